@@ -101,7 +101,7 @@ def build_python_module() -> str:
     cmd += [f"-I{p}" for p in inc]
     cmd += [os.path.join(CSRC, "binding.cpp"), "-o", out,
             f"-L{HERE}", "-lsma_hip", "-Wl,-rpath,$ORIGIN",
-            f"-L{torch_lib}", "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_python",
+            f"-L{torch_lib}", "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python",
             f"-Wl,-rpath,{torch_lib}"]
     _run(cmd)
     return out

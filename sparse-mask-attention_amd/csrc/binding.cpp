@@ -16,6 +16,10 @@
 //       instead of pack_mask + forward; `packed_out`, if given, receives what pack_mask would
 //       return and `map_out` what tile_map would return for it; `bool_mask_supported(q, k, v, mask)`
 //       says whether it applies)
+//   attention(q, k, v, mask, mask_packed, tile_map, autograd) -> Tensor or None   (not in the reference:
+//       everything python/sparse_attention.py does for one call - conversions, padding, allocation,
+//       launches and the autograd node - without returning to Python in between; None when an
+//       argument is not what the Python layer's own checks demand, which then say what is wrong)
 //
 // Differences, all on the safe side: `lse` may be None (the reference's own inference wrapper
 // passes None, python/sparse_attention.py:170-171); every tensor argument is checked (device,
@@ -28,8 +32,16 @@
 // entries / heads.
 // This file is host-only C++ (compiled by g++); all GPU code lives behind include/sma.h.
 #include <torch/extension.h>
+#include <ATen/EmptyTensor.h>
+#include <ATen/hip/impl/HIPCachingAllocatorMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/python_cpp_function.h>
+#include <torch/csrc/autograd/saved_variable.h>
+
+#include <cmath>
+#include <mutex>
 
 #include "sma.h"
 
@@ -38,6 +50,20 @@ namespace {
 void check_status(int st, const char *what)
 {
     TORCH_CHECK(st == SMA_OK, what, " failed: ", sma_strerror(st), " (code ", st, ")");
+}
+
+// Uninitialised tensors straight from PyTorch's caching allocator of the current device (the callers
+// hold the device guard), without the dispatcher in between.
+torch::Tensor empty_rows(c10::IntArrayRef sizes, c10::IntArrayRef strides, at::ScalarType dtype)
+{
+    static c10::Allocator *const allocator = c10::hip::HIPCachingAllocatorMasqueradingAsCUDA::get();
+    return torch::Tensor(at::detail::empty_strided_generic(sizes, strides, allocator, c10::DispatchKeySet(c10::DispatchKey::CUDA), dtype));
+}
+
+torch::Tensor empty_dense(c10::IntArrayRef sizes, at::ScalarType dtype)
+{
+    static c10::Allocator *const allocator = c10::hip::HIPCachingAllocatorMasqueradingAsCUDA::get();
+    return torch::Tensor(at::detail::empty_generic(sizes, allocator, c10::DispatchKeySet(c10::DispatchKey::CUDA), dtype, c10::nullopt));
 }
 
 // Descriptor of a [B,H,N,D] tensor for the strided C entry points.  Extents of size 1 get stride 0
@@ -248,7 +274,7 @@ void backward(const torch::Tensor &dout, const torch::Tensor &q, const torch::Te
     const uint32_t *map_ptr = map_pointer(tile_map, mask_packed, q);
 
     const c10::DeviceGuard guard(q.device());
-    torch::Tensor delta = torch::empty({B, H, N}, lse.options());      // workspace of the C entry point
+    torch::Tensor delta = empty_dense({B, H, N}, at::kFloat);      // workspace of the C entry point
     hipStream_t stream = c10::hip::getCurrentHIPStream(q.device().index()).stream();
     const int st = sma_attn_bwd_map_strided(&d[0], &d[1], &d[2], &d[3], &d[4], lse.data_ptr<float>(),
                                             reinterpret_cast<const uint32_t *>(mask_packed.data_ptr<int32_t>()),
@@ -270,7 +296,7 @@ torch::Tensor pack_mask(const torch::Tensor &mask)
     TORCH_CHECK(B <= INT32_MAX && H <= INT32_MAX && N <= INT32_MAX, "extent too large");
     const c10::DeviceGuard guard(m.device());
     // Every word is written by the kernel, so no zero-fill is needed.
-    torch::Tensor packed = torch::empty({B, H, N, (N + 31) / 32}, m.options().dtype(torch::kInt32));
+    torch::Tensor packed = empty_dense({B, H, N, (N + 31) / 32}, at::kInt);
     hipStream_t stream = c10::hip::getCurrentHIPStream(m.device().index()).stream();
     const int st = sma_pack_mask(reinterpret_cast<const uint8_t *>(m.data_ptr<bool>()),
                                  reinterpret_cast<uint32_t *>(packed.data_ptr<int32_t>()), (int)B,
@@ -290,12 +316,262 @@ torch::Tensor tile_map(const torch::Tensor &mask_packed)
     TORCH_CHECK(B <= INT32_MAX && H <= INT32_MAX && N <= 131072, "extent too large");
     const int64_t T = (N + 63) / 64;
     const c10::DeviceGuard guard(mask_packed.device());
-    torch::Tensor map = torch::empty({B, H, T, 2, (T + 31) / 32}, mask_packed.options());    // every word is written
+    torch::Tensor map = empty_dense({B, H, T, 2, (T + 31) / 32}, at::kInt);    // every word is written
     hipStream_t stream = c10::hip::getCurrentHIPStream(mask_packed.device().index()).stream();
     const int st = sma_tile_map(reinterpret_cast<const uint32_t *>(mask_packed.data_ptr<int32_t>()),
                                 reinterpret_cast<uint32_t *>(map.data_ptr<int32_t>()), (int)B, (int)H, (int)N, stream);
     check_status(st, "sma_tile_map");
     return map;
+}
+
+// ---- one call of the Python layer, whole --------------------------------------------------------
+//
+// What bounds a small call is the host, not the GPU: the kernels of a 128-token request take 5 us,
+// the same steps written in Python 11 us for the forward and 105 us for forward + backward (measured
+// with 3 kernels of 10 us each in flight).  So the conversions, the allocations, the choice of the
+// kernel and the autograd node live here; Python only calls `attention` and, when it declines,
+// explains why.
+
+using torch::Tensor;
+
+// An uninitialised tensor like t (its strides too, where they leave no gaps), what torch.empty_like gives.
+Tensor empty_like_rows(const Tensor &t)
+{
+    if (t.is_contiguous()) return empty_dense(t.sizes(), t.scalar_type());
+    if (t.is_non_overlapping_and_dense()) return empty_rows(t.sizes(), t.strides(), t.scalar_type());
+    return at::empty_like(t.detach());
+}
+
+// Whether the kernels can address t as it is: contiguous last dimension, the strides of the others
+// non-negative multiples of 8 elements, 16-byte aligned storage.
+bool addressable(const Tensor &t)
+{
+    if (t.stride(3) != 1 && t.size(3) != 1) return false;
+    if (reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 != 0) return false;
+    for (int d = 0; d < 3; ++d)
+        if (t.size(d) > 1 && (t.stride(d) < 0 || t.stride(d) % 8 != 0)) return false;
+    return true;
+}
+
+// q, k, v or a gradient as the kernels take it: 16-bit elements of type `dtype`, head dim Dk (zeros
+// after the tensor's own), addressable.
+Tensor kernel_rows(const Tensor &t, at::ScalarType dtype, int64_t Dk)
+{
+    Tensor r = t.scalar_type() == dtype ? t : t.to(dtype);
+    if (r.size(3) != Dk) return at::constant_pad_nd(r, {0, Dk - r.size(3)});
+    return addressable(r) ? r : r.contiguous();
+}
+
+// The mask with its expanded (stride 0) batch / head extents taken back to 1: it is then read once
+// and shared.
+Tensor unexpand(Tensor m)
+{
+    if (m.size(0) > 1 && m.stride(0) == 0) m = m.narrow(0, 0, 1);
+    if (m.size(1) > 1 && m.stride(1) == 0) m = m.narrow(1, 0, 1);
+    return m.is_contiguous() ? m : m.contiguous();
+}
+
+struct Call {                       // one problem as the kernels see it
+    Tensor q, k, v;                 // kernel_rows of the caller's
+    Tensor mask;                    // the boolean mask, unexpanded; undefined if only the packed one is there
+    Tensor packed, map;             // packed mask and tile map, either may be undefined
+    int64_t B, H, N, D;             // the caller's extents
+    double scale;
+};
+
+// Forward of `c` into `out`; with `lse` defined, the packed mask is left in c.packed and, if
+// `want_map`, the tile map in c.map, for the backward.
+void run_forward(Call &c, Tensor &out, const Tensor &lse, bool want_map)
+{
+    const bool training = lse.defined();
+    const c10::optional<Tensor> lse_arg = training ? c10::optional<Tensor>(lse) : c10::nullopt;
+    if (!c.packed.defined() && bool_mask_supported(c.q, c.k, c.v, c.mask)) {
+        c10::optional<Tensor> packed_out, map_out;
+        if (training) {
+            const int64_t T = (c.N + 63) / 64;
+            c.packed = empty_dense({c.mask.size(0), c.mask.size(1), c.N, (c.N + 31) / 32}, at::kInt);
+            packed_out = c.packed;
+            if (want_map) {
+                c.map = empty_dense({c.mask.size(0), c.mask.size(1), T, 2, (T + 31) / 32}, at::kInt);
+                map_out = c.map;
+            }
+        }
+        forward_bool_mask(c.q, c.k, c.v, c.mask, out, lse_arg, c.scale, training, packed_out, map_out);
+        return;
+    }
+    if (!c.packed.defined()) {
+        c.packed = pack_mask(c.mask);
+        if (training && want_map) c.map = tile_map(c.packed);
+    }
+    forward(c.q, c.k, c.v, c.packed, out, lse_arg, c.scale, training,
+            c.map.defined() ? c10::optional<Tensor>(c.map) : c10::nullopt);
+}
+
+// The autograd node of one training forward.
+struct SparseAttentionBackward : public torch::autograd::Node {
+    std::mutex mutex;
+    torch::autograd::SavedVariable q, k, v, out, lse, packed;
+    Tensor map;                     // undefined without a tile map
+    double scale = 1.0;
+    at::ScalarType grad_dtype = at::kHalf;      // what the caller's q, k, v are made of ...
+    int64_t grad_D = 0;                         // ... and their head dim
+    bool out_is_output = false;     // `out` is the tensor handed to the caller (nothing was converted)
+
+    std::string name() const override { return "SparseAttentionFunctionBackward"; }
+
+    void release_variables() override
+    {
+        std::lock_guard<std::mutex> lock(mutex);
+        for (torch::autograd::SavedVariable *s : {&q, &k, &v, &out, &lse, &packed}) s->reset_data();
+        map.reset();
+    }
+
+    torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override
+    {
+        if (!grads[0].defined()) return {Tensor(), Tensor(), Tensor()};
+        std::lock_guard<std::mutex> lock(mutex);
+        const Tensor tq = q.unpack(), tk = k.unpack(), tv = v.unpack();
+        const Tensor tout = out.unpack(out_is_output ? shared_from_this() : nullptr);
+        const Tensor tlse = lse.unpack(), tpacked = packed.unpack();
+        at::NoGradGuard no_grad;
+        const c10::DeviceGuard guard(tq.device());
+        const Tensor dout = kernel_rows(grads[0], tq.scalar_type(), tq.size(3));
+        Tensor d[3] = {empty_like_rows(tq), empty_like_rows(tk), empty_like_rows(tv)};
+        backward(dout, tq, tk, tv, tout, tlse, tpacked, d[0], d[1], d[2], scale,
+                 map.defined() ? c10::optional<Tensor>(map) : c10::nullopt);
+        for (Tensor &t : d) {
+            if (t.size(3) != grad_D) t = t.narrow(3, 0, grad_D);
+            if (t.scalar_type() != grad_dtype) t = t.to(grad_dtype);
+        }
+        return {d[0], d[1], d[2]};
+    }
+};
+
+// Output of one call: out, with its autograd node when q, k or v want gradients and `autograd`.
+Tensor run_call(const Tensor &q, const Tensor &k, const Tensor &v, Call &c, bool want_map, bool autograd)
+{
+    const at::ScalarType dtype = q.scalar_type();
+    const at::ScalarType kdt = dtype == at::kFloat ? at::kBFloat16 : dtype;
+    const int64_t Dk = c.D <= 32 ? 32 : (c.D <= 64 ? 64 : 128);
+    const bool tracked = autograd && torch::autograd::compute_requires_grad(q, k, v);
+    std::shared_ptr<SparseAttentionBackward> node;
+    if (tracked) {
+        node = std::make_shared<SparseAttentionBackward>();
+        node->set_next_edges(torch::autograd::collect_next_edges(q, k, v));
+    }
+    const c10::DeviceGuard guard(q.device());
+    at::AutoDispatchBelowADInplaceOrView below_autograd;
+    c.q = kernel_rows(q, kdt, Dk);
+    c.k = kernel_rows(k, kdt, Dk);
+    c.v = kernel_rows(v, kdt, Dk);
+    Tensor out = empty_like_rows(c.q), lse;
+    if (tracked) lse = empty_dense({c.B, c.H, c.N}, at::kFloat);
+    run_forward(c, out, lse, want_map);
+    Tensor result = out;
+    if (Dk != c.D) result = result.narrow(3, 0, c.D);
+    if (kdt != dtype) result = result.to(dtype);
+    if (!tracked) return result;
+    torch::autograd::set_history(result, node);
+    node->out_is_output = result.is_same(out);
+    node->q = torch::autograd::SavedVariable(c.q, false);
+    node->k = torch::autograd::SavedVariable(c.k, false);
+    node->v = torch::autograd::SavedVariable(c.v, false);
+    node->out = torch::autograd::SavedVariable(out, node->out_is_output);
+    node->lse = torch::autograd::SavedVariable(lse, false);
+    node->packed = torch::autograd::SavedVariable(c.packed, false);
+    node->map = c.map;
+    node->scale = c.scale;
+    node->grad_dtype = dtype;
+    node->grad_D = c.D;
+    return result;
+}
+
+// sparse_attention / sparse_attention_func of the Python layer.  `tile_map` is None, True (leave a map
+// behind for the backward) or a tensor.  None is returned, before anything has been done, for
+// arguments that the Python layer refuses or has to prepare first (a boolean mask shorter than one
+// 16-byte copy per row is packed there).
+c10::optional<Tensor> attention(const Tensor &q, const Tensor &k, const Tensor &v, const c10::optional<Tensor> &mask,
+                                const c10::optional<Tensor> &mask_packed, const py::object &tile_map, bool autograd)
+{
+    const at::ScalarType dtype = q.scalar_type();
+    if (!q.is_cuda() || q.dim() != 4 || k.sizes() != q.sizes() || v.sizes() != q.sizes() || k.device() != q.device() ||
+        v.device() != q.device())
+        return c10::nullopt;
+    if (dtype == at::kHalf || dtype == at::kBFloat16) {
+        if (k.scalar_type() != dtype || v.scalar_type() != dtype) return c10::nullopt;
+    } else if (dtype != at::kFloat) {
+        return c10::nullopt;
+    }
+    Call c;
+    c.B = q.size(0), c.H = q.size(1), c.N = q.size(2), c.D = q.size(3);
+    if (c.D < 1 || c.D > 128) return c10::nullopt;
+    auto shared_or = [](int64_t have, int64_t want) { return have == 1 || have == want; };
+    const bool want_map = tile_map.ptr() == Py_True;
+    const bool has_map = !want_map && !tile_map.is_none();
+    if (mask_packed.has_value() && mask_packed->defined()) {
+        const Tensor &p = *mask_packed;
+        if (p.scalar_type() != at::kInt || p.dim() != 4 || !shared_or(p.size(0), c.B) || !shared_or(p.size(1), c.H) ||
+            p.size(2) != c.N || p.size(3) != (c.N + 31) / 32 || p.device() != q.device() || (want_map && autograd))
+            return c10::nullopt;
+        c.packed = p;
+        if (has_map) c.map = tile_map.cast<Tensor>();
+    } else {
+        if (!mask.has_value() || !mask->defined() || has_map) return c10::nullopt;
+        const Tensor &m = *mask;
+        if (m.scalar_type() != at::kBool || m.device() != q.device() || m.dim() != 4 || !shared_or(m.size(0), c.B) ||
+            !shared_or(m.size(1), c.H) || m.size(2) != c.N || m.size(3) != c.N || (c.N < 16 && q.numel() > 0))
+            return c10::nullopt;
+        c.mask = unexpand(m);
+    }
+    c.scale = 1.0 / std::sqrt((double)c.D);
+    return run_call(q, k, v, c, want_map, autograd);
+}
+
+// SparseAttentionFunction.apply of the Python layer: the same with the scale given and q, k, v in a
+// head dim and type that the kernels have.
+Tensor attention_function(const Tensor &q, const Tensor &k, const Tensor &v, const c10::optional<Tensor> &mask_packed,
+                          const c10::optional<Tensor> &mask, double scale, const py::object &tile_map)
+{
+    TORCH_CHECK(q.dim() == 4 && k.sizes() == q.sizes() && v.sizes() == q.sizes(), "q, k, v must have the same 4D shape");
+    Call c;
+    c.B = q.size(0), c.H = q.size(1), c.N = q.size(2), c.D = q.size(3);
+    const bool want_map = tile_map.ptr() == Py_True;
+    if (mask_packed.has_value() && mask_packed->defined()) {
+        c.packed = *mask_packed;
+        if (!want_map && !tile_map.is_none()) c.map = tile_map.cast<Tensor>();
+    } else {
+        TORCH_CHECK(mask.has_value() && mask->defined() && mask->dim() == 4, "a mask or a packed mask is needed");
+        c.mask = unexpand(*mask);
+    }
+    c.scale = scale;
+    return run_call(q, k, v, c, want_map, true);
+}
+
+// The Python type of the node, so that grad_fn shows what it carries.
+PyObject *node_tile_map(PyObject *self, void *)
+{
+    const auto *node = static_cast<SparseAttentionBackward *>(reinterpret_cast<torch::autograd::THPCppFunction *>(self)->cdata.get());
+    if (!node->map.defined()) Py_RETURN_NONE;
+    return THPVariable_Wrap(node->map);
+}
+
+PyObject *node_scale(PyObject *self, void *)
+{
+    const auto *node = static_cast<SparseAttentionBackward *>(reinterpret_cast<torch::autograd::THPCppFunction *>(self)->cdata.get());
+    return PyFloat_FromDouble(node->scale);
+}
+
+void register_node_type()
+{
+    using namespace torch::autograd;
+    static PyTypeObject type;
+    static PyGetSetDef properties[] = {THP_FUNCTION_DEFAULT_PROPERTIES,
+                                       {"tile_map", node_tile_map, nullptr, nullptr, nullptr},
+                                       {"scale", node_scale, nullptr, nullptr, nullptr},
+                                       {nullptr, nullptr, nullptr, nullptr, nullptr}};
+    _initFunctionPyTypeObject(type, "SparseAttentionFunctionBackward", properties, nullptr);
+    Py_INCREF(&type);
+    registerCppFunction(typeid(SparseAttentionBackward), &type);
 }
 
 }  // namespace
@@ -323,5 +599,11 @@ PYBIND11_MODULE(sparse_attn_cuda, m)
           py::arg("k"), py::arg("v"), py::arg("mask"));
     m.def("pack_mask", &pack_mask, "Pack a bool mask into uint32 words (returned as int32)",
           py::arg("mask"));
+    m.def("attention", &attention, "One call of the Python layer; None if its arguments need the checks made there",
+          py::arg("q"), py::arg("k"), py::arg("v"), py::arg("mask"), py::arg("mask_packed"), py::arg("tile_map"),
+          py::arg("autograd"));
+    m.def("attention_function", &attention_function, "Forward with an autograd node, scale given", py::arg("q"),
+          py::arg("k"), py::arg("v"), py::arg("mask_packed"), py::arg("mask"), py::arg("scale"), py::arg("tile_map"));
+    register_node_type();
     m.def("version", []() { return sma_version(); });
 }

@@ -56,7 +56,6 @@ import os
 import sys
 
 import torch
-from torch.autograd import Function
 
 _PKG_DIR = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 if _PKG_DIR not in sys.path:
@@ -107,56 +106,22 @@ def sparse_attention_ref(q, k, v, mask):
 # autograd
 # ----------------------------------------------------------------------------------------------
 
-class SparseAttentionFunction(Function):
+class SparseAttentionFunction:
     """forward = fused HIP kernel (saves LSE); backward = the HIP dQ and dK/dV kernels.
+
+    The autograd node itself is native (csrc/binding.cpp, SparseAttentionBackward): in a small training
+    step the host is what takes time, and a node written in Python made it twice as long.
 
     ``mask_packed`` may be None: the mask is then read as it is by the one-launch forward, which
     leaves the packed words the backward uses (and, with ``tile_map=True``, the mask's tile map) as
-    by-products, or packed first where that kernel does not apply."""
+    by-products, or packed first where that kernel does not apply.  ``tile_map=True`` is not the
+    default because a mask without empty blocks (any random one) would pay for a by-product that
+    nothing can use."""
 
     @staticmethod
-    def forward(ctx, q, k, v, mask_packed, mask_bool, scale, seq_len, tile_map=None):
+    def apply(q, k, v, mask_packed, mask_bool, scale, seq_len, tile_map=None):
         _require_ext(q)
-        B, H, N, _ = q.shape
-        q, k, v = _rows(q), _rows(k), _rows(v)
-        out = torch.empty_like(q)
-        lse = torch.empty(B, H, N, device=q.device, dtype=torch.float32)
-        if mask_packed is None:
-            mask_bool = _unexpand(mask_bool)
-            if sparse_attn_cuda.bool_mask_supported(q, k, v, mask_bool):
-                mask_packed = torch.empty(mask_bool.shape[0], mask_bool.shape[1], N, (N + 31) // 32,
-                                          device=q.device, dtype=torch.int32)
-                # tile_map=True: the caller says the mask has empty 64 x 64 blocks; the same launch
-                # then leaves the mask's tile map behind and the backward visits only the blocks
-                # that hold something.  Not by default: a mask without empty blocks (any random one)
-                # would pay for a by-product that nothing can use.
-                if tile_map is True:
-                    T = (N + 63) // 64
-                    tile_map = torch.empty(mask_bool.shape[0], mask_bool.shape[1], T, 2, (T + 31) // 32,
-                                           device=q.device, dtype=torch.int32)
-                else:
-                    tile_map = None
-                sparse_attn_cuda.forward_bool_mask(q, k, v, mask_bool, out, lse, scale, True, mask_packed, tile_map)
-                ctx.save_for_backward(q, k, v, out, lse, mask_packed)
-                ctx.scale = scale
-                ctx.tile_map = tile_map
-                return out
-            mask_packed = pack_mask(mask_bool)
-            tile_map = sparse_attn_cuda.tile_map(mask_packed) if tile_map is True else None
-        sparse_attn_cuda.forward(q, k, v, mask_packed, out, lse, scale, True, tile_map)
-        ctx.save_for_backward(q, k, v, out, lse, mask_packed)
-        ctx.scale = scale
-        ctx.tile_map = tile_map
-        return out
-
-    @staticmethod
-    def backward(ctx, dout):
-        q, k, v, out, lse, mask_packed = ctx.saved_tensors
-        dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-        # the call the reference makes at python/sparse_attention.py:91-94
-        sparse_attn_cuda.backward(_rows(dout.to(q.dtype)), q, k, v, out, lse, mask_packed,
-                                  dq, dk, dv, ctx.scale, getattr(ctx, "tile_map", None))
-        return dq, dk, dv, None, None, None, None, None
+        return sparse_attn_cuda.attention_function(q, k, v, mask_packed, mask_bool, scale, tile_map)
 
 
 def backward_recompute(q, k, v, out, lse, mask_bool, dout, scale):
@@ -209,17 +174,26 @@ def _unexpand(mask: torch.Tensor) -> torch.Tensor:
 
 
 
-
-
-def _pad_head_dim(q, k, v):
-    """q, k, v with their head dim zero-padded to the next one the kernels have (32, 64 or 128)."""
-    D = q.shape[-1]
-    assert 1 <= D <= 128, "head_dim must be at most 128"
-    Dk = 32 if D <= 32 else (64 if D <= 64 else 128)
-    if D == Dk:
-        return q, k, v
-    pad = (0, Dk - D)
-    return tuple(torch.nn.functional.pad(t, pad) for t in (q, k, v))
+def _declined(q, k, v, mask, mask_packed, tile_map, autograd):
+    """What ``sparse_attn_cuda.attention`` did not take: the checks that say what is wrong with the
+    arguments, and the one thing it leaves to be done beforehand, packing a mask of fewer than 16 columns
+    (shorter than one copy of the kernel that reads the boolean mask)."""
+    _check_inputs(q, k, v, mask, mask_packed)
+    if autograd:
+        assert tile_map is None or tile_map is True or mask_packed is not None, "a tile_map tensor belongs to a mask_packed"
+        assert not (tile_map is True and mask_packed is not None), "with mask_packed, pass the result of tile_map(mask_packed)"
+    else:
+        assert tile_map is None or tile_map is True or mask_packed is not None, "tile_map belongs to a mask_packed"
+    _require_ext(q)
+    assert 1 <= q.shape[-1] <= 128, "head_dim must be at most 128"
+    if mask_packed is None and q.shape[2] < 16:
+        mask_packed = pack_mask(_unexpand(mask))
+        if tile_map is True:
+            tile_map = sparse_attn_cuda.tile_map(mask_packed) if autograd else None
+    out = sparse_attn_cuda.attention(q, k, v, None, mask_packed, tile_map, autograd) if mask_packed is not None else None
+    if out is None:
+        raise RuntimeError("Unsupported dtype, need BF16 or FP16 (or FP32), the same for q, k and v, on one device")
+    return out
 
 
 def sparse_attention(q, k, v, mask, mask_packed=None, tile_map=None):
@@ -237,59 +211,14 @@ def sparse_attention(q, k, v, mask, mask_packed=None, tile_map=None):
     the forward then leaves the map behind for the backward (about 1 us at N = 512; off by default,
     because a mask without empty blocks gains nothing from it).
     """
-    _check_inputs(q, k, v, mask, mask_packed)
-    assert tile_map is None or tile_map is True or mask_packed is not None, "a tile_map tensor belongs to a mask_packed"
-    assert not (tile_map is True and mask_packed is not None), "with mask_packed, pass the result of tile_map(mask_packed)"
-    _require_ext(q)
-    if not (torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)):
-        # nothing will be differentiated: no LSE, and the mask can be read without packing it
-        return sparse_attention_func(q, k, v, mask, mask_packed, tile_map)
-    B, H, N, D = q.shape
-    scale = 1.0 / math.sqrt(D)
-
-    orig_dtype = q.dtype
-    if orig_dtype == torch.float32:
-        q, k, v = q.bfloat16(), k.bfloat16(), v.bfloat16()
-
-    q, k, v = _pad_head_dim(q, k, v)              # differentiable: the gradients are sliced back
-    out = SparseAttentionFunction.apply(q, k, v, mask_packed, mask, scale, N, tile_map)[..., :D]
-
-    if orig_dtype == torch.float32:
-        out = out.float()
-    return out
+    out = sparse_attn_cuda.attention(q, k, v, mask, mask_packed, tile_map, True) if HAS_CUDA_EXT else None
+    return out if out is not None else _declined(q, k, v, mask, mask_packed, tile_map, True)
 
 
 def sparse_attention_func(q, k, v, mask, mask_packed=None, tile_map=None):
     """Inference-only variant of :func:`sparse_attention`: no autograd graph, no LSE."""
-    _check_inputs(q, k, v, mask, mask_packed)
-    if tile_map is True:        # a hint for the backward only
-        tile_map = None
-    assert tile_map is None or mask_packed is not None, "tile_map belongs to a mask_packed"
-    _require_ext(q)
-    D = q.shape[-1]
-    scale = 1.0 / math.sqrt(D)
-
-    orig_dtype = q.dtype
-    if orig_dtype == torch.float32:
-        q, k, v = q.bfloat16(), k.bfloat16(), v.bfloat16()
-
-    with torch.no_grad():
-        q, k, v = _pad_head_dim(q, k, v)
-        q, k, v = _rows(q), _rows(k), _rows(v)
-        if mask_packed is None:
-            mask = _unexpand(mask)
-            if sparse_attn_cuda.bool_mask_supported(q, k, v, mask):
-                out = torch.empty_like(q)
-                sparse_attn_cuda.forward_bool_mask(q, k, v, mask, out, None, scale, False)
-                return (out[..., :D].float() if orig_dtype == torch.float32 else out[..., :D])
-            mask_packed = pack_mask(mask)
-        out = torch.empty_like(q)
-        sparse_attn_cuda.forward(q, k, v, mask_packed, out, None, scale, False, tile_map)
-        out = out[..., :D]
-
-    if orig_dtype == torch.float32:
-        out = out.float()
-    return out
+    out = sparse_attn_cuda.attention(q, k, v, mask, mask_packed, tile_map, False) if HAS_CUDA_EXT else None
+    return out if out is not None else _declined(q, k, v, mask, mask_packed, tile_map, False)
 
 
 # ----------------------------------------------------------------------------------------------
