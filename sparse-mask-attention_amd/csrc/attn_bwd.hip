@@ -167,7 +167,7 @@ __global__ __launch_bounds__(NTHREADS, HDIM == 128 ? 2 : 3) void attn_bwd_dq_ker
     const int l32 = lane & 31, hh = lane >> 5;
     const int nid = renumber_block();
     const int bh = (int)fastdiv((uint32_t)nid, a.div_qtiles);
-    const int qt = nid - bh * a.qtiles;
+    const int qt = a.qtiles - 1 - (nid - bh * a.qtiles);      // last rows first, as in the forward
     const int N = a.N, nw = (N + 31) >> 5;
     const int T = (N + BN - 1) / BN;
     const bool ragged = (N & (BN - 1)) != 0;

@@ -138,7 +138,9 @@ __global__ __launch_bounds__(NTHREADS, HDIM == 128 ? 2 : 3) void attn_fwd_kernel
 
     const int nid = renumber_block();
     const int bh = (int)fastdiv((uint32_t)nid, a.div_qtiles);
-    const int qt = nid - bh * a.qtiles;
+    // last rows first: where rows keep more keys the later they come (causal masks), the longest
+    // work-groups of a head start first and the shortest fill the end of the launch
+    const int qt = a.qtiles - 1 - (nid - bh * a.qtiles);
     const int N = a.N, nw = (N + 31) >> 5;
     const int T = (N + BN - 1) / BN;
     const bool ragged = (N & (BN - 1)) != 0;

@@ -117,13 +117,17 @@ int sma_device_check(void *stream)
 int sma_pack_mask_map(const uint8_t *mask, uint32_t *packed, uint32_t *tile_map, int B, int H, int N,
                       void *stream)
 {
-    // what sma_tile_map would refuse is refused before anything is written
-    if (tile_map != nullptr && B >= 0 && H >= 0 &&
-        (N > 131072 || !below_2_31((long long)B * H, (N + 63) / 64) || misaligned(tile_map, 4)))
-        return misaligned(tile_map, 4) ? SMA_ERR_ALIGNMENT : SMA_ERR_BAD_SHAPE;
-    const int st = sma_pack_mask(mask, packed, B, H, N, stream);
-    if (st != SMA_OK || tile_map == nullptr) return st;
-    return sma_tile_map(packed, tile_map, B, H, N, stream);
+    if (tile_map == nullptr) return sma_pack_mask(mask, packed, B, H, N, stream);
+    if (B < 0 || H < 0 || N < 0) return SMA_ERR_BAD_SHAPE;
+    const long long slabs = (long long)B * H;
+    if (misaligned(tile_map, 4)) return SMA_ERR_ALIGNMENT;
+    if (N > 131072 || !below_2_31(slabs, (N + 63) / 64)) return SMA_ERR_BAD_SHAPE;
+    if (slabs == 0 || N == 0) return SMA_OK;
+    if (mask == nullptr || packed == nullptr) return SMA_ERR_NULL_POINTER;
+    if (!below_2_31(slabs, N) || !below_2_31(slabs * N, (N + 31) / 32)) return SMA_ERR_BAD_SHAPE;
+    if (misaligned(packed, 4)) return SMA_ERR_ALIGNMENT;
+    const hipError_t e = sma::launch_pack_mask_map(mask, packed, tile_map, slabs, N, static_cast<hipStream_t>(stream));
+    return e == hipSuccess ? SMA_OK : SMA_ERR_LAUNCH;
 }
 
 int sma_pack_mask(const uint8_t *mask, uint32_t *packed, int B, int H, int N, void *stream)

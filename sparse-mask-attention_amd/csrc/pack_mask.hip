@@ -252,6 +252,73 @@ __global__ __launch_bounds__(64) void unaligned_probe_kernel(unsigned char *src,
 // thread ORs what its words say into per-key-tile flags in LDS, and the first tw threads write the
 // words.  No atomics on global memory, nothing to clear beforehand, deterministic.
 constexpr int MAP_MAX_TW = 64;      // key tiles per query tile <= 2048, i.e. N <= 131072
+
+// Packed words and tile map in one pass over the mask, N >= 8 at any address.  One work-group per
+// 64 rows x 512 columns: exactly one byte (8 key tiles) of a block row's "some" and "full" words,
+// so no two work-groups share a byte and nothing is combined through memory.  Each of the 8
+// wavefronts packs 8 rows like pack_row_kernel (four 8-byte loads in flight per lane) and keeps the
+// OR of what its lanes saw; eight neighbouring lanes are one key tile.  Bound by the latency of
+// two rounds of loads when the mask is small, by HBM when it is large (1 byte in per entry):
+// [1, 1, 4096, 4096] in 6 us, [16, 12, 1024, 1024] in 35 us (6.4 TB/s), in place of two launches.
+constexpr int PACK_MAP_THREADS = 512;
+__global__ __launch_bounds__(PACK_MAP_THREADS) void pack_map_kernel(const uint8_t *__restrict__ mask,
+                                                                    uint32_t *__restrict__ packed,
+                                                                    uint8_t *__restrict__ map, int N, int nw,
+                                                                    int qblocks, int segs, int tw)
+{
+    __shared__ unsigned long long flags[PACK_MAP_THREADS / 64][2];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int rb = blockIdx.x / segs, seg = blockIdx.x - rb * segs;       // rb: slab * qblocks + block of 64 rows
+    const int slab = rb / qblocks, qb = rb - slab * qblocks;
+    const int col = seg * 512 + lane * 8;
+    const int over = col + 8 - N;                       // columns of this lane's eight that lie beyond the row
+    const uint32_t valid = over <= 0 ? 0xffu : (over < 8 ? 0xffu >> over : 0u);
+    const int w = seg * 16 + (lane >> 2);
+    bool some = false, hole = false;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        u32x2 d[4];
+        const uint8_t *p[4];
+        const int row0 = qb * 64 + wave * 8 + s * 4;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {                   // rows beyond N repeat row N - 1 and change nothing
+            const int row = row0 + u < N ? row0 + u : N - 1;
+            p[u] = mask + ((size_t)slab * N + row) * N + (over <= 0 ? col : N - 8);
+        }
+        load8_any(d, p);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            uint64_t v = ((uint64_t)d[u].y << 32) | d[u].x;
+            if (over > 0) v = over < 8 ? v >> (8 * over) : 0ull;
+            uint32_t b = __builtin_amdgcn_udot4(nonzero_bytes((uint32_t)v), 0x08040201u, 0u, false);
+            b = __builtin_amdgcn_udot4(nonzero_bytes((uint32_t)(v >> 32)), 0x80402010u, b, false);
+            some |= b != 0u;
+            hole |= b != valid;
+            b <<= 8 * (lane & 3);
+            b |= __shfl_xor(b, 1, 64);
+            b |= __shfl_xor(b, 2, 64);
+            if (row0 + u < N && (lane & 3) == 0 && w < nw) packed[((size_t)slab * N + row0 + u) * nw + w] = b;
+        }
+    }
+    const unsigned long long bs = __builtin_amdgcn_ballot_w64(some), bh = __builtin_amdgcn_ballot_w64(hole);
+    if (lane == 0) { flags[wave][0] = bs; flags[wave][1] = bh; }
+    __syncthreads();
+    // thread 0: "some", thread 1: "full"; the last segment also clears what is left of its word
+    if (threadIdx.x < 2) {
+        unsigned long long f = 0ull;
+        for (int i = 0; i < PACK_MAP_THREADS / 64; ++i) f |= flags[i][threadIdx.x];
+        uint32_t bits = 0u;
+        for (int i = 0; i < 8; ++i) bits |= (((f >> (8 * i)) & 0xffull) != 0ull) ? 1u << i : 0u;
+        const int tiles = (N - seg * 512 + 63) / 64;
+        const uint32_t in_range = tiles >= 8 ? 0xffu : (1u << tiles) - 1u;
+        if (threadIdx.x == 1) bits = ~bits;
+        uint8_t *dst = map + ((size_t)rb * 2 + threadIdx.x) * 4 * tw;
+        dst[seg] = (uint8_t)(bits & in_range);
+        if (seg == segs - 1)
+            for (int i = segs; i < 4 * tw; ++i) dst[i] = 0;
+    }
+}
+
 __global__ __launch_bounds__(PACK_THREADS) void tile_map_kernel(const uint32_t *__restrict__ packed,
                                                                 uint32_t *__restrict__ map,
                                                                 int N, int nw, int qblocks, int tw)
@@ -287,6 +354,21 @@ __global__ __launch_bounds__(PACK_THREADS) void tile_map_kernel(const uint32_t *
 }
 
 }  // namespace
+
+hipError_t launch_pack_mask_map(const uint8_t *mask, uint32_t *packed, uint32_t *map, long long slabs, int N,
+                                hipStream_t stream)
+{
+    if (slabs == 0 || N == 0) return hipSuccess;
+    const int nw = (N + 31) / 32, qblocks = (N + 63) / 64, tw = (qblocks + 31) / 32, segs = (N + 511) / 512;
+    const long long groups = slabs * qblocks * segs;
+    if (N < 8 || groups >= (1ll << 31) || unaligned_access_state(stream) == 0) {
+        const hipError_t e = launch_pack_mask(mask, packed, slabs * N, N, stream);
+        return e == hipSuccess ? launch_tile_map(packed, map, slabs, N, stream) : e;
+    }
+    hipLaunchKernelGGL(pack_map_kernel, dim3((unsigned)groups), dim3(PACK_MAP_THREADS), 0, stream, mask, packed,
+                       reinterpret_cast<uint8_t *>(map), N, nw, qblocks, segs, tw);
+    return hipGetLastError();
+}
 
 hipError_t launch_tile_map(const uint32_t *packed, uint32_t *map, long long slabs, int N, hipStream_t stream)
 {

@@ -103,4 +103,8 @@ int unaligned_access_state(hipStream_t stream);
 // tile map [slabs, ceil(N/64), 2, ceil(ceil(N/64)/32)] of packed words [slabs, N, ceil(N/32)]
 hipError_t launch_tile_map(const uint32_t *packed, uint32_t *map, long long slabs, int N, hipStream_t stream);
 
+// both of the above in one pass over the mask
+hipError_t launch_pack_mask_map(const uint8_t *mask, uint32_t *packed, uint32_t *map, long long slabs, int N,
+                                hipStream_t stream);
+
 }  // namespace sma
