@@ -24,7 +24,7 @@ extern "C" {
 #define SMA_OK                 0
 #define SMA_ERR_NULL_POINTER  -1   /* a required pointer is NULL */
 #define SMA_ERR_BAD_SHAPE     -2   /* a negative extent, or an extent beyond the 32-bit index range */
-#define SMA_ERR_HEAD_DIM      -3   /* head_dim other than 32, 64 or 128 */
+#define SMA_ERR_HEAD_DIM      -3   /* head_dim other than 32, 64 or 128 (the *_call entry points: not a multiple of 8 up to 128) */
 #define SMA_ERR_DTYPE         -4   /* dtype other than SMA_DTYPE_F16 / SMA_DTYPE_BF16 */
 #define SMA_ERR_SCALE         -5   /* scale is NaN or infinite */
 #define SMA_ERR_LAUNCH        -6   /* the HIP runtime refused the launch (hipGetLastError) */
@@ -293,6 +293,52 @@ int sma_attn_bwd_map_strided(const sma_tensor *dout, const sma_tensor *q, const 
                              const uint32_t *tile_map, const sma_tensor *dq, const sma_tensor *dk,
                              const sma_tensor *dv, float *delta_ws, int B, int H, int N, int D, float scale,
                              int dtype, void *stream);
+
+/* Forward and backward with everything optional in one argument block, for what the functions above do
+ * not take: any head dim that is a multiple of 8 up to 128 without padding copies (the kernels exist
+ * for 32, 64, 96 and 128; D = 80 runs in the one for 96), and fp32 results next to or instead of the
+ * bf16 ones (the rounded bf16 values widened; dtype must be bf16), for callers that keep fp32 tensors.
+ * Pointers that are marked optional may be NULL; everything else is as in sma_attn_fwd_map_strided,
+ * sma_attn_fwd_bool_mask_strided and sma_attn_bwd_map_strided.
+ *
+ * No counterpart in the reference, which converts and pads with tensor operations
+ * (python/sparse_attention.py:140-142,151-152).
+ */
+typedef struct sma_fwd_call {
+    const sma_tensor *q, *k, *v;
+    const sma_tensor *out;                  /* optional if out_f32 is given */
+    const sma_tensor *out_f32;              /* optional: float elements, strides multiples of 8 */
+    const uint8_t *mask;                    /* boolean mask (strides in bytes), or NULL to use ... */
+    const uint32_t *mask_packed;            /* ... the packed one (strides in words) */
+    int64_t mask_stride_b, mask_stride_h;
+    const uint32_t *tile_map;               /* optional, with mask_packed */
+    float *lse;                             /* optional */
+    uint32_t *packed_out, *map_out;         /* optional, with mask */
+    int B, H, N, D;
+    float scale;
+    int dtype;
+} sma_fwd_call;
+int sma_attn_fwd_call(const sma_fwd_call *call, void *stream);
+
+typedef struct sma_bwd_call {
+    const sma_tensor *dout, *q, *k, *v, *out;
+    const sma_tensor *dq, *dk, *dv;         /* 16-bit elements, or floats if grads_f32 */
+    const float *lse;
+    const uint32_t *mask_packed;
+    int64_t mask_stride_b, mask_stride_h;
+    const uint32_t *tile_map;               /* optional */
+    float *delta_ws;
+    int B, H, N, D;
+    float scale;
+    int dtype;
+    int grads_f32;
+} sma_bwd_call;
+int sma_attn_bwd_call(const sma_bwd_call *call, void *stream);
+
+/* bf16 copies (round to nearest even) of `count` <= 3 float arrays of n elements each, one launch; n is a
+ * multiple of 8, all pointers 16-byte aligned.  src and dst are host arrays of device pointers.
+ */
+int sma_to_bf16(const float *const *src, uint16_t *const *dst, int count, long long n, void *stream);
 
 #ifdef __cplusplus
 }

@@ -23,6 +23,8 @@ import shutil
 import subprocess
 import sys
 import sysconfig
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -33,6 +35,7 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 LIB_NAME = "libsma_hip.so"
 MODULE_NAME = "sparse_attn_cuda"
 HIP_SOURCES = ["attn_fwd.hip", "attn_bwd.hip", "pack_mask.hip", "capi.hip"]
+FWD_HEAD_DIMS = (32, 64, 96, 128)      # attn_fwd.hip is compiled once for each, for their kernels
 PROBE_DIR = os.path.join(HERE, "benchprobe")
 PROBE_LIB_NAME = "libsma_probe.so"
 GPU_ARCH = "gfx950"
@@ -79,10 +82,18 @@ HIPCC_FLAGS = [f"--offload-arch={GPU_ARCH}", "-O3", "-std=c++17", "-fno-finite-m
 
 def build_hip_library() -> str:
     out = lib_path()
-    cmd = [hipcc_path()] + HIPCC_FLAGS + ["-fPIC", "-shared"]
-    cmd += [os.path.join(CSRC, s) for s in HIP_SOURCES]
-    cmd += ["-o", out, f"-Wl,-rpath,{os.path.join(ROCM, 'lib')}", "-Wl,-soname," + LIB_NAME]
-    _run(cmd)
+    jobs = [(s, []) for s in HIP_SOURCES] + [("attn_fwd.hip", [f"-DSMA_FWD_HEAD_DIM={d}"]) for d in FWD_HEAD_DIMS]
+    with tempfile.TemporaryDirectory() as tmp:
+        def compile_one(job):
+            i, (source, defines) = job
+            obj = os.path.join(tmp, f"{i}.o")
+            _run([hipcc_path()] + HIPCC_FLAGS + defines + ["-fPIC", "-c", os.path.join(CSRC, source), "-o", obj])
+            return obj
+
+        with ThreadPoolExecutor(max_workers=8) as pool:
+            objects = list(pool.map(compile_one, enumerate(jobs)))
+        _run([hipcc_path(), f"--offload-arch={GPU_ARCH}", "-fPIC", "-shared"] + objects +
+             ["-o", out, f"-Wl,-rpath,{os.path.join(ROCM, 'lib')}", "-Wl,-soname," + LIB_NAME])
     return out
 
 

@@ -35,8 +35,9 @@
 // halves, the others (dQ, dK, dV) fill one pair of accumulators per half.  The dK/dV kernel would
 // need 128 accumulator registers for that; it is therefore launched twice, once for dK and once
 // for dV (S is formed in both).  Head dim 32 uses half a tile: the copies fill the upper half of
-// every LDS row with a second copy of the lower half (global chunk index & 3), which is never read;
-// contractions over the head dim take two MFMA steps and the outputs have one 32-column block.
+// every LDS row with copies of the row's last 16 bytes, which are never read;
+// contractions over the head dim take two MFMA steps and the outputs have one 32-column block.  Head dim 96
+// is 128 with such a half tile as its second half: six steps, three blocks.
 #include "attn_common.h"
 
 namespace sma {
@@ -66,9 +67,11 @@ template <int NH> struct Cfg {
 // position ^ bitrev3((row >> 1) & 7).
 struct TileCopy {
     uint32_t chunk[2];      // byte offset of the lane's global chunk inside its row
+    uint32_t chunk2[2];     // the same for the second column half
     int row[2];
 };
-__device__ __forceinline__ TileCopy make_tile_copy(int wave, int lane, int chunk_mask)
+// last_chunk: the row's last 16-byte chunk, which stands in for those beyond it
+__device__ __forceinline__ TileCopy make_tile_copy(int wave, int lane, int last_chunk)
 {
     TileCopy c;
 #pragma unroll
@@ -76,7 +79,9 @@ __device__ __forceinline__ TileCopy make_tile_copy(int wave, int lane, int chunk
         const int row = 8 * (2 * wave + j) + (lane >> 3);
         const int pos = lane & 7;
         c.row[j] = row;
-        c.chunk[j] = (uint32_t)(((pos ^ bitrev3((row >> 1) & 7)) & chunk_mask) << 4);
+        const int chunk = pos ^ bitrev3((row >> 1) & 7);
+        c.chunk[j] = (uint32_t)(chunk < last_chunk ? chunk : last_chunk) << 4;
+        c.chunk2[j] = (uint32_t)(chunk + 8 < last_chunk ? chunk + 8 : last_chunk) << 4;
     }
     return c;
 }
@@ -91,9 +96,9 @@ __device__ __forceinline__ void issue_tile(uint32_t dst, const uint16_t *mat, ui
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const int r = c.row[j] < last ? c.row[j] : last;
-        const uint32_t voff = __umul24(r, 2u * sn) + c.chunk[j];
-        async_copy_b128(dst + wave * 2048 + j * 1024, src, voff);
-        if constexpr (NH == 2) async_copy_b128(dst + TILE_BYTES + wave * 2048 + j * 1024, src + HD, voff);
+        const uint32_t row = __umul24(r, 2u * sn);
+        async_copy_b128(dst + wave * 2048 + j * 1024, src, row + c.chunk[j]);
+        if constexpr (NH == 2) async_copy_b128(dst + TILE_BYTES + wave * 2048 + j * 1024, src, row + c.chunk2[j]);
     }
 }
 // Zero the rows >= N of the `parts` consecutive 64-column tiles that start at dst.
@@ -139,23 +144,45 @@ __device__ __forceinline__ TileRead make_tile_read(int lane)
     return r;
 }
 
-// 16 bytes (8 elements) of row `row` (row stride sn elements) at element offset `col`.
-__device__ __forceinline__ u32x4 load_frag(const uint16_t *mat, int sn, int row, int col)
+// The fragments of one row of a matrix (row stride sn elements, D columns): 8 elements at columns
+// 16s + 8hh, zeros beyond the row.  `full` (D is the kernel's own head dim) is wave-uniform: the common
+// case loads straight.
+template <int KS>
+__device__ __forceinline__ void load_row(u32x4 (&f)[KS], const uint16_t *mat, uint32_t sn, int row, int hh, int D)
 {
-    return *reinterpret_cast<const u32x4 *>(mat + (size_t)row * sn + col);
+    const uint16_t *p = mat + (size_t)row * sn + 8 * hh;
+    if (D == 16 * KS) {
+#pragma unroll
+        for (int s = 0; s < KS; ++s) f[s] = *reinterpret_cast<const u32x4 *>(p + 16 * s);
+    } else {
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+            f[s] = 16 * s + 8 * hh < D ? *reinterpret_cast<const u32x4 *>(p + 16 * s) : u32x4{0u, 0u, 0u, 0u};
+    }
+}
+
+// Stores rows row0 .. row0 + 31 of a gradient, in 16 bits or (WIDE) fp32.  A template argument: both ways in
+// one kernel, chosen at run time, cost 2 to 4 % of the backward of many short sequences, whose epilogues are a
+// large part of it.
+template <bool BF16, bool WIDE, int OB>
+__device__ __forceinline__ void store_gradient(const f32x16 (&acc)[OB], float mult, uint32_t lds_wave, const AttnBwdArgs &a,
+                                               const Rows &r, int bi, int hi, int row0, int lane)
+{
+    const Rows none = {nullptr, 0u, 0u, 0u};
+    store_rows<BF16, OB>(acc, mult, lds_wave, 0, block_dst(WIDE ? none : r, WIDE ? r : none, bi, hi, row0, a.D), !WIDE, WIDE,
+                         row0, a.N, lane);
 }
 
 // ------------------------------------------------------------------------------------------------
 // dQ (and delta)
 // ------------------------------------------------------------------------------------------------
-template <bool BF16, int HDIM>
-__global__ __launch_bounds__(NTHREADS, HDIM == 128 ? 2 : 3) void attn_bwd_dq_kernel(const AttnBwdArgs a)
+template <bool BF16, int HDIM, bool WIDE>
+__global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_bwd_dq_kernel(const AttnBwdArgs a)
 {
     using E = Elem<BF16>;
-    constexpr int NH = HDIM == 128 ? 2 : 1;       // 64-column tiles per matrix
+    constexpr int NH = HDIM > 64 ? 2 : 1;         // 64-column tiles per matrix
     constexpr int KS = HDIM / 16;                 // MFMA steps of a contraction over the head dim
     constexpr int OB = HDIM / 32;                 // 32-column accumulator blocks of an output
-    constexpr int CHM = HDIM == 32 ? 3 : 7;       // 16-byte chunks per global row, minus one
     using C = Cfg<NH>;
     constexpr int STAGE_BYTES = C::STAGE_BYTES, OFF_AUX = C::OFF_AUX, OFF_LUT = C::OFF_LUT;
     __shared__ __attribute__((aligned(1024))) unsigned char smem[C::LDS_BYTES];
@@ -181,25 +208,21 @@ __global__ __launch_bounds__(NTHREADS, HDIM == 128 ? 2 : 3) void attn_bwd_dq_ker
     // ---- this lane's query row: q^T and dO^T fragments (B operands), delta, lse ----
     const int qrow = qt * BM + wave * 32 + l32;
     const int qr = qrow < N ? qrow : N - 1;
-    u32x4 qf[KS], dof[KS];
+    u32x4 qf[KS], dof[KS], of[KS];
+    load_row(qf, qb, a.q.sn, qr, hh, a.D);
+    load_row(dof, dob, a.dout.sn, qr, hh, a.D);
+    load_row(of, ob, a.out.sn, qr, hh, a.D);
     float delta = 0.f;
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-        const int col = 16 * s + 8 * hh;
-        u32x4 tq = load_frag(qb, a.q.sn, qr, col);
-        const u32x4 td = load_frag(dob, a.dout.sn, qr, col);
-        const u32x4 to = load_frag(ob, a.out.sn, qr, col);
+    for (int s = 0; s < KS; ++s)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            delta += E::up1((uint16_t)(td[i] & 0xffffu)) * E::up1((uint16_t)(to[i] & 0xffffu)) +
-                     E::up1((uint16_t)(td[i] >> 16)) * E::up1((uint16_t)(to[i] >> 16));
-            const float lo = E::up1((uint16_t)(tq[i] & 0xffffu)) * a.q_scale;
-            const float hi = E::up1((uint16_t)(tq[i] >> 16)) * a.q_scale;
-            tq[i] = (uint32_t)E::cvt1(lo) | ((uint32_t)E::cvt1(hi) << 16);
+            delta += E::up1((uint16_t)(dof[s][i] & 0xffffu)) * E::up1((uint16_t)(of[s][i] & 0xffffu)) +
+                     E::up1((uint16_t)(dof[s][i] >> 16)) * E::up1((uint16_t)(of[s][i] >> 16));
+            const float lo = E::up1((uint16_t)(qf[s][i] & 0xffffu)) * a.q_scale;
+            const float hi = E::up1((uint16_t)(qf[s][i] >> 16)) * a.q_scale;
+            qf[s][i] = (uint32_t)E::cvt1(lo) | ((uint32_t)E::cvt1(hi) << 16);
         }
-        qf[s] = tq;
-        dof[s] = td;
-    }
     delta = xhalf_sum(delta);
     if (qrow < N && hh == 0) a.delta[(size_t)bh * N + qrow] = delta;
     const float lse_row = a.lse[(size_t)bh * N + qr];
@@ -207,7 +230,7 @@ __global__ __launch_bounds__(NTHREADS, HDIM == 128 ? 2 : 3) void attn_bwd_dq_ker
     const float L = (qrow >= N || lse_row == -__builtin_inff()) ? __builtin_inff() : lse_row * LOG2E;
 
     // ---- copies ----
-    const TileCopy tc = make_tile_copy(wave, lane, CHM);
+    const TileCopy tc = make_tile_copy(wave, lane, (a.D >> 3) - 1);
     const TileRead tr = make_tile_read(lane);
     const int mrow = qt * BM + wave * 32 + (lane >> 1);
     const uint32_t m_voff = (uint32_t)(((size_t)(mrow < N ? mrow : N - 1) * nw + (lane & 1)) * 4);
@@ -321,15 +344,7 @@ __global__ __launch_bounds__(NTHREADS, HDIM == 128 ? 2 : 3) void attn_bwd_dq_ker
     __syncthreads();              // every wave is done reading the stages
     const int row0 = qt * BM + wave * 32;
     if (row0 < N) {
-        uint16_t *dst = slab(a.dq, bi, hi) + (size_t)row0 * a.dq.sn;
-        if constexpr (HDIM == 32) {
-            store_block<BF16, 32>(oacc[0], oacc[0], a.scale, lds0 + wave * 4096, dst, a.dq.sn, row0, N, lane);
-        } else {
-#pragma unroll
-            for (int half = 0; half < NH; ++half)
-                store_block<BF16>(oacc[2 * half], oacc[2 * half + 1], a.scale, lds0 + wave * 4096,
-                                  dst + half * HD, a.dq.sn, row0, N, lane);
-        }
+        store_gradient<BF16, WIDE>(oacc, a.scale, lds0 + wave * 4096, a, a.dq, bi, hi, row0, lane);
     }
 }
 
@@ -338,14 +353,13 @@ __global__ __launch_bounds__(NTHREADS, HDIM == 128 ? 2 : 3) void attn_bwd_dq_ker
 // ------------------------------------------------------------------------------------------------
 // DK / DV: which of the two gradients this instance produces (both for head dim 64; one per launch
 // for head dim 128, where both sets of accumulators do not fit the register file).
-template <bool BF16, int HDIM, bool DK, bool DV, bool POSTMUL>
+template <bool BF16, int HDIM, bool DK, bool DV, bool POSTMUL, bool WIDE>
 __global__ __launch_bounds__(NTHREADS, 2) void attn_bwd_dkv_kernel(const AttnBwdArgs a)
 {
     using E = Elem<BF16>;
-    constexpr int NH = HDIM == 128 ? 2 : 1;
+    constexpr int NH = HDIM > 64 ? 2 : 1;
     constexpr int KS = HDIM / 16;
     constexpr int OB = HDIM / 32;
-    constexpr int CHM = HDIM == 32 ? 3 : 7;
     using C = Cfg<NH>;
     constexpr int STAGE_BYTES = C::STAGE_BYTES, OFF_AUX = C::OFF_AUX;
     __shared__ __attribute__((aligned(1024))) unsigned char smem[C::LDS_BYTES];
@@ -379,22 +393,19 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_bwd_dkv_kernel(const AttnBwd
     const uint32_t key_w = key < N ? 1u : 0u;         // width of the bit field that holds this key's mask bit
     const int wi = (key0 >> 5) < nw ? (key0 >> 5) : nw - 1;     // this wave's mask word of a row
     u32x4 kf[KS], vf[DK ? KS : 1];
+    load_row(kf, kb, a.k.sn, kr, hh, a.D);
+    if constexpr (DK) load_row(vf, vb, a.v.sn, kr, hh, a.D);
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-        const int col = 16 * s + 8 * hh;
-        u32x4 tk = load_frag(kb, a.k.sn, kr, col);
-        if constexpr (DK) vf[s] = load_frag(vb, a.v.sn, kr, col);
+    for (int s = 0; s < KS; ++s)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const float lo = E::up1((uint16_t)(tk[i] & 0xffffu)) * a.q_scale;
-            const float hi = E::up1((uint16_t)(tk[i] >> 16)) * a.q_scale;
-            tk[i] = (uint32_t)E::cvt1(lo) | ((uint32_t)E::cvt1(hi) << 16);
+            const float lo = E::up1((uint16_t)(kf[s][i] & 0xffffu)) * a.q_scale;
+            const float hi = E::up1((uint16_t)(kf[s][i] >> 16)) * a.q_scale;
+            kf[s][i] = (uint32_t)E::cvt1(lo) | ((uint32_t)E::cvt1(hi) << 16);
         }
-        kf[s] = tk;
-    }
 
     // ---- copies: Q tile, dO tile; per wave its mask word of the 64 rows; lse (wave 0), delta (wave 1)
-    const TileCopy tc = make_tile_copy(wave, lane, CHM);
+    const TileCopy tc = make_tile_copy(wave, lane, (a.D >> 3) - 1);
     const TileRead tr = make_tile_read(lane);
     auto issue = [&](int t, int st) {
         const int r0 = t * BN;
@@ -557,33 +568,33 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_bwd_dkv_kernel(const AttnBwd
     WAIT_VMCNT(0);
     __syncthreads();
     if (wave_valid) {
-        uint16_t *dk_dst = slab(a.dk, bi, hi) + (size_t)key0 * a.dk.sn;
-        uint16_t *dv_dst = slab(a.dv, bi, hi) + (size_t)key0 * a.dv.sn;
-        if constexpr (HDIM == 32) {
-            if constexpr (DK) store_block<BF16, 32>(dkacc[0], dkacc[0], a.scale, lds0 + wave * 4096, dk_dst, a.dk.sn, key0, N, lane);
-            if constexpr (DV) store_block<BF16, 32>(dvacc[0], dvacc[0], 1.0f, lds0 + wave * 4096, dv_dst, a.dv.sn, key0, N, lane);
-        } else {
-#pragma unroll
-            for (int half = 0; half < NH; ++half) {
-                if constexpr (DK)
-                    store_block<BF16>(dkacc[2 * half], dkacc[2 * half + 1], a.scale, lds0 + wave * 4096,
-                                      dk_dst + half * HD, a.dk.sn, key0, N, lane);
-                if constexpr (DV)
-                    store_block<BF16>(dvacc[2 * half], dvacc[2 * half + 1], 1.0f, lds0 + wave * 4096,
-                                      dv_dst + half * HD, a.dv.sn, key0, N, lane);
-            }
-        }
+        if constexpr (DK) store_gradient<BF16, WIDE>(dkacc, a.scale, lds0 + wave * 4096, a, a.dk, bi, hi, key0, lane);
+        if constexpr (DV) store_gradient<BF16, WIDE>(dvacc, 1.0f, lds0 + wave * 4096, a, a.dv, bi, hi, key0, lane);
     }
 }
 
-// Launches the dK/dV instance for (dtype, head dim, gradients) with or without the post-multiplier.
-template <bool BF16, int HDIM, bool DK, bool DV>
-void launch_dkv(bool postmul, dim3 grid, dim3 block, hipStream_t stream, const AttnBwdArgs &a)
+template <bool BF16, int HDIM, bool POSTMUL, bool WIDE>
+void launch_pair(dim3 grid, dim3 block, hipStream_t stream, const AttnBwdArgs &a)
 {
-    if (postmul)
-        hipLaunchKernelGGL((attn_bwd_dkv_kernel<BF16, HDIM, DK, DV, true>), grid, block, 0, stream, a);
+    // dQ first: it also fills the delta workspace that the dK/dV kernel reads (same stream)
+    hipLaunchKernelGGL((attn_bwd_dq_kernel<BF16, HDIM, WIDE>), grid, block, 0, stream, a);
+    if constexpr (HDIM == 128) {
+        hipLaunchKernelGGL((attn_bwd_dkv_kernel<BF16, HDIM, true, false, POSTMUL, WIDE>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((attn_bwd_dkv_kernel<BF16, HDIM, false, true, POSTMUL, WIDE>), grid, block, 0, stream, a);
+    } else {
+        hipLaunchKernelGGL((attn_bwd_dkv_kernel<BF16, HDIM, true, true, POSTMUL, WIDE>), grid, block, 0, stream, a);
+    }
+}
+template <int HDIM>
+void launch_head_dim(bool bf16, dim3 grid, dim3 block, hipStream_t stream, const AttnBwdArgs &a)
+{
+    const bool postmul = a.post_mul != 1.0f;       // exp2(pm * s) needs its multiplication only then
+    if (a.grads_f32)                               // fp32 callers compute in bf16
+        postmul ? launch_pair<true, HDIM, true, true>(grid, block, stream, a) : launch_pair<true, HDIM, false, true>(grid, block, stream, a);
+    else if (bf16)
+        postmul ? launch_pair<true, HDIM, true, false>(grid, block, stream, a) : launch_pair<true, HDIM, false, false>(grid, block, stream, a);
     else
-        hipLaunchKernelGGL((attn_bwd_dkv_kernel<BF16, HDIM, DK, DV, false>), grid, block, 0, stream, a);
+        postmul ? launch_pair<false, HDIM, true, false>(grid, block, stream, a) : launch_pair<false, HDIM, false, false>(grid, block, stream, a);
 }
 
 }  // namespace
@@ -595,35 +606,13 @@ hipError_t launch_attn_bwd(const AttnBwdArgs &args, bool bf16, hipStream_t strea
     a.div_H = make_fastdiv((uint32_t)a.H);
     const long long groups = (long long)a.BH * a.qtiles;
     if (groups == 0) return hipSuccess;
+    if (a.grads_f32 && !bf16) return hipErrorInvalidValue;
     const dim3 grid((unsigned)groups), block(NTHREADS);
-    const bool postmul = a.post_mul != 1.0f;       // exp2(pm * s) needs its multiplication only then
-    // dQ first: it also fills the delta workspace that the dK/dV kernel reads (same stream).
-    if (a.D == 2 * HD) {
-        if (bf16) {
-            hipLaunchKernelGGL((attn_bwd_dq_kernel<true, 128>), grid, block, 0, stream, a);
-            launch_dkv<true, 128, true, false>(postmul, grid, block, stream, a);
-            launch_dkv<true, 128, false, true>(postmul, grid, block, stream, a);
-        } else {
-            hipLaunchKernelGGL((attn_bwd_dq_kernel<false, 128>), grid, block, 0, stream, a);
-            launch_dkv<false, 128, true, false>(postmul, grid, block, stream, a);
-            launch_dkv<false, 128, false, true>(postmul, grid, block, stream, a);
-        }
-    } else if (a.D == HD) {
-        if (bf16) {
-            hipLaunchKernelGGL((attn_bwd_dq_kernel<true, 64>), grid, block, 0, stream, a);
-            launch_dkv<true, 64, true, true>(postmul, grid, block, stream, a);
-        } else {
-            hipLaunchKernelGGL((attn_bwd_dq_kernel<false, 64>), grid, block, 0, stream, a);
-            launch_dkv<false, 64, true, true>(postmul, grid, block, stream, a);
-        }
-    } else {
-        if (bf16) {
-            hipLaunchKernelGGL((attn_bwd_dq_kernel<true, 32>), grid, block, 0, stream, a);
-            launch_dkv<true, 32, true, true>(postmul, grid, block, stream, a);
-        } else {
-            hipLaunchKernelGGL((attn_bwd_dq_kernel<false, 32>), grid, block, 0, stream, a);
-            launch_dkv<false, 32, true, true>(postmul, grid, block, stream, a);
-        }
+    switch (kernel_head_dim(a.D)) {
+    case 128: launch_head_dim<128>(bf16, grid, block, stream, a); break;
+    case 96: launch_head_dim<96>(bf16, grid, block, stream, a); break;
+    case 64: launch_head_dim<64>(bf16, grid, block, stream, a); break;
+    default: launch_head_dim<32>(bf16, grid, block, stream, a); break;
     }
     return hipGetLastError();
 }

@@ -12,6 +12,7 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef short i16x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -151,14 +152,37 @@ __device__ __forceinline__ void async_copy_b32_at(uint32_t lds_base, const void 
 #define WAIT_VMCNT(n) asm volatile("s_waitcnt vmcnt(" #n ")" ::: "memory")
 
 
+// Where a wavefront's 32 x COLS block of results goes: 16-bit rows, 32-bit rows (the rounded values
+// widened), or both; a null pointer leaves one out.
+struct BlockDst {
+    uint16_t *h;            // first row, first of the COLS columns
+    float *f;
+    uint32_t h_sn, f_sn;    // row strides in elements
+    int cols;               // columns of the tensor from there on: columns beyond are not stored
+};
+__device__ __forceinline__ BlockDst block_dst(const Rows &h, const Rows &f, int b, int hd, int row0, int D)
+{
+    BlockDst d;
+    d.h = h.p != nullptr ? slab(h, b, hd) + (size_t)row0 * h.sn : nullptr;
+    d.f = f.p != nullptr ? reinterpret_cast<float *>(f.p) + ((size_t)b * f.sb8 + (size_t)hd * f.sh8) * 8 + (size_t)row0 * f.sn
+                         : nullptr;
+    d.h_sn = h.sn;
+    d.f_sn = f.sn;
+    d.cols = D;
+    return d;
+}
+__device__ __forceinline__ BlockDst columns_from(const BlockDst &d, int col)
+{
+    return BlockDst{d.h + col, d.f + col, d.h_sn, d.f_sn, d.cols - col};
+}
+
 // Transposed store of a 32 x COLS accumulator block (COLS = 64: acc[dblk][4g+j] = value(row l32,
 // column 32dblk + 8g + 4hh + j) with acc = {acc0, acc1}; COLS = 32: acc0 only) times `mult`, through
-// 4 KiB of wave-private LDS, as whole 2*COLS-byte pieces of rows (dst_row0: first row, first of the
-// COLS columns; sn: row stride in elements).  Non-temporal stores: what is written is not read
-// again by the kernel and should not displace its inputs from the caches.
+// 4 KiB of wave-private LDS, as whole pieces of rows.  Non-temporal stores: what is written is not
+// read again by the kernel and should not displace its inputs from the caches.
 template <bool BF16, int COLS = 64>
 __device__ __forceinline__ void store_block(const f32x16 &acc0, const f32x16 &acc1, float mult, uint32_t lds_wave,
-                                            uint16_t *dst_row0, int sn, int row0, int N, int lane)
+                                            const BlockDst &dst, bool has_h, bool has_f, int row0, int N, int lane)
 {
     const f32x16 acc[2] = {acc0, acc1};
     using E = Elem<BF16>;
@@ -177,15 +201,66 @@ __device__ __forceinline__ void store_block(const f32x16 &acc0, const f32x16 &ac
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     constexpr int LPR = COLS / 8;                 // lanes (16-byte chunks) per row
+    constexpr int STEPS = LPR / 2;
+    const int pos = lane % LPR, row_in = lane / LPR;
+    u32x4 v[STEPS];
 #pragma unroll
-    for (int j = 0; j < LPR / 2; ++j) {
-        const int row = (64 / LPR) * j + lane / LPR, pos = lane % LPR;
-        const u32x4 v = lds_read_b128(lds_wave + row * 128 + ((pos ^ ((row >> 1) & 7)) << 4));
-        if (row0 + row < N) __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(dst_row0 + (size_t)row * sn + pos * 8));
+    for (int j = 0; j < STEPS; ++j) {
+        const int row = (64 / LPR) * j + row_in;
+        v[j] = lds_read_b128(lds_wave + row * 128 + ((pos ^ ((row >> 1) & 7)) << 4));
     }
+    // every branch on `has_h`, `has_f` and `whole` is wave-uniform and taken once, not per row: tested row by row
+    // the stores of the two kernels of the backward cost 3 us of 110 (64 x 16 heads, N = 256)
+    const bool whole = row0 + 32 <= N && dst.cols >= COLS;
+    auto each = [&](auto store) __attribute__((always_inline)) {
+        if (whole) {
+#pragma unroll
+            for (int j = 0; j < STEPS; ++j) store(j, (64 / LPR) * j + row_in);
+        } else {
+#pragma unroll
+            for (int j = 0; j < STEPS; ++j) {
+                const int row = (64 / LPR) * j + row_in;
+                if (row0 + row < N && pos * 8 < dst.cols) store(j, row);
+            }
+        }
+    };
+    if (has_h)
+        each([&](int j, int row) __attribute__((always_inline)) {
+            __builtin_nontemporal_store(v[j], reinterpret_cast<u32x4 *>(dst.h + (size_t)row * dst.h_sn + pos * 8));
+        });
+    if (has_f)
+        each([&](int j, int row) __attribute__((always_inline)) {
+            f32x4 lo, hi;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                lo[2 * i] = E::up1((uint16_t)(v[j][i] & 0xffffu));
+                lo[2 * i + 1] = E::up1((uint16_t)(v[j][i] >> 16));
+                hi[2 * i] = E::up1((uint16_t)(v[j][2 + i] & 0xffffu));
+                hi[2 * i + 1] = E::up1((uint16_t)(v[j][2 + i] >> 16));
+            }
+            f32x4 *f = reinterpret_cast<f32x4 *>(dst.f + (size_t)row * dst.f_sn + pos * 8);
+            __builtin_nontemporal_store(lo, f);
+            __builtin_nontemporal_store(hi, f + 1);
+        });
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// The same for all 32-column blocks of an output row (acc[2 * half + dblk]); `stride` LDS bytes between the
+// areas of the two column halves (0: one after the other through the same 4 KiB).
+template <bool BF16, int OB>
+__device__ __forceinline__ void store_rows(const f32x16 (&acc)[OB], float mult, uint32_t lds_wave, uint32_t stride,
+                                           const BlockDst &dst, bool has_h, bool has_f, int row0, int N, int lane)
+{
+    if constexpr (OB == 1) {
+        store_block<BF16, 32>(acc[0], acc[0], mult, lds_wave, dst, has_h, has_f, row0, N, lane);
+    } else {
+        store_block<BF16>(acc[0], acc[1], mult, lds_wave, dst, has_h, has_f, row0, N, lane);
+        if constexpr (OB == 3)
+            store_block<BF16, 32>(acc[2], acc[2], mult, lds_wave + stride, columns_from(dst, 64), has_h, has_f, row0, N, lane);
+        if constexpr (OB == 4)
+            store_block<BF16>(acc[2], acc[3], mult, lds_wave + stride, columns_from(dst, 64), has_h, has_f, row0, N, lane);
+    }
 }
 
 }  // namespace

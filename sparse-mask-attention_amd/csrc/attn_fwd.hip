@@ -65,9 +65,11 @@ constexpr float SUM_LIMIT = 16384.0f;     // a lane's 32 weights of a tile sum t
 //        QK^T chain runs over both halves of K and q, and P multiplies each half of V into its own
 //        pair of accumulators.  A stage is twice as large (32 KiB) and the kernel needs about 224
 //        registers, so two work-groups share a CU.
-//   32   half a tile: the copies fill the upper half of every LDS row with a second copy of the
-//        lower half (global chunk index & 3), which is never read; the QK^T chain has two steps
-//        instead of four and P multiplies one 32-column block of V.
+//   32   half a tile: the copies fill the upper half of every LDS row with copies of the row's last
+//        16 bytes, which are never read; the QK^T chain has two steps instead of four and P multiplies
+//        one 32-column block of V.
+//   96   128 with such a half tile as its second half: six steps, three blocks.  D = 80 and 96 ran in the
+//        128 kernel before, through zero-padded copies (16 x 8 heads, N = 1088, D = 96: 156 -> 81 us)
 //
 // BYTEMASK: the mask arrives as the caller's boolean bytes (one per score, 0 or 1) instead of packed
 // words.  Each wavefront copies the 32 x 64 bytes of a tile for its rows into LDS and turns them
@@ -116,18 +118,20 @@ template <int N> __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_
 // slower, and the launcher leaves it off.
 template <bool BF16, bool POSTMUL, bool PACKED_ROWS, int HDIM, bool BYTEMASK = false, bool BYPRODUCTS = false,
           bool PAIRS = false>
-__global__ __launch_bounds__(NTHREADS, HDIM == 128 ? 2 : 3) void attn_fwd_kernel(const AttnArgs a)
+__global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(const AttnArgs a)
 {
     static_assert(!PAIRS || (BYTEMASK && HDIM <= 64), "PAIRS: byte mask, two byte slots");
     using E = Elem<BF16>;
-    constexpr int NH = HDIM == 128 ? 2 : 1;       // 64-column tiles per matrix
+    constexpr int NH = HDIM > 64 ? 2 : 1;         // 64-column tiles per matrix
     constexpr int KS = HDIM / 16;                 // MFMA steps of the QK^T chain
     constexpr int OB = HDIM / 32;                 // 32-column accumulator blocks of O
-    constexpr int CHM = HDIM == 32 ? 3 : 7;       // 16-byte chunks per global row, minus one
+    // second column half at a constant distance from the first in every row
+    constexpr bool SAME_HALVES = HDIM == 128 && PACKED_ROWS;
     using C = Cfg<NH, BYTEMASK>;
     constexpr int NSTAGE = C::NSTAGE, STAGE_BYTES = C::STAGE_BYTES, OFF_MASK = C::OFF_MASK, OFF_LUT = C::OFF_LUT;
     constexpr int MASK_SLOT = C::MASK_SLOT;
-    constexpr int D = HDIM;
+    const int D = PACKED_ROWS ? HDIM : a.D;
+    const int last_chunk = (D >> 3) - 1;          // 16-byte chunks per global row, minus one
     __shared__ __attribute__((aligned(1024))) unsigned char smem[C::LDS_BYTES];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(LDS_PTR(unsigned char))smem;
 
@@ -177,7 +181,7 @@ __global__ __launch_bounds__(NTHREADS, HDIM == 128 ? 2 : 3) void attn_fwd_kernel
                                                                        bi * a.mask.sb + hi * a.mask.sh)
                                   : slab(a.mask, bi, hi);
     const uint32_t q_sn = PACKED_ROWS ? D : a.q.sn, k_sn = PACKED_ROWS ? D : a.k.sn;       // row strides, elements
-    const uint32_t v_sn = PACKED_ROWS ? D : a.v.sn, o_sn = PACKED_ROWS ? D : a.out.sn;
+    const uint32_t v_sn = PACKED_ROWS ? D : a.v.sn;
     const uint32_t q_rb = 2u * q_sn, k_rb = 2u * k_sn, v_rb = 2u * v_sn;                   // row pitch, bytes
 
     // ---- mask words: wave-private async copies, slot = tile % NSTAGE, lane i -> (row i/2, word i%2) ----
@@ -385,7 +389,9 @@ __global__ __launch_bounds__(NTHREADS, HDIM == 128 ? 2 : 3) void attn_fwd_kernel
     // One global_load_lds_dwordx4 fills 1 KiB = 8 tile rows.  Wave w copies row blocks 2w, 2w+1 of
     // K and of V.  Lane i fills LDS chunk (row = 8*blk + i/8, position i%8) with the global chunk
     // position ^ swz(row):   K: swz(row) = (row >> 1) & 7      V: swz(row) = bitrev3((row >> 1) & 7)
-    uint32_t kv_voff[2][2];
+    // (a chunk beyond the row's last is read as that one)
+    auto chunk_at = [&](int c) __attribute__((always_inline)) -> uint32_t { return (uint32_t)(c < last_chunk ? c : last_chunk) << 4; };
+    uint32_t kv_voff[2][2], kv_voff2[2][2];       // first and second column half
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const int row = 8 * (2 * wave + j) + (lane >> 3);
@@ -393,14 +399,17 @@ __global__ __launch_bounds__(NTHREADS, HDIM == 128 ? 2 : 3) void attn_fwd_kernel
         const int f = (row >> 1) & 7;
         const int fr = bitrev3(f);
         // row pitches are below 2^24 bytes (checked by the C-ABI layer): full-rate 24-bit multiplies
-        kv_voff[0][j] = __umul24(row, k_rb) + (((pos ^ f) & CHM) << 4);
-        kv_voff[1][j] = __umul24(row, v_rb) + (((pos ^ fr) & CHM) << 4);
+        kv_voff[0][j] = __umul24(row, k_rb) + chunk_at(pos ^ f);
+        kv_voff[1][j] = __umul24(row, v_rb) + chunk_at(pos ^ fr);
+        kv_voff2[0][j] = SAME_HALVES ? kv_voff[0][j] + 2 * HD : __umul24(row, k_rb) + chunk_at(8 + (pos ^ f));
+        kv_voff2[1][j] = SAME_HALVES ? kv_voff[1][j] + 2 * HD : __umul24(row, v_rb) + chunk_at(8 + (pos ^ fr));
     }
     const uint32_t kv_dst = lds0 + wave * 2048;
     auto issue_kv = [&](int t, auto stage_c) __attribute__((always_inline)) {
         constexpr int SO = decltype(stage_c)::value * STAGE_BYTES;
         const int key0 = t * BN;
         uint32_t ko[2] = {kv_voff[0][0], kv_voff[0][1]}, vo[2] = {kv_voff[1][0], kv_voff[1][1]};
+        uint32_t ko2[2] = {kv_voff2[0][0], kv_voff2[0][1]}, vo2[2] = {kv_voff2[1][0], kv_voff2[1][1]};
         if (ragged && t == T - 1) {           // rows beyond N: copy row N-1 instead (zeroed later)
             int last0 = key0;
             asm volatile("" : "+s"(last0));   // opaque: keeps this once-only arithmetic out of the loop's registers
@@ -408,21 +417,30 @@ __global__ __launch_bounds__(NTHREADS, HDIM == 128 ? 2 : 3) void attn_fwd_kernel
             for (int j = 0; j < 2; ++j) {
                 const int row = 8 * (2 * wave + j) + (lane >> 3);
                 const int over = last0 + row - (N - 1);
-                if (over > 0) { ko[j] -= __umul24(over, k_rb); vo[j] -= __umul24(over, v_rb); }
+                if (over > 0) {
+                    ko[j] -= __umul24(over, k_rb); vo[j] -= __umul24(over, v_rb);
+                    ko2[j] -= __umul24(over, k_rb); vo2[j] -= __umul24(over, v_rb);
+                }
             }
         }
         const uint16_t *ksrc = kb + (size_t)key0 * k_sn, *vsrc = vb + (size_t)key0 * v_sn;
         async_copy_b128_at<SO>(kv_dst, ksrc, ko[0]);
         async_copy_b128_at<SO + 1024>(kv_dst, ksrc, ko[1]);
-        if constexpr (NH == 2) {              // second column half: 128 bytes further along each row
+        if constexpr (SAME_HALVES) {          // 128 bytes further along each row
             async_copy_b128_at<SO + TILE_BYTES>(kv_dst, ksrc + HD, ko[0]);
             async_copy_b128_at<SO + TILE_BYTES + 1024>(kv_dst, ksrc + HD, ko[1]);
+        } else if constexpr (NH == 2) {
+            async_copy_b128_at<SO + TILE_BYTES>(kv_dst, ksrc, ko2[0]);
+            async_copy_b128_at<SO + TILE_BYTES + 1024>(kv_dst, ksrc, ko2[1]);
         }
         async_copy_b128_at<SO + C::OFF_V>(kv_dst, vsrc, vo[0]);
         async_copy_b128_at<SO + C::OFF_V + 1024>(kv_dst, vsrc, vo[1]);
-        if constexpr (NH == 2) {
+        if constexpr (SAME_HALVES) {
             async_copy_b128_at<SO + C::OFF_V + TILE_BYTES>(kv_dst, vsrc + HD, vo[0]);
             async_copy_b128_at<SO + C::OFF_V + TILE_BYTES + 1024>(kv_dst, vsrc + HD, vo[1]);
+        } else if constexpr (NH == 2) {
+            async_copy_b128_at<SO + C::OFF_V + TILE_BYTES>(kv_dst, vsrc, vo2[0]);
+            async_copy_b128_at<SO + C::OFF_V + TILE_BYTES + 1024>(kv_dst, vsrc, vo2[1]);
         }
     };
     auto zero_tail_rows = [&](int t, int stage) __attribute__((always_inline)) {   // after the copies of the last tile have landed
@@ -479,9 +497,9 @@ __global__ __launch_bounds__(NTHREADS, HDIM == 128 ? 2 : 3) void attn_fwd_kernel
             const int row = 8 * j + (lane >> 3);
             const int pos = lane & 7;
             const int lrow = row < last ? row : last;
-            const uint32_t voff = __umul24(lrow, q_rb) + (((pos ^ ((row >> 1) & 7)) & CHM) << 4);
-            async_copy_b128(dst + j * 1024, qsrc, voff);
-            if constexpr (NH == 2) async_copy_b128(dst + 16384 + j * 1024, qsrc + HD, voff);
+            const int c = pos ^ ((row >> 1) & 7);
+            async_copy_b128(dst + j * 1024, qsrc, __umul24(lrow, q_rb) + chunk_at(c));
+            if constexpr (NH == 2) async_copy_b128(dst + 16384 + j * 1024, qsrc, __umul24(lrow, q_rb) + chunk_at(8 + c));
         }
     }
     using std::integral_constant;
@@ -536,6 +554,7 @@ __global__ __launch_bounds__(NTHREADS, HDIM == 128 ? 2 : 3) void attn_fwd_kernel
             const float hi = E::up1((uint16_t)(t[i] >> 16)) * a.q_scale;
             t[i] = (uint32_t)E::cvt1(lo) | ((uint32_t)E::cvt1(hi) << 16);
         }
+        if (!PACKED_ROWS && 2 * s + hh > last_chunk) t = u32x4{0u, 0u, 0u, 0u};      // beyond the row: adds nothing
         qf[s] = t;
     }
 
@@ -808,16 +827,9 @@ __global__ __launch_bounds__(NTHREADS, HDIM == 128 ? 2 : 3) void attn_fwd_kernel
     const float inv = (l_tot > 0.f) ? 1.0f / l_tot : 0.f;
     {
         const int row0 = qt * BM + wave * 32;
-        uint16_t *ob = slab(a.out, bi, hi) + (size_t)row0 * o_sn;
         const uint32_t ebase = lds0 + (uint32_t)(visits & 1) * STAGE_BYTES + wave * 4096;
-        if constexpr (HDIM == 32) {
-            store_block<BF16, 32>(oacc[0], oacc[0], inv, ebase, ob, (int)o_sn, row0, N, lane);
-        } else {
-#pragma unroll
-            for (int half = 0; half < NH; ++half)
-                store_block<BF16>(oacc[2 * half], oacc[2 * half + 1], inv, ebase + half * 16384,
-                                  ob + half * HD, (int)o_sn, row0, N, lane);
-        }
+        store_rows<BF16, OB>(oacc, inv, ebase, 16384, block_dst(a.out, a.out32, bi, hi, row0, D), a.out.p != nullptr,
+                             BF16 && a.out32.p != nullptr, row0, N, lane);       // fp32 callers compute in bf16
     }
     if (qrow < N) {
         if (a.lse != nullptr && hh == 0) {
@@ -831,6 +843,46 @@ __global__ __launch_bounds__(NTHREADS, HDIM == 128 ? 2 : 3) void attn_fwd_kernel
 }
 
 }  // namespace
+
+// The instance for (element type, post-multiplier, row strides) and the kind of mask: 0 packed words, 1
+// boolean bytes, 2 the same with by-products, 3 and 4 those with two tiles' bytes per request.  This file is
+// compiled once per head dim for the instances, side by side, and once for the launcher.
+typedef void (*FwdKernel)(const AttnArgs);
+#ifdef SMA_FWD_HEAD_DIM
+template <int HDIM, bool BF16, bool POSTMUL, bool PACKED_ROWS> FwdKernel pick_mask_kind(int mask_kind)
+{
+    switch (mask_kind) {
+    case 0: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM>;
+    case 1: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true>;
+    case 2: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true>;
+    }
+    if constexpr (HDIM <= 64) {
+        if (mask_kind == 3) return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, false, true>;
+        return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true, true>;
+    }
+    return nullptr;
+}
+template <int HDIM> FwdKernel pick(int variant, int mask_kind)
+{
+    switch (variant) {
+    case 0: return pick_mask_kind<HDIM, false, false, false>(mask_kind);
+    case 1: return pick_mask_kind<HDIM, false, false, true>(mask_kind);
+    case 2: return pick_mask_kind<HDIM, false, true, false>(mask_kind);
+    case 3: return pick_mask_kind<HDIM, false, true, true>(mask_kind);
+    case 4: return pick_mask_kind<HDIM, true, false, false>(mask_kind);
+    case 5: return pick_mask_kind<HDIM, true, false, true>(mask_kind);
+    case 6: return pick_mask_kind<HDIM, true, true, false>(mask_kind);
+    default: return pick_mask_kind<HDIM, true, true, true>(mask_kind);
+    }
+}
+#define SMA_NAME2(d) fwd_kernel_##d
+#define SMA_NAME(d) SMA_NAME2(d)
+FwdKernel SMA_NAME(SMA_FWD_HEAD_DIM)(int variant, int mask_kind) { return pick<SMA_FWD_HEAD_DIM>(variant, mask_kind); }
+#else
+FwdKernel fwd_kernel_32(int variant, int mask_kind);
+FwdKernel fwd_kernel_64(int variant, int mask_kind);
+FwdKernel fwd_kernel_96(int variant, int mask_kind);
+FwdKernel fwd_kernel_128(int variant, int mask_kind);
 
 // Number of compute units of the current device (cached per device ordinal).
 static int compute_units()
@@ -858,75 +910,21 @@ hipError_t launch_attn_fwd(const AttnArgs &args, bool bf16, hipStream_t stream)
     a.tail_start = (groups > 2 * cus && groups <= 3 * cus) ? 0 : (int)groups;
     const dim3 grid((unsigned)groups), block(NTHREADS);
     const bool postmul = a.post_mul != 1.0f;
-    const int D = a.D;
-    const bool packed = (int)a.q.sn == D && (int)a.k.sn == D && (int)a.v.sn == D && (int)a.out.sn == D;
-    if (D == 2 * HD) a.tail_start = (int)groups;              // two work-groups per CU: nobody yields
-    void (*kernel)(const AttnArgs) = nullptr;
-    const int variant = (bf16 ? 4 : 0) | (postmul ? 2 : 0) | (packed ? 1 : 0);
-#define SMA_FWD_VARIANTS(HDIM)                                                          \
-    switch (variant) {                                                                 \
-    case 0: kernel = attn_fwd_kernel<false, false, false, HDIM>; break;                \
-    case 1: kernel = attn_fwd_kernel<false, false, true, HDIM>; break;                 \
-    case 2: kernel = attn_fwd_kernel<false, true, false, HDIM>; break;                 \
-    case 3: kernel = attn_fwd_kernel<false, true, true, HDIM>; break;                  \
-    case 4: kernel = attn_fwd_kernel<true, false, false, HDIM>; break;                 \
-    case 5: kernel = attn_fwd_kernel<true, false, true, HDIM>; break;                  \
-    case 6: kernel = attn_fwd_kernel<true, true, false, HDIM>; break;                  \
-    default: kernel = attn_fwd_kernel<true, true, true, HDIM>; break;                  \
-    }
-#define SMA_FWD_BYTEMASK_VARIANTS(HDIM)                                                 \
-    switch (variant | (byproducts ? 8 : 0)) {                                          \
-    case 0: kernel = attn_fwd_kernel<false, false, false, HDIM, true>; break;          \
-    case 1: kernel = attn_fwd_kernel<false, false, true, HDIM, true>; break;           \
-    case 2: kernel = attn_fwd_kernel<false, true, false, HDIM, true>; break;           \
-    case 3: kernel = attn_fwd_kernel<false, true, true, HDIM, true>; break;            \
-    case 4: kernel = attn_fwd_kernel<true, false, false, HDIM, true>; break;           \
-    case 5: kernel = attn_fwd_kernel<true, false, true, HDIM, true>; break;            \
-    case 6: kernel = attn_fwd_kernel<true, true, false, HDIM, true>; break;            \
-    case 7: kernel = attn_fwd_kernel<true, true, true, HDIM, true>; break;             \
-    case 8: kernel = attn_fwd_kernel<false, false, false, HDIM, true, true>; break;    \
-    case 9: kernel = attn_fwd_kernel<false, false, true, HDIM, true, true>; break;     \
-    case 10: kernel = attn_fwd_kernel<false, true, false, HDIM, true, true>; break;    \
-    case 11: kernel = attn_fwd_kernel<false, true, true, HDIM, true, true>; break;     \
-    case 12: kernel = attn_fwd_kernel<true, false, false, HDIM, true, true>; break;    \
-    case 13: kernel = attn_fwd_kernel<true, false, true, HDIM, true, true>; break;     \
-    case 14: kernel = attn_fwd_kernel<true, true, false, HDIM, true, true>; break;     \
-    default: kernel = attn_fwd_kernel<true, true, true, HDIM, true, true>; break;      \
-    }
-#define SMA_FWD_PAIRS_VARIANTS(HDIM)                                                    \
-    switch (variant | (byproducts ? 8 : 0)) {                                          \
-    case 0: kernel = attn_fwd_kernel<false, false, false, HDIM, true, false, true>; break;   \
-    case 1: kernel = attn_fwd_kernel<false, false, true, HDIM, true, false, true>; break;    \
-    case 2: kernel = attn_fwd_kernel<false, true, false, HDIM, true, false, true>; break;    \
-    case 3: kernel = attn_fwd_kernel<false, true, true, HDIM, true, false, true>; break;     \
-    case 4: kernel = attn_fwd_kernel<true, false, false, HDIM, true, false, true>; break;    \
-    case 5: kernel = attn_fwd_kernel<true, false, true, HDIM, true, false, true>; break;     \
-    case 6: kernel = attn_fwd_kernel<true, true, false, HDIM, true, false, true>; break;     \
-    case 7: kernel = attn_fwd_kernel<true, true, true, HDIM, true, false, true>; break;      \
-    case 8: kernel = attn_fwd_kernel<false, false, false, HDIM, true, true, true>; break;    \
-    case 9: kernel = attn_fwd_kernel<false, false, true, HDIM, true, true, true>; break;     \
-    case 10: kernel = attn_fwd_kernel<false, true, false, HDIM, true, true, true>; break;    \
-    case 11: kernel = attn_fwd_kernel<false, true, true, HDIM, true, true, true>; break;     \
-    case 12: kernel = attn_fwd_kernel<true, false, false, HDIM, true, true, true>; break;    \
-    case 13: kernel = attn_fwd_kernel<true, false, true, HDIM, true, true, true>; break;     \
-    case 14: kernel = attn_fwd_kernel<true, true, false, HDIM, true, true, true>; break;     \
-    default: kernel = attn_fwd_kernel<true, true, true, HDIM, true, true, true>; break;      \
-    }
+    const int D = kernel_head_dim(a.D);
+    const bool packed = a.D == D && (int)a.q.sn == D && (int)a.k.sn == D && (int)a.v.sn == D;
+    if (D > HD) a.tail_start = (int)groups;                   // two work-groups per CU: nobody yields
     const bool byproducts = a.mask_out != nullptr || a.map_out != nullptr;
     // two tiles' mask bytes per request (see PAIRS at the kernel), unless the grid is the single round
     // of work-groups in step for which tail_start was set to 0 above
-    const bool pairs = a.byte_mask && D <= 64 && a.N % (2 * BN) == 0 && a.tail_start != 0;
-    if (pairs) {
-        if (D == 32) { SMA_FWD_PAIRS_VARIANTS(32) } else { SMA_FWD_PAIRS_VARIANTS(64) }
-    } else if (a.byte_mask) {
-        if (a.N < 16) return hipErrorInvalidValue;          // a row holds at least one 16-byte copy (checked by the C-ABI layer)
-        if (D == 32) { SMA_FWD_BYTEMASK_VARIANTS(32) } else if (D == 64) { SMA_FWD_BYTEMASK_VARIANTS(64) } else { SMA_FWD_BYTEMASK_VARIANTS(128) }
-    } else if (D == 32) { SMA_FWD_VARIANTS(32) } else if (D == 64) { SMA_FWD_VARIANTS(64) } else { SMA_FWD_VARIANTS(128) }
-#undef SMA_FWD_VARIANTS
-#undef SMA_FWD_BYTEMASK_VARIANTS
-#undef SMA_FWD_PAIRS_VARIANTS
+    const bool pairs = a.byte_mask && D <= HD && a.N % (2 * BN) == 0 && a.tail_start != 0;
+    if (a.byte_mask && a.N < 16) return hipErrorInvalidValue;  // a row holds at least one 16-byte copy (checked by the C-ABI layer)
+    const int mask_kind = !a.byte_mask ? 0 : (pairs ? 3 : 1) + (byproducts ? 1 : 0);
+    const int variant = (bf16 ? 4 : 0) | (postmul ? 2 : 0) | (packed ? 1 : 0);
+    const FwdKernel kernel = D == 32 ? fwd_kernel_32(variant, mask_kind) : D == 64 ? fwd_kernel_64(variant, mask_kind)
+                             : D == 96 ? fwd_kernel_96(variant, mask_kind) : fwd_kernel_128(variant, mask_kind);
     hipLaunchKernelGGL(kernel, grid, block, 0, stream, a);
     return hipGetLastError();
 }
+#endif
 
 }  // namespace sma

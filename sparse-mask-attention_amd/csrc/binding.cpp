@@ -334,14 +334,6 @@ torch::Tensor tile_map(const torch::Tensor &mask_packed)
 
 using torch::Tensor;
 
-// An uninitialised tensor like t (its strides too, where they leave no gaps), what torch.empty_like gives.
-Tensor empty_like_rows(const Tensor &t)
-{
-    if (t.is_contiguous()) return empty_dense(t.sizes(), t.scalar_type());
-    if (t.is_non_overlapping_and_dense()) return empty_rows(t.sizes(), t.strides(), t.scalar_type());
-    return at::empty_like(t.detach());
-}
-
 // Whether the kernels can address t as it is: contiguous last dimension, the strides of the others
 // non-negative multiples of 8 elements, 16-byte aligned storage.
 bool addressable(const Tensor &t)
@@ -353,13 +345,44 @@ bool addressable(const Tensor &t)
     return true;
 }
 
-// q, k, v or a gradient as the kernels take it: 16-bit elements of type `dtype`, head dim Dk (zeros
-// after the tensor's own), addressable.
-Tensor kernel_rows(const Tensor &t, at::ScalarType dtype, int64_t Dk)
+// Head dim of the kernels' tensors for one of the caller's: the next multiple of 8 (16 bytes).
+int64_t padded_head_dim(int64_t D) { return (D + 7) / 8 * 8; }
+
+// q, k, v or a gradient as the kernels take them: 16-bit elements of type `dtype`, head dim Dk (zeros after the
+// tensor's own), addressable.  fp32 tensors that leave no gaps, all of one size, are converted in one launch that
+// keeps their layout; the caller holds the device guard.
+template <size_t COUNT>
+void kernel_rows(const Tensor *const (&from)[COUNT], Tensor *const (&to)[COUNT], at::ScalarType dtype, int64_t Dk)
 {
-    Tensor r = t.scalar_type() == dtype ? t : t.to(dtype);
-    if (r.size(3) != Dk) return at::constant_pad_nd(r, {0, Dk - r.size(3)});
-    return addressable(r) ? r : r.contiguous();
+    bool flat = dtype == at::kBFloat16 && COUNT <= 3;
+    for (const Tensor *t : from)
+        flat = flat && t->scalar_type() == at::kFloat && t->size(3) == Dk && t->is_non_overlapping_and_dense() && t->stride(3) == 1 &&
+               t->numel() == from[0]->numel() && reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0;
+    if (flat) {
+        const float *src[COUNT];
+        uint16_t *dst[COUNT];
+        for (size_t i = 0; i < COUNT; ++i) {
+            *to[i] = from[i]->is_contiguous() ? empty_dense(from[i]->sizes(), dtype) : empty_rows(from[i]->sizes(), from[i]->strides(), dtype);
+            src[i] = static_cast<const float *>(from[i]->data_ptr());
+            dst[i] = static_cast<uint16_t *>(to[i]->data_ptr());
+        }
+        hipStream_t stream = c10::hip::getCurrentHIPStream(from[0]->device().index()).stream();
+        check_status(sma_to_bf16(src, dst, (int)COUNT, from[0]->numel(), stream), "sma_to_bf16");
+        return;
+    }
+    for (size_t i = 0; i < COUNT; ++i) {
+        Tensor r = from[i]->scalar_type() == dtype ? *from[i] : from[i]->to(dtype);
+        if (r.size(3) != Dk) r = at::constant_pad_nd(r, {0, Dk - r.size(3)});
+        *to[i] = addressable(r) ? r : r.contiguous();
+    }
+}
+
+// An uninitialised tensor laid out like t, of another element type.
+Tensor empty_like_rows(const Tensor &t, at::ScalarType dtype)
+{
+    if (t.is_contiguous()) return empty_dense(t.sizes(), dtype);
+    if (t.is_non_overlapping_and_dense()) return empty_rows(t.sizes(), t.strides(), dtype);
+    return at::empty_like(t.detach(), t.options().dtype(dtype));
 }
 
 // The mask with its expanded (stride 0) batch / head extents taken back to 1: it is then read once
@@ -405,36 +428,55 @@ void pack_with_map(Call &c)
     check_status(st, "sma_pack_mask_map");
 }
 
-// Forward of `c` into `out`; with `lse` defined, the packed mask is left in c.packed and, if
-// `want_map` or if one was made anyway, the tile map in c.map, for the backward.
-void run_forward(Call &c, Tensor &out, const Tensor &lse, bool want_map)
+// Whether the forward can read c's boolean mask as it is (c.mask is contiguous, q, k and v addressable).
+bool reads_bytes(const Call &c)
+{
+    if (c.N < 16 || c.N * c.N >= (int64_t(1) << 31)) return false;
+    // the kernel copies mask rows from whatever byte address they start at: the library checks once
+    // per device that such copies are served (always, under ROCm); where not, the mask is packed
+    return sma_device_check(c10::hip::getCurrentHIPStream(c.q.device().index()).stream()) == SMA_OK;
+}
+
+// Forward of `c` into `out` and / or its fp32 copy `out_f32`; with `lse` defined, the packed mask is left in
+// c.packed and, if `want_map` or if one was made anyway, the tile map in c.map, for the backward.
+void run_forward(Call &c, const Tensor &out, const Tensor &out_f32, const Tensor &lse, bool want_map)
 {
     const bool training = lse.defined();
-    const c10::optional<Tensor> lse_arg = training ? c10::optional<Tensor>(lse) : c10::nullopt;
-    if (!c.packed.defined()) {
-        if (pack_first(c)) {
+    const int64_t T = (c.N + 63) / 64;
+    TORCH_CHECK(c.B <= INT32_MAX && c.H <= INT32_MAX && c.N <= INT32_MAX, "extent too large");
+    sma_fwd_call f = {};
+    if (!c.packed.defined() && c.q.numel() > 0) {
+        if (pack_first(c) || (training && want_map && !reads_bytes(c))) {
             pack_with_map(c);
-        } else if (bool_mask_supported(c.q, c.k, c.v, c.mask)) {
-            c10::optional<Tensor> packed_out, map_out;
+        } else if (reads_bytes(c)) {
+            f.mask = reinterpret_cast<const uint8_t *>(c.mask.data_ptr<bool>());
+            f.mask_stride_b = c.mask.size(0) == 1 ? 0 : c.mask.size(1) * c.N * c.N;
+            f.mask_stride_h = c.mask.size(1) == 1 ? 0 : c.N * c.N;
             if (training) {
-                const int64_t T = (c.N + 63) / 64;
                 c.packed = empty_dense({c.mask.size(0), c.mask.size(1), c.N, (c.N + 31) / 32}, at::kInt);
-                packed_out = c.packed;
-                if (want_map) {
-                    c.map = empty_dense({c.mask.size(0), c.mask.size(1), T, 2, (T + 31) / 32}, at::kInt);
-                    map_out = c.map;
-                }
+                f.packed_out = reinterpret_cast<uint32_t *>(c.packed.data_ptr<int32_t>());
             }
-            forward_bool_mask(c.q, c.k, c.v, c.mask, out, lse_arg, c.scale, training, packed_out, map_out);
-            return;
-        } else if (training && want_map) {
-            pack_with_map(c);
-        } else {
-            c.packed = pack_mask(c.mask);
+            if (training && want_map) {
+                c.map = empty_dense({c.mask.size(0), c.mask.size(1), T, 2, (T + 31) / 32}, at::kInt);
+                f.map_out = reinterpret_cast<uint32_t *>(c.map.data_ptr<int32_t>());
+            }
         }
     }
-    forward(c.q, c.k, c.v, c.packed, out, lse_arg, c.scale, training,
-            c.map.defined() ? c10::optional<Tensor>(c.map) : c10::nullopt);
+    if (!f.mask) {
+        if (!c.packed.defined()) c.packed = pack_mask(c.mask);
+        mask_strides(c.packed, c.q, &f.mask_stride_b, &f.mask_stride_h);
+        f.mask_packed = reinterpret_cast<const uint32_t *>(c.packed.data_ptr<int32_t>());
+        f.tile_map = map_pointer(c.map.defined() ? c10::optional<Tensor>(c.map) : c10::nullopt, c.packed, c.q);
+    }
+    sma_tensor t[5] = {rows_of(c.q, "q"), rows_of(c.k, "k"), rows_of(c.v, "v")};
+    f.q = &t[0], f.k = &t[1], f.v = &t[2];
+    if (out.defined()) t[3] = rows_of(out, "out"), f.out = &t[3];
+    if (out_f32.defined()) t[4] = rows_of(out_f32, "out"), f.out_f32 = &t[4];
+    f.lse = training ? lse.data_ptr<float>() : nullptr;
+    f.B = (int)c.B, f.H = (int)c.H, f.N = (int)c.N, f.D = (int)c.q.size(3);
+    f.scale = (float)c.scale;
+    f.dtype = c.q.scalar_type() == at::kBFloat16 ? SMA_DTYPE_BF16 : SMA_DTYPE_F16;
+    check_status(sma_attn_fwd_call(&f, c10::hip::getCurrentHIPStream(c.q.device().index()).stream()), "sma_attn_fwd_call");
 }
 
 // The autograd node of one training forward.
@@ -466,14 +508,33 @@ struct SparseAttentionBackward : public torch::autograd::Node {
         const Tensor tlse = lse.unpack(), tpacked = packed.unpack();
         at::NoGradGuard no_grad;
         const c10::DeviceGuard guard(tq.device());
-        const Tensor dout = kernel_rows(grads[0], tq.scalar_type(), tq.size(3));
-        Tensor d[3] = {empty_like_rows(tq), empty_like_rows(tk), empty_like_rows(tv)};
-        backward(dout, tq, tk, tv, tout, tlse, tpacked, d[0], d[1], d[2], scale,
-                 map.defined() ? c10::optional<Tensor>(map) : c10::nullopt);
-        for (Tensor &t : d) {
-            if (t.size(3) != grad_D) t = t.narrow(3, 0, grad_D);
-            if (t.scalar_type() != grad_dtype) t = t.to(grad_dtype);
-        }
+        Tensor dout;
+        kernel_rows<1>({&grads[0]}, {&dout}, tq.scalar_type(), tq.size(3));
+        // the gradients in the caller's type and layout at once, unless its rows are no multiple of 16 bytes
+        const bool direct = grad_D == tq.size(3);
+        const at::ScalarType made = direct ? grad_dtype : tq.scalar_type();
+        Tensor d[3] = {empty_like_rows(tq, made), empty_like_rows(tk, made), empty_like_rows(tv, made)};
+        const int64_t B = tq.size(0), H = tq.size(1), N = tq.size(2);
+        Tensor delta = empty_dense({B, H, N}, at::kFloat);             // workspace of the C entry point
+        sma_tensor t[8] = {rows_of(dout, "dout"), rows_of(tq, "q"), rows_of(tk, "k"), rows_of(tv, "v"), rows_of(tout, "out"),
+                           rows_of(d[0], "dq"), rows_of(d[1], "dk"), rows_of(d[2], "dv")};
+        sma_bwd_call c = {};
+        c.dout = &t[0], c.q = &t[1], c.k = &t[2], c.v = &t[3], c.out = &t[4], c.dq = &t[5], c.dk = &t[6], c.dv = &t[7];
+        c.lse = tlse.data_ptr<float>();
+        mask_strides(tpacked, tq, &c.mask_stride_b, &c.mask_stride_h);
+        c.mask_packed = reinterpret_cast<const uint32_t *>(tpacked.data_ptr<int32_t>());
+        c.tile_map = map_pointer(map.defined() ? c10::optional<Tensor>(map) : c10::nullopt, tpacked, tq);
+        c.delta_ws = delta.data_ptr<float>();
+        c.B = (int)B, c.H = (int)H, c.N = (int)N, c.D = (int)tq.size(3);
+        c.scale = (float)scale;
+        c.dtype = tq.scalar_type() == at::kBFloat16 ? SMA_DTYPE_BF16 : SMA_DTYPE_F16;
+        c.grads_f32 = made == at::kFloat;
+        check_status(sma_attn_bwd_call(&c, c10::hip::getCurrentHIPStream(tq.device().index()).stream()), "sma_attn_bwd_call");
+        if (!direct)
+            for (Tensor &g : d) {
+                g = g.narrow(3, 0, grad_D);
+                if (g.scalar_type() != grad_dtype) g = g.to(grad_dtype);
+            }
         return {d[0], d[1], d[2]};
     }
 };
@@ -483,7 +544,7 @@ Tensor run_call(const Tensor &q, const Tensor &k, const Tensor &v, Call &c, bool
 {
     const at::ScalarType dtype = q.scalar_type();
     const at::ScalarType kdt = dtype == at::kFloat ? at::kBFloat16 : dtype;
-    const int64_t Dk = c.D <= 32 ? 32 : (c.D <= 64 ? 64 : 128);
+    const int64_t Dk = padded_head_dim(c.D);
     const bool map_shown = want_map || c.map.defined();
     const bool tracked = autograd && torch::autograd::compute_requires_grad(q, k, v);
     std::shared_ptr<SparseAttentionBackward> node;
@@ -493,15 +554,19 @@ Tensor run_call(const Tensor &q, const Tensor &k, const Tensor &v, Call &c, bool
     }
     const c10::DeviceGuard guard(q.device());
     at::AutoDispatchBelowADInplaceOrView below_autograd;
-    c.q = kernel_rows(q, kdt, Dk);
-    c.k = kernel_rows(k, kdt, Dk);
-    c.v = kernel_rows(v, kdt, Dk);
-    Tensor out = empty_like_rows(c.q), lse;
+    kernel_rows<3>({&q, &k, &v}, {&c.q, &c.k, &c.v}, kdt, Dk);
+    // fp32 callers get their result from the kernel itself; the 16-bit one is then made for the backward only
+    const bool wide = kdt != dtype && Dk == c.D;
+    Tensor out, result, lse;
+    if (!wide || tracked) out = empty_like_rows(c.q, kdt);
+    if (wide) result = empty_like_rows(c.q, dtype);
     if (tracked) lse = empty_dense({c.B, c.H, c.N}, at::kFloat);
-    run_forward(c, out, lse, want_map);
-    Tensor result = out;
-    if (Dk != c.D) result = result.narrow(3, 0, c.D);
-    if (kdt != dtype) result = result.to(dtype);
+    run_forward(c, out, result, lse, want_map);
+    if (!wide) {
+        result = out;
+        if (Dk != c.D) result = result.narrow(3, 0, c.D);
+        if (kdt != dtype) result = result.to(dtype);
+    }
     if (!tracked) return result;
     torch::autograd::set_history(result, node);
     node->out_is_output = result.is_same(out);

@@ -26,13 +26,14 @@ inline sma_tensor dense(const void *p, int H, int N, int D)
 // Checks one strided [B,H,N,D] tensor and converts it; SMA_OK or an error code.  An output
 // (`written`) must not fold several rows onto one address: a row stride below D or a zero stride
 // over an extent above 1 would make rows or work-groups overwrite each other.
-int to_rows(const sma_tensor *t, int B, int H, int N, int D, bool written, sma::Rows *r)
+int to_rows(const sma_tensor *t, int B, int H, int N, int D, bool written, sma::Rows *r, bool f32 = false)
 {
     if (t == nullptr || t->data == nullptr) return SMA_ERR_NULL_POINTER;
     if (misaligned(t->data, 16)) return SMA_ERR_ALIGNMENT;
     if (t->stride_b < 0 || t->stride_h < 0 || t->stride_n < 0) return SMA_ERR_STRIDE;
     if ((t->stride_b | t->stride_h | t->stride_n) & 7) return SMA_ERR_STRIDE;
-    if ((long long)(N - 1) * t->stride_n * 2 + 2 * D >= (1ll << 31)) return SMA_ERR_STRIDE;
+    const int size = f32 ? 4 : 2;
+    if ((long long)(N - 1) * t->stride_n * size + size * D >= (1ll << 31)) return SMA_ERR_STRIDE;
     if (t->stride_b >= (1ll << 35) || t->stride_h >= (1ll << 35) || t->stride_n >= (1ll << 23)) return SMA_ERR_STRIDE;
     if (written && ((N > 1 && t->stride_n < D) || (H > 1 && t->stride_h == 0) || (B > 1 && t->stride_b == 0)))
         return SMA_ERR_STRIDE;
@@ -169,6 +170,9 @@ static void last_tile_masks(int N, uint32_t *m0, uint32_t *m1)
     *m1 = v1 >= 32 ? 0xffffffffu : ((1u << v1) - 1u);
 }
 
+// The head dims of the reference-shaped entry points; sma_attn_fwd_call / sma_attn_bwd_call take more.
+static bool plain_head_dim(int D) { return D == 32 || D == 64 || D == 128; }
+
 int sma_attn_bwd_map_strided(const sma_tensor *dout, const sma_tensor *q, const sma_tensor *k,
                              const sma_tensor *v, const sma_tensor *out, const float *lse,
                              const uint32_t *mask_packed, int64_t mask_stride_b, int64_t mask_stride_h,
@@ -176,45 +180,57 @@ int sma_attn_bwd_map_strided(const sma_tensor *dout, const sma_tensor *q, const 
                              const sma_tensor *dv, float *delta_ws, int B, int H, int N, int D, float scale,
                              int dtype, void *stream)
 {
+    if (B >= 0 && H >= 0 && N >= 0 && D >= 0 && !plain_head_dim(D)) return SMA_ERR_HEAD_DIM;
+    const sma_bwd_call c = {dout, q, k, v, out, dq, dk, dv, lse, mask_packed, mask_stride_b, mask_stride_h, tile_map,
+                            delta_ws, B, H, N, D, scale, dtype, 0};
+    return sma_attn_bwd_call(&c, stream);
+}
+
+int sma_attn_bwd_call(const sma_bwd_call *c, void *stream)
+{
+    if (c == nullptr) return SMA_ERR_NULL_POINTER;
+    const int B = c->B, H = c->H, N = c->N, D = c->D;
     if (B < 0 || H < 0 || N < 0 || D < 0) return SMA_ERR_BAD_SHAPE;
-    if (D != 32 && D != 64 && D != 128) return SMA_ERR_HEAD_DIM;
-    if (dtype != SMA_DTYPE_F16 && dtype != SMA_DTYPE_BF16) return SMA_ERR_DTYPE;
-    if (!isfinite(scale)) return SMA_ERR_SCALE;
+    if (D == 0 || D % 8 != 0 || D > 128) return SMA_ERR_HEAD_DIM;
+    if (c->dtype != SMA_DTYPE_F16 && c->dtype != SMA_DTYPE_BF16) return SMA_ERR_DTYPE;
+    if (!isfinite(c->scale)) return SMA_ERR_SCALE;
     const long long BH = (long long)B * H;
     if (BH == 0 || N == 0) return SMA_OK;
-    if (!lse || !mask_packed || !delta_ws) return SMA_ERR_NULL_POINTER;
+    if (c->grads_f32 && c->dtype != SMA_DTYPE_BF16) return SMA_ERR_DTYPE;
+    if (!c->lse || !c->mask_packed || !c->delta_ws) return SMA_ERR_NULL_POINTER;
     const long long qtiles = (N + 127) / 128;
     if (!below_2_31(BH, qtiles) || !below_2_31(BH, N)) return SMA_ERR_BAD_SHAPE;
     // a lane's byte offset into the packed mask of one (b,h) is a 32-bit register
     if ((long long)N * ((N + 31) / 32) * 4 >= (1ll << 32)) return SMA_ERR_BAD_SHAPE;
-    if (misaligned(mask_packed, 4) || misaligned(lse, 4) || misaligned(delta_ws, 4) || (tile_map && misaligned(tile_map, 4)))
+    if (misaligned(c->mask_packed, 4) || misaligned(c->lse, 4) || misaligned(c->delta_ws, 4) || (c->tile_map && misaligned(c->tile_map, 4)))
         return SMA_ERR_ALIGNMENT;
-    if (tile_map && N > 131072) return SMA_ERR_BAD_SHAPE;
-    if (mask_stride_b < 0 || mask_stride_h < 0) return SMA_ERR_STRIDE;
+    if (c->tile_map && N > 131072) return SMA_ERR_BAD_SHAPE;
+    if (c->mask_stride_b < 0 || c->mask_stride_h < 0) return SMA_ERR_STRIDE;
 
     sma::AttnBwdArgs a;
-    const sma_tensor *in[8] = {dout, q, k, v, out, dq, dk, dv};
+    const sma_tensor *in[8] = {c->dout, c->q, c->k, c->v, c->out, c->dq, c->dk, c->dv};
     sma::Rows *to[8] = {&a.dout, &a.q, &a.k, &a.v, &a.out, &a.dq, &a.dk, &a.dv};
     for (int i = 0; i < 8; ++i) {
-        const int st = to_rows(in[i], B, H, N, D, i >= 5, to[i]);
+        const int st = to_rows(in[i], B, H, N, D, i >= 5, to[i], i >= 5 && c->grads_f32);
         if (st != SMA_OK) return st;
     }
-    a.lse = lse;
-    a.mask = sma::PackedMask{mask_packed, mask_stride_b, mask_stride_h};
-    a.delta = delta_ws;
-    a.tile_map = tile_map;
+    a.lse = c->lse;
+    a.mask = sma::PackedMask{c->mask_packed, c->mask_stride_b, c->mask_stride_h};
+    a.delta = c->delta_ws;
+    a.tile_map = c->tile_map;
+    a.grads_f32 = c->grads_f32 != 0;
     const long long map_words = sma_tile_map_words(N);
-    a.map_sh = (H > 1 && mask_stride_h != 0) ? map_words : 0;
-    a.map_sb = (B > 1 && mask_stride_b != 0) ? ((H > 1 && mask_stride_h != 0) ? (long long)H : 1ll) * map_words : 0;
+    a.map_sh = (H > 1 && c->mask_stride_h != 0) ? map_words : 0;
+    a.map_sb = (B > 1 && c->mask_stride_b != 0) ? ((H > 1 && c->mask_stride_h != 0) ? (long long)H : 1ll) * map_words : 0;
     a.BH = (int)BH;
     a.H = H;
     a.N = N;
     a.D = D;
     a.qtiles = (int)qtiles;
-    a.scale = scale;
-    split_scale(scale, &a.q_scale, &a.post_mul);
+    a.scale = c->scale;
+    split_scale(c->scale, &a.q_scale, &a.post_mul);
     last_tile_masks(N, &a.last_mask0, &a.last_mask1);
-    const hipError_t e = sma::launch_attn_bwd(a, dtype == SMA_DTYPE_BF16, static_cast<hipStream_t>(stream));
+    const hipError_t e = sma::launch_attn_bwd(a, c->dtype == SMA_DTYPE_BF16, static_cast<hipStream_t>(stream));
     return e == hipSuccess ? SMA_OK : SMA_ERR_LAUNCH;
 }
 
@@ -246,48 +262,71 @@ int sma_attn_fwd_map_strided(const sma_tensor *q, const sma_tensor *k, const sma
                              const uint32_t *tile_map, const sma_tensor *out, float *lse, int B, int H,
                              int N, int D, float scale, int dtype, void *stream)
 {
+    if (B >= 0 && H >= 0 && N >= 0 && D >= 0 && !plain_head_dim(D)) return SMA_ERR_HEAD_DIM;
+    if (B > 0 && H > 0 && N > 0 && !out) return SMA_ERR_NULL_POINTER;
+    const sma_fwd_call c = {q, k, v, out, nullptr, nullptr, mask_packed, mask_stride_b, mask_stride_h, tile_map, lse,
+                            nullptr, nullptr, B, H, N, D, scale, dtype};
+    return sma_attn_fwd_call(&c, stream);
+}
+
+int sma_attn_fwd_call(const sma_fwd_call *c, void *stream)
+{
+    if (c == nullptr) return SMA_ERR_NULL_POINTER;
+    const int B = c->B, H = c->H, N = c->N, D = c->D;
+    const bool bytes = c->mask != nullptr;
     if (B < 0 || H < 0 || N < 0 || D < 0) return SMA_ERR_BAD_SHAPE;
-    if (D != 32 && D != 64 && D != 128) return SMA_ERR_HEAD_DIM;
-    if (dtype != SMA_DTYPE_F16 && dtype != SMA_DTYPE_BF16) return SMA_ERR_DTYPE;
-    if (!isfinite(scale)) return SMA_ERR_SCALE;
+    if (D == 0 || D % 8 != 0 || D > 128) return SMA_ERR_HEAD_DIM;
+    if (c->dtype != SMA_DTYPE_F16 && c->dtype != SMA_DTYPE_BF16) return SMA_ERR_DTYPE;
+    if (!isfinite(c->scale)) return SMA_ERR_SCALE;
     const long long BH = (long long)B * H;
     if (BH == 0 || N == 0) return SMA_OK;
-    if (!mask_packed) return SMA_ERR_NULL_POINTER;
+    if (!bytes && !c->mask_packed) return SMA_ERR_NULL_POINTER;
+    if (!c->out && !c->out_f32) return SMA_ERR_NULL_POINTER;
+    if (c->out_f32 && c->dtype != SMA_DTYPE_BF16) return SMA_ERR_DTYPE;
+    if (bytes && N < 16) return SMA_ERR_BAD_SHAPE;               // a row holds at least one 16-byte copy
     const long long qtiles = (N + 127) / 128;
     if (!below_2_31(BH, qtiles) || !below_2_31(BH, N)) return SMA_ERR_BAD_SHAPE;
-    // a lane's byte offset into the packed mask of one (b,h) is a 32-bit register
-    if ((long long)N * ((N + 31) / 32) * 4 >= (1ll << 32)) return SMA_ERR_BAD_SHAPE;
-    if (misaligned(mask_packed, 4) || (lse && misaligned(lse, 4)) || (tile_map && misaligned(tile_map, 4)))
+    // a lane's byte offset into the mask of one (b,h) is a 32-bit register
+    if (bytes ? (long long)N * N >= (1ll << 31) : (long long)N * ((N + 31) / 32) * 4 >= (1ll << 32)) return SMA_ERR_BAD_SHAPE;
+    if ((!bytes && misaligned(c->mask_packed, 4)) || (c->lse && misaligned(c->lse, 4)) || (c->tile_map && misaligned(c->tile_map, 4)) ||
+        (c->packed_out && misaligned(c->packed_out, 4)) || (c->map_out && misaligned(c->map_out, 4)))
         return SMA_ERR_ALIGNMENT;
-    if (tile_map && N > 131072) return SMA_ERR_BAD_SHAPE;      // the limit of sma_tile_map, which makes the maps
-    if (mask_stride_b < 0 || mask_stride_h < 0) return SMA_ERR_STRIDE;
+    if (c->tile_map && N > 131072) return SMA_ERR_BAD_SHAPE;     // the limit of sma_tile_map, which makes the maps
+    // the kernel collects the map in 32 words of 32 key tiles per wavefront (N <= 65536; the limit on
+    // N * N above is the tighter one)
+    if (c->map_out && (N + 63) / 64 > 32 * 32) return SMA_ERR_BAD_SHAPE;
+    if (c->mask_stride_b < 0 || c->mask_stride_h < 0) return SMA_ERR_STRIDE;
 
     sma::AttnArgs a;
-    const sma_tensor *in[4] = {q, k, v, out};
-    sma::Rows *to[4] = {&a.q, &a.k, &a.v, &a.out};
-    for (int i = 0; i < 4; ++i) {
-        const int st = to_rows(in[i], B, H, N, D, i == 3, to[i]);
+    const sma_tensor *in[5] = {c->q, c->k, c->v, c->out, c->out_f32};
+    sma::Rows *to[5] = {&a.q, &a.k, &a.v, &a.out, &a.out32};
+    for (int i = 0; i < 5; ++i) {
+        *to[i] = sma::Rows{nullptr, 0u, 0u, 0u};
+        if (i >= 3 && in[i] == nullptr) continue;
+        const int st = to_rows(in[i], B, H, N, D, i >= 3, to[i], i == 4);
         if (st != SMA_OK) return st;
     }
-    a.mask = sma::PackedMask{mask_packed, mask_stride_b, mask_stride_h};
-    a.lse = lse;
+    // mask rows start at any byte address: the kernel's 16-byte copies rely on the device serving them
+    if (bytes && sma::unaligned_access_state(static_cast<hipStream_t>(stream)) == 0) return SMA_ERR_DEVICE;
+    a.mask = sma::PackedMask{bytes ? reinterpret_cast<const uint32_t *>(c->mask) : c->mask_packed, c->mask_stride_b, c->mask_stride_h};
+    a.lse = c->lse;
     a.BH = (int)BH;
     a.H = H;
     a.N = N;
     a.D = D;
-    a.byte_mask = 0;
-    a.mask_out = nullptr;
-    a.map_out = nullptr;
+    a.byte_mask = bytes;
+    a.mask_out = bytes ? c->packed_out : nullptr;
+    a.map_out = bytes ? c->map_out : nullptr;
     // the map is contiguous [Bm, Hm, ...] with the mask's own Bm, Hm (1 where the mask is shared)
-    a.tile_map = tile_map;
+    a.tile_map = bytes ? nullptr : c->tile_map;
     const long long map_words = sma_tile_map_words(N);
-    a.map_sh = (H > 1 && mask_stride_h != 0) ? map_words : 0;
-    a.map_sb = (B > 1 && mask_stride_b != 0) ? ((H > 1 && mask_stride_h != 0) ? (long long)H : 1ll) * map_words : 0;
+    a.map_sh = (H > 1 && c->mask_stride_h != 0) ? map_words : 0;
+    a.map_sb = (B > 1 && c->mask_stride_b != 0) ? ((H > 1 && c->mask_stride_h != 0) ? (long long)H : 1ll) * map_words : 0;
     a.qtiles = (int)qtiles;
-    split_scale(scale, &a.q_scale, &a.post_mul);
+    split_scale(c->scale, &a.q_scale, &a.post_mul);
     last_tile_masks(N, &a.last_mask0, &a.last_mask1);
 
-    const hipError_t e = sma::launch_attn_fwd(a, dtype == SMA_DTYPE_BF16, static_cast<hipStream_t>(stream));
+    const hipError_t e = sma::launch_attn_fwd(a, c->dtype == SMA_DTYPE_BF16, static_cast<hipStream_t>(stream));
     return e == hipSuccess ? SMA_OK : SMA_ERR_LAUNCH;
 }
 
@@ -334,51 +373,30 @@ int sma_attn_fwd_bool_mask_strided(const sma_tensor *q, const sma_tensor *k, con
                                    const sma_tensor *out, float *lse, uint32_t *packed_out, uint32_t *map_out,
                                    int B, int H, int N, int D, float scale, int dtype, void *stream)
 {
-    if (B < 0 || H < 0 || N < 0 || D < 0) return SMA_ERR_BAD_SHAPE;
-    if (D != 32 && D != 64 && D != 128) return SMA_ERR_HEAD_DIM;
-    if (dtype != SMA_DTYPE_F16 && dtype != SMA_DTYPE_BF16) return SMA_ERR_DTYPE;
-    if (!isfinite(scale)) return SMA_ERR_SCALE;
-    const long long BH = (long long)B * H;
-    if (BH == 0 || N == 0) return SMA_OK;
-    if (!mask) return SMA_ERR_NULL_POINTER;
-    if (N < 16) return SMA_ERR_BAD_SHAPE;               // a row holds at least one 16-byte copy
-    const long long qtiles = (N + 127) / 128;
-    if (!below_2_31(BH, qtiles) || !below_2_31(BH, N)) return SMA_ERR_BAD_SHAPE;
-    // a lane's byte offset into the mask of one (b,h) is a 32-bit register
-    if ((long long)N * N >= (1ll << 31)) return SMA_ERR_BAD_SHAPE;
-    if ((lse && misaligned(lse, 4)) || (packed_out && misaligned(packed_out, 4)) || (map_out && misaligned(map_out, 4)))
-        return SMA_ERR_ALIGNMENT;
-    // the kernel collects the map in 32 words of 32 key tiles per wavefront (N <= 65536; the limit on
-    // N * N above is the tighter one)
-    if (map_out && (N + 63) / 64 > 32 * 32) return SMA_ERR_BAD_SHAPE;
-    if (mask_stride_b < 0 || mask_stride_h < 0) return SMA_ERR_STRIDE;
-
-    sma::AttnArgs a;
-    const sma_tensor *in[4] = {q, k, v, out};
-    sma::Rows *to[4] = {&a.q, &a.k, &a.v, &a.out};
-    for (int i = 0; i < 4; ++i) {
-        const int st = to_rows(in[i], B, H, N, D, i == 3, to[i]);
-        if (st != SMA_OK) return st;
+    if (B >= 0 && H >= 0 && N >= 0 && D >= 0 && !plain_head_dim(D)) return SMA_ERR_HEAD_DIM;
+    const sma_fwd_call c = {q, k, v, out, nullptr, mask, nullptr, mask_stride_b, mask_stride_h, nullptr, lse,
+                            packed_out, map_out, B, H, N, D, scale, dtype};
+    if (!mask || !out) {        // nothing to attend with: the checks of the rest first
+        const uint8_t none = 0;
+        sma_fwd_call d = c;
+        d.mask = &none;
+        d.B = B > 0 ? 0 : B;
+        const int st = sma_attn_fwd_call(&d, stream);
+        return st != SMA_OK ? st : (B == 0 || H == 0 || N == 0) ? SMA_OK : SMA_ERR_NULL_POINTER;
     }
-    // mask rows start at any byte address: the kernel's 16-byte copies rely on the device serving them
-    if (sma::unaligned_access_state(static_cast<hipStream_t>(stream)) == 0) return SMA_ERR_DEVICE;
-    a.mask = sma::PackedMask{reinterpret_cast<const uint32_t *>(mask), mask_stride_b, mask_stride_h};
-    a.lse = lse;
-    a.BH = (int)BH;
-    a.H = H;
-    a.N = N;
-    a.D = D;
-    a.byte_mask = 1;
-    a.mask_out = packed_out;
-    a.map_out = map_out;
-    a.tile_map = nullptr;
-    a.map_sb = a.map_sh = 0;
-    a.qtiles = (int)qtiles;
-    split_scale(scale, &a.q_scale, &a.post_mul);
-    last_tile_masks(N, &a.last_mask0, &a.last_mask1);
+    return sma_attn_fwd_call(&c, stream);
+}
 
-    const hipError_t e = sma::launch_attn_fwd(a, dtype == SMA_DTYPE_BF16, static_cast<hipStream_t>(stream));
-    return e == hipSuccess ? SMA_OK : SMA_ERR_LAUNCH;
+int sma_to_bf16(const float *const *src, uint16_t *const *dst, int count, long long n, void *stream)
+{
+    if (count < 0 || count > 3 || n < 0 || n % 8 != 0) return SMA_ERR_BAD_SHAPE;
+    if (count == 0 || n == 0) return SMA_OK;
+    if (src == nullptr || dst == nullptr) return SMA_ERR_NULL_POINTER;
+    for (int i = 0; i < count; ++i) {
+        if (src[i] == nullptr || dst[i] == nullptr) return SMA_ERR_NULL_POINTER;
+        if (misaligned(src[i], 16) || misaligned(dst[i], 16)) return SMA_ERR_ALIGNMENT;
+    }
+    return sma::launch_to_bf16(src, dst, count, n, static_cast<hipStream_t>(stream)) == hipSuccess ? SMA_OK : SMA_ERR_LAUNCH;
 }
 
 int sma_attn_bwd(const void *dout, const void *q, const void *k, const void *v, const void *out,

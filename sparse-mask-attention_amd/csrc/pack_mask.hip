@@ -33,6 +33,8 @@ namespace sma {
 namespace {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int PACK_THREADS = 256;
 constexpr int PACK_UNROLL = 2;
@@ -353,7 +355,44 @@ __global__ __launch_bounds__(PACK_THREADS) void tile_map_kernel(const uint32_t *
     }
 }
 
+// fp32 arrays -> bf16, 8 elements per thread and step.  Streaming: q, k and v of a call go in one launch
+// (blockIdx.y names the array), where a conversion and a zero-padding pass per tensor took six.
+struct ToBf16Args {
+    const f32x4 *src[3];
+    u32x4 *dst[3];
+    long long chunks;               // of 8 elements
+};
+__global__ __launch_bounds__(PACK_THREADS) void to_bf16_kernel(const ToBf16Args a)
+{
+    const f32x4 *src = a.src[blockIdx.y];
+    u32x4 *dst = a.dst[blockIdx.y];
+    for (long long i = (long long)blockIdx.x * PACK_THREADS + threadIdx.x; i < a.chunks; i += (long long)gridDim.x * PACK_THREADS) {
+        const f32x4 lo = __builtin_nontemporal_load(src + 2 * i), hi = __builtin_nontemporal_load(src + 2 * i + 1);
+        u32x4 o;
+        o.x = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)lo.x, (__bf16)lo.y});
+        o.y = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)lo.z, (__bf16)lo.w});
+        o.z = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)hi.x, (__bf16)hi.y});
+        o.w = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)hi.z, (__bf16)hi.w});
+        dst[i] = o;
+    }
+}
+
 }  // namespace
+
+hipError_t launch_to_bf16(const float *const *src, uint16_t *const *dst, int count, long long n, hipStream_t stream)
+{
+    if (n == 0 || count == 0) return hipSuccess;
+    ToBf16Args a;
+    for (int i = 0; i < 3; ++i) {
+        a.src[i] = reinterpret_cast<const f32x4 *>(src[i < count ? i : 0]);
+        a.dst[i] = reinterpret_cast<u32x4 *>(dst[i < count ? i : 0]);
+    }
+    a.chunks = n / 8;
+    const long long blocks = (a.chunks + PACK_THREADS - 1) / PACK_THREADS;
+    hipLaunchKernelGGL(to_bf16_kernel, dim3((unsigned)(blocks < 8192 ? blocks : 8192), (unsigned)count), dim3(PACK_THREADS), 0,
+                       stream, a);
+    return hipGetLastError();
+}
 
 hipError_t launch_pack_mask_map(const uint8_t *mask, uint32_t *packed, uint32_t *map, long long slabs, int N,
                                 hipStream_t stream)

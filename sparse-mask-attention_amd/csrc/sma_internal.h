@@ -47,10 +47,10 @@ __host__ __device__ inline uint32_t fastdiv(uint32_t n, FastDiv f)
 struct AttnArgs {
     Rows q, k, v;                   // inputs (never written)
     PackedMask mask;                // byte_mask != 0: p names boolean bytes [Bm, Hm, N, N], strides in bytes
-    Rows out;
+    Rows out, out32;                // 16-bit output and its fp32 copy (p names floats); p == nullptr: not wanted
     float *lse;                     // [BH, N] contiguous, or nullptr
     int BH, H, N;
-    int D;                          // head dim: 32, 64 or 128
+    int D;                          // head dim: a multiple of 8 up to 128
     int byte_mask;                  // the mask is the caller's boolean tensor, not packed words
     uint32_t *mask_out;             // byte_mask only: nullptr, or where to leave the packed words [Bm, Hm, N, nw]
     uint32_t *map_out;              // byte_mask only: nullptr, or where to leave the tile map (layout as tile_map below)
@@ -78,12 +78,13 @@ struct AttnBwdArgs {
     Rows dout, q, k, v, out;                   // inputs (never written)
     const float *lse;                          // [BH, N] natural-log-sum-exp saved by the forward
     PackedMask mask;
-    Rows dq, dk, dv;
+    Rows dq, dk, dv;                           // outputs: 16-bit elements, or floats if grads_f32
+    int grads_f32;
     float *delta;                              // [BH, N] workspace: sum_d dout * out per query row
     const uint32_t *tile_map;                  // nullptr, or the tile map of the mask (as in AttnArgs)
     long long map_sb, map_sh;
     int BH, H, N;
-    int D;                                     // head dim: 32, 64 or 128
+    int D;                                     // head dim: a multiple of 8 up to 128
     int qtiles;                                // ceil(N / 128)
     FastDiv div_qtiles, div_H;                 // filled in by the launcher
     float scale;                               // as given by the caller
@@ -91,8 +92,15 @@ struct AttnBwdArgs {
     uint32_t last_mask0, last_mask1;
 };
 
+// The kernels exist for head dims of 32, 64, 96 and 128; any multiple of 8 in between runs in the next larger
+// one: the copies fill an LDS row beyond the tensor's with its last 16 bytes once more, the fragments that the
+// wavefronts hold in registers are zero there, and results beyond it are not stored.
+inline int kernel_head_dim(int D) { return D <= 32 ? 32 : D <= 64 ? 64 : D <= 96 ? 96 : 128; }
+
 hipError_t launch_attn_fwd(const AttnArgs &a, bool bf16, hipStream_t stream);
 hipError_t launch_attn_bwd(const AttnBwdArgs &a, bool bf16, hipStream_t stream);
+// fp32 -> bf16 (round to nearest even), `count` (at most 3) arrays of n elements, n a multiple of 8
+hipError_t launch_to_bf16(const float *const *src, uint16_t *const *dst, int count, long long n, hipStream_t stream);
 hipError_t launch_pack_mask(const uint8_t *mask, uint32_t *packed, long long rows, int N,
                             hipStream_t stream);
 // Whether the current device serves 8- and 16-byte loads from unaligned addresses (the row packers
