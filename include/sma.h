@@ -141,7 +141,7 @@ int sma_attn_fwd_map(const void *q, const void *k, const void *v, const uint32_t
  *   delta_ws            float [B,H,N] workspace owned by the caller; holds sum_d dout*out per query
  *                       row on return (the library never allocates)
  *
- * Two launches on `stream` (dq, then dk and dv; three for D = 128: dq, dk, dv); no atomics, results are
+ * Two launches on `stream` (dq, then dk and dv); no atomics, results are
  * bit-reproducible.
  *
  * Replaces: void sparse_attention_bwd_bf16(const SparseAttentionParams&, const void* dout,

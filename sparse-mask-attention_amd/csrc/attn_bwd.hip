@@ -32,9 +32,7 @@
 //
 // Head dim 128 (NH = 2) is handled as two column halves of 64: every streamed matrix is kept in LDS
 // as two 64-column tiles, the products that contract over the head dim (S, dP) run over both
-// halves, the others (dQ, dK, dV) fill one pair of accumulators per half.  The dK/dV kernel would
-// need 128 accumulator registers for that; it is therefore launched twice, once for dK and once
-// for dV (S is formed in both).  Head dim 32 uses half a tile: the copies fill the upper half of
+// halves, the others (dQ, dK, dV) fill one pair of accumulators per half.  Head dim 32 uses half a tile: the copies fill the upper half of
 // every LDS row with copies of the row's last 16 bytes, which are never read;
 // contractions over the head dim take two MFMA steps and the outputs have one 32-column block.  Head dim 96
 // is 128 with such a half tile as its second half: six steps, three blocks.
@@ -351,17 +349,33 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_bwd_dq_kerne
 // ------------------------------------------------------------------------------------------------
 // dK and dV
 // ------------------------------------------------------------------------------------------------
-// DK / DV: which of the two gradients this instance produces (both for head dim 64; one per launch
-// for head dim 128, where both sets of accumulators do not fit the register file).
-template <bool BF16, int HDIM, bool DK, bool DV, bool POSTMUL, bool WIDE>
-__global__ __launch_bounds__(NTHREADS, 2) void attn_bwd_dkv_kernel(const AttnBwdArgs a)
+// NW wavefronts of 32 keys each.  Up to head dim 96 the K and V fragments of a wavefront's keys stay in
+// registers.  At 128 (VLDS) the accumulators of dK and dV take 128 registers; the V fragments then wait in LDS,
+// 16 bytes per lane and fragment in the order the lanes read them.  Both gradients in one kernel form S once
+// where a kernel for each formed it twice: 2783 -> 2032 us on 4 x 32 heads, N = 4096 (1.08 PFLOP/s over four
+// products).
+template <int HDIM, int NW> struct DkvCfg {
+    static constexpr bool VLDS = HDIM == 128;
+    static constexpr int NH = HDIM > 64 ? 2 : 1;
+    static constexpr int STAGE_BYTES = 2 * NH * TILE_BYTES;
+    static constexpr int OFF_B = NH * TILE_BYTES;           // dO inside a stage
+    static constexpr int AUX = NW * 256 + 512;              // per wavefront its mask words of 64 rows, then lse, delta
+    static constexpr int OFF_AUX = NSTAGE * STAGE_BYTES;
+    static constexpr int OFF_FRAG = OFF_AUX + NSTAGE * AUX; // V fragments of each wavefront
+    static constexpr int FRAG = VLDS ? HDIM / 16 * 1024 : 0;
+    static constexpr int LDS_BYTES = OFF_FRAG + NW * FRAG;
+};
+template <bool BF16, int HDIM, int NW, bool POSTMUL, bool WIDE>
+__global__ __launch_bounds__(64 * NW, HDIM == 128 ? NW / 4 : 2) void attn_bwd_dkv_kernel(const AttnBwdArgs a)
 {
     using E = Elem<BF16>;
     constexpr int NH = HDIM > 64 ? 2 : 1;
     constexpr int KS = HDIM / 16;
     constexpr int OB = HDIM / 32;
-    using C = Cfg<NH>;
-    constexpr int STAGE_BYTES = C::STAGE_BYTES, OFF_AUX = C::OFF_AUX;
+    using C = DkvCfg<HDIM, NW>;
+    constexpr int STAGE_BYTES = C::STAGE_BYTES, OFF_AUX = C::OFF_AUX, AUX_BYTES = C::AUX;
+    constexpr int OFF_LSE = NW * 256, OFF_DELTA = OFF_LSE + 256;       // inside the small data of a stage
+    constexpr bool VLDS = C::VLDS;
     __shared__ __attribute__((aligned(1024))) unsigned char smem[C::LDS_BYTES];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(LDS_PTR(unsigned char))smem;
 
@@ -370,8 +384,8 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_bwd_dkv_kernel(const AttnBwd
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, hh = lane >> 5;
     const int nid = renumber_block();
-    const int bh = (int)fastdiv((uint32_t)nid, a.div_qtiles);
-    const int kt = nid - bh * a.qtiles;
+    const int bh = (int)fastdiv((uint32_t)nid, a.div_ktiles);
+    const int kt = nid - bh * a.ktiles;
     const int N = a.N, nw = (N + 31) >> 5;
     const int T = (N + BN - 1) / BN;
     const bool ragged = (N & (BN - 1)) != 0;
@@ -385,45 +399,54 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_bwd_dkv_kernel(const AttnBwd
     const float *lse_b = a.lse + (size_t)bh * N, *delta_b = a.delta + (size_t)bh * N;
 
     // ---- this lane's key: K^T (scaled) and V^T fragments, B operands ----
-    const int key0 = kt * BM + wave * 32;
+    const int key0 = kt * (32 * NW) + wave * 32;
     const bool wave_valid = key0 < N;                 // wave-uniform: some key of this wave exists
     const int key = key0 + l32;
     const int kr = key < N ? key : N - 1;
     const uint32_t key_ok = key < N ? 0xffffffffu : 0u;
     const uint32_t key_w = key < N ? 1u : 0u;         // width of the bit field that holds this key's mask bit
     const int wi = (key0 >> 5) < nw ? (key0 >> 5) : nw - 1;     // this wave's mask word of a row
-    u32x4 kf[KS], vf[DK ? KS : 1];
-    load_row(kf, kb, a.k.sn, kr, hh, a.D);
-    if constexpr (DK) load_row(vf, vb, a.v.sn, kr, hh, a.D);
+    const uint32_t frag = lds0 + C::OFF_FRAG + wave * C::FRAG + lane * 16;
+    u32x4 kf[KS], vf[VLDS ? 1 : KS];
+    {
+        u32x4 v_all[KS];
+        load_row(kf, kb, a.k.sn, kr, hh, a.D);
+        load_row(v_all, vb, a.v.sn, kr, hh, a.D);
 #pragma unroll
-    for (int s = 0; s < KS; ++s)
+        for (int s = 0; s < KS; ++s) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float lo = E::up1((uint16_t)(kf[s][i] & 0xffffu)) * a.q_scale;
-            const float hi = E::up1((uint16_t)(kf[s][i] >> 16)) * a.q_scale;
-            kf[s][i] = (uint32_t)E::cvt1(lo) | ((uint32_t)E::cvt1(hi) << 16);
+            for (int i = 0; i < 4; ++i) {
+                const float lo = E::up1((uint16_t)(kf[s][i] & 0xffffu)) * a.q_scale;
+                const float hi = E::up1((uint16_t)(kf[s][i] >> 16)) * a.q_scale;
+                kf[s][i] = (uint32_t)E::cvt1(lo) | ((uint32_t)E::cvt1(hi) << 16);
+            }
+            if constexpr (VLDS) *(LDS_PTR(u32x4))(uintptr_t)(frag + s * 1024) = v_all[s];
+            else vf[VLDS ? 0 : s] = v_all[s];
         }
+    }
 
     // ---- copies: Q tile, dO tile; per wave its mask word of the 64 rows; lse (wave 0), delta (wave 1)
-    const TileCopy tc = make_tile_copy(wave, lane, (a.D >> 3) - 1);
+    // (eight wavefronts: the first four copy Q, the others dO)
+    const int cw = wave & 3;
+    const TileCopy tc = make_tile_copy(cw, lane, (a.D >> 3) - 1);
     const TileRead tr = make_tile_read(lane);
     auto issue = [&](int t, int st) {
         const int r0 = t * BN;
         const int row = r0 + lane < N ? r0 + lane : N - 1;
         const uint32_t aux = lds0 + OFF_AUX + st * AUX_BYTES;
         async_copy_b32(aux + wave * 256, mb + wi, (uint32_t)((size_t)row * nw * 4));
-        if (wave == 0) async_copy_b32(aux + 1024, lse_b, (uint32_t)(row * 4));
-        if (wave == 1) async_copy_b32(aux + 1280, delta_b, (uint32_t)(row * 4));
-        issue_tile<NH>(lds0 + st * STAGE_BYTES, qb, a.q.sn, r0, N, tc, wave);
-        issue_tile<NH>(lds0 + st * STAGE_BYTES + C::OFF_B, dob, a.dout.sn, r0, N, tc, wave);
+        if (wave == 0) async_copy_b32(aux + OFF_LSE, lse_b, (uint32_t)(row * 4));
+        if (wave == 1) async_copy_b32(aux + OFF_DELTA, delta_b, (uint32_t)(row * 4));
+        if (NW == 4 || wave < 4) issue_tile<NH>(lds0 + st * STAGE_BYTES, qb, a.q.sn, r0, N, tc, cw);
+        if (NW == 4 || wave >= 4) issue_tile<NH>(lds0 + st * STAGE_BYTES + C::OFF_B, dob, a.dout.sn, r0, N, tc, cw);
     };
     // With a tile map only the blocks of 64 query rows in which the mask keeps something for this
-    // work-group's 128 keys (its two key tiles 2kt, 2kt+1: neighbouring bits of one word of the
-    // row block's "live" bits) are visited: lane r of a wavefront looks at row block 64c + r, a
+    // work-group's keys (NW / 2 key tiles: neighbouring bits of one word of the row block's "live"
+    // bits) are visited: lane r of a wavefront looks at row block 64c + r, a
     // ballot turns the 64 answers into the bits that are walked.  Every wavefront does the same.
     const int TW = (T + 31) >> 5;
     const uint32_t *mapc = a.tile_map != nullptr
-        ? a.tile_map + bi * a.map_sb + hi * a.map_sh + ((2 * kt) >> 5) : nullptr;
+        ? a.tile_map + bi * a.map_sb + hi * a.map_sh + ((NW / 2 * kt) >> 5) : nullptr;
     int cur_c = -1;
     unsigned long long live_c = 0ull;
     auto next_tile = [&]() __attribute__((always_inline)) -> int {     // next live row block, T if there is none
@@ -431,7 +454,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_bwd_dkv_kernel(const AttnBwd
             if (64 * ++cur_c >= T) return T;
             const int r = 64 * cur_c + lane;
             bool lv = r < T;
-            if (mapc != nullptr && lv) lv = ((mapc[(size_t)r * 2 * TW] >> ((2 * kt) & 31)) & 3u) != 0u;
+            if (mapc != nullptr && lv) lv = ((mapc[(size_t)r * 2 * TW] >> ((NW / 2 * kt) & 31)) & ((1u << (NW / 2)) - 1u)) != 0u;
             live_c = __builtin_amdgcn_ballot_w64(lv);
         }
         const int b = __builtin_ctzll(live_c);
@@ -441,37 +464,44 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_bwd_dkv_kernel(const AttnBwd
     const int t_first = next_tile();
     if (t_first < T) issue(t_first, 0);
 
-    f32x16 dkacc[DK ? OB : 1], dvacc[DV ? OB : 1];      // [2 * half + dblk]: 32 columns each
+    f32x16 dkacc[OB], dvacc[OB];      // [2 * half + dblk]: 32 columns each
 #pragma unroll
     for (int b = 0; b < OB; ++b)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            if constexpr (DK) dkacc[b][i] = 0.f;
-            if constexpr (DV) dvacc[b][i] = 0.f;
+            dkacc[b][i] = 0.f;
+            dvacc[b][i] = 0.f;
         }
+
+    // bases of this lane's reads of the small data; opaque, because beyond 64 KiB the compiler would otherwise
+    // keep a register for every sum of base and offset (40 of them) instead of using the offset field
+    uint32_t aux_rows = lds0 + OFF_AUX + 16 * hh, aux_words = aux_rows + wave * 256, aux_lane = lds0 + OFF_AUX + 4 * lane;
+    if constexpr (OFF_AUX >= 65536) asm volatile("" : "+v"(aux_rows), "+v"(aux_words), "+v"(aux_lane));
 
     // one q tile; the ring stage is a compile-time constant so that every LDS address of the body is
     // a register plus an immediate
     auto tile = [&](int t, int t_next, auto st_c) __attribute__((always_inline)) {
         constexpr int st = decltype(st_c)::value;
         const uint32_t so = lds0 + st * STAGE_BYTES;
-        const uint32_t aux = lds0 + OFF_AUX + st * AUX_BYTES;
         WAIT_VMCNT(0);
         if (wave == 0) {
             // lse of the tile's rows -> what the score accumulators start from, -lse * log2(e) / pm, so
             // that exp2(pm * accumulator) is the probability; rows that kept nothing or lie beyond N
             // -> -inf (probability 0)
-            const uint32_t p = aux + 1024 + lane * 4;
+            const uint32_t p = aux_lane + st * AUX_BYTES + OFF_LSE;
             const float l = *(LDS_PTR(float))(uintptr_t)p;
             const bool dead = (t * BN + lane >= N) || (l == -__builtin_inff());
             *(LDS_PTR(float))(uintptr_t)p = dead ? -__builtin_inff() : l * lse_mul;
         }
         if (wave == 1) {
             // -delta: the dP accumulators start from it
-            const uint32_t p = aux + 1280 + lane * 4;
+            const uint32_t p = aux_lane + st * AUX_BYTES + OFF_DELTA;
             *(LDS_PTR(float))(uintptr_t)p = -*(LDS_PTR(float))(uintptr_t)p;
         }
-        if (ragged && t == T - 1) zero_tile_tail(so, 2 * NH, t * BN, N, tc, wave, lane);
+        if (ragged && t == T - 1) {
+            if (NW == 4) zero_tile_tail(so, 2 * NH, t * BN, N, tc, cw, lane);
+            else zero_tile_tail(so + (wave >> 2) * C::OFF_B, NH, t * BN, N, tc, cw, lane);
+        }
         __syncthreads();
         if (t_next < T) issue(t_next, st ^ 1);
         if (!wave_valid) return;
@@ -479,12 +509,12 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_bwd_dkv_kernel(const AttnBwd
 #pragma unroll
         for (int blk = 0; blk < 2; ++blk) {
             // element 4g+j of an accumulator <-> query row 32blk + 8g + 4hh + j of the tile
-            const uint32_t rsel = (uint32_t)((32 * blk + 4 * hh) * 4);
+            auto mask_words = [&](int g) __attribute__((always_inline)) { return lds_read_b128(aux_words + st * AUX_BYTES + 128 * blk + 32 * g); };
             u32x4 mw[4];
             uint32_t any = 0u;
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                mw[g] = lds_read_b128(aux + wave * 256 + rsel + 32 * g);
+                mw[g] = mask_words(g);
                 any |= mw[g].x | mw[g].y | mw[g].z | mw[g].w;
             }
             if (__builtin_amdgcn_ballot_w64((((any >> l32) & 1u) & key_ok) != 0u) == 0ull) continue;
@@ -494,9 +524,8 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_bwd_dkv_kernel(const AttnBwd
             f32x16 sacc, dacc;
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const u32x4 Lr = lds_read_b128(aux + 1024 + rsel + 32 * g);
-                u32x4 Dr = {0u, 0u, 0u, 0u};
-                if constexpr (DK) Dr = lds_read_b128(aux + 1280 + rsel + 32 * g);
+                const u32x4 Lr = lds_read_b128(aux_rows + st * AUX_BYTES + OFF_LSE + 128 * blk + 32 * g);
+                const u32x4 Dr = lds_read_b128(aux_rows + st * AUX_BYTES + OFF_DELTA + 128 * blk + 32 * g);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     sacc[4 * g + j] = __builtin_bit_cast(float, (uint32_t)Lr[j]);
@@ -506,33 +535,30 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_bwd_dkv_kernel(const AttnBwd
 #pragma unroll
             for (int s = 0; s < KS; ++s)
                 sacc = E::mfma(lds_read_b128(tr.rowaddr[s & 3] + so + (s >> 2) * TILE_BYTES + 4096 * blk), kf[s], sacc);
-            if constexpr (DK) {
 #pragma unroll
-                for (int s = 0; s < KS; ++s)
-                    dacc = E::mfma(lds_read_b128(tr.rowaddr[s & 3] + so + C::OFF_B + (s >> 2) * TILE_BYTES + 4096 * blk),
-                                   vf[s], dacc);
+            for (int s = 0; s < KS; ++s) {
+                const u32x4 vs = VLDS ? lds_read_b128(frag + s * 1024) : vf[VLDS ? 0 : s];
+                dacc = E::mfma(lds_read_b128(tr.rowaddr[s & 3] + so + C::OFF_B + (s >> 2) * TILE_BYTES + 4096 * blk), vs, dacc);
             }
 
-            uint32_t pp[2][4] = {}, ps[2][4] = {};       // the one a single-gradient instance leaves unused is dropped
+            if constexpr (VLDS) asm volatile("" ::: "memory");      // the words are read once more, not kept
+            uint32_t pp[2][4], ps[2][4];
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 float p[4], d[4];
+                const u32x4 mg = VLDS ? mask_words(g) : mw[g];
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const uint32_t keep = (uint32_t)__builtin_amdgcn_sbfe((int)mw[g][j], (uint32_t)l32, key_w);
+                    const uint32_t keep = (uint32_t)__builtin_amdgcn_sbfe((int)mg[j], (uint32_t)l32, key_w);
                     const float e = __builtin_amdgcn_exp2f(POSTMUL ? sacc[4 * g + j] * pm : sacc[4 * g + j]);
                     p[j] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, e) & keep);
                     d[j] = p[j] * dacc[4 * g + j];
                 }
                 // elements 4g .. 4g+3 are pairs (2i, 2i+1) with i = 2(g & 1), 2(g & 1) + 1 of u = g >> 1
-                if constexpr (DV) {
-                    pp[g >> 1][2 * (g & 1)] = E::pack2_rne(p[0], p[1]);
-                    pp[g >> 1][2 * (g & 1) + 1] = E::pack2_rne(p[2], p[3]);
-                }
-                if constexpr (DK) {
-                    ps[g >> 1][2 * (g & 1)] = E::pack2_rne(d[0], d[1]);
-                    ps[g >> 1][2 * (g & 1) + 1] = E::pack2_rne(d[2], d[3]);
-                }
+                pp[g >> 1][2 * (g & 1)] = E::pack2_rne(p[0], p[1]);
+                pp[g >> 1][2 * (g & 1) + 1] = E::pack2_rne(p[2], p[3]);
+                ps[g >> 1][2 * (g & 1)] = E::pack2_rne(d[0], d[1]);
+                ps[g >> 1][2 * (g & 1) + 1] = E::pack2_rne(d[2], d[3]);
             }
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
@@ -542,18 +568,14 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_bwd_dkv_kernel(const AttnBwd
 #pragma unroll
                 for (int b = 0; b < OB; ++b) {
                     const uint32_t ho = off + (b >> 1) * TILE_BYTES;
-                    if constexpr (DK) {                              // dK^T += Q^T dS
-                        const u32x2 qlo = lds_read_tr16_b64(tr.traddr[b & 1][0] + ho);
-                        const u32x2 qhi = lds_read_tr16_b64(tr.traddr[b & 1][1] + ho);
-                        const u32x4 qa = {qlo.x, qlo.y, qhi.x, qhi.y};
-                        dkacc[b] = E::mfma(qa, bs, dkacc[b]);
-                    }
-                    if constexpr (DV) {                              // dV^T += dO^T P
-                        const u32x2 dlo = lds_read_tr16_b64(tr.traddr[b & 1][0] + ho + C::OFF_B);
-                        const u32x2 dhi = lds_read_tr16_b64(tr.traddr[b & 1][1] + ho + C::OFF_B);
-                        const u32x4 da = {dlo.x, dlo.y, dhi.x, dhi.y};
-                        dvacc[b] = E::mfma(da, bp, dvacc[b]);
-                    }
+                    const u32x2 qlo = lds_read_tr16_b64(tr.traddr[b & 1][0] + ho);          // dK^T += Q^T dS
+                    const u32x2 qhi = lds_read_tr16_b64(tr.traddr[b & 1][1] + ho);
+                    const u32x4 qa = {qlo.x, qlo.y, qhi.x, qhi.y};
+                    dkacc[b] = E::mfma(qa, bs, dkacc[b]);
+                    const u32x2 dlo = lds_read_tr16_b64(tr.traddr[b & 1][0] + ho + C::OFF_B);       // dV^T += dO^T P
+                    const u32x2 dhi = lds_read_tr16_b64(tr.traddr[b & 1][1] + ho + C::OFF_B);
+                    const u32x4 da = {dlo.x, dlo.y, dhi.x, dhi.y};
+                    dvacc[b] = E::mfma(da, bp, dvacc[b]);
                 }
             }
         }
@@ -568,33 +590,44 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_bwd_dkv_kernel(const AttnBwd
     WAIT_VMCNT(0);
     __syncthreads();
     if (wave_valid) {
-        if constexpr (DK) store_gradient<BF16, WIDE>(dkacc, a.scale, lds0 + wave * 4096, a, a.dk, bi, hi, key0, lane);
-        if constexpr (DV) store_gradient<BF16, WIDE>(dvacc, 1.0f, lds0 + wave * 4096, a, a.dv, bi, hi, key0, lane);
+        store_gradient<BF16, WIDE>(dkacc, a.scale, lds0 + wave * 4096, a, a.dk, bi, hi, key0, lane);
+        store_gradient<BF16, WIDE>(dvacc, 1.0f, lds0 + wave * 4096, a, a.dv, bi, hi, key0, lane);
     }
 }
 
 template <bool BF16, int HDIM, bool POSTMUL, bool WIDE>
-void launch_pair(dim3 grid, dim3 block, hipStream_t stream, const AttnBwdArgs &a)
+void launch_pair(hipStream_t stream, const AttnBwdArgs &args)
 {
+    AttnBwdArgs a = args;
     // dQ first: it also fills the delta workspace that the dK/dV kernel reads (same stream)
-    hipLaunchKernelGGL((attn_bwd_dq_kernel<BF16, HDIM, WIDE>), grid, block, 0, stream, a);
-    if constexpr (HDIM == 128) {
-        hipLaunchKernelGGL((attn_bwd_dkv_kernel<BF16, HDIM, true, false, POSTMUL, WIDE>), grid, block, 0, stream, a);
-        hipLaunchKernelGGL((attn_bwd_dkv_kernel<BF16, HDIM, false, true, POSTMUL, WIDE>), grid, block, 0, stream, a);
-    } else {
-        hipLaunchKernelGGL((attn_bwd_dkv_kernel<BF16, HDIM, true, true, POSTMUL, WIDE>), grid, block, 0, stream, a);
-    }
+    hipLaunchKernelGGL((attn_bwd_dq_kernel<BF16, HDIM, WIDE>), dim3((unsigned)(a.BH * a.qtiles)), dim3(NTHREADS), 0, stream, a);
+    auto dkv = [&](auto nw_c) {
+        constexpr int NW = decltype(nw_c)::value;
+        a.ktiles = (a.N + 32 * NW - 1) / (32 * NW);
+        a.div_ktiles = make_fastdiv((uint32_t)a.ktiles);
+        hipLaunchKernelGGL((attn_bwd_dkv_kernel<BF16, HDIM, NW, POSTMUL, WIDE>), dim3((unsigned)(a.BH * a.ktiles)), dim3(64 * NW), 0,
+                           stream, a);
+    };
+    // Head dim 128: eight wavefronts read Q and dO once per 256 keys and keep two of themselves on a SIMD, four
+    // leave a CU to one work-group; but a grid that four-wavefront work-groups do not fill takes them (1 x 8 heads,
+    // N = 1024: 74 against 87 us), and so do short keys of which 256 at a time would leave a sixth or more idle.
+    // Elsewhere eight win: 16 x 12, N = 1024: 373 against 431 us.
+    const long long groups = (long long)a.BH * a.qtiles;
+    if (HDIM == 128 && groups > compute_units() && (a.qtiles % 2 == 0 || a.qtiles >= 5))
+        dkv(std::integral_constant<int, HDIM == 128 ? 8 : 4>{});
+    else
+        dkv(std::integral_constant<int, 4>{});
 }
 template <int HDIM>
-void launch_head_dim(bool bf16, dim3 grid, dim3 block, hipStream_t stream, const AttnBwdArgs &a)
+void launch_head_dim(bool bf16, hipStream_t stream, const AttnBwdArgs &a)
 {
     const bool postmul = a.post_mul != 1.0f;       // exp2(pm * s) needs its multiplication only then
     if (a.grads_f32)                               // fp32 callers compute in bf16
-        postmul ? launch_pair<true, HDIM, true, true>(grid, block, stream, a) : launch_pair<true, HDIM, false, true>(grid, block, stream, a);
+        postmul ? launch_pair<true, HDIM, true, true>(stream, a) : launch_pair<true, HDIM, false, true>(stream, a);
     else if (bf16)
-        postmul ? launch_pair<true, HDIM, true, false>(grid, block, stream, a) : launch_pair<true, HDIM, false, false>(grid, block, stream, a);
+        postmul ? launch_pair<true, HDIM, true, false>(stream, a) : launch_pair<true, HDIM, false, false>(stream, a);
     else
-        postmul ? launch_pair<false, HDIM, true, false>(grid, block, stream, a) : launch_pair<false, HDIM, false, false>(grid, block, stream, a);
+        postmul ? launch_pair<false, HDIM, true, false>(stream, a) : launch_pair<false, HDIM, false, false>(stream, a);
 }
 
 }  // namespace
@@ -604,15 +637,13 @@ hipError_t launch_attn_bwd(const AttnBwdArgs &args, bool bf16, hipStream_t strea
     AttnBwdArgs a = args;
     a.div_qtiles = make_fastdiv((uint32_t)a.qtiles);
     a.div_H = make_fastdiv((uint32_t)a.H);
-    const long long groups = (long long)a.BH * a.qtiles;
-    if (groups == 0) return hipSuccess;
+    if ((long long)a.BH * a.qtiles == 0) return hipSuccess;
     if (a.grads_f32 && !bf16) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)groups), block(NTHREADS);
     switch (kernel_head_dim(a.D)) {
-    case 128: launch_head_dim<128>(bf16, grid, block, stream, a); break;
-    case 96: launch_head_dim<96>(bf16, grid, block, stream, a); break;
-    case 64: launch_head_dim<64>(bf16, grid, block, stream, a); break;
-    default: launch_head_dim<32>(bf16, grid, block, stream, a); break;
+    case 128: launch_head_dim<128>(bf16, stream, a); break;
+    case 96: launch_head_dim<96>(bf16, stream, a); break;
+    case 64: launch_head_dim<64>(bf16, stream, a); break;
+    default: launch_head_dim<32>(bf16, stream, a); break;
     }
     return hipGetLastError();
 }

@@ -885,7 +885,7 @@ FwdKernel fwd_kernel_96(int variant, int mask_kind);
 FwdKernel fwd_kernel_128(int variant, int mask_kind);
 
 // Number of compute units of the current device (cached per device ordinal).
-static int compute_units()
+int compute_units()
 {
     static std::atomic<int> cached[64];      // 0 = not asked yet; threads may race to store the same value
     int dev = 0;

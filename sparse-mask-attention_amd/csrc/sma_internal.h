@@ -86,7 +86,8 @@ struct AttnBwdArgs {
     int BH, H, N;
     int D;                                     // head dim: a multiple of 8 up to 128
     int qtiles;                                // ceil(N / 128)
-    FastDiv div_qtiles, div_H;                 // filled in by the launcher
+    int ktiles;                                // key tiles (work-groups of the dK/dV kernel) per (b,h) ...
+    FastDiv div_qtiles, div_ktiles, div_H;     // ... and these: filled in by the launcher
     float scale;                               // as given by the caller
     float q_scale, post_mul;                   // as in AttnArgs
     uint32_t last_mask0, last_mask1;
@@ -96,6 +97,9 @@ struct AttnBwdArgs {
 // one: the copies fill an LDS row beyond the tensor's with its last 16 bytes once more, the fragments that the
 // wavefronts hold in registers are zero there, and results beyond it are not stored.
 inline int kernel_head_dim(int D) { return D <= 32 ? 32 : D <= 64 ? 64 : D <= 96 ? 96 : 128; }
+
+// Number of compute units of the current device (asked for once).
+int compute_units();
 
 hipError_t launch_attn_fwd(const AttnArgs &a, bool bf16, hipStream_t stream);
 hipError_t launch_attn_bwd(const AttnBwdArgs &a, bool bf16, hipStream_t stream);
