@@ -76,8 +76,8 @@ constexpr float SUM_LIMIT = 16384.0f;     // a lane's 32 weights of a tile sum t
 // into the two words per row itself (eight dot products with the weights 1, 2, 4 .. 128 per lane
 // and one exchange between the lane halves): the separate packing pass, its launch and the
 // round trip of the words through memory disappear for a mask that is used once.
-template <int NH, bool BYTEMASK> struct Cfg {
-    static constexpr int NSTAGE = 2;                                // ring of two stages: copies run one tile ahead
+template <int NH, bool BYTEMASK, bool SPLIT> struct Cfg {
+    static constexpr int NSTAGE = SPLIT ? 4 : 2; // SPLIT: one K and one V buffer for each of the four wavefronts, else                               // ring of two stages: copies run one tile ahead
     static constexpr int MASK_COPIES = BYTEMASK ? 2 : 1;
     static constexpr int COPIES = MASK_COPIES + 4 * NH;             // async copies per wave and tile
     // LDS map (bytes)
@@ -89,15 +89,16 @@ template <int NH, bool BYTEMASK> struct Cfg {
     // enough, at the price of waiting for those reads before the requests (3 % on the headline
     // workload, which is why two are used where they fit)
     static constexpr int OFF_MASK = NSTAGE * STAGE_BYTES;
-    static constexpr int BYTE_SLOTS = NH == 1 ? 2 : 1;
+    static constexpr int BYTE_SLOTS = NH == 1 && !SPLIT ? 2 : 1;
     static constexpr int MASK_SLOT = BYTEMASK ? (BYTE_SLOTS - 1) * 8192 : 1024;     // distance between the slots
-    static constexpr int OFF_LUT = OFF_MASK + (BYTEMASK ? BYTE_SLOTS * 8192 : NSTAGE * 1024);   // 16 x 16 B
+    static constexpr int OFF_LUT = OFF_MASK + (BYTEMASK ? BYTE_SLOTS * 8192 : SPLIT ? 1024 : NSTAGE * 1024);   // 16 x 16 B
     // byte mask only: the tile-map bits the wavefronts collect, [4 waves][MAP_WORDS][some, hole],
     // and one arrival counter per pair of wavefronts (block of 64 rows)
     static constexpr int MAP_WORDS = 32;                            // 32 x 32 key tiles: N <= 65536
+    // (SPLIT writes them to memory at once)
     static constexpr int OFF_MAP = OFF_LUT + 256;
     static constexpr int OFF_MAP_ARRIVED = OFF_MAP + 4 * MAP_WORDS * 8;
-    static constexpr int LDS_BYTES = BYTEMASK ? OFF_MAP_ARRIVED + 16 : OFF_MAP;
+    static constexpr int LDS_BYTES = BYTEMASK && !SPLIT ? OFF_MAP_ARRIVED + 16 : OFF_MAP;
 };
 
 template <int N> __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory"); }
@@ -116,18 +117,25 @@ template <int N> __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_
 // step (the even-progress case of the launcher, e.g. the headline shape): there the first visit,
 // which waits for twice the bytes, is not hidden behind other work-groups' work, it measured 1 to 4 %
 // slower, and the launcher leaves it off.
+// SPLIT: for grids that leave most of the chip idle.  The four wavefronts of a work-group share 32 query
+// rows and take every fourth key tile each, with a K and a V buffer of their own: no barriers, four times
+// the work-groups, a quarter of the serial chain; what they found is combined through LDS at the end.
+// K of the next tile is requested when the scores of this one are formed, V when its products are.
+// Measured, D = 64, packed mask: 1 x 4 heads, N = 4096: 55 -> 31 us, 1 x 1: 55 -> 23 us; 2 x 8, N = 1024: 16.6
+// -> 11.1 us; 4 x 8, N = 512: 10.1 -> 7.9 us.  A wavefront now copies 16 KB per tile instead of 4, and a tile takes
+// 1.4 times as long.
 template <bool BF16, bool POSTMUL, bool PACKED_ROWS, int HDIM, bool BYTEMASK = false, bool BYPRODUCTS = false,
-          bool PAIRS = false>
-__global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(const AttnArgs a)
+          bool PAIRS = false, bool SPLIT = false>
+__global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ? 2 : 3) void attn_fwd_kernel(const AttnArgs a)
 {
-    static_assert(!PAIRS || (BYTEMASK && HDIM <= 64), "PAIRS: byte mask, two byte slots");
+    static_assert(!PAIRS || (BYTEMASK && HDIM <= 64 && !SPLIT), "PAIRS: byte mask, two byte slots");
     using E = Elem<BF16>;
     constexpr int NH = HDIM > 64 ? 2 : 1;         // 64-column tiles per matrix
     constexpr int KS = HDIM / 16;                 // MFMA steps of the QK^T chain
     constexpr int OB = HDIM / 32;                 // 32-column accumulator blocks of O
     // second column half at a constant distance from the first in every row
     constexpr bool SAME_HALVES = HDIM == 128 && PACKED_ROWS;
-    using C = Cfg<NH, BYTEMASK>;
+    using C = Cfg<NH, BYTEMASK, SPLIT>;
     constexpr int NSTAGE = C::NSTAGE, STAGE_BYTES = C::STAGE_BYTES, OFF_MASK = C::OFF_MASK, OFF_LUT = C::OFF_LUT;
     constexpr int MASK_SLOT = C::MASK_SLOT;
     const int D = PACKED_ROWS ? HDIM : a.D;
@@ -145,6 +153,7 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
     // last rows first: where rows keep more keys the later they come (causal masks), the longest
     // work-groups of a head start first and the shortest fill the end of the launch
     const int qt = a.qtiles - 1 - (nid - bh * a.qtiles);
+    const int row_base = SPLIT ? qt * 32 : qt * BM + wave * 32;          // this wavefront's 32 query rows
     const int N = a.N, nw = (N + 31) >> 5;
     const int T = (N + BN - 1) / BN;
     const bool ragged = (N & (BN - 1)) != 0;
@@ -160,8 +169,8 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
     const uint32_t *mapw = nullptr, *mapw2 = nullptr;       // the two 64-row blocks (the same one if the second does not exist)
     if constexpr (!BYTEMASK) {
         if (a.tile_map != nullptr) {
-            mapw = a.tile_map + bi * a.map_sb + hi * a.map_sh + (size_t)(2 * qt) * 2 * TW;
-            mapw2 = (2 * qt + 1 < T) ? mapw + 2 * TW : mapw;
+            mapw = a.tile_map + bi * a.map_sb + hi * a.map_sh + (size_t)(SPLIT ? qt >> 1 : 2 * qt) * 2 * TW;
+            mapw2 = (!SPLIT && 2 * qt + 1 < T) ? mapw + 2 * TW : mapw;
         }
     }
     // The first map words are read here, with ordinary (scalar) loads, long before they are needed:
@@ -193,14 +202,14 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
     // every chunk that would reach beyond the row's end is read from the 16 bytes before that end
     // instead, so that nothing after the mask's last byte is touched; the bits of the chunk that
     // holds the end are shifted to their places below, those of later chunks cleared as pad bits.
-    const int mrow = BYTEMASK ? 0 : qt * BM + wave * 32 + (lane >> 1);
+    const int mrow = BYTEMASK ? 0 : row_base + (lane >> 1);
     const uint32_t m_voff = BYTEMASK ? 0u : (uint32_t)(((size_t)(mrow < N ? mrow : N - 1) * nw + (lane & 1)) * 4);
     uint32_t mb_voff[2] = {0u, 0u}, mb_chunk[2] = {0u, 0u};
     if constexpr (BYTEMASK) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const int row = 16 * j + (lane >> 2);
-            const int grow = qt * BM + wave * 32 + row;
+            const int grow = row_base + row;
             mb_chunk[j] = (uint32_t)(((lane & 3) ^ ((row >> 2) & 3)) << 4);
             mb_voff[j] = (uint32_t)(grow < N ? grow : N - 1) * (uint32_t)N + mb_chunk[j];
         }
@@ -241,7 +250,7 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
     uint32_t pair_voff = 0u;
     if constexpr (PAIRS) {
         const int row = lane >> 3;
-        pair_voff = (uint32_t)(qt * BM + wave * 32 + row) * (uint32_t)N + (uint32_t)(((lane & 7) ^ (row >> 1)) << 4);
+        pair_voff = (uint32_t)(row_base + row) * (uint32_t)N + (uint32_t)(((lane & 7) ^ (row >> 1)) << 4);
     }
     auto issue_mask_pair = [&](int p) __attribute__((always_inline)) {      // bytes of tiles 2p and 2p + 1
         const uint8_t *src = reinterpret_cast<const uint8_t *>(mb) + (size_t)p * (2 * BN);
@@ -253,7 +262,7 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
     };
     // BYTEMASK: where this lane's row of packed words goes, if the caller wants them ([Bm, Hm, N, nw]
     // like the mask; a mask shared between batch entries / heads is written by the first of them)
-    const int qrow = qt * BM + wave * 32 + l32;
+    const int qrow = row_base + l32;
     uint32_t *words_out = nullptr;
     // ... and where the tile map of this work-group's two blocks of 64 rows goes ([Bm, Hm, T, 2, TW]).
     // Each wavefront notes per key tile whether its 32 rows hold a set bit and whether they hold a
@@ -270,10 +279,10 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
         const int Hm = a.mask.sh != 0 ? a.H : 1;
         const size_t slab_m = (size_t)((a.mask.sb != 0 ? bi : 0) * Hm + (a.mask.sh != 0 ? hi : 0));
         if (a.mask_out != nullptr && writer) words_out = a.mask_out + (slab_m * N + (qrow < N ? qrow : 0)) * nw;
-        if (a.map_out != nullptr && writer) map_dst = a.map_out + (slab_m * T + 2 * qt) * 2 * TW;
+        if (a.map_out != nullptr && writer) map_dst = a.map_out + (slab_m * T + (SPLIT ? qt >> 1 : 2 * qt)) * 2 * TW;
     }
     const uint32_t map_lds = lds0 + C::OFF_MAP + wave * (C::MAP_WORDS * 8);
-    if constexpr (BYPRODUCTS) {     // ordered before any arrival by the barriers of the main loop (T >= 1)
+    if constexpr (BYPRODUCTS && !SPLIT) {     // ordered before any arrival by the barriers of the main loop (T >= 1)
         if (tid < 2) *(LDS_PTR(uint32_t))(uintptr_t)(lds0 + C::OFF_MAP_ARRIVED + 4 * tid) = 0u;
     }
     const uint32_t maddr = BYTEMASK ? lds0 + OFF_MASK + wave * 2048 + l32 * 64 : lds0 + OFF_MASK + wave * 256 + l32 * 8;
@@ -336,9 +345,18 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
                 const uint32_t valid = x == T - 1 ? (hh ? a.last_mask1 : a.last_mask0) : 0xffffffffu;
                 const uint32_t some = __builtin_amdgcn_ballot_w64(mine != 0u) != 0ull ? 1u : 0u;
                 const uint32_t hole = __builtin_amdgcn_ballot_w64(mine != valid) != 0ull ? 1u : 0u;
+                if constexpr (SPLIT) {
+                    // the block's other 32 rows belong to another work-group: into the words at once, which were
+                    // set to "nothing kept" and "everything kept" before the launch
+                    if (lane == 0) {
+                        if (some) atomicOr(map_dst + (x >> 5), 1u << (x & 31));
+                        if (hole) atomicAnd(map_dst + TW + (x >> 5), ~(1u << (x & 31)));
+                    }
+                }
                 some_acc |= some << (x & 31);
                 hole_acc |= hole << (x & 31);
-                if ((x & 31) == 31 || x == T - 1) {
+                if (SPLIT) {
+                } else if ((x & 31) == 31 || x == T - 1) {
                     if (lane == 0) *(LDS_PTR(u32x2))(uintptr_t)(map_lds + (uint32_t)(x >> 5) * 8) = u32x2{some_acc, hole_acc};
                     some_acc = hole_acc = 0u;
                 }
@@ -352,7 +370,11 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
             // the lower lane half keeps the words of tiles 4g and 4g + 1, the upper half those of
             // tiles 4g + 2 and 4g + 3, and after every fourth tile each lane stores 16 bytes: 32
             // consecutive bytes of each row per store instruction.
-            if (BYPRODUCTS && words_out != nullptr) {
+            if (SPLIT && BYPRODUCTS && words_out != nullptr && qrow < N && hh == 0) {
+                words_out[2 * x] = w.x;
+                if (2 * x + 1 < nw) words_out[2 * x + 1] = w.y;
+            }
+            if (!SPLIT && BYPRODUCTS && words_out != nullptr) {
                 const int j = x & 3;
                 const bool turn = hh == (j >> 1);
                 if ((j & 1) == 0) {
@@ -394,7 +416,7 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
     uint32_t kv_voff[2][2], kv_voff2[2][2];       // first and second column half
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-        const int row = 8 * (2 * wave + j) + (lane >> 3);
+        const int row = 8 * (SPLIT ? j : 2 * wave + j) + (lane >> 3);       // SPLIT: the wave copies rows 16i + these too
         const int pos = lane & 7;
         const int f = (row >> 1) & 7;
         const int fr = bitrev3(f);
@@ -443,6 +465,50 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
             async_copy_b128_at<SO + C::OFF_V + TILE_BYTES + 1024>(kv_dst, vsrc, vo2[1]);
         }
     };
+    // SPLIT: all 64 rows of one matrix by one wavefront, 16 rows (two copies) at a time; the swizzles repeat
+    // every 16 rows
+    const uint32_t split_dst = lds0 + wave * STAGE_BYTES;
+    auto issue_own = [&](int t, const uint16_t *mat, uint32_t sn, uint32_t rb, const uint32_t (&off)[2], const uint32_t (&off2)[2],
+                         auto at_c) __attribute__((always_inline)) {
+        constexpr int AT = decltype(at_c)::value;
+        const int key0 = t * BN;
+        const uint16_t *src = mat + (size_t)key0 * sn;
+        const bool cut = ragged && t == T - 1;
+        auto group = [&](auto i_c) __attribute__((always_inline)) {
+            constexpr int I = decltype(i_c)::value;
+            uint32_t o[2] = {off[0], off[1]}, o2[2] = {off2[0], off2[1]};
+            if (cut) {                        // rows beyond N: copy row N-1 instead (zeroed later)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const int r = 8 * j + (lane >> 3), over = key0 + 16 * I + r - (N - 1);
+                    // what goes down by more than the lane's own rows is taken from the base's below
+                    const uint32_t up = over > 0 ? __umul24(over, rb) : 0u;
+                    o[j] += __umul24(16 * I, rb) - up;
+                    o2[j] += __umul24(16 * I, rb) - up;
+                }
+            }
+            const uint16_t *p = cut ? src : src + (size_t)(16 * I) * sn;
+            async_copy_b128_at<AT + 2048 * I>(split_dst, p, o[0]);
+            async_copy_b128_at<AT + 2048 * I + 1024>(split_dst, p, o[1]);
+            if constexpr (NH == 2) {
+                async_copy_b128_at<AT + TILE_BYTES + 2048 * I>(split_dst, p, o2[0]);
+                async_copy_b128_at<AT + TILE_BYTES + 2048 * I + 1024>(split_dst, p, o2[1]);
+            }
+        };
+        group(std::integral_constant<int, 0>{});
+        group(std::integral_constant<int, 1>{});
+        group(std::integral_constant<int, 2>{});
+        group(std::integral_constant<int, 3>{});
+    };
+    auto issue_own_k = [&](int t) __attribute__((always_inline)) { issue_own(t, kb, k_sn, k_rb, kv_voff[0], kv_voff2[0], std::integral_constant<int, 0>{}); };
+    auto issue_own_v = [&](int t) __attribute__((always_inline)) { issue_own(t, vb, v_sn, v_rb, kv_voff[1], kv_voff2[1], std::integral_constant<int, C::OFF_V>{}); };
+    auto zero_own_rows = [&](int t, int at) __attribute__((always_inline)) {
+        for (int r = (lane >> 3); r < BN; r += 8)
+            if (t * BN + r >= N)
+#pragma unroll
+                for (int half = 0; half < NH; ++half)
+                    *(LDS_PTR(u32x4))(uintptr_t)(split_dst + at + half * TILE_BYTES + r * 128 + (lane & 7) * 16) = u32x4{0u, 0u, 0u, 0u};
+    };
     auto zero_tail_rows = [&](int t, int stage) __attribute__((always_inline)) {   // after the copies of the last tile have landed
         const int key0 = t * BN;
 #pragma unroll
@@ -464,6 +530,7 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
     //   with i = lane % 16, G = (lane % 32) / 16                     -> vaddr[dblk][x] + 4096*blk + 2048*u
     uint32_t kaddr[4], vaddr[2][2];
     {
+        const uint32_t lds0 = SPLIT ? split_dst : (uint32_t)(uintptr_t)(LDS_PTR(unsigned char))smem;
         const int fk = (l32 >> 1) & 7;
 #pragma unroll
         for (int s = 0; s < 4; ++s) kaddr[s] = lds0 + l32 * 128 + (((2 * s + hh) ^ fk) << 4);
@@ -485,13 +552,14 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
     const uint32_t nib_shift = 4u - 4u * hh;
 
     // ================================ prologue: one memory round trip ================================
+    constexpr int Q_HALF = SPLIT ? 4096 : 16384;         // between the column halves of the staged q
     // Requested at once, oldest first: q (this wave's 32 rows, staged through the second K/V stage,
     // which the prologue leaves unused, K-swizzled), then K/V and the mask words of tile 0.
     {
-        const int qbase = qt * BM + wave * 32 < N ? qt * BM + wave * 32 : N - 1;   // wave-uniform
+        const int qbase = row_base < N ? row_base : N - 1;   // wave-uniform
         const uint16_t *qsrc = qb + (size_t)qbase * q_sn;
         const int last = N - 1 - qbase;                      // rows beyond N re-read row N-1
-        const uint32_t dst = lds0 + (NSTAGE - 1) * STAGE_BYTES + wave * 4096;
+        const uint32_t dst = SPLIT ? split_dst + C::OFF_V : lds0 + (NSTAGE - 1) * STAGE_BYTES + wave * 4096;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int row = 8 * j + (lane >> 3);
@@ -499,12 +567,14 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
             const int lrow = row < last ? row : last;
             const int c = pos ^ ((row >> 1) & 7);
             async_copy_b128(dst + j * 1024, qsrc, __umul24(lrow, q_rb) + chunk_at(c));
-            if constexpr (NH == 2) async_copy_b128(dst + 16384 + j * 1024, qsrc, __umul24(lrow, q_rb) + chunk_at(8 + c));
+            if constexpr (NH == 2) async_copy_b128(dst + Q_HALF + j * 1024, qsrc, __umul24(lrow, q_rb) + chunk_at(8 + c));
         }
     }
     using std::integral_constant;
     uint32_t live_w = has_map ? (first_w | first_w2) : 0xffffffffu;
     if ((T & 31) != 0 && TW == 1) live_w &= (1u << (T & 31)) - 1u;
+    const uint32_t own_tiles = SPLIT ? 0x11111111u << wave : 0xffffffffu;
+    live_w &= own_tiles;
     const int n_visits = TW == 1 ? __builtin_popcount(live_w) : T;
     // Walk over the set bits of the "live" words: `live_w` holds the bits of word `cur_w` that have
     // not been visited yet.  Words beyond the first (N > 2048) are fetched when the walk gets there.
@@ -518,7 +588,7 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
                              : "=&s"(lv), "=&s"(lv2) : "s"(mapw + cur_w), "s"(mapw2 + cur_w) : "memory");
             lv |= lv2;
             if (cur_w == TW - 1 && (T & 31) != 0) lv &= (1u << (T & 31)) - 1u;
-            live_w = lv;
+            live_w = lv & own_tiles;
         }
         const int b = __builtin_ctz(live_w);
         live_w &= live_w - 1u;
@@ -526,7 +596,10 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
     };
     const int t_first = next_tile();
     if (t_first < T) {
-        if constexpr (PAIRS) {          // the first pair's bytes before K/V: the walk below counts on that order
+        if constexpr (SPLIT) {          // V waits until q, which sits in its buffer, has been read
+            issue_own_k(t_first);
+            issue_mask(t_first, integral_constant<int, 0>{});
+        } else if constexpr (PAIRS) {   // the first pair's bytes before K/V: the walk below counts on that order
             issue_mask_pair(0);
             issue_kv(t_first, integral_constant<int, 0>{});
         } else {
@@ -539,7 +612,8 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
         reinterpret_cast<float *>(smem + OFF_LUT)[tid] = (((tid >> 2) >> (tid & 3)) & 1) ? 0.f : -__builtin_inff();
     const bool even_progress = NH == 1 && (int)blockIdx.x >= a.tail_start;   // three work-groups per CU
     if (even_progress && n_visits >= 4) __builtin_amdgcn_s_setprio(3);
-    if (PAIRS) wait_vmcnt<8>();                   // q has landed; 4 mask and 4 K/V copies may still be in flight
+    if (SPLIT) { if (t_first < T) wait_vmcnt<8 * NH + C::MASK_COPIES>(); else wait_vmcnt<0>(); }
+    else if (PAIRS) wait_vmcnt<8>();                   // q has landed; 4 mask and 4 K/V copies may still be in flight
     else if (t_first < T) wait_vmcnt<C::COPIES>();     // q has landed; the copies of the first tile may still be in flight
     else wait_vmcnt<0>();
     // ---- Q^T as MFMA B operands, scaled by scale*log2(e)/post_mul:
@@ -547,7 +621,7 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
     u32x4 qf[KS];
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
-        u32x4 t = lds_read_b128(kaddr[s & 3] + (NSTAGE - 1) * STAGE_BYTES + (s >> 2) * 16384 + wave * 4096);
+        u32x4 t = lds_read_b128(kaddr[s & 3] + (SPLIT ? C::OFF_V + (s >> 2) * Q_HALF : (NSTAGE - 1) * STAGE_BYTES + (s >> 2) * Q_HALF + wave * 4096));
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const float lo = E::up1((uint16_t)(t[i] & 0xffffu)) * a.q_scale;
@@ -556,6 +630,11 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
         }
         if (!PACKED_ROWS && 2 * s + hh > last_chunk) t = u32x4{0u, 0u, 0u, 0u};      // beyond the row: adds nothing
         qf[s] = t;
+    }
+
+    if constexpr (SPLIT) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (t_first < T) issue_own_v(t_first);
     }
 
     // ---- running state: one query row per lane; both lane halves hold the same ref ----
@@ -592,8 +671,12 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
 
     // One key tile for this wavefront.  `so` (LDS offset of the stage) is a compile-time constant
     // in every call, so all LDS addresses below are a register plus an immediate.
-    auto compute_tile = [&](const u32x2 w2, const uint32_t so) __attribute__((always_inline)) {
-        if (__builtin_amdgcn_ballot_w64((w2.x | w2.y) != 0u) == 0ull) return;
+    // (SPLIT: `after_scores` runs when K has been read, `before_values` before V is.)
+    auto compute_tile_with = [&](const u32x2 w2, const uint32_t so, auto after_scores, auto before_values) __attribute__((always_inline)) {
+        if (__builtin_amdgcn_ballot_w64((w2.x | w2.y) != 0u) == 0ull) {
+            after_scores();
+            return;
+        }
         // ---- S^T: sacc[blk][4g+j] = log2 weight / pm of (key 32blk + 8g + 4hh + j, query l32) ----
         f32x16 sacc[2];
         // The K fragments of MFMA step s + 1 are requested before the MFMAs of step s are issued, the
@@ -630,6 +713,7 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
             sacc[1] = E::mfma(kf[s & 1][1], qf[s], sacc[1]);
             __builtin_amdgcn_sched_barrier(0);
         }
+        after_scores();
         // ---- the row maximum of the tile is taken only when it can matter ----
         // Moves the reference point when a row's scores leave the window [r-8, r+8] upwards, or when
         // the first kept score of a row lies below it.
@@ -701,6 +785,7 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
             lsum = exponentials();
         }
         l_run += lsum;
+        before_values();
         // ---- O^T += V^T * P^T : oacc[b][4g+j] = out(query l32, d = 32b + 8g + 4hh + j) ----
 #pragma unroll
         for (int blk = 0; blk < 2; ++blk)
@@ -717,6 +802,10 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
                     oacc[b] = E::mfma(va, pv, oacc[b]);
                 }
             }
+    };
+
+    auto compute_tile = [&](const u32x2 w2, const uint32_t so) __attribute__((always_inline)) {
+        compute_tile_with(w2, so, [] {}, [] {});
     };
 
     // ================================ main loop ================================
@@ -752,7 +841,29 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
         }
         compute_tile(w2, (uint32_t)(SLOT * STAGE_BYTES));
     };
-    if constexpr (PAIRS) {
+    if constexpr (SPLIT) {
+        __syncthreads();              // the table of the mask bias
+        for (int t = t_first, tn; t < T; t = tn) {
+            tn = next_tile();
+            wait_vmcnt<8 * NH>();     // K and the mask of tile t; its V may still be on its way
+            if (ragged && t == T - 1) zero_own_rows(t, 0);
+            const u32x2 w2 = mask_words(t, 0);
+            compute_tile_with(w2, 0u,
+                [&]() __attribute__((always_inline)) {
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                    if (tn < T) {
+                        issue_own_k(tn);
+                        issue_mask(tn, integral_constant<int, 0>{});
+                    }
+                },
+                [&]() __attribute__((always_inline)) {
+                    if (tn < T) wait_vmcnt<8 * NH + C::MASK_COPIES>(); else wait_vmcnt<0>();
+                    if (ragged && t == T - 1) zero_own_rows(t, C::OFF_V);
+                });
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (tn < T) issue_own_v(tn);
+        }
+    } else if constexpr (PAIRS) {
         // Every tile is visited (there is no tile map with a boolean mask) and their number is even.
         // Copies in flight, oldest first, at the top of an even visit t: the bytes of the pair
         // (t, t + 1), then K/V of t; after its barrier K/V of t + 1 and then the bytes of the next
@@ -794,7 +905,53 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
     }
     wait_vmcnt<0>();              // no copy may outlive the work-group's LDS allocation
 
-    if constexpr (BYPRODUCTS) {
+    if constexpr (SPLIT) {
+        // Wavefronts 1 to 3 leave their sums in their own buffers, wavefront 0 adds them to its own, all of them
+        // moved to the largest reference point of those that have met a kept key.
+        const bool seen = rmax > -__builtin_inff();
+        if (wave != 0) {
+#pragma unroll
+            for (int b = 0; b < OB; ++b)
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    *(LDS_PTR(f32x4))(uintptr_t)(split_dst + (4 * b + g) * 1024 + lane * 16) =
+                        f32x4{oacc[b][4 * g], oacc[b][4 * g + 1], oacc[b][4 * g + 2], oacc[b][4 * g + 3]};
+            *(LDS_PTR(f32x2))(uintptr_t)(split_dst + OB * 4096 + lane * 8) = f32x2{seen ? ref : -__builtin_inff(), l_run};
+        }
+        __syncthreads();
+        if (wave != 0) return;
+        f32x2 of_wave[4];
+        of_wave[0] = f32x2{seen ? ref : -__builtin_inff(), l_run};
+        float top = of_wave[0].x;
+#pragma unroll
+        for (int w = 1; w < 4; ++w) {
+            of_wave[w] = *(LDS_PTR(const f32x2))(uintptr_t)(lds0 + w * STAGE_BYTES + OB * 4096 + lane * 8);
+            top = __builtin_fmaxf(top, of_wave[w].x);
+        }
+        ref = top > -__builtin_inff() ? top : 0.f;
+        l_run = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            // a wavefront that has met no kept key of the row has nothing to add (its factor is 0)
+            const float d = of_wave[w].x - ref;
+            const float f = __builtin_amdgcn_exp2f(POSTMUL ? d * pm : d);
+            l_run = __builtin_fmaf(of_wave[w].y, f, l_run);
+#pragma unroll
+            for (int b = 0; b < OB; ++b)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    if (w == 0) {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) oacc[b][4 * g + j] *= f;
+                    } else {
+                        const f32x4 o = *(LDS_PTR(const f32x4))(uintptr_t)(lds0 + w * STAGE_BYTES + (4 * b + g) * 1024 + lane * 16);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) oacc[b][4 * g + j] = __builtin_fmaf(o[j], f, oacc[b][4 * g + j]);
+                    }
+                }
+        }
+    }
+    if constexpr (BYPRODUCTS && !SPLIT) {
         if (map_dst != nullptr) {
             const int rb = wave >> 1;                          // block of 64 rows
             uint32_t before = 0u;
@@ -826,9 +983,9 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
     const float l_tot = xhalf_sum(l_run);
     const float inv = (l_tot > 0.f) ? 1.0f / l_tot : 0.f;
     {
-        const int row0 = qt * BM + wave * 32;
-        const uint32_t ebase = lds0 + (uint32_t)(visits & 1) * STAGE_BYTES + wave * 4096;
-        store_rows<BF16, OB>(oacc, inv, ebase, 16384, block_dst(a.out, a.out32, bi, hi, row0, D), a.out.p != nullptr,
+        const int row0 = row_base;
+        const uint32_t ebase = SPLIT ? lds0 : lds0 + (uint32_t)(visits & 1) * STAGE_BYTES + wave * 4096;
+        store_rows<BF16, OB>(oacc, inv, ebase, SPLIT ? 4096 : 16384, block_dst(a.out, a.out32, bi, hi, row0, D), a.out.p != nullptr,
                              BF16 && a.out32.p != nullptr, row0, N, lane);       // fp32 callers compute in bf16
     }
     if (qrow < N) {
@@ -845,7 +1002,8 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_fwd_kernel(c
 }  // namespace
 
 // The instance for (element type, post-multiplier, row strides) and the kind of mask: 0 packed words, 1
-// boolean bytes, 2 the same with by-products, 3 and 4 those with two tiles' bytes per request.  This file is
+// boolean bytes, 2 the same with by-products, 3 and 4 those with two tiles' bytes per request, 5 to 7 the first
+// three with the keys split between the wavefronts.  This file is
 // compiled once per head dim for the instances, side by side, and once for the launcher.
 typedef void (*FwdKernel)(const AttnArgs);
 #ifdef SMA_FWD_HEAD_DIM
@@ -855,6 +1013,9 @@ template <int HDIM, bool BF16, bool POSTMUL, bool PACKED_ROWS> FwdKernel pick_ma
     case 0: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM>;
     case 1: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true>;
     case 2: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true>;
+    case 5: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, false, false, false, true>;
+    case 6: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, false, false, true>;
+    case 7: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true, false, true>;
     }
     if constexpr (HDIM <= 64) {
         if (mask_kind == 3) return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, false, true>;
@@ -899,15 +1060,28 @@ int compute_units()
 hipError_t launch_attn_fwd(const AttnArgs &args, bool bf16, hipStream_t stream)
 {
     AttnArgs a = args;
-    a.div_qtiles = make_fastdiv((uint32_t)a.qtiles);
     a.div_H = make_fastdiv((uint32_t)a.H);
-    const long long groups = (long long)a.BH * a.qtiles;
+    long long groups = (long long)a.BH * a.qtiles;
     if (groups == 0) return hipSuccess;
     // Only a grid that is resident all at once with three work-groups on (almost) every CU evens out
     // its progress; with several rounds oldest-first is what frees slots for the waiting ones, and
     // applying it to the last round only measured neutral.
     const long long cus = compute_units();
-    a.tail_start = (groups > 2 * cus && groups <= 3 * cus) ? 0 : (int)groups;
+    // Keys split between the wavefronts (SPLIT at the kernel): while all work-groups of 32 rows are resident
+    // at once, two on a CU up to head dim 64 and one beyond, and there are three key tiles or more to share.  Beyond
+    // that line the fewer, longer work-groups of 128 rows win (8 x 8 heads, N = 512, D = 64: 11.2 against 14.8 us).
+    // By the shape alone, so that every way of giving the same mask gives the same bits.
+    const bool split = a.N > 2 * BN && 2 * groups <= (a.D <= HD ? cus : cus / 2);
+    if (split) {
+        a.qtiles = (a.N + 31) / 32;
+        groups = (long long)a.BH * a.qtiles;
+        if (a.map_out != nullptr) {
+            const hipError_t e = launch_tile_map_start(a.map_out, a.map_slabs, a.N, stream);
+            if (e != hipSuccess) return e;
+        }
+    }
+    a.div_qtiles = make_fastdiv((uint32_t)a.qtiles);
+    a.tail_start = (!split && groups > 2 * cus && groups <= 3 * cus) ? 0 : (int)groups;
     const dim3 grid((unsigned)groups), block(NTHREADS);
     const bool postmul = a.post_mul != 1.0f;
     const int D = kernel_head_dim(a.D);
@@ -916,9 +1090,9 @@ hipError_t launch_attn_fwd(const AttnArgs &args, bool bf16, hipStream_t stream)
     const bool byproducts = a.mask_out != nullptr || a.map_out != nullptr;
     // two tiles' mask bytes per request (see PAIRS at the kernel), unless the grid is the single round
     // of work-groups in step for which tail_start was set to 0 above
-    const bool pairs = a.byte_mask && D <= HD && a.N % (2 * BN) == 0 && a.tail_start != 0;
+    const bool pairs = !split && a.byte_mask && D <= HD && a.N % (2 * BN) == 0 && a.tail_start != 0;
     if (a.byte_mask && a.N < 16) return hipErrorInvalidValue;  // a row holds at least one 16-byte copy (checked by the C-ABI layer)
-    const int mask_kind = !a.byte_mask ? 0 : (pairs ? 3 : 1) + (byproducts ? 1 : 0);
+    const int mask_kind = (split ? 5 : 0) + (!a.byte_mask ? 0 : (pairs ? 3 : 1) + (byproducts ? 1 : 0));
     const int variant = (bf16 ? 4 : 0) | (postmul ? 2 : 0) | (packed ? 1 : 0);
     const FwdKernel kernel = D == 32 ? fwd_kernel_32(variant, mask_kind) : D == 64 ? fwd_kernel_64(variant, mask_kind)
                              : D == 96 ? fwd_kernel_96(variant, mask_kind) : fwd_kernel_128(variant, mask_kind);

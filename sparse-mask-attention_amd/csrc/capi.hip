@@ -317,6 +317,7 @@ int sma_attn_fwd_call(const sma_fwd_call *c, void *stream)
     a.byte_mask = bytes;
     a.mask_out = bytes ? c->packed_out : nullptr;
     a.map_out = bytes ? c->map_out : nullptr;
+    a.map_slabs = (long long)(c->mask_stride_b != 0 ? B : 1) * (c->mask_stride_h != 0 ? H : 1);
     // the map is contiguous [Bm, Hm, ...] with the mask's own Bm, Hm (1 where the mask is shared)
     a.tile_map = bytes ? nullptr : c->tile_map;
     const long long map_words = sma_tile_map_words(N);

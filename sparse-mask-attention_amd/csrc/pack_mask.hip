@@ -355,6 +355,17 @@ __global__ __launch_bounds__(PACK_THREADS) void tile_map_kernel(const uint32_t *
     }
 }
 
+// Tile map before the first mask entry is looked at: no block keeps anything, every block is full.
+__global__ __launch_bounds__(PACK_THREADS) void tile_map_start_kernel(uint32_t *__restrict__ map, long long words, int T, int tw)
+{
+    const long long i = (long long)blockIdx.x * PACK_THREADS + threadIdx.x;
+    if (i >= words) return;
+    const int w = (int)(i % (2 * tw));
+    uint32_t x = 0u;
+    if (w >= tw) x = (w == 2 * tw - 1 && (T & 31)) ? (1u << (T & 31)) - 1u : 0xffffffffu;
+    map[i] = x;
+}
+
 // fp32 arrays -> bf16, 8 elements per thread and step.  Streaming: q, k and v of a call go in one launch
 // (blockIdx.y names the array), where a conversion and a zero-padding pass per tensor took six.
 struct ToBf16Args {
@@ -391,6 +402,15 @@ hipError_t launch_to_bf16(const float *const *src, uint16_t *const *dst, int cou
     const long long blocks = (a.chunks + PACK_THREADS - 1) / PACK_THREADS;
     hipLaunchKernelGGL(to_bf16_kernel, dim3((unsigned)(blocks < 8192 ? blocks : 8192), (unsigned)count), dim3(PACK_THREADS), 0,
                        stream, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_tile_map_start(uint32_t *map, long long slabs, int N, hipStream_t stream)
+{
+    const int T = (N + 63) / 64, tw = (T + 31) / 32;
+    const long long words = slabs * T * 2 * tw;
+    hipLaunchKernelGGL(tile_map_start_kernel, dim3((unsigned)((words + PACK_THREADS - 1) / PACK_THREADS)), dim3(PACK_THREADS), 0,
+                       stream, map, words, T, tw);
     return hipGetLastError();
 }
 

@@ -54,6 +54,7 @@ struct AttnArgs {
     int byte_mask;                  // the mask is the caller's boolean tensor, not packed words
     uint32_t *mask_out;             // byte_mask only: nullptr, or where to leave the packed words [Bm, Hm, N, nw]
     uint32_t *map_out;              // byte_mask only: nullptr, or where to leave the tile map (layout as tile_map below)
+    long long map_slabs;            // (batch entry, head) pairs of the mask
     // packed mask only: nullptr, or the tile map [Bm, Hm, T, 2, ceil(T/32)] (T = ceil(N/64)): per block
     // of 64 query rows one bit per 64-key tile "some mask bit set", then one bit per key tile "all
     // mask bits set"; strides between batch entries / heads in words, 0 = shared
@@ -115,6 +116,8 @@ int unaligned_access_state(hipStream_t stream);
 // tile map [slabs, ceil(N/64), 2, ceil(ceil(N/64)/32)] of packed words [slabs, N, ceil(N/32)]
 hipError_t launch_tile_map(const uint32_t *packed, uint32_t *map, long long slabs, int N, hipStream_t stream);
 
+// a tile map from which bits are then taken and to which bits are added: nothing kept, everything kept
+hipError_t launch_tile_map_start(uint32_t *map, long long slabs, int N, hipStream_t stream);
 // both of the above in one pass over the mask
 hipError_t launch_pack_mask_map(const uint8_t *mask, uint32_t *packed, uint32_t *map, long long slabs, int N,
                                 hipStream_t stream);
