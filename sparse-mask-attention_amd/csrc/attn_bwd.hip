@@ -359,13 +359,14 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_bwd_dq_kerne
 // ------------------------------------------------------------------------------------------------
 // dK and dV
 // ------------------------------------------------------------------------------------------------
-// NW wavefronts of 32 keys each.  Up to head dim 96 the K and V fragments of a wavefront's keys stay in
-// registers.  At 128 (VLDS) the accumulators of dK and dV take 128 registers; the V fragments then wait in LDS,
-// 16 bytes per lane and fragment in the order the lanes read them.  Both gradients in one kernel form S once
-// where a kernel for each formed it twice: 2783 -> 2032 us on 4 x 32 heads, N = 4096 (1.08 PFLOP/s over four
-// products).
-template <int HDIM, int NW> struct DkvCfg {
-    static constexpr bool VLDS = HDIM == 128;
+// NW wavefronts of 32 keys each.  The K fragments of a wavefront's keys stay in registers, and the V fragments where they
+// fit.  VLDS: they wait in LDS, 16 bytes per lane and fragment in the order the lanes read them, and the mask words are
+// read twice instead of kept.
+//   128  the accumulators of dK and dV take 128 registers; both gradients in one kernel form S once where a kernel
+//        for each formed it twice: 2783 -> 2032 us on 4 x 32 heads, N = 4096 (1.08 PFLOP/s over four products)
+//   64   166 registers instead of 198: three work-groups on a CU instead of two, where the grid has them (see the
+//        launcher): 16 x 12 heads, N = 512: 41.0 -> 37.3 us (691 TFLOP/s)
+template <int HDIM, int NW, bool VLDS> struct DkvCfg {
     static constexpr int NH = HDIM > 64 ? 2 : 1;
     static constexpr int STAGE_BYTES = 2 * NH * TILE_BYTES;
     static constexpr int OFF_B = NH * TILE_BYTES;           // dO inside a stage
@@ -375,17 +376,16 @@ template <int HDIM, int NW> struct DkvCfg {
     static constexpr int FRAG = VLDS ? HDIM / 16 * 1024 : 0;
     static constexpr int LDS_BYTES = OFF_FRAG + NW * FRAG;
 };
-template <bool BF16, int HDIM, int NW, bool POSTMUL, bool WIDE>
-__global__ __launch_bounds__(64 * NW, HDIM == 128 ? NW / 4 : 2) void attn_bwd_dkv_kernel(const AttnBwdArgs a)
+template <bool BF16, int HDIM, int NW, bool VLDS, bool POSTMUL, bool WIDE>
+__global__ __launch_bounds__(64 * NW, HDIM == 128 ? NW / 4 : VLDS ? 3 : 2) void attn_bwd_dkv_kernel(const AttnBwdArgs a)
 {
     using E = Elem<BF16>;
     constexpr int NH = HDIM > 64 ? 2 : 1;
     constexpr int KS = HDIM / 16;
     constexpr int OB = HDIM / 32;
-    using C = DkvCfg<HDIM, NW>;
+    using C = DkvCfg<HDIM, NW, VLDS>;
     constexpr int STAGE_BYTES = C::STAGE_BYTES, OFF_AUX = C::OFF_AUX, AUX_BYTES = C::AUX;
     constexpr int OFF_LSE = NW * 256, OFF_DELTA = OFF_LSE + 256;       // inside the small data of a stage
-    constexpr bool VLDS = C::VLDS;
     __shared__ __attribute__((aligned(1024))) unsigned char smem[C::LDS_BYTES];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(LDS_PTR(unsigned char))smem;
 
@@ -484,9 +484,10 @@ __global__ __launch_bounds__(64 * NW, HDIM == 128 ? NW / 4 : 2) void attn_bwd_dk
         }
 
     // bases of this lane's reads of the small data; opaque, because beyond 64 KiB the compiler would otherwise
-    // keep a register for every sum of base and offset (40 of them) instead of using the offset field
+    // keep a register for every sum of base and offset (40 of them) instead of using the offset field, and at 64
+    // three work-groups on a CU leave no register to spare
     uint32_t aux_rows = lds0 + OFF_AUX + 16 * hh, aux_words = aux_rows + wave * 256, aux_lane = lds0 + OFF_AUX + 4 * lane;
-    if constexpr (OFF_AUX >= 65536) asm volatile("" : "+v"(aux_rows), "+v"(aux_words), "+v"(aux_lane));
+    if constexpr (VLDS || OFF_AUX >= 65536) asm volatile("" : "+v"(aux_rows), "+v"(aux_words), "+v"(aux_lane));
 
     // one q tile; the ring stage is a compile-time constant so that every LDS address of the body is
     // a register plus an immediate
@@ -941,22 +942,30 @@ void launch_pair(hipStream_t stream, const AttnBwdArgs &args)
     }
     // dQ first: it also fills the delta workspace that the dK/dV kernel reads (same stream)
     hipLaunchKernelGGL((attn_bwd_dq_kernel<BF16, HDIM, WIDE>), dim3((unsigned)(a.BH * a.qtiles)), dim3(NTHREADS), 0, stream, a);
-    auto dkv = [&](auto nw_c) {
+    auto dkv = [&](auto nw_c, auto vlds_c) {
         constexpr int NW = decltype(nw_c)::value;
         a.ktiles = (a.N + 32 * NW - 1) / (32 * NW);
         a.div_ktiles = make_fastdiv((uint32_t)a.ktiles);
-        hipLaunchKernelGGL((attn_bwd_dkv_kernel<BF16, HDIM, NW, POSTMUL, WIDE>), dim3((unsigned)(a.BH * a.ktiles)), dim3(64 * NW), 0,
-                           stream, a);
+        hipLaunchKernelGGL((attn_bwd_dkv_kernel<BF16, HDIM, NW, decltype(vlds_c)::value, POSTMUL, WIDE>),
+                           dim3((unsigned)(a.BH * a.ktiles)), dim3(64 * NW), 0, stream, a);
     };
-    // Head dim 128: eight wavefronts read Q and dO once per 256 keys and keep two of themselves on a SIMD, four
-    // leave a CU to one work-group; but a grid that four-wavefront work-groups do not fill takes them (1 x 8 heads,
-    // N = 1024: 74 against 87 us), and so do short keys of which 256 at a time would leave a sixth or more idle.
-    // Elsewhere eight win: 16 x 12, N = 1024: 373 against 431 us.
-    const long long groups = (long long)a.BH * a.qtiles;
-    if (HDIM == 128 && groups > compute_units() && (a.qtiles % 2 == 0 || a.qtiles >= 5))
-        dkv(std::integral_constant<int, HDIM == 128 ? 8 : 4>{});
-    else
-        dkv(std::integral_constant<int, 4>{});
+    using four = std::integral_constant<int, 4>;
+    const long long groups = (long long)a.BH * a.qtiles, cus = compute_units();
+    if constexpr (HDIM == 128) {
+        // Eight wavefronts read Q and dO once per 256 keys and keep two of themselves on a SIMD, four
+        // leave a CU to one work-group; but a grid that four-wavefront work-groups do not fill takes them (1 x 8 heads,
+        // N = 1024: 74 against 87 us), and so do short keys of which 256 at a time would leave a sixth or more idle.
+        // Elsewhere eight win: 16 x 12, N = 1024: 373 against 431 us.
+        if (groups > cus && (a.qtiles % 2 == 0 || a.qtiles >= 5)) dkv(std::integral_constant<int, 8>{}, std::true_type{});
+        else dkv(four{}, std::true_type{});
+    } else if (HDIM == 64 && groups > 2 * cus && (2 * groups <= 7 * cus || groups > 4 * cus)) {
+        // Three work-groups on a CU.  A grid that two of them on each CU hold does not need the third and pays for the reads
+        // (whole backward, 128 heads, N = 448: 39.0 against 38.1 us), two full rounds of two are as fast as one and a
+        // third of three (64 heads, N = 2048: 277 against 273 us); beyond, 5 to 9 % (256 heads, N = 300: 41.6 against 45.4).
+        dkv(four{}, std::integral_constant<bool, HDIM == 64>{});
+    } else {
+        dkv(four{}, std::false_type{});
+    }
 }
 template <int HDIM>
 void launch_head_dim(bool bf16, hipStream_t stream, const AttnBwdArgs &a)
