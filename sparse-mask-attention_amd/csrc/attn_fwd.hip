@@ -77,7 +77,8 @@ constexpr float SUM_LIMIT = 16384.0f;     // a lane's 32 weights of a tile sum t
 // and one exchange between the lane halves): the separate packing pass, its launch and the
 // round trip of the words through memory disappear for a mask that is used once.
 template <int NH, bool BYTEMASK, bool SPLIT> struct Cfg {
-    static constexpr int NSTAGE = SPLIT ? 4 : 2; // SPLIT: one K and one V buffer for each of the four wavefronts, else                               // ring of two stages: copies run one tile ahead
+    // SPLIT: one K and one V buffer for each of the four wavefronts, else a ring of two stages: copies run one tile ahead
+    static constexpr int NSTAGE = SPLIT ? 4 : 2;
     static constexpr int MASK_COPIES = BYTEMASK ? 2 : 1;
     static constexpr int COPIES = MASK_COPIES + 4 * NH;             // async copies per wave and tile
     // LDS map (bytes)
@@ -117,6 +118,11 @@ template <int N> __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_
 // step (the even-progress case of the launcher, e.g. the headline shape): there the first visit,
 // which waits for twice the bytes, is not hidden behind other work-groups' work, it measured 1 to 4 %
 // slower, and the launcher leaves it off.
+// AHEAD (like PAIRS, any other N): a tile's mask bytes are requested two tiles ahead.  A wave has turned its bytes of a
+// tile into words before it requests others, so the tile's own slot takes those of the tile after next.  Rows that
+// start anywhere come as parts of two cache lines, and one tile's time does not cover what a mask that is in no cache
+// takes: 8 x 16 heads, N = 1000, bf16: 60.5 -> 55.8 us.  Not where the whole grid is one round in step, whose first
+// requests all come at once and where it costs 1.6 % (16 x 12, N = 512: 20.2 -> 20.6 us).
 // SPLIT: for grids that leave most of the chip idle.  The four wavefronts of a work-group share 32 query
 // rows and take every fourth key tile each, with a K and a V buffer of their own: no barriers, four times
 // the work-groups, a quarter of the serial chain; what they found is combined through LDS at the end.
@@ -125,10 +131,11 @@ template <int N> __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_
 // -> 11.1 us; 4 x 8, N = 512: 10.1 -> 7.9 us.  A wavefront now copies 16 KB per tile instead of 4, and a tile takes
 // 1.4 times as long.
 template <bool BF16, bool POSTMUL, bool PACKED_ROWS, int HDIM, bool BYTEMASK = false, bool BYPRODUCTS = false,
-          bool PAIRS = false, bool SPLIT = false>
+          int FETCH = 0, bool SPLIT = false>
 __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ? 2 : 3) void attn_fwd_kernel(const AttnArgs a)
 {
-    static_assert(!PAIRS || (BYTEMASK && HDIM <= 64 && !SPLIT), "PAIRS: byte mask, two byte slots");
+    static_assert(FETCH == 0 || (BYTEMASK && HDIM <= 64 && !SPLIT), "PAIRS, AHEAD: byte mask, two byte slots");
+    constexpr bool PAIRS = FETCH == 1, AHEAD = FETCH == 2;
     using E = Elem<BF16>;
     constexpr int NH = HDIM > 64 ? 2 : 1;         // 64-column tiles per matrix
     constexpr int KS = HDIM / 16;                 // MFMA steps of the QK^T chain
@@ -595,6 +602,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         return 32 * cur_w + b;
     };
     const int t_first = next_tile();
+    const bool even_progress = NH == 1 && (int)blockIdx.x >= a.tail_start;   // three work-groups per CU
     if (t_first < T) {
         if constexpr (SPLIT) {          // V waits until q, which sits in its buffer, has been read
             issue_own_k(t_first);
@@ -605,15 +613,16 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         } else {
             issue_kv(t_first, integral_constant<int, 0>{});
             issue_mask(t_first, integral_constant<int, 0>{});
+            if (AHEAD && T > 1) issue_mask(1, integral_constant<int, 1>{});
         }
     }
     // small LDS table for the mask: entry n (16 B) holds four floats, float j = (bit j of n) ? 0 : -inf
     if (tid < 64)
         reinterpret_cast<float *>(smem + OFF_LUT)[tid] = (((tid >> 2) >> (tid & 3)) & 1) ? 0.f : -__builtin_inff();
-    const bool even_progress = NH == 1 && (int)blockIdx.x >= a.tail_start;   // three work-groups per CU
     if (even_progress && n_visits >= 4) __builtin_amdgcn_s_setprio(3);
     if (SPLIT) { if (t_first < T) wait_vmcnt<8 * NH + C::MASK_COPIES>(); else wait_vmcnt<0>(); }
     else if (PAIRS) wait_vmcnt<8>();                   // q has landed; 4 mask and 4 K/V copies may still be in flight
+    else if (AHEAD && T > 1) wait_vmcnt<C::COPIES + C::MASK_COPIES>();
     else if (t_first < T) wait_vmcnt<C::COPIES>();     // q has landed; the copies of the first tile may still be in flight
     else wait_vmcnt<0>();
     // ---- Q^T as MFMA B operands, scaled by scale*log2(e)/post_mul:
@@ -831,13 +840,18 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
             else if (visits == (3 * n_visits) / 4) __builtin_amdgcn_s_setprio(0);
         }
         ++visits;
-        wait_vmcnt<0>();          // the copies of tile t (the only ones in flight) have landed
+        // the copies of tile t have landed; the mask bytes of the next may be in flight, they are always the youngest
+        if (AHEAD && t + 1 < T) wait_vmcnt<C::MASK_COPIES>(); else wait_vmcnt<0>();
         if (ragged && t == T - 1) zero_tail_rows(t, SLOT);
         __syncthreads();          // tile t landed for every wave; the stage of the previous visit is free
         const u32x2 w2 = mask_words(t, SLOT);
         if (t_next < T) {       // K/V first: the MFMA operands are what the next visit needs first (1-2 % with a byte mask)
             issue_kv(t_next, integral_constant<int, SLOT2>{});
-            issue_mask(t_next, integral_constant<int, SLOT2>{});
+            if constexpr (!AHEAD) issue_mask(t_next, integral_constant<int, SLOT2>{});
+        }
+        if (AHEAD && t + 2 < T) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // this wave's bytes of tile t have been read
+            issue_mask(t + 2, integral_constant<int, SLOT>{});
         }
         compute_tile(w2, (uint32_t)(SLOT * STAGE_BYTES));
     };
@@ -1003,7 +1017,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
 
 // The instance for (element type, post-multiplier, row strides) and the kind of mask: 0 packed words, 1
 // boolean bytes, 2 the same with by-products, 3 and 4 those with two tiles' bytes per request, 5 to 7 the first
-// three with the keys split between the wavefronts.  This file is
+// three with the keys split between the wavefronts, 8 and 9 (1 and 2) with the bytes two tiles ahead.  This file is
 // compiled once per head dim for the instances, side by side, and once for the launcher.
 typedef void (*FwdKernel)(const AttnArgs);
 #ifdef SMA_FWD_HEAD_DIM
@@ -1013,13 +1027,17 @@ template <int HDIM, bool BF16, bool POSTMUL, bool PACKED_ROWS> FwdKernel pick_ma
     case 0: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM>;
     case 1: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true>;
     case 2: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true>;
-    case 5: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, false, false, false, true>;
-    case 6: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, false, false, true>;
-    case 7: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true, false, true>;
+    case 5: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, false, false, 0, true>;
+    case 6: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, false, 0, true>;
+    case 7: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true, 0, true>;
     }
     if constexpr (HDIM <= 64) {
-        if (mask_kind == 3) return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, false, true>;
-        return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true, true>;
+        switch (mask_kind) {
+        case 3: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, false, 1>;
+        case 4: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true, 1>;
+        case 8: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, false, 2>;
+        case 9: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true, 2>;
+        }
     }
     return nullptr;
 }
@@ -1088,11 +1106,11 @@ hipError_t launch_attn_fwd(const AttnArgs &args, bool bf16, hipStream_t stream)
     const bool packed = a.D == D && (int)a.q.sn == D && (int)a.k.sn == D && (int)a.v.sn == D;
     if (D > HD) a.tail_start = (int)groups;                   // two work-groups per CU: nobody yields
     const bool byproducts = a.mask_out != nullptr || a.map_out != nullptr;
-    // two tiles' mask bytes per request (see PAIRS at the kernel), unless the grid is the single round
-    // of work-groups in step for which tail_start was set to 0 above
-    const bool pairs = !split && a.byte_mask && D <= HD && a.N % (2 * BN) == 0 && a.tail_start != 0;
+    // two tiles' mask bytes per request, or the bytes two tiles ahead (see PAIRS and AHEAD at the kernel), unless the grid
+    // is the single round of work-groups in step for which tail_start was set to 0 above
+    const bool further = !split && a.byte_mask && D <= HD && a.tail_start != 0;
     if (a.byte_mask && a.N < 16) return hipErrorInvalidValue;  // a row holds at least one 16-byte copy (checked by the C-ABI layer)
-    const int mask_kind = (split ? 5 : 0) + (!a.byte_mask ? 0 : (pairs ? 3 : 1) + (byproducts ? 1 : 0));
+    const int mask_kind = (split ? 5 : 0) + (!a.byte_mask ? 0 : (!further ? 1 : a.N % (2 * BN) == 0 ? 3 : 8) + (byproducts ? 1 : 0));
     const int variant = (bf16 ? 4 : 0) | (postmul ? 2 : 0) | (packed ? 1 : 0);
     const FwdKernel kernel = D == 32 ? fwd_kernel_32(variant, mask_kind) : D == 64 ? fwd_kernel_64(variant, mask_kind)
                              : D == 96 ? fwd_kernel_96(variant, mask_kind) : fwd_kernel_128(variant, mask_kind);
