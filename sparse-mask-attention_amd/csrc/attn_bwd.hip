@@ -1,4 +1,4 @@
-// Masked-attention backward for gfx950 (MI355X), head_dim 32, 64 or 128, fp16 / bf16, fp32 accumulate.
+// Masked-attention backward for gfx950 (MI355X), head_dim 32, 64, 96 or 128, fp16 / bf16, fp32 accumulate.
 //
 // The reference declares a backward launcher (csrc/sparse_attention.h:57-64) and its Python API
 // calls sparse_attn_cuda.backward (python/sparse_attention.py:91-94), but neither was ever
@@ -611,7 +611,7 @@ __global__ __launch_bounds__(64 * NW, HDIM == 128 ? NW / 4 : VLDS ? 3 : 2) void 
 // ------------------------------------------------------------------------------------------------
 // N <= 32 NW keys and head dim <= 64: one work-group holds a whole head, a wavefront 32 of its keys, as in the dK/dV
 // kernel.  S, dP and the exponentials are formed once (the two kernels form them twice: 7 products instead of 5) and
-// q, k, v, dO are read once.  What is bound by memory and by the length of a work-group's prologue gains most:
+// q, k, v, dO come from memory once.  What is bound by memory and by the length of a work-group's prologue gains most:
 // 64 x 16 heads, N = 256, D = 64: 104 us for the two kernels, 90 us here (3.6 TB/s of what has to move; one work-group
 // of 8 wavefronts on a CU, whose loads nothing else hides), 1024 heads, N = 128: 41.7 -> 33.0 us.
 //   K            in LDS too, for dQ

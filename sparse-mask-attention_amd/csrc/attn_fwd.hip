@@ -1,4 +1,4 @@
-// Fused masked-attention forward for gfx950 (MI355X), head_dim 32, 64 or 128, fp16 / bf16, fp32 accumulate.
+// Fused masked-attention forward for gfx950 (MI355X), head_dim 32, 64, 96 or 128, fp16 / bf16, fp32 accumulate.
 //
 // Stands in for sparse_attn_wmma_full_fp16 (csrc/sparse_attention.cu:82-412 of the reference) and
 // for its scalar bf16 kernel (csrc/sparse_attention.cu:418-543); the design below is specific to
