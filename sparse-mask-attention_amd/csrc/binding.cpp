@@ -564,7 +564,12 @@ Tensor run_call(const Tensor &q, const Tensor &k, const Tensor &v, Call &c, bool
     run_forward(c, out, result, lse, want_map);
     if (!wide) {
         result = out;
-        if (Dk != c.D) result = result.narrow(3, 0, c.D);
+        if (Dk != c.D) {
+            result = result.narrow(3, 0, c.D);
+            // made below autograd, such a view counts versions of its own: with the count of the tensor that the
+            // backward reads, a change of the result in place is noticed there
+            if (tracked) torch::autograd::impl::set_version_counter(result, torch::autograd::impl::version_counter(out));
+        }
         if (kdt != dtype) result = result.to(dtype);
     }
     if (!tracked) return result;
