@@ -589,6 +589,53 @@ Tensor run_call(const Tensor &q, const Tensor &k, const Tensor &v, Call &c, bool
     return result;
 }
 
+// What is wrong with the tensors of one call, or nullptr.  Everything below reaches them through raw pointers, with
+// offsets computed from q's extents, so each entry point asks here first.
+const char *refusal(const Tensor &q, const Tensor &k, const Tensor &v, const c10::optional<Tensor> &mask,
+                    const c10::optional<Tensor> &mask_packed)
+{
+    if (!q.is_cuda()) return "q must be a GPU tensor";
+    if (q.dim() != 4 || k.sizes() != q.sizes() || v.sizes() != q.sizes()) return "q, k, v must have the same 4D shape";
+    if (k.device() != q.device() || v.device() != q.device()) return "q, k, v must be on the same device";
+    const at::ScalarType dtype = q.scalar_type();
+    if (dtype != at::kHalf && dtype != at::kBFloat16 && dtype != at::kFloat) return "Unsupported dtype, need BF16 or FP16 (or FP32)";
+    if (dtype != at::kFloat && (k.scalar_type() != dtype || v.scalar_type() != dtype)) return "q, k, v must have the same dtype";
+    const int64_t B = q.size(0), H = q.size(1), N = q.size(2), D = q.size(3);
+    if (D < 1 || D > 128) return "head_dim must be at most 128";
+    auto shared_or = [](int64_t have, int64_t want) { return have == 1 || have == want; };
+    if (mask_packed.has_value() && mask_packed->defined()) {
+        const Tensor &p = *mask_packed;
+        if (p.device() != q.device()) return "mask_packed must be on q's device";
+        if (p.scalar_type() != at::kInt || p.dim() != 4 || !shared_or(p.size(0), B) || !shared_or(p.size(1), H) || p.size(2) != N ||
+            p.size(3) != (N + 31) / 32)
+            return "mask_packed must be int32 [B or 1, H or 1, N, ceil(N/32)]";
+        return nullptr;
+    }
+    if (!mask.has_value() || !mask->defined()) return "a mask or a packed mask is needed";
+    const Tensor &m = *mask;
+    if (m.device() != q.device()) return "mask must be on q's device";
+    if (m.scalar_type() != at::kBool || m.dim() != 4 || !shared_or(m.size(0), B) || !shared_or(m.size(1), H) || m.size(2) != N ||
+        m.size(3) != N)
+        return "mask must be bool [B or 1, H or 1, N, N]";
+    return nullptr;
+}
+
+// The problem of a call whose tensors have passed the checks above; `tile_map` is a tensor's Python object or nullptr.
+Call problem(const Tensor &q, const c10::optional<Tensor> &mask, const c10::optional<Tensor> &mask_packed, const py::object *tile_map,
+             double scale)
+{
+    Call c;
+    c.B = q.size(0), c.H = q.size(1), c.N = q.size(2), c.D = q.size(3);
+    if (mask_packed.has_value() && mask_packed->defined()) {
+        c.packed = *mask_packed;
+        if (tile_map) c.map = tile_map->cast<Tensor>();
+    } else {
+        c.mask = unexpand(*mask);
+    }
+    c.scale = scale;
+    return c;
+}
+
 // sparse_attention / sparse_attention_func of the Python layer.  `tile_map` is None, True (leave a map
 // behind for the backward) or a tensor.  None is returned, before anything has been done, for
 // arguments that the Python layer refuses or has to prepare first (a boolean mask shorter than one
@@ -596,57 +643,27 @@ Tensor run_call(const Tensor &q, const Tensor &k, const Tensor &v, Call &c, bool
 c10::optional<Tensor> attention(const Tensor &q, const Tensor &k, const Tensor &v, const c10::optional<Tensor> &mask,
                                 const c10::optional<Tensor> &mask_packed, const py::object &tile_map, bool autograd)
 {
-    const at::ScalarType dtype = q.scalar_type();
-    if (!q.is_cuda() || q.dim() != 4 || k.sizes() != q.sizes() || v.sizes() != q.sizes() || k.device() != q.device() ||
-        v.device() != q.device())
-        return c10::nullopt;
-    if (dtype == at::kHalf || dtype == at::kBFloat16) {
-        if (k.scalar_type() != dtype || v.scalar_type() != dtype) return c10::nullopt;
-    } else if (dtype != at::kFloat) {
-        return c10::nullopt;
-    }
-    Call c;
-    c.B = q.size(0), c.H = q.size(1), c.N = q.size(2), c.D = q.size(3);
-    if (c.D < 1 || c.D > 128) return c10::nullopt;
-    auto shared_or = [](int64_t have, int64_t want) { return have == 1 || have == want; };
+    if (refusal(q, k, v, mask, mask_packed) != nullptr) return c10::nullopt;
+    const bool packed = mask_packed.has_value() && mask_packed->defined();
     const bool want_map = tile_map.ptr() == Py_True;
     const bool has_map = !want_map && !tile_map.is_none();
-    if (mask_packed.has_value() && mask_packed->defined()) {
-        const Tensor &p = *mask_packed;
-        if (p.scalar_type() != at::kInt || p.dim() != 4 || !shared_or(p.size(0), c.B) || !shared_or(p.size(1), c.H) ||
-            p.size(2) != c.N || p.size(3) != (c.N + 31) / 32 || p.device() != q.device() || (want_map && autograd))
-            return c10::nullopt;
-        c.packed = p;
-        if (has_map) c.map = tile_map.cast<Tensor>();
-    } else {
-        if (!mask.has_value() || !mask->defined() || has_map) return c10::nullopt;
-        const Tensor &m = *mask;
-        if (m.scalar_type() != at::kBool || m.device() != q.device() || m.dim() != 4 || !shared_or(m.size(0), c.B) ||
-            !shared_or(m.size(1), c.H) || m.size(2) != c.N || m.size(3) != c.N || (c.N < 16 && q.numel() > 0))
-            return c10::nullopt;
-        c.mask = unexpand(m);
-    }
-    c.scale = 1.0 / std::sqrt((double)c.D);
+    if (packed ? want_map && autograd : has_map || (q.size(2) < 16 && q.numel() > 0)) return c10::nullopt;
+    Call c = problem(q, mask, mask_packed, has_map ? &tile_map : nullptr, 1.0 / std::sqrt((double)q.size(3)));
     return run_call(q, k, v, c, want_map, autograd);
 }
 
-// SparseAttentionFunction.apply of the Python layer: the same with the scale given and q, k, v in a
-// head dim and type that the kernels have.
+// SparseAttentionFunction.apply of the Python layer: the same with the scale given, for q, k and v of 16 bits (nothing
+// is converted), whose wrong arguments are errors.  Without a packed mask, a tile map given as a tensor is not used.
 Tensor attention_function(const Tensor &q, const Tensor &k, const Tensor &v, const c10::optional<Tensor> &mask_packed,
                           const c10::optional<Tensor> &mask, double scale, const py::object &tile_map)
 {
-    TORCH_CHECK(q.dim() == 4 && k.sizes() == q.sizes() && v.sizes() == q.sizes(), "q, k, v must have the same 4D shape");
-    Call c;
-    c.B = q.size(0), c.H = q.size(1), c.N = q.size(2), c.D = q.size(3);
+    const char *const why = refusal(q, k, v, mask, mask_packed);
+    TORCH_CHECK(why == nullptr, why);
+    TORCH_CHECK(q.scalar_type() != at::kFloat, "Unsupported dtype, need BF16 or FP16");
+    const bool packed = mask_packed.has_value() && mask_packed->defined();
     const bool want_map = tile_map.ptr() == Py_True;
-    if (mask_packed.has_value() && mask_packed->defined()) {
-        c.packed = *mask_packed;
-        if (!want_map && !tile_map.is_none()) c.map = tile_map.cast<Tensor>();
-    } else {
-        TORCH_CHECK(mask.has_value() && mask->defined() && mask->dim() == 4, "a mask or a packed mask is needed");
-        c.mask = unexpand(*mask);
-    }
-    c.scale = scale;
+    TORCH_CHECK(!(packed && want_map), "with mask_packed, pass the result of tile_map(mask_packed)");
+    Call c = problem(q, mask, mask_packed, !want_map && !tile_map.is_none() ? &tile_map : nullptr, scale);
     return run_call(q, k, v, c, want_map, true);
 }
 

@@ -57,3 +57,33 @@ def test_an_fp32_output_may_be_changed_in_place(sa, dev, D):
         change(sa.sparse_attention(leaf, k, v, mask)).backward(do)
         got.append(leaf.grad)
     assert torch.equal(*got)
+
+
+def test_the_function_behind_the_api_refuses_what_it_cannot_address(sa, dev):
+    """SparseAttentionFunction.apply makes the checks of sparse_attention, before anything is launched: the kernels
+    address every tensor by q's extents."""
+    q, k, v, do, mask = _problem(dev)
+    packed = sa.pack_mask(mask)
+    tm = sa.sparse_attn_cuda.tile_map(packed)
+    N = q.shape[2]
+
+    def call(q=q, k=k, v=v, packed=None, mask=mask, tile_map=None):
+        return sa.SparseAttentionFunction.apply(q, k, v, packed, mask, 0.125, N, tile_map)
+
+    wrong = [dict(mask=None)]
+    wrong += [dict(mask=m) for m in (mask[:, :, :, :-1], mask[:, :, :-1], mask[:, :, :64, :64], mask[:1].expand(3, 2, N, N), mask[0],
+                                     mask[:, :1].expand(2, 4, N, N), mask.to(torch.uint8), mask.half(), mask.cpu())]
+    wrong += [dict(packed=p) for p in (packed[:, :, :-1], packed[..., :-1], packed[0], packed.float(), packed.long(), packed.cpu(),
+                                       packed.expand(2, 2, N, 3).transpose(2, 3).contiguous().transpose(2, 3),
+                                       packed[:1].expand(3, 2, N, 3))]
+    wrong += [dict(q=t(q), k=t(k), v=t(v)) for t in (torch.Tensor.double, torch.Tensor.float, torch.Tensor.int, torch.Tensor.cpu,
+                                                     lambda x: x[0], lambda x: torch.cat([x, x, x], -1))]
+    wrong += [{name: t(x)} for name, x in (("k", k), ("v", v))
+              for t in (torch.Tensor.float, torch.Tensor.bfloat16, torch.Tensor.cpu, lambda x: x[:, :, :-1], lambda x: x[..., :32])]
+    wrong += [dict(packed=packed, tile_map=t) for t in (True, tm[:, :, :1], tm.cpu(), tm.float(), 3)]
+    for args in wrong:
+        with pytest.raises(RuntimeError):
+            call(**args)
+    want = sa.sparse_attention_func(q, k, v, mask)
+    for args in ({}, dict(mask=mask, tile_map=True), dict(mask=None, packed=packed), dict(mask=None, packed=packed, tile_map=tm)):
+        assert torch.equal(call(**args), want)
