@@ -305,6 +305,9 @@ torch::Tensor pack_mask(const torch::Tensor &mask)
     return packed;
 }
 
+// Longest sequence that a tile map is made for (sma_tile_map, sma_pack_mask_map).
+constexpr int64_t MAP_MAX_N = 131072;
+
 // tile_map(mask_packed): [Bm, Hm, N, ceil(N/32)] int32 -> [Bm, Hm, T, 2, ceil(T/32)] int32, T = ceil(N/64).
 torch::Tensor tile_map(const torch::Tensor &mask_packed)
 {
@@ -313,7 +316,7 @@ torch::Tensor tile_map(const torch::Tensor &mask_packed)
                 "mask_packed must be a contiguous int32 [B, H, N, ceil(N/32)] tensor");
     const int64_t B = mask_packed.size(0), H = mask_packed.size(1), N = mask_packed.size(2);
     TORCH_CHECK(mask_packed.size(3) == (N + 31) / 32, "mask_packed must be [B, H, N, ceil(N/32)]");
-    TORCH_CHECK(B <= INT32_MAX && H <= INT32_MAX && N <= 131072, "extent too large");
+    TORCH_CHECK(B <= INT32_MAX && H <= INT32_MAX && N <= MAP_MAX_N, "extent too large");
     const int64_t T = (N + 63) / 64;
     const c10::DeviceGuard guard(mask_packed.device());
     torch::Tensor map = empty_dense({B, H, T, 2, (T + 31) / 32}, at::kInt);    // every word is written
@@ -408,10 +411,11 @@ struct Call {                       // one problem as the kernels see it
 // no room for bytes in LDS.  Measured (4 x 32 heads, one mask for the heads of a batch entry or for all):
 // N = 1000, random: 49.3 us either way; N = 2048, causal: 128 -> 111 us forward, 514 -> 458 us
 // forward + backward; 8 x 16 heads, N = 512: 15 -> 19 us.  The line lies at 2^27 scores.
+// A sequence too long for a map is packed without one, further down, like any whose bytes the kernel cannot address.
 bool pack_first(const Call &c)
 {
     const int64_t heads = c.B * c.H, masks = c.mask.size(0) * c.mask.size(1);
-    return heads >= 4 * masks && (double)heads * c.N * c.N >= (double)(1 << 27);
+    return c.N <= MAP_MAX_N && heads >= 4 * masks && (double)heads * c.N * c.N >= (double)(1 << 27);
 }
 
 // Packed words and tile map of the boolean mask, in one launch.

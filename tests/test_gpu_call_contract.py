@@ -87,3 +87,22 @@ def test_the_function_behind_the_api_refuses_what_it_cannot_address(sa, dev):
     want = sa.sparse_attention_func(q, k, v, mask)
     for args in ({}, dict(mask=mask, tile_map=True), dict(mask=None, packed=packed), dict(mask=None, packed=packed, tile_map=tm)):
         assert torch.equal(call(**args), want)
+
+
+def test_a_shared_mask_longer_than_a_tile_map_allows(sa, dev):
+    """N > 131072, one mask for four heads: packed without a map.  Every row keeps three keys, one of them the last."""
+    N, D = 131136, 32
+    g = torch.Generator().manual_seed(3)
+    q, k, v = (torch.randn(1, 4, N, D, generator=g).half().to(dev) for _ in range(3))
+    mask = torch.eye(N, dtype=torch.bool, device=dev)[None, None]
+    mask[..., 5] = True
+    mask[..., N - 1] = True
+    leaf = q.clone().requires_grad_(True)
+    out = sa.sparse_attention_func(q, k, v, mask)
+    assert torch.equal(out, sa.sparse_attention(leaf, k, v, mask).detach())
+    keys = torch.stack([torch.full((N,), 5, device=dev), torch.full((N,), N - 1, device=dev), torch.arange(N, device=dev)], 1)
+    s = (q.float()[:, :, :, None] * k.float()[:, :, keys]).sum(-1) * D ** -0.5                  # [1, 4, N, 3]
+    s[:, :, 5, 2] = s[:, :, N - 1, 2] = -float("inf")                                           # the same key a second time
+    want = (torch.softmax(s, -1)[..., None] * v.float()[:, :, keys]).sum(-2)
+    # weights (rounded toward zero, numerator and denominator alike) and output of 11 bits
+    assert torch.allclose(out.float(), want, atol=1e-2, rtol=1e-2)
