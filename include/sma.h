@@ -307,7 +307,8 @@ int sma_attn_bwd_map_strided(const sma_tensor *dout, const sma_tensor *q, const 
 typedef struct sma_fwd_call {
     const sma_tensor *q, *k, *v;
     const sma_tensor *out;                  /* optional if out_f32 is given */
-    const sma_tensor *out_f32;              /* optional: float elements, strides multiples of 8 */
+    const sma_tensor *out_f32;              /* optional: float elements, strides multiples of 8,
+                                               (N-1)*stride_n*4 + 4*D < 2^31 */
     const uint8_t *mask;                    /* boolean mask (strides in bytes), or NULL to use ... */
     const uint32_t *mask_packed;            /* ... the packed one (strides in words) */
     int64_t mask_stride_b, mask_stride_h;
@@ -322,7 +323,7 @@ int sma_attn_fwd_call(const sma_fwd_call *call, void *stream);
 
 typedef struct sma_bwd_call {
     const sma_tensor *dout, *q, *k, *v, *out;
-    const sma_tensor *dq, *dk, *dv;         /* 16-bit elements, or floats if grads_f32 */
+    const sma_tensor *dq, *dk, *dv;         /* 16-bit elements, or floats if grads_f32 (limits as out_f32) */
     const float *lse;
     const uint32_t *mask_packed;
     int64_t mask_stride_b, mask_stride_h;

@@ -388,6 +388,13 @@ Tensor empty_like_rows(const Tensor &t, at::ScalarType dtype)
     return at::empty_like(t.detach(), t.options().dtype(dtype));
 }
 
+// Whether the kernels reach every row of an fp32 tensor laid out like t (a kernel tensor, 16 bits): a lane's byte
+// offset inside one (b, h) slab has 31 bits, half the rows of a 16-bit one.
+bool reaches_f32(const Tensor &t)
+{
+    return t.numel() == 0 || (t.size(2) - 1) * t.stride(2) * 4 + t.size(3) * 4 < (int64_t(1) << 31);
+}
+
 // The mask with its expanded (stride 0) batch / head extents taken back to 1: it is then read once
 // and shared.
 Tensor unexpand(Tensor m)
@@ -514,8 +521,9 @@ struct SparseAttentionBackward : public torch::autograd::Node {
         const c10::DeviceGuard guard(tq.device());
         Tensor dout;
         kernel_rows<1>({&grads[0]}, {&dout}, tq.scalar_type(), tq.size(3));
-        // the gradients in the caller's type and layout at once, unless its rows are no multiple of 16 bytes
-        const bool direct = grad_D == tq.size(3);
+        // the gradients in the caller's type and layout at once, unless its rows are no multiple of 16 bytes or too far apart
+        const bool direct = grad_D == tq.size(3) &&
+                            (grad_dtype == tq.scalar_type() || (reaches_f32(tq) && reaches_f32(tk) && reaches_f32(tv)));
         const at::ScalarType made = direct ? grad_dtype : tq.scalar_type();
         Tensor d[3] = {empty_like_rows(tq, made), empty_like_rows(tk, made), empty_like_rows(tv, made)};
         const int64_t B = tq.size(0), H = tq.size(1), N = tq.size(2);
@@ -536,7 +544,7 @@ struct SparseAttentionBackward : public torch::autograd::Node {
         check_status(sma_attn_bwd_call(&c, c10::hip::getCurrentHIPStream(tq.device().index()).stream()), "sma_attn_bwd_call");
         if (!direct)
             for (Tensor &g : d) {
-                g = g.narrow(3, 0, grad_D);
+                if (g.size(3) != grad_D) g = g.narrow(3, 0, grad_D);
                 if (g.scalar_type() != grad_dtype) g = g.to(grad_dtype);
             }
         return {d[0], d[1], d[2]};
@@ -559,8 +567,9 @@ Tensor run_call(const Tensor &q, const Tensor &k, const Tensor &v, Call &c, bool
     const c10::DeviceGuard guard(q.device());
     at::AutoDispatchBelowADInplaceOrView below_autograd;
     kernel_rows<3>({&q, &k, &v}, {&c.q, &c.k, &c.v}, kdt, Dk);
-    // fp32 callers get their result from the kernel itself; the 16-bit one is then made for the backward only
-    const bool wide = kdt != dtype && Dk == c.D;
+    // fp32 callers get their result from the kernel itself (unless its rows are too far apart); the 16-bit one is then made
+    // for the backward only
+    const bool wide = kdt != dtype && Dk == c.D && reaches_f32(c.q);
     Tensor out, result, lse;
     if (!wide || tracked) out = empty_like_rows(c.q, kdt);
     if (wide) result = empty_like_rows(c.q, dtype);

@@ -106,3 +106,28 @@ def test_a_shared_mask_longer_than_a_tile_map_allows(sa, dev):
     want = (torch.softmax(s, -1)[..., None] * v.float()[:, :, keys]).sum(-2)
     # weights (rounded toward zero, numerator and denominator alike) and output of 11 bits
     assert torch.allclose(out.float(), want, atol=1e-2, rtol=1e-2)
+
+
+def test_fp32_rows_further_apart_than_the_kernels_store_them(sa, dev):
+    """[B, N, H, D] with H * D = 131072: the slab of a head passes 2^31 bytes in fp32, not in the 16 bits that the
+    kernels compute in.  The same heads in a tensor of their own are stored as fp32 by the kernels: the same bits."""
+    N, H, D = 4100, 1024, 128
+    g = torch.Generator(device=dev).manual_seed(4)
+    q, k, v, do = (torch.randn(1, N, H, D, device=dev, generator=g).transpose(1, 2) for _ in range(4))
+    assert (N - 1) * H * D * 4 + 4 * D >= 2 ** 31 > (N - 1) * H * D * 2 + 2 * D
+    mask = torch.rand(1, 1, N, N, device=dev, generator=g) < 0.3
+    mask[..., 64:] &= torch.rand(N, 1, device=dev, generator=g) < 0.01          # few tiles with anything in them
+    mask |= torch.eye(N, dtype=torch.bool, device=dev)
+
+    def run(heads):
+        few = heads < H
+        leaves = [(t[:, :heads].contiguous() if few else t).detach().requires_grad_(True) for t in (q, k, v)]
+        out = sa.sparse_attention(*leaves, mask)
+        with torch.no_grad():
+            assert torch.equal(out, sa.sparse_attention(*leaves, mask))
+        assert out.dtype == torch.float32 and out.stride() == leaves[0].stride()
+        return [out.detach()] + list(torch.autograd.grad(out, leaves, do[:, :heads].contiguous() if few else do))
+
+    wide, few = run(H), run(256)
+    for name, a, b in zip(("out", "dq", "dk", "dv"), wide, few):
+        assert a.dtype == torch.float32 and torch.equal(a[:, :256], b), name
