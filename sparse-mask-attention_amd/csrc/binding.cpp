@@ -551,6 +551,13 @@ struct SparseAttentionBackward : public torch::autograd::Node {
     }
 };
 
+// Forward-mode AD has no formula here: a tangent is refused, not dropped.
+void refuse_tangents(const Tensor &q, const Tensor &k, const Tensor &v)
+{
+    for (const Tensor *t : {&q, &k, &v})
+        TORCH_CHECK_NOT_IMPLEMENTED(!t->_fw_grad(/*level=*/0).defined(), "sparse attention does not support forward mode AD");
+}
+
 // Output of one call: out, with its autograd node when q, k or v want gradients and `autograd`.
 Tensor run_call(const Tensor &q, const Tensor &k, const Tensor &v, Call &c, bool want_map, bool autograd)
 {
@@ -561,6 +568,7 @@ Tensor run_call(const Tensor &q, const Tensor &k, const Tensor &v, Call &c, bool
     const bool tracked = autograd && torch::autograd::compute_requires_grad(q, k, v);
     std::shared_ptr<SparseAttentionBackward> node;
     if (tracked) {
+        refuse_tangents(q, k, v);
         node = std::make_shared<SparseAttentionBackward>();
         node->set_next_edges(torch::autograd::collect_next_edges(q, k, v));
     }
@@ -672,6 +680,7 @@ Tensor attention_function(const Tensor &q, const Tensor &k, const Tensor &v, con
 {
     const char *const why = refusal(q, k, v, mask, mask_packed);
     TORCH_CHECK(why == nullptr, why);
+    refuse_tangents(q, k, v);
     TORCH_CHECK(q.scalar_type() != at::kFloat, "Unsupported dtype, need BF16 or FP16");
     const bool packed = mask_packed.has_value() && mask_packed->defined();
     const bool want_map = tile_map.ptr() == Py_True;

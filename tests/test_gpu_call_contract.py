@@ -5,6 +5,7 @@ import sys
 
 import pytest
 import torch
+import torch.autograd.forward_ad as fwd_ad
 
 pytestmark = pytest.mark.gpu
 
@@ -131,3 +132,21 @@ def test_fp32_rows_further_apart_than_the_kernels_store_them(sa, dev):
     wide, few = run(H), run(256)
     for name, a, b in zip(("out", "dq", "dk", "dv"), wide, few):
         assert a.dtype == torch.float32 and torch.equal(a[:, :256], b), name
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_a_tangent_is_refused_and_not_dropped(sa, dev, dtype):
+    q, k, v, do, mask = _problem(dev, dtype=dtype)
+    for which in range(3):
+        leaves = [t.clone().requires_grad_(True) for t in (q, k, v)]
+        with fwd_ad.dual_level():
+            leaves[which] = fwd_ad.make_dual(leaves[which], torch.ones_like(q))
+            with pytest.raises(NotImplementedError, match="forward mode"):
+                sa.sparse_attention(*leaves, mask)
+            if dtype == torch.float16:
+                plain = [t.detach() for t in (q, k, v)]
+                plain[which] = fwd_ad.make_dual(plain[which], torch.ones_like(q))
+                for tensors in (leaves, plain):
+                    with pytest.raises(NotImplementedError, match="forward mode"):
+                        sa.SparseAttentionFunction.apply(*tensors, None, mask, 0.125, q.shape[2])
+        assert torch.equal(sa.sparse_attention(*leaves, mask), sa.sparse_attention_func(q, k, v, mask))      # the level is over
