@@ -492,7 +492,7 @@ void run_forward(Call &c, const Tensor &out, const Tensor &out_f32, const Tensor
 
 // The autograd node of one training forward.
 struct SparseAttentionBackward : public torch::autograd::Node {
-    std::mutex mutex;
+    std::recursive_mutex mutex;     // (a saved-tensor hook that the backward calls may look at saved_tensors)
     torch::autograd::SavedVariable q, k, v, out, lse, packed;
     Tensor map;                     // undefined without a tile map
     bool map_shown = false;         // the caller gave the map or asked for it
@@ -505,7 +505,7 @@ struct SparseAttentionBackward : public torch::autograd::Node {
 
     void release_variables() override
     {
-        std::lock_guard<std::mutex> lock(mutex);
+        std::lock_guard<std::recursive_mutex> lock(mutex);
         for (torch::autograd::SavedVariable *s : {&q, &k, &v, &out, &lse, &packed}) s->reset_data();
         map.reset();
     }
@@ -513,7 +513,7 @@ struct SparseAttentionBackward : public torch::autograd::Node {
     torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override
     {
         if (!grads[0].defined()) return {Tensor(), Tensor(), Tensor()};
-        std::lock_guard<std::mutex> lock(mutex);
+        std::lock_guard<std::recursive_mutex> lock(mutex);
         const Tensor tq = q.unpack(), tk = k.unpack(), tv = v.unpack();
         const Tensor tout = out.unpack(out_is_output ? shared_from_this() : nullptr);
         const Tensor tlse = lse.unpack(), tpacked = packed.unpack();
@@ -703,6 +703,28 @@ PyObject *node_scale(PyObject *self, void *)
     return PyFloat_FromDouble(node->scale);
 }
 
+// What the backward will use: q, k, v, out, lse and the packed mask as the kernels take them, for as long as the
+// backward can still run.  (Waiting for the lock and unpacking happen without the interpreter's lock: the backward holds the first
+// while a saved-tensor hook may ask for the second.)
+PyObject *node_saved_tensors(PyObject *self, void *)
+{
+    HANDLE_TH_ERRORS
+    const std::shared_ptr<torch::autograd::Node> keep = reinterpret_cast<torch::autograd::THPCppFunction *>(self)->cdata;
+    auto *node = static_cast<SparseAttentionBackward *>(keep.get());
+    std::vector<Tensor> saved;
+    {
+        const py::gil_scoped_release no_gil;
+        const std::lock_guard<std::recursive_mutex> lock(node->mutex);
+        for (const torch::autograd::SavedVariable *s : {&node->q, &node->k, &node->v}) saved.push_back(s->unpack());
+        saved.push_back(node->out.unpack(node->out_is_output ? keep : nullptr));
+        for (const torch::autograd::SavedVariable *s : {&node->lse, &node->packed}) saved.push_back(s->unpack());
+    }
+    py::tuple result(saved.size());
+    for (size_t i = 0; i < saved.size(); ++i) result[i] = py::reinterpret_steal<py::object>(THPVariable_Wrap(saved[i]));
+    return result.release().ptr();
+    END_HANDLE_TH_ERRORS
+}
+
 void register_node_type()
 {
     using namespace torch::autograd;
@@ -710,6 +732,7 @@ void register_node_type()
     static PyGetSetDef properties[] = {THP_FUNCTION_DEFAULT_PROPERTIES,
                                        {"tile_map", node_tile_map, nullptr, nullptr, nullptr},
                                        {"scale", node_scale, nullptr, nullptr, nullptr},
+                                       {"saved_tensors", node_saved_tensors, nullptr, nullptr, nullptr},
                                        {nullptr, nullptr, nullptr, nullptr, nullptr}};
     _initFunctionPyTypeObject(type, "SparseAttentionFunctionBackward", properties, nullptr);
     Py_INCREF(&type);

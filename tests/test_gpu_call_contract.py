@@ -150,3 +150,39 @@ def test_a_tangent_is_refused_and_not_dropped(sa, dev, dtype):
                     with pytest.raises(NotImplementedError, match="forward mode"):
                         sa.SparseAttentionFunction.apply(*tensors, None, mask, 0.125, q.shape[2])
         assert torch.equal(sa.sparse_attention(*leaves, mask), sa.sparse_attention_func(q, k, v, mask))      # the level is over
+
+
+@pytest.mark.parametrize("D", [60, 64])
+def test_the_node_shows_what_it_saved(sa, dev, D):
+    """grad_fn.saved_tensors: q, k, v, out, lse and the packed mask, until the backward has freed them."""
+    q, k, v, do, mask = _problem(dev, D=D)
+    leaf = q.clone().requires_grad_(True)
+    out = sa.sparse_attention(leaf, k, v, mask)
+    for _ in range(2):
+        saved = out.grad_fn.saved_tensors
+        assert len(saved) == 6
+        for a, b in zip(saved, (q, k, v, out.detach())):
+            assert torch.equal(a[..., :D], b) and not a[..., D:].any()
+        s = (q.float() @ k.float().transpose(-1, -2) * D ** -0.5).masked_fill(~mask, -float("inf"))
+        assert torch.allclose(saved[4], torch.logsumexp(s, -1), atol=2e-3)
+        assert torch.equal(saved[5], sa.pack_mask(mask))
+        out.backward(do, retain_graph=True)
+    if D == 64:
+        assert saved[0] is leaf and saved[3].grad_fn is out.grad_fn
+    out.backward(do)
+    with pytest.raises(RuntimeError, match="freed"):
+        out.grad_fn.saved_tensors
+    # through hooks, and from inside of one that the backward calls
+    seen = []
+
+    def unpack(t):
+        seen.append(t)
+        if len(seen) == 7:
+            assert len(out.grad_fn.saved_tensors) == 6
+        return t
+
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.clone(), unpack):
+        out = sa.sparse_attention(leaf, k, v, mask)
+    assert len(out.grad_fn.saved_tensors) == 6 and len(seen) == 6
+    out.backward(do)
+    assert len(seen) == 18
