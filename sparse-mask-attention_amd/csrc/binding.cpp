@@ -510,6 +510,21 @@ struct SparseAttentionBackward : public torch::autograd::Node {
         map.reset();
     }
 
+    // Saved-tensor hooks give back what they like; the kernels address it by raw pointers.  (The packed mask and the map
+    // are checked where their strides are taken.)
+    void check_saved(const Tensor &grad, std::initializer_list<const Tensor *> rows, const Tensor &tlse) const
+    {
+        const at::ScalarType kdt = grad_dtype == at::kFloat ? at::kBFloat16 : grad_dtype;
+        const int64_t B = grad.size(0), H = grad.size(1), N = grad.size(2);
+        for (const Tensor *t : rows)
+            TORCH_CHECK(t->device() == grad.device() && t->scalar_type() == kdt && t->dim() == 4 && t->size(0) == B && t->size(1) == H &&
+                            t->size(2) == N && t->size(3) == padded_head_dim(grad_D),
+                        "a saved tensor came back with another device, dtype or shape");
+        TORCH_CHECK(tlse.device() == grad.device() && tlse.scalar_type() == at::kFloat && tlse.dim() == 3 && tlse.size(0) == B &&
+                        tlse.size(1) == H && tlse.size(2) == N && tlse.is_contiguous(),
+                    "the saved lse came back with another device, dtype, shape or layout");
+    }
+
     torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override
     {
         if (!grads[0].defined()) return {Tensor(), Tensor(), Tensor()};
@@ -518,6 +533,7 @@ struct SparseAttentionBackward : public torch::autograd::Node {
         const Tensor tout = out.unpack(out_is_output ? shared_from_this() : nullptr);
         const Tensor tlse = lse.unpack(), tpacked = packed.unpack();
         at::NoGradGuard no_grad;
+        check_saved(grads[0], {&tq, &tk, &tv, &tout}, tlse);
         const c10::DeviceGuard guard(tq.device());
         Tensor dout;
         kernel_rows<1>({&grads[0]}, {&dout}, tq.scalar_type(), tq.size(3));

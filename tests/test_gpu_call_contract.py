@@ -186,3 +186,28 @@ def test_the_node_shows_what_it_saved(sa, dev, D):
     assert len(out.grad_fn.saved_tensors) == 6 and len(seen) == 6
     out.backward(do)
     assert len(seen) == 18
+
+
+@pytest.mark.parametrize("D", [60, 64])
+def test_what_saved_tensor_hooks_give_back_is_checked(sa, dev, D):
+    """The backward addresses what it saved by the gradient's extents: hooks that change device, type or shape are an
+    error, as they were for a function written in Python; hooks that give back an equal tensor are fine."""
+    q, k, v, do, mask = _problem(dev, D=D)
+
+    def grads(which, change):
+        leaves = [t.clone().requires_grad_(True) for t in (q, k, v)]
+        count = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: (len(count), count.append(0), t.detach().clone())[::2],
+                                                      lambda p: change(p[1]) if p[0] == which else p[1]):
+            out = sa.sparse_attention(*leaves, mask)
+        assert len(count) == 6
+        return torch.autograd.grad(out, leaves, do)
+
+    want = grads(-1, None)
+    for which in range(6):
+        for a, b in zip(want, grads(which, lambda t: t.cpu().to(dev))):
+            assert torch.equal(a, b)
+        for change in (torch.Tensor.cpu, torch.Tensor.double, lambda t: t[:, :, :-1], lambda t: t[:0], lambda t: t[0],
+                       lambda t: t[..., :-8] if t.size(-1) > 8 else t[..., :-1]):
+            with pytest.raises(RuntimeError):
+                grads(which, change)
