@@ -561,7 +561,7 @@ struct SparseAttentionBackward : public torch::autograd::Node {
         if (!direct)
             for (Tensor &g : d) {
                 if (g.size(3) != grad_D) g = g.narrow(3, 0, grad_D);
-                if (g.scalar_type() != grad_dtype) g = g.to(grad_dtype);
+                g = g.scalar_type() != grad_dtype ? g.to(grad_dtype) : g.contiguous();      // without the padding's gaps
             }
         return {d[0], d[1], d[2]};
     }

@@ -211,3 +211,13 @@ def test_what_saved_tensor_hooks_give_back_is_checked(sa, dev, D):
                        lambda t: t[..., :-8] if t.size(-1) > 8 else t[..., :-1]):
             with pytest.raises(RuntimeError):
                 grads(which, change)
+
+
+@pytest.mark.parametrize("D", [60, 64, 80])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_gradients_leave_no_gaps(sa, dev, D, dtype):
+    """Gradients of contiguous tensors are contiguous, also where the kernels compute with padded rows."""
+    q, k, v, do, mask = _problem(dev, D=D, dtype=dtype)
+    leaves = [t.clone().requires_grad_(True) for t in (q, k, v)]
+    for g in torch.autograd.grad(sa.sparse_attention(*leaves, mask), leaves, do):
+        assert g.is_contiguous() and g.view(-1).numel() == q.numel()
