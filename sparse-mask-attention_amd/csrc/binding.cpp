@@ -39,6 +39,7 @@
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_cpp_function.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <cmath>
 #include <mutex>
@@ -676,11 +677,11 @@ Call problem(const Tensor &q, const c10::optional<Tensor> &mask, const c10::opti
 // sparse_attention / sparse_attention_func of the Python layer.  `tile_map` is None, True (leave a map
 // behind for the backward) or a tensor.  None is returned, before anything has been done, for
 // arguments that the Python layer refuses or has to prepare first (a boolean mask shorter than one
-// 16-byte copy per row is packed there).
+// 16-byte copy per row is packed there), and while torch.jit traces, which sees nothing of a native call.
 c10::optional<Tensor> attention(const Tensor &q, const Tensor &k, const Tensor &v, const c10::optional<Tensor> &mask,
                                 const c10::optional<Tensor> &mask_packed, const py::object &tile_map, bool autograd)
 {
-    if (refusal(q, k, v, mask, mask_packed) != nullptr) return c10::nullopt;
+    if (refusal(q, k, v, mask, mask_packed) != nullptr || torch::jit::tracer::isTracing()) return c10::nullopt;
     const bool packed = mask_packed.has_value() && mask_packed->defined();
     const bool want_map = tile_map.ptr() == Py_True;
     const bool has_map = !want_map && !tile_map.is_none();

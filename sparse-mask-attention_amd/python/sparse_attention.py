@@ -121,7 +121,33 @@ class SparseAttentionFunction:
     @staticmethod
     def apply(q, k, v, mask_packed, mask_bool, scale, seq_len, tile_map=None):
         _require_ext(q)
+        if torch.jit.is_tracing():
+            return _TracedCall.apply(SparseAttentionFunction.apply, q, k, v, mask_packed, mask_bool, scale, seq_len, tile_map)
         return sparse_attn_cuda.attention_function(q, k, v, mask_packed, mask_bool, scale, tile_map)
+
+
+class _TracedCall(torch.autograd.Function):
+    """``call(q, k, v, *rest)`` as one operation of a ``torch.jit`` trace, which records operations of PyTorch and sees
+    nothing of a native call.  The call itself, made with the tracer off, and its native node do the work."""
+
+    @staticmethod
+    def forward(ctx, call, q, k, v, *rest):
+        state = torch._C._get_tracing_state()
+        torch._C._set_tracing_state(None)
+        try:
+            with torch.enable_grad():
+                ctx.inputs = [t.detach().requires_grad_(wanted) for t, wanted in zip((q, k, v), ctx.needs_input_grad[1:4])]
+                ctx.output = call(*ctx.inputs, *rest)
+            out = ctx.output.detach()
+        finally:
+            torch._C._set_tracing_state(state)
+        ctx.others = len(rest)
+        return out.clone()              # known to the tracer, and free to be changed in place
+
+    @staticmethod
+    def backward(ctx, dout):
+        grads = iter(torch.autograd.grad(ctx.output, [t for t in ctx.inputs if t.requires_grad], dout, retain_graph=True))
+        return (None, *(next(grads) if t.requires_grad else None for t in ctx.inputs), *[None] * ctx.others)
 
 
 def backward_recompute(q, k, v, out, lse, mask_bool, dout, scale):
@@ -178,6 +204,8 @@ def _declined(q, k, v, mask, mask_packed, tile_map, autograd):
     """What ``sparse_attn_cuda.attention`` did not take: the checks that say what is wrong with the
     arguments, and the one thing it leaves to be done beforehand, packing a mask of fewer than 16 columns
     (shorter than one copy of the kernel that reads the boolean mask)."""
+    if torch.jit.is_tracing():
+        return _TracedCall.apply(sparse_attention if autograd else sparse_attention_func, q, k, v, mask, mask_packed, tile_map)
     _check_inputs(q, k, v, mask, mask_packed)
     if autograd:
         assert tile_map is None or tile_map is True or mask_packed is not None, "a tile_map tensor belongs to a mask_packed"

@@ -221,3 +221,40 @@ def test_gradients_leave_no_gaps(sa, dev, D, dtype):
     leaves = [t.clone().requires_grad_(True) for t in (q, k, v)]
     for g in torch.autograd.grad(sa.sparse_attention(*leaves, mask), leaves, do):
         assert g.is_contiguous() and g.view(-1).numel() == q.numel()
+
+
+@pytest.mark.parametrize("D", [60, 64])
+@pytest.mark.parametrize("entry", ["sparse_attention", "sparse_attention_func", "apply", "packed"])
+@pytest.mark.filterwarnings("ignore:.*torch.jit.*:DeprecationWarning")
+def test_a_trace_records_the_call(sa, dev, D, entry):
+    """torch.jit.trace: the call is an operation of the trace, computed anew from the inputs and masks of each run."""
+
+    class Model(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.weight = torch.nn.Parameter(torch.linspace(0.5, 1.5, D).half())
+
+        def forward(self, x, k, v, mask):
+            q = x * self.weight
+            if entry == "apply":
+                return sa.SparseAttentionFunction.apply(q, k, v, None, mask, 0.125, x.shape[2]) * 2
+            if entry == "packed":
+                return sa.sparse_attention(q, k, v, None, mask) * 2
+            return getattr(sa, entry)(q, k, v, mask) * 2
+
+    model = Model().to(dev)
+    inputs = []
+    for seed in (1, 2):
+        q, k, v, do, mask = _problem(dev, D=D, seed=seed)
+        inputs.append((q, k, v, sa.pack_mask(mask) if entry == "packed" else mask))
+    for tracked in (True, False):
+        with torch.set_grad_enabled(tracked and entry != "sparse_attention_func"):
+            traced = torch.jit.trace(model, inputs[0], check_trace=False)
+            for args in reversed(inputs):
+                got, want = traced(*args), model(*args)
+                assert torch.equal(got, want)
+                if want.requires_grad:
+                    a, b = (torch.autograd.grad(o, model.weight, do)[0] for o in (got, want))
+                    assert torch.equal(a, b)
+    with pytest.raises(AssertionError):
+        torch.jit.trace(lambda x, m: sa.sparse_attention(x, x, x, m), (q, mask[..., :-1]), check_trace=False)
