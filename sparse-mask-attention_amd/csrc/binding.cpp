@@ -586,7 +586,8 @@ Tensor run_call(const Tensor &q, const Tensor &k, const Tensor &v, Call &c, bool
     std::shared_ptr<SparseAttentionBackward> node;
     if (tracked) {
         refuse_tangents(q, k, v);
-        node = std::make_shared<SparseAttentionBackward>();
+        // freed node by node like PyTorch's own, not by recursion along a chain of them
+        node = std::shared_ptr<SparseAttentionBackward>(new SparseAttentionBackward(), torch::autograd::deleteNode);
         node->set_next_edges(torch::autograd::collect_next_edges(q, k, v));
     }
     const c10::DeviceGuard guard(q.device());

@@ -2,6 +2,7 @@
 launched, and limits lie where the documentation puts them."""
 import importlib
 import sys
+import threading
 
 import pytest
 import torch
@@ -258,3 +259,22 @@ def test_a_trace_records_the_call(sa, dev, D, entry):
                     assert torch.equal(a, b)
     with pytest.raises(AssertionError):
         torch.jit.trace(lambda x, m: sa.sparse_attention(x, x, x, m), (q, mask[..., :-1]), check_trace=False)
+
+
+def test_a_long_chain_of_calls_is_freed(sa, dev):
+    """Each call's query is the output of the one before: the graph is one node after the other.  Freed by recursion,
+    20000 of them take more than the 256 KiB of stack that they are freed on here."""
+    q = torch.randn(1, 1, 16, 32, device=dev, dtype=torch.float16)
+    mask = torch.ones(1, 1, 16, 16, dtype=torch.bool, device=dev)
+    leaf = q.clone().requires_grad_(True)
+    chain = [leaf]
+    for _ in range(20000):
+        chain[0] = sa.sparse_attention(chain[0], q, q, mask)
+    before = threading.stack_size(256 * 1024)
+    try:
+        thread = threading.Thread(target=chain.clear)
+        thread.start()
+    finally:
+        threading.stack_size(before)
+    thread.join()
+    assert torch.equal(sa.sparse_attention(leaf, q, q, mask), sa.sparse_attention_func(q, q, q, mask))
