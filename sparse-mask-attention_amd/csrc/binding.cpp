@@ -691,15 +691,15 @@ c10::optional<Tensor> attention(const Tensor &q, const Tensor &k, const Tensor &
     return run_call(q, k, v, c, want_map, autograd);
 }
 
-// SparseAttentionFunction.apply of the Python layer: the same with the scale given, for q, k and v of 16 bits (nothing
-// is converted), whose wrong arguments are errors.  Without a packed mask, a tile map given as a tensor is not used.
+// SparseAttentionFunction.apply of the Python layer: the same with the scale given, for q, k and v of one type, whose
+// wrong arguments are errors.  Without a packed mask, a tile map given as a tensor is not used.
 Tensor attention_function(const Tensor &q, const Tensor &k, const Tensor &v, const c10::optional<Tensor> &mask_packed,
                           const c10::optional<Tensor> &mask, double scale, const py::object &tile_map)
 {
     const char *const why = refusal(q, k, v, mask, mask_packed);
     TORCH_CHECK(why == nullptr, why);
     refuse_tangents(q, k, v);
-    TORCH_CHECK(q.scalar_type() != at::kFloat, "Unsupported dtype, need BF16 or FP16");
+    TORCH_CHECK(k.scalar_type() == q.scalar_type() && v.scalar_type() == q.scalar_type(), "q, k, v must have the same dtype");
     const bool packed = mask_packed.has_value() && mask_packed->defined();
     const bool want_map = tile_map.ptr() == Py_True;
     TORCH_CHECK(!(packed && want_map), "with mask_packed, pass the result of tile_map(mask_packed)");

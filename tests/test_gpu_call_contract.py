@@ -78,10 +78,11 @@ def test_the_function_behind_the_api_refuses_what_it_cannot_address(sa, dev):
     wrong += [dict(packed=p) for p in (packed[:, :, :-1], packed[..., :-1], packed[0], packed.float(), packed.long(), packed.cpu(),
                                        packed.expand(2, 2, N, 3).transpose(2, 3).contiguous().transpose(2, 3),
                                        packed[:1].expand(3, 2, N, 3))]
-    wrong += [dict(q=t(q), k=t(k), v=t(v)) for t in (torch.Tensor.double, torch.Tensor.float, torch.Tensor.int, torch.Tensor.cpu,
+    wrong += [dict(q=t(q), k=t(k), v=t(v)) for t in (torch.Tensor.double, torch.Tensor.int, torch.Tensor.cpu,
                                                      lambda x: x[0], lambda x: torch.cat([x, x, x], -1))]
     wrong += [{name: t(x)} for name, x in (("k", k), ("v", v))
               for t in (torch.Tensor.float, torch.Tensor.bfloat16, torch.Tensor.cpu, lambda x: x[:, :, :-1], lambda x: x[..., :32])]
+    wrong += [dict(q=q.float(), k=k.float()), dict(q=q.float(), v=v.float()), dict(q=q.float(), k=k.float(), v=v.double())]
     wrong += [dict(packed=packed, tile_map=t) for t in (True, tm[:, :, :1], tm.cpu(), tm.float(), 3)]
     for args in wrong:
         with pytest.raises(RuntimeError):
@@ -89,6 +90,8 @@ def test_the_function_behind_the_api_refuses_what_it_cannot_address(sa, dev):
     want = sa.sparse_attention_func(q, k, v, mask)
     for args in ({}, dict(mask=mask, tile_map=True), dict(mask=None, packed=packed), dict(mask=None, packed=packed, tile_map=tm)):
         assert torch.equal(call(**args), want)
+    wide = [t.float() for t in (q, k, v)]
+    assert torch.equal(call(*wide), sa.sparse_attention_func(*wide, mask))
 
 
 def test_a_shared_mask_longer_than_a_tile_map_allows(sa, dev):
