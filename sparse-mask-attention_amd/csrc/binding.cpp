@@ -153,6 +153,18 @@ void forward(const torch::Tensor &q, const torch::Tensor &k, const torch::Tensor
     check_status(st, "sma_attn_fwd_map_strided");
 }
 
+// Whether the kernels can address t as it is: contiguous last dimension, the strides of the others
+// non-negative multiples of 8 elements, 16-byte aligned storage.
+bool addressable(const torch::Tensor &t)
+{
+    if (t.dim() != 4) return false;
+    if (t.stride(3) != 1 && t.size(3) != 1) return false;
+    if (reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 != 0) return false;
+    for (int d = 0; d < 3; ++d)
+        if (t.size(d) > 1 && (t.stride(d) < 0 || t.stride(d) % 8 != 0)) return false;
+    return true;
+}
+
 // Limits of sma_attn_fwd_bool_mask, so that callers can choose between it and pack_mask + forward
 // without provoking an error: q, k, v with contiguous rows and strides that are multiples of 8
 // elements, head dim 32, 64 or 128, 16 <= N < 46341, a contiguous bool mask [1|B, 1|H, N, N].
@@ -162,14 +174,8 @@ bool bool_mask_supported(const torch::Tensor &q, const torch::Tensor &k, const t
     if (!q.is_cuda() || q.dim() != 4 || mask.dim() != 4) return false;
     const int64_t B = q.size(0), H = q.size(1), N = q.size(2), D = q.size(3);
     if (!(D == 32 || D == 64 || D == 128) || N < 16 || N * N >= (int64_t(1) << 31)) return false;
-    // q, k, v as the strided entry points take them: rows contiguous, other strides multiples of 8
-    // elements, 16-byte aligned storage
-    for (const torch::Tensor *t : {&q, &k, &v}) {
-        if (t->dim() != 4 || t->sizes() != q.sizes() || (t->stride(3) != 1 && t->size(3) != 1)) return false;
-        if (reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 != 0) return false;
-        for (int d = 0; d < 3; ++d)
-            if (t->size(d) > 1 && (t->stride(d) < 0 || t->stride(d) % 8 != 0)) return false;
-    }
+    for (const torch::Tensor *t : {&q, &k, &v})
+        if (t->sizes() != q.sizes() || !addressable(*t)) return false;
     if (mask.scalar_type() != at::kBool || !mask.is_contiguous() || mask.device() != q.device()) return false;
     if (!((mask.size(0) == B || mask.size(0) == 1) && (mask.size(1) == H || mask.size(1) == 1) &&
           mask.size(2) == N && mask.size(3) == N))
@@ -337,17 +343,6 @@ torch::Tensor tile_map(const torch::Tensor &mask_packed)
 // explains why.
 
 using torch::Tensor;
-
-// Whether the kernels can address t as it is: contiguous last dimension, the strides of the others
-// non-negative multiples of 8 elements, 16-byte aligned storage.
-bool addressable(const Tensor &t)
-{
-    if (t.stride(3) != 1 && t.size(3) != 1) return false;
-    if (reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 != 0) return false;
-    for (int d = 0; d < 3; ++d)
-        if (t.size(d) > 1 && (t.stride(d) < 0 || t.stride(d) % 8 != 0)) return false;
-    return true;
-}
 
 // Head dim of the kernels' tensors for one of the caller's: the next multiple of 8 (16 bytes).
 int64_t padded_head_dim(int64_t D) { return (D + 7) / 8 * 8; }
@@ -780,6 +775,8 @@ PYBIND11_MODULE(sparse_attn_cuda, m)
     m.def("bool_mask_supported", &bool_mask_supported,
           "Whether forward_bool_mask applies to these tensors (else use pack_mask + forward)", py::arg("q"),
           py::arg("k"), py::arg("v"), py::arg("mask"));
+    m.def("addressable", &addressable,
+          "Whether the kernels take a [B, H, N, D] tensor as it is (else a contiguous copy of it)", py::arg("t"));
     m.def("pack_mask", &pack_mask, "Pack a bool mask into uint32 words (returned as int32)",
           py::arg("mask"));
     m.def("attention", &attention, "One call of the Python layer; None if its arguments need the checks made there",

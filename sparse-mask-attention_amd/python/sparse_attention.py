@@ -73,10 +73,9 @@ except ImportError as exc:  # the API stays importable; any compute call reports
 
 def _rows(t: torch.Tensor) -> torch.Tensor:
     """t itself if the kernels can address it (contiguous last dimension, the strides of the other
-    dimensions multiples of 8 elements, 16-byte aligned storage), else a contiguous copy."""
-    ok = (t.stride(-1) == 1 or t.size(-1) == 1) and t.data_ptr() % 16 == 0 and all(
-        st % 8 == 0 for st, n in zip(t.stride()[:-1], t.shape[:-1]) if n > 1)
-    return t if ok else t.contiguous()
+    dimensions multiples of 8 elements, 16-byte aligned storage), else a contiguous copy: what a call does
+    with q, k and v, by the rule that it goes by."""
+    return t if sparse_attn_cuda.addressable(t) else t.contiguous()
 
 
 def _require_ext(t: torch.Tensor) -> None:

@@ -227,3 +227,24 @@ def test_bench_passes_on_recorded_traffic_only_for_the_sources_it_was_recorded_f
     assert bench.measured_traffic("C3", "pack_mask_kernel") is None            # no summary
     (csrc / "pack_mask.hip").write_text("// changed\n")
     assert bench.measured_traffic("C2", "pack_mask_kernel") is None            # recorded for other code
+
+
+@pytest.mark.parametrize("view, ok", [
+    (lambda q: q, True),
+    (lambda q: q.transpose(1, 2), True),
+    (lambda q: q[:, :, ::2], True),
+    (lambda q: q[..., :60], True),                       # rows stay 64 apart
+    (lambda q: q[:1, :1, :1].expand(2, 3, 10, 64), True),
+    (lambda q: q[..., 8:16], True),
+    (lambda q: q[..., 4:12], False),                     # 8 bytes into a row
+    (lambda q: q[..., ::2], False),
+    (lambda q: q.transpose(2, 3), False),
+    (lambda q: q[..., :60].contiguous(), False),         # rows 60 apart
+    (lambda q: q[..., :60].contiguous()[:1, :1, :1], True),
+    (lambda q: q[0], False),
+])
+def test_which_tensors_the_kernels_take_as_they_are(view, ok):
+    sa = sys.modules["python.sparse_attention"]
+    t = view(torch.zeros(2, 3, 10, 64, dtype=torch.float16))
+    assert sa.sparse_attn_cuda.addressable(t) == ok
+    assert (sa._rows(t) is t) == (ok or t.is_contiguous())
