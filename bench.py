@@ -110,6 +110,7 @@ KERNEL_SOURCES = {
     "pack_mask_kernel": ("pack_mask.hip", "sma_internal.h"),
     "attn_bwd_dq_kernel": ("attn_bwd.hip", "attn_common.h", "sma_internal.h"),
     "attn_bwd_dkv_kernel": ("attn_bwd.hip", "attn_common.h", "sma_internal.h"),
+    "attn_bwd_short_kernel": ("attn_bwd.hip", "attn_common.h", "sma_internal.h"),
 }
 
 
@@ -371,6 +372,8 @@ def main():
     del mp
     attn_tflops = w.dense_flops / (attn_ms * 1e-3) / 1e12
     pack_gbps = w.pack_bytes / (pack_ms * 1e-3) / 1e9
+    # the workloads of at most 256 keys run the backward that holds a whole head in one work-group
+    bwd_kernels = ("attn_bwd_short_kernel",) if w.N <= 256 else ("attn_bwd_dq_kernel", "attn_bwd_dkv_kernel")
     result = {
         "metric": "dense_equiv_tflops_sparse_attention_fwd_incl_pack_mask",
         "value": round(value, 3),
@@ -422,10 +425,10 @@ def main():
                           "frac_cold": round(w.pack_bytes / (pack_cold_ms * 1e-3) / 1e9 / harness.MI355X_HBM_GBPS, 4),
                           "cache_note": "frac: same mask every launch (last-level cache warm); frac_cold: HBM",
                           "traffic": measured_traffic(w.name, "pack_mask_kernel"), "algorithmic_bytes": w.pack_bytes},
-        "roofline_bwd": {"kernel": "attn_bwd_dq_kernel + attn_bwd_dkv_kernel", "bound": "mfma",
+        "roofline_bwd": {"kernel": " + ".join(bwd_kernels), "bound": "mfma",
                          "achieved": round(bwd_tflops, 2), "peak": harness.MI355X_MFMA_F16_TFLOPS,
                          "unit": "TFLOP/s", "frac": round(bwd_tflops / harness.MI355X_MFMA_F16_TFLOPS, 4),
-                         "traffic": measured_traffic(w.name, "attn_bwd_dq_kernel", "attn_bwd_dkv_kernel"), "algorithmic_bytes": w.bwd_bytes},
+                         "traffic": measured_traffic(w.name, *bwd_kernels), "algorithmic_bytes": w.bwd_bytes},
     }
 
     result["roofline_attn"].update(roofline_ceiling(w.dense_flops, w.attn_bytes, attn_tflops))

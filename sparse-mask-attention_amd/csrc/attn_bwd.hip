@@ -365,7 +365,7 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_bwd_dq_kerne
 //   128  the accumulators of dK and dV take 128 registers; both gradients in one kernel form S once where a kernel
 //        for each formed it twice: 2783 -> 2032 us on 4 x 32 heads, N = 4096 (1.08 PFLOP/s over four products)
 //   64   166 registers instead of 198: three work-groups on a CU instead of two, where the grid has them (see the
-//        launcher): 16 x 12 heads, N = 512: 41.0 -> 37.3 us (691 TFLOP/s)
+//        launcher): 16 x 12 heads, N = 512, this kernel alone on warm inputs: 41.0 -> 37.3 us (691 TFLOP/s)
 template <int HDIM, int NW, bool VLDS> struct DkvCfg {
     static constexpr int NH = HDIM > 64 ? 2 : 1;
     static constexpr int STAGE_BYTES = 2 * NH * TILE_BYTES;
@@ -612,8 +612,9 @@ __global__ __launch_bounds__(64 * NW, HDIM == 128 ? NW / 4 : VLDS ? 3 : 2) void 
 // N <= 32 NW keys and head dim <= 64: one work-group holds a whole head, a wavefront 32 of its keys, as in the dK/dV
 // kernel.  S, dP and the exponentials are formed once (the two kernels form them twice: 7 products instead of 5) and
 // q, k, v, dO come from memory once.  What is bound by memory and by the length of a work-group's prologue gains most:
-// 64 x 16 heads, N = 256, D = 64: 104 us for the two kernels, 90 us here (3.6 TB/s of what has to move; one work-group
-// of 8 wavefronts on a CU, whose loads nothing else hides), 1024 heads, N = 128: 41.7 -> 33.0 us.
+// forward and backward on inputs that no cache holds, the two kernels -> this one: 1024 heads, N = 128, D = 64: 65.0 ->
+// 56.1 us.  With more keys a CU holds one work-group of 8 wavefronts, whose loads nothing else hides, and the gain goes with
+// the number of rounds: N = 256, D = 64, 256 heads: 46.0 -> 39.9 us, 512: 84.9 -> 75.7, 1024: 150.6 -> 146.0, 2048: 297 -> 297.
 //   K            in LDS too, for dQ
 //   scaled Q     (the operand of S, rounded as the forward rounds it, so that the probabilities fit its lse) beside the
 //                Q that dK needs: each wavefront scales the rows it has copied
@@ -923,11 +924,13 @@ void launch_pair(hipStream_t stream, const AttnBwdArgs &args)
 {
     AttnBwdArgs a = args;
     if constexpr (HDIM <= 64) {
-        // A whole head in one work-group (see attn_bwd_short_kernel).  Up to 128 keys always: 4 heads, N = 64, D = 32:
-        // 7.8 -> 5.3 us, 1024 heads, N = 128, D = 64: 41.7 -> 33.0 us.  With more keys a CU holds only one of the
-        // eight-wavefront work-groups, and its time is that of its whole rounds: for head dims above 32 where the last
-        // round is at least three quarters full (256 heads, N = 256, D = 64: 28.2 -> 24.2 us, 1024: 104 -> 90 us; but
-        // 384: 40.2 -> 41.7 us, and D = 32, 1024: 57.8 -> 61.7 us).
+        // A whole head in one work-group (see attn_bwd_short_kernel).  Up to 128 keys always: forward + backward, inputs from
+        // memory, 4 heads, N = 64, D = 32: 11.7 -> 9.0 us, 2048 heads, N = 128, D = 64: 118.6 -> 107.5 us, 4 to 30 % between.
+        // With more keys a CU holds only one of the eight-wavefront work-groups, and its time is that of its whole
+        // rounds: for head dims above 32 where the last round is at least three quarters full.  N = 256, D = 64, the same
+        // measure: 192 heads 40.5 -> 35.4 us, 256: 46.0 -> 39.9, 1024: 150.6 -> 146.0, 2048: 297 either way (causal
+        // mask: 274 -> 279); half a round, 384 heads, would go 61.9 -> 63.4.  (D = 32, 1024 heads, the backward alone
+        // on warm inputs: 57.8 -> 61.7 us.)
         const long long cus = compute_units(), last = cus > 0 ? a.BH % cus : 0;
         if (a.N <= 128 || (a.N <= 256 && HDIM > 32 && (last == 0 || 4 * last >= 3 * cus))) {
             const dim3 grid((unsigned)a.BH);
@@ -960,8 +963,11 @@ void launch_pair(hipStream_t stream, const AttnBwdArgs &args)
         else dkv(four{}, std::true_type{});
     } else if (HDIM == 64 && groups > 2 * cus && (2 * groups <= 7 * cus || groups > 4 * cus)) {
         // Three work-groups on a CU.  A grid that two of them on each CU hold does not need the third and pays for the reads
-        // (whole backward, 128 heads, N = 448: 39.0 against 38.1 us), two full rounds of two are as fast as one and a
-        // third of three (64 heads, N = 2048: 277 against 273 us); beyond, 5 to 9 % (256 heads, N = 300: 41.6 against 45.4).
+        // (128 heads, N = 448, the backward alone: 39.0 against 38.1 us), and from 3.5 to 4 per CU two full rounds of two
+        // are as fast as one and a third of three.  Forward + backward, inputs from memory, two -> three: 2 to 3 per CU gain 2.5 to
+        // 6.5 % (172 heads, N = 300: 59.3 -> 55.6 us; 192, N = 512: 95.6 -> 92.5; 48, N = 2048: 296 -> 288), 3 to 3.5 nothing (224,
+        // N = 512: 117.6 either way) to 1.2 % the other way (56, N = 2048: 374.6 -> 379.3), beyond 4 1 to 3.5 % (400, N = 300:
+        // 100.6 -> 97.2; 96, N = 2048: 570 -> 561).
         dkv(four{}, std::integral_constant<bool, HDIM == 64>{});
     } else {
         dkv(four{}, std::false_type{});
