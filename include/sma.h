@@ -141,8 +141,9 @@ int sma_attn_fwd_map(const void *q, const void *k, const void *v, const uint32_t
  *   delta_ws            float [B,H,N] workspace owned by the caller; holds sum_d dout*out per query
  *                       row on return (the library never allocates)
  *
- * Two launches on `stream` (dq, then dk and dv); no atomics, results are
- * bit-reproducible.
+ * One or two launches on `stream`: sequences of up to 128 keys with D up to 64, and many of up to 256 with
+ * D above 32, run in one kernel that holds a whole head in a work-group; others in two (dq, then dk and dv).
+ * No atomics, results are bit-reproducible.
  *
  * Replaces: void sparse_attention_bwd_bf16(const SparseAttentionParams&, const void* dout,
  *           void* dq, void* dk, void* dv, cudaStream_t), declared csrc/sparse_attention.h:57-64 and
@@ -153,9 +154,9 @@ int sma_attn_bwd(const void *dout, const void *q, const void *k, const void *v, 
                  const float *lse, const uint32_t *mask_packed, void *dq, void *dk, void *dv,
                  float *delta_ws, int B, int H, int N, int D, float scale, int dtype, void *stream);
 
-/* sma_attn_bwd with a tile map (see sma_tile_map) of the same packed mask: both kernels visit only
- * the 64 x 64 blocks in which the mask keeps something.  tile_map == NULL is sma_attn_bwd; the
- * gradients are the same bit for bit.  sma_attn_bwd_map_strided is the strided form (map
+/* sma_attn_bwd with a tile map (see sma_tile_map) of the same packed mask: the two kernels visit only
+ * the 64 x 64 blocks in which the mask keeps something (the one for short sequences has no use for the map
+ * and does not read it).  tile_map == NULL is sma_attn_bwd; the gradients are the same bit for bit.  sma_attn_bwd_map_strided is the strided form (map
  * contiguous [Bm,Hm,T,2,TW] with the mask's own Bm, Hm).
  */
 int sma_attn_bwd_map(const void *dout, const void *q, const void *k, const void *v, const void *out,
@@ -166,7 +167,7 @@ int sma_attn_bwd_map(const void *dout, const void *q, const void *k, const void 
 
 /* sma_attn_bwd without the workspace argument, for callers that cannot allocate device memory at
  * all (code running under HIP graph capture, tight serving loops, harnesses that forbid
- * hipMalloc): the per-row sums that the two kernels exchange live in a fixed array inside the
+ * hipMalloc): the per-row sums (delta_ws of sma_attn_bwd) live in a fixed array inside the
  * library's device image (SMA_STATIC_WS_ROWS floats = 4 MiB, held by every GPU the library has
  * been called on until the process ends).  Arguments and results are exactly those of
  * sma_attn_bwd.  The call allocates nothing; B*H*N > SMA_STATIC_WS_ROWS returns SMA_ERR_WORKSPACE

@@ -20,11 +20,14 @@
 //       everything python/sparse_attention.py does for one call - conversions, padding, allocation,
 //       launches and the autograd node - without returning to Python in between; None when an
 //       argument is not what the Python layer's own checks demand, which then say what is wrong)
+//   attention_function(q, k, v, mask_packed, mask, scale, tile_map) -> Tensor   (SparseAttentionFunction.apply: the same
+//       with the scale given; wrong arguments raise)
+//   addressable(t) -> bool   (whether the kernels take a tensor as it is)
 //
 // Differences, all on the safe side: `lse` may be None (the reference's own inference wrapper
 // passes None, python/sparse_attention.py:170-171); every tensor argument is checked (device,
-// dtype, shape, layout, head_dim 32, 64 or 128) instead of only `q`; launches go to the current HIP
-// stream of q's device under a device guard; a failed launch raises RuntimeError.
+// dtype, shape, layout, head_dim 32, 64 or 128, or any up to 128 in `attention` and
+// `attention_function`) instead of only `q`; launches go to the current HIP stream of q's device under a device guard; a failed launch raises RuntimeError.
 // q, k, v, out and the gradients need not be contiguous: any view whose last dimension is
 // contiguous and whose other strides are multiples of 8 elements is passed on with its strides
 // (the reference reserves such strides, csrc/sparse_attention.h:30-33, and ignores them), and

@@ -1,17 +1,17 @@
-"""Sparse-mask attention: the user-facing Python API, unchanged from the reference.
+"""Sparse-mask attention: the user-facing Python API, with the reference's functions and arguments.
 
 Mirrors ``python/sparse_attention.py`` of the reference (line numbers below refer to it):
 
 * ``sparse_attention(q, k, v, mask)``       :120-154  autograd-aware entry point
 * ``sparse_attention_func(q, k, v, mask)``  :157-177  inference-only variant (no LSE, no graph)
 * ``pack_mask(mask)``                       :184-201  bool [B,H,N,N] -> int32 [B,H,N,ceil(N/32)]
-* ``SparseAttentionFunction``               :49-113   the autograd.Function behind the first
+* ``SparseAttentionFunction``               :49-113   what ``sparse_attention`` differentiates, with the scale given
 * ``sparse_attention_ref``                  :24-42    the plain-PyTorch statement of the operator
 * ``generate_random_sparse_mask``           :204-211
 
-``q, k, v`` are ``[B, H, N, D]`` fp16 / bf16 tensors on an MI355X, D = 64 as in the reference, 32 or
-128 (other head dims up to 128 are zero-padded to the next of these, see below) (fp32 inputs are computed in
-bf16 and returned as fp32, as in the reference :140-142,151-152); ``mask`` is a bool
+``q, k, v`` are ``[B, H, N, D]`` fp16 / bf16 tensors on an MI355X, D = 64 as in the reference or any other up to
+128 (multiples of 8 as they are, others zero-padded to the next multiple of 8, see below); fp32 inputs are computed in
+bf16 and returned as fp32, as in the reference :140-142,151-152.  ``mask`` is a bool
 ``[B, H, N, N]`` tensor, True = attend.  Query rows that attend to nothing give zeros.
 
 What differs from the reference, on purpose:
@@ -45,9 +45,12 @@ What differs from the reference, on purpose:
   Worth it for a mask that is used many times; ``tile_map`` returns None when too few visits would
   disappear for the walk to pay.
 * ``.backward()`` works.  The reference calls a ``sparse_attn_cuda.backward`` that was never
-  written (:91-94); here that function exists (two HIP kernels, dQ and dK/dV, from the saved
-  log-sum-exp and the packed mask).  ``backward_recompute`` states the same gradients with PyTorch
+  written (:91-94); here that function exists (HIP kernels, from the saved log-sum-exp and the packed mask: dQ and
+  dK/dV, or one for short sequences).  ``backward_recompute`` states the same gradients with PyTorch
   ops (the reference's own formulas, :97-111) for cross-checks.
+* ``SparseAttentionFunction`` has ``apply`` and nothing else of a ``torch.autograd.Function``: its node is native.  The node
+  shows ``saved_tensors``, ``scale`` and ``tile_map``.  Forward-mode AD is refused (``NotImplementedError``), and a
+  ``torch.jit`` trace records each call as one operation.
 """
 from __future__ import annotations
 
@@ -106,10 +109,11 @@ def sparse_attention_ref(q, k, v, mask):
 # ----------------------------------------------------------------------------------------------
 
 class SparseAttentionFunction:
-    """forward = fused HIP kernel (saves LSE); backward = the HIP dQ and dK/dV kernels.
+    """forward = fused HIP kernel (saves LSE); backward = the HIP backward kernels.
 
     The autograd node itself is native (csrc/binding.cpp, SparseAttentionBackward): in a small training
-    step the host is what takes time, and a node written in Python made it twice as long.
+    step the host is what takes time, and a node written in Python made it twice as long.  Tensors are checked as
+    ``sparse_attention`` checks them, and q, k and v have one type; what is wrong raises ``RuntimeError``.
 
     ``mask_packed`` may be None: the mask is then read as it is by the one-launch forward, which
     leaves the packed words the backward uses (and, with ``tile_map=True``, the mask's tile map) as
@@ -226,8 +230,8 @@ def _declined(q, k, v, mask, mask_packed, tile_map, autograd):
 def sparse_attention(q, k, v, mask, mask_packed=None, tile_map=None):
     """Masked attention with autograd support.
 
-    q, k, v: ``[B, H, N, D]`` (D = 32, 64 or 128; other D <= 128 are zero-padded) bf16 / fp16 / fp32;  mask: bool ``[B, H, N, N]``, True = keep
-    (a leading extent of 1 shares the mask between batch entries / heads).
+    q, k, v: ``[B, H, N, D]`` (D <= 128; off multiples of 8 at the price of padding copies) bf16 / fp16 / fp32;
+    mask: bool ``[B, H, N, N]``, True = keep (a leading extent of 1 shares the mask between batch entries / heads).
     Returns a tensor of q's shape and original dtype.
 
     ``mask_packed`` (optional, not in the reference): the result of ``pack_mask(mask)`` kept from an
