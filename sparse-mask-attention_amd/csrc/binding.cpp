@@ -27,7 +27,8 @@
 // Differences, all on the safe side: `lse` may be None (the reference's own inference wrapper
 // passes None, python/sparse_attention.py:170-171); every tensor argument is checked (device,
 // dtype, shape, layout, head_dim 32, 64 or 128, or any up to 128 in `attention` and
-// `attention_function`) instead of only `q`; launches go to the current HIP stream of q's device under a device guard; a failed launch raises RuntimeError.
+// `attention_function`) instead of only `q`; launches go to the current HIP stream of q's device
+// under a device guard; a failed launch raises RuntimeError.
 // q, k, v, out and the gradients need not be contiguous: any view whose last dimension is
 // contiguous and whose other strides are multiples of 8 elements is passed on with its strides
 // (the reference reserves such strides, csrc/sparse_attention.h:30-33, and ignores them), and
