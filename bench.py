@@ -108,9 +108,9 @@ KERNEL_SOURCES = {
     "attn_fwd_kernel": ("attn_fwd.hip", "attn_common.h", "sma_internal.h"),
     "attn_fwd_bool_mask_kernel": ("attn_fwd.hip", "attn_common.h", "sma_internal.h"),
     "pack_mask_kernel": ("pack_mask.hip", "sma_internal.h"),
-    "attn_bwd_dq_kernel": ("attn_bwd.hip", "attn_common.h", "sma_internal.h"),
-    "attn_bwd_dkv_kernel": ("attn_bwd.hip", "attn_common.h", "sma_internal.h"),
-    "attn_bwd_short_kernel": ("attn_bwd.hip", "attn_common.h", "sma_internal.h"),
+    "attn_bwd_dq_kernel": ("attn_bwd.hip", "attn_bwd_common.h", "attn_common.h", "sma_internal.h"),
+    "attn_bwd_dkv_kernel": ("attn_bwd.hip", "attn_bwd_common.h", "attn_common.h", "sma_internal.h"),
+    "attn_bwd_head_kernel": ("attn_bwd_head.hip", "attn_bwd_common.h", "attn_common.h", "sma_internal.h"),
 }
 
 
@@ -372,8 +372,8 @@ def main():
     del mp
     attn_tflops = w.dense_flops / (attn_ms * 1e-3) / 1e12
     pack_gbps = w.pack_bytes / (pack_ms * 1e-3) / 1e9
-    # the workloads of at most 256 keys run the backward that holds a whole head in one work-group
-    bwd_kernels = ("attn_bwd_short_kernel",) if w.N <= 256 else ("attn_bwd_dq_kernel", "attn_bwd_dkv_kernel")
+    # the workloads of at most 512 keys run the backward that holds a whole head in one work-group
+    bwd_kernels = ("attn_bwd_head_kernel",) if w.N <= 512 else ("attn_bwd_dq_kernel", "attn_bwd_dkv_kernel")
     result = {
         "metric": "dense_equiv_tflops_sparse_attention_fwd_incl_pack_mask",
         "value": round(value, 3),

@@ -8,8 +8,8 @@
 //     dV = P^T dO          dP = dO V^T          delta_i = sum_d dO_id O_id  (= sum_j P_ij dP_ij)
 //     dS = P o (dP - delta) * scale             dQ = dS K            dK = dS^T Q
 //
-// No atomics, bit-reproducible.  Short sequences take attn_bwd_short_kernel (one launch, described there), others
-// two kernels:
+// No atomics, bit-reproducible.  Sequences of which a work-group holds a whole head take attn_bwd_head.hip's kernel, others
+// two:
 //
 //   attn_bwd_dq_kernel   one work-group = 128 query rows, walks the key tiles exactly like the
 //                        forward: S^T = K Q^T and dP^T = V dO^T on the MFMA (lane = query row, so
@@ -37,7 +37,7 @@
 // every LDS row with copies of the row's last 16 bytes, which are never read;
 // contractions over the head dim take two MFMA steps and the outputs have one 32-column block.  Head dim 96
 // is 128 with such a half tile as its second half: six steps, three blocks.
-#include "attn_common.h"
+#include "attn_bwd_common.h"
 
 namespace sma {
 namespace {
@@ -49,7 +49,6 @@ constexpr int NTHREADS = 256;
 constexpr int TILE_BYTES = BN * HD * 2;
 constexpr int NSTAGE = 2;
 constexpr int AUX_BYTES = 2048;                             // small per-tile data of a stage
-constexpr float LOG2E = 1.4426950408889634f;
 
 // LDS map (bytes) for head dim 64 * NH: a stage holds the NH column halves of the first streamed
 // matrix, then those of the second.
@@ -111,65 +110,6 @@ __device__ __forceinline__ void zero_tile_tail(uint32_t dst, int parts, int r0, 
             for (int part = 0; part < parts; ++part)
                 *(LDS_PTR(u32x4))(uintptr_t)(dst + part * TILE_BYTES + wave * 2048 + j * 1024 + lane * 16) = z;
         }
-}
-
-// Per-lane LDS read offsets inside a tile (add the tile's base and 4096 per block of 32 rows).
-//   rowaddr[s]       ds_read_b128: row l32, columns 16s + 8hh .. +7          (A operand, k-step s)
-//   traddr[dblk][x]  ds_read_b64_tr_b16: rows 8x + 4hh + (i >> 2) (+16u), columns 32dblk + 16G +
-//                    4(i & 3) .. +3, i = lane % 16, G = (lane % 32) / 16     (A operand = tile^T)
-struct TileRead {
-    uint32_t rowaddr[4];
-    uint32_t traddr[2][2];
-};
-__device__ __forceinline__ TileRead make_tile_read(int lane)
-{
-    TileRead r;
-    const int l32 = lane & 31, hh = lane >> 5;
-    const int fk = bitrev3((l32 >> 1) & 7);
-#pragma unroll
-    for (int s = 0; s < 4; ++s) r.rowaddr[s] = (uint32_t)(l32 * 128 + (((2 * s + hh) ^ fk) << 4));
-    const int i16 = lane & 15, G = l32 >> 4;
-    const int r3 = 4 * hh + (i16 >> 2);
-#pragma unroll
-    for (int x = 0; x < 2; ++x) {
-        const int row = 8 * x + r3;
-        const int fr = bitrev3((row >> 1) & 7);
-#pragma unroll
-        for (int dblk = 0; dblk < 2; ++dblk) {
-            const int chunk = 4 * dblk + 2 * G + ((i16 & 3) >> 1);
-            r.traddr[dblk][x] = (uint32_t)(row * 128 + ((chunk ^ fr) << 4) + ((i16 & 1) << 3));
-        }
-    }
-    return r;
-}
-
-// The fragments of one row of a matrix (row stride sn elements, D columns): 8 elements at columns
-// 16s + 8hh, zeros beyond the row.  `full` (D is the kernel's own head dim) is wave-uniform: the common
-// case loads straight.
-template <int KS>
-__device__ __forceinline__ void load_row(u32x4 (&f)[KS], const uint16_t *mat, uint32_t sn, int row, int hh, int D)
-{
-    const uint16_t *p = mat + (size_t)row * sn + 8 * hh;
-    if (D == 16 * KS) {
-#pragma unroll
-        for (int s = 0; s < KS; ++s) f[s] = *reinterpret_cast<const u32x4 *>(p + 16 * s);
-    } else {
-#pragma unroll
-        for (int s = 0; s < KS; ++s)
-            f[s] = 16 * s + 8 * hh < D ? *reinterpret_cast<const u32x4 *>(p + 16 * s) : u32x4{0u, 0u, 0u, 0u};
-    }
-}
-
-// Stores rows row0 .. row0 + 31 of a gradient, in 16 bits or (WIDE) fp32.  A template argument: both ways in
-// one kernel, chosen at run time, cost 2 to 4 % of the backward of many short sequences, whose epilogues are a
-// large part of it.
-template <bool BF16, bool WIDE, int OB>
-__device__ __forceinline__ void store_gradient(const f32x16 (&acc)[OB], float mult, uint32_t lds_wave, const AttnBwdArgs &a,
-                                               const Rows &r, int bi, int hi, int row0, int lane)
-{
-    const Rows none = {nullptr, 0u, 0u, 0u};
-    store_rows<BF16, OB>(acc, mult, lds_wave, 0, block_dst(WIDE ? none : r, WIDE ? r : none, bi, hi, row0, a.D), !WIDE, WIDE,
-                         row0, a.N, lane);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -606,343 +546,10 @@ __global__ __launch_bounds__(64 * NW, HDIM == 128 ? NW / 4 : VLDS ? 3 : 2) void 
     }
 }
 
-// ------------------------------------------------------------------------------------------------
-// all three gradients of a short sequence
-// ------------------------------------------------------------------------------------------------
-// N <= 32 NW keys and head dim <= 64: one work-group holds a whole head, a wavefront 32 of its keys, as in the dK/dV
-// kernel.  S, dP and the exponentials are formed once (the two kernels form them twice: 7 products instead of 5) and
-// q, k, v, dO come from memory once.  What is bound by memory and by the length of a work-group's prologue gains most:
-// forward and backward on inputs that no cache holds, the two kernels -> this one: 1024 heads, N = 128, D = 64: 65.0 ->
-// 56.1 us.  With more keys a CU holds one work-group of 8 wavefronts, whose loads nothing else hides, and the gain goes with
-// the number of rounds: N = 256, D = 64, 256 heads: 46.0 -> 39.9 us, 512: 84.9 -> 75.7, 1024: 150.6 -> 146.0, 2048: 297 -> 297.
-//   K            in LDS too, for dQ
-//   scaled Q     (the operand of S, rounded as the forward rounds it, so that the probabilities fit its lse) beside the
-//                Q that dK needs: each wavefront scales the rows it has copied
-//   lse, delta   of all rows and the mask words of each wavefront's keys in LDS from the start; Q and dO through a ring
-//                of two stages of 64 rows
-//   dS           of a tile goes to LDS as [key][row], rows of 128 bytes like every other tile, so that the transposing
-//                reads give the B operand of dQ^T = K^T dS^T; after every second tile the wavefronts share
-//                the 128 rows of dQ.  No sums between work-groups: bit-reproducible.
-template <int NW> struct ShortCfg {
-    static constexpr int KEYS = 32 * NW;                                    // and rows, at most
-    static constexpr int OFF_STAGE = KEYS * 128;
-    static constexpr int STAGE_BYTES = 2 * TILE_BYTES;                      // Q, dO
-    static constexpr int NSTAGES = NW == 2 ? 1 : 2;
-    static constexpr int OFF_DS = OFF_STAGE + NSTAGES * STAGE_BYTES;
-    // the second tile's dS; NW = 4 has no third tile, its first stage is free by then
-    static constexpr int OFF_DS2 = NW == 8 ? OFF_DS + KEYS * 128 : OFF_STAGE;
-    static constexpr int OFF_QS = OFF_DS + (NW == 8 ? 2 : 1) * KEYS * 128;  // scaled Q: of each stage, or (LDS of two
-    static constexpr int QS_BYTES = NW == 8 ? TILE_BYTES : 0;               // work-groups on a CU) of one tile only
-    static constexpr int OFF_WORDS = OFF_QS + TILE_BYTES + QS_BYTES;
-    static constexpr int OFF_LSE = OFF_WORDS + NW * KEYS * 4;
-    static constexpr int OFF_DELTA = OFF_LSE + KEYS * 4;
-    static constexpr int LDS_BYTES = OFF_DELTA + KEYS * 4;
-};
-template <bool BF16, int HDIM, int NW, bool POSTMUL, bool WIDE>
-__global__ __launch_bounds__(64 * NW, 2) void attn_bwd_short_kernel(const AttnBwdArgs a)
-{
-    using E = Elem<BF16>;
-    using C = ShortCfg<NW>;
-    constexpr int KS = HDIM / 16, OB = HDIM / 32;
-    __shared__ __attribute__((aligned(1024))) unsigned char smem[C::LDS_BYTES];
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(LDS_PTR(unsigned char))smem;
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int l32 = lane & 31, hh = lane >> 5;
-    const int bh = renumber_block();
-    const int N = a.N, nw = (N + 31) >> 5;
-    const int T = (N + BN - 1) / BN;
-    const float pm = POSTMUL ? a.post_mul : 1.0f;
-    const float lse_mul = -LOG2E / pm;                // pm is a power of two: exact
-
-    const int bi = (int)fastdiv((uint32_t)bh, a.div_H), hi = bh - bi * a.H;
-    const uint16_t *qb = slab(a.q, bi, hi), *dob = slab(a.dout, bi, hi), *ob = slab(a.out, bi, hi);
-    const uint16_t *kb = slab(a.k, bi, hi), *vb = slab(a.v, bi, hi);
-    const uint32_t *mb = slab(a.mask, bi, hi);
-
-    // ---- copies.  Eight rows of a 64-row tile at a time, swizzled as everywhere; rows >= N repeat row N - 1 and are
-    // set to zero by the wavefront that copied them, once they have landed
-    const int last_chunk = (a.D >> 3) - 1;
-    auto copy_rows = [&](uint32_t tile, const uint16_t *mat, uint32_t sn, int row0, int part) __attribute__((always_inline)) {
-        const int row = 8 * part + (lane >> 3);
-        const int chunk = (lane & 7) ^ bitrev3((row >> 1) & 7);
-        const int r = row0 + row < N ? row0 + row : N - 1;
-        async_copy_b128(tile + part * 1024, mat, __umul24(r, 2u * sn) + ((uint32_t)(chunk < last_chunk ? chunk : last_chunk) << 4));
-    };
-    auto zero_rows = [&](uint32_t tile, int row0, int part) __attribute__((always_inline)) {
-        if (row0 + 8 * part + (lane >> 3) >= N)
-            *(LDS_PTR(u32x4))(uintptr_t)(tile + part * 1024 + lane * 16) = u32x4{0u, 0u, 0u, 0u};
-    };
-    auto copy_tile = [&](int t, int st) __attribute__((always_inline)) {
-        const uint32_t so = lds0 + C::OFF_STAGE + st * C::STAGE_BYTES;
-#pragma unroll
-        for (int j = 0; j < 8 / NW; ++j) {
-            copy_rows(so, qb, a.q.sn, t * BN, wave * (8 / NW) + j);
-            copy_rows(so + TILE_BYTES, dob, a.dout.sn, t * BN, wave * (8 / NW) + j);
-        }
-    };
-    const int key0 = wave * 32;                       // this wavefront's keys; of delta and lse, its rows
-    const bool wave_valid = key0 < N;                 // wave-uniform
-    const int wi = wave < nw ? wave : nw - 1;         // its mask word of a row
-    const uint32_t k_tile = lds0 + (wave >> 1) * TILE_BYTES;
-    for (int t = 0; t < T; ++t) {
-        const int row = t * BN + lane < N ? t * BN + lane : N - 1;
-        async_copy_b32(lds0 + C::OFF_WORDS + wave * (C::KEYS * 4) + t * 256, mb + wi, (uint32_t)(row * nw * 4));
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) copy_rows(k_tile, kb, a.k.sn, (wave >> 1) * BN, 4 * (wave & 1) + j);
-    copy_tile(0, 0);
-
-    // ---- K^T and V^T fragments of this lane's key, delta and lse of its row
-    const int key = key0 + l32;
-    const int kr = key < N ? key : N - 1;
-    const uint32_t key_ok = key < N ? 0xffffffffu : 0u;
-    const uint32_t key_w = key < N ? 1u : 0u;         // width of the bit field that holds this key's mask bit
-    u32x4 kf[KS], vf[KS];
-    {
-        u32x4 dof[KS], of[KS];
-        load_row(kf, kb, a.k.sn, kr, hh, a.D);
-        load_row(vf, vb, a.v.sn, kr, hh, a.D);
-        load_row(dof, dob, a.dout.sn, kr, hh, a.D);
-        load_row(of, ob, a.out.sn, kr, hh, a.D);
-        const float l = a.lse[(size_t)bh * N + kr];
-        float delta = 0.f;
-#pragma unroll
-        for (int s = 0; s < KS; ++s)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                delta += E::up1((uint16_t)(dof[s][i] & 0xffffu)) * E::up1((uint16_t)(of[s][i] & 0xffffu)) +
-                         E::up1((uint16_t)(dof[s][i] >> 16)) * E::up1((uint16_t)(of[s][i] >> 16));
-        delta = xhalf_sum(delta);
-        // rows that kept nothing or lie beyond N: probability 0
-        const bool dead = key >= N || l == -__builtin_inff();
-        if (hh == 0) {
-            *(LDS_PTR(float))(uintptr_t)(lds0 + C::OFF_LSE + 4 * key) = dead ? -__builtin_inff() : l * lse_mul;
-            *(LDS_PTR(float))(uintptr_t)(lds0 + C::OFF_DELTA + 4 * key) = -delta;
-            if (key < N) a.delta[(size_t)bh * N + key] = delta;
-        }
-    }
-    if (NW > 2 && T > 1) copy_tile(1, 1);             // not before the loads above, whose arrival awaits all older requests
-
-    const TileRead tr = make_tile_read(lane);
-    f32x16 dkacc[OB], dvacc[OB];
-#pragma unroll
-    for (int b = 0; b < OB; ++b)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            dkacc[b][i] = 0.f;
-            dvacc[b][i] = 0.f;
-        }
-    // this lane's place in a dS tile: row = its key, columns 32blk + 8g + 4hh .. +3 of the 64 query rows
-    uint32_t ds_row = lds0 + C::OFF_DS + key * 128 + 8 * hh;
-    const uint32_t ds_swz = (uint32_t)bitrev3((l32 >> 1) & 7);
-    uint32_t rows_at = lds0 + C::OFF_WORDS + 16 * hh, words_at = rows_at + wave * (C::KEYS * 4);
-    asm volatile("" : "+v"(ds_row), "+v"(rows_at), "+v"(words_at));         // opaque: see the dK/dV kernel
-
-    // ---- one tile of 64 query rows: dV, dK, and dS into LDS
-    auto tile = [&](int t, auto st_c) __attribute__((always_inline)) {
-        constexpr int st = decltype(st_c)::value;
-        constexpr uint32_t SO = C::OFF_STAGE + st * C::STAGE_BYTES;
-        constexpr int DS = (st == 0 ? C::OFF_DS : C::OFF_DS2) - C::OFF_DS;
-        const uint32_t so = lds0 + SO;
-        const uint32_t rows = rows_at + t * 256, words = words_at + t * 256;
-#pragma unroll
-        for (int blk = 0; blk < 2; ++blk) {
-            // element 4g+j of an accumulator <-> query row 32blk + 8g + 4hh + j of the tile
-            u32x4 mw[4];
-            uint32_t any = 0u;
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                mw[g] = lds_read_b128(words + 128 * blk + 32 * g);
-                any |= mw[g].x | mw[g].y | mw[g].z | mw[g].w;
-            }
-            auto put_ds = [&](int g, u32x2 v) __attribute__((always_inline)) {
-                *(LDS_PTR(u32x2))(uintptr_t)(ds_row + DS + (((4 * blk + g) ^ ds_swz) << 4)) = v;
-            };
-            if (__builtin_amdgcn_ballot_w64((((any >> l32) & 1u) & key_ok) != 0u) == 0ull) {
-#pragma unroll
-                for (int g = 0; g < 4; ++g) put_ds(g, u32x2{0u, 0u});
-                continue;
-            }
-            f32x16 sacc, dacc;
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const u32x4 Lr = lds_read_b128(rows + (C::OFF_LSE - C::OFF_WORDS) + 128 * blk + 32 * g);
-                const u32x4 Dr = lds_read_b128(rows + (C::OFF_DELTA - C::OFF_WORDS) + 128 * blk + 32 * g);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    sacc[4 * g + j] = __builtin_bit_cast(float, (uint32_t)Lr[j]);
-                    dacc[4 * g + j] = __builtin_bit_cast(float, (uint32_t)Dr[j]);
-                }
-            }
-#pragma unroll
-            for (int s = 0; s < KS; ++s) sacc = E::mfma(lds_read_b128(tr.rowaddr[s] + lds0 + C::OFF_QS + st * C::QS_BYTES + 4096 * blk), kf[s], sacc);
-#pragma unroll
-            for (int s = 0; s < KS; ++s) dacc = E::mfma(lds_read_b128(tr.rowaddr[s] + so + TILE_BYTES + 4096 * blk), vf[s], dacc);
-            uint32_t pp[2][4], ps[2][4];
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                float p[4], d[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t keep = (uint32_t)__builtin_amdgcn_sbfe((int)mw[g][j], (uint32_t)l32, key_w);
-                    const float e = __builtin_amdgcn_exp2f(POSTMUL ? sacc[4 * g + j] * pm : sacc[4 * g + j]);
-                    p[j] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, e) & keep);
-                    d[j] = p[j] * dacc[4 * g + j];
-                }
-                pp[g >> 1][2 * (g & 1)] = E::pack2_rne(p[0], p[1]);
-                pp[g >> 1][2 * (g & 1) + 1] = E::pack2_rne(p[2], p[3]);
-                const u32x2 ds = {E::pack2_rne(d[0], d[1]), E::pack2_rne(d[2], d[3])};
-                ps[g >> 1][2 * (g & 1)] = ds.x;
-                ps[g >> 1][2 * (g & 1) + 1] = ds.y;
-                put_ds(g, ds);
-            }
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const u32x4 bp = {pp[u][0], pp[u][1], pp[u][2], pp[u][3]};
-                const u32x4 bs = {ps[u][0], ps[u][1], ps[u][2], ps[u][3]};
-                const uint32_t off = so + 4096 * blk + 2048 * u;
-#pragma unroll
-                for (int b = 0; b < OB; ++b) {
-                    const u32x2 qlo = lds_read_tr16_b64(tr.traddr[b][0] + off), qhi = lds_read_tr16_b64(tr.traddr[b][1] + off);
-                    dkacc[b] = E::mfma(u32x4{qlo.x, qlo.y, qhi.x, qhi.y}, bs, dkacc[b]);              // dK^T += Q^T dS
-                    const u32x2 dlo = lds_read_tr16_b64(tr.traddr[b][0] + off + TILE_BYTES);
-                    const u32x2 dhi = lds_read_tr16_b64(tr.traddr[b][1] + off + TILE_BYTES);
-                    dvacc[b] = E::mfma(u32x4{dlo.x, dlo.y, dhi.x, dhi.y}, bp, dvacc[b]);              // dV^T += dO^T P
-                }
-            }
-        }
-    };
-    // after the copies of a tile have landed
-    auto land = [&](int t, int st) __attribute__((always_inline)) {
-        const uint32_t so = lds0 + C::OFF_STAGE + st * C::STAGE_BYTES, qs = lds0 + C::OFF_QS + st * C::QS_BYTES;
-        if (C::QS_BYTES == 0 && t > 0) __syncthreads();             // the tile before has been read
-#pragma unroll
-        for (int j = 0; j < 8 / NW; ++j) {
-            const int part = wave * (8 / NW) + j;
-            if ((t + 1) * BN > N) {
-                zero_rows(so, t * BN, part);
-                zero_rows(so + TILE_BYTES, t * BN, part);
-            }
-            u32x4 x = lds_read_b128(so + part * 1024 + lane * 16);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float lo = E::up1((uint16_t)(x[i] & 0xffffu)) * a.q_scale;
-                const float hi = E::up1((uint16_t)(x[i] >> 16)) * a.q_scale;
-                x[i] = (uint32_t)E::cvt1(lo) | ((uint32_t)E::cvt1(hi) << 16);
-            }
-            *(LDS_PTR(u32x4))(uintptr_t)(qs + part * 1024 + lane * 16) = x;
-        }
-        __syncthreads();
-    };
-
-    // ---- dQ of up to 128 rows from row0 on: blocks of 32 rows x 32 columns, eight wavefronts one each, fewer the
-    // columns of 32 rows
-    constexpr int QB = NW == 8 ? 1 : OB;              // column blocks of a wavefront
-    const int rb = NW == 8 ? wave >> 1 : wave;
-    const int cb = NW == 8 ? wave & 1 : 0;            // the first of them
-    auto store_dq = [&](int row0) __attribute__((always_inline)) {
-        if (row0 + 32 * rb >= N || cb >= OB) return;
-        f32x16 acc[QB];
-#pragma unroll
-        for (int b = 0; b < QB; ++b)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[b][i] = 0.f;
-        const uint32_t ds = lds0 + (rb >> 1 ? C::OFF_DS2 : C::OFF_DS);
-        const uint32_t b0 = ds + tr.traddr[0][0] + (rb & 1 ? tr.traddr[1][0] - tr.traddr[0][0] : 0u);
-        const uint32_t b1 = ds + tr.traddr[0][1] + (rb & 1 ? tr.traddr[1][1] - tr.traddr[0][1] : 0u);
-        const uint32_t a0 = lds0 + tr.traddr[0][0] + (cb ? tr.traddr[1][0] - tr.traddr[0][0] : 0u);
-        const uint32_t a1 = lds0 + tr.traddr[0][1] + (cb ? tr.traddr[1][1] - tr.traddr[0][1] : 0u);
-        // keys, 32 at a time: the wavefronts beyond the last key have left no dS
-#pragma unroll
-        for (int kb32 = 0; kb32 < NW; ++kb32) {
-            if (32 * kb32 >= N) break;
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const uint32_t off = 4096 * kb32 + 2048 * u;
-                const u32x2 dlo = lds_read_tr16_b64(b0 + off), dhi = lds_read_tr16_b64(b1 + off);
-                const u32x4 dsf = {dlo.x, dlo.y, dhi.x, dhi.y};
-#pragma unroll
-                for (int b = 0; b < QB; ++b) {
-                    const u32x2 klo = lds_read_tr16_b64((b == 0 ? a0 : lds0 + tr.traddr[b][0]) + off);
-                    const u32x2 khi = lds_read_tr16_b64((b == 0 ? a1 : lds0 + tr.traddr[b][1]) + off);
-                    acc[b] = E::mfma(u32x4{klo.x, klo.y, khi.x, khi.y}, dsf, acc[b]);
-                }
-            }
-        }
-        // a lane has columns 8g + 4hh .. +3 of its row: LDS is in use, so they go out as they are (8 or 16 bytes)
-        const int row = row0 + 32 * rb + l32;
-        if (row < N) {
-            const BlockDst d = block_dst(WIDE ? Rows{nullptr, 0u, 0u, 0u} : a.dq, WIDE ? a.dq : Rows{nullptr, 0u, 0u, 0u}, bi, hi, row, a.D);
-#pragma unroll
-            for (int b = 0; b < QB; ++b)
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const int col = 32 * (cb + b) + 8 * g;
-                    if (col >= a.D) continue;
-                    const u32x2 h = {E::pack2_rne(acc[b][4 * g] * a.scale, acc[b][4 * g + 1] * a.scale),
-                                     E::pack2_rne(acc[b][4 * g + 2] * a.scale, acc[b][4 * g + 3] * a.scale)};
-                    if constexpr (WIDE)
-                        *reinterpret_cast<f32x4 *>(d.f + col + 4 * hh) =
-                            f32x4{E::up1((uint16_t)(h.x & 0xffffu)), E::up1((uint16_t)(h.x >> 16)), E::up1((uint16_t)(h.y & 0xffffu)),
-                                  E::up1((uint16_t)(h.y >> 16))};
-                    else
-                        *reinterpret_cast<u32x2 *>(d.h + col + 4 * hh) = h;
-                }
-        }
-    };
-
-    if (NW > 2 && T > 1) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(16 / NW) : "memory");        // all but the second tile
-    else WAIT_VMCNT(0);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) zero_rows(k_tile, (wave >> 1) * BN, 4 * (wave & 1) + j);
-    for (int t = 0; t < T; t += 2) {
-        if (t > 0) WAIT_VMCNT(0);
-        land(t, 0);
-        if (wave_valid) tile(t, std::integral_constant<int, 0>{});
-        if (NW > 2 && t + 1 < T) {
-            WAIT_VMCNT(0);
-            land(t + 1, 1);                           // every wavefront is done with the first stage
-            if (NW > 4 && t + 2 < T) copy_tile(t + 2, 0);
-            if (wave_valid) tile(t + 1, std::integral_constant<int, C::NSTAGES - 1>{});
-        }
-        __syncthreads();                              // dS is complete, the second stage is free
-        if (NW > 4 && t + 3 < T) copy_tile(t + 3, 1);
-        store_dq(t * BN);
-    }
-    __syncthreads();                                  // K has been read: its place serves the transposed stores
-    if (wave_valid) {
-        store_gradient<BF16, WIDE>(dkacc, a.scale, lds0 + wave * 4096, a, a.dk, bi, hi, key0, lane);
-        store_gradient<BF16, WIDE>(dvacc, 1.0f, lds0 + wave * 4096, a, a.dv, bi, hi, key0, lane);
-    }
-}
-
 template <bool BF16, int HDIM, bool POSTMUL, bool WIDE>
 void launch_pair(hipStream_t stream, const AttnBwdArgs &args)
 {
     AttnBwdArgs a = args;
-    if constexpr (HDIM <= 64) {
-        // A whole head in one work-group (see attn_bwd_short_kernel).  Up to 128 keys always: forward + backward, inputs from
-        // memory, 4 heads, N = 64, D = 32: 11.7 -> 9.0 us, 2048 heads, N = 128, D = 64: 118.6 -> 107.5 us, 4 to 30 % between.
-        // With more keys a CU holds only one of the eight-wavefront work-groups, and its time is that of its whole
-        // rounds: for head dims above 32 where the last round is at least three quarters full.  N = 256, D = 64, the same
-        // measure: 192 heads 40.5 -> 35.4 us, 256: 46.0 -> 39.9, 1024: 150.6 -> 146.0, 2048: 297 either way (causal
-        // mask: 274 -> 279); half a round, 384 heads, would go 61.9 -> 63.4.  (D = 32, 1024 heads, the backward alone
-        // on warm inputs: 57.8 -> 61.7 us.)
-        const long long cus = compute_units(), last = cus > 0 ? a.BH % cus : 0;
-        if (a.N <= 128 || (a.N <= 256 && HDIM > 32 && (last == 0 || 4 * last >= 3 * cus))) {
-            const dim3 grid((unsigned)a.BH);
-            if (a.N <= 64)
-                hipLaunchKernelGGL((attn_bwd_short_kernel<BF16, HDIM, 2, POSTMUL, WIDE>), grid, dim3(128), 0, stream, a);
-            else if (a.N <= 128)
-                hipLaunchKernelGGL((attn_bwd_short_kernel<BF16, HDIM, 4, POSTMUL, WIDE>), grid, dim3(256), 0, stream, a);
-            else if constexpr (HDIM > 32)
-                hipLaunchKernelGGL((attn_bwd_short_kernel<BF16, HDIM, 8, POSTMUL, WIDE>), grid, dim3(512), 0, stream, a);
-            return;
-        }
-    }
     // dQ first: it also fills the delta workspace that the dK/dV kernel reads (same stream)
     hipLaunchKernelGGL((attn_bwd_dq_kernel<BF16, HDIM, WIDE>), dim3((unsigned)(a.BH * a.qtiles)), dim3(NTHREADS), 0, stream, a);
     auto dkv = [&](auto nw_c, auto vlds_c) {
@@ -994,6 +601,7 @@ hipError_t launch_attn_bwd(const AttnBwdArgs &args, bool bf16, hipStream_t strea
     a.div_H = make_fastdiv((uint32_t)a.H);
     if ((long long)a.BH * a.qtiles == 0) return hipSuccess;
     if (a.grads_f32 && !bf16) return hipErrorInvalidValue;
+    if (launch_attn_bwd_head(a, bf16, stream)) return hipGetLastError();
     switch (kernel_head_dim(a.D)) {
     case 128: launch_head_dim<128>(bf16, stream, a); break;
     case 96: launch_head_dim<96>(bf16, stream, a); break;

@@ -1,0 +1,71 @@
+// Device-side helpers that the backward kernels share (attn_bwd.hip, attn_bwd_head.hip): the per-lane read addresses of
+// a tile, the fragments of a row, the stores of a gradient.
+#pragma once
+#include "attn_common.h"
+
+namespace sma {
+namespace {
+
+constexpr float LOG2E = 1.4426950408889634f;
+
+// Per-lane LDS read offsets inside a tile (add the tile's base and 4096 per block of 32 rows).
+//   rowaddr[s]       ds_read_b128: row l32, columns 16s + 8hh .. +7          (A operand, k-step s)
+//   traddr[dblk][x]  ds_read_b64_tr_b16: rows 8x + 4hh + (i >> 2) (+16u), columns 32dblk + 16G +
+//                    4(i & 3) .. +3, i = lane % 16, G = (lane % 32) / 16     (A operand = tile^T)
+struct TileRead {
+    uint32_t rowaddr[4];
+    uint32_t traddr[2][2];
+};
+__device__ __forceinline__ TileRead make_tile_read(int lane)
+{
+    TileRead r;
+    const int l32 = lane & 31, hh = lane >> 5;
+    const int fk = bitrev3((l32 >> 1) & 7);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) r.rowaddr[s] = (uint32_t)(l32 * 128 + (((2 * s + hh) ^ fk) << 4));
+    const int i16 = lane & 15, G = l32 >> 4;
+    const int r3 = 4 * hh + (i16 >> 2);
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+        const int row = 8 * x + r3;
+        const int fr = bitrev3((row >> 1) & 7);
+#pragma unroll
+        for (int dblk = 0; dblk < 2; ++dblk) {
+            const int chunk = 4 * dblk + 2 * G + ((i16 & 3) >> 1);
+            r.traddr[dblk][x] = (uint32_t)(row * 128 + ((chunk ^ fr) << 4) + ((i16 & 1) << 3));
+        }
+    }
+    return r;
+}
+
+// The fragments of one row of a matrix (row stride sn elements, D columns): 8 elements at columns
+// 16s + 8hh, zeros beyond the row.  `full` (D is the kernel's own head dim) is wave-uniform: the common
+// case loads straight.
+template <int KS>
+__device__ __forceinline__ void load_row(u32x4 (&f)[KS], const uint16_t *mat, uint32_t sn, int row, int hh, int D)
+{
+    const uint16_t *p = mat + (size_t)row * sn + 8 * hh;
+    if (D == 16 * KS) {
+#pragma unroll
+        for (int s = 0; s < KS; ++s) f[s] = *reinterpret_cast<const u32x4 *>(p + 16 * s);
+    } else {
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+            f[s] = 16 * s + 8 * hh < D ? *reinterpret_cast<const u32x4 *>(p + 16 * s) : u32x4{0u, 0u, 0u, 0u};
+    }
+}
+
+// Stores rows row0 .. row0 + 31 of a gradient, in 16 bits or (WIDE) fp32.  A template argument: both ways in
+// one kernel, chosen at run time, cost 2 to 4 % of the backward of many short sequences, whose epilogues are a
+// large part of it.
+template <bool BF16, bool WIDE, int OB>
+__device__ __forceinline__ void store_gradient(const f32x16 (&acc)[OB], float mult, uint32_t lds_wave, const AttnBwdArgs &a,
+                                               const Rows &r, int bi, int hi, int row0, int lane)
+{
+    const Rows none = {nullptr, 0u, 0u, 0u};
+    store_rows<BF16, OB>(acc, mult, lds_wave, 0, block_dst(WIDE ? none : r, WIDE ? r : none, bi, hi, row0, a.D), !WIDE, WIDE,
+                         row0, a.N, lane);
+}
+
+}  // namespace
+}  // namespace sma

@@ -1,0 +1,518 @@
+// dQ, dK and dV of a whole head in one work-group: sequences of at most 128 (head dims 96 and 128, four wavefronts), 256
+// (eight) or 512 keys (head dims 32 and 64, 64 keys to a wavefront).  The formulas are those at the top of attn_bwd.hip.
+//
+// S, dP and the exponentials are formed once where the two kernels of attn_bwd.hip form them twice (five N x N x D products
+// instead of seven), q, k, v and dO come from memory once, and there is one launch.  No sums between work-groups:
+// bit-reproducible.
+//   wavefront    32 KB keys, KB = 1 or 2 (lane = key, as in the dK/dV kernel); dK and dV are its accumulators, V fragments stay in
+//                registers.  With KB = 2 every Q and dO operand that is read from LDS serves two products.
+//   rows         32 at a time, in a ring of two stages: Q, dO, the mask words of each wavefront's keys, and Q scaled and rounded as
+//                the forward does it, so that the probabilities fit its lse (the wavefront that copied eight rows scales
+//                them; as VALU work of every wavefront instead it cost 4 us of 62 on 192 heads, N = 512, D = 64).
+//   K            all of it in LDS, both as the operand of S and, read transposed, of dQ
+//   dS           to LDS as [key][row], 64 bytes a key; after the next barrier the wavefronts share dQ^T = K^T dS^T of the 32 rows
+//                in blocks of 16 x 16.  Eight wavefronts have two such buffers and one barrier for 32 rows; four have one,
+//                so that two work-groups share a CU, and two barriers.
+// Swizzles: Q and dO as everywhere in the backward (bitrev3 of row / 2), K by 16 bytes with the bits of row / 2 in the order (2, 0, 1)
+// and dS by 8 bytes with those of key / 4 in the order (1, 2, 0): their row accesses and the transposing reads of 16 keys x 16
+// columns that dQ needs are free of bank conflicts (2.3 cycles a read on a full CU, 2.1 for a linear one).
+//
+// Forward + backward with every step's inputs from memory, in us, before (two kernels, up to 256 keys at head dims up to 64 an
+// earlier form of this one) -> now:
+//   D =  64   N = 512: 192 heads 90.9 -> 84.8, 256: 123.7 -> 101.7;  N = 256: 512 heads 73.9 -> 70.9, 2048: 282 -> 248;
+//             1024 heads: N = 160 94.2 -> 80.1;  2048 heads: N = 128 106.0 -> 98.4, N = 32 41.3 -> 37.2
+//   D = 128   N = 256: 256 heads 72.7 -> 63.1, 1024: 274 -> 236;  1024 heads: N = 128 123.1 -> 93.7, N = 64 70.0 -> 49.0
+//   D =  32   1024 heads, N = 256: 90.7 -> 82.8;  D = 96: 1024 heads, N = 128: 86.1 -> 77.1
+// What bounds it: on 256 heads, N = 512, D = 64 (fp16, 62 us) a SIMD's 6500 cycles for 32 rows hold 2560 of the matrix cores, about 2700
+// of the vector ALU and, for the CU, 3200 of LDS; the barrier keeps the eight wavefronts in the same phase, which is bound by one of
+// them at a time.  Starting half of the wavefronts with dQ and half with S changed nothing.  Many short sequences are bound by
+// memory: 2048 heads, N = 32: 4.2 TB/s.
+#include <type_traits>
+
+#include "attn_bwd_common.h"
+
+namespace sma {
+namespace {
+
+template <int HDIM, int NW, int KB> struct HeadCfg {
+    static constexpr int NH = HDIM > 64 ? 2 : 1;                    // column halves of 64
+    static constexpr int KEYS = 32 * NW * KB;                       // and rows, at most
+    static constexpr int K_HALF = KEYS * 128;
+    static constexpr int OFF_DS = NH * K_HALF;
+    static constexpr int DS_BYTES = KEYS * 64;                      // dS of 32 rows: [key][row]
+    static constexpr int DS_BUFS = NW == 8 ? 2 : 1;
+    static constexpr int PART = NH * 4096;                          // 32 rows of one matrix
+    static constexpr bool LAND = !(NW == 4 && NH == 2);             // scaled Q in LDS (there two work-groups would not fit)
+    static constexpr int OFF_WORDS = (LAND ? 3 : 2) * PART;         // a stage: Q, dO, scaled Q, each wavefront's mask words
+    static constexpr int STAGE_BYTES = OFF_WORDS + NW * 256;
+    static constexpr int OFF_STAGE = OFF_DS + DS_BUFS * DS_BYTES;
+    static constexpr int OFF_LSE = OFF_STAGE + 2 * STAGE_BYTES;
+    static constexpr int OFF_DELTA = OFF_LSE + KEYS * 4;
+    static constexpr int LDS_BYTES = OFF_DELTA + KEYS * 4;
+};
+
+// 16 x 16 x 32 products
+template <bool BF16> __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c)
+{
+    if constexpr (BF16)
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ u32x4 tr_pair(uint32_t lo, uint32_t hi)
+{
+    const u32x2 x = lds_read_tr16_b64(lo), y = lds_read_tr16_b64(hi);
+    return u32x4{x.x, x.y, y.x, y.y};
+}
+
+template <bool BF16, int HDIM, int NW, int KB, bool WIDE>
+__global__ __launch_bounds__(64 * NW, HDIM <= 64 && KB == 1 && NW == 4 ? 3 : 2) void attn_bwd_head_kernel(const AttnBwdArgs a)
+{
+    using E = Elem<BF16>;
+    using C = HeadCfg<HDIM, NW, KB>;
+    constexpr int NH = C::NH, KS = HDIM / 16, OB = HDIM / 32;
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[C::LDS_BYTES];
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(LDS_PTR(unsigned char))smem;
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, hh = lane >> 5;
+    const int bh = renumber_block();
+    const int N = a.N, nw = (N + 31) >> 5;
+    const int RB = (N + 31) >> 5;                     // blocks of 32 rows
+    const float pm = a.post_mul;
+
+    const int bi = (int)fastdiv((uint32_t)bh, a.div_H), hi = bh - bi * a.H;
+    const uint16_t *qb = slab(a.q, bi, hi), *dob = slab(a.dout, bi, hi), *ob = slab(a.out, bi, hi);
+    const uint16_t *kb_ = slab(a.k, bi, hi), *vb = slab(a.v, bi, hi);
+    const uint32_t *mb = slab(a.mask, bi, hi);
+
+    // ---- copies
+    const int last_chunk = (a.D >> 3) - 1;
+    auto chunk_at = [&](int c) __attribute__((always_inline)) -> uint32_t { return (uint32_t)(c < last_chunk ? c : last_chunk) << 4; };
+    auto k_swizzle = [](int row) __attribute__((always_inline)) { const int p = (row >> 1) & 7; return (p & 4) | ((p & 1) << 1) | ((p >> 1) & 1); };
+    const int key0 = wave * (32 * KB);                // this wavefront's keys; of delta and lse, its rows
+    const bool wave_valid = key0 < N;                 // wave-uniform
+    const int part = wave & 3;
+    auto issue = [&](int i, auto st_c) __attribute__((always_inline)) {
+        constexpr int SO = C::OFF_STAGE + decltype(st_c)::value * C::STAGE_BYTES;
+        int ln = lane;
+        asm volatile("" : "+v"(ln));                  // the few sums below are made again each time instead of kept
+        const int prow = 8 * part + (ln >> 3);        // the row of a stage that this lane copies 16 bytes of
+        const int pc = (ln & 7) ^ bitrev3((prow >> 1) & 7);
+        const uint32_t pchunk = chunk_at(pc), pchunk2 = chunk_at(8 + pc);
+        const int row = 32 * i + prow < N ? 32 * i + prow : N - 1;
+        auto rows = [&](auto off_c, const uint16_t *mat, uint32_t sn) __attribute__((always_inline)) {
+            constexpr int AT = SO + decltype(off_c)::value;
+            const uint32_t r = __umul24(row, 2u * sn);
+            async_copy_b128_at<AT>(lds0 + part * 1024, mat, r + pchunk);
+            if constexpr (NH == 2) async_copy_b128_at<AT + 4096>(lds0 + part * 1024, mat, r + pchunk2);
+        };
+        if (NW == 4 || wave < 4) rows(std::integral_constant<int, 0>{}, qb, a.q.sn);
+        if (NW == 4 || wave >= 4) rows(std::integral_constant<int, C::PART>{}, dob, a.dout.sn);
+        const int mword = KB == 2 ? wave * 2 + (ln >> 5) : wave, wi = mword < nw ? mword : nw - 1;
+        const int mrow = 32 * i + (ln & 31) < N ? 32 * i + (ln & 31) : N - 1;
+        async_copy_b32_at<SO + C::OFF_WORDS>(lds0 + wave * 256, mb, (uint32_t)((mrow * nw + wi) * 4));
+    };
+#pragma unroll
+    for (int j = 0; j < 4 * KB; ++j) {                // its rows of K
+        const int row = key0 + 8 * j + (lane >> 3), r = row < N ? row : N - 1;
+        const int chunk = (lane & 7) ^ k_swizzle(row);
+        const uint32_t off = __umul24(r, 2u * a.k.sn);
+        async_copy_b128(lds0 + key0 * 128 + j * 1024, kb_, off + chunk_at(chunk));
+        if constexpr (NH == 2) async_copy_b128(lds0 + C::K_HALF + key0 * 128 + j * 1024, kb_, off + chunk_at(8 + chunk));
+    }
+    issue(0, std::integral_constant<int, 0>{});
+
+    // ---- V^T fragments of this lane's keys, delta and lse of its rows
+    u32x4 vf[KB][KS];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+        const int key = key0 + 32 * kb + l32, kr = key < N ? key : N - 1;
+        u32x4 dof[KS], of[KS];
+        const uint16_t *vp = vb + (size_t)kr * a.v.sn, *dop = dob + (size_t)kr * a.dout.sn, *op = ob + (size_t)kr * a.out.sn;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {                // columns beyond the row's end: its last ones, set to zero
+            const int col = 16 * s + 8 * hh, at = col < a.D ? col : a.D - 8;
+            const uint32_t ok = col < a.D ? 0xffffffffu : 0u;
+            vf[kb][s] = *reinterpret_cast<const u32x4 *>(vp + at) & ok;
+            dof[s] = *reinterpret_cast<const u32x4 *>(dop + at) & ok;
+            of[s] = *reinterpret_cast<const u32x4 *>(op + at);
+        }
+        const float l = a.lse[(size_t)bh * N + kr];
+        float delta = 0.f;
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                delta += E::up1((uint16_t)(dof[s][i] & 0xffffu)) * E::up1((uint16_t)(of[s][i] & 0xffffu)) +
+                         E::up1((uint16_t)(dof[s][i] >> 16)) * E::up1((uint16_t)(of[s][i] >> 16));
+        delta = xhalf_sum(delta);
+        // rows that kept nothing or lie beyond N: probability 0
+        const bool dead = key >= N || l == -__builtin_inff();
+        if (hh == 0) {
+            *(LDS_PTR(float))(uintptr_t)(lds0 + C::OFF_LSE + 4 * key) = dead ? -__builtin_inff() : -l * LOG2E;
+            *(LDS_PTR(float))(uintptr_t)(lds0 + C::OFF_DELTA + 4 * key) = -delta;
+            if (key < N) a.delta[(size_t)bh * N + key] = delta;
+        }
+    }
+    const bool keys_end = key0 + 32 * KB > N;         // wave-uniform: some of this wavefront's keys do not exist
+
+    f32x16 dkacc[KB][OB], dvacc[KB][OB];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int b = 0; b < OB; ++b)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                dkacc[kb][b][i] = 0.f;
+                dvacc[kb][b][i] = 0.f;
+            }
+
+    // ---- read addresses
+    // One register per pattern: a step along a row flips bits of the swizzled chunk, eight (four) rows further down flip
+    // another and add their bytes; the rest is an immediate.
+    uint32_t row_at = lds0 + C::OFF_STAGE + make_tile_read(lane).rowaddr[0], col_at = lds0 + C::OFF_STAGE + make_tile_read(lane).traddr[0][0];
+    uint32_t key_at = lds0 + (key0 + l32) * 128 + ((hh ^ k_swizzle(l32)) << 4);
+    auto ds_swizzle = [](int key) __attribute__((always_inline)) { const int x = key >> 2; return ((x & 2) << 1) | ((x & 4) >> 1) | (x & 1); };
+    uint32_t ds_at = lds0 + C::OFF_DS + (key0 + l32) * 64 + ((hh ^ ds_swizzle(l32)) << 3);
+    uint32_t half_at = lds0 + 16 * hh, lane_at = lds0 + 4 * lane;      // rows 8g + 4hh .. of the small data; this lane's word
+
+    // dQ^T = K^T dS^T in blocks of 16 columns x 16 rows
+    constexpr int NDB = HDIM / 16;
+    constexpr int RH = NW >= 2 * NDB ? 1 : 2;         // row halves of a wavefront
+    constexpr int PASSES = (NDB + NW - 1) / NW;   // its blocks of columns, NW apart: 64 columns
+    static_assert(PASSES == 1 || NW == 4, "the blocks of a wavefront lie in different column halves");
+    const int db = RH == 1 ? wave % NDB : wave, rh0 = RH == 1 ? wave / NDB : 0;
+    unsigned char *dq_slab = reinterpret_cast<unsigned char *>(a.dq.p) + ((size_t)bi * a.dq.sb8 + (size_t)hi * a.dq.sh8) * (WIDE ? 32 : 16);
+    const bool dq_wave = RH == 1 ? wave < 2 * NDB : wave < NDB;
+    uint32_t dq_k, dq_s;
+    {
+        const int i16 = lane & 15, key = 8 * (lane >> 4) + (i16 >> 2);
+        dq_k = lds0 + (db >> 2) * C::K_HALF + key * 128 + (((2 * (db & 3) + ((i16 & 3) >> 1)) ^ k_swizzle(key)) << 4) + ((i16 & 1) << 3);
+        dq_s = lds0 + C::OFF_DS + key * 64 + (((4 * rh0 + (i16 & 3)) ^ ds_swizzle(key)) << 3);
+    }
+
+    // q as the forward multiplies it (scaled, rounded once more), so that the probabilities fit its lse
+    auto scaled = [&](u32x4 x) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            x[j] = E::pack2_rne(E::up1((uint16_t)(x[j] & 0xffffu)) * a.q_scale, E::up1((uint16_t)(x[j] >> 16)) * a.q_scale);
+        return x;
+    };
+    auto land = [&](auto st_c) __attribute__((always_inline)) {      // ... of the rows that this wavefront has copied
+        if constexpr (C::LAND) {
+            if (NW == 8 && wave >= 4) return;
+            const uint32_t at = lane_at * 4 - 3 * lds0 + (C::OFF_STAGE + decltype(st_c)::value * C::STAGE_BYTES + part * 1024);
+#pragma unroll
+            for (int half = 0; half < NH; ++half)
+                *(LDS_PTR(u32x4))(uintptr_t)(at + 2 * C::PART + half * 4096) = scaled(lds_read_b128(at + half * 4096));
+        }
+    };
+    // ---- 32 query rows: dV, dK, and dS into LDS
+    auto rows32 = [&](int i, auto st_c) __attribute__((always_inline)) {
+        constexpr int st = decltype(st_c)::value;
+        constexpr int DS = C::DS_BUFS == 2 ? st * C::DS_BYTES : 0;
+        constexpr int SB = st * C::STAGE_BYTES;
+        // opaque: the compiler would keep a register for every address that follows from these
+        asm volatile("" : "+v"(row_at), "+v"(col_at), "+v"(key_at), "+v"(ds_at), "+v"(half_at), "+v"(lane_at));
+        const uint32_t word_at = lane_at + (C::OFF_STAGE + SB + C::OFF_WORDS + wave * 256), words_at = half_at + (C::OFF_STAGE + SB + C::OFF_WORDS + wave * 256);
+        uint32_t word = *(LDS_PTR(const uint32_t))(uintptr_t)(word_at);
+        if (keys_end) {                               // nothing is kept of keys beyond N, whatever their bits
+            int ln = lane;
+            asm volatile("" : "+v"(ln));
+            const int left = N - key0 - (KB == 2 ? ln & 32 : 0);
+            word &= left >= 32 ? 0xffffffffu : left > 0 ? (1u << left) - 1u : 0u;
+            *(LDS_PTR(uint32_t))(uintptr_t)(word_at) = word;
+        }
+        const bool live = wave_valid && __builtin_amdgcn_ballot_w64(word != 0u) != 0ull;
+        // dQ leaves out the wavefronts that have kept nothing; their flags take the place of the rows before these in lse
+        if (i > 0) {
+            if (lane == 0) *(LDS_PTR(uint32_t))(uintptr_t)(lds0 + C::OFF_LSE + 128 * (i - 1) + 4 * wave) = live ? 1u : 0u;
+        } else if (!live) {
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) *(LDS_PTR(u32x2))(uintptr_t)((ds_at ^ (16 * g)) + DS + 2048 * kb) = u32x2{0u, 0u};
+        }
+        if (!live) return;
+        // Operands are requested a step ahead of their use, and scheduling barriers hold that order: left alone, the compiler
+        // requests each just before it is needed, since registers are short, and the wavefront sits out some 30 LDS round
+        // trips one after the other.
+        const uint32_t rows = half_at + (C::OFF_LSE + i * 128);
+        auto q_frag = [&](int s) __attribute__((always_inline)) { return lds_read_b128((row_at ^ (32 * (s & 3))) + SB + (C::LAND ? 2 * C::PART : 0) + (s >> 2) * 4096); };
+        auto o_frag = [&](int s) __attribute__((always_inline)) { return lds_read_b128((row_at ^ (32 * (s & 3))) + SB + C::PART + (s >> 2) * 4096); };
+        auto k_frag = [&](int s, int kb) __attribute__((always_inline)) { return lds_read_b128((key_at ^ (32 * (s & 3))) + (s >> 2) * C::K_HALF + kb * 4096); };
+        auto mask_of = [&](int kb, int g) __attribute__((always_inline)) { return lds_read_b128(words_at + 128 * kb + 32 * g); };
+        auto lse_of = [&](int g) __attribute__((always_inline)) { return lds_read_b128(rows + 32 * g); };
+        f32x16 sacc[KB], dacc[KB];
+        auto from_delta = [&](int kb) __attribute__((always_inline)) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const u32x4 Dr = lds_read_b128(rows + (C::OFF_DELTA - C::OFF_LSE) + 32 * g);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) dacc[kb][4 * g + j] = __builtin_bit_cast(float, (uint32_t)Dr[j]);
+            }
+        };
+        if (NW == 8) __builtin_amdgcn_s_setprio(0);
+        u32x4 raw[2], qf[2], kf[2][KB], of[2], mg[2], Lr[2];
+        if constexpr (C::LAND) {
+            qf[0] = q_frag(0);
+        } else {
+            raw[0] = q_frag(0);
+            raw[1] = q_frag(1);
+        }
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+            kf[0][kb] = k_frag(0, kb);
+#pragma unroll
+            for (int e = 0; e < 16; ++e) sacc[kb][e] = 0.f;
+        }
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            if constexpr (!C::LAND) qf[s & 1] = scaled(raw[s & 1]);
+            if (s + 1 < KS) {
+                if constexpr (C::LAND) qf[(s + 1) & 1] = q_frag(s + 1);
+                else if (s + 2 < KS) raw[s & 1] = q_frag(s + 2);
+#pragma unroll
+                for (int kb = 0; kb < KB; ++kb) kf[(s + 1) & 1][kb] = k_frag(s + 1, kb);
+            } else {
+                from_delta(0);
+                of[0] = o_frag(0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb) sacc[kb] = E::mfma(qf[s & 1], kf[s & 1][kb], sacc[kb]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            if (s + 1 < KS) {
+                of[(s + 1) & 1] = o_frag(s + 1);
+            } else {
+                mg[0] = mask_of(0, 0);
+                Lr[0] = lse_of(0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            dacc[0] = E::mfma(of[s & 1], vf[0][s], dacc[0]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // P and dS, four rows at a time; with two blocks of keys the second's dP in the midst of the first's
+        uint32_t pp[KB][2][4], ps[KB][2][4];
+        u32x4 qa[2], oa[2];
+        auto columns = [&](int n) __attribute__((always_inline)) {           // Q^T and dO^T operands of the n-th pair of products
+            const int u = n / OB, b = n % OB, at = SB + 2048 * u + (b >> 1) * 4096;
+            const uint32_t c0 = col_at ^ (64 * (b & 1)), c1 = col_at ^ (64 * (b & 1) + 16);
+            oa[n & 1] = tr_pair(c0 + at + C::PART, c1 + at + 1024 + C::PART);
+            qa[n & 1] = tr_pair(c0 + at, c1 + at + 1024);
+        };
+#pragma unroll
+        for (int n = 0; n < 4 * KB; ++n) {
+            const int kb = n / 4, g = n % 4;
+            if (n + 1 < 4 * KB) {
+                mg[(n + 1) & 1] = mask_of((n + 1) / 4, (n + 1) % 4);
+                Lr[(n + 1) & 1] = lse_of((n + 1) % 4);
+            } else {
+                columns(0);
+            }
+            if (KB == 2 && n == 3) of[0] = o_frag(0);
+            __builtin_amdgcn_sched_barrier(0);
+            float p[4], d[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t keep = (uint32_t)__builtin_amdgcn_sbfe((int)mg[n & 1][j], (uint32_t)lane, 1u);       // bit lane % 32
+                const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[kb][4 * g + j], pm, __builtin_bit_cast(float, (uint32_t)Lr[n & 1][j])));
+                p[j] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, e) & keep);
+                d[j] = p[j] * dacc[kb][4 * g + j];
+            }
+            pp[kb][g >> 1][2 * (g & 1)] = E::pack2_rne(p[0], p[1]);
+            pp[kb][g >> 1][2 * (g & 1) + 1] = E::pack2_rne(p[2], p[3]);
+            const u32x2 ds = {E::pack2_rne(d[0], d[1]), E::pack2_rne(d[2], d[3])};
+            ps[kb][g >> 1][2 * (g & 1)] = ds.x;
+            ps[kb][g >> 1][2 * (g & 1) + 1] = ds.y;
+            *(LDS_PTR(u32x2))(uintptr_t)((ds_at ^ (16 * g)) + DS + 2048 * kb) = ds;
+            __builtin_amdgcn_sched_barrier(0);
+            if (KB == 2 && n == 3) {
+                from_delta(KB - 1);
+#pragma unroll
+                for (int s = 0; s < KS; ++s) {
+                    if (s + 1 < KS) of[(s + 1) & 1] = o_frag(s + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    dacc[KB - 1] = E::mfma(of[s & 1], vf[KB - 1][s], dacc[KB - 1]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        }
+#pragma unroll
+        for (int n = 0; n < 2 * OB; ++n) {
+            const int u = n / OB, b = n % OB;
+            if (n + 1 < 2 * OB) columns(n + 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb) {
+                dvacc[kb][b] = E::mfma(oa[n & 1], u32x4{pp[kb][u][0], pp[kb][u][1], pp[kb][u][2], pp[kb][u][3]}, dvacc[kb][b]);
+                dkacc[kb][b] = E::mfma(qa[n & 1], u32x4{ps[kb][u][0], ps[kb][u][1], ps[kb][u][2], ps[kb][u][3]}, dkacc[kb][b]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    // ---- dQ of the 32 rows whose dS is complete
+    auto dq32 = [&](int i, auto buf_c) __attribute__((always_inline)) {
+        constexpr int BUF = C::DS_BUFS == 2 ? decltype(buf_c)::value : 0;
+        if (!dq_wave) return;
+        // The hardware serves the oldest wavefronts first; here the others would wait twice as long for their LDS reads, and all
+        // of them for those at the next barrier: 61.9 -> 57.9 us on 192 heads, N = 512, D = 64
+        if (NW == 8 && wave >= NW / 2) __builtin_amdgcn_s_setprio(1);
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
+        uint32_t live = (1u << NW) - 1u;
+        if (i > 0) live &= (uint32_t)__builtin_amdgcn_ballot_w64(*(LDS_PTR(const uint32_t))(uintptr_t)(lds0 + C::OFF_LSE + 128 * (i - 1) + 4 * (ln & (NW - 1))) != 0u);
+#pragma unroll
+        for (int pass = 0; pass < PASSES; ++pass) {
+            if (pass > 0 && wave + NW * pass >= NDB) break;
+            constexpr int CH = RH == 1 ? 2 : 1;           // chains of products of a block
+            f32x4 acc[RH][CH];
+#pragma unroll
+            for (int r = 0; r < RH; ++r)
+#pragma unroll
+                for (int c = 0; c < CH; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+            asm volatile("" : "+v"(dq_k), "+v"(dq_s));
+            constexpr int DEPTH = 2;                      // products whose operands are on their way
+            u32x4 kt[DEPTH], dst[DEPTH][RH];
+            auto fetch = [&](int ks) __attribute__((always_inline)) {
+                constexpr int AT = BUF * C::DS_BYTES;
+                kt[ks % DEPTH] = tr_pair(dq_k + (pass * C::K_HALF + 4096 * ks), (dq_k ^ 16) + (pass * C::K_HALF + 4096 * ks + 512));
+#pragma unroll
+                for (int r = 0; r < RH; ++r)
+                    dst[ks % DEPTH][r] = tr_pair((dq_s ^ (32 * r)) + (AT + 2048 * ks), (dq_s ^ (32 * r + 8)) + (AT + 2048 * ks + 256));
+            };
+            auto product = [&](int ks) __attribute__((always_inline)) {
+#pragma unroll
+                for (int r = 0; r < RH; ++r) acc[r][ks % CH] = mfma16<BF16>(kt[ks % DEPTH], dst[ks % DEPTH][r], acc[r][ks % CH]);
+            };
+            if (live == (1u << NW) - 1u) {
+#pragma unroll
+                for (int ks = 0; ks < NW * KB; ++ks) {
+                    if (ks == 0) {
+#pragma unroll
+                        for (int d = 0; d < DEPTH; ++d) fetch(d);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    product(ks);
+                    if (ks + DEPTH < NW * KB) fetch(ks + DEPTH);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            } else {
+#pragma unroll
+                for (int w = 0; w < NW; ++w)
+                    if (live >> w & 1u) {
+#pragma unroll
+                        for (int kb = 0; kb < KB; ++kb) {
+                            fetch(w * KB + kb);
+                            product(w * KB + kb);
+                        }
+                    }
+            }
+            const int col = 16 * db + 64 * pass + 4 * (ln >> 4);
+#pragma unroll
+            for (int r = 0; r < RH; ++r) {
+                if constexpr (CH == 2) acc[r][0] += acc[r][1];
+                const int row = 32 * i + 16 * (rh0 + r) + (ln & 15);
+                if (row >= N || col >= a.D) continue;
+                const uint32_t at = (uint32_t)row * a.dq.sn + (uint32_t)col;          // elements: a slab's bytes fit 31 bits
+                const u32x2 h = {E::pack2_rne(acc[r][0][0] * a.scale, acc[r][0][1] * a.scale), E::pack2_rne(acc[r][0][2] * a.scale, acc[r][0][3] * a.scale)};
+                if constexpr (WIDE)
+                    *reinterpret_cast<f32x4 *>(dq_slab + 4 * at) = f32x4{E::up1((uint16_t)(h.x & 0xffffu)), E::up1((uint16_t)(h.x >> 16)),
+                                                                  E::up1((uint16_t)(h.y & 0xffffu)), E::up1((uint16_t)(h.y >> 16))};
+                else
+                    *reinterpret_cast<u32x2 *>(dq_slab + 2 * at) = h;
+            }
+        }
+    };
+
+    WAIT_VMCNT(0);
+    if (a.D < HDIM && lane < 32 * KB) {               // columns of K beyond the row's end add nothing to the scores
+        for (int c = last_chunk + 1; c < 2 * KS; ++c)
+            *(LDS_PTR(u32x4))(uintptr_t)(lds0 + (c >> 3) * C::K_HALF + (key0 + lane) * 128 + (((c & 7) ^ k_swizzle(lane)) << 4)) = u32x4{0u, 0u, 0u, 0u};
+    }
+    auto iteration = [&](int i, auto st_c) __attribute__((always_inline)) {
+        constexpr int st = decltype(st_c)::value;
+        using same = std::integral_constant<int, st>;
+        using other = std::integral_constant<int, st ^ 1>;
+        __syncthreads();                              // these 32 rows have landed; the other stage is done with
+        if (i + 1 < RB) issue(i + 1, other{});
+        if constexpr (C::DS_BUFS == 2) {
+            if (i > 0) dq32(i - 1, other{});
+            if (i < RB) rows32(i, same{});
+            WAIT_VMCNT(0);
+            if (i + 1 < RB) land(other{});
+        } else {
+            rows32(i, same{});
+            WAIT_VMCNT(0);
+            if (i + 1 < RB) land(other{});
+            __syncthreads();
+            dq32(i, same{});                          // its stores are nothing that the next rows wait for
+        }
+    };
+    land(std::integral_constant<int, 0>{});
+    constexpr int EXTRA = C::DS_BUFS == 2 ? 1 : 0;    // dQ of the last rows
+    for (int i = 0; i < RB + EXTRA; i += 2) {
+        iteration(i, std::integral_constant<int, 0>{});
+        if (i + 1 < RB + EXTRA) iteration(i + 1, std::integral_constant<int, 1>{});
+    }
+    __syncthreads();
+    if (wave_valid) {
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+            if (key0 + 32 * kb >= N) break;
+            store_gradient<BF16, WIDE>(dkacc[kb], a.scale, lds0 + wave * 4096, a, a.dk, bi, hi, key0 + 32 * kb, lane);
+            store_gradient<BF16, WIDE>(dvacc[kb], 1.0f, lds0 + wave * 4096, a, a.dv, bi, hi, key0 + 32 * kb, lane);
+        }
+    }
+}
+
+template <bool BF16, int HDIM, int NW, int KB, bool WIDE> void launch(hipStream_t stream, const AttnBwdArgs &a)
+{
+    hipLaunchKernelGGL((attn_bwd_head_kernel<BF16, HDIM, NW, KB, WIDE>), dim3((unsigned)a.BH), dim3(64 * NW), 0, stream, a);
+}
+template <bool BF16, bool WIDE> bool pick(hipStream_t stream, const AttnBwdArgs &a)
+{
+    // Up to 128 keys always (see the figures at the top).  129 to 256 keys: eight wavefronts of 32 keys while every head has a CU of its
+    // own (D = 64, N = 256, the backward alone on warm inputs: 64 heads 19.7 us, four wavefronts of 64 keys 23.1; 256: 25.5, 27.9),
+    // beyond that the four, two work-groups to a CU (300: 44.4 against 38.4; 512: 50.2, 48.3).  At head dims 96 and 128 only eight
+    // fit; below a head for every second CU the two kernels' more, shorter work-groups win from 193 keys on (96 heads, N = 256, D = 128:
+    // 31.7 against 33.8 us; N = 192: 26.8 against 26.3).
+    // 257 to 512 keys: a work-group has a CU for itself and a round takes the same time however few heads it holds, so 70 % of
+    // the places of all rounds must be taken (D = 64, N = 512, two kernels against this one: 128 heads 46.8, 55.4 us; 192: 66.9, 61.4;
+    // 300: 102, 115; 350: 119, 121; 384: 126, 119; 448: 149, 125).
+    const int D = kernel_head_dim(a.D), N = a.N;
+    const long long cus = compute_units(), rounds = cus > 0 ? (a.BH + cus - 1) / cus : 1;
+    const bool own_cu = a.BH <= cus, half_filled = 2 * (long long)a.BH >= cus, filled = 10 * (long long)a.BH >= 7 * rounds * cus;
+    auto narrow = [&](auto d_c) {
+        constexpr int HDIM = decltype(d_c)::value;
+        if (N <= 128) launch<BF16, HDIM, 4, 1, WIDE>(stream, a);
+        else if (N <= 256) own_cu ? launch<BF16, HDIM, 8, 1, WIDE>(stream, a) : launch<BF16, HDIM, 4, 2, WIDE>(stream, a);
+        else if (N <= 512 && filled) launch<BF16, HDIM, 8, 2, WIDE>(stream, a);
+        else return false;
+        return true;
+    };
+    auto wide = [&](auto d_c) {
+        constexpr int HDIM = decltype(d_c)::value;
+        if (N <= 128) launch<BF16, HDIM, 4, 1, WIDE>(stream, a);
+        else if (N <= 192 || (N <= 256 && half_filled)) launch<BF16, HDIM, 8, 1, WIDE>(stream, a);
+        else return false;
+        return true;
+    };
+    return D == 32 ? narrow(std::integral_constant<int, 32>{}) : D == 64 ? narrow(std::integral_constant<int, 64>{})
+           : D == 96 ? wide(std::integral_constant<int, 96>{}) : wide(std::integral_constant<int, 128>{});
+}
+
+}  // namespace
+
+bool launch_attn_bwd_head(const AttnBwdArgs &a, bool bf16, hipStream_t stream)
+{
+    return a.grads_f32 ? pick<true, true>(stream, a) : bf16 ? pick<true, false>(stream, a) : pick<false, false>(stream, a);
+}
+
+}  // namespace sma

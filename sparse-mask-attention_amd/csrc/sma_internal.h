@@ -104,6 +104,8 @@ int compute_units();
 
 hipError_t launch_attn_fwd(const AttnArgs &a, bool bf16, hipStream_t stream);
 hipError_t launch_attn_bwd(const AttnBwdArgs &a, bool bf16, hipStream_t stream);
+// ... by the kernel that holds a whole head in one work-group, where that is the faster; false: nothing was launched
+bool launch_attn_bwd_head(const AttnBwdArgs &a, bool bf16, hipStream_t stream);
 // fp32 -> bf16 (round to nearest even), `count` (at most 3) arrays of n elements, n a multiple of 8
 hipError_t launch_to_bf16(const float *const *src, uint16_t *const *dst, int count, long long n, hipStream_t stream);
 hipError_t launch_pack_mask(const uint8_t *mask, uint32_t *packed, long long rows, int N,
