@@ -6,9 +6,11 @@
 // bit-reproducible.
 //   wavefront    32 KB keys, KB = 1 or 2 (lane = key, as in the dK/dV kernel); dK and dV are its accumulators, V fragments stay in
 //                registers.  With KB = 2 every Q and dO operand that is read from LDS serves two products.
-//   rows         32 at a time, in a ring of two stages: Q, dO, the mask words of each wavefront's keys, and Q scaled and rounded as
-//                the forward does it, so that the probabilities fit its lse (the wavefront that copied eight rows scales
-//                them; as VALU work of every wavefront instead it cost 4 us of 62 on 192 heads, N = 512, D = 64).
+//   rows         32 at a time, in a ring of two stages: Q, dO, the mask words of each wavefront's keys.  The wavefront that has copied
+//                eight rows also forms their delta (O comes with them) and Q scaled and rounded as the forward does it, so that
+//                the probabilities fit its lse, in the place of O.  Delta of all rows before the first, as the two kernels have it,
+//                made every work-group begin with twice the bytes while nothing is computed: 64.6 -> 57.7 us on 192 heads, N = 512,
+//                D = 64, 175 -> 156 on 1024, N = 256, D = 128.  Scaling by every wavefront for itself: 4 us more on the first.
 //   K            all of it in LDS, both as the operand of S and, read transposed, of dQ
 //   dS           to LDS as [key][row], 64 bytes a key; after the next barrier the wavefronts share dQ^T = K^T dS^T of the 32 rows
 //                in blocks of 16 x 16.  Eight wavefronts have two such buffers and one barrier for 32 rows; four have one,
@@ -17,16 +19,16 @@
 // and dS by 8 bytes with those of key / 4 in the order (1, 2, 0): their row accesses and the transposing reads of 16 keys x 16
 // columns that dQ needs are free of bank conflicts (2.3 cycles a read on a full CU, 2.1 for a linear one).
 //
-// Forward + backward with every step's inputs from memory, in us, before (two kernels, up to 256 keys at head dims up to 64 an
-// earlier form of this one) -> now:
-//   D =  64   N = 512: 192 heads 90.9 -> 84.8, 256: 123.7 -> 101.7;  N = 256: 512 heads 73.9 -> 70.9, 2048: 282 -> 248;
-//             1024 heads: N = 160 94.2 -> 80.1;  2048 heads: N = 128 106.0 -> 98.4, N = 32 41.3 -> 37.2
-//   D = 128   N = 256: 256 heads 72.7 -> 63.1, 1024: 274 -> 236;  1024 heads: N = 128 123.1 -> 93.7, N = 64 70.0 -> 49.0
-//   D =  32   1024 heads, N = 256: 90.7 -> 82.8;  D = 96: 1024 heads, N = 128: 86.1 -> 77.1
-// What bounds it: on 256 heads, N = 512, D = 64 (fp16, 62 us) a SIMD's 6500 cycles for 32 rows hold 2560 of the matrix cores, about 2700
-// of the vector ALU and, for the CU, 3200 of LDS; the barrier keeps the eight wavefronts in the same phase, which is bound by one of
-// them at a time.  Starting half of the wavefronts with dQ and half with S changed nothing.  Many short sequences are bound by
-// memory: 2048 heads, N = 32: 4.2 TB/s.
+// The backward alone, inputs in turn, in us, before (two kernels, up to 256 keys at head dims up to 64 an earlier form of this
+// one) -> now:
+//   D =  64   N = 512: 192 heads 69.5 -> 57.7, 256: 93.6 -> 66.4;  N = 256: 1024 heads 102.4 -> 81.6, causal 95.7 -> 75.6, 256: 26.8 -> 24.7;
+//             2048 heads, N = 32: 26.6 -> 20.0
+//   D = 128   N = 256: 256 heads 54.0 -> 40.4, 1024: 212 -> 156;  1024 heads: N = 128 98.8 -> 64.3, N = 64 54.9 -> 31.9
+//   D =  32   1024 heads, N = 256: 66.1 -> 53.7;  192, N = 512: 45.3 -> 39.8;   D = 96   1024 heads, N = 128: 57.1 -> 48.1
+// What bounds it: on 256 heads, N = 512, D = 64 (66 us) a SIMD's 5800 cycles for 32 rows hold 2560 of the matrix cores, about 2700 of the
+// vector ALU and, for the CU, 3200 of LDS; the barrier keeps the eight wavefronts in the same phase, which is bound by one of them at a
+// time.  Starting half of the wavefronts with dQ and half with S changed nothing.  Prologue and epilogue, some 20000 cycles
+// of 130000, move 256 KB of every CU at what memory gives.
 #include <type_traits>
 
 #include "attn_bwd_common.h"
@@ -43,12 +45,13 @@ template <int HDIM, int NW, int KB> struct HeadCfg {
     static constexpr int DS_BUFS = NW == 8 ? 2 : 1;
     static constexpr int PART = NH * 4096;                          // 32 rows of one matrix
     static constexpr bool LAND = !(NW == 4 && NH == 2);             // scaled Q in LDS (there two work-groups would not fit)
-    static constexpr int OFF_WORDS = (LAND ? 3 : 2) * PART;         // a stage: Q, dO, scaled Q, each wavefront's mask words
-    static constexpr int STAGE_BYTES = OFF_WORDS + NW * 256;
+    // a stage: Q, dO, scaled Q (before that O, of which delta is formed), each wavefront's mask words, lse and delta
+    static constexpr int OFF_WORDS = (LAND ? 3 : 2) * PART;
+    static constexpr int OFF_LSE = OFF_WORDS + NW * 256, OFF_DELTA = OFF_LSE + 256;       // (a copy fills 64 places of lse)
+    static constexpr int STAGE_BYTES = OFF_DELTA + 128;
     static constexpr int OFF_STAGE = OFF_DS + DS_BUFS * DS_BYTES;
-    static constexpr int OFF_LSE = OFF_STAGE + 2 * STAGE_BYTES;
-    static constexpr int OFF_DELTA = OFF_LSE + KEYS * 4;
-    static constexpr int LDS_BYTES = OFF_DELTA + KEYS * 4;
+    static constexpr int OFF_LIVE = OFF_STAGE + 2 * STAGE_BYTES;    // [buffer][wavefront]
+    static constexpr int LDS_BYTES = OFF_LIVE + 64;
 };
 
 // 16 x 16 x 32 products
@@ -92,9 +95,10 @@ __global__ __launch_bounds__(64 * NW, HDIM <= 64 && KB == 1 && NW == 4 ? 3 : 2) 
     const int last_chunk = (a.D >> 3) - 1;
     auto chunk_at = [&](int c) __attribute__((always_inline)) -> uint32_t { return (uint32_t)(c < last_chunk ? c : last_chunk) << 4; };
     auto k_swizzle = [](int row) __attribute__((always_inline)) { const int p = (row >> 1) & 7; return (p & 4) | ((p & 1) << 1) | ((p >> 1) & 1); };
-    const int key0 = wave * (32 * KB);                // this wavefront's keys; of delta and lse, its rows
+    const int key0 = wave * (32 * KB);                // this wavefront's keys
     const bool wave_valid = key0 < N;                 // wave-uniform
     const int part = wave & 3;
+    u32x4 o_next[C::LAND ? 1 : NH];                   // O where it does not go through LDS
     auto issue = [&](int i, auto st_c) __attribute__((always_inline)) {
         constexpr int SO = C::OFF_STAGE + decltype(st_c)::value * C::STAGE_BYTES;
         int ln = lane;
@@ -109,8 +113,21 @@ __global__ __launch_bounds__(64 * NW, HDIM <= 64 && KB == 1 && NW == 4 ? 3 : 2) 
             async_copy_b128_at<AT>(lds0 + part * 1024, mat, r + pchunk);
             if constexpr (NH == 2) async_copy_b128_at<AT + 4096>(lds0 + part * 1024, mat, r + pchunk2);
         };
-        if (NW == 4 || wave < 4) rows(std::integral_constant<int, 0>{}, qb, a.q.sn);
-        if (NW == 4 || wave >= 4) rows(std::integral_constant<int, C::PART>{}, dob, a.dout.sn);
+        if (wave < 4) {
+            rows(std::integral_constant<int, 0>{}, qb, a.q.sn);
+            rows(std::integral_constant<int, C::PART>{}, dob, a.dout.sn);
+            if constexpr (C::LAND) {
+                rows(std::integral_constant<int, 2 * C::PART>{}, ob, a.out.sn);
+            } else {
+                const uint32_t r = __umul24(row, 2u * a.out.sn);
+                o_next[0] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const unsigned char *>(ob) + (r + pchunk));
+                o_next[NH - 1] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const unsigned char *>(ob) + (r + pchunk2));
+            }
+        }
+        if (wave == NW - 1) {
+            const int lrow = 32 * i + (ln & 31) < N ? 32 * i + (ln & 31) : N - 1;
+            async_copy_b32_at<SO + C::OFF_LSE>(lds0, a.lse + (size_t)bh * N, (uint32_t)(lrow * 4));
+        }
         const int mword = KB == 2 ? wave * 2 + (ln >> 5) : wave, wi = mword < nw ? mword : nw - 1;
         const int mrow = 32 * i + (ln & 31) < N ? 32 * i + (ln & 31) : N - 1;
         async_copy_b32_at<SO + C::OFF_WORDS>(lds0 + wave * 256, mb, (uint32_t)((mrow * nw + wi) * 4));
@@ -125,38 +142,19 @@ __global__ __launch_bounds__(64 * NW, HDIM <= 64 && KB == 1 && NW == 4 ? 3 : 2) 
     }
     issue(0, std::integral_constant<int, 0>{});
 
-    // ---- V^T fragments of this lane's keys, delta and lse of its rows
+    // ---- V^T fragments of this lane's keys
     u32x4 vf[KB][KS];
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
         const int key = key0 + 32 * kb + l32, kr = key < N ? key : N - 1;
-        u32x4 dof[KS], of[KS];
-        const uint16_t *vp = vb + (size_t)kr * a.v.sn, *dop = dob + (size_t)kr * a.dout.sn, *op = ob + (size_t)kr * a.out.sn;
+        const uint16_t *vp = vb + (size_t)kr * a.v.sn;
 #pragma unroll
         for (int s = 0; s < KS; ++s) {                // columns beyond the row's end: its last ones, set to zero
-            const int col = 16 * s + 8 * hh, at = col < a.D ? col : a.D - 8;
-            const uint32_t ok = col < a.D ? 0xffffffffu : 0u;
-            vf[kb][s] = *reinterpret_cast<const u32x4 *>(vp + at) & ok;
-            dof[s] = *reinterpret_cast<const u32x4 *>(dop + at) & ok;
-            of[s] = *reinterpret_cast<const u32x4 *>(op + at);
-        }
-        const float l = a.lse[(size_t)bh * N + kr];
-        float delta = 0.f;
-#pragma unroll
-        for (int s = 0; s < KS; ++s)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                delta += E::up1((uint16_t)(dof[s][i] & 0xffffu)) * E::up1((uint16_t)(of[s][i] & 0xffffu)) +
-                         E::up1((uint16_t)(dof[s][i] >> 16)) * E::up1((uint16_t)(of[s][i] >> 16));
-        delta = xhalf_sum(delta);
-        // rows that kept nothing or lie beyond N: probability 0
-        const bool dead = key >= N || l == -__builtin_inff();
-        if (hh == 0) {
-            *(LDS_PTR(float))(uintptr_t)(lds0 + C::OFF_LSE + 4 * key) = dead ? -__builtin_inff() : -l * LOG2E;
-            *(LDS_PTR(float))(uintptr_t)(lds0 + C::OFF_DELTA + 4 * key) = -delta;
-            if (key < N) a.delta[(size_t)bh * N + key] = delta;
+            const int col = 16 * s + 8 * hh;
+            vf[kb][s] = *reinterpret_cast<const u32x4 *>(vp + (col < a.D ? col : a.D - 8)) & (col < a.D ? 0xffffffffu : 0u);
         }
     }
+    if (tid < 16) *(LDS_PTR(uint32_t))(uintptr_t)(lds0 + C::OFF_LIVE + 4 * tid) = 0u;
     const bool keys_end = key0 + 32 * KB > N;         // wave-uniform: some of this wavefront's keys do not exist
 
     f32x16 dkacc[KB][OB], dvacc[KB][OB];
@@ -201,17 +199,46 @@ __global__ __launch_bounds__(64 * NW, HDIM <= 64 && KB == 1 && NW == 4 ? 3 : 2) 
             x[j] = E::pack2_rne(E::up1((uint16_t)(x[j] & 0xffffu)) * a.q_scale, E::up1((uint16_t)(x[j] >> 16)) * a.q_scale);
         return x;
     };
-    auto land = [&](auto st_c) __attribute__((always_inline)) {      // ... of the rows that this wavefront has copied
-        if constexpr (C::LAND) {
-            if (NW == 8 && wave >= 4) return;
-            const uint32_t at = lane_at * 4 - 3 * lds0 + (C::OFF_STAGE + decltype(st_c)::value * C::STAGE_BYTES + part * 1024);
+    // after the copies of 32 rows, by the wavefronts that have made them: delta, scaled Q (in the place of O), lse
+    auto land = [&](int i, auto st_c) __attribute__((always_inline)) {
+        constexpr int SO = C::OFF_STAGE + decltype(st_c)::value * C::STAGE_BYTES;
+        if (wave < 4) {
+            int ln = lane;
+            asm volatile("" : "+v"(ln));
+            const int prow = 8 * part + (ln >> 3), chunk = (ln & 7) ^ bitrev3((prow >> 1) & 7);
+            const uint32_t at = lds0 + 16 * ln + (SO + part * 1024);
+            float delta = 0.f;
 #pragma unroll
-            for (int half = 0; half < NH; ++half)
-                *(LDS_PTR(u32x4))(uintptr_t)(at + 2 * C::PART + half * 4096) = scaled(lds_read_b128(at + half * 4096));
+            for (int half = 0; half < NH; ++half) {
+                const u32x4 x = lds_read_b128(at + C::PART + half * 4096);
+                const u32x4 o = C::LAND ? lds_read_b128(at + 2 * C::PART + half * 4096) : o_next[C::LAND ? 0 : half];
+                float d = 0.f;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    d = __builtin_fmaf(E::up1((uint16_t)(x[j] & 0xffffu)), E::up1((uint16_t)(o[j] & 0xffffu)), d);
+                    d = __builtin_fmaf(E::up1((uint16_t)(x[j] >> 16)), E::up1((uint16_t)(o[j] >> 16)), d);
+                }
+                delta += chunk + 8 * half <= last_chunk ? d : 0.f;            // beyond the row's end its last columns stand once more
+                if constexpr (C::LAND) *(LDS_PTR(u32x4))(uintptr_t)(at + 2 * C::PART + half * 4096) = scaled(lds_read_b128(at + half * 4096));
+            }
+            // the eight lanes of a row
+            delta += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, delta), 0xB1, 0xf, 0xf, true));
+            delta += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, delta), 0x4E, 0xf, 0xf, true));
+            delta += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, delta), 0x141, 0xf, 0xf, true));
+            if ((ln & 7) == 0) {
+                *(LDS_PTR(float))(uintptr_t)(lds0 + (SO + C::OFF_DELTA) + 4 * prow) = -delta;
+                if (32 * i + prow < N) a.delta[(size_t)bh * N + 32 * i + prow] = delta;
+            }
+        }
+        if (wave == NW - 1 && lane < 32) {
+            const uint32_t at = lane_at + (SO + C::OFF_LSE);
+            const float l = *(LDS_PTR(float))(uintptr_t)at;
+            // rows that kept nothing or lie beyond N: probability 0
+            *(LDS_PTR(float))(uintptr_t)at = 32 * i + lane >= N || l == -__builtin_inff() ? -__builtin_inff() : -l * LOG2E;
         }
     };
     // ---- 32 query rows: dV, dK, and dS into LDS
-    auto rows32 = [&](int i, auto st_c) __attribute__((always_inline)) {
+    auto rows32 = [&](auto st_c) __attribute__((always_inline)) {
         constexpr int st = decltype(st_c)::value;
         constexpr int DS = C::DS_BUFS == 2 ? st * C::DS_BYTES : 0;
         constexpr int SB = st * C::STAGE_BYTES;
@@ -226,21 +253,13 @@ __global__ __launch_bounds__(64 * NW, HDIM <= 64 && KB == 1 && NW == 4 ? 3 : 2) 
             word &= left >= 32 ? 0xffffffffu : left > 0 ? (1u << left) - 1u : 0u;
             *(LDS_PTR(uint32_t))(uintptr_t)(word_at) = word;
         }
-        const bool live = wave_valid && __builtin_amdgcn_ballot_w64(word != 0u) != 0ull;
-        // dQ leaves out the wavefronts that have kept nothing; their flags take the place of the rows before these in lse
-        if (i > 0) {
-            if (lane == 0) *(LDS_PTR(uint32_t))(uintptr_t)(lds0 + C::OFF_LSE + 128 * (i - 1) + 4 * wave) = live ? 1u : 0u;
-        } else if (!live) {
-#pragma unroll
-            for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-                for (int g = 0; g < 4; ++g) *(LDS_PTR(u32x2))(uintptr_t)((ds_at ^ (16 * g)) + DS + 2048 * kb) = u32x2{0u, 0u};
-        }
+        const bool live = __builtin_amdgcn_ballot_w64(word != 0u) != 0ull;         // dQ leaves out the others
+        if (lane == 0) *(LDS_PTR(uint32_t))(uintptr_t)(lds0 + C::OFF_LIVE + (C::DS_BUFS == 2 ? 32 * st : 0) + 4 * wave) = live ? 1u : 0u;
         if (!live) return;
         // Operands are requested a step ahead of their use, and scheduling barriers hold that order: left alone, the compiler
         // requests each just before it is needed, since registers are short, and the wavefront sits out some 30 LDS round
         // trips one after the other.
-        const uint32_t rows = half_at + (C::OFF_LSE + i * 128);
+        const uint32_t rows = half_at + (C::OFF_STAGE + SB + C::OFF_LSE);
         auto q_frag = [&](int s) __attribute__((always_inline)) { return lds_read_b128((row_at ^ (32 * (s & 3))) + SB + (C::LAND ? 2 * C::PART : 0) + (s >> 2) * 4096); };
         auto o_frag = [&](int s) __attribute__((always_inline)) { return lds_read_b128((row_at ^ (32 * (s & 3))) + SB + C::PART + (s >> 2) * 4096); };
         auto k_frag = [&](int s, int kb) __attribute__((always_inline)) { return lds_read_b128((key_at ^ (32 * (s & 3))) + (s >> 2) * C::K_HALF + kb * 4096); };
@@ -366,8 +385,8 @@ __global__ __launch_bounds__(64 * NW, HDIM <= 64 && KB == 1 && NW == 4 ? 3 : 2) 
         if (NW == 8 && wave >= NW / 2) __builtin_amdgcn_s_setprio(1);
         int ln = lane;
         asm volatile("" : "+v"(ln));
-        uint32_t live = (1u << NW) - 1u;
-        if (i > 0) live &= (uint32_t)__builtin_amdgcn_ballot_w64(*(LDS_PTR(const uint32_t))(uintptr_t)(lds0 + C::OFF_LSE + 128 * (i - 1) + 4 * (ln & (NW - 1))) != 0u);
+        const uint32_t flag = *(LDS_PTR(const uint32_t))(uintptr_t)(lds0 + (C::OFF_LIVE + 32 * BUF) + 4 * (ln & (NW - 1)));
+        const uint32_t live = (uint32_t)__builtin_amdgcn_ballot_w64(flag != 0u) & ((1u << NW) - 1u);
 #pragma unroll
         for (int pass = 0; pass < PASSES; ++pass) {
             if (pass > 0 && wave + NW * pass >= NDB) break;
@@ -444,18 +463,18 @@ __global__ __launch_bounds__(64 * NW, HDIM <= 64 && KB == 1 && NW == 4 ? 3 : 2) 
         if (i + 1 < RB) issue(i + 1, other{});
         if constexpr (C::DS_BUFS == 2) {
             if (i > 0) dq32(i - 1, other{});
-            if (i < RB) rows32(i, same{});
+            if (wave_valid && i < RB) rows32(same{});
             WAIT_VMCNT(0);
-            if (i + 1 < RB) land(other{});
+            if (i + 1 < RB) land(i + 1, other{});
         } else {
-            rows32(i, same{});
+            if (wave_valid) rows32(same{});
             WAIT_VMCNT(0);
-            if (i + 1 < RB) land(other{});
+            if (i + 1 < RB) land(i + 1, other{});
             __syncthreads();
             dq32(i, same{});                          // its stores are nothing that the next rows wait for
         }
     };
-    land(std::integral_constant<int, 0>{});
+    land(0, std::integral_constant<int, 0>{});
     constexpr int EXTRA = C::DS_BUFS == 2 ? 1 : 0;    // dQ of the last rows
     for (int i = 0; i < RB + EXTRA; i += 2) {
         iteration(i, std::integral_constant<int, 0>{});
@@ -478,17 +497,18 @@ template <bool BF16, int HDIM, int NW, int KB, bool WIDE> void launch(hipStream_
 }
 template <bool BF16, bool WIDE> bool pick(hipStream_t stream, const AttnBwdArgs &a)
 {
-    // Up to 128 keys always (see the figures at the top).  129 to 256 keys: eight wavefronts of 32 keys while every head has a CU of its
-    // own (D = 64, N = 256, the backward alone on warm inputs: 64 heads 19.7 us, four wavefronts of 64 keys 23.1; 256: 25.5, 27.9),
-    // beyond that the four, two work-groups to a CU (300: 44.4 against 38.4; 512: 50.2, 48.3).  At head dims 96 and 128 only eight
-    // fit; below a head for every second CU the two kernels' more, shorter work-groups win from 193 keys on (96 heads, N = 256, D = 128:
-    // 31.7 against 33.8 us; N = 192: 26.8 against 26.3).
-    // 257 to 512 keys: a work-group has a CU for itself and a round takes the same time however few heads it holds, so 70 % of
-    // the places of all rounds must be taken (D = 64, N = 512, two kernels against this one: 128 heads 46.8, 55.4 us; 192: 66.9, 61.4;
-    // 300: 102, 115; 350: 119, 121; 384: 126, 119; 448: 149, 125).
+    // Backward alone, inputs in turn, the two kernels of attn_bwd.hip against this one:
+    // up to 256 keys it is the faster at any number of heads (D = 64, N = 256: 8 heads 18.8, 17.6 us, 96: 21.1, 19.2; D = 128: 32 heads 28.7, 25.6).
+    // 129 to 256 keys at head dims up to 64: eight wavefronts of 32 keys while every head has a CU of its own (64 heads 19.7 us, four
+    // wavefronts of 64 keys 23.1; 256: 25.5, 27.9), beyond that the four, two work-groups to a CU (300: 44.4 against 38.4).
+    // 257 to 512 keys: a work-group has a CU for itself and a round takes the same time however few heads it holds, so that
+    // most of the places must be taken, five eighths or, where fewer than 385 keys leave wavefronts without any and at head dims up to 32 after
+    // the first round, three quarters.  D = 64, N = 512: 128 heads 50.9, 53.3 us; 160: 63.7, 56.1; 300: 109.1, 110.0; 320: 111.3, 110.6; 600: 201,
+    // 173; N = 300: 160 heads 33.3, 34.4, 320: 63.5, 70.7; N = 320: 192 heads 41.4, 36; D = 32, N = 512: 160 heads 42.5, 39.4, 320: 71.5, 78.8.
     const int D = kernel_head_dim(a.D), N = a.N;
     const long long cus = compute_units(), rounds = cus > 0 ? (a.BH + cus - 1) / cus : 1;
-    const bool own_cu = a.BH <= cus, half_filled = 2 * (long long)a.BH >= cus, filled = 10 * (long long)a.BH >= 7 * rounds * cus;
+    const bool own_cu = a.BH <= cus;
+    const bool filled = 8 * (long long)a.BH >= (N > 384 && (D == 64 || rounds == 1) ? 5 : 6) * rounds * cus;
     auto narrow = [&](auto d_c) {
         constexpr int HDIM = decltype(d_c)::value;
         if (N <= 128) launch<BF16, HDIM, 4, 1, WIDE>(stream, a);
@@ -500,7 +520,7 @@ template <bool BF16, bool WIDE> bool pick(hipStream_t stream, const AttnBwdArgs 
     auto wide = [&](auto d_c) {
         constexpr int HDIM = decltype(d_c)::value;
         if (N <= 128) launch<BF16, HDIM, 4, 1, WIDE>(stream, a);
-        else if (N <= 192 || (N <= 256 && half_filled)) launch<BF16, HDIM, 8, 1, WIDE>(stream, a);
+        else if (N <= 256) launch<BF16, HDIM, 8, 1, WIDE>(stream, a);
         else return false;
         return true;
     };
