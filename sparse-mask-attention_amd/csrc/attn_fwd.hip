@@ -110,7 +110,7 @@ template <int N> __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_
 // BYPRODUCTS (with BYTEMASK): the caller wants the packed words and / or the tile map of the mask
 // left behind; a separate instantiation, so that the kernel of a caller who wants neither carries
 // none of that code (it measured 1.5 % on the headline workload even when switched off at run time).
-// PAIRS (with BYTEMASK, head dims up to 64, N a multiple of 128): the mask bytes of
+// PAIRS (FETCH != 0, with BYTEMASK, head dims up to 64): the mask bytes of
 // TWO key tiles are requested at once, every second visit: 128 bytes per row, i.e. whole cache lines
 // where one tile's 64 bytes are half of one.  The forward from the boolean mask measured 1 to 5 %
 // faster this way on random masks of every length tried (128 to 2048) and 7 % on the
@@ -118,11 +118,10 @@ template <int N> __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_
 // step (the even-progress case of the launcher, e.g. the headline shape): there the first visit,
 // which waits for twice the bytes, is not hidden behind other work-groups' work, it measured 1 to 4 %
 // slower, and the launcher leaves it off.
-// AHEAD (like PAIRS, any other N): a tile's mask bytes are requested two tiles ahead.  A wave has turned its bytes of a
-// tile into words before it requests others, so the tile's own slot takes those of the tile after next.  Rows that
-// start anywhere come as parts of two cache lines, and one tile's time does not cover what a mask that is in no cache
-// takes: 8 x 16 heads, N = 1000, bf16: 60.5 -> 55.8 us.  Not where the whole grid is one round in step, whose first
-// requests all come at once and where it costs 1.6 % (16 x 12, N = 512: 20.2 -> 20.6 us).
+// FETCH = 1: N a multiple of 128: no row and no pair ends within a request.  FETCH = 2: any N; the ends cost registers and 2 % (8 x 16
+// heads, N = 1024: 55.9 -> 57.3 us), so the lengths that have none keep their own.  Against one tile's bytes requested two
+// tiles ahead, which is what other lengths had before: 8 x 16 heads, bf16, N = 1000: 61.3 -> 59.0 us, 960: 57.1 -> 55.0; 4 x 16,
+// N = 2000: 109 -> 105; D = 32, 16 x 16, N = 1000: 90.6 -> 86.3; up to 500 keys the same.
 // SPLIT: for grids that leave most of the chip idle.  The four wavefronts of a work-group share 32 query
 // rows and take every fourth key tile each, with a K and a V buffer of their own: no barriers, four times
 // the work-groups, a quarter of the serial chain; what they found is combined through LDS at the end.
@@ -134,8 +133,8 @@ template <bool BF16, bool POSTMUL, bool PACKED_ROWS, int HDIM, bool BYTEMASK = f
           int FETCH = 0, bool SPLIT = false>
 __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ? 2 : 3) void attn_fwd_kernel(const AttnArgs a)
 {
-    static_assert(FETCH == 0 || (BYTEMASK && HDIM <= 64 && !SPLIT), "PAIRS, AHEAD: byte mask, two byte slots");
-    constexpr bool PAIRS = FETCH == 1, AHEAD = FETCH == 2;
+    static_assert(FETCH == 0 || (BYTEMASK && HDIM <= 64 && !SPLIT), "PAIRS: byte mask, two byte slots");
+    constexpr bool PAIRS = FETCH != 0, WHOLE = FETCH == 1;
     using E = Elem<BF16>;
     constexpr int NH = HDIM > 64 ? 2 : 1;         // 64-column tiles per matrix
     constexpr int KS = HDIM / 16;                 // MFMA steps of the QK^T chain
@@ -252,20 +251,49 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     };
     // PAIRS: four copies per wave and pair of tiles; lane i of copy j fills (row 8j + i/8, position i%8)
     // from the row's chunk (i%8) ^ ((row >> 1) & 7).  (row >> 1) & 7 is (i/8 >> 1) for j = 0, 2 and that
-    // plus 4 for j = 1, 3: one lane offset and the same with chunk bit 2 flipped (N is a multiple of
-    // 128, so the low seven bits of the offset are the chunk alone).
+    // plus 4 for j = 1, 3.  In a pair that the row ends in, chunks move back as in issue_mask.
     uint32_t pair_voff = 0u;
-    if constexpr (PAIRS) {
-        const int row = lane >> 3;
-        pair_voff = (uint32_t)(row_base + row) * (uint32_t)N + (uint32_t)(((lane & 7) ^ (row >> 1)) << 4);
-    }
+    if constexpr (PAIRS) pair_voff = (uint32_t)(row_base + (lane >> 3)) * (uint32_t)N + (uint32_t)(((lane & 7) ^ (lane >> 4)) << 4);
     auto issue_mask_pair = [&](int p) __attribute__((always_inline)) {      // bytes of tiles 2p and 2p + 1
         const uint8_t *src = reinterpret_cast<const uint8_t *>(mb) + (size_t)p * (2 * BN);
         const uint32_t dst = lds0 + wave * 4096;
-        async_copy_b128_at<OFF_MASK>(dst, src, pair_voff);
-        async_copy_b128_at<OFF_MASK + 1024>(dst, src + (size_t)8 * N, pair_voff ^ 64u);
-        async_copy_b128_at<OFF_MASK + 2048>(dst, src + (size_t)16 * N, pair_voff);
-        async_copy_b128_at<OFF_MASK + 3072>(dst, src + (size_t)24 * N, pair_voff ^ 64u);
+        if constexpr (WHOLE) {                   // the low seven bits of the lane offset are the chunk alone
+            async_copy_b128_at<OFF_MASK>(dst, src, pair_voff);
+            async_copy_b128_at<OFF_MASK + 1024>(dst, src + (size_t)8 * N, pair_voff ^ 64u);
+            async_copy_b128_at<OFF_MASK + 2048>(dst, src + (size_t)16 * N, pair_voff);
+            async_copy_b128_at<OFF_MASK + 3072>(dst, src + (size_t)24 * N, pair_voff ^ 64u);
+            return;
+        }
+        int ln = lane;
+        asm volatile("" : "+v"(ln));             // opaque: what follows from it is made anew each time instead of kept in registers
+        const uint32_t chunk = (uint32_t)(((ln & 7) ^ (ln >> 4)) << 4);
+        uint32_t vo[4] = {pair_voff, pair_voff + 64u - 2u * (chunk & 64u), 0u, 0u};
+        vo[2] = vo[0];
+        vo[3] = vo[1];
+        size_t step = (size_t)8 * N;                                         // eight rows
+        if (row_base + 32 > N) {                                             // rows beyond N: copy row N - 1 instead
+            step = 0;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int grow = row_base + 8 * j + (ln >> 3);
+                vo[j] = (uint32_t)(grow < N ? grow : N - 1) * (uint32_t)N + (chunk ^ (64u * (j & 1)));
+            }
+        }
+        const uint32_t row_end = (uint32_t)(N - p * (2 * BN));               // bytes of the row left
+        if (row_end < 2u * BN) {
+            const uint32_t back = p > 0 ? 16u : 0u;
+            src -= back;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t end = (chunk ^ (64u * (j & 1))) + 16u;
+                vo[j] += back;
+                if (end > row_end) vo[j] -= end - row_end;
+            }
+        }
+        async_copy_b128_at<OFF_MASK>(dst, src, vo[0]);
+        async_copy_b128_at<OFF_MASK + 1024>(dst, src + step, vo[1]);
+        async_copy_b128_at<OFF_MASK + 2048>(dst, src + 2 * step, vo[2]);
+        async_copy_b128_at<OFF_MASK + 3072>(dst, src + 3 * step, vo[3]);
     };
     // BYTEMASK: where this lane's row of packed words goes, if the caller wants them ([Bm, Hm, N, nw]
     // like the mask; a mask shared between batch entries / heads is written by the first of them)
@@ -613,7 +641,6 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         } else {
             issue_kv(t_first, integral_constant<int, 0>{});
             issue_mask(t_first, integral_constant<int, 0>{});
-            if (AHEAD && T > 1) issue_mask(1, integral_constant<int, 1>{});
         }
     }
     // small LDS table for the mask: entry n (16 B) holds four floats, float j = (bit j of n) ? 0 : -inf
@@ -622,7 +649,6 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     if (even_progress && n_visits >= 4) __builtin_amdgcn_s_setprio(3);
     if (SPLIT) { if (t_first < T) wait_vmcnt<8 * NH + C::MASK_COPIES>(); else wait_vmcnt<0>(); }
     else if (PAIRS) wait_vmcnt<8>();                   // q has landed; 4 mask and 4 K/V copies may still be in flight
-    else if (AHEAD && T > 1) wait_vmcnt<C::COPIES + C::MASK_COPIES>();
     else if (t_first < T) wait_vmcnt<C::COPIES>();     // q has landed; the copies of the first tile may still be in flight
     else wait_vmcnt<0>();
     // ---- Q^T as MFMA B operands, scaled by scale*log2(e)/post_mul:
@@ -840,18 +866,13 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
             else if (visits == (3 * n_visits) / 4) __builtin_amdgcn_s_setprio(0);
         }
         ++visits;
-        // the copies of tile t have landed; the mask bytes of the next may be in flight, they are always the youngest
-        if (AHEAD && t + 1 < T) wait_vmcnt<C::MASK_COPIES>(); else wait_vmcnt<0>();
+        wait_vmcnt<0>();          // the copies of tile t have landed
         if (ragged && t == T - 1) zero_tail_rows(t, SLOT);
         __syncthreads();          // tile t landed for every wave; the stage of the previous visit is free
         const u32x2 w2 = mask_words(t, SLOT);
         if (t_next < T) {       // K/V first: the MFMA operands are what the next visit needs first (1-2 % with a byte mask)
             issue_kv(t_next, integral_constant<int, SLOT2>{});
-            if constexpr (!AHEAD) issue_mask(t_next, integral_constant<int, SLOT2>{});
-        }
-        if (AHEAD && t + 2 < T) {
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // this wave's bytes of tile t have been read
-            issue_mask(t + 2, integral_constant<int, SLOT>{});
+            issue_mask(t_next, integral_constant<int, SLOT2>{});
         }
         compute_tile(w2, (uint32_t)(SLOT * STAGE_BYTES));
     };
@@ -878,7 +899,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
             if (tn < T) issue_own_v(tn);
         }
     } else if constexpr (PAIRS) {
-        // Every tile is visited (there is no tile map with a boolean mask) and their number is even.
+        // Every tile is visited (there is no tile map with a boolean mask).
         // Copies in flight, oldest first, at the top of an even visit t: the bytes of the pair
         // (t, t + 1), then K/V of t; after its barrier K/V of t + 1 and then the bytes of the next
         // pair are requested, and the odd visit requests K/V of t + 2 after its barrier: the bytes of
@@ -897,14 +918,18 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
             progress();
             wait_vmcnt<4>();                                  // this wave's bytes of the pair have landed
             const u32x2 w_even = mask_words(t, 0, 0);
-            const u32x2 w_odd = mask_words(t + 1, 0, 1);
+            u32x2 w_odd = {0u, 0u};
+            if (WHOLE || t + 1 < T) w_odd = mask_words(t + 1, 0, 1);
             wait_vmcnt<0>();                                  // K/V of tile t
+            if (!WHOLE && ragged && t == T - 1) zero_tail_rows(t, 0);
             __syncthreads();
-            issue_kv(t + 1, integral_constant<int, 1>{});
+            if (WHOLE || t + 1 < T) issue_kv(t + 1, integral_constant<int, 1>{});
             if (t + 2 < T) issue_mask_pair((t >> 1) + 1);     // the words above are in registers: the bytes may go
             compute_tile(w_even, 0u);
+            if (!WHOLE && t + 1 >= T) break;
             progress();
             if (t + 2 < T) wait_vmcnt<4>(); else wait_vmcnt<0>();   // K/V of tile t + 1 (the next pair's bytes may be on their way)
+            if (!WHOLE && ragged && t + 1 == T - 1) zero_tail_rows(t + 1, 1);
             __syncthreads();
             if (t + 2 < T) issue_kv(t + 2, integral_constant<int, 0>{});
             compute_tile(w_odd, (uint32_t)STAGE_BYTES);
@@ -1017,7 +1042,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
 
 // The instance for (element type, post-multiplier, row strides) and the kind of mask: 0 packed words, 1
 // boolean bytes, 2 the same with by-products, 3 and 4 those with two tiles' bytes per request, 5 to 7 the first
-// three with the keys split between the wavefronts, 8 and 9 (1 and 2) with the bytes two tiles ahead.  This file is
+// three with the keys split between the wavefronts, 8 and 9 as 3 and 4 at any N.  This file is
 // compiled once per head dim for the instances, side by side, and once for the launcher.
 typedef void (*FwdKernel)(const AttnArgs);
 #ifdef SMA_FWD_HEAD_DIM
@@ -1106,8 +1131,8 @@ hipError_t launch_attn_fwd(const AttnArgs &args, bool bf16, hipStream_t stream)
     const bool packed = a.D == D && (int)a.q.sn == D && (int)a.k.sn == D && (int)a.v.sn == D;
     if (D > HD) a.tail_start = (int)groups;                   // two work-groups per CU: nobody yields
     const bool byproducts = a.mask_out != nullptr || a.map_out != nullptr;
-    // two tiles' mask bytes per request, or the bytes two tiles ahead (see PAIRS and AHEAD at the kernel), unless the grid
-    // is the single round of work-groups in step for which tail_start was set to 0 above
+    // two tiles' mask bytes per request (see PAIRS at the kernel), unless the grid is the single round of work-groups in
+    // step for which tail_start was set to 0 above
     const bool further = !split && a.byte_mask && D <= HD && a.tail_start != 0;
     if (a.byte_mask && a.N < 16) return hipErrorInvalidValue;  // a row holds at least one 16-byte copy (checked by the C-ABI layer)
     const int mask_kind = (split ? 5 : 0) + (!a.byte_mask ? 0 : (!further ? 1 : a.N % (2 * BN) == 0 ? 3 : 8) + (byproducts ? 1 : 0));
