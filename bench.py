@@ -20,7 +20,7 @@ Prints ONE JSON line.  Besides the whole-step figure it carries
   roofline_attn the packed-mask forward kernel alone against the MFMA peak (with the tile map of the
                 mask where walking it saves enough visits to pay);
   roofline_pack the packer alone against the HBM peak;
-  roofline_bwd  the backward (its two kernels, one call) against the MFMA peak, 2.5 x the forward's FLOP;
+  roofline_bwd  the backward (its kernels, one call) against the MFMA peak, 2.5 x the forward's FLOP;
   cpu_baseline  the oracle's PyTorch formulation of the same workload on the host cores.
 Every roofline carries two timings.  The plain ones repeat the launch on the same tensors, as the
 reference's protocol does (run.py:172-183): the working set of the headline workload (57 to 101 MB)
@@ -110,6 +110,8 @@ KERNEL_SOURCES = {
     "pack_mask_kernel": ("pack_mask.hip", "sma_internal.h"),
     "attn_bwd_dq_kernel": ("attn_bwd.hip", "attn_bwd_common.h", "attn_common.h", "sma_internal.h"),
     "attn_bwd_dkv_kernel": ("attn_bwd.hip", "attn_bwd_common.h", "attn_common.h", "sma_internal.h"),
+    "attn_bwd_delta_kernel": ("attn_bwd.hip", "attn_bwd_common.h", "attn_common.h", "sma_internal.h"),
+    "attn_bwd_both_kernel": ("attn_bwd.hip", "attn_bwd_common.h", "attn_common.h", "sma_internal.h"),
     "attn_bwd_head_kernel": ("attn_bwd_head.hip", "attn_bwd_common.h", "attn_common.h", "sma_internal.h"),
 }
 
@@ -372,8 +374,11 @@ def main():
     del mp
     attn_tflops = w.dense_flops / (attn_ms * 1e-3) / 1e12
     pack_gbps = w.pack_bytes / (pack_ms * 1e-3) / 1e9
-    # the workloads of at most 512 keys run the backward that holds a whole head in one work-group
-    bwd_kernels = ("attn_bwd_head_kernel",) if w.N <= 512 else ("attn_bwd_dq_kernel", "attn_bwd_dkv_kernel")
+    # the workloads of at most 512 keys run the backward that holds a whole head in one work-group, those with a tile map dQ and
+    # dK/dV in one launch
+    bwd_kernels = (("attn_bwd_head_kernel",) if w.N <= 512 else
+                   ("attn_bwd_delta_kernel", "attn_bwd_both_kernel") if tmap is not None else
+                   ("attn_bwd_dq_kernel", "attn_bwd_dkv_kernel"))
     result = {
         "metric": "dense_equiv_tflops_sparse_attention_fwd_incl_pack_mask",
         "value": round(value, 3),

@@ -9,7 +9,7 @@
 //     dS = P o (dP - delta) * scale             dQ = dS K            dK = dS^T Q
 //
 // No atomics, bit-reproducible.  Sequences of which a work-group holds a whole head take attn_bwd_head.hip's kernel, others
-// two:
+// two, or both in one launch (attn_bwd_both_kernel):
 //
 //   attn_bwd_dq_kernel   one work-group = 128 query rows, walks the key tiles exactly like the
 //                        forward: S^T = K Q^T and dP^T = V dO^T on the MFMA (lane = query row, so
@@ -115,8 +115,17 @@ __device__ __forceinline__ void zero_tile_tail(uint32_t dst, int parts, int r0, 
 // ------------------------------------------------------------------------------------------------
 // dQ (and delta)
 // ------------------------------------------------------------------------------------------------
-template <bool BF16, int HDIM, bool WIDE>
-__global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_bwd_dq_kernel(const AttnBwdArgs a)
+// Two products of 16-bit pairs more.  Delta is formed in the same order, and so with the same bits, by the dQ kernel and by attn_bwd_delta_kernel:
+// by fmas over the 8 elements of a chunk and then of the one 8 chunks further, then chunks 2s and 2s + 1, then pairs of these.
+template <bool BF16> __device__ __forceinline__ float add_products(uint32_t x, uint32_t y, float sum)
+{
+    using E = Elem<BF16>;
+    sum = __builtin_fmaf(E::up1((uint16_t)(x & 0xffffu)), E::up1((uint16_t)(y & 0xffffu)), sum);
+    return __builtin_fmaf(E::up1((uint16_t)(x >> 16)), E::up1((uint16_t)(y >> 16)), sum);
+}
+// HAVE_DELTA: attn_bwd_delta_kernel has left it
+template <bool BF16, int HDIM, bool WIDE, bool HAVE_DELTA>
+__device__ __forceinline__ void dq_rows(const AttnBwdArgs &a, unsigned char *smem, int bh, int qt)
 {
     using E = Elem<BF16>;
     constexpr int NH = HDIM > 64 ? 2 : 1;         // 64-column tiles per matrix
@@ -124,16 +133,12 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_bwd_dq_kerne
     constexpr int OB = HDIM / 32;                 // 32-column accumulator blocks of an output
     using C = Cfg<NH>;
     constexpr int STAGE_BYTES = C::STAGE_BYTES, OFF_AUX = C::OFF_AUX, OFF_LUT = C::OFF_LUT;
-    __shared__ __attribute__((aligned(1024))) unsigned char smem[C::LDS_BYTES];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(LDS_PTR(unsigned char))smem;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, hh = lane >> 5;
-    const int nid = renumber_block();
-    const int bh = (int)fastdiv((uint32_t)nid, a.div_qtiles);
-    const int qt = a.qtiles - 1 - (nid - bh * a.qtiles);      // last rows first, as in the forward
     const int N = a.N, nw = (N + 31) >> 5;
     const int T = (N + BN - 1) / BN;
     const bool ragged = (N & (BN - 1)) != 0;
@@ -150,20 +155,22 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_bwd_dq_kerne
     u32x4 qf[KS], dof[KS], of[KS];
     load_row(qf, qb, a.q.sn, qr, hh, a.D);
     load_row(dof, dob, a.dout.sn, qr, hh, a.D);
-    load_row(of, ob, a.out.sn, qr, hh, a.D);
-    float delta = 0.f;
+    float delta = 0.f, d4[4] = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (HAVE_DELTA) delta = a.delta[(size_t)bh * N + qr];
+    else load_row(of, ob, a.out.sn, qr, hh, a.D);
 #pragma unroll
     for (int s = 0; s < KS; ++s)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            delta += E::up1((uint16_t)(dof[s][i] & 0xffffu)) * E::up1((uint16_t)(of[s][i] & 0xffffu)) +
-                     E::up1((uint16_t)(dof[s][i] >> 16)) * E::up1((uint16_t)(of[s][i] >> 16));
+            if constexpr (!HAVE_DELTA) d4[s & 3] = add_products<BF16>(dof[s][i], of[s][i], d4[s & 3]);
             const float lo = E::up1((uint16_t)(qf[s][i] & 0xffffu)) * a.q_scale;
             const float hi = E::up1((uint16_t)(qf[s][i] >> 16)) * a.q_scale;
             qf[s][i] = (uint32_t)E::cvt1(lo) | ((uint32_t)E::cvt1(hi) << 16);
         }
-    delta = xhalf_sum(delta);
-    if (qrow < N && hh == 0) a.delta[(size_t)bh * N + qrow] = delta;
+    if constexpr (!HAVE_DELTA) {
+        delta = (xhalf_sum(d4[0]) + xhalf_sum(d4[1])) + (xhalf_sum(d4[2]) + xhalf_sum(d4[3]));
+        if (qrow < N && hh == 0) a.delta[(size_t)bh * N + qrow] = delta;
+    }
     const float lse_row = a.lse[(size_t)bh * N + qr];
     // p = exp2(pm * s - L); rows that kept nothing (lse = -inf) and rows beyond N get L = +inf
     const float L = (qrow >= N || lse_row == -__builtin_inff()) ? __builtin_inff() : lse_row * LOG2E;
@@ -296,6 +303,15 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_bwd_dq_kerne
     }
 }
 
+template <bool BF16, int HDIM, bool WIDE>
+__global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_bwd_dq_kernel(const AttnBwdArgs a)
+{
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[Cfg<(HDIM > 64 ? 2 : 1)>::LDS_BYTES];
+    const int nid = renumber_block();
+    const int bh = (int)fastdiv((uint32_t)nid, a.div_qtiles);
+    dq_rows<BF16, HDIM, WIDE, false>(a, smem, bh, a.qtiles - 1 - (nid - bh * a.qtiles));      // last rows first, as in the forward
+}
+
 // ------------------------------------------------------------------------------------------------
 // dK and dV
 // ------------------------------------------------------------------------------------------------
@@ -317,7 +333,7 @@ template <int HDIM, int NW, bool VLDS> struct DkvCfg {
     static constexpr int LDS_BYTES = OFF_FRAG + NW * FRAG;
 };
 template <bool BF16, int HDIM, int NW, bool VLDS, bool POSTMUL, bool WIDE>
-__global__ __launch_bounds__(64 * NW, HDIM == 128 ? NW / 4 : VLDS ? 3 : 2) void attn_bwd_dkv_kernel(const AttnBwdArgs a)
+__device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *smem, int bh, int kt)
 {
     using E = Elem<BF16>;
     constexpr int NH = HDIM > 64 ? 2 : 1;
@@ -326,16 +342,12 @@ __global__ __launch_bounds__(64 * NW, HDIM == 128 ? NW / 4 : VLDS ? 3 : 2) void 
     using C = DkvCfg<HDIM, NW, VLDS>;
     constexpr int STAGE_BYTES = C::STAGE_BYTES, OFF_AUX = C::OFF_AUX, AUX_BYTES = C::AUX;
     constexpr int OFF_LSE = NW * 256, OFF_DELTA = OFF_LSE + 256;       // inside the small data of a stage
-    __shared__ __attribute__((aligned(1024))) unsigned char smem[C::LDS_BYTES];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(LDS_PTR(unsigned char))smem;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, hh = lane >> 5;
-    const int nid = renumber_block();
-    const int bh = (int)fastdiv((uint32_t)nid, a.div_ktiles);
-    const int kt = nid - bh * a.ktiles;
     const int N = a.N, nw = (N + 31) >> 5;
     const int T = (N + BN - 1) / BN;
     const bool ragged = (N & (BN - 1)) != 0;
@@ -546,10 +558,79 @@ __global__ __launch_bounds__(64 * NW, HDIM == 128 ? NW / 4 : VLDS ? 3 : 2) void 
     }
 }
 
+template <bool BF16, int HDIM, int NW, bool VLDS, bool POSTMUL, bool WIDE>
+__global__ __launch_bounds__(64 * NW, HDIM == 128 ? NW / 4 : VLDS ? 3 : 2) void attn_bwd_dkv_kernel(const AttnBwdArgs a)
+{
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[DkvCfg<HDIM, NW, VLDS>::LDS_BYTES];
+    const int nid = renumber_block();
+    const int bh = (int)fastdiv((uint32_t)nid, a.div_ktiles);
+    dkv_keys<BF16, HDIM, NW, VLDS, POSTMUL, WIDE>(a, smem, bh, nid - bh * a.ktiles);
+}
+
+// ------------------------------------------------------------------------------------------------
+// both in one launch
+// ------------------------------------------------------------------------------------------------
+// The work-groups of a head follow each other, those of its keys (which take longer) first.  What that gives: a grid that is
+// resident all at once runs both kinds side by side instead of one after the other; where rows and keys have unequal work the ends of the
+// one fill with the other; and q, k, v and dO of a head come from memory once.  What it costs: delta beforehand, in a
+// launch of its own, and dK/dV at the occupancy of both.  The backward alone, two launches -> this, in us:
+//   one round     8 heads, N = 512: 29.6 -> 20.1;  64, N = 700: 51.3 -> 46.4;  20, N = 2048: 118 -> 105;  1, N = 4096: 173 -> 105;  D = 32: 8 heads, N = 333: 19.2 ->
+//                 12.9;  D = 128: 16 heads, N = 512: 44.4 -> 30.4;  4, N = 4096: 259 -> 168
+//   blocks, map   forward + backward, 12 heads, N = 1024: batch 16 156 -> 149, 8 86.7 -> 82.0, 4 66.9 -> 55.2;  D = 96, batch 8: 135 -> 124;
+//                 16 x 12, N = 700: 104.9 -> 95.2;  2 x 8, N = 4096: 178 -> 165
+// Beyond one round and without a map it is left off: 192 heads, N = 1024: 214 -> 221; 60, N = 1000 (1.25 rounds): 74 -> 84 (causal masks would gain:
+// 128, N = 1000: 125 -> 109, but the launcher doesn't see them); D = 32 with a map: 384 heads, N = 600: 94.2 -> 96.6.
+//
+// Delta of every row, eight lanes a row: whole lines at once (two lanes a row, with the fragments' access, took 10 us more of 150 on 16 x 12
+// heads, N = 1024)
+template <bool BF16> __global__ __launch_bounds__(NTHREADS) void attn_bwd_delta_kernel(const AttnBwdArgs a)
+{
+    const int N = a.N, bh = (int)fastdiv(blockIdx.x, a.div_qtiles), bi = (int)fastdiv((uint32_t)bh, a.div_H), hi = bh - bi * a.H;
+    const uint16_t *dob = slab(a.dout, bi, hi), *ob = slab(a.out, bi, hi);
+    const int c = threadIdx.x & 7;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int row = ((int)blockIdx.x - bh * a.qtiles) * BM + 32 * j + (int)(threadIdx.x >> 3), r = row < N ? row : N - 1;
+        float d = 0.f;
+        for (int chunk = c; 8 * chunk < a.D; chunk += 8) {
+            const u32x4 x = *reinterpret_cast<const u32x4 *>(dob + (size_t)r * a.dout.sn + 8 * chunk);
+            const u32x4 y = *reinterpret_cast<const u32x4 *>(ob + (size_t)r * a.out.sn + 8 * chunk);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) d = add_products<BF16>(x[i], y[i], d);
+        }
+        // lane ^ 1, then lane ^ 2, then 7 - lane
+        d += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, d), 0xB1, 0xf, 0xf, true));
+        d += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, d), 0x4E, 0xf, 0xf, true));
+        d += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, d), 0x141, 0xf, 0xf, true));
+        if (row < N && c == 0) a.delta[(size_t)bh * N + row] = d;
+    }
+}
+template <bool BF16, int HDIM, bool POSTMUL, bool WIDE>
+__global__ __launch_bounds__(NTHREADS, HDIM == 128 ? 1 : HDIM > 64 ? 2 : 3) void attn_bwd_both_kernel(const AttnBwdArgs a)
+{
+    constexpr bool VLDS = HDIM == 64 || HDIM == 128;
+    constexpr int DQ = Cfg<(HDIM > 64 ? 2 : 1)>::LDS_BYTES, DKV = DkvCfg<HDIM, 4, VLDS>::LDS_BYTES;
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[DQ > DKV ? DQ : DKV];
+    const int nid = renumber_block();
+    const int bh = (int)fastdiv((uint32_t)nid, a.div_ktiles), i = nid - bh * 2 * a.qtiles;
+    if (i < a.qtiles) dkv_keys<BF16, HDIM, 4, VLDS, POSTMUL, WIDE>(a, smem, bh, i);
+    else dq_rows<BF16, HDIM, WIDE, true>(a, smem, bh, 2 * a.qtiles - 1 - i);
+}
+
 template <bool BF16, int HDIM, bool POSTMUL, bool WIDE>
 void launch_pair(hipStream_t stream, const AttnBwdArgs &args)
 {
     AttnBwdArgs a = args;
+    const long long groups = (long long)a.BH * a.qtiles, cus = compute_units();
+    // Both kinds of work-groups in one launch (see attn_bwd_both_kernel): while all are resident at once, or with a tile map
+    if (2 * groups <= (HDIM == 128 ? 1 : HDIM > 64 ? 2 : 3) * cus ||
+        (a.tile_map != nullptr && (HDIM == 64 || HDIM == 96) && groups < (1ll << 30))) {
+        a.ktiles = a.qtiles;
+        a.div_ktiles = make_fastdiv((uint32_t)(2 * a.qtiles));
+        hipLaunchKernelGGL((attn_bwd_delta_kernel<BF16>), dim3((unsigned)groups), dim3(NTHREADS), 0, stream, a);
+        hipLaunchKernelGGL((attn_bwd_both_kernel<BF16, HDIM, POSTMUL, WIDE>), dim3((unsigned)(2 * groups)), dim3(NTHREADS), 0, stream, a);
+        return;
+    }
     // dQ first: it also fills the delta workspace that the dK/dV kernel reads (same stream)
     hipLaunchKernelGGL((attn_bwd_dq_kernel<BF16, HDIM, WIDE>), dim3((unsigned)(a.BH * a.qtiles)), dim3(NTHREADS), 0, stream, a);
     auto dkv = [&](auto nw_c, auto vlds_c) {
@@ -560,7 +641,6 @@ void launch_pair(hipStream_t stream, const AttnBwdArgs &args)
                            dim3((unsigned)(a.BH * a.ktiles)), dim3(64 * NW), 0, stream, a);
     };
     using four = std::integral_constant<int, 4>;
-    const long long groups = (long long)a.BH * a.qtiles, cus = compute_units();
     if constexpr (HDIM == 128) {
         // Eight wavefronts read Q and dO once per 256 keys and keep two of themselves on a SIMD, four
         // leave a CU to one work-group; but a grid that four-wavefront work-groups do not fill takes them (1 x 8 heads,
