@@ -367,6 +367,7 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
     const int kr = key < N ? key : N - 1;
     const uint32_t key_ok = key < N ? 0xffffffffu : 0u;
     const uint32_t key_w = key < N ? 1u : 0u;         // width of the bit field that holds this key's mask bit
+    const uint32_t wave_keys = N - key0 >= 32 ? 0xffffffffu : N > key0 ? (1u << (N - key0)) - 1u : 0u;      // of them the existing ones
     const int wi = (key0 >> 5) < nw ? (key0 >> 5) : nw - 1;     // this wave's mask word of a row
     const uint32_t frag = lds0 + C::OFF_FRAG + wave * C::FRAG + lane * 16;
     u32x4 kf[KS], vf[VLDS ? 1 : KS];
@@ -469,18 +470,31 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
         if (t_next < T) issue(t_next, st ^ 1);
         if (!wave_valid) return;
 
+        // VLDS: which rows keep any of this wavefront's keys, by one word a lane: the four 16-byte reads of the words themselves, of a
+        // kernel whose LDS is nearly always busy, then come once and not twice, and not at all where nothing is kept.  The backward alone: 192 heads, N = 1024,
+        // D = 64 215.0 -> 210.3 us; 4 x 32, N = 4096, D = 128 3397 -> 3366; in one launch with dQ and by a map, a random
+        // mask, forward + backward, 32 heads, N = 4096 675 -> 646.
+        unsigned long long live_rows = ~0ull;
+        if constexpr (VLDS) {
+            const uint32_t w = *(LDS_PTR(const uint32_t))(uintptr_t)(aux_lane + wave * 256 + st * AUX_BYTES);
+            live_rows = __builtin_amdgcn_ballot_w64((w & wave_keys) != 0u);
+        }
 #pragma unroll
         for (int blk = 0; blk < 2; ++blk) {
             // element 4g+j of an accumulator <-> query row 32blk + 8g + 4hh + j of the tile
             auto mask_words = [&](int g) __attribute__((always_inline)) { return lds_read_b128(aux_words + st * AUX_BYTES + 128 * blk + 32 * g); };
             u32x4 mw[4];
-            uint32_t any = 0u;
+            if constexpr (VLDS) {
+                if ((uint32_t)(live_rows >> (32 * blk)) == 0u) continue;
+            } else {
+                uint32_t any = 0u;
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                mw[g] = mask_words(g);
-                any |= mw[g].x | mw[g].y | mw[g].z | mw[g].w;
+                for (int g = 0; g < 4; ++g) {
+                    mw[g] = mask_words(g);
+                    any |= mw[g].x | mw[g].y | mw[g].z | mw[g].w;
+                }
+                if (__builtin_amdgcn_ballot_w64((((any >> l32) & 1u) & key_ok) != 0u) == 0ull) continue;
             }
-            if (__builtin_amdgcn_ballot_w64((((any >> l32) & 1u) & key_ok) != 0u) == 0ull) continue;
 
             // the accumulators start from the rows' -lse (scaled) and -delta, read straight into them:
             // the products then leave s - lse and dP - delta, with no subtraction per element
@@ -504,7 +518,6 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
                 dacc = E::mfma(lds_read_b128(tr.rowaddr[s & 3] + so + C::OFF_B + (s >> 2) * TILE_BYTES + 4096 * blk), vs, dacc);
             }
 
-            if constexpr (VLDS) asm volatile("" ::: "memory");      // the words are read once more, not kept
             uint32_t pp[2][4], ps[2][4];
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
