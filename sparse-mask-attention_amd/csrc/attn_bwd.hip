@@ -589,10 +589,13 @@ __global__ __launch_bounds__(64 * NW, HDIM == 128 ? NW / 4 : VLDS ? 3 : 2) void 
 // launch of its own, and dK/dV at the occupancy of both.  The backward alone, two launches -> this, in us:
 //   one round     8 heads, N = 512: 29.6 -> 20.1;  64, N = 700: 51.3 -> 46.4;  20, N = 2048: 118 -> 105;  1, N = 4096: 173 -> 105;  D = 32: 8 heads, N = 333: 19.2 ->
 //                 12.9;  D = 128: 16 heads, N = 512: 44.4 -> 30.4;  4, N = 4096: 259 -> 168
-//   blocks, map   forward + backward, 12 heads, N = 1024: batch 16 156 -> 149, 8 86.7 -> 82.0, 4 66.9 -> 55.2;  D = 96, batch 8: 135 -> 124;
+//   blocks, map   forward + backward, 12 heads, N = 1024: batch 16 156 -> 149, 8 86.7 -> 82.0, 4 66.9 -> 55.2;
 //                 16 x 12, N = 700: 104.9 -> 95.2;  2 x 8, N = 4096: 178 -> 165
+//   random, map   (one of a mask in which nothing can be skipped) 16 x 12 heads, N = 1024: 274.2 -> 275.5;  4 x 32, N = 2048: 687.7 -> 685.1;
+//                 4 x 8, N = 4096: 672 -> 646;  3 x 12, N = 2048: 228.8 -> 206.5;  4 x 8, N = 2048, a third more than a round: 186 -> 190 (causal 168 -> 148)
 // Beyond one round and without a map it is left off: 192 heads, N = 1024: 214 -> 221; 60, N = 1000 (1.25 rounds): 74 -> 84 (causal masks would gain:
-// 128, N = 1000: 125 -> 109, but the launcher doesn't see them); D = 32 with a map: 384 heads, N = 600: 94.2 -> 96.6.
+// 128, N = 1000: 125 -> 109, but the launcher doesn't see them; D = 32 with a map: 384 heads, N = 600: 94.2 -> 96.6;
+// D = 96 with a map: blocks 8 x 12, N = 1024 145 -> 131, but 8 x 16, N = 2048 443 -> 447, and a random mask 907 -> 932).
 //
 // Delta of every row, eight lanes a row: whole lines at once (two lanes a row, with the fragments' access, took 10 us more of 150 on 16 x 12
 // heads, N = 1024)
@@ -637,7 +640,7 @@ void launch_pair(hipStream_t stream, const AttnBwdArgs &args)
     const long long groups = (long long)a.BH * a.qtiles, cus = compute_units();
     // Both kinds of work-groups in one launch (see attn_bwd_both_kernel): while all are resident at once, or with a tile map
     if (2 * groups <= (HDIM == 128 ? 1 : HDIM > 64 ? 2 : 3) * cus ||
-        (a.tile_map != nullptr && (HDIM == 64 || HDIM == 96) && groups < (1ll << 30))) {
+        (a.tile_map != nullptr && HDIM == 64 && groups < (1ll << 30))) {
         a.ktiles = a.qtiles;
         a.div_ktiles = make_fastdiv((uint32_t)(2 * a.qtiles));
         hipLaunchKernelGGL((attn_bwd_delta_kernel<BF16>), dim3((unsigned)groups), dim3(NTHREADS), 0, stream, a);

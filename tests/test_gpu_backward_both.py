@@ -1,4 +1,4 @@
-"""The backward whose dQ and dK/dV work-groups share a launch (grids of one round; with a tile map any grid at head dims 64 and 96)."""
+"""The backward whose dQ and dK/dV work-groups share a launch (grids of one round; with a tile map any grid at head dim 64)."""
 import importlib
 import sys
 
