@@ -321,6 +321,10 @@ typedef struct sma_fwd_call {
     int dtype;
 } sma_fwd_call;
 int sma_attn_fwd_call(const sma_fwd_call *call, void *stream);
+/* The same with q in fp32 (limits as out_f32; dtype must be bf16): the kernel rounds it (to nearest even), which is as if
+ * sma_to_bf16 had been called on it first, and leaves the rounded q in `q_rounded` if that is not NULL.
+ */
+int sma_attn_fwd_call_q32(const sma_fwd_call *call, const sma_tensor *q_rounded, void *stream);
 
 typedef struct sma_bwd_call {
     const sma_tensor *dout, *q, *k, *v, *out;

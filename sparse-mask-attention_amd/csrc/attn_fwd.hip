@@ -130,7 +130,7 @@ template <int N> __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_
 // -> 11.1 us; 4 x 8, N = 512: 10.1 -> 7.9 us.  A wavefront now copies 16 KB per tile instead of 4, and a tile takes
 // 1.4 times as long.
 template <bool BF16, bool POSTMUL, bool PACKED_ROWS, int HDIM, bool BYTEMASK = false, bool BYPRODUCTS = false,
-          int FETCH = 0, bool SPLIT = false>
+          int FETCH = 0, bool SPLIT = false, bool WIDE_Q = false>
 __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ? 2 : 3) void attn_fwd_kernel(const AttnArgs a)
 {
     static_assert(FETCH == 0 || (BYTEMASK && HDIM <= 64 && !SPLIT), "PAIRS: byte mask, two byte slots");
@@ -590,17 +590,35 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     constexpr int Q_HALF = SPLIT ? 4096 : 16384;         // between the column halves of the staged q
     // Requested at once, oldest first: q (this wave's 32 rows, staged through the second K/V stage,
     // which the prologue leaves unused, K-swizzled), then K/V and the mask words of tile 0.
+    // WIDE_Q (q in fp32): the same pieces through registers, rounded once the copies below are on their way.  q is read by one
+    // work-group alone, so this replaces a pass over it: 6 bytes an element instead of 8 with the rounded q kept, 4 without.  Separate
+    // pass -> this: forward, 384 heads, N = 200: 32.1 -> 29.1 us; 192, N = 512: 46.1 -> 44.4; 96, N = 577, D = 80: 42.0 -> 40.9;
+    // forward + backward, the last 121.8 -> 119.9, 64, N = 1000, D = 128: 218.0 -> 213.4.  As an instance of its own: decided at run time, the
+    // other element types' loops came out 0.5 to 1 % slower.
+    const uint32_t q_dst = SPLIT ? split_dst + C::OFF_V : lds0 + (NSTAGE - 1) * STAGE_BYTES + wave * 4096;
+    f32x4 wide[WIDE_Q ? 4 * NH : 1][2];
     {
         const int qbase = row_base < N ? row_base : N - 1;   // wave-uniform
         const uint16_t *qsrc = qb + (size_t)qbase * q_sn;
         const int last = N - 1 - qbase;                      // rows beyond N re-read row N-1
-        const uint32_t dst = SPLIT ? split_dst + C::OFF_V : lds0 + (NSTAGE - 1) * STAGE_BYTES + wave * 4096;
+        const uint32_t dst = q_dst;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int row = 8 * j + (lane >> 3);
             const int pos = lane & 7;
             const int lrow = row < last ? row : last;
             const int c = pos ^ ((row >> 1) & 7);
+            if constexpr (WIDE_Q) {
+                const float *src = reinterpret_cast<const float *>(a.q.p) + ((size_t)bi * a.q.sb8 + (size_t)hi * a.q.sh8) * 8 +
+                                   (size_t)(qbase + lrow) * q_sn;
+#pragma unroll
+                for (int half = 0; half < NH; ++half) {
+                    const f32x4 *x = reinterpret_cast<const f32x4 *>(src + (chunk_at(8 * half + c) >> 1));
+                    wide[NH * j + half][0] = x[0];
+                    wide[NH * j + half][1] = x[1];
+                }
+                continue;
+            }
             async_copy_b128(dst + j * 1024, qsrc, __umul24(lrow, q_rb) + chunk_at(c));
             if constexpr (NH == 2) async_copy_b128(dst + Q_HALF + j * 1024, qsrc, __umul24(lrow, q_rb) + chunk_at(8 + c));
         }
@@ -641,6 +659,21 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         } else {
             issue_kv(t_first, integral_constant<int, 0>{});
             issue_mask(t_first, integral_constant<int, 0>{});
+        }
+    }
+    if constexpr (WIDE_Q) {
+        uint16_t *q16 = a.q16.p != nullptr && (!SPLIT || wave == 0) ? slab(a.q16, bi, hi) : nullptr;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int row = 8 * j + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
+#pragma unroll
+            for (int half = 0; half < NH; ++half) {
+                const f32x4 lo = wide[NH * j + half][0], hi4 = wide[NH * j + half][1];
+                const u32x4 t = {E::pack2_rne(lo.x, lo.y), E::pack2_rne(lo.z, lo.w), E::pack2_rne(hi4.x, hi4.y), E::pack2_rne(hi4.z, hi4.w)};
+                *(LDS_PTR(u32x4))(uintptr_t)(q_dst + half * Q_HALF + j * 1024 + lane * 16) = t;
+                if (q16 != nullptr && row_base + row < N && 8 * half + c <= last_chunk)
+                    *reinterpret_cast<u32x4 *>(q16 + (size_t)(row_base + row) * a.q16.sn + 8 * (8 * half + c)) = t;
+            }
         }
     }
     // small LDS table for the mask: entry n (16 B) holds four floats, float j = (bit j of n) ? 0 : -inf
@@ -1040,28 +1073,28 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
 
 }  // namespace
 
-// The instance for (element type, post-multiplier, row strides) and the kind of mask: 0 packed words, 1
+// The instance for (fp32 q, element type, post-multiplier, row strides) and the kind of mask: 0 packed words, 1
 // boolean bytes, 2 the same with by-products, 3 and 4 those with two tiles' bytes per request, 5 to 7 the first
 // three with the keys split between the wavefronts, 8 and 9 as 3 and 4 at any N.  This file is
 // compiled once per head dim for the instances, side by side, and once for the launcher.
 typedef void (*FwdKernel)(const AttnArgs);
 #ifdef SMA_FWD_HEAD_DIM
-template <int HDIM, bool BF16, bool POSTMUL, bool PACKED_ROWS> FwdKernel pick_mask_kind(int mask_kind)
+template <int HDIM, bool BF16, bool POSTMUL, bool PACKED_ROWS, bool WIDE_Q = false> FwdKernel pick_mask_kind(int mask_kind)
 {
     switch (mask_kind) {
-    case 0: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM>;
-    case 1: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true>;
-    case 2: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true>;
-    case 5: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, false, false, 0, true>;
-    case 6: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, false, 0, true>;
-    case 7: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true, 0, true>;
+    case 0: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, false, false, 0, false, WIDE_Q>;
+    case 1: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, false, 0, false, WIDE_Q>;
+    case 2: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true, 0, false, WIDE_Q>;
+    case 5: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, false, false, 0, true, WIDE_Q>;
+    case 6: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, false, 0, true, WIDE_Q>;
+    case 7: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true, 0, true, WIDE_Q>;
     }
     if constexpr (HDIM <= 64) {
         switch (mask_kind) {
-        case 3: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, false, 1>;
-        case 4: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true, 1>;
-        case 8: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, false, 2>;
-        case 9: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true, 2>;
+        case 3: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, false, 1, false, WIDE_Q>;
+        case 4: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true, 1, false, WIDE_Q>;
+        case 8: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, false, 2, false, WIDE_Q>;
+        case 9: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true, 2, false, WIDE_Q>;
         }
     }
     return nullptr;
@@ -1076,7 +1109,11 @@ template <int HDIM> FwdKernel pick(int variant, int mask_kind)
     case 4: return pick_mask_kind<HDIM, true, false, false>(mask_kind);
     case 5: return pick_mask_kind<HDIM, true, false, true>(mask_kind);
     case 6: return pick_mask_kind<HDIM, true, true, false>(mask_kind);
-    default: return pick_mask_kind<HDIM, true, true, true>(mask_kind);
+    case 7: return pick_mask_kind<HDIM, true, true, true>(mask_kind);
+    case 12: return pick_mask_kind<HDIM, true, false, false, true>(mask_kind);
+    case 13: return pick_mask_kind<HDIM, true, false, true, true>(mask_kind);
+    case 14: return pick_mask_kind<HDIM, true, true, false, true>(mask_kind);
+    default: return pick_mask_kind<HDIM, true, true, true, true>(mask_kind);
     }
 }
 #define SMA_NAME2(d) fwd_kernel_##d
@@ -1134,9 +1171,10 @@ hipError_t launch_attn_fwd(const AttnArgs &args, bool bf16, hipStream_t stream)
     // two tiles' mask bytes per request (see PAIRS at the kernel), unless the grid is the single round of work-groups in
     // step for which tail_start was set to 0 above
     const bool further = !split && a.byte_mask && D <= HD && a.tail_start != 0;
+    if (a.q_f32 && !bf16) return hipErrorInvalidValue;         // fp32 callers compute in bf16
     if (a.byte_mask && a.N < 16) return hipErrorInvalidValue;  // a row holds at least one 16-byte copy (checked by the C-ABI layer)
     const int mask_kind = (split ? 5 : 0) + (!a.byte_mask ? 0 : (!further ? 1 : a.N % (2 * BN) == 0 ? 3 : 8) + (byproducts ? 1 : 0));
-    const int variant = (bf16 ? 4 : 0) | (postmul ? 2 : 0) | (packed ? 1 : 0);
+    const int variant = (a.q_f32 ? 8 : 0) | (bf16 ? 4 : 0) | (postmul ? 2 : 0) | (packed ? 1 : 0);
     const FwdKernel kernel = D == 32 ? fwd_kernel_32(variant, mask_kind) : D == 64 ? fwd_kernel_64(variant, mask_kind)
                              : D == 96 ? fwd_kernel_96(variant, mask_kind) : fwd_kernel_128(variant, mask_kind);
     hipLaunchKernelGGL(kernel, grid, block, 0, stream, a);

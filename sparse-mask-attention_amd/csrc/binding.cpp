@@ -355,24 +355,34 @@ int64_t padded_head_dim(int64_t D) { return (D + 7) / 8 * 8; }
 // tensor's own), addressable.  fp32 tensors that leave no gaps, all of one size, are converted in one launch that
 // keeps their layout; the caller holds the device guard.
 template <size_t COUNT>
-void kernel_rows(const Tensor *const (&from)[COUNT], Tensor *const (&to)[COUNT], at::ScalarType dtype, int64_t Dk)
+bool flat_f32(const Tensor *const (&from)[COUNT], int64_t Dk)
 {
-    bool flat = dtype == at::kBFloat16 && COUNT <= 3;
+    bool flat = COUNT <= 3;
     for (const Tensor *t : from)
         flat = flat && t->scalar_type() == at::kFloat && t->size(3) == Dk && t->is_non_overlapping_and_dense() && t->stride(3) == 1 &&
                t->numel() == from[0]->numel() && reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0;
-    if (flat) {
-        const float *src[COUNT];
-        uint16_t *dst[COUNT];
-        for (size_t i = 0; i < COUNT; ++i) {
-            *to[i] = from[i]->is_contiguous() ? empty_dense(from[i]->sizes(), dtype) : empty_rows(from[i]->sizes(), from[i]->strides(), dtype);
-            src[i] = static_cast<const float *>(from[i]->data_ptr());
-            dst[i] = static_cast<uint16_t *>(to[i]->data_ptr());
-        }
-        hipStream_t stream = c10::hip::getCurrentHIPStream(from[0]->device().index()).stream();
-        check_status(sma_to_bf16(src, dst, (int)COUNT, from[0]->numel(), stream), "sma_to_bf16");
-        return;
+    return flat;
+}
+Tensor empty_flat(const Tensor &t, at::ScalarType dtype)
+{
+    return t.is_contiguous() ? empty_dense(t.sizes(), dtype) : empty_rows(t.sizes(), t.strides(), dtype);
+}
+template <size_t COUNT> void flat_rows(const Tensor *const (&from)[COUNT], Tensor *const (&to)[COUNT])
+{
+    const float *src[COUNT];
+    uint16_t *dst[COUNT];
+    for (size_t i = 0; i < COUNT; ++i) {
+        *to[i] = empty_flat(*from[i], at::kBFloat16);
+        src[i] = static_cast<const float *>(from[i]->data_ptr());
+        dst[i] = static_cast<uint16_t *>(to[i]->data_ptr());
     }
+    hipStream_t stream = c10::hip::getCurrentHIPStream(from[0]->device().index()).stream();
+    check_status(sma_to_bf16(src, dst, (int)COUNT, from[0]->numel(), stream), "sma_to_bf16");
+}
+template <size_t COUNT>
+void kernel_rows(const Tensor *const (&from)[COUNT], Tensor *const (&to)[COUNT], at::ScalarType dtype, int64_t Dk)
+{
+    if (dtype == at::kBFloat16 && flat_f32(from, Dk)) return flat_rows(from, to);
     for (size_t i = 0; i < COUNT; ++i) {
         Tensor r = from[i]->scalar_type() == dtype ? *from[i] : from[i]->to(dtype);
         if (r.size(3) != Dk) r = at::constant_pad_nd(r, {0, Dk - r.size(3)});
@@ -406,6 +416,7 @@ Tensor unexpand(Tensor m)
 
 struct Call {                       // one problem as the kernels see it
     Tensor q, k, v;                 // kernel_rows of the caller's
+    Tensor q32;                     // undefined, or the fp32 q that the kernel itself rounds (into q, if there is a backward; else q is q32)
     Tensor mask;                    // the boolean mask, unexpanded; undefined if only the packed one is there
     Tensor packed, map;             // packed mask and tile map, either may be undefined
     int64_t B, H, N, D;             // the caller's extents
@@ -479,14 +490,20 @@ void run_forward(Call &c, const Tensor &out, const Tensor &out_f32, const Tensor
         f.mask_packed = reinterpret_cast<const uint32_t *>(c.packed.data_ptr<int32_t>());
         f.tile_map = map_pointer(c.map.defined() ? c10::optional<Tensor>(c.map) : c10::nullopt, c.packed, c.q);
     }
-    sma_tensor t[5] = {rows_of(c.q, "q"), rows_of(c.k, "k"), rows_of(c.v, "v")};
+    sma_tensor t[6] = {rows_of(c.q32.defined() ? c.q32 : c.q, "q"), rows_of(c.k, "k"), rows_of(c.v, "v")};
     f.q = &t[0], f.k = &t[1], f.v = &t[2];
     if (out.defined()) t[3] = rows_of(out, "out"), f.out = &t[3];
     if (out_f32.defined()) t[4] = rows_of(out_f32, "out"), f.out_f32 = &t[4];
     f.lse = training ? lse.data_ptr<float>() : nullptr;
     f.B = (int)c.B, f.H = (int)c.H, f.N = (int)c.N, f.D = (int)c.q.size(3);
     f.scale = (float)c.scale;
-    f.dtype = c.q.scalar_type() == at::kBFloat16 ? SMA_DTYPE_BF16 : SMA_DTYPE_F16;
+    f.dtype = c.q.scalar_type() == at::kHalf ? SMA_DTYPE_F16 : SMA_DTYPE_BF16;
+    if (c.q32.defined()) {
+        if (training) t[5] = rows_of(c.q, "q");
+        check_status(sma_attn_fwd_call_q32(&f, training ? &t[5] : nullptr,
+                                           c10::hip::getCurrentHIPStream(c.q.device().index()).stream()), "sma_attn_fwd_call_q32");
+        return;
+    }
     check_status(sma_attn_fwd_call(&f, c10::hip::getCurrentHIPStream(c.q.device().index()).stream()), "sma_attn_fwd_call");
 }
 
@@ -591,7 +608,14 @@ Tensor run_call(const Tensor &q, const Tensor &k, const Tensor &v, Call &c, bool
     }
     const c10::DeviceGuard guard(q.device());
     at::AutoDispatchBelowADInplaceOrView below_autograd;
-    kernel_rows<3>({&q, &k, &v}, {&c.q, &c.k, &c.v}, kdt, Dk);
+    // q is read once and can be rounded where it is read; k and v are read once per 128 query rows
+    if (dtype == at::kFloat && flat_f32<3>({&q, &k, &v}, Dk) && reaches_f32(q)) {
+        flat_rows<2>({&k, &v}, {&c.k, &c.v});
+        c.q32 = q;
+        c.q = tracked ? empty_flat(q, kdt) : q;
+    } else {
+        kernel_rows<3>({&q, &k, &v}, {&c.q, &c.k, &c.v}, kdt, Dk);
+    }
     // fp32 callers get their result from the kernel itself (unless its rows are too far apart); the 16-bit one is then made
     // for the backward only
     const bool wide = kdt != dtype && Dk == c.D && reaches_f32(c.q);

@@ -269,7 +269,8 @@ int sma_attn_fwd_map_strided(const sma_tensor *q, const sma_tensor *k, const sma
     return sma_attn_fwd_call(&c, stream);
 }
 
-int sma_attn_fwd_call(const sma_fwd_call *c, void *stream)
+// q_f32: c->q holds floats, and q_rounded (optional) receives what the kernel made of them
+static int fwd_call(const sma_fwd_call *c, bool q_f32, const sma_tensor *q_rounded, void *stream)
 {
     if (c == nullptr) return SMA_ERR_NULL_POINTER;
     const int B = c->B, H = c->H, N = c->N, D = c->D;
@@ -282,7 +283,7 @@ int sma_attn_fwd_call(const sma_fwd_call *c, void *stream)
     if (BH == 0 || N == 0) return SMA_OK;
     if (!bytes && !c->mask_packed) return SMA_ERR_NULL_POINTER;
     if (!c->out && !c->out_f32) return SMA_ERR_NULL_POINTER;
-    if (c->out_f32 && c->dtype != SMA_DTYPE_BF16) return SMA_ERR_DTYPE;
+    if ((c->out_f32 || q_f32) && c->dtype != SMA_DTYPE_BF16) return SMA_ERR_DTYPE;
     if (bytes && N < 16) return SMA_ERR_BAD_SHAPE;               // a row holds at least one 16-byte copy
     const long long qtiles = (N + 127) / 128;
     if (!below_2_31(BH, qtiles) || !below_2_31(BH, N)) return SMA_ERR_BAD_SHAPE;
@@ -298,16 +299,17 @@ int sma_attn_fwd_call(const sma_fwd_call *c, void *stream)
     if (c->mask_stride_b < 0 || c->mask_stride_h < 0) return SMA_ERR_STRIDE;
 
     sma::AttnArgs a;
-    const sma_tensor *in[5] = {c->q, c->k, c->v, c->out, c->out_f32};
-    sma::Rows *to[5] = {&a.q, &a.k, &a.v, &a.out, &a.out32};
-    for (int i = 0; i < 5; ++i) {
+    const sma_tensor *in[6] = {c->q, c->k, c->v, c->out, c->out_f32, q_rounded};
+    sma::Rows *to[6] = {&a.q, &a.k, &a.v, &a.out, &a.out32, &a.q16};
+    for (int i = 0; i < 6; ++i) {
         *to[i] = sma::Rows{nullptr, 0u, 0u, 0u};
         if (i >= 3 && in[i] == nullptr) continue;
-        const int st = to_rows(in[i], B, H, N, D, i >= 3, to[i], i == 4);
+        const int st = to_rows(in[i], B, H, N, D, i >= 3, to[i], i == 4 || (i == 0 && q_f32));
         if (st != SMA_OK) return st;
     }
     // mask rows start at any byte address: the kernel's 16-byte copies rely on the device serving them
     if (bytes && sma::unaligned_access_state(static_cast<hipStream_t>(stream)) == 0) return SMA_ERR_DEVICE;
+    a.q_f32 = q_f32;
     a.mask = sma::PackedMask{bytes ? reinterpret_cast<const uint32_t *>(c->mask) : c->mask_packed, c->mask_stride_b, c->mask_stride_h};
     a.lse = c->lse;
     a.BH = (int)BH;
@@ -329,6 +331,13 @@ int sma_attn_fwd_call(const sma_fwd_call *c, void *stream)
 
     const hipError_t e = sma::launch_attn_fwd(a, c->dtype == SMA_DTYPE_BF16, static_cast<hipStream_t>(stream));
     return e == hipSuccess ? SMA_OK : SMA_ERR_LAUNCH;
+}
+
+int sma_attn_fwd_call(const sma_fwd_call *c, void *stream) { return fwd_call(c, false, nullptr, stream); }
+
+int sma_attn_fwd_call_q32(const sma_fwd_call *c, const sma_tensor *q_rounded, void *stream)
+{
+    return fwd_call(c, true, q_rounded, stream);
 }
 
 int sma_attn_fwd_strided(const sma_tensor *q, const sma_tensor *k, const sma_tensor *v,

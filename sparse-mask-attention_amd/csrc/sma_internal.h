@@ -46,6 +46,8 @@ __host__ __device__ inline uint32_t fastdiv(uint32_t n, FastDiv f)
 // Arguments of the fused forward kernel, already validated by the C-ABI layer.
 struct AttnArgs {
     Rows q, k, v;                   // inputs (never written)
+    Rows q16;                       // with q_f32: where to leave q's rounded rows, p == nullptr: nowhere
+    int q_f32;                      // q.p names floats (bf16 kernels)
     PackedMask mask;                // byte_mask != 0: p names boolean bytes [Bm, Hm, N, N], strides in bytes
     Rows out, out32;                // 16-bit output and its fp32 copy (p names floats); p == nullptr: not wanted
     float *lse;                     // [BH, N] contiguous, or nullptr
