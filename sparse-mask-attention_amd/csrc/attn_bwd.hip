@@ -16,7 +16,7 @@
 //                        lse and delta are per-lane scalars and the mask enters as the accumulator's
 //                        initial value), dS^T packed to 16 bit is the B operand of dQ^T += K^T dS^T
 //                        (K^T by transposing LDS reads).  Also writes delta to the workspace.
-//   attn_bwd_dkv_kernel  one work-group = 128 keys (lane = key), walks the query tiles:
+//   attn_bwd_dkv_kernel  one work-group = 128 or 256 keys (lane = key), walks the query tiles:
 //                        S = Q K^T and dP = dO V^T with K, V fragments held in registers; -lse and
 //                        -delta of the tile's rows are read from LDS (broadcast reads) straight
 //                        into the accumulators as their initial values, so the products leave
@@ -332,7 +332,7 @@ template <int HDIM, int NW, bool VLDS> struct DkvCfg {
     static constexpr int FRAG = VLDS ? HDIM / 16 * 1024 : 0;
     static constexpr int LDS_BYTES = OFF_FRAG + NW * FRAG;
 };
-template <bool BF16, int HDIM, int NW, bool VLDS, bool POSTMUL, bool WIDE>
+template <bool BF16, int HDIM, int NW, bool VLDS, bool POSTMUL, bool WIDE, bool HALVES = false>
 __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *smem, int bh, int kt)
 {
     using E = Elem<BF16>;
@@ -361,7 +361,16 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
     const float *lse_b = a.lse + (size_t)bh * N, *delta_b = a.delta + (size_t)bh * N;
 
     // ---- this lane's key: K^T (scaled) and V^T fragments, B operands ----
-    const int key0 = kt * (32 * NW) + wave * 32;
+    // HALVES: a work-group of half the keys, in which the wavefronts of either half take 32 rows of every tile and their sums are added at the
+    // end.  One CU holds one work-group of eight wavefronts, so a grid just beyond a round took two: its last heads, where work-groups of 128 keys
+    // hold them all at once, come in such ones, each three quarters as long as a whole one.  The backward alone, before -> now, in us:
+    //   36 heads, N = 2048: 377 -> 343 (causal 281 -> 247);  48: 394 -> 365;  68: 596 -> 560;  72, N = 1000: 206 -> 192;  18, N = 4000,
+    //   causal: 489 -> 421;  forward + backward, 40, N = 2048, one mask in blocks: 276 -> 248.  Of 35 grids one lost: 24 heads, N = 3000, causal,
+    //   whose short work-groups had filled the second round by themselves: 286 -> 301.
+    static_assert(!HALVES || (NW == 8 && VLDS && OB * 2 * 4096 * 4 <= C::LDS_BYTES), "four wavefronts' sums fit the LDS");
+    constexpr int KW = HALVES ? 4 : NW;               // wavefronts side by side on different keys
+    const int half = HALVES ? wave >> 2 : 0;          // ... and which 32 rows of every tile this one takes
+    const int key0 = kt * (32 * KW) + (HALVES ? wave & 3 : wave) * 32;
     const bool wave_valid = key0 < N;                 // wave-uniform: some key of this wave exists
     const int key = key0 + l32;
     const int kr = key < N ? key : N - 1;
@@ -392,7 +401,14 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
     // (eight wavefronts: the first four copy Q, the others dO)
     const int cw = wave & 3;
     const TileCopy tc = make_tile_copy(cw, lane, (a.D >> 3) - 1);
-    const TileRead tr = make_tile_read(lane);
+    TileRead tr = make_tile_read(lane);
+    if constexpr (HALVES) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            tr.rowaddr[i] += 4096 * half;
+            tr.traddr[i >> 1][i & 1] += 4096 * half;
+        }
+    }
     auto issue = [&](int t, int st) {
         const int r0 = t * BN;
         const int row = r0 + lane < N ? r0 + lane : N - 1;
@@ -404,12 +420,12 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
         if (NW == 4 || wave >= 4) issue_tile<NH>(lds0 + st * STAGE_BYTES + C::OFF_B, dob, a.dout.sn, r0, N, tc, cw);
     };
     // With a tile map only the blocks of 64 query rows in which the mask keeps something for this
-    // work-group's keys (NW / 2 key tiles: neighbouring bits of one word of the row block's "live"
+    // work-group's keys (KW / 2 key tiles: neighbouring bits of one word of the row block's "live"
     // bits) are visited: lane r of a wavefront looks at row block 64c + r, a
     // ballot turns the 64 answers into the bits that are walked.  Every wavefront does the same.
     const int TW = (T + 31) >> 5;
     const uint32_t *mapc = a.tile_map != nullptr
-        ? a.tile_map + bi * a.map_sb + hi * a.map_sh + ((NW / 2 * kt) >> 5) : nullptr;
+        ? a.tile_map + bi * a.map_sb + hi * a.map_sh + ((KW / 2 * kt) >> 5) : nullptr;
     int cur_c = -1;
     unsigned long long live_c = 0ull;
     auto next_tile = [&]() __attribute__((always_inline)) -> int {     // next live row block, T if there is none
@@ -417,7 +433,7 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
             if (64 * ++cur_c >= T) return T;
             const int r = 64 * cur_c + lane;
             bool lv = r < T;
-            if (mapc != nullptr && lv) lv = ((mapc[(size_t)r * 2 * TW] >> ((NW / 2 * kt) & 31)) & ((1u << (NW / 2)) - 1u)) != 0u;
+            if (mapc != nullptr && lv) lv = ((mapc[(size_t)r * 2 * TW] >> ((KW / 2 * kt) & 31)) & ((1u << (KW / 2)) - 1u)) != 0u;
             live_c = __builtin_amdgcn_ballot_w64(lv);
         }
         const int b = __builtin_ctzll(live_c);
@@ -440,6 +456,8 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
     // keep a register for every sum of base and offset (40 of them) instead of using the offset field, and at 64
     // three work-groups on a CU leave no register to spare
     uint32_t aux_rows = lds0 + OFF_AUX + 16 * hh, aux_words = aux_rows + wave * 256, aux_lane = lds0 + OFF_AUX + 4 * lane;
+    aux_rows += 128 * half;
+    aux_words += 128 * half;
     if constexpr (VLDS || OFF_AUX >= 65536) asm volatile("" : "+v"(aux_rows), "+v"(aux_words), "+v"(aux_lane));
 
     // one q tile; the ring stage is a compile-time constant so that every LDS address of the body is
@@ -477,10 +495,10 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
         unsigned long long live_rows = ~0ull;
         if constexpr (VLDS) {
             const uint32_t w = *(LDS_PTR(const uint32_t))(uintptr_t)(aux_lane + wave * 256 + st * AUX_BYTES);
-            live_rows = __builtin_amdgcn_ballot_w64((w & wave_keys) != 0u);
+            live_rows = __builtin_amdgcn_ballot_w64((w & wave_keys) != 0u) >> (32 * half);
         }
 #pragma unroll
-        for (int blk = 0; blk < 2; ++blk) {
+        for (int blk = 0; blk < (HALVES ? 1 : 2); ++blk) {
             // element 4g+j of an accumulator <-> query row 32blk + 8g + 4hh + j of the tile
             auto mask_words = [&](int g) __attribute__((always_inline)) { return lds_read_b128(aux_words + st * AUX_BYTES + 128 * blk + 32 * g); };
             u32x4 mw[4];
@@ -565,6 +583,39 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
     }
     WAIT_VMCNT(0);
     __syncthreads();
+    if constexpr (HALVES) {
+        // the sums over the other 32 rows of every tile, from the wavefront that has the same keys
+        const uint32_t sums = lds0 + (wave & 3) * (OB * 8192) + lane * 16;
+        if (half == 1 && wave_valid) {
+#pragma unroll
+            for (int b = 0; b < OB; ++b)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    *(LDS_PTR(f32x4))(uintptr_t)(sums + (4 * b + g) * 1024) =
+                        f32x4{dkacc[b][4 * g], dkacc[b][4 * g + 1], dkacc[b][4 * g + 2], dkacc[b][4 * g + 3]};
+                    *(LDS_PTR(f32x4))(uintptr_t)(sums + (4 * (OB + b) + g) * 1024) =
+                        f32x4{dvacc[b][4 * g], dvacc[b][4 * g + 1], dvacc[b][4 * g + 2], dvacc[b][4 * g + 3]};
+                }
+        }
+        __syncthreads();
+        if (half == 1 || !wave_valid) return;
+#pragma unroll
+        for (int b = 0; b < OB; ++b) {
+            __builtin_amdgcn_sched_barrier(0);            // one block's sums in registers at a time
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const f32x4 x = *(LDS_PTR(f32x4))(uintptr_t)(sums + (4 * b + g) * 1024), y = *(LDS_PTR(f32x4))(uintptr_t)(sums + (4 * (OB + b) + g) * 1024);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    dkacc[b][4 * g + j] += x[j];
+                    dvacc[b][4 * g + j] += y[j];
+                }
+            }
+        }
+        store_gradient<BF16, WIDE>(dkacc, a.scale, lds0 + wave * (OB * 8192), a, a.dk, bi, hi, key0, lane);      // over its own sums
+        store_gradient<BF16, WIDE>(dvacc, 1.0f, lds0 + wave * (OB * 8192), a, a.dv, bi, hi, key0, lane);
+        return;
+    }
     if (wave_valid) {
         store_gradient<BF16, WIDE>(dkacc, a.scale, lds0 + wave * 4096, a, a.dk, bi, hi, key0, lane);
         store_gradient<BF16, WIDE>(dvacc, 1.0f, lds0 + wave * 4096, a, a.dv, bi, hi, key0, lane);
@@ -575,7 +626,16 @@ template <bool BF16, int HDIM, int NW, bool VLDS, bool POSTMUL, bool WIDE>
 __global__ __launch_bounds__(64 * NW, HDIM == 128 ? NW / 4 : VLDS ? 3 : 2) void attn_bwd_dkv_kernel(const AttnBwdArgs a)
 {
     __shared__ __attribute__((aligned(1024))) unsigned char smem[DkvCfg<HDIM, NW, VLDS>::LDS_BYTES];
-    const int nid = renumber_block();
+    if constexpr (HDIM == 128 && NW == 8) {
+        const int late = (int)blockIdx.x - a.whole_groups;
+        if (late >= 0) {
+            const int i = renumber_block(late, (int)gridDim.x - a.whole_groups);
+            const int h = (int)fastdiv((uint32_t)i, a.div_qtiles);
+            dkv_keys<BF16, HDIM, NW, VLDS, POSTMUL, WIDE, true>(a, smem, a.whole_heads + h, i - h * a.qtiles);
+            return;
+        }
+    }
+    const int nid = HDIM == 128 && NW == 8 ? renumber_block((int)blockIdx.x, a.whole_groups) : renumber_block();
     const int bh = (int)fastdiv((uint32_t)nid, a.div_ktiles);
     dkv_keys<BF16, HDIM, NW, VLDS, POSTMUL, WIDE>(a, smem, bh, nid - bh * a.ktiles);
 }
@@ -653,16 +713,25 @@ void launch_pair(hipStream_t stream, const AttnBwdArgs &args)
         constexpr int NW = decltype(nw_c)::value;
         a.ktiles = (a.N + 32 * NW - 1) / (32 * NW);
         a.div_ktiles = make_fastdiv((uint32_t)a.ktiles);
+        long long launched = (long long)a.BH * a.ktiles;
+        if constexpr (HDIM == 128 && NW == 8) {
+            // heads beyond the last full round in work-groups of 128 keys, if these are one round at most (see HALVES at the kernel)
+            const long long full = cus > 0 ? (launched - 1) / cus * cus / a.ktiles : a.BH, rest = a.BH - full;
+            a.whole_heads = rest * a.qtiles <= cus ? (int)full : a.BH;
+            a.whole_groups = a.whole_heads * a.ktiles;
+            launched = a.whole_groups + (long long)(a.BH - a.whole_heads) * a.qtiles;
+        }
         hipLaunchKernelGGL((attn_bwd_dkv_kernel<BF16, HDIM, NW, decltype(vlds_c)::value, POSTMUL, WIDE>),
-                           dim3((unsigned)(a.BH * a.ktiles)), dim3(64 * NW), 0, stream, a);
+                           dim3((unsigned)launched), dim3(64 * NW), 0, stream, a);
     };
     using four = std::integral_constant<int, 4>;
     if constexpr (HDIM == 128) {
-        // Eight wavefronts read Q and dO once per 256 keys and keep two of themselves on a SIMD, four
-        // leave a CU to one work-group; but a grid that four-wavefront work-groups do not fill takes them (1 x 8 heads,
-        // N = 1024: 74 against 87 us), and so do short keys of which 256 at a time would leave a sixth or more idle.
-        // Elsewhere eight win: 16 x 12, N = 1024: 373 against 431 us.
-        if (groups > cus && (a.qtiles % 2 == 0 || a.qtiles >= 5)) dkv(std::integral_constant<int, 8>{}, std::true_type{});
+        // Eight wavefronts read Q and dO once per 256 keys and keep two of themselves on a SIMD, four leave a CU to one work-group:
+        // 16 x 12 heads, N = 1024: 373 against 431 us.  A grid that four fill no more than once takes eight on 128 keys (the rows between
+        // them, HALVES) from 641 keys on: 16 heads, N = 2048 145 -> 136 us, 6, N = 4000 256 -> 232, 28, N = 1088 81.0 -> 79.4;
+        // 40, N = 700 57.2 either way, 60, N = 512 46.6 -> 47.9.  Four stay there, and on short keys of which 256 at a
+        // time would leave a sixth or more idle (300 heads, N = 384, by halves: 134 -> 141).
+        if (groups > cus ? a.qtiles % 2 == 0 || a.qtiles >= 5 : a.qtiles > 5) dkv(std::integral_constant<int, 8>{}, std::true_type{});
         else dkv(four{}, std::true_type{});
     } else if (HDIM == 64 && groups > 2 * cus && (2 * groups <= 7 * cus || groups > 4 * cus)) {
         // Three work-groups on a CU.  A grid that two of them on each CU hold does not need the third and pays for the reads

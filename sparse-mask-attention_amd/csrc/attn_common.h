@@ -92,13 +92,13 @@ __device__ __forceinline__ int bitrev3(int f) { return ((f & 1) << 2) | (f & 2) 
 // id; the number returned gives each XCD (own L2) a contiguous range of (b,h) pairs, with the
 // tiles of one (b,h) dispatched next to each other: the matrices of a head are then fetched into
 // one L2 only.
-__device__ __forceinline__ int renumber_block()
+__device__ __forceinline__ int renumber_block(int bid, int total)
 {
-    const int total = gridDim.x, bid = blockIdx.x;
     const int xcd = bid & 7, j = bid >> 3;
     const int base = total >> 3, rem = total & 7;
     return xcd * base + (xcd < rem ? xcd : rem) + j;
 }
+__device__ __forceinline__ int renumber_block() { return renumber_block((int)blockIdx.x, (int)gridDim.x); }
 
 // max / sum of a value with its partner in the other lane half (lane l <-> lane l ^ 32).
 // v_permlane32_swap(a, b) leaves {own a | partner's b, partner's a | own b} in lanes < 32 | >= 32.

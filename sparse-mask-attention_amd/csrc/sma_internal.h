@@ -91,6 +91,7 @@ struct AttnBwdArgs {
     int qtiles;                                // ceil(N / 128)
     int ktiles;                                // key tiles (work-groups of the dK/dV kernel) per (b,h) ...
     FastDiv div_qtiles, div_ktiles, div_H;     // ... and these: filled in by the launcher
+    int whole_heads, whole_groups;             // head dim 128, eight wavefronts: the heads, and their work-groups, of 256 keys each
     float scale;                               // as given by the caller
     float q_scale, post_mul;                   // as in AttnArgs
     uint32_t last_mask0, last_mask1;
