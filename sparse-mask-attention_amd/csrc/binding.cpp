@@ -608,8 +608,10 @@ Tensor run_call(const Tensor &q, const Tensor &k, const Tensor &v, Call &c, bool
     }
     const c10::DeviceGuard guard(q.device());
     at::AutoDispatchBelowADInplaceOrView below_autograd;
-    // q is read once and can be rounded where it is read; k and v are read once per 128 query rows
-    if (dtype == at::kFloat && flat_f32<3>({&q, &k, &v}, Dk) && reaches_f32(q)) {
+    // q is read once and can be rounded where it is read; k and v are read once per 128 query rows.  From 2^19 elements on: below, the pass
+    // over all three is as long as the one over two, and the forward's first loads are longer (forward, separate pass -> this: 16 heads,
+    // N = 64 6.6 -> 6.95 us; 32, N = 200, D = 64 10.55 either way, D = 128 15.3 -> 14.9; 64, N = 256 14.4 -> 13.2)
+    if (dtype == at::kFloat && q.numel() >= (int64_t(1) << 19) && flat_f32<3>({&q, &k, &v}, Dk) && reaches_f32(q)) {
         flat_rows<2>({&k, &v}, {&c.k, &c.v});
         c.q32 = q;
         c.q = tracked ? empty_flat(q, kdt) : q;

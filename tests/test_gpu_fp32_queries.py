@@ -8,8 +8,9 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-# keys split between wavefronts, one row block, edges of tiles and of 16-byte pieces, two mask tiles per request at any N and at multiples of 128
-@pytest.mark.parametrize("heads, N", [(3, 200), (3, 1), (5, 16), (6, 129), (96, 577), (100, 1000), (110, 1024)])
+# below the size from which the forward does it; keys split between wavefronts (up to head dim 64, at 128), one row block, edges of tiles and
+# of 16-byte pieces, two mask tiles per request at any N and at multiples of 128
+@pytest.mark.parametrize("heads, N", [(3, 200), (3, 1), (62, 200), (30, 193), (2000, 33), (3000, 16), (520, 129), (96, 577), (100, 1000), (110, 1024)])
 @pytest.mark.parametrize("D", [8, 32, 64, 80, 128])
 @pytest.mark.parametrize("layout", ["bhnd", "bnhd"])
 def test_same_bits_as_from_rounded_tensors(dev, heads, N, D, layout):
