@@ -130,9 +130,14 @@ template <int N> __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_
 // -> 11.1 us; 4 x 8, N = 512: 10.1 -> 7.9 us.  A wavefront now copies 16 KB per tile instead of 4, and a tile takes
 // 1.4 times as long.
 template <bool BF16, bool POSTMUL, bool PACKED_ROWS, int HDIM, bool BYTEMASK = false, bool BYPRODUCTS = false,
-          int FETCH = 0, bool SPLIT = false, bool WIDE_Q = false>
+          int FETCH = 0, bool SPLIT = false, bool WIDE_Q = false, bool HALVES = false>
 __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ? 2 : 3) void attn_fwd_kernel(const AttnArgs a)
 {
+    // HALVES: a work-group of 64 rows, two wavefronts to each 32 of them, which take 32 keys of every tile each and add their
+    // sums at the end.  A grid that leaves CUs without any 128-row work-group then has one on (almost) each, and a visit's chain of products,
+    // exponentials and products is half as long.  Forward, before -> now, D = 128: 7 heads, N = 2048 46.1 -> 36.1 us (packed 42.5 -> 32.0); 16,
+    // N = 1024 25.7 -> 21.0; 32, N = 512 15.6 -> 13.6; 32, N = 263 11.6 -> 10.7; D = 80: 5 heads, N = 3000 62.3 -> 52.3; 64, N = 192 8.7 -> 8.2.
+    static_assert(!HALVES || (HDIM > 64 && FETCH == 0 && !SPLIT), "HALVES: one tile's bytes at a time");
     static_assert(FETCH == 0 || (BYTEMASK && HDIM <= 64 && !SPLIT), "PAIRS: byte mask, two byte slots");
     constexpr bool PAIRS = FETCH != 0, WHOLE = FETCH == 1;
     using E = Elem<BF16>;
@@ -159,7 +164,8 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     // last rows first: where rows keep more keys the later they come (causal masks), the longest
     // work-groups of a head start first and the shortest fill the end of the launch
     const int qt = a.qtiles - 1 - (nid - bh * a.qtiles);
-    const int row_base = SPLIT ? qt * 32 : qt * BM + wave * 32;          // this wavefront's 32 query rows
+    const int half = HALVES ? wave >> 1 : 0;                             // which 32 keys of every tile
+    const int row_base = SPLIT ? qt * 32 : HALVES ? qt * 64 + (wave & 1) * 32 : qt * BM + wave * 32;     // this wavefront's 32 query rows
     const int N = a.N, nw = (N + 31) >> 5;
     const int T = (N + BN - 1) / BN;
     const bool ragged = (N & (BN - 1)) != 0;
@@ -175,8 +181,8 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     const uint32_t *mapw = nullptr, *mapw2 = nullptr;       // the two 64-row blocks (the same one if the second does not exist)
     if constexpr (!BYTEMASK) {
         if (a.tile_map != nullptr) {
-            mapw = a.tile_map + bi * a.map_sb + hi * a.map_sh + (size_t)(SPLIT ? qt >> 1 : 2 * qt) * 2 * TW;
-            mapw2 = (!SPLIT && 2 * qt + 1 < T) ? mapw + 2 * TW : mapw;
+            mapw = a.tile_map + bi * a.map_sb + hi * a.map_sh + (size_t)(SPLIT ? qt >> 1 : HALVES ? qt : 2 * qt) * 2 * TW;
+            mapw2 = (!SPLIT && !HALVES && 2 * qt + 1 < T) ? mapw + 2 * TW : mapw;
         }
     }
     // The first map words are read here, with ordinary (scalar) loads, long before they are needed:
@@ -310,11 +316,11 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     uint32_t some_acc = 0u, hole_acc = 0u;
     u32x4 pend = {0u, 0u, 0u, 0u};        // packed words waiting to be stored, see mask_words
     if constexpr (BYPRODUCTS) {
-        const bool writer = (a.mask.sb != 0 || bi == 0) && (a.mask.sh != 0 || hi == 0);
+        const bool writer = (a.mask.sb != 0 || bi == 0) && (a.mask.sh != 0 || hi == 0) && half == 0;
         const int Hm = a.mask.sh != 0 ? a.H : 1;
         const size_t slab_m = (size_t)((a.mask.sb != 0 ? bi : 0) * Hm + (a.mask.sh != 0 ? hi : 0));
         if (a.mask_out != nullptr && writer) words_out = a.mask_out + (slab_m * N + (qrow < N ? qrow : 0)) * nw;
-        if (a.map_out != nullptr && writer) map_dst = a.map_out + (slab_m * T + (SPLIT ? qt >> 1 : 2 * qt)) * 2 * TW;
+        if (a.map_out != nullptr && writer) map_dst = a.map_out + (slab_m * T + (SPLIT ? qt >> 1 : HALVES ? qt : 2 * qt)) * 2 * TW;
     }
     const uint32_t map_lds = lds0 + C::OFF_MAP + wave * (C::MAP_WORDS * 8);
     if constexpr (BYPRODUCTS && !SPLIT) {     // ordered before any arrival by the barriers of the main loop (T >= 1)
@@ -662,7 +668,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         }
     }
     if constexpr (WIDE_Q) {
-        uint16_t *q16 = a.q16.p != nullptr && (!SPLIT || wave == 0) ? slab(a.q16, bi, hi) : nullptr;
+        uint16_t *q16 = a.q16.p != nullptr && (SPLIT ? wave == 0 : half == 0) ? slab(a.q16, bi, hi) : nullptr;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int row = 8 * j + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
@@ -704,6 +710,13 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (t_first < T) issue_own_v(t_first);
     }
+    if constexpr (HALVES) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            kaddr[i] += 4096 * half;
+            vaddr[i >> 1][i & 1] += 4096 * half;
+        }
+    }
 
     // ---- running state: one query row per lane; both lane halves hold the same ref ----
     f32x16 oacc[OB];                    // [2 * half + dblk]: 32 columns each
@@ -740,23 +753,25 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     // One key tile for this wavefront.  `so` (LDS offset of the stage) is a compile-time constant
     // in every call, so all LDS addresses below are a register plus an immediate.
     // (SPLIT: `after_scores` runs when K has been read, `before_values` before V is.)
-    auto compute_tile_with = [&](const u32x2 w2, const uint32_t so, auto after_scores, auto before_values) __attribute__((always_inline)) {
+    constexpr int KB = HALVES ? 1 : 2;            // blocks of 32 keys that a wavefront takes of a tile
+    auto compute_tile_with = [&](const u32x2 both, const uint32_t so, auto after_scores, auto before_values) __attribute__((always_inline)) {
+        const u32x2 w2 = HALVES ? u32x2{half ? both.y : both.x, 0u} : both;
         if (__builtin_amdgcn_ballot_w64((w2.x | w2.y) != 0u) == 0ull) {
             after_scores();
             return;
         }
         // ---- S^T: sacc[blk][4g+j] = log2 weight / pm of (key 32blk + 8g + 4hh + j, query l32) ----
-        f32x16 sacc[2];
+        f32x16 sacc[KB];
         // The K fragments of MFMA step s + 1 are requested before the MFMAs of step s are issued, the
         // first pair before the table look-ups below.  The scheduling barriers hold that order: left
         // alone, the compiler requests each pair just before its MFMAs (it saves eight registers)
         // and the wavefront sits out four LDS round trips per tile one after the other.
         u32x4 kf[2][2];
         kf[0][0] = lds_read_b128(kaddr[0] + so);
-        kf[0][1] = lds_read_b128(kaddr[0] + so + 4096);
+        if constexpr (!HALVES) kf[0][1] = lds_read_b128(kaddr[0] + so + 4096);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int blk = 0; blk < 2; ++blk) {
+        for (int blk = 0; blk < KB; ++blk) {
             const uint32_t wa = (blk == 0 ? w2.x : w2.y) << nib_shift;
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
@@ -767,18 +782,18 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         }
         if (ref_used) {               // wave-uniform: some row of this wavefront has r != 0
             sacc[0] = E::mfma(ones, refb, sacc[0]);
-            sacc[1] = E::mfma(ones, refb, sacc[1]);
+            if constexpr (!HALVES) sacc[KB - 1] = E::mfma(ones, refb, sacc[KB - 1]);
         }
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
             if (s + 1 < KS) {
                 const uint32_t ka = kaddr[(s + 1) & 3] + so + ((s + 1) >> 2) * TILE_BYTES;
                 kf[(s + 1) & 1][0] = lds_read_b128(ka);
-                kf[(s + 1) & 1][1] = lds_read_b128(ka + 4096);
+                if constexpr (!HALVES) kf[(s + 1) & 1][1] = lds_read_b128(ka + 4096);
             }
             __builtin_amdgcn_sched_barrier(0);
             sacc[0] = E::mfma(kf[s & 1][0], qf[s], sacc[0]);
-            sacc[1] = E::mfma(kf[s & 1][1], qf[s], sacc[1]);
+            if constexpr (!HALVES) sacc[KB - 1] = E::mfma(kf[s & 1][1], qf[s], sacc[KB - 1]);
             __builtin_amdgcn_sched_barrier(0);
         }
         after_scores();
@@ -788,7 +803,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         auto recentre = [&]() __attribute__((always_inline)) {
             float mx = -__builtin_inff();
 #pragma unroll
-            for (int blk = 0; blk < 2; ++blk)
+            for (int blk = 0; blk < KB; ++blk)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) mx = __builtin_fmaxf(mx, sacc[blk][i]);
             mx = xhalf_max(mx);
@@ -809,7 +824,8 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
                 for (int i = 0; i < 16; ++i) {
 #pragma unroll
                     for (int b = 0; b < OB; ++b) oacc[b][i] *= alpha;
-                    sacc[0][i] += delta; sacc[1][i] += delta;
+                    sacc[0][i] += delta;
+                    if constexpr (!HALVES) sacc[KB - 1][i] += delta;
                 }
                 rmax = top + delta;
             } else {
@@ -817,11 +833,11 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
             }
         };
         // probabilities, packed as the B operands of the PV product; returns this lane's sum of them
-        uint32_t pb[2][2][4];
+        uint32_t pb[KB][2][4];
         auto exponentials = [&]() __attribute__((always_inline)) -> float {
             float lsum = 0.f;
 #pragma unroll
-            for (int blk = 0; blk < 2; ++blk)
+            for (int blk = 0; blk < KB; ++blk)
 #pragma unroll
                 for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -856,7 +872,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         before_values();
         // ---- O^T += V^T * P^T : oacc[b][4g+j] = out(query l32, d = 32b + 8g + 4hh + j) ----
 #pragma unroll
-        for (int blk = 0; blk < 2; ++blk)
+        for (int blk = 0; blk < KB; ++blk)
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
                 const u32x4 pv = {pb[blk][u][0], pb[blk][u][1], pb[blk][u][2], pb[blk][u][3]};
@@ -1025,13 +1041,13 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     }
     if constexpr (BYPRODUCTS && !SPLIT) {
         if (map_dst != nullptr) {
-            const int rb = wave >> 1;                          // block of 64 rows
+            const int rb = HALVES ? 0 : wave >> 1;             // block of 64 rows
             uint32_t before = 0u;
             if (lane == 0)
                 before = __hip_atomic_fetch_add((LDS_PTR(uint32_t))(uintptr_t)(lds0 + C::OFF_MAP_ARRIVED + 4 * rb), 1u,
                                                 __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
             before = __builtin_amdgcn_readfirstlane(before);
-            if (before == 1u && lane < TW && 2 * qt + rb < T) {
+            if (before == 1u && lane < TW && (HALVES || 2 * qt + rb < T)) {
                 const int w = lane;                            // word of 32 key tiles
                 const uint32_t src = lds0 + C::OFF_MAP + (uint32_t)(2 * rb) * (C::MAP_WORDS * 8) + (uint32_t)w * 8;
                 const u32x2 x0 = lds_read_b64(src), x1 = lds_read_b64(src + C::MAP_WORDS * 8);
@@ -1041,6 +1057,41 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
                 dst[TW + w] = ~(x0.y | x1.y) & in_range;
             }
         }
+    }
+
+    constexpr int HALF_SUMS = OB * 4096 + 1024;          // of one wavefront
+    if constexpr (HALVES) {
+        // Wavefronts 2 and 3 leave their sums for 0 and 1, which have the same rows, both moved to the larger reference point of
+        // those that have met a kept key.
+        const uint32_t sums = lds0 + (wave & 1) * HALF_SUMS;
+        const bool seen = rmax > -__builtin_inff();
+        __syncthreads();                                  // the last tile has been read by all
+        if (half == 1) {
+#pragma unroll
+            for (int b = 0; b < OB; ++b)
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    *(LDS_PTR(f32x4))(uintptr_t)(sums + (4 * b + g) * 1024 + lane * 16) =
+                        f32x4{oacc[b][4 * g], oacc[b][4 * g + 1], oacc[b][4 * g + 2], oacc[b][4 * g + 3]};
+            *(LDS_PTR(f32x2))(uintptr_t)(sums + OB * 4096 + lane * 8) = f32x2{seen ? ref : -__builtin_inff(), l_run};
+        }
+        __syncthreads();
+        if (half == 1) return;
+        const f32x2 other = *(LDS_PTR(const f32x2))(uintptr_t)(sums + OB * 4096 + lane * 8);
+        const float mine = seen ? ref : -__builtin_inff(), top = __builtin_fmaxf(mine, other.x);
+        ref = top > -__builtin_inff() ? top : 0.f;
+        // one that has met no kept key of the row has nothing to add (its factor is 0)
+        const float dm = mine - ref, d = other.x - ref;
+        const float fm = __builtin_amdgcn_exp2f(POSTMUL ? dm * pm : dm), f = __builtin_amdgcn_exp2f(POSTMUL ? d * pm : d);
+        l_run = __builtin_fmaf(other.y, f, l_run * fm);
+#pragma unroll
+        for (int b = 0; b < OB; ++b)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const f32x4 o = *(LDS_PTR(const f32x4))(uintptr_t)(sums + (4 * b + g) * 1024 + lane * 16);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) oacc[b][4 * g + j] = __builtin_fmaf(o[j], f, oacc[b][4 * g + j] * fm);
+            }
     }
 
     // ---- epilogue ----
@@ -1056,8 +1107,8 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     const float inv = (l_tot > 0.f) ? 1.0f / l_tot : 0.f;
     {
         const int row0 = row_base;
-        const uint32_t ebase = SPLIT ? lds0 : lds0 + (uint32_t)(visits & 1) * STAGE_BYTES + wave * 4096;
-        store_rows<BF16, OB>(oacc, inv, ebase, SPLIT ? 4096 : 16384, block_dst(a.out, a.out32, bi, hi, row0, D), a.out.p != nullptr,
+        const uint32_t ebase = SPLIT ? lds0 : HALVES ? lds0 + 2 * HALF_SUMS + wave * 4096 : lds0 + (uint32_t)(visits & 1) * STAGE_BYTES + wave * 4096;
+        store_rows<BF16, OB>(oacc, inv, ebase, SPLIT ? 4096 : HALVES ? 8192 : 16384, block_dst(a.out, a.out32, bi, hi, row0, D), a.out.p != nullptr,
                              BF16 && a.out32.p != nullptr, row0, N, lane);       // fp32 callers compute in bf16
     }
     if (qrow < N) {
@@ -1075,7 +1126,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
 
 // The instance for (fp32 q, element type, post-multiplier, row strides) and the kind of mask: 0 packed words, 1
 // boolean bytes, 2 the same with by-products, 3 and 4 those with two tiles' bytes per request, 5 to 7 the first
-// three with the keys split between the wavefronts, 8 and 9 as 3 and 4 at any N.  This file is
+// three with the keys split between the wavefronts, 8 and 9 as 3 and 4 at any N, 10 to 12 the first three in halves.  This file is
 // compiled once per head dim for the instances, side by side, and once for the launcher.
 typedef void (*FwdKernel)(const AttnArgs);
 #ifdef SMA_FWD_HEAD_DIM
@@ -1095,6 +1146,13 @@ template <int HDIM, bool BF16, bool POSTMUL, bool PACKED_ROWS, bool WIDE_Q = fal
         case 4: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true, 1, false, WIDE_Q>;
         case 8: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, false, 2, false, WIDE_Q>;
         case 9: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true, 2, false, WIDE_Q>;
+        }
+    }
+    if constexpr (HDIM > 64) {
+        switch (mask_kind) {
+        case 10: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, false, false, 0, false, WIDE_Q, true>;
+        case 11: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, false, 0, false, WIDE_Q, true>;
+        case 12: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true, 0, false, WIDE_Q, true>;
         }
     }
     return nullptr;
@@ -1160,6 +1218,15 @@ hipError_t launch_attn_fwd(const AttnArgs &args, bool bf16, hipStream_t stream)
             if (e != hipSuccess) return e;
         }
     }
+    // Beyond that line work-groups of 64 rows (HALVES at the kernel) while one on a CU holds them all, at head dims beyond 64.  With two on a
+    // CU they lose (8 x 8 heads, N = 512, D = 128: 17.0 -> 17.8 us), up to 64, where three share a CU, they gain and lose by turns (packed, 48 heads,
+    // N = 1024: 24.3 -> 22.2; 64, N = 512: 11.7 -> 12.1, boolean 13.1), and up to 128 keys there is nothing to share (6.6 us either way).
+    // The split stays ahead where it fits: 8 heads, N = 1024 16.9 against 21.3 us.
+    const bool halves = !split && a.D > HD && a.N > 2 * BN && (long long)a.BH * ((a.N + 63) / 64) <= cus;
+    if (halves) {
+        a.qtiles = (a.N + 63) / 64;
+        groups = (long long)a.BH * a.qtiles;
+    }
     a.div_qtiles = make_fastdiv((uint32_t)a.qtiles);
     a.tail_start = (!split && groups > 2 * cus && groups <= 3 * cus) ? 0 : (int)groups;
     const dim3 grid((unsigned)groups), block(NTHREADS);
@@ -1170,10 +1237,10 @@ hipError_t launch_attn_fwd(const AttnArgs &args, bool bf16, hipStream_t stream)
     const bool byproducts = a.mask_out != nullptr || a.map_out != nullptr;
     // two tiles' mask bytes per request (see PAIRS at the kernel), unless the grid is the single round of work-groups in
     // step for which tail_start was set to 0 above
-    const bool further = !split && a.byte_mask && D <= HD && a.tail_start != 0;
+    const bool further = !split && !halves && a.byte_mask && D <= HD && a.tail_start != 0;
     if (a.q_f32 && !bf16) return hipErrorInvalidValue;         // fp32 callers compute in bf16
     if (a.byte_mask && a.N < 16) return hipErrorInvalidValue;  // a row holds at least one 16-byte copy (checked by the C-ABI layer)
-    const int mask_kind = (split ? 5 : 0) + (!a.byte_mask ? 0 : (!further ? 1 : a.N % (2 * BN) == 0 ? 3 : 8) + (byproducts ? 1 : 0));
+    const int mask_kind = (split ? 5 : halves ? 10 : 0) + (!a.byte_mask ? 0 : (!further ? 1 : a.N % (2 * BN) == 0 ? 3 : 8) + (byproducts ? 1 : 0));
     const int variant = (a.q_f32 ? 8 : 0) | (bf16 ? 4 : 0) | (postmul ? 2 : 0) | (packed ? 1 : 0);
     const FwdKernel kernel = D == 32 ? fwd_kernel_32(variant, mask_kind) : D == 64 ? fwd_kernel_64(variant, mask_kind)
                              : D == 96 ? fwd_kernel_96(variant, mask_kind) : fwd_kernel_128(variant, mask_kind);
