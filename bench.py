@@ -433,7 +433,7 @@ def main():
         "roofline_bwd": {"kernel": " + ".join(bwd_kernels), "bound": "mfma",
                          "achieved": round(bwd_tflops, 2), "peak": harness.MI355X_MFMA_F16_TFLOPS,
                          "unit": "TFLOP/s", "frac": round(bwd_tflops / harness.MI355X_MFMA_F16_TFLOPS, 4),
-                         "traffic": measured_traffic(w.name, *bwd_kernels), "algorithmic_bytes": w.bwd_bytes},
+                         "traffic": measured_traffic(w.name, *bwd_kernels), "algorithmic_bytes": w.bwd_bytes(*bwd_kernels)},
     }
 
     result["roofline_attn"].update(roofline_ceiling(w.dense_flops, w.attn_bytes, attn_tflops))

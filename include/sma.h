@@ -154,9 +154,9 @@ int sma_attn_bwd(const void *dout, const void *q, const void *k, const void *v, 
                  const float *lse, const uint32_t *mask_packed, void *dq, void *dk, void *dv,
                  float *delta_ws, int B, int H, int N, int D, float scale, int dtype, void *stream);
 
-/* sma_attn_bwd with a tile map (see sma_tile_map) of the same packed mask: the two kernels visit only
- * the 64 x 64 blocks in which the mask keeps something (the one for short sequences has no use for the map
- * and does not read it).  tile_map == NULL is sma_attn_bwd; the gradients are the same bit for bit.  sma_attn_bwd_map_strided is the strided form (map
+/* sma_attn_bwd with a tile map (see sma_tile_map) of the same packed mask: the dQ and dK/dV kernels visit only
+ * the 64 x 64 blocks in which the mask keeps something (the one that holds a whole head, up to 256 or 512 keys, has no use
+ * for the map and does not read it).  tile_map == NULL is sma_attn_bwd; the gradients are the same bit for bit.  sma_attn_bwd_map_strided is the strided form (map
  * contiguous [Bm,Hm,T,2,TW] with the mask's own Bm, Hm).
  */
 int sma_attn_bwd_map(const void *dout, const void *q, const void *k, const void *v, const void *out,

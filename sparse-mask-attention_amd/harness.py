@@ -62,15 +62,17 @@ class Workload:
         S and dP are formed in both)."""
         return 10 * self.B * self.H * self.N * self.N * self.D
 
-    @property
-    def bwd_bytes(self) -> int:
-        """Algorithmic bytes of one backward (both launches): the dQ kernel reads q, k, v, dout, out,
-        the mask and lse and writes dq and delta; the dK/dV kernel reads q, k, v, dout, the mask, lse
-        and delta and writes dk and dv."""
+    def bwd_bytes(self, *kernels: str) -> int:
+        """Algorithmic bytes of the backward kernels named: dQ reads q, k, v, dout, out, the mask and lse and writes dq and delta; dK/dV
+        reads q, k, v, dout, the mask, lse and delta and writes dk and dv; the one for both reads what dK/dV reads and writes
+        all three; delta reads dout and out; the one of a whole head reads everything once and writes the three gradients."""
         mat = self.B * self.H * self.N * self.D * 2
         mask = 4 * self.B * self.H * self.N * self.n_words
         vec = 4 * self.B * self.H * self.N
-        return (6 * mat + mask + 2 * vec) + (6 * mat + mask + 2 * vec)
+        of = {"attn_bwd_dq_kernel": 6 * mat + mask + 2 * vec, "attn_bwd_dkv_kernel": 6 * mat + mask + 2 * vec,
+              "attn_bwd_both_kernel": 7 * mat + mask + 2 * vec, "attn_bwd_delta_kernel": 2 * mat + vec,
+              "attn_bwd_head_kernel": 8 * mat + mask + vec}
+        return sum(of[k] for k in kernels)
 
     @property
     def pack_bytes(self) -> int:

@@ -46,7 +46,7 @@ What differs from the reference, on purpose:
   disappear for the walk to pay.
 * ``.backward()`` works.  The reference calls a ``sparse_attn_cuda.backward`` that was never
   written (:91-94); here that function exists (HIP kernels, from the saved log-sum-exp and the packed mask: dQ and
-  dK/dV, or one for short sequences).  ``backward_recompute`` states the same gradients with PyTorch
+  dK/dV, or one for a whole head).  ``backward_recompute`` states the same gradients with PyTorch
   ops (the reference's own formulas, :97-111) for cross-checks.
 * ``SparseAttentionFunction`` has ``apply`` and nothing else of a ``torch.autograd.Function``: its node is native.  The node
   shows ``saved_tensors``, ``scale`` and ``tile_map``.  Forward-mode AD is refused (``NotImplementedError``), and a
