@@ -6,6 +6,7 @@ import sys
 import pytest
 import torch
 
+from _launches import launches, places
 from oracle import sma_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -50,3 +51,32 @@ def test_against_the_oracle(dev, N, D, heads, dtype):
             for got, ref, name in zip(grads, refs, ("dq", "dk", "dv")):
                 err = (got[b:b + 1, h:h + 1].float().cpu() - ref).abs()
                 assert (err <= floor + 1e-2 * ref.abs().max() + rtol * ref.abs()).all(), (name, b, h, scale, float(err.max()))
+
+
+# Heads as 32nds of a round of one work-group on a CU; with a tile map the kernels that visit only live tiles are ahead on grids that
+# leave part of their last round empty (and up to 384 keys after the first round on all).
+@pytest.mark.parametrize("N, D, part, map_given, whole", [
+    (512, 64, 24, False, True), (512, 64, 24, True, True), (512, 64, 16, False, False),
+    (512, 64, 40, False, True), (512, 64, 40, True, False), (512, 64, 60, True, True), (512, 64, 75, True, False),
+    (320, 64, 24, False, True), (320, 64, 24, True, True), (320, 64, 50, False, False), (320, 64, 60, False, True), (320, 64, 64, True, False),
+    (512, 32, 44, False, False), (512, 32, 50, False, True), (512, 32, 50, True, False), (512, 32, 64, True, True), (384, 32, 64, True, False)])
+def test_grids_that_take_it(dev, N, D, part, map_given, whole):
+    importlib.import_module("python.sparse_attention")
+    sa = sys.modules["python.sparse_attention"]
+    heads = part * places() // 32
+    g = torch.Generator(device=dev).manual_seed(N + part)
+    q, k, v, do = (torch.randn(1, heads, N, D, device=dev, generator=g).half() for _ in range(4))
+    nb = (N + 63) // 64
+    blocks = (torch.rand(1, 1, nb, nb, device=dev, generator=g) < 0.25) | torch.eye(nb, dtype=torch.bool, device=dev)
+    mask = blocks.repeat_interleave(64, 2)[:, :, :N].repeat_interleave(64, 3)[..., :N].contiguous()
+    packed = sa.pack_mask(mask)
+    leaves = [t.requires_grad_(True) for t in (q, k, v)]
+    out = sa.sparse_attention(*leaves, None, mask_packed=packed, tile_map=sa.tile_map(packed, min_skip=0.0) if map_given else None)
+    grads = []
+    kernels = [name for name, _, _ in launches(lambda: grads.extend(torch.autograd.grad(out, leaves, do)))]
+    assert (kernels == ["attn_bwd_head_kernel"]) == whole, kernels
+    h = heads - 1
+    refs = O.sparse_attention_bwd_ref(*(t[:, h:h + 1].detach().float().cpu() for t in (q, k, v)), mask.cpu(), do[:, h:h + 1].float().cpu(), scale=D ** -0.5)
+    for got, ref, name in zip(grads, refs, ("dq", "dk", "dv")):          # the bound of the test above
+        err = (got[:, h:h + 1].float().cpu() - ref).abs()
+        assert (err <= 1e-4 + 1e-2 * ref.abs().max() + 1e-2 * ref.abs()).all(), (name, float(err.max()))
