@@ -498,7 +498,10 @@ template <bool BF16, int HDIM, int NW, int KB, bool WIDE> void launch(hipStream_
 template <bool BF16, bool WIDE> bool pick(hipStream_t stream, const AttnBwdArgs &a)
 {
     // Backward alone, inputs in turn, the two kernels of attn_bwd.hip against this one:
-    // up to 256 keys it is the faster at any number of heads (D = 64, N = 256: 8 heads 18.8, 17.6 us, 96: 21.1, 19.2; D = 128: 32 heads 28.7, 25.6).
+    // up to 256 keys it is the faster (D = 64, N = 256: 85 heads 19.1, 18.9 us, 256: 31.0, 24.0; 8 heads, N = 128: 9.8, 9.2; D = 128: 85 heads 30.9, 27.8),
+    // except from 129 keys on (head dim 128: 193) where both rows and both keys of every head have a CU for themselves, side by side
+    // in one launch: there this one leaves CUs idle (8 heads, N = 256: D = 64 13.3, 17.5 us, D = 32 10.4, 14.1, D = 96 15.5, 21.9, D = 128 20.0, 25.2;
+    // 64 heads 15.0, 18.5;  N = 160, 8 heads: D = 64 11.6, 12.5, D = 128 17.5, 17.1).
     // 129 to 256 keys at head dims up to 64: eight wavefronts of 32 keys while every head has a CU of its own (64 heads 19.7 us, four
     // wavefronts of 64 keys 23.1; 256: 25.5, 27.9), beyond that the four, two work-groups to a CU (300: 44.4 against 38.4).
     // 257 to 512 keys: a work-group has a CU for itself and a round takes the same time however few heads it holds, so that
@@ -512,6 +515,7 @@ template <bool BF16, bool WIDE> bool pick(hipStream_t stream, const AttnBwdArgs 
     // 480 95.3, 95.7;  N = 320: 600 70.9, 85.8 / 79.7, 88.0;  1000 111, 118.
     const int D = kernel_head_dim(a.D), N = a.N;
     const long long cus = compute_units(), rounds = cus > 0 ? (a.BH + cus - 1) / cus : 1;
+    if (N > (D == 128 ? 192 : 128) && 4 * (long long)a.BH <= cus) return false;
     const bool own_cu = a.BH <= cus, map = a.tile_map != nullptr;
     const int need = rounds == 1 ? (N > 384 ? 18 : 20) : N <= 384 ? (map ? 33 : rounds == 2 ? 27 : 29) : (D == 64 ? 20 : 24) + (map ? 6 : 0);
     const bool filled = 32 * (long long)a.BH >= need * rounds * cus;
