@@ -539,6 +539,8 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
             uint32_t pp[2][4], ps[2][4];
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
+                // (one wait for the words less far ahead, or four registers more than there are: each reload in this loop waits for the copies)
+                if constexpr (HALVES && POSTMUL) if (g == 1) __builtin_amdgcn_sched_barrier(0);
                 float p[4], d[4];
                 const u32x4 mg = VLDS ? mask_words(g) : mw[g];
 #pragma unroll
@@ -599,20 +601,24 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
         }
         __syncthreads();
         if (half == 1 || !wave_valid) return;
+        // One gradient after the other: with both sums in registers at once 17 to 20 of them were spilled, here and because of their allocation to the
+        // whole kernel, which took 256 registers for 246 (36 heads, N = 2048, the backward alone: 329.6 -> 327.8 us; 128, N = 4096: 3326 -> 3308).
+        auto add = [&](f32x16 (&acc)[OB], uint32_t at) __attribute__((always_inline)) {
 #pragma unroll
-        for (int b = 0; b < OB; ++b) {
-            __builtin_amdgcn_sched_barrier(0);            // one block's sums in registers at a time
+            for (int b = 0; b < OB; ++b) {
+                __builtin_amdgcn_sched_barrier(0);        // one block's sums in registers at a time
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const f32x4 x = *(LDS_PTR(f32x4))(uintptr_t)(sums + (4 * b + g) * 1024), y = *(LDS_PTR(f32x4))(uintptr_t)(sums + (4 * (OB + b) + g) * 1024);
+                for (int g = 0; g < 4; ++g) {
+                    const f32x4 x = *(LDS_PTR(f32x4))(uintptr_t)(at + (4 * b + g) * 1024);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    dkacc[b][4 * g + j] += x[j];
-                    dvacc[b][4 * g + j] += y[j];
+                    for (int j = 0; j < 4; ++j) acc[b][4 * g + j] += x[j];
                 }
             }
-        }
+        };
+        add(dkacc, sums);
         store_gradient<BF16, WIDE>(dkacc, a.scale, lds0 + wave * (OB * 8192), a, a.dk, bi, hi, key0, lane);      // over its own sums
+        __builtin_amdgcn_sched_barrier(0);
+        add(dvacc, sums + OB * 4096);
         store_gradient<BF16, WIDE>(dvacc, 1.0f, lds0 + wave * (OB * 8192), a, a.dv, bi, hi, key0, lane);
         return;
     }
