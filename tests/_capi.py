@@ -37,6 +37,14 @@ class SmaTensor(ctypes.Structure):
         return cls(t.data_ptr(), t.stride(0), t.stride(1), t.stride(2))
 
 
+class SmaFwdCall(ctypes.Structure):
+    """struct sma_fwd_call of include/sma.h."""
+    _fields_ = ([(n, ctypes.POINTER(SmaTensor)) for n in ("q", "k", "v", "out", "out_f32")] +
+                [("mask", ctypes.c_void_p), ("mask_packed", ctypes.c_void_p), ("mask_stride_b", ctypes.c_int64), ("mask_stride_h", ctypes.c_int64)] +
+                [(n, ctypes.c_void_p) for n in ("tile_map", "lse", "packed_out", "map_out")] +
+                [(n, ctypes.c_int) for n in "BHND"] + [("scale", ctypes.c_float), ("dtype", ctypes.c_int)])
+
+
 def load():
     global _lib
     if _lib is None:
@@ -83,6 +91,10 @@ def load():
         lib.sma_attn_fwd_bool_mask_map.argtypes = [vp, vp, vp, vp, i64, i64, vp, vp, vp, vp, ci, ci, ci, ci, cf, ci, vp]
         lib.sma_attn_fwd_bool_mask_strided.restype = ci
         lib.sma_attn_fwd_bool_mask_strided.argtypes = [tp, tp, tp, vp, i64, i64, tp, vp, vp, vp, ci, ci, ci, ci, cf, ci, vp]
+        lib.sma_attn_fwd_call.restype = ci
+        lib.sma_attn_fwd_call.argtypes = [ctypes.POINTER(SmaFwdCall), vp]
+        lib.sma_attn_fwd_call_q32.restype = ci
+        lib.sma_attn_fwd_call_q32.argtypes = [ctypes.POINTER(SmaFwdCall), tp, vp]
         _lib = lib
     return _lib
 
