@@ -505,19 +505,22 @@ template <bool BF16, bool WIDE> bool pick(hipStream_t stream, const AttnBwdArgs 
     // 129 to 256 keys at head dims up to 64: eight wavefronts of 32 keys while every head has a CU of its own (64 heads 19.7 us, four
     // wavefronts of 64 keys 23.1; 256: 25.5, 27.9), beyond that the four, two work-groups to a CU (300: 44.4 against 38.4).
     // 257 to 512 keys: a work-group has a CU for itself and a round takes the same time however few heads it holds, so that
-    // most of the places must be taken, `need` of 32.  Up to 384 keys a quarter or more of the wavefronts have no keys, at head dims up to 32 the others'
-    // products are cheaper, and with a tile map the others visit only the tiles that hold something, where here every row is visited by
-    // all and skipped by wavefront: after the first round each of the three asks for more.  Random masks, D = 64 (others, this one, us):
-    //   N = 512   128 heads 46.5, 51.7;  150 57.8, 53.4;  320 105.1, 106.9;  400 133.9, 116.7;  600 188, 167
-    //   N = 320   160 heads 32.1, 33.8;  175 38.3, 34.3;  400 69.0, 71.1;  440 79.3, 73.5;  1000 155, 149;  1300 193, 210
-    //   D = 32    N = 512: 160 heads 41.8, 38.2;  320 69.4, 77.7;  400 88.6, 80.0;  600 124, 121;   N = 384: 400 54.7, 59.5;  480 63.4, 62.8
-    // and with a map, of blocks kept by a quarter / causal, N = 512: 160 heads 42.0, 47.9 / 52.1, 47.2;  320 69.8, 90.5 / 88.4, 94.0;  600 121, 138 / 153, 144;
-    // 480 95.3, 95.7;  N = 320: 600 70.9, 85.8 / 79.7, 88.0;  1000 111, 118.
+    // most of the places must be taken, `need` of 32: more up to 384 keys, where a quarter or more of the wavefronts have no keys, and after the
+    // first round at head dims up to 32, whose products are cheaper.  With a tile map the others visit only the tiles that hold
+    // something, where here all rows are visited and wavefronts skip; but the gradients are the same bits with and without a map, so
+    // the line is one for all masks.  Random masks without a map (others, this one, us), where they differ from it in sign after the stroke blocks kept by a quarter,
+    // with a map:
+    //   D = 64   N = 512: 128 heads 46.5, 51.7;  160 59.2, 52.7 / 42.0, 48.0;  330 111, 106 / 73, 91;  400 134, 117 / 83, 94;  480 155, 125;  600 188, 167 / 121, 138
+    //            N = 320: 160 heads 32.1, 33.8;  175 38.3, 34.3;  400 69.0, 71.1;  440 79.3, 73.5 / 53.9, 59.6;  1000 155, 149 / 111, 118;  1300 193, 210
+    //   D = 32   N = 512: 160 heads 41.8, 38.2;  320 69.4, 77.7;  400 88.6, 80.0 / 57.7, 66.3;  600 124, 121 / 80, 98;  700 137, 125 / 88, 100
+    //            N = 384: 400 heads 54.7, 59.5;  480 63.4, 62.8;  768 92.5, 91.5 / 67.5, 79.2;  1300 148, 159
+    // Over 2000 such grids, masks and maps the kernel taken is on average 0.6 % behind the better one for random and causal masks, 2.7 % for blocks with a map.
     const int D = kernel_head_dim(a.D), N = a.N;
     const long long cus = compute_units(), rounds = cus > 0 ? (a.BH + cus - 1) / cus : 1;
     if (N > (D == 128 ? 192 : 128) && 4 * (long long)a.BH <= cus) return false;
-    const bool own_cu = a.BH <= cus, map = a.tile_map != nullptr;
-    const int need = rounds == 1 ? (N > 384 ? 18 : 20) : N <= 384 ? (map ? 33 : rounds == 2 ? 27 : 29) : (D == 64 ? 20 : 24) + (map ? 6 : 0);
+    const bool own_cu = a.BH <= cus;
+    const int need = rounds == 1 ? (N > 384 ? 20 : 22) : N > 384 ? (D == 64 ? 23 : rounds == 2 ? 24 : 26) : D == 64 ? (rounds == 2 ? 27 : 29)
+                                                                                                              : rounds == 2 ? 30 : 33;
     const bool filled = 32 * (long long)a.BH >= need * rounds * cus;
     auto narrow = [&](auto d_c) {
         constexpr int HDIM = decltype(d_c)::value;

@@ -6,6 +6,7 @@ import sys
 import pytest
 import torch
 
+from _launches import launches
 from oracle import sma_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -40,9 +41,13 @@ def test_halves_against_the_oracle(dev, heads, N, D, dtype, scale):
     leaves = [t.detach().requires_grad_(True) for t in (q, k, v)]
     scale = D ** -0.5 if scale is None else scale
     packed = sa.pack_mask(mask)
-    out = sa.SparseAttentionFunction.apply(*leaves, None, mask, scale, N)
-    again = sa.SparseAttentionFunction.apply(*leaves, packed, None, scale, N)
-    mapped = sa.SparseAttentionFunction.apply(*leaves, packed, None, scale, N, sa.tile_map(packed, min_skip=0.0))
+    tile_map = sa.tile_map(packed, min_skip=0.0)
+    made = []
+    ran = launches(lambda: made.extend([sa.SparseAttentionFunction.apply(*leaves, None, mask, scale, N),
+                                        sa.SparseAttentionFunction.apply(*leaves, packed, None, scale, N),
+                                        sa.SparseAttentionFunction.apply(*leaves, packed, None, scale, N, tile_map)]))
+    assert [args[9] for name, args, _ in ran if name == "attn_fwd_kernel"] == ["true"] * 3, ran           # HALVES
+    out, again, mapped = made
     assert torch.equal(out, again) and torch.equal(out, mapped)
     lse, words = out.grad_fn.saved_tensors[4:6]
     assert torch.equal(lse, again.grad_fn.saved_tensors[4]) and torch.equal(words.view_as(packed), packed)      # by-products
@@ -78,7 +83,10 @@ def test_map_by_product(dev, heads, N):
     mask[:, :, 40:50] = False
     q, k, v, do = (torch.randn(1, heads, N, 128, device=dev, generator=g).half() for _ in range(4))
     leaves = [t.requires_grad_(True) for t in (q, k, v)]
-    out = sa.sparse_attention(*leaves, mask, tile_map=True)
+    outs = []
+    ran = launches(lambda: outs.append(sa.sparse_attention(*leaves, mask, tile_map=True)))
+    assert [args[9] for name, args, _ in ran if name == "attn_fwd_kernel"] == ["true"], ran
+    out = outs[0]
     made = out.grad_fn.tile_map
     assert torch.equal(made.flatten(), sa.tile_map(sa.pack_mask(mask), min_skip=0.0).flatten())
     plain = sa.sparse_attention(*leaves, mask)
