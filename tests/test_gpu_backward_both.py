@@ -5,6 +5,7 @@ import sys
 import pytest
 import torch
 
+from _launches import launches
 from oracle import sma_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -30,7 +31,9 @@ def test_one_round_against_the_oracle(dev, N, D, dtype):
     mask[0, :, :, 192:320] = False                                    # a work-group's keys without any
     leaves = [t.detach().requires_grad_(True) for t in (q, k, v)]
     out = sa.sparse_attention(*leaves, mask.to(dev))
-    grads = torch.autograd.grad(out, leaves, do, retain_graph=True)
+    grads = []
+    kernels = [name for name, _, _ in launches(lambda: grads.extend(torch.autograd.grad(out, leaves, do, retain_graph=True)))]
+    assert kernels[-2:] == ["attn_bwd_delta_kernel", "attn_bwd_both_kernel"], kernels
     assert all(torch.equal(x, y) for x, y in zip(grads, torch.autograd.grad(out, leaves, do)))
     rtol = 1e-2 if dtype == torch.float16 else 2e-2
     for b, h in ((0, 0), (1, 2)):
@@ -55,6 +58,10 @@ def test_same_bits_with_a_tile_map(dev, D, heads, N, dtype):
     tile_map = sa.tile_map(packed, min_skip=0.0)
     assert tile_map is not None
     leaves = [t.requires_grad_(True) for t in (q, k, v)]
-    with_map = torch.autograd.grad(sa.sparse_attention(*leaves, None, mask_packed=packed, tile_map=tile_map), leaves, do)
-    without = torch.autograd.grad(sa.sparse_attention(*leaves, None, mask_packed=packed), leaves, do)
+    ways = []
+    for given, one in ((tile_map, D == 64), (None, False)):
+        out = sa.sparse_attention(*leaves, None, mask_packed=packed, tile_map=given)
+        ran = launches(lambda: ways.append(torch.autograd.grad(out, leaves, do)))
+        assert any(name == "attn_bwd_both_kernel" for name, _, _ in ran) == one, ran
+    with_map, without = ways
     assert all(torch.equal(x, y) for x, y in zip(with_map, without))
