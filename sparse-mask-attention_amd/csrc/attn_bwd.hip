@@ -365,8 +365,9 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
     // end.  One CU holds one work-group of eight wavefronts, so a grid just beyond a round took two: its last heads, where work-groups of 128 keys
     // hold them all at once, come in such ones, each three quarters as long as a whole one.  The backward alone, before -> now, in us:
     //   36 heads, N = 2048: 377 -> 343 (causal 281 -> 247);  48: 394 -> 365;  68: 596 -> 560;  72, N = 1000: 206 -> 192;  18, N = 4000,
-    //   causal: 489 -> 421;  forward + backward, 40, N = 2048, one mask in blocks: 276 -> 248.  Of 35 grids one lost: 24 heads, N = 3000, causal,
-    //   whose short work-groups had filled the second round by themselves: 286 -> 301.
+    //   causal: 489 -> 421;  forward + backward, 40, N = 2048, one mask in blocks: 276 -> 248.  Of 70 grids of 17 to 96 heads, random, causal and causal
+    //   with a map, one lost: 24 heads, N = 3000, causal without a map, whose short work-groups fill the second round by themselves: 271 -> 286 (with a
+    //   map 254 either way, random 514 -> 462).
     static_assert(!HALVES || (NW == 8 && VLDS && OB * 2 * 4096 * 4 <= C::LDS_BYTES), "four wavefronts' sums fit the LDS");
     constexpr int KW = HALVES ? 4 : NW;               // wavefronts side by side on different keys
     const int half = HALVES ? wave >> 2 : 0;          // ... and which 32 rows of every tile this one takes
@@ -660,7 +661,10 @@ __global__ __launch_bounds__(64 * NW, HDIM == 128 ? NW / 4 : HDIM == 32 ? 4 : VL
 //   blocks, map   forward + backward, 12 heads, N = 1024: batch 16 156 -> 149, 8 86.7 -> 82.0, 4 66.9 -> 55.2;
 //                 16 x 12, N = 700: 104.9 -> 95.2;  2 x 8, N = 4096: 178 -> 165
 //   random, map   (one of a mask in which nothing can be skipped) 16 x 12 heads, N = 1024: 274.2 -> 275.5;  4 x 32, N = 2048: 687.7 -> 685.1;
-//                 4 x 8, N = 4096: 672 -> 646;  3 x 12, N = 2048: 228.8 -> 206.5;  4 x 8, N = 2048, a third more than a round: 186 -> 190 (causal 168 -> 148)
+//                 4 x 8, N = 4096: 672 -> 646;  3 x 12, N = 2048: 228.8 -> 206.5
+//   up to a third beyond full rounds, with a map    random masks lose, those that a map is made for gain: 16 heads, N = 4096 random 260 -> 272, causal
+//                 229 -> 185, blocks 135 -> 117;  13, N = 4096 237 -> 251, 220 -> 173, 131 -> 113;  64, N = 1024 79.1 -> 82.0, 68.2 -> 63.2, 52.5 ->
+//                 49.1;  70, N = 700 52.5 -> 55.1, 44.1 -> 43.4, 42.1 -> 36.6
 // Beyond one round and without a map it is left off: 192 heads, N = 1024: 214 -> 221; 60, N = 1000 (1.25 rounds): 74 -> 84 (causal masks would gain:
 // 128, N = 1000: 125 -> 109, but the launcher doesn't see them; D = 32 with a map: 384 heads, N = 600: 94.2 -> 96.6;
 // D = 96 with a map: blocks 8 x 12, N = 1024 145 -> 131, but 8 x 16, N = 2048 443 -> 447, and a random mask 907 -> 932).

@@ -497,24 +497,26 @@ template <bool BF16, int HDIM, int NW, int KB, bool WIDE> void launch(hipStream_
 }
 template <bool BF16, bool WIDE> bool pick(hipStream_t stream, const AttnBwdArgs &a)
 {
-    // Backward alone, inputs in turn, the two kernels of attn_bwd.hip against this one:
-    // up to 256 keys it is the faster (D = 64, N = 256: 85 heads 19.1, 18.9 us, 256: 31.0, 24.0; 8 heads, N = 128: 9.8, 9.2; D = 128: 85 heads 30.9, 27.8),
+    // Backward alone, inputs in turn, the kernels of attn_bwd.hip against this one, in us:
+    // up to 256 keys it is the faster (D = 64, N = 256: 85 heads 19.1, 18.9, 256: 31.0, 24.0; 8 heads, N = 128: 9.8, 9.2; D = 128: 85 heads 30.9, 27.8),
     // except from 129 keys on (head dim 128: 193) where both rows and both keys of every head have a CU for themselves, side by side
-    // in one launch: there this one leaves CUs idle (8 heads, N = 256: D = 64 13.3, 17.5 us, D = 32 10.4, 14.1, D = 96 15.5, 21.9, D = 128 20.0, 25.2;
+    // in one launch: there this one leaves CUs idle (8 heads, N = 256: D = 64 13.3, 17.5, D = 32 10.4, 14.1, D = 96 15.5, 21.9, D = 128 20.0, 25.2;
     // 64 heads 15.0, 18.5;  N = 160, 8 heads: D = 64 11.6, 12.5, D = 128 17.5, 17.1).
-    // 129 to 256 keys at head dims up to 64: eight wavefronts of 32 keys while every head has a CU of its own (64 heads 19.7 us, four
-    // wavefronts of 64 keys 23.1; 256: 25.5, 27.9), beyond that the four, two work-groups to a CU (300: 44.4 against 38.4).
+    // 129 to 256 keys at head dims up to 64: eight wavefronts of 32 keys while every head has a CU of its own (256 heads 25.5, four
+    // wavefronts of 64 keys 27.9), beyond that the four, two work-groups to a CU (300: 44.4 against 38.4).
     // 257 to 512 keys: a work-group has a CU for itself and a round takes the same time however few heads it holds, so that
-    // most of the places must be taken, `need` of 32: more up to 384 keys, where a quarter or more of the wavefronts have no keys, and after the
-    // first round at head dims up to 32, whose products are cheaper.  With a tile map the others visit only the tiles that hold
-    // something, where here all rows are visited and wavefronts skip; but the gradients are the same bits with and without a map, so
-    // the line is one for all masks.  Random masks without a map (others, this one, us), where they differ from it in sign after the stroke blocks kept by a quarter,
-    // with a map:
-    //   D = 64   N = 512: 128 heads 46.5, 51.7;  160 59.2, 52.7 / 42.0, 48.0;  330 111, 106 / 73, 91;  400 134, 117 / 83, 94;  480 155, 125;  600 188, 167 / 121, 138
-    //            N = 320: 160 heads 32.1, 33.8;  175 38.3, 34.3;  400 69.0, 71.1;  440 79.3, 73.5 / 53.9, 59.6;  1000 155, 149 / 111, 118;  1300 193, 210
+    // most of the places must be taken, `need` of 32: more up to 384 keys, where a quarter or more of the wavefronts have no keys, and after
+    // the first round at head dims up to 32, whose products are cheaper.  With a tile map the others visit only the tiles that hold
+    // something, where here all rows are visited and wavefronts skip; but the gradients are the same bits with and without a map, so the line is
+    // one for all masks.  Random masks without a map, and after the stroke blocks kept by a quarter, with one:
+    //   D = 64   N = 512: 128 heads 46.5, 51.7;  160 59.2, 52.7 / 42.0, 48.0;  330 111, 106 / 73, 91;  400 134, 117 / 83, 94;  480 155, 125;
+    //            600 188, 167 / 121, 138
+    //            N = 320: 160 heads 32.1, 33.8;  175 38.3, 34.3;  400 69.0, 71.1;  440 79.3, 73.5 / 53.9, 59.6;  1000 155, 149 / 111, 118;
+    //            1300 193, 210 (N = 300)
     //   D = 32   N = 512: 160 heads 41.8, 38.2;  320 69.4, 77.7;  400 88.6, 80.0 / 57.7, 66.3;  600 124, 121 / 80, 98;  700 137, 125 / 88, 100
-    //            N = 384: 400 heads 54.7, 59.5;  480 63.4, 62.8;  768 92.5, 91.5 / 67.5, 79.2;  1300 148, 159
-    // Over 2000 such grids, masks and maps the kernel taken is on average 0.6 % behind the better one for random and causal masks, 2.7 % for blocks with a map.
+    //            N = 384: 400 heads 54.7, 59.5;  480 63.4, 62.8;  768 92.5, 91.5 / 67.5, 79.2;  1300 148, 159 (N = 350)
+    // Over 2000 such grids, masks and maps the kernel taken is on average 0.6 % behind the better one for random and causal masks, 2.7 % for
+    // blocks with a map.
     const int D = kernel_head_dim(a.D), N = a.N;
     const long long cus = compute_units(), rounds = cus > 0 ? (a.BH + cus - 1) / cus : 1;
     if (N > (D == 128 ? 192 : 128) && 4 * (long long)a.BH <= cus) return false;

@@ -597,10 +597,11 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     // Requested at once, oldest first: q (this wave's 32 rows, staged through the second K/V stage,
     // which the prologue leaves unused, K-swizzled), then K/V and the mask words of tile 0.
     // WIDE_Q (q in fp32): the same pieces through registers, rounded once the copies below are on their way.  q is read by one
-    // work-group alone, so this replaces a pass over it: 6 bytes an element instead of 8 with the rounded q kept, 4 without.  Separate
-    // pass -> this: forward, 384 heads, N = 200: 32.1 -> 29.1 us; 192, N = 512: 46.1 -> 44.4; 96, N = 577, D = 80: 42.0 -> 40.9;
-    // forward + backward, the last 121.8 -> 119.9, 64, N = 1000, D = 128: 218.0 -> 213.4.  As an instance of its own: decided at run time, the
-    // other element types' loops came out 0.5 to 1 % slower.
+    // work-group alone, so this replaces a pass over it: 6 bytes an element instead of 8 with the rounded q kept, 4 without.  Conversion and
+    // forward, separate pass -> this: 192 heads, N = 512, D = 128: 75.8 -> 69.8 us, D = 64: 42.9 -> 39.8; with the rounded q kept 81.2 -> 79.8 and
+    // 46.4 -> 44.8.  Where it does not pay stands at its callers' rule (forward_rounds_q in binding.cpp).  What it could give and does not: the
+    // compiler's waits for these loads also wait for the copies issued after them, which it knows nothing of.  As an instance of its own: decided at
+    // run time, the other element types' loops came out 0.5 to 1 % slower.
     const uint32_t q_dst = SPLIT ? split_dst + C::OFF_V : lds0 + (NSTAGE - 1) * STAGE_BYTES + wave * 4096;
     f32x4 wide[WIDE_Q ? 4 * NH : 1][2];
     {
