@@ -142,7 +142,7 @@ int sma_attn_fwd_map(const void *q, const void *k, const void *v, const uint32_t
  *                       row on return (the library never allocates)
  *
  * One or two launches on `stream`: sequences of up to 256 keys, and with D up to 64 many of up to 512, run in one kernel that holds
- * a whole head in a work-group; others, and few heads of more than 128 keys, in two (dq, then dk and dv; or delta, then both).
+ * a whole head in a work-group; others in two (dq, then dk and dv; or delta, then both).
  * No atomics, results are bit-reproducible.
  *
  * Replaces: void sparse_attention_bwd_bf16(const SparseAttentionParams&, const void* dout,

@@ -498,10 +498,11 @@ template <bool BF16, int HDIM, int NW, int KB, bool WIDE> void launch(hipStream_
 template <bool BF16, bool WIDE> bool pick(hipStream_t stream, const AttnBwdArgs &a)
 {
     // Backward alone, inputs in turn, the kernels of attn_bwd.hip against this one, in us:
-    // up to 256 keys it is the faster (D = 64, N = 256: 85 heads 19.1, 18.9, 256: 31.0, 24.0; 8 heads, N = 128: 9.8, 9.2; D = 128: 85 heads 30.9, 27.8),
-    // except from 129 keys on (head dim 128: 193) where both rows and both keys of every head have a CU for themselves, side by side
-    // in one launch: there this one leaves CUs idle (8 heads, N = 256: D = 64 13.3, 17.5, D = 32 10.4, 14.1, D = 96 15.5, 21.9, D = 128 20.0, 25.2;
-    // 64 heads 15.0, 18.5;  N = 160, 8 heads: D = 64 11.6, 12.5, D = 128 17.5, 17.1).
+    // up to 256 keys always (D = 64, N = 256: 85 heads 19.1, 18.9, 256: 31.0, 24.0; 8 heads, N = 128: 9.8, 9.2; D = 128: 85 heads 30.9, 27.8).  From
+    // 129 keys on few heads, of which the others give the rows and the keys a CU each, side by side in one launch, would be faster there (8
+    // heads, N = 256: D = 64 13.3, 17.5, D = 128 20.0, 25.2; 64 heads 15.0, 18.5; more than 64 not), but dK and dV would be further from 64 bits than
+    // they are: the others' dK/dV kernel scales and rounds k where the forward rounded scaled q (relative 2-norm of dK, bf16, N = 256, D = 64: 0.00312
+    // against 0.00287; 0.00052 against 0.00050 in fp16 at N = 512).
     // 129 to 256 keys at head dims up to 64: eight wavefronts of 32 keys while every head has a CU of its own (256 heads 25.5, four
     // wavefronts of 64 keys 27.9), beyond that the four, two work-groups to a CU (300: 44.4 against 38.4).
     // 257 to 512 keys: a work-group has a CU for itself and a round takes the same time however few heads it holds, so that
@@ -519,7 +520,6 @@ template <bool BF16, bool WIDE> bool pick(hipStream_t stream, const AttnBwdArgs 
     // blocks with a map.
     const int D = kernel_head_dim(a.D), N = a.N;
     const long long cus = compute_units(), rounds = cus > 0 ? (a.BH + cus - 1) / cus : 1;
-    if (N > (D == 128 ? 192 : 128) && 4 * (long long)a.BH <= cus) return false;
     const bool own_cu = a.BH <= cus;
     const int need = rounds == 1 ? (N > 384 ? 20 : 22) : N > 384 ? (D == 64 ? 23 : rounds == 2 ? 24 : 26) : D == 64 ? (rounds == 2 ? 27 : 29)
                                                                                                               : rounds == 2 ? 30 : 33;

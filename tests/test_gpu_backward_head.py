@@ -55,29 +55,6 @@ def test_against_the_oracle(dev, N, D, heads, dtype):
                 assert (err <= floor + 1e-2 * ref.abs().max() + rtol * ref.abs()).all(), (name, b, h, scale, float(err.max()))
 
 
-# Few heads of 129 keys or more (193 at head dim 128): rows and keys of a head on CUs of their own, in one launch.
-@pytest.mark.parametrize("N, D, part, whole", [
-    (128, 64, 1, True), (129, 64, 1, False), (256, 64, 8, False), (256, 64, 9, True), (160, 32, 8, False), (256, 96, 8, False), (200, 80, 9, True),
-    (192, 128, 8, True), (193, 128, 8, False), (256, 128, 9, True)])
-def test_few_heads(dev, N, D, part, whole):
-    importlib.import_module("python.sparse_attention")
-    sa = sys.modules["python.sparse_attention"]
-    heads = part * places() // 32
-    g = torch.Generator(device=dev).manual_seed(N + part)
-    q, k, v, do = (torch.randn(1, heads, N, D, device=dev, generator=g).half() for _ in range(4))
-    mask = torch.rand(1, heads, N, N, device=dev, generator=g) < 0.3
-    leaves = [t.requires_grad_(True) for t in (q, k, v)]
-    out = sa.sparse_attention(*leaves, mask)
-    grads = []
-    kernels = [name for name, _, _ in launches(lambda: grads.extend(torch.autograd.grad(out, leaves, do)))]
-    assert kernels == (["attn_bwd_head_kernel"] if whole else ["attn_bwd_delta_kernel", "attn_bwd_both_kernel"])
-    h = heads - 1
-    refs = O.sparse_attention_bwd_ref(*(t[:, h:h + 1].detach().float().cpu() for t in (q, k, v)), mask[:, h:h + 1].cpu(), do[:, h:h + 1].float().cpu(), scale=D ** -0.5)
-    for got, ref, name in zip(grads, refs, ("dq", "dk", "dv")):          # the bound of the test above
-        err = (got[:, h:h + 1].float().cpu() - ref).abs()
-        assert (err <= 1e-4 + 1e-2 * ref.abs().max() + 1e-2 * ref.abs()).all(), (name, float(err.max()))
-
-
 # Heads as 32nds of a round of one work-group on a CU.  Gradients are the same bits with and without a tile map, so it is the same kernel.
 @pytest.mark.parametrize("N, D, part, whole", [
     (512, 64, 16, False), (512, 64, 20, True), (385, 64, 24, True), (512, 64, 40, False), (512, 64, 48, True), (385, 64, 80, True), (512, 64, 66, False),
