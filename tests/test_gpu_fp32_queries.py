@@ -46,10 +46,10 @@ def test_same_bits_as_from_rounded_tensors(dev, heads, N, D, layout):
             assert torch.equal(a.float().nan_to_num(nan=7e37, posinf=8e37, neginf=9e37), b.float().nan_to_num(nan=7e37, posinf=8e37, neginf=9e37))
 
 
-# Inference from 2^20 elements on; training from 512 keys on, head dims beyond 32, unless every head has a boolean mask of its own.
+# Inference from 11 * 2^16 elements on; training from 2^20 and 512 keys on, head dims beyond 32, unless every head has a boolean mask of its own.
 @pytest.mark.parametrize("heads, N, D, training, masks, rounds", [
-    (64, 256, 64, False, "own", True), (64, 255, 64, False, "own", False), (256, 128, 32, False, "shared", True), (64, 64, 128, False, "packed", False),
-    (64, 512, 64, True, "shared", True), (64, 512, 64, True, "packed", True), (64, 512, 64, True, "own", False), (64, 511, 80, True, "shared", False),
+    (44, 256, 64, False, "own", True), (44, 255, 64, False, "own", False), (256, 128, 32, False, "shared", True), (64, 64, 128, False, "packed", False),
+    (64, 512, 64, True, "shared", True), (64, 512, 64, True, "packed", True), (64, 512, 64, True, "own", False), (31, 512, 64, True, "packed", False), (64, 511, 80, True, "shared", False),
     (1000, 64, 64, True, "shared", False), (512, 64, 128, True, "packed", False), (96, 577, 32, True, "shared", False), (96, 577, 80, True, "shared", True)])
 def test_which_forward_rounds_q(dev, heads, N, D, training, masks, rounds):
     importlib.import_module("python.sparse_attention")
