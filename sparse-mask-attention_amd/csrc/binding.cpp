@@ -593,9 +593,9 @@ void refuse_tangents(const Tensor &q, const Tensor &k, const Tensor &v)
 
 // Whether the forward itself rounds q of fp32 callers: q is read once and can be rounded where it is read; k and v are read once per 128 query
 // rows.  What it costs is a longer way to the first tile.  Conversion and forward, pass over all three -> this, in us (heads, N, D):
-//   inference from 0.8 million elements on gains nearly everywhere (-8 to +0.5 % of 200 grids from 2^20 on, and of 160 between): 64, 256, 64 12.5 -> 11.7;
-//             192, 512, 128 75.8 -> 69.8;  128, 1000, 32 51.0 -> 49.8.  Around 0.72 million nothing is gained on average, -1.4 % at head dim 64, +0.5 at
-//             128.  Below: 64, 128, 64 9.2 -> 9.7;  128, 128, 32 9.3 -> 9.6;  64, 64, 128 9.4 -> 10.1
+//   inference from 2^20 elements on -8 to +0.5 % (200 grids): 64, 256, 64 12.5 -> 11.7;  192, 512, 128 75.8 -> 69.8;  128, 1000, 32 51.0 -> 49.8.  0.8 to
+//             1 million: -6 to +4 %, -1 to -3 on average;  around 0.72 million -1.4 % on average at head dim 64, +0.5 at 128.  Below: 64, 128, 64
+//             9.2 -> 9.7;  128, 128, 32 9.3 -> 9.6;  64, 64, 128 9.4 -> 10.1
 //   training  (from 2^20 elements on) it also writes the rounded rows.  Long sequences hide that: 160, 768, 128 113.5 -> 108.2;  96, 512, 80 36.7 -> 34.7;
 //             200, 1024, 64 117 -> 112;  at worst 300, 512, 80 92.3 -> 94.1.  Short ones don't (512, 64, 128 24.6 -> 27.3;  200, 320, 80 43.7 -> 47.3;
 //             192, 200, 128 33.5 -> 34.2), nor does head dim 32 (300, 512 42.3 -> 43.9), and where every head has a boolean mask of its own, whose bytes
