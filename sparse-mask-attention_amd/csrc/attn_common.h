@@ -18,6 +18,10 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
+// Which way a wave-uniform branch usually goes: the usual way falls through, the other is placed out of line.
+#define LIKELY(c) __builtin_expect(c, 1)
+#define UNLIKELY(c) __builtin_expect(c, 0)
+
 #define LDS_PTR(T) __attribute__((address_space(3))) T *
 
 // First element of the (b, h) slab of a strided tensor / of the packed mask.
@@ -144,6 +148,13 @@ template <int OFF>
 __device__ __forceinline__ void async_copy_b128_at(uint32_t lds_base, const void *base, uint32_t voff) {
     asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                  :: "s"(lds_base), "v"(voff), "s"(base), "n"(OFF) : "memory", "scc", "m0");
+}
+// ... two of them, in one statement: between two statements the compiler puts a wait state of its own
+template <int OFF, int OFF2>
+__device__ __forceinline__ void async_copy2_b128_at(uint32_t lds_base, const void *base, uint32_t voff, uint32_t voff2) {
+    asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %3\n\t"
+                 "s_add_u32 m0, %0, %5\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3"
+                 :: "s"(lds_base), "v"(voff), "v"(voff2), "s"(base), "n"(OFF), "n"(OFF2) : "memory", "scc", "m0");
 }
 template <int OFF>
 __device__ __forceinline__ void async_copy_b32_at(uint32_t lds_base, const void *base, uint32_t voff) {

@@ -169,6 +169,8 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     const int N = a.N, nw = (N + 31) >> 5;
     const int T = (N + BN - 1) / BN;
     const bool ragged = (N & (BN - 1)) != 0;
+    const int cut_tile = ragged ? T - 1 : -1;                            // the tile that the keys end in
+    const int odd_tile = (nw & 1) ? T - 1 : -1;                          // the tile of which there is one word: it is read twice
     const float pm = POSTMUL ? a.post_mul : 1.0f;
 
     const int bi = (int)fastdiv((uint32_t)bh, a.div_H), hi = bh - bi * a.H;
@@ -215,7 +217,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     // instead, so that nothing after the mask's last byte is touched; the bits of the chunk that
     // holds the end are shifted to their places below, those of later chunks cleared as pad bits.
     const int mrow = BYTEMASK ? 0 : row_base + (lane >> 1);
-    const uint32_t m_voff = BYTEMASK ? 0u : (uint32_t)(((size_t)(mrow < N ? mrow : N - 1) * nw + (lane & 1)) * 4);
+    uint32_t m_voff = BYTEMASK ? 0u : (uint32_t)(((size_t)(mrow < N ? mrow : N - 1) * nw + (lane & 1)) * 4);
     uint32_t mb_voff[2] = {0u, 0u}, mb_chunk[2] = {0u, 0u};
     if constexpr (BYTEMASK) {
 #pragma unroll
@@ -230,11 +232,10 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     auto issue_mask = [&](int x, auto slot_c) __attribute__((always_inline)) {
         constexpr int SLOT = decltype(slot_c)::value;
         if constexpr (BYTEMASK) {
-            const uint8_t *src = reinterpret_cast<const uint8_t *>(mb) + (size_t)x * BN;
+            const uint8_t *src = reinterpret_cast<const uint8_t *>(mb) + (uint32_t)x * (uint32_t)BN;
             // a single slot is refilled: this wave's reads of the previous tile's bytes must be over
             if constexpr (C::BYTE_SLOTS == 1) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            uint32_t vo[2] = {mb_voff[0], mb_voff[1]};
-            if (ragged && x == T - 1) {
+            if (UNLIKELY(x == cut_tile)) {        // (no tile follows it)
                 const uint32_t row_end = (uint32_t)(N - x * BN);       // bytes of the row left in this tile
                 // the lane offsets are unsigned: what is taken from them below is first taken from the
                 // base (a tile that is not the first has 64 bytes of the row before it; in the first,
@@ -243,16 +244,15 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
                 src -= back;
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
-                    vo[j] += back;
-                    if (mb_chunk[j] + 16 > row_end) vo[j] -= mb_chunk[j] + 16 - row_end;
+                    mb_voff[j] += back;
+                    if (mb_chunk[j] + 16 > row_end) mb_voff[j] -= mb_chunk[j] + 16 - row_end;
                 }
             }
-            async_copy_b128_at<OFF_MASK + SLOT * MASK_SLOT>(mask_dst, src, vo[0]);
-            async_copy_b128_at<OFF_MASK + SLOT * MASK_SLOT + 1024>(mask_dst, src, vo[1]);
+            async_copy_b128_at<OFF_MASK + SLOT * MASK_SLOT>(mask_dst, src, mb_voff[0]);
+            async_copy_b128_at<OFF_MASK + SLOT * MASK_SLOT + 1024>(mask_dst, src, mb_voff[1]);
         } else {
-            uint32_t voff = m_voff;
-            if (2 * x + 1 >= nw) voff -= (lane & 1) * 4;           // odd word count: re-read the last word
-            async_copy_b32_at<OFF_MASK + SLOT * MASK_SLOT>(mask_dst, mb + 2 * x, voff);
+            if (UNLIKELY(x == odd_tile)) m_voff -= (lane & 1) * 4;      // the last tile: none follows it
+            async_copy_b32_at<OFF_MASK + SLOT * MASK_SLOT>(mask_dst, mb + 2u * (uint32_t)x, m_voff);
         }
     };
     // PAIRS: four copies per wave and pair of tiles; lane i of copy j fills (row 8j + i/8, position i%8)
@@ -351,7 +351,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
             // mask PyTorch itself made) need none of it: one look at the wavefront's 2 KiB decides.
             const uint32_t other = (d0.x | d0.y | d0.z | d0.w | d1.x | d1.y | d1.z | d1.w) & 0xfefefefeu;
             uint32_t mine;
-            if (__builtin_amdgcn_ballot_w64(other != 0u) == 0ull) {
+            if (LIKELY(__builtin_amdgcn_ballot_w64(other != 0u) == 0ull)) {
                 uint32_t b0 = __builtin_amdgcn_udot4(d0.x, 0x08040201u, 0u, false);
                 uint32_t b1 = __builtin_amdgcn_udot4(d0.z, 0x08040201u, 0u, false);
                 uint32_t b2 = __builtin_amdgcn_udot4(d1.x, 0x08040201u, 0u, false);
@@ -373,7 +373,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
                 // each partial value is 128 x (8 bits): bits 7..14
                 mine = (b0 >> 7) | (b1 << 1) | (b2 << 9) | (b3 << 17);
             }
-            if (x == T - 1) {
+            if (UNLIKELY(x == cut_tile)) {
                 // the chunk that holds the row's end was copied from 16 bytes before that end: its
                 // bits move down to their places (zeros follow them)
                 const int row_end = N - x * BN, part = row_end >> 4, shift = (16 - (row_end & 15)) & 15;
@@ -442,9 +442,10 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
             }
         } else {
             w = lds_read_b64(maddr + slot * MASK_SLOT);
-            const bool last = (x == T - 1);
-            w.x &= last ? a.last_mask0 : 0xffffffffu;
-            w.y &= last ? a.last_mask1 : 0xffffffffu;
+            if (UNLIKELY(x == cut_tile)) {
+                w.x &= a.last_mask0;
+                w.y &= a.last_mask1;
+            }
         }
         return w;
     };
@@ -471,9 +472,9 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     auto issue_kv = [&](int t, auto stage_c) __attribute__((always_inline)) {
         constexpr int SO = decltype(stage_c)::value * STAGE_BYTES;
         const int key0 = t * BN;
-        uint32_t ko[2] = {kv_voff[0][0], kv_voff[0][1]}, vo[2] = {kv_voff[1][0], kv_voff[1][1]};
-        uint32_t ko2[2] = {kv_voff2[0][0], kv_voff2[0][1]}, vo2[2] = {kv_voff2[1][0], kv_voff2[1][1]};
-        if (ragged && t == T - 1) {           // rows beyond N: copy row N-1 instead (zeroed later)
+        const uint16_t *ksrc = reinterpret_cast<const uint16_t *>(reinterpret_cast<const char *>(kb) + (uint32_t)key0 * k_rb);
+        const uint16_t *vsrc = reinterpret_cast<const uint16_t *>(reinterpret_cast<const char *>(vb) + (uint32_t)key0 * v_rb);
+        if (UNLIKELY(t == cut_tile)) {        // rows beyond N: copy row N-1 instead (zeroed later); no tile follows this one
             int last0 = key0;
             asm volatile("" : "+s"(last0));   // opaque: keeps this once-only arithmetic out of the loop's registers
 #pragma unroll
@@ -481,29 +482,22 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
                 const int row = 8 * (2 * wave + j) + (lane >> 3);
                 const int over = last0 + row - (N - 1);
                 if (over > 0) {
-                    ko[j] -= __umul24(over, k_rb); vo[j] -= __umul24(over, v_rb);
-                    ko2[j] -= __umul24(over, k_rb); vo2[j] -= __umul24(over, v_rb);
+                    kv_voff[0][j] -= __umul24(over, k_rb); kv_voff[1][j] -= __umul24(over, v_rb);
+                    kv_voff2[0][j] -= __umul24(over, k_rb); kv_voff2[1][j] -= __umul24(over, v_rb);
                 }
             }
         }
-        const uint16_t *ksrc = kb + (size_t)key0 * k_sn, *vsrc = vb + (size_t)key0 * v_sn;
-        async_copy_b128_at<SO>(kv_dst, ksrc, ko[0]);
-        async_copy_b128_at<SO + 1024>(kv_dst, ksrc, ko[1]);
+        async_copy2_b128_at<SO, SO + 1024>(kv_dst, ksrc, kv_voff[0][0], kv_voff[0][1]);
         if constexpr (SAME_HALVES) {          // 128 bytes further along each row
-            async_copy_b128_at<SO + TILE_BYTES>(kv_dst, ksrc + HD, ko[0]);
-            async_copy_b128_at<SO + TILE_BYTES + 1024>(kv_dst, ksrc + HD, ko[1]);
+            async_copy2_b128_at<SO + TILE_BYTES, SO + TILE_BYTES + 1024>(kv_dst, ksrc + HD, kv_voff[0][0], kv_voff[0][1]);
         } else if constexpr (NH == 2) {
-            async_copy_b128_at<SO + TILE_BYTES>(kv_dst, ksrc, ko2[0]);
-            async_copy_b128_at<SO + TILE_BYTES + 1024>(kv_dst, ksrc, ko2[1]);
+            async_copy2_b128_at<SO + TILE_BYTES, SO + TILE_BYTES + 1024>(kv_dst, ksrc, kv_voff2[0][0], kv_voff2[0][1]);
         }
-        async_copy_b128_at<SO + C::OFF_V>(kv_dst, vsrc, vo[0]);
-        async_copy_b128_at<SO + C::OFF_V + 1024>(kv_dst, vsrc, vo[1]);
+        async_copy2_b128_at<SO + C::OFF_V, SO + C::OFF_V + 1024>(kv_dst, vsrc, kv_voff[1][0], kv_voff[1][1]);
         if constexpr (SAME_HALVES) {
-            async_copy_b128_at<SO + C::OFF_V + TILE_BYTES>(kv_dst, vsrc + HD, vo[0]);
-            async_copy_b128_at<SO + C::OFF_V + TILE_BYTES + 1024>(kv_dst, vsrc + HD, vo[1]);
+            async_copy2_b128_at<SO + C::OFF_V + TILE_BYTES, SO + C::OFF_V + TILE_BYTES + 1024>(kv_dst, vsrc + HD, kv_voff[1][0], kv_voff[1][1]);
         } else if constexpr (NH == 2) {
-            async_copy_b128_at<SO + C::OFF_V + TILE_BYTES>(kv_dst, vsrc, vo2[0]);
-            async_copy_b128_at<SO + C::OFF_V + TILE_BYTES + 1024>(kv_dst, vsrc, vo2[1]);
+            async_copy2_b128_at<SO + C::OFF_V + TILE_BYTES, SO + C::OFF_V + TILE_BYTES + 1024>(kv_dst, vsrc, kv_voff2[1][0], kv_voff2[1][1]);
         }
     };
     // SPLIT: all 64 rows of one matrix by one wavefront, 16 rows (two copies) at a time; the swizzles repeat
@@ -514,7 +508,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         constexpr int AT = decltype(at_c)::value;
         const int key0 = t * BN;
         const uint16_t *src = mat + (size_t)key0 * sn;
-        const bool cut = ragged && t == T - 1;
+        const bool cut = t == cut_tile;
         auto group = [&](auto i_c) __attribute__((always_inline)) {
             constexpr int I = decltype(i_c)::value;
             uint32_t o[2] = {off[0], off[1]}, o2[2] = {off2[0], off2[1]};
@@ -638,10 +632,11 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     const int n_visits = TW == 1 ? __builtin_popcount(live_w) : T;
     // Walk over the set bits of the "live" words: `live_w` holds the bits of word `cur_w` that have
     // not been visited yet.  Words beyond the first (N > 2048) are fetched when the walk gets there.
-    int cur_w = 0;
+    int base_t = 0, cur_w = 0;
     auto next_tile = [&]() __attribute__((always_inline)) -> int {     // next live tile, T if there is none; wave-uniform
-        while (live_w == 0u) {
+        while (UNLIKELY(live_w == 0u)) {
             if (++cur_w >= TW) return T;
+            base_t = 32 * cur_w;
             uint32_t lv = 0xffffffffu, lv2 = 0u;
             if (mapw != nullptr)
                 asm volatile("s_load_dword %0, %2, 0x0\n\ts_load_dword %1, %3, 0x0\n\ts_waitcnt lgkmcnt(0)"
@@ -652,7 +647,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         }
         const int b = __builtin_ctz(live_w);
         live_w &= live_w - 1u;
-        return 32 * cur_w + b;
+        return base_t + b;
     };
     const int t_first = next_tile();
     const bool even_progress = NH == 1 && (int)blockIdx.x >= a.tail_start;   // three work-groups per CU
@@ -686,7 +681,11 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     // small LDS table for the mask: entry n (16 B) holds four floats, float j = (bit j of n) ? 0 : -inf
     if (tid < 64)
         reinterpret_cast<float *>(smem + OFF_LUT)[tid] = (((tid >> 2) >> (tid & 3)) & 1) ? 0.f : -__builtin_inff();
-    if (even_progress && n_visits >= 4) __builtin_amdgcn_s_setprio(3);
+    int yield_at = -1;                  // the visit at which this wave next lowers its priority
+    if (even_progress && n_visits >= 4) {
+        __builtin_amdgcn_s_setprio(3);
+        yield_at = n_visits / 4;
+    }
     if (SPLIT) { if (t_first < T) wait_vmcnt<8 * NH + C::MASK_COPIES>(); else wait_vmcnt<0>(); }
     else if (PAIRS) wait_vmcnt<8>();                   // q has landed; 4 mask and 4 K/V copies may still be in flight
     else if (t_first < T) wait_vmcnt<C::COPIES>();     // q has landed; the copies of the first tile may still be in flight
@@ -727,10 +726,10 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         for (int i = 0; i < 16; ++i) oacc[b][i] = 0.f;
     float ref = 0.f;                    // reference point r, in accumulator units (log2 / pm)
     float rmax = -__builtin_inff();     // largest score seen when the maximum was last taken, minus r; -inf = no kept key yet
-    bool all_seen = false;              // wave-uniform: every row of this wavefront has met a kept key
+    int all_seen = 0;                   // wave-uniform: every row of this wavefront has met a kept key
     float l_run = 0.f;                  // this lane's share of sum exp2(pm * (score - r))
     u32x4 refb = {0u, 0u, 0u, 0u};      // -r as four 16-bit terms (lane half 0 only), B operand
-    bool ref_used = false;              // false while r == 0 for every row: the extra MFMA is skipped
+    int ref_used = 0;                   // wave-uniform: 0 while r == 0 for every row: the extra MFMA is skipped
     u32x4 ones = {E::ONES, E::ONES, E::ONES, E::ONES};
     asm volatile("" : "+v"(ones));      // keep the constant operand resident in registers
 
@@ -757,7 +756,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     constexpr int KB = HALVES ? 1 : 2;            // blocks of 32 keys that a wavefront takes of a tile
     auto compute_tile_with = [&](const u32x2 both, const uint32_t so, auto after_scores, auto before_values) __attribute__((always_inline)) {
         const u32x2 w2 = HALVES ? u32x2{half ? both.y : both.x, 0u} : both;
-        if (__builtin_amdgcn_ballot_w64((w2.x | w2.y) != 0u) == 0ull) {
+        if (UNLIKELY(__builtin_amdgcn_ballot_w64((w2.x | w2.y) != 0u) == 0ull)) {
             after_scores();
             return;
         }
@@ -781,7 +780,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
                 for (int j = 0; j < 4; ++j) sacc[blk][4 * g + j] = __builtin_bit_cast(float, (uint32_t)b[j]);
             }
         }
-        if (ref_used) {               // wave-uniform: some row of this wavefront has r != 0
+        if (UNLIKELY(ref_used)) {               // wave-uniform: some row of this wavefront has r != 0
             sacc[0] = E::mfma(ones, refb, sacc[0]);
             if constexpr (!HALVES) sacc[KB - 1] = E::mfma(ones, refb, sacc[KB - 1]);
         }
@@ -812,14 +811,14 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
             const bool first = (rmax == -__builtin_inff());
             const bool move = (mxs > WINDOW_LOG2) | (first & (mxs < -WINDOW_LOG2) & (mx > -__builtin_inff()));
             const float top = __builtin_fmaxf(rmax, mx);
-            if (__builtin_amdgcn_ballot_w64(move) != 0ull) {
+            if (UNLIKELY(__builtin_amdgcn_ballot_w64(move) != 0ull)) {
                 // every row of the wavefront re-centres on its own largest score so far
                 const bool any = top > -__builtin_inff();
                 const float new_ref = set_ref(any ? ref + top : ref);
                 const float delta = ref - new_ref;                       // ~ -top
                 const float alpha = first ? 1.0f : __builtin_amdgcn_exp2f(POSTMUL ? delta * pm : delta);
                 ref = new_ref;
-                ref_used = true;
+                ref_used = 1;
                 l_run *= alpha;
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
@@ -858,16 +857,20 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         // infinity or a NaN makes a lane's sum of 32 weights exceed SUM_LIMIT, and no weight that
         // the window would have let pass (<= 2^8) can.  Only then are the maximum taken, the
         // reference moved and the exponentials redone.
-        bool with_max = false;
-        if (!all_seen) with_max = __builtin_amdgcn_ballot_w64((rmax == -__builtin_inff()) & ((w2.x | w2.y) != 0u)) != 0ull;
-        if (with_max) {
-            recentre();
-            all_seen = __builtin_amdgcn_ballot_w64(rmax == -__builtin_inff()) == 0ull;
+        int with_max = 0;
+        if (UNLIKELY(!all_seen)) {
+            if (__builtin_amdgcn_ballot_w64((rmax == -__builtin_inff()) & ((w2.x | w2.y) != 0u)) != 0ull) {
+                with_max = 1;
+                recentre();
+                all_seen = __builtin_amdgcn_readfirstlane(__builtin_amdgcn_ballot_w64(rmax == -__builtin_inff()) == 0ull ? 1 : 0);
+            }
         }
         float lsum = exponentials();
-        if (!with_max && __builtin_amdgcn_ballot_w64(!(lsum <= SUM_LIMIT)) != 0ull) {
-            recentre();
-            lsum = exponentials();
+        if (UNLIKELY(__builtin_amdgcn_ballot_w64(!(lsum <= SUM_LIMIT)) != 0ull)) {
+            if (!with_max) {
+                recentre();
+                lsum = exponentials();
+            }
         }
         l_run += lsum;
         before_values();
@@ -894,6 +897,12 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     };
 
     // ================================ main loop ================================
+    // What a visit spends beside its products and exponentials is scalar: some 60 instructions for the walk, the copies' addresses and the
+    // rare cases.  The branches say which way they go (UNLIKELY), so that the usual way falls through and what rarely runs lies behind the
+    // loop; wave-uniform flags are numbers in scalar registers, tile offsets 32 bits, and the copies of the tile that the keys end in change
+    // the lanes' offsets in place, since none follows it.  Before -> now, one binary each in turn: 192 heads, D = 64, packed, N = 2048
+    // 237.4 -> 229.5 us, N = 1024 64.4 -> 62.3, blocks with a map 38.0 -> 35.8; 8 heads, N = 3958, boolean 64.8 -> 58.7; D = 128, 128 heads,
+    // N = 4096 1063 -> 1036, causal 619 -> 595; where the mask's bytes bound it (192, N = 512) 24.2 -> 23.9.
     // The tiles visited: every tile whose "some bit set" bit is on (all of them without a map), in
     // ascending order; the prologue has requested the first.  The i-th visit uses stage and mask
     // slot i % 2; the loop is unrolled by 2 so that these are constants.
@@ -904,23 +913,32 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     // (A ring of three stages, copies two tiles ahead, measured the same to 2 % slower on every
     // workload and costs 18 KB more LDS.)
     int visits = 0;
+    // The hardware serves the oldest wave first, so of three co-resident work-groups one
+    // finishes early and the last runs alone, at a worse rate than three together.  When
+    // no other work-group waits for the slot, a wave therefore yields as it advances.
+    auto progress = [&]() __attribute__((always_inline)) {
+        if (UNLIKELY(visits == yield_at)) {
+            if (visits == n_visits / 4) {
+                __builtin_amdgcn_s_setprio(2);
+                yield_at = n_visits / 2;
+            } else if (visits == n_visits / 2) {
+                __builtin_amdgcn_s_setprio(1);
+                yield_at = (3 * n_visits) / 4;
+            } else {
+                __builtin_amdgcn_s_setprio(0);
+            }
+        }
+        ++visits;
+    };
     auto visit = [&](const int t, const int t_next, auto slot_c) __attribute__((always_inline)) {
         constexpr int SLOT = decltype(slot_c)::value;
         constexpr int SLOT2 = SLOT ^ 1;       // the stage freed by the barrier below
-        if (even_progress) {
-            // The hardware serves the oldest wave first, so of three co-resident work-groups one
-            // finishes early and the last runs alone, at a worse rate than three together.  When
-            // no other work-group waits for the slot, a wave therefore yields as it advances.
-            if (visits == n_visits / 4) __builtin_amdgcn_s_setprio(2);
-            else if (visits == n_visits / 2) __builtin_amdgcn_s_setprio(1);
-            else if (visits == (3 * n_visits) / 4) __builtin_amdgcn_s_setprio(0);
-        }
-        ++visits;
+        progress();
         wait_vmcnt<0>();          // the copies of tile t have landed
-        if (ragged && t == T - 1) zero_tail_rows(t, SLOT);
+        if (UNLIKELY(t == cut_tile)) zero_tail_rows(t, SLOT);
         __syncthreads();          // tile t landed for every wave; the stage of the previous visit is free
         const u32x2 w2 = mask_words(t, SLOT);
-        if (t_next < T) {       // K/V first: the MFMA operands are what the next visit needs first (1-2 % with a byte mask)
+        if (LIKELY(t_next < T)) {       // K/V first: the MFMA operands are what the next visit needs first (1-2 % with a byte mask)
             issue_kv(t_next, integral_constant<int, SLOT2>{});
             issue_mask(t_next, integral_constant<int, SLOT2>{});
         }
@@ -931,7 +949,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         for (int t = t_first, tn; t < T; t = tn) {
             tn = next_tile();
             wait_vmcnt<8 * NH>();     // K and the mask of tile t; its V may still be on its way
-            if (ragged && t == T - 1) zero_own_rows(t, 0);
+            if (UNLIKELY(t == cut_tile)) zero_own_rows(t, 0);
             const u32x2 w2 = mask_words(t, 0);
             compute_tile_with(w2, 0u,
                 [&]() __attribute__((always_inline)) {
@@ -943,7 +961,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
                 },
                 [&]() __attribute__((always_inline)) {
                     if (tn < T) wait_vmcnt<8 * NH + C::MASK_COPIES>(); else wait_vmcnt<0>();
-                    if (ragged && t == T - 1) zero_own_rows(t, C::OFF_V);
+                    if (UNLIKELY(t == cut_tile)) zero_own_rows(t, C::OFF_V);
                 });
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             if (tn < T) issue_own_v(tn);
@@ -956,14 +974,6 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         // a pair are always followed by exactly four younger copies when they are needed.  (The stores
         // of the by-products, when asked for, only add to the count: copies complete in the order of
         // their requests, so "at most four outstanding" still means that all older copies are in.)
-        auto progress = [&]() __attribute__((always_inline)) {
-            if (even_progress) {
-                if (visits == n_visits / 4) __builtin_amdgcn_s_setprio(2);
-                else if (visits == n_visits / 2) __builtin_amdgcn_s_setprio(1);
-                else if (visits == (3 * n_visits) / 4) __builtin_amdgcn_s_setprio(0);
-            }
-            ++visits;
-        };
         for (int t = 0; t < T; t += 2) {
             progress();
             wait_vmcnt<4>();                                  // this wave's bytes of the pair have landed
@@ -971,17 +981,17 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
             u32x2 w_odd = {0u, 0u};
             if (WHOLE || t + 1 < T) w_odd = mask_words(t + 1, 0, 1);
             wait_vmcnt<0>();                                  // K/V of tile t
-            if (!WHOLE && ragged && t == T - 1) zero_tail_rows(t, 0);
+            if (!WHOLE && UNLIKELY(t == cut_tile)) zero_tail_rows(t, 0);
             __syncthreads();
             if (WHOLE || t + 1 < T) issue_kv(t + 1, integral_constant<int, 1>{});
-            if (t + 2 < T) issue_mask_pair((t >> 1) + 1);     // the words above are in registers: the bytes may go
+            if (LIKELY(t + 2 < T)) issue_mask_pair((t >> 1) + 1);     // the words above are in registers: the bytes may go
             compute_tile(w_even, 0u);
             if (!WHOLE && t + 1 >= T) break;
             progress();
             if (t + 2 < T) wait_vmcnt<4>(); else wait_vmcnt<0>();   // K/V of tile t + 1 (the next pair's bytes may be on their way)
-            if (!WHOLE && ragged && t + 1 == T - 1) zero_tail_rows(t + 1, 1);
+            if (!WHOLE && UNLIKELY(t + 1 == cut_tile)) zero_tail_rows(t + 1, 1);
             __syncthreads();
-            if (t + 2 < T) issue_kv(t + 2, integral_constant<int, 0>{});
+            if (LIKELY(t + 2 < T)) issue_kv(t + 2, integral_constant<int, 0>{});
             compute_tile(w_odd, (uint32_t)STAGE_BYTES);
         }
     } else
