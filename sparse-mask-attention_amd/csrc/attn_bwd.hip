@@ -26,8 +26,19 @@
 //                        unrolled by the two ring stages, so every LDS address in it is a
 //                        register plus an immediate.
 //
+// Products of 16 x 16 x 32: what bounds these kernels at head dims 96 and 128 is the power the matrix cores draw, which lowers the clock, and a
+// stream of these on random operands sustains 1904 TFLOP/s at 1.89 GHz where 32 x 32 x 16 sustains 1689 at 1.69.  A lane holds two rows (dQ) or two
+// keys (dK/dV), 16 apart, and every operand that is read from LDS serves both; of lse, delta and mask words half as many reads are left.  They are short, so
+// operands are requested two or three steps (of two products) ahead and the vector work of one step lies between the products of
+// another; scheduling barriers hold that order.  The compiler's own order, each read just before its use: dK/dV 1878 -> 2090 us on 4 x 32 heads,
+// N = 4096, D = 128; with it 1657, the matrix cores busy 62 % of the cycles at 2.03 GHz (before 57 % at 1.95); dQ 1405 -> 1345 -> 1275 us.
+// The backward alone, 32 x 32 x 16 -> this, in us, random masks unless noted:
+//   192 heads, N = 1024   D = 32 128 -> 120, 64 200 -> 184 (blocks, map 101 -> 97), 96 274 -> 254, 128 353 -> 318 (blocks, map 219 -> 200)
+//   128 heads, N = 2048   D = 32 315 -> 294, 64 484 -> 440, 96 673 -> 613, 128 857 -> 780;  causal, N = 2000: 218 -> 210, 299 -> 280, 437 -> 410, 598 -> 550
+//   8 heads, N = 3000     D = 32 64.8 -> 61.5, 64 81.0 -> 75.5, 96 113 -> 98, 128 174 -> 155
+//
 // Tiles (64 rows x 64 x 16 bit) are copied global -> LDS by global_load_lds_dwordx4 into two
-// stages, one tile ahead; the 16-byte chunks of a row are XOR-swizzled with bitrev3((row >> 1) & 7),
+// stages, one tile ahead; the 16-byte chunks of a row are XOR-swizzled with swizzle16((row >> 1) & 7),
 // which keeps both the row reads (ds_read_b128) and the transposing reads (ds_read_b64_tr_b16) of
 // the same tile free of bank conflicts.
 //
@@ -35,8 +46,8 @@
 // as two 64-column tiles, the products that contract over the head dim (S, dP) run over both
 // halves, the others (dQ, dK, dV) fill one pair of accumulators per half.  Head dim 32 uses half a tile: the copies fill the upper half of
 // every LDS row with copies of the row's last 16 bytes, which are never read;
-// contractions over the head dim take two MFMA steps and the outputs have one 32-column block.  Head dim 96
-// is 128 with such a half tile as its second half: six steps, three blocks.
+// contractions over the head dim take one MFMA step and the outputs have two 16-column blocks.  Head dim 96
+// is 128 with such a half tile as its second half: three steps, six blocks.
 #include "attn_bwd_common.h"
 
 namespace sma {
@@ -62,7 +73,7 @@ template <int NH> struct Cfg {
 
 // Per-lane constants of the tile copies: wave w copies row blocks 2w and 2w+1 (8 rows each) of a
 // 64-row tile; lane i fills LDS chunk (row 8*blk + i/8, position i%8) with global chunk
-// position ^ bitrev3((row >> 1) & 7).
+// position ^ swizzle16((row >> 1) & 7).
 struct TileCopy {
     uint32_t chunk[2];      // byte offset of the lane's global chunk inside its row
     uint32_t chunk2[2];     // the same for the second column half
@@ -77,7 +88,7 @@ __device__ __forceinline__ TileCopy make_tile_copy(int wave, int lane, int last_
         const int row = 8 * (2 * wave + j) + (lane >> 3);
         const int pos = lane & 7;
         c.row[j] = row;
-        const int chunk = pos ^ bitrev3((row >> 1) & 7);
+        const int chunk = pos ^ swizzle16((row >> 1) & 7);
         c.chunk[j] = (uint32_t)(chunk < last_chunk ? chunk : last_chunk) << 4;
         c.chunk2[j] = (uint32_t)(chunk + 8 < last_chunk ? chunk + 8 : last_chunk) << 4;
     }
@@ -129,8 +140,9 @@ __device__ __forceinline__ void dq_rows(const AttnBwdArgs &a, unsigned char *sme
 {
     using E = Elem<BF16>;
     constexpr int NH = HDIM > 64 ? 2 : 1;         // 64-column tiles per matrix
-    constexpr int KS = HDIM / 16;                 // MFMA steps of a contraction over the head dim
-    constexpr int OB = HDIM / 32;                 // 32-column accumulator blocks of an output
+    constexpr int KS = HDIM / 32;                 // MFMA steps of a contraction over the head dim
+    constexpr int DB = HDIM / 16;                 // 16-column accumulator blocks of an output
+    constexpr int AHEAD = HDIM <= 64 ? 2 : 3;     // steps by which an operand is requested before its use
     using C = Cfg<NH>;
     constexpr int STAGE_BYTES = C::STAGE_BYTES, OFF_AUX = C::OFF_AUX, OFF_LUT = C::OFF_LUT;
     const uint32_t lds0 = (uint32_t)(uintptr_t)(LDS_PTR(unsigned char))smem;
@@ -138,7 +150,7 @@ __device__ __forceinline__ void dq_rows(const AttnBwdArgs &a, unsigned char *sme
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int l32 = lane & 31, hh = lane >> 5;
+    const int l16 = lane & 15, q4 = lane >> 4;
     const int N = a.N, nw = (N + 31) >> 5;
     const int T = (N + BN - 1) / BN;
     const bool ragged = (N & (BN - 1)) != 0;
@@ -149,35 +161,42 @@ __device__ __forceinline__ void dq_rows(const AttnBwdArgs &a, unsigned char *sme
     const uint16_t *qb = slab(a.q, bi, hi), *dob = slab(a.dout, bi, hi), *ob = slab(a.out, bi, hi);
     const uint32_t *mb = slab(a.mask, bi, hi);
 
-    // ---- this lane's query row: q^T and dO^T fragments (B operands), delta, lse ----
-    const int qrow = qt * BM + wave * 32 + l32;
-    const int qr = qrow < N ? qrow : N - 1;
-    u32x4 qf[KS], dof[KS], of[KS];
-    load_row(qf, qb, a.q.sn, qr, hh, a.D);
-    load_row(dof, dob, a.dout.sn, qr, hh, a.D);
-    float delta = 0.f, d4[4] = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (HAVE_DELTA) delta = a.delta[(size_t)bh * N + qr];
-    else load_row(of, ob, a.out.sn, qr, hh, a.D);
+    // ---- this lane's two query rows: q^T and dO^T fragments (B operands), delta, lse ----
+    u32x4 qf[2][KS], dof[2][KS];
+    float L[2];                         // p = exp2(pm * s - L); rows that kept nothing (lse = -inf) and rows beyond N get L = +inf
+    f32x4 from_delta[2];                // what the dP accumulators start from
 #pragma unroll
-    for (int s = 0; s < KS; ++s)
+    for (int qb_ = 0; qb_ < 2; ++qb_) {
+        const int qrow = qt * BM + wave * 32 + 16 * qb_ + l16;
+        const int qr = qrow < N ? qrow : N - 1;
+        u32x4 of[KS];
+        load_row16(qf[qb_], qb, a.q.sn, qr, q4, a.D);
+        load_row16(dof[qb_], dob, a.dout.sn, qr, q4, a.D);
+        float delta = 0.f, d2[2] = {0.f, 0.f};
+        if constexpr (HAVE_DELTA) delta = a.delta[(size_t)bh * N + qr];
+        else load_row16(of, ob, a.out.sn, qr, q4, a.D);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            if constexpr (!HAVE_DELTA) d4[s & 3] = add_products<BF16>(dof[s][i], of[s][i], d4[s & 3]);
-            const float lo = E::up1((uint16_t)(qf[s][i] & 0xffffu)) * a.q_scale;
-            const float hi = E::up1((uint16_t)(qf[s][i] >> 16)) * a.q_scale;
-            qf[s][i] = (uint32_t)E::cvt1(lo) | ((uint32_t)E::cvt1(hi) << 16);
+        for (int s = 0; s < KS; ++s)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if constexpr (!HAVE_DELTA) d2[s & 1] = add_products<BF16>(dof[qb_][s][i], of[s][i], d2[s & 1]);
+                const float lo = E::up1((uint16_t)(qf[qb_][s][i] & 0xffffu)) * a.q_scale;
+                const float hi = E::up1((uint16_t)(qf[qb_][s][i] >> 16)) * a.q_scale;
+                qf[qb_][s][i] = (uint32_t)E::cvt1(lo) | ((uint32_t)E::cvt1(hi) << 16);
+            }
+        if constexpr (!HAVE_DELTA) {
+            delta = xhalf_sum(xrow_sum(d2[0])) + xhalf_sum(xrow_sum(d2[1]));
+            if (qrow < N && q4 == 0) a.delta[(size_t)bh * N + qrow] = delta;
         }
-    if constexpr (!HAVE_DELTA) {
-        delta = (xhalf_sum(d4[0]) + xhalf_sum(d4[1])) + (xhalf_sum(d4[2]) + xhalf_sum(d4[3]));
-        if (qrow < N && hh == 0) a.delta[(size_t)bh * N + qrow] = delta;
+        const float lse_row = a.lse[(size_t)bh * N + qr];
+        L[qb_] = (qrow >= N || lse_row == -__builtin_inff()) ? __builtin_inff() : lse_row * LOG2E;
+        from_delta[qb_] = f32x4{-delta, -delta, -delta, -delta};
     }
-    const float lse_row = a.lse[(size_t)bh * N + qr];
-    // p = exp2(pm * s - L); rows that kept nothing (lse = -inf) and rows beyond N get L = +inf
-    const float L = (qrow >= N || lse_row == -__builtin_inff()) ? __builtin_inff() : lse_row * LOG2E;
+    // kept, the first MFMAs of a tile read them in place
+    asm volatile("" : "+v"(from_delta[0]), "+v"(from_delta[1]));
 
     // ---- copies ----
     const TileCopy tc = make_tile_copy(wave, lane, (a.D >> 3) - 1);
-    const TileRead tr = make_tile_read(lane);
     const int mrow = qt * BM + wave * 32 + (lane >> 1);
     const uint32_t m_voff = (uint32_t)(((size_t)(mrow < N ? mrow : N - 1) * nw + (lane & 1)) * 4);
     auto issue = [&](int t, int st) {
@@ -215,21 +234,17 @@ __device__ __forceinline__ void dq_rows(const AttnBwdArgs &a, unsigned char *sme
     if (tid < 64)
         reinterpret_cast<float *>(smem + OFF_LUT)[tid] = (((tid >> 2) >> (tid & 3)) & 1) ? 0.f : -__builtin_inff();
 
-    f32x16 oacc[OB];                    // [2 * half + dblk]: 32 columns of dQ each
+    f32x4 oacc[2][DB];                  // 16 columns of dQ of 16 rows each
 #pragma unroll
-    for (int b = 0; b < OB; ++b)
+    for (int x = 0; x < 2; ++x)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) oacc[b][i] = 0.f;
+        for (int b = 0; b < DB; ++b) oacc[x][b] = f32x4{0.f, 0.f, 0.f, 0.f};
     const uint32_t lut_addr = lds0 + OFF_LUT;
-    const uint32_t nib_shift = 4u - 4u * hh;
-    f32x16 from_delta;                  // what the dP accumulators start from; kept, the first MFMA of a tile reads it in place
-#pragma unroll
-    for (int i = 0; i < 16; ++i) from_delta[i] = -delta;
-    asm volatile("" : "+v"(from_delta));
+    const uint32_t nib_rotate = (4u * q4 + 28u) & 31u;     // right: the nibble of keys 4q4 .. 4q4 + 3 comes to bits 4 .. 7
 
-    // one key tile; the ring stage is a compile-time constant, as in the dK/dV kernel: 22 address sums per tile less.
-    // With dP's accumulators started from -delta (no subtraction per element) 1466 -> 1412 us on 4 x 32 heads, N = 4096,
-    // D = 128, 1.17 PFLOP/s, where the clock is down to 1.8 GHz under the matrix cores' load
+    uint32_t row_at = make_tile_read16(lane).row, col_at = make_tile_read16(lane).col;
+    // one key tile; the ring stage is a compile-time constant, as in the dK/dV kernel, so that every LDS address is a register plus an
+    // immediate.  4 x 32 heads, N = 4096, D = 128: 1275 us, 1.29 PFLOP/s, the matrix cores busy two thirds of the time at 1.86 GHz
     auto tile = [&](int t, int t_next, auto st_c) __attribute__((always_inline)) {
         constexpr int st = decltype(st_c)::value;
         const uint32_t so = lds0 + st * STAGE_BYTES;
@@ -238,55 +253,97 @@ __device__ __forceinline__ void dq_rows(const AttnBwdArgs &a, unsigned char *sme
         __syncthreads();          // tile t of every wave landed; the other stage is free
         if (t_next < T) issue(t_next, st ^ 1);
 
-        u32x2 w2 = lds_read_b64(lds0 + OFF_AUX + st * AUX_BYTES + wave * 256 + l32 * 8);
-        if (t == T - 1) { w2.x &= a.last_mask0; w2.y &= a.last_mask1; }
-        if (__builtin_amdgcn_ballot_w64((w2.x | w2.y) != 0u) == 0ull) return;
+        // Steps of two products each: S^T of 32 keys (mask bias as initial value), dP^T of them, then the same of the other 32, then dQ^T += K^T dS^T.
+        // Element j of [kb][x] <-> key 32blk + 16kb + 4q4 + j, row 16x + l16.
+        asm volatile("" : "+v"(row_at), "+v"(col_at));       // or the compiler keeps a register for every address that follows from these
+        auto k_row = [&](int blk, int n) __attribute__((always_inline)) {        // step n: key block n & 1, columns 32 (n >> 1)
+            return lds_read_b128((row_at ^ (64 * ((n >> 1) & 1))) + so + (n >> 2) * TILE_BYTES + 4096 * blk + 2048 * (n & 1));
+        };
+        auto v_row = [&](int blk, int n) __attribute__((always_inline)) {
+            return lds_read_b128((row_at ^ (64 * ((n >> 1) & 1))) + so + C::OFF_B + (n >> 2) * TILE_BYTES + 4096 * blk + 2048 * (n & 1));
+        };
+        auto k_col = [&](int blk, int b) __attribute__((always_inline)) {
+            const uint32_t ko = (col_at ^ (32 * (b & 3))) + so + (b >> 2) * TILE_BYTES + 4096 * blk;
+            const u32x2 lo = lds_read_tr16_b64(ko), hi = lds_read_tr16_b64(ko + 2048);
+            return u32x4{lo.x, lo.y, hi.x, hi.y};
+        };
+        // The operands of a step are requested AHEAD steps before it, and scheduling barriers hold that order: left alone, the compiler
+        // requests each just before its use.
+        constexpr int PH = 2 * KS;                    // steps of a phase
+        u32x4 ring[AHEAD + 1];
+        auto fetch = [&](int n) __attribute__((always_inline)) {
+            u32x4 &r = ring[n % (AHEAD + 1)];
+            if (n < PH) r = k_row(0, n);
+            else if (n < 2 * PH) r = v_row(0, n - PH);
+            else if (n < 3 * PH) r = k_row(1, n - 2 * PH);
+            else if (n < 4 * PH) r = v_row(1, n - 3 * PH);
+            else if (n < 4 * PH + DB) r = k_col(0, n - 4 * PH);
+            else if (n < 4 * PH + 2 * DB) r = k_col(1, n - 4 * PH - DB);
+        };
+        u32x2 w2[2];
+#pragma unroll
+        for (int x = 0; x < 2; ++x) w2[x] = lds_read_b64(lds0 + OFF_AUX + st * AUX_BYTES + wave * 256 + 128 * x + l16 * 8);
+#pragma unroll
+        for (int n = 0; n < AHEAD; ++n) fetch(n);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+            if (t == T - 1) { w2[x].x &= a.last_mask0; w2[x].y &= a.last_mask1; }
+        if (__builtin_amdgcn_ballot_w64((w2[0].x | w2[0].y | w2[1].x | w2[1].y) != 0u) == 0ull) return;
 
-        // Per block of 32 keys: S^T (mask bias as initial value) and dP^T, element [4g+j] <-> key
-        // 32blk + 8g + 4hh + j, then dS^T / scale = P^T o (dP^T - delta), packed as B operands.
-        uint32_t pb[2][2][4];
+        u32x4 pb[2][2];
+        f32x4 sacc[2][2][2], dacc[2][2][2];           // [blk]: a block's registers are free again when its dS is packed
+        auto bias = [&](int blk) __attribute__((always_inline)) {
 #pragma unroll
-        for (int blk = 0; blk < 2; ++blk) {
-            f32x16 sacc, dacc = from_delta;
-            const uint32_t wa = (blk == 0 ? w2.x : w2.y) << nib_shift;
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const u32x4 b = lds_read_b128(lut_addr + ((wa >> (8 * g)) & 0xF0u));
-#pragma unroll
-                for (int j = 0; j < 4; ++j) sacc[4 * g + j] = __builtin_bit_cast(float, (uint32_t)b[j]);
+            for (int x = 0; x < 2; ++x) {
+                const uint32_t w = blk == 0 ? w2[x].x : w2[x].y;
+                const uint32_t wa = __builtin_amdgcn_alignbit(w, w, nib_rotate);
+                sacc[blk][0][x] = __builtin_bit_cast(f32x4, lds_read_b128(lut_addr + (wa & 0xF0u)));
+                sacc[blk][1][x] = __builtin_bit_cast(f32x4, lds_read_b128(lut_addr + ((wa >> 16) & 0xF0u)));
             }
+        };
+        auto weight = [&](int blk, int e) __attribute__((always_inline)) {       // element e of 16
+            const int kb = e >> 3, x = (e >> 2) & 1, j = e & 3;
+            sacc[blk][kb][x][j] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[blk][kb][x][j], pm, -L[x]));
+        };
+        auto dscore = [&](int blk, int i) __attribute__((always_inline)) {       // dS^T / scale = P^T o (dP^T - delta), pair i of 8, packed as B operand
+            const int kb = i >> 2, x = (i >> 1) & 1, j = 2 * (i & 1);
+            pb[blk][x][2 * kb + (i & 1)] = E::pack2_rne(sacc[blk][kb][x][j] * dacc[blk][kb][x][j], sacc[blk][kb][x][j + 1] * dacc[blk][kb][x][j + 1]);
+        };
+        bias(0);
 #pragma unroll
-            for (int s = 0; s < KS; ++s) {
-                const uint32_t ra = tr.rowaddr[s & 3] + so + (s >> 2) * TILE_BYTES + 4096 * blk;
-                sacc = E::mfma(lds_read_b128(ra), qf[s], sacc);
-                dacc = E::mfma(lds_read_b128(ra + C::OFF_B), dof[s], dacc);
-            }
+        for (int n = 0; n < 4 * PH + 2 * DB; ++n) {
+            fetch(n + AHEAD);
+            if (n == 2 * PH - 2) bias(1);
+            __builtin_amdgcn_sched_barrier(0);
+            const u32x4 &r = ring[n % (AHEAD + 1)];
+            const int ph = n / PH, m = n % PH, blk = ph >> 1, kb = m & 1, c = m >> 1;
+            if (n >= 4 * PH) {
+                const int k = n - 4 * PH, b = k % DB;
 #pragma unroll
-            for (int u = 0; u < 2; ++u)
+                for (int x = 0; x < 2; ++x) oacc[x][b] = E::mfma16(r, pb[k / DB][x], oacc[x][b]);
+                if (k < DB) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int e = 8 * u + 2 * i;
-                    const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[e], pm, -L));
-                    const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[e + 1], pm, -L));
-                    pb[blk][u][i] = E::pack2_rne(p0 * dacc[e], p1 * dacc[e + 1]);
+                    for (int i = 0; i < (8 + DB - 1) / DB; ++i)
+                        if (k * ((8 + DB - 1) / DB) + i < 8) dscore(1, k * ((8 + DB - 1) / DB) + i);
                 }
+            } else if (ph == 0 || ph == 2) {
+#pragma unroll
+                for (int x = 0; x < 2; ++x) sacc[blk][kb][x] = E::mfma16(r, qf[x][c], sacc[blk][kb][x]);
+                if (ph == 2) {
+#pragma unroll
+                    for (int i = 0; i < (8 + PH - 1) / PH; ++i)
+                        if (m * ((8 + PH - 1) / PH) + i < 8) dscore(0, m * ((8 + PH - 1) / PH) + i);
+                }
+            } else {
+#pragma unroll
+                for (int x = 0; x < 2; ++x) dacc[blk][kb][x] = E::mfma16(r, dof[x][c], c == 0 ? from_delta[x] : dacc[blk][kb][x]);
+#pragma unroll
+                for (int i = 0; i < (16 + PH - 1) / PH; ++i)
+                    if (m * ((16 + PH - 1) / PH) + i < 16) weight(blk, m * ((16 + PH - 1) / PH) + i);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        // dQ^T += K^T dS^T
-#pragma unroll
-        for (int blk = 0; blk < 2; ++blk)
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const u32x4 pv = {pb[blk][u][0], pb[blk][u][1], pb[blk][u][2], pb[blk][u][3]};
-                const uint32_t off = so + 4096 * blk + 2048 * u;
-#pragma unroll
-                for (int b = 0; b < OB; ++b) {
-                    const uint32_t ko = off + (b >> 1) * TILE_BYTES;
-                    const u32x2 lo = lds_read_tr16_b64(tr.traddr[b & 1][0] + ko);
-                    const u32x2 hi = lds_read_tr16_b64(tr.traddr[b & 1][1] + ko);
-                    const u32x4 va = {lo.x, lo.y, hi.x, hi.y};
-                    oacc[b] = E::mfma(va, pv, oacc[b]);
-                }
-            }
     };
     for (int t = t_first; t < T;) {
         const int tn = next_tile();
@@ -299,7 +356,7 @@ __device__ __forceinline__ void dq_rows(const AttnBwdArgs &a, unsigned char *sme
     __syncthreads();              // every wave is done reading the stages
     const int row0 = qt * BM + wave * 32;
     if (row0 < N) {
-        store_gradient<BF16, WIDE>(oacc, a.scale, lds0 + wave * 4096, a, a.dq, bi, hi, row0, lane);
+        store_gradient16<BF16, WIDE>(oacc, a.scale, lds0 + wave * 4096, a, a.dq, bi, hi, row0, lane);
     }
 }
 
@@ -316,10 +373,9 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_bwd_dq_kerne
 // dK and dV
 // ------------------------------------------------------------------------------------------------
 // NW wavefronts of 32 keys each.  The K fragments of a wavefront's keys stay in registers, and the V fragments where they
-// fit.  VLDS: they wait in LDS, 16 bytes per lane and fragment in the order the lanes read them, and the mask words are
-// read twice instead of kept.
+// fit.  VLDS: they wait in LDS, 16 bytes per lane and fragment in the order the lanes read them.
 //   128  the accumulators of dK and dV take 128 registers; both gradients in one kernel form S once where a kernel
-//        for each formed it twice: 2783 -> 2032 us on 4 x 32 heads, N = 4096 (1.08 PFLOP/s over four products)
+//        for each formed it twice: 2783 -> 2032 us on 4 x 32 heads, N = 4096 (now 1657, 1.33 PFLOP/s over four products)
 //   64   166 registers instead of 198: three work-groups on a CU instead of two, where the grid has them (see the
 //        launcher): 16 x 12 heads, N = 512, this kernel alone on warm inputs: 41.0 -> 37.3 us (691 TFLOP/s)
 template <int HDIM, int NW, bool VLDS> struct DkvCfg {
@@ -337,8 +393,9 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
 {
     using E = Elem<BF16>;
     constexpr int NH = HDIM > 64 ? 2 : 1;
-    constexpr int KS = HDIM / 16;
-    constexpr int OB = HDIM / 32;
+    constexpr int KS = HDIM / 32;
+    constexpr int DB = HDIM / 16;
+    constexpr int AHEAD = VLDS || HDIM == 32 ? 2 : 3;             // one more where there are registers for it
     using C = DkvCfg<HDIM, NW, VLDS>;
     constexpr int STAGE_BYTES = C::STAGE_BYTES, OFF_AUX = C::OFF_AUX, AUX_BYTES = C::AUX;
     constexpr int OFF_LSE = NW * 256, OFF_DELTA = OFF_LSE + 256;       // inside the small data of a stage
@@ -347,7 +404,7 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int l32 = lane & 31, hh = lane >> 5;
+    const int l16 = lane & 15, q4 = lane >> 4;
     const int N = a.N, nw = (N + 31) >> 5;
     const int T = (N + BN - 1) / BN;
     const bool ragged = (N & (BN - 1)) != 0;
@@ -356,11 +413,11 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
 
     const int bi = (int)fastdiv((uint32_t)bh, a.div_H), hi = bh - bi * a.H;
     const uint16_t *qb = slab(a.q, bi, hi), *dob = slab(a.dout, bi, hi);
-    const uint16_t *kb = slab(a.k, bi, hi), *vb = slab(a.v, bi, hi);
+    const uint16_t *kb_ = slab(a.k, bi, hi), *vb = slab(a.v, bi, hi);
     const uint32_t *mb = slab(a.mask, bi, hi);
     const float *lse_b = a.lse + (size_t)bh * N, *delta_b = a.delta + (size_t)bh * N;
 
-    // ---- this lane's key: K^T (scaled) and V^T fragments, B operands ----
+    // ---- this lane's two keys: K^T (scaled) and V^T fragments, B operands ----
     // HALVES: a work-group of half the keys, in which the wavefronts of either half take 32 rows of every tile and their sums are added at the
     // end.  One CU holds one work-group of eight wavefronts, so a grid just beyond a round took two: its last heads, where work-groups of 128 keys
     // hold them all at once, come in such ones, each three quarters as long as a whole one.  The backward alone, before -> now, in us:
@@ -368,33 +425,31 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
     //   causal: 489 -> 421;  forward + backward, 40, N = 2048, one mask in blocks: 276 -> 248.  Of 70 grids of 17 to 96 heads, random, causal and causal
     //   with a map, one lost: 24 heads, N = 3000, causal without a map, whose short work-groups fill the second round by themselves: 271 -> 286 (with a
     //   map 254 either way, random 514 -> 462).
-    static_assert(!HALVES || (NW == 8 && VLDS && OB * 2 * 4096 * 4 <= C::LDS_BYTES), "four wavefronts' sums fit the LDS");
+    static_assert(!HALVES || (NW == 8 && VLDS && DB * 4096 * 4 <= C::LDS_BYTES), "four wavefronts' sums fit the LDS");
     constexpr int KW = HALVES ? 4 : NW;               // wavefronts side by side on different keys
     const int half = HALVES ? wave >> 2 : 0;          // ... and which 32 rows of every tile this one takes
     const int key0 = kt * (32 * KW) + (HALVES ? wave & 3 : wave) * 32;
     const bool wave_valid = key0 < N;                 // wave-uniform: some key of this wave exists
-    const int key = key0 + l32;
-    const int kr = key < N ? key : N - 1;
-    const uint32_t key_ok = key < N ? 0xffffffffu : 0u;
-    const uint32_t key_w = key < N ? 1u : 0u;         // width of the bit field that holds this key's mask bit
     const uint32_t wave_keys = N - key0 >= 32 ? 0xffffffffu : N > key0 ? (1u << (N - key0)) - 1u : 0u;      // of them the existing ones
     const int wi = (key0 >> 5) < nw ? (key0 >> 5) : nw - 1;     // this wave's mask word of a row
     const uint32_t frag = lds0 + C::OFF_FRAG + wave * C::FRAG + lane * 16;
-    u32x4 kf[KS], vf[VLDS ? 1 : KS];
-    {
+    u32x4 kf[2][KS], vf[2][VLDS ? 1 : KS];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+        const int key = key0 + 16 * kb + l16;         // a key beyond N has sums that are not stored
         u32x4 v_all[KS];
-        load_row(kf, kb, a.k.sn, kr, hh, a.D);
-        load_row(v_all, vb, a.v.sn, kr, hh, a.D);
+        load_row16(kf[kb], kb_, a.k.sn, key < N ? key : N - 1, q4, a.D);
+        load_row16(v_all, vb, a.v.sn, key < N ? key : N - 1, q4, a.D);
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const float lo = E::up1((uint16_t)(kf[s][i] & 0xffffu)) * a.q_scale;
-                const float hi = E::up1((uint16_t)(kf[s][i] >> 16)) * a.q_scale;
-                kf[s][i] = (uint32_t)E::cvt1(lo) | ((uint32_t)E::cvt1(hi) << 16);
+                const float lo = E::up1((uint16_t)(kf[kb][s][i] & 0xffffu)) * a.q_scale;
+                const float hi = E::up1((uint16_t)(kf[kb][s][i] >> 16)) * a.q_scale;
+                kf[kb][s][i] = (uint32_t)E::cvt1(lo) | ((uint32_t)E::cvt1(hi) << 16);
             }
-            if constexpr (VLDS) *(LDS_PTR(u32x4))(uintptr_t)(frag + s * 1024) = v_all[s];
-            else vf[VLDS ? 0 : s] = v_all[s];
+            if constexpr (VLDS) *(LDS_PTR(u32x4))(uintptr_t)(frag + (kb * KS + s) * 1024) = v_all[s];
+            else vf[kb][VLDS ? 0 : s] = v_all[s];
         }
     }
 
@@ -402,14 +457,6 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
     // (eight wavefronts: the first four copy Q, the others dO)
     const int cw = wave & 3;
     const TileCopy tc = make_tile_copy(cw, lane, (a.D >> 3) - 1);
-    TileRead tr = make_tile_read(lane);
-    if constexpr (HALVES) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            tr.rowaddr[i] += 4096 * half;
-            tr.traddr[i >> 1][i & 1] += 4096 * half;
-        }
-    }
     auto issue = [&](int t, int st) {
         const int r0 = t * BN;
         const int row = r0 + lane < N ? r0 + lane : N - 1;
@@ -444,23 +491,21 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
     const int t_first = next_tile();
     if (t_first < T) issue(t_first, 0);
 
-    f32x16 dkacc[OB], dvacc[OB];      // [2 * half + dblk]: 32 columns each
+    f32x4 dkacc[2][DB], dvacc[2][DB];     // 16 columns of 16 keys each
 #pragma unroll
-    for (int b = 0; b < OB; ++b)
+    for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            dkacc[b][i] = 0.f;
-            dvacc[b][i] = 0.f;
-        }
+        for (int b = 0; b < DB; ++b) dkacc[kb][b] = dvacc[kb][b] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     // bases of this lane's reads of the small data; opaque, because beyond 64 KiB the compiler would otherwise
     // keep a register for every sum of base and offset (40 of them) instead of using the offset field, and at 64
     // three work-groups on a CU leave no register to spare
-    uint32_t aux_rows = lds0 + OFF_AUX + 16 * hh, aux_words = aux_rows + wave * 256, aux_lane = lds0 + OFF_AUX + 4 * lane;
+    uint32_t aux_rows = lds0 + OFF_AUX + 16 * q4, aux_words = aux_rows + wave * 256, aux_lane = lds0 + OFF_AUX + 4 * lane;
     aux_rows += 128 * half;
     aux_words += 128 * half;
     if constexpr (VLDS || OFF_AUX >= 65536) asm volatile("" : "+v"(aux_rows), "+v"(aux_words), "+v"(aux_lane));
 
+    uint32_t row_at = make_tile_read16(lane).row + 4096 * half, col_at = make_tile_read16(lane).col + 4096 * half;
     // one q tile; the ring stage is a compile-time constant so that every LDS address of the body is
     // a register plus an immediate
     auto tile = [&](int t, int t_next, auto st_c) __attribute__((always_inline)) {
@@ -489,91 +534,102 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
         if (t_next < T) issue(t_next, st ^ 1);
         if (!wave_valid) return;
 
-        // VLDS: which rows keep any of this wavefront's keys, by one word a lane: the four 16-byte reads of the words themselves, of a
-        // kernel whose LDS is nearly always busy, then come once and not twice, and not at all where nothing is kept.  The backward alone: 192 heads, N = 1024,
-        // D = 64 215.0 -> 210.3 us; 4 x 32, N = 4096, D = 128 3397 -> 3366; in one launch with dQ and by a map, a random
-        // mask, forward + backward, 32 heads, N = 4096 675 -> 646.
-        unsigned long long live_rows = ~0ull;
-        if constexpr (VLDS) {
-            const uint32_t w = *(LDS_PTR(const uint32_t))(uintptr_t)(aux_lane + wave * 256 + st * AUX_BYTES);
-            live_rows = __builtin_amdgcn_ballot_w64((w & wave_keys) != 0u) >> (32 * half);
-        }
+        // which rows keep any of this wavefront's keys, by one word a lane
+        const uint32_t w = *(LDS_PTR(const uint32_t))(uintptr_t)(aux_lane + wave * 256 + st * AUX_BYTES);
+        const unsigned long long live_rows = __builtin_amdgcn_ballot_w64((w & wave_keys) != 0u) >> (32 * half);
 #pragma unroll
         for (int blk = 0; blk < (HALVES ? 1 : 2); ++blk) {
-            // element 4g+j of an accumulator <-> query row 32blk + 8g + 4hh + j of the tile
-            auto mask_words = [&](int g) __attribute__((always_inline)) { return lds_read_b128(aux_words + st * AUX_BYTES + 128 * blk + 32 * g); };
-            u32x4 mw[4];
-            if constexpr (VLDS) {
-                if ((uint32_t)(live_rows >> (32 * blk)) == 0u) continue;
-            } else {
-                uint32_t any = 0u;
+            if ((uint32_t)(live_rows >> (32 * blk)) == 0u) continue;
+            asm volatile("" : "+v"(row_at), "+v"(col_at));
+            // Element j of [rb][kb] <-> query row 32blk + 16rb + 4q4 + j of the tile, key 16kb + l16.
+            // Steps of two products each: S (PH of them), dP (as many), dV (DB), dK (DB).  The operands of a step are requested AHEAD steps
+            // before it, and scheduling barriers hold that order: left alone, the compiler requests each just before its use.  The exponentials
+            // go beside dP's products, dS is formed beside dV's.
+            constexpr int PH = 2 * KS;
+            auto row = [&](int n) __attribute__((always_inline)) -> uint32_t {           // row block n & 1, columns 32 (n >> 1)
+                return (row_at ^ (64 * ((n >> 1) & 1))) + so + (n >> 2) * TILE_BYTES + 4096 * blk + 2048 * (n & 1);
+            };
+            auto col = [&](int b, int off) __attribute__((always_inline)) {
+                const uint32_t at = (col_at ^ (32 * (b & 3))) + so + off + (b >> 2) * TILE_BYTES + 4096 * blk;
+                const u32x2 lo = lds_read_tr16_b64(at), hi = lds_read_tr16_b64(at + 2048);
+                return u32x4{lo.x, lo.y, hi.x, hi.y};
+            };
+            auto rows_data = [&](int off, int rb) __attribute__((always_inline)) {
+                return __builtin_bit_cast(f32x4, lds_read_b128(aux_rows + st * AUX_BYTES + off + 128 * blk + 64 * rb));
+            };
+            auto mask_words = [&](int rb) __attribute__((always_inline)) { return lds_read_b128(aux_words + st * AUX_BYTES + 128 * blk + 64 * rb); };
+            u32x4 ring[AHEAD + 1], vs[2][2], mw[2], pp[2], ps[2];
+            auto fetch = [&](int n) __attribute__((always_inline)) {
+                u32x4 &r = ring[n % (AHEAD + 1)];
+                if (n < PH) r = lds_read_b128(row(n));
+                else if (n < 2 * PH) r = lds_read_b128(row(n - PH) + C::OFF_B);
+                else if (n < 2 * PH + DB) r = col(n - 2 * PH, C::OFF_B);
+                else if (n < 2 * PH + 2 * DB) r = col(n - 2 * PH - DB, 0);
+            };
+            auto fetch_v = [&](int c) __attribute__((always_inline)) {
 #pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    mw[g] = mask_words(g);
-                    any |= mw[g].x | mw[g].y | mw[g].z | mw[g].w;
+                for (int kb = 0; kb < 2; ++kb) vs[c & 1][kb] = VLDS ? lds_read_b128(frag + (kb * KS + c) * 1024) : vf[kb][VLDS ? 0 : c];
+            };
+            // the accumulators start from the rows' -lse (scaled) and -delta (the same for both blocks of keys): the products then leave
+            // s - lse and dP - delta, with no subtraction per element
+            f32x4 sacc[2][2], dacc[2][2];
+#pragma unroll
+            for (int rb = 0; rb < 2; ++rb) sacc[rb][0] = sacc[rb][1] = rows_data(OFF_LSE, rb);
+#pragma unroll
+            for (int n = 0; n < AHEAD; ++n) fetch(n);
+#pragma unroll
+            for (int n = 0; n < 2 * PH + 2 * DB; ++n) {
+                fetch(n + AHEAD);
+                const int m = n % PH, rb = m & 1, c = m >> 1;
+                if (n == PH - 2) {
+                    fetch_v(0);
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) dacc[i][0] = dacc[i][1] = rows_data(OFF_DELTA, i);
                 }
-                if (__builtin_amdgcn_ballot_w64((((any >> l32) & 1u) & key_ok) != 0u) == 0ull) continue;
-            }
-
-            // the accumulators start from the rows' -lse (scaled) and -delta, read straight into them:
-            // the products then leave s - lse and dP - delta, with no subtraction per element
-            f32x16 sacc, dacc;
+                if (n == PH - 1) mw[0] = mask_words(0);
+                if (n == PH + PH / 2 - 1) mw[1] = mask_words(1);
+                if (n >= PH && n < 2 * PH && rb == 0 && c + 1 < KS) fetch_v(c + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                const u32x4 &r = ring[n % (AHEAD + 1)];
+                if (n < PH) {
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const u32x4 Lr = lds_read_b128(aux_rows + st * AUX_BYTES + OFF_LSE + 128 * blk + 32 * g);
-                const u32x4 Dr = lds_read_b128(aux_rows + st * AUX_BYTES + OFF_DELTA + 128 * blk + 32 * g);
+                    for (int kb = 0; kb < 2; ++kb) sacc[rb][kb] = E::mfma16(r, kf[kb][c], sacc[rb][kb]);
+                } else if (n < 2 * PH) {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    sacc[4 * g + j] = __builtin_bit_cast(float, (uint32_t)Lr[j]);
-                    dacc[4 * g + j] = __builtin_bit_cast(float, (uint32_t)Dr[j]);
+                    for (int kb = 0; kb < 2; ++kb) dacc[rb][kb] = E::mfma16(r, vs[c & 1][kb], dacc[rb][kb]);
+#pragma unroll
+                    for (int i = 0; i < (16 + PH - 1) / PH; ++i) {
+                        const int e = m * ((16 + PH - 1) / PH) + i, er = e >> 3, ek = (e >> 2) & 1, j = e & 3;
+                        if (e < 16) {
+                            const uint32_t keep = (uint32_t)__builtin_amdgcn_sbfe((int)mw[er][j], (uint32_t)(l16 + 16 * ek), 1u);
+                            const float x = __builtin_amdgcn_exp2f(POSTMUL ? sacc[er][ek][j] * pm : sacc[er][ek][j]);
+                            float p = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & keep);
+                            asm volatile("" : "+v"(p));              // here: the compiler would keep both operands of all 16 for the first use
+                            sacc[er][ek][j] = p;
+                        }
+                    }
+                    if (n == 2 * PH - 1) {
+#pragma unroll
+                        for (int i = 0; i < 8; ++i)
+                            pp[(i >> 1) & 1][2 * (i >> 2) + (i & 1)] =
+                                E::pack2_rne(sacc[i >> 2][(i >> 1) & 1][2 * (i & 1)], sacc[i >> 2][(i >> 1) & 1][2 * (i & 1) + 1]);
+                    }
+                } else if (n < 2 * PH + DB) {          // dV^T += dO^T P
+                    const int b = n - 2 * PH;
+#pragma unroll
+                    for (int kb = 0; kb < 2; ++kb) dvacc[kb][b] = E::mfma16(r, pp[kb], dvacc[kb][b]);
+#pragma unroll
+                    for (int q = 0; q < (8 + DB - 1) / DB; ++q) {
+                        const int i = b * ((8 + DB - 1) / DB) + q, ir = i >> 2, ik = (i >> 1) & 1, j = 2 * (i & 1);
+                        if (i < 8)
+                            ps[ik][2 * ir + (i & 1)] = E::pack2_rne(sacc[ir][ik][j] * dacc[ir][ik][j], sacc[ir][ik][j + 1] * dacc[ir][ik][j + 1]);
+                    }
+                } else {                               // dK^T += Q^T dS
+                    const int b = n - 2 * PH - DB;
+#pragma unroll
+                    for (int kb = 0; kb < 2; ++kb) dkacc[kb][b] = E::mfma16(r, ps[kb], dkacc[kb][b]);
                 }
-            }
-#pragma unroll
-            for (int s = 0; s < KS; ++s)
-                sacc = E::mfma(lds_read_b128(tr.rowaddr[s & 3] + so + (s >> 2) * TILE_BYTES + 4096 * blk), kf[s], sacc);
-#pragma unroll
-            for (int s = 0; s < KS; ++s) {
-                const u32x4 vs = VLDS ? lds_read_b128(frag + s * 1024) : vf[VLDS ? 0 : s];
-                dacc = E::mfma(lds_read_b128(tr.rowaddr[s & 3] + so + C::OFF_B + (s >> 2) * TILE_BYTES + 4096 * blk), vs, dacc);
-            }
-
-            uint32_t pp[2][4], ps[2][4];
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                // (one wait for the words less far ahead, or four registers more than there are: each reload in this loop waits for the copies)
-                if constexpr (HALVES && POSTMUL) if (g == 1) __builtin_amdgcn_sched_barrier(0);
-                float p[4], d[4];
-                const u32x4 mg = VLDS ? mask_words(g) : mw[g];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t keep = (uint32_t)__builtin_amdgcn_sbfe((int)mg[j], (uint32_t)l32, key_w);
-                    const float e = __builtin_amdgcn_exp2f(POSTMUL ? sacc[4 * g + j] * pm : sacc[4 * g + j]);
-                    p[j] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, e) & keep);
-                    d[j] = p[j] * dacc[4 * g + j];
-                }
-                // elements 4g .. 4g+3 are pairs (2i, 2i+1) with i = 2(g & 1), 2(g & 1) + 1 of u = g >> 1
-                pp[g >> 1][2 * (g & 1)] = E::pack2_rne(p[0], p[1]);
-                pp[g >> 1][2 * (g & 1) + 1] = E::pack2_rne(p[2], p[3]);
-                ps[g >> 1][2 * (g & 1)] = E::pack2_rne(d[0], d[1]);
-                ps[g >> 1][2 * (g & 1) + 1] = E::pack2_rne(d[2], d[3]);
-            }
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const u32x4 bp = {pp[u][0], pp[u][1], pp[u][2], pp[u][3]};
-                const u32x4 bs = {ps[u][0], ps[u][1], ps[u][2], ps[u][3]};
-                const uint32_t off = so + 4096 * blk + 2048 * u;
-#pragma unroll
-                for (int b = 0; b < OB; ++b) {
-                    const uint32_t ho = off + (b >> 1) * TILE_BYTES;
-                    const u32x2 qlo = lds_read_tr16_b64(tr.traddr[b & 1][0] + ho);          // dK^T += Q^T dS
-                    const u32x2 qhi = lds_read_tr16_b64(tr.traddr[b & 1][1] + ho);
-                    const u32x4 qa = {qlo.x, qlo.y, qhi.x, qhi.y};
-                    dkacc[b] = E::mfma(qa, bs, dkacc[b]);
-                    const u32x2 dlo = lds_read_tr16_b64(tr.traddr[b & 1][0] + ho + C::OFF_B);       // dV^T += dO^T P
-                    const u32x2 dhi = lds_read_tr16_b64(tr.traddr[b & 1][1] + ho + C::OFF_B);
-                    const u32x4 da = {dlo.x, dlo.y, dhi.x, dhi.y};
-                    dvacc[b] = E::mfma(da, bp, dvacc[b]);
-                }
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
     };
@@ -588,44 +644,39 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
     __syncthreads();
     if constexpr (HALVES) {
         // the sums over the other 32 rows of every tile, from the wavefront that has the same keys
-        const uint32_t sums = lds0 + (wave & 3) * (OB * 8192) + lane * 16;
+        const uint32_t sums = lds0 + (wave & 3) * (DB * 4096) + lane * 16;
         if (half == 1 && wave_valid) {
 #pragma unroll
-            for (int b = 0; b < OB; ++b)
+            for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    *(LDS_PTR(f32x4))(uintptr_t)(sums + (4 * b + g) * 1024) =
-                        f32x4{dkacc[b][4 * g], dkacc[b][4 * g + 1], dkacc[b][4 * g + 2], dkacc[b][4 * g + 3]};
-                    *(LDS_PTR(f32x4))(uintptr_t)(sums + (4 * (OB + b) + g) * 1024) =
-                        f32x4{dvacc[b][4 * g], dvacc[b][4 * g + 1], dvacc[b][4 * g + 2], dvacc[b][4 * g + 3]};
+                for (int b = 0; b < DB; ++b) {
+                    *(LDS_PTR(f32x4))(uintptr_t)(sums + (kb * DB + b) * 1024) = dkacc[kb][b];
+                    *(LDS_PTR(f32x4))(uintptr_t)(sums + ((2 + kb) * DB + b) * 1024) = dvacc[kb][b];
                 }
         }
         __syncthreads();
         if (half == 1 || !wave_valid) return;
         // One gradient after the other: with both sums in registers at once 17 to 20 of them were spilled, here and because of their allocation to the
         // whole kernel, which took 256 registers for 246 (36 heads, N = 2048, the backward alone: 329.6 -> 327.8 us; 128, N = 4096: 3326 -> 3308).
-        auto add = [&](f32x16 (&acc)[OB], uint32_t at) __attribute__((always_inline)) {
+        auto add = [&](f32x4 (&acc)[2][DB], uint32_t at) __attribute__((always_inline)) {
 #pragma unroll
-            for (int b = 0; b < OB; ++b) {
-                __builtin_amdgcn_sched_barrier(0);        // one block's sums in registers at a time
+            for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const f32x4 x = *(LDS_PTR(f32x4))(uintptr_t)(at + (4 * b + g) * 1024);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) acc[b][4 * g + j] += x[j];
+                for (int b = 0; b < DB; ++b) {
+                    if (b % 4 == 0) __builtin_amdgcn_sched_barrier(0);        // four blocks' sums in registers at a time
+                    acc[kb][b] += *(LDS_PTR(const f32x4))(uintptr_t)(at + (kb * DB + b) * 1024);
                 }
-            }
         };
         add(dkacc, sums);
-        store_gradient<BF16, WIDE>(dkacc, a.scale, lds0 + wave * (OB * 8192), a, a.dk, bi, hi, key0, lane);      // over its own sums
+        store_gradient16<BF16, WIDE>(dkacc, a.scale, lds0 + wave * (DB * 4096), a, a.dk, bi, hi, key0, lane);      // over its own sums
         __builtin_amdgcn_sched_barrier(0);
-        add(dvacc, sums + OB * 4096);
-        store_gradient<BF16, WIDE>(dvacc, 1.0f, lds0 + wave * (OB * 8192), a, a.dv, bi, hi, key0, lane);
+        add(dvacc, sums + DB * 2048);
+        store_gradient16<BF16, WIDE>(dvacc, 1.0f, lds0 + wave * (DB * 4096), a, a.dv, bi, hi, key0, lane);
         return;
     }
     if (wave_valid) {
-        store_gradient<BF16, WIDE>(dkacc, a.scale, lds0 + wave * 4096, a, a.dk, bi, hi, key0, lane);
-        store_gradient<BF16, WIDE>(dvacc, 1.0f, lds0 + wave * 4096, a, a.dv, bi, hi, key0, lane);
+        store_gradient16<BF16, WIDE>(dkacc, a.scale, lds0 + wave * 4096, a, a.dk, bi, hi, key0, lane);
+        store_gradient16<BF16, WIDE>(dvacc, 1.0f, lds0 + wave * 4096, a, a.dv, bi, hi, key0, lane);
     }
 }
 

@@ -38,6 +38,10 @@ template <> struct Elem<false> {
         return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
                                                       __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
     }
+    static __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
+                                                      __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+    }
     // Two probabilities -> one packed register with the cheapest conversion the format has (fp16:
     // v_cvt_pkrtz, round toward zero); the row sum is taken over the SAME rounded values, so
     // numerator and denominator stay consistent whatever the rounding.
@@ -65,6 +69,10 @@ template <> struct Elem<true> {
     static constexpr uint32_t ONES = 0x3f803f80u;           // two bf16 1.0
     static __device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                       __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
                                                        __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
     }
     static __device__ __forceinline__ uint32_t pack2_prob(float a, float b) {
@@ -114,6 +122,12 @@ __device__ __forceinline__ float xhalf_max(float x) {
 __device__ __forceinline__ float xhalf_sum(float x) {
     const uint32_t u = __builtin_bit_cast(uint32_t, x);
     const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
+}
+// The same with the partner in the neighbouring row of 16 lanes (lane l <-> lane l ^ 16).
+__device__ __forceinline__ float xrow_sum(float x) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, x);
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
     return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
 }
 
@@ -188,27 +202,13 @@ __device__ __forceinline__ BlockDst columns_from(const BlockDst &d, int col)
     return BlockDst{d.h + col, d.f + col, d.h_sn, d.f_sn, d.cols - col};
 }
 
-// Transposed store of a 32 x COLS accumulator block (COLS = 64: acc[dblk][4g+j] = value(row l32,
-// column 32dblk + 8g + 4hh + j) with acc = {acc0, acc1}; COLS = 32: acc0 only) times `mult`, through
-// 4 KiB of wave-private LDS, as whole pieces of rows.  Non-temporal stores: what is written is not
+// The second half of a transposed store: a 32 x COLS block of 16-bit results that lies in 4 KiB of wave-private LDS (row r at 128 r, its
+// 16-byte chunks at their position ^ (r / 2) % 8) goes out as whole pieces of rows.  Non-temporal stores: what is written is not
 // read again by the kernel and should not displace its inputs from the caches.
-template <bool BF16, int COLS = 64>
-__device__ __forceinline__ void store_block(const f32x16 &acc0, const f32x16 &acc1, float mult, uint32_t lds_wave,
-                                            const BlockDst &dst, bool has_h, bool has_f, int row0, int N, int lane)
+template <bool BF16, int COLS>
+__device__ __forceinline__ void store_landed(uint32_t lds_wave, const BlockDst &dst, bool has_h, bool has_f, int row0, int N, int lane)
 {
-    const f32x16 acc[2] = {acc0, acc1};
     using E = Elem<BF16>;
-    const int l32 = lane & 31, hh = lane >> 5;
-    const uint32_t wrow = lds_wave + l32 * 128 + hh * 8;
-    const int fo = (l32 >> 1) & 7;
-#pragma unroll
-    for (int dblk = 0; dblk < COLS / 32; ++dblk)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const u32x2 o = {E::pack2_rne(acc[dblk][4 * g + 0] * mult, acc[dblk][4 * g + 1] * mult),
-                             E::pack2_rne(acc[dblk][4 * g + 2] * mult, acc[dblk][4 * g + 3] * mult)};
-            *(LDS_PTR(u32x2))(uintptr_t)(wrow + (((4 * dblk + g) ^ fo) << 4)) = o;
-        }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -258,6 +258,27 @@ __device__ __forceinline__ void store_block(const f32x16 &acc0, const f32x16 &ac
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
+// Transposed store of a 32 x COLS accumulator block (COLS = 64: acc[dblk][4g+j] = value(row l32,
+// column 32dblk + 8g + 4hh + j) with acc = {acc0, acc1}; COLS = 32: acc0 only) times `mult`.
+template <bool BF16, int COLS = 64>
+__device__ __forceinline__ void store_block(const f32x16 &acc0, const f32x16 &acc1, float mult, uint32_t lds_wave,
+                                            const BlockDst &dst, bool has_h, bool has_f, int row0, int N, int lane)
+{
+    const f32x16 acc[2] = {acc0, acc1};
+    using E = Elem<BF16>;
+    const int l32 = lane & 31, hh = lane >> 5;
+    const uint32_t wrow = lds_wave + l32 * 128 + hh * 8;
+    const int fo = (l32 >> 1) & 7;
+#pragma unroll
+    for (int dblk = 0; dblk < COLS / 32; ++dblk)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const u32x2 o = {E::pack2_rne(acc[dblk][4 * g + 0] * mult, acc[dblk][4 * g + 1] * mult),
+                             E::pack2_rne(acc[dblk][4 * g + 2] * mult, acc[dblk][4 * g + 3] * mult)};
+            *(LDS_PTR(u32x2))(uintptr_t)(wrow + (((4 * dblk + g) ^ fo) << 4)) = o;
+        }
+    store_landed<BF16, COLS>(lds_wave, dst, has_h, has_f, row0, N, lane);
+}
 // The same for all 32-column blocks of an output row (acc[2 * half + dblk]); `stride` LDS bytes between the
 // areas of the two column halves (0: one after the other through the same 4 KiB).
 template <bool BF16, int OB>
@@ -273,6 +294,34 @@ __device__ __forceinline__ void store_rows(const f32x16 (&acc)[OB], float mult, 
         if constexpr (OB == 4)
             store_block<BF16>(acc[2], acc[3], mult, lds_wave + stride, columns_from(dst, 64), has_h, has_f, row0, N, lane);
     }
+}
+
+// The same from accumulators of 16 x 16 products: acc[rb][db][j] = value(row 16rb + lane % 16, column 16db + 4 (lane / 16) + j).
+template <bool BF16, int COLS, int DB0, int NB>
+__device__ __forceinline__ void store_block16(const f32x4 (&acc)[2][NB], float mult, uint32_t lds_wave,
+                                              const BlockDst &dst, bool has_h, bool has_f, int row0, int N, int lane)
+{
+    using E = Elem<BF16>;
+    const int l16 = lane & 15, q4 = lane >> 4;
+    const uint32_t wrow = lds_wave + l16 * 128 + (q4 & 1) * 8;
+    const int chunk = (q4 >> 1) ^ (l16 >> 1);
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+        for (int db = 0; db < COLS / 16; ++db) {
+            const f32x4 x = acc[rb][DB0 + db] * mult;
+            const u32x2 o = {E::pack2_rne(x[0], x[1]), E::pack2_rne(x[2], x[3])};
+            *(LDS_PTR(u32x2))(uintptr_t)(wrow + 2048 * rb + ((chunk ^ (2 * db)) << 4)) = o;
+        }
+    store_landed<BF16, COLS>(lds_wave, dst, has_h, has_f, row0, N, lane);
+}
+template <bool BF16, int NB>
+__device__ __forceinline__ void store_rows16(const f32x4 (&acc)[2][NB], float mult, uint32_t lds_wave,
+                                             const BlockDst &dst, bool has_h, bool has_f, int row0, int N, int lane)
+{
+    store_block16<BF16, NB == 2 ? 32 : 64, 0>(acc, mult, lds_wave, dst, has_h, has_f, row0, N, lane);
+    if constexpr (NB > 4)
+        store_block16<BF16, NB == 6 ? 32 : 64, 4>(acc, mult, lds_wave, columns_from(dst, 64), has_h, has_f, row0, N, lane);
 }
 
 }  // namespace
