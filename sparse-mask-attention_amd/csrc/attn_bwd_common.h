@@ -93,7 +93,8 @@ __device__ __forceinline__ void store_gradient16(const f32x4 (&acc)[2][NB], floa
                                                  const Rows &r, int bi, int hi, int row0, int lane)
 {
     const Rows none = {nullptr, 0u, 0u, 0u};
-    store_rows16<BF16>(acc, mult, lds_wave, block_dst(WIDE ? none : r, WIDE ? r : none, bi, hi, row0, a.D), !WIDE, WIDE, row0, a.N, lane);
+    const float both[2] = {mult, mult};
+    store_rows16<BF16>(acc, both, lds_wave, 0, block_dst(WIDE ? none : r, WIDE ? r : none, bi, hi, row0, a.D), !WIDE, WIDE, row0, a.N, lane);
 }
 
 }  // namespace

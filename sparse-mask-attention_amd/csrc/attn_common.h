@@ -124,7 +124,25 @@ __device__ __forceinline__ float xhalf_sum(float x) {
     const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
     return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
 }
-// The same with the partner in the neighbouring row of 16 lanes (lane l <-> lane l ^ 16).
+// Products of 16 x 16 leave a lane values of the two rows 16x + lane % 16, x = 0, 1.  From these the largest / the sum of row lane % 32, in both
+// lane halves, and from something of row lane % 32 (in both halves) that of the lane's two.
+// v_permlane16_swap(a, b) leaves {a's lanes of even | b's of even sixteens, a's of odd | b's of odd sixteens} in even | odd sixteens.
+__device__ __forceinline__ float rows_max(float x0, float x1) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, x0), __builtin_bit_cast(uint32_t, x1), false, false);
+    return xhalf_max(__builtin_fmaxf(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1])));
+}
+__device__ __forceinline__ float rows_sum(float x0, float x1) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, x0), __builtin_bit_cast(uint32_t, x1), false, false);
+    return xhalf_sum(__builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]));
+}
+struct RowPair {
+    uint32_t w[2];
+};
+__device__ __forceinline__ RowPair of_rows(uint32_t u) {
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return RowPair{{(uint32_t)r[0], (uint32_t)r[1]}};
+}
+// The sum of a value and its partner's in the neighbouring sixteen (lane l <-> lane l ^ 16).
 __device__ __forceinline__ float xrow_sum(float x) {
     const uint32_t u = __builtin_bit_cast(uint32_t, x);
     const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
@@ -298,7 +316,7 @@ __device__ __forceinline__ void store_rows(const f32x16 (&acc)[OB], float mult, 
 
 // The same from accumulators of 16 x 16 products: acc[rb][db][j] = value(row 16rb + lane % 16, column 16db + 4 (lane / 16) + j).
 template <bool BF16, int COLS, int DB0, int NB>
-__device__ __forceinline__ void store_block16(const f32x4 (&acc)[2][NB], float mult, uint32_t lds_wave,
+__device__ __forceinline__ void store_block16(const f32x4 (&acc)[2][NB], const float (&mult)[2], uint32_t lds_wave,
                                               const BlockDst &dst, bool has_h, bool has_f, int row0, int N, int lane)
 {
     using E = Elem<BF16>;
@@ -309,19 +327,19 @@ __device__ __forceinline__ void store_block16(const f32x4 (&acc)[2][NB], float m
     for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
         for (int db = 0; db < COLS / 16; ++db) {
-            const f32x4 x = acc[rb][DB0 + db] * mult;
+            const f32x4 x = acc[rb][DB0 + db] * mult[rb];
             const u32x2 o = {E::pack2_rne(x[0], x[1]), E::pack2_rne(x[2], x[3])};
             *(LDS_PTR(u32x2))(uintptr_t)(wrow + 2048 * rb + ((chunk ^ (2 * db)) << 4)) = o;
         }
     store_landed<BF16, COLS>(lds_wave, dst, has_h, has_f, row0, N, lane);
 }
 template <bool BF16, int NB>
-__device__ __forceinline__ void store_rows16(const f32x4 (&acc)[2][NB], float mult, uint32_t lds_wave,
+__device__ __forceinline__ void store_rows16(const f32x4 (&acc)[2][NB], const float (&mult)[2], uint32_t lds_wave, uint32_t stride,
                                              const BlockDst &dst, bool has_h, bool has_f, int row0, int N, int lane)
 {
     store_block16<BF16, NB == 2 ? 32 : 64, 0>(acc, mult, lds_wave, dst, has_h, has_f, row0, N, lane);
     if constexpr (NB > 4)
-        store_block16<BF16, NB == 6 ? 32 : 64, 4>(acc, mult, lds_wave, columns_from(dst, 64), has_h, has_f, row0, N, lane);
+        store_block16<BF16, NB == 6 ? 32 : 64, 4>(acc, mult, lds_wave + stride, columns_from(dst, 64), has_h, has_f, row0, N, lane);
 }
 
 }  // namespace

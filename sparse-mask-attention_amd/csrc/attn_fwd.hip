@@ -9,20 +9,31 @@
 //                 Three work-groups fit a CU (<= 168 VGPRs, ~34 KB LDS each): one wavefront of
 //                 each per SIMD, so that the softmax VALU work of one overlaps the MFMAs of another.
 //   wavefront   = 32 query rows.  It computes S^T = K_tile (64x64) * Q^T (64x32) with
-//                 v_mfma_f32_32x32x16, so every lane owns ONE query row (lane % 32) and 32 of the
-//                 tile's 64 keys: the online softmax is a per-lane register loop plus a single
-//                 exchange between lane l and lane l+32 (v_permlane32_swap).  P^T is already in
+//                 v_mfma_f32_16x16x32, so every lane owns two query rows (lane % 16 and 16 more) and 16 of the
+//                 tile's 64 keys: the online softmax is a per-lane register loop, and what is looked at once
+//                 a tile or less (maximum, reference point, total) is kept for row lane % 32 by two
+//                 exchanges (v_permlane16_swap, v_permlane32_swap).  P^T is already in
 //                 the B-operand layout of O^T += V^T * P^T: probabilities never leave registers.
+//                 The long grids run at the clock that the matrix cores' power leaves, and 16 x 16 x 32 draws
+//                 less than 32 x 32 x 16 (a stream on random operands: 1904 TFLOP/s at 1.89 GHz, 1689 at 1.69).
+//                 These products are short, so their operands are requested two or three steps of two
+//                 products ahead (four or more of V while the exponentials run), in an order that scheduling barriers
+//                 hold.  Forward, 32 x 32 x 16 with operands one step ahead -> this, in us:
+//                   packed, 128 heads, N = 2048    D = 32 99 -> 96, 64 147 -> 138, 96 213 -> 200, 128 257 -> 239
+//                   causal, 128 heads, N = 2000    D = 64 105 -> 102, 96 148 -> 144, 128 175 -> 167
+//                   boolean, 128 heads, N = 1000   D = 64 49.5 -> 48.4, 128 76.9 -> 74.8;  1024 heads, N = 200: D = 64 30.0 -> 29.9
+//                   packed, 192 heads, N = 1024    D = 64 59.3 -> 56.5 (blocks, map 37.3 -> 36.9), 128 106 -> 100 (62.2 -> 61.2)
+//                 A call of one or two tiles takes the same cycles as before.
 //   K/V tiles   = copied global -> LDS by global_load_lds_dwordx4 (no VGPR staging) into a ring of
 //                 two stages, one tile ahead of the one being computed.  Rows are 128 B; the
 //                 16-byte chunks of a row are XOR-swizzled (the permutation is applied to the
 //                 global address of each lane; the LDS side of such a load is always linear) so
-//                 that K's ds_read_b128 (32 consecutive rows, same column) and V's
-//                 ds_read_b64_tr_b16 (transposing read, 8 consecutive rows x 64 B) are free of
+//                 that K's ds_read_b128 (16 consecutive rows x 64 B) and V's
+//                 ds_read_b64_tr_b16 (transposing read, 16 consecutive rows x 32 B) are free of
 //                 bank conflicts on the 64-bank LDS.
 //   mask        = each wavefront copies the two packed words per query row of a tile into LDS with
-//                 one global_load_lds_dword, one tile ahead.  A lane reads the two words of its
-//                 row; each nibble selects one of 16 rows of a small LDS table of four floats that
+//                 one global_load_lds_dword, one tile ahead.  A lane reads the two words of
+//                 row lane % 32 and has those of its two rows by an exchange; each nibble selects one of 16 rows of a small LDS table of four floats that
 //                 are 0 (keep) or -inf (drop); one ds_read_b128 of that row initialises four
 //                 accumulator registers of the QK^T MFMA chain.  Masking costs no VALU work per score.
 //   exponent    = q is multiplied by scale*log2(e) when it is loaded, and the reference point of
@@ -66,9 +77,9 @@ constexpr float SUM_LIMIT = 16384.0f;     // a lane's 32 weights of a tile sum t
 //        pair of accumulators.  A stage is twice as large (32 KiB) and the kernel needs about 224
 //        registers, so two work-groups share a CU.
 //   32   half a tile: the copies fill the upper half of every LDS row with copies of the row's last
-//        16 bytes, which are never read; the QK^T chain has two steps instead of four and P multiplies
-//        one 32-column block of V.
-//   96   128 with such a half tile as its second half: six steps, three blocks.  D = 80 and 96 ran in the
+//        16 bytes, which are never read; the QK^T chain has one step instead of two and P multiplies
+//        two 16-column blocks of V.
+//   96   128 with such a half tile as its second half: three steps, six blocks.  D = 80 and 96 ran in the
 //        128 kernel before, through zero-padded copies (16 x 8 heads, N = 1088, D = 96: 156 -> 81 us)
 //
 // BYTEMASK: the mask arrives as the caller's boolean bytes (one per score, 0 or 1) instead of packed
@@ -81,7 +92,7 @@ template <int NH, bool BYTEMASK, bool SPLIT> struct Cfg {
     static constexpr int NSTAGE = SPLIT ? 4 : 2;
     static constexpr int MASK_COPIES = BYTEMASK ? 2 : 1;
     static constexpr int COPIES = MASK_COPIES + 4 * NH;             // async copies per wave and tile
-    // LDS map (bytes)
+    // LDS map (bytes), after the 256 of the table of the mask bias, which lies first: a read's immediate offset reaches 64 KiB
     static constexpr int STAGE_BYTES = 2 * NH * TILE_BYTES;         // K halves, then V halves
     static constexpr int OFF_V = NH * TILE_BYTES;                   // V inside a stage
     // mask: packed words in NSTAGE slots of 4 waves x 64 words; bytes in slots of 4 waves x 2 KiB,
@@ -92,14 +103,14 @@ template <int NH, bool BYTEMASK, bool SPLIT> struct Cfg {
     static constexpr int OFF_MASK = NSTAGE * STAGE_BYTES;
     static constexpr int BYTE_SLOTS = NH == 1 && !SPLIT ? 2 : 1;
     static constexpr int MASK_SLOT = BYTEMASK ? (BYTE_SLOTS - 1) * 8192 : 1024;     // distance between the slots
-    static constexpr int OFF_LUT = OFF_MASK + (BYTEMASK ? BYTE_SLOTS * 8192 : SPLIT ? 1024 : NSTAGE * 1024);   // 16 x 16 B
     // byte mask only: the tile-map bits the wavefronts collect, [4 waves][MAP_WORDS][some, hole],
     // and one arrival counter per pair of wavefronts (block of 64 rows)
     static constexpr int MAP_WORDS = 32;                            // 32 x 32 key tiles: N <= 65536
     // (SPLIT writes them to memory at once)
-    static constexpr int OFF_MAP = OFF_LUT + 256;
+    static constexpr int OFF_MAP = OFF_MASK + (BYTEMASK ? BYTE_SLOTS * 8192 : SPLIT ? 1024 : NSTAGE * 1024);
     static constexpr int OFF_MAP_ARRIVED = OFF_MAP + 4 * MAP_WORDS * 8;
-    static constexpr int LDS_BYTES = BYTEMASK && !SPLIT ? OFF_MAP_ARRIVED + 16 : OFF_MAP;
+    static constexpr int LUT_BYTES = 256;                           // 16 x 16 B
+    static constexpr int LDS_BYTES = LUT_BYTES + (BYTEMASK && !SPLIT ? OFF_MAP_ARRIVED + 16 : OFF_MAP);
 };
 
 template <int N> __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory"); }
@@ -142,22 +153,25 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     constexpr bool PAIRS = FETCH != 0, WHOLE = FETCH == 1;
     using E = Elem<BF16>;
     constexpr int NH = HDIM > 64 ? 2 : 1;         // 64-column tiles per matrix
-    constexpr int KS = HDIM / 16;                 // MFMA steps of the QK^T chain
-    constexpr int OB = HDIM / 32;                 // 32-column accumulator blocks of O
+    constexpr int KS = HDIM / 32;                 // MFMA steps of the QK^T chain
+    constexpr int DB = HDIM / 16;                 // 16-column accumulator blocks of O
+    constexpr int AHEAD = SPLIT ? 4 : HDIM <= 64 ? 2 : 3;              // steps by which an operand is requested before its use: scores
+    constexpr int V_AHEAD = SPLIT ? DB * 2 < 8 ? DB * 2 : 8 : HDIM <= 64 ? 4 : 6;             // ... and values, when the scores' registers are free
     // second column half at a constant distance from the first in every row
     constexpr bool SAME_HALVES = HDIM == 128 && PACKED_ROWS;
     using C = Cfg<NH, BYTEMASK, SPLIT>;
-    constexpr int NSTAGE = C::NSTAGE, STAGE_BYTES = C::STAGE_BYTES, OFF_MASK = C::OFF_MASK, OFF_LUT = C::OFF_LUT;
+    constexpr int NSTAGE = C::NSTAGE, STAGE_BYTES = C::STAGE_BYTES, OFF_MASK = C::OFF_MASK;
     constexpr int MASK_SLOT = C::MASK_SLOT;
     const int D = PACKED_ROWS ? HDIM : a.D;
     const int last_chunk = (D >> 3) - 1;          // 16-byte chunks per global row, minus one
     __shared__ __attribute__((aligned(1024))) unsigned char smem[C::LDS_BYTES];
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(LDS_PTR(unsigned char))smem;
+    const uint32_t lut_addr = (uint32_t)(uintptr_t)(LDS_PTR(unsigned char))smem, lds0 = lut_addr + C::LUT_BYTES;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int l32 = lane & 31, hh = lane >> 5;
+    const int l32 = lane & 31, hh = lane >> 5;       // mask: a row and a half of its words
+    const int l16 = lane & 15, q4 = lane >> 4;       // products: rows l16 and 16 + l16
 
     const int nid = renumber_block();
     const int bh = (int)fastdiv((uint32_t)nid, a.div_qtiles);
@@ -558,33 +572,18 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         }
     };
 
-    // ---- per-lane LDS read addresses (stage 0, first column half); everything else is an immediate offset ----
-    // K operand (blk, s): row 32*blk + l32, chunk 2s + hh           -> kaddr[s] + 4096*blk
-    // V operand (dblk, blk, u, x), read by ds_read_b64_tr_b16: the lane supplies
-    //   row 32blk + 16u + 8x + 4hh + (i >> 2), columns 32dblk + 16G + 4(i & 3) .. +3
-    //   with i = lane % 16, G = (lane % 32) / 16                     -> vaddr[dblk][x] + 4096*blk + 2048*u
-    uint32_t kaddr[4], vaddr[2][2];
+    // ---- per-lane LDS read addresses (stage 0, first column half, first columns); everything else flips bits or is an immediate offset ----
+    // K operand (block of 16 keys kb, step c): row 16kb + l16, chunk 4c + q4           -> (k_at ^ 64 (c % 2)) + 2048kb
+    // V operand (16 columns db, block of 32 keys), read by ds_read_b64_tr_b16: the lane supplies
+    //   rows 16x + 4q4 + (l16 >> 2), columns 16db + 4(l16 & 3) .. +3, x = 0, 1                -> (v_at ^ 32 (db % 4)) + 2048x
+    uint32_t k_at, v_at;
     {
-        const uint32_t lds0 = SPLIT ? split_dst : (uint32_t)(uintptr_t)(LDS_PTR(unsigned char))smem;
-        const int fk = (l32 >> 1) & 7;
-#pragma unroll
-        for (int s = 0; s < 4; ++s) kaddr[s] = lds0 + l32 * 128 + (((2 * s + hh) ^ fk) << 4);
-        const int i16 = lane & 15, G = l32 >> 4;
-        const int r3 = 4 * hh + (i16 >> 2);
-#pragma unroll
-        for (int x = 0; x < 2; ++x) {
-            const int row = 8 * x + r3;
-            const int f = (row >> 1) & 7;
-            const int fr = bitrev3(f);
-#pragma unroll
-            for (int dblk = 0; dblk < 2; ++dblk) {
-                const int chunk = 4 * dblk + 2 * G + ((i16 & 3) >> 1);
-                vaddr[dblk][x] = lds0 + C::OFF_V + row * 128 + ((chunk ^ fr) << 4) + ((i16 & 1) << 3);
-            }
-        }
+        const uint32_t own0 = SPLIT ? split_dst : lds0;
+        const int r = 4 * q4 + (l16 >> 2);
+        k_at = own0 + l16 * 128 + ((q4 ^ (l16 >> 1)) << 4);
+        v_at = own0 + C::OFF_V + r * 128 + ((((l16 & 3) >> 1) ^ bitrev3(r >> 1)) << 4) + ((l16 & 1) << 3);
     }
-    const uint32_t lut_addr = lds0 + OFF_LUT;
-    const uint32_t nib_shift = 4u - 4u * hh;
+    const uint32_t nib_rotate = (4u * q4 + 28u) & 31u;     // right: the nibble of keys 4q4 .. 4q4 + 3 comes to bits 4 .. 7
 
     // ================================ prologue: one memory round trip ================================
     constexpr int Q_HALF = SPLIT ? 4096 : 16384;         // between the column halves of the staged q
@@ -629,11 +628,19 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     if ((T & 31) != 0 && TW == 1) live_w &= (1u << (T & 31)) - 1u;
     const uint32_t own_tiles = SPLIT ? 0x11111111u << wave : 0xffffffffu;
     live_w &= own_tiles;
-    const int n_visits = TW == 1 ? __builtin_popcount(live_w) : T;
+    const int n_visits = !BYTEMASK && TW == 1 ? __builtin_popcount(live_w) : T;
+    // (BYTEMASK: there is no map, and every tile, or every fourth of SPLIT, is visited.)
     // Walk over the set bits of the "live" words: `live_w` holds the bits of word `cur_w` that have
     // not been visited yet.  Words beyond the first (N > 2048) are fetched when the walk gets there.
     int base_t = 0, cur_w = 0;
+    constexpr int STRIDE = SPLIT ? 4 : 1;
+    int upcoming = SPLIT ? wave : 0;
     auto next_tile = [&]() __attribute__((always_inline)) -> int {     // next live tile, T if there is none; wave-uniform
+        if constexpr (BYTEMASK) {
+            const int t = upcoming < T ? upcoming : T;
+            upcoming += STRIDE;
+            return t;
+        }
         while (UNLIKELY(live_w == 0u)) {
             if (++cur_w >= TW) return T;
             base_t = 32 * cur_w;
@@ -680,7 +687,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     }
     // small LDS table for the mask: entry n (16 B) holds four floats, float j = (bit j of n) ? 0 : -inf
     if (tid < 64)
-        reinterpret_cast<float *>(smem + OFF_LUT)[tid] = (((tid >> 2) >> (tid & 3)) & 1) ? 0.f : -__builtin_inff();
+        reinterpret_cast<float *>(smem)[tid] = (((tid >> 2) >> (tid & 3)) & 1) ? 0.f : -__builtin_inff();
     int yield_at = -1;                  // the visit at which this wave next lowers its priority
     if (even_progress && n_visits >= 4) {
         __builtin_amdgcn_s_setprio(3);
@@ -691,47 +698,46 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     else if (t_first < T) wait_vmcnt<C::COPIES>();     // q has landed; the copies of the first tile may still be in flight
     else wait_vmcnt<0>();
     // ---- Q^T as MFMA B operands, scaled by scale*log2(e)/post_mul:
-    //      lane holds query row l32, d = 16*s + 8*hh .. +7
-    u32x4 qf[KS];
+    //      lane holds query rows 16x + l16, d = 32*c + 8*q4 .. +7
+    u32x4 qf[2][KS];
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-        u32x4 t = lds_read_b128(kaddr[s & 3] + (SPLIT ? C::OFF_V + (s >> 2) * Q_HALF : (NSTAGE - 1) * STAGE_BYTES + (s >> 2) * Q_HALF + wave * 4096));
+    for (int x = 0; x < 2; ++x)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float lo = E::up1((uint16_t)(t[i] & 0xffffu)) * a.q_scale;
-            const float hi = E::up1((uint16_t)(t[i] >> 16)) * a.q_scale;
-            t[i] = (uint32_t)E::cvt1(lo) | ((uint32_t)E::cvt1(hi) << 16);
+        for (int c = 0; c < KS; ++c) {
+            u32x4 t = lds_read_b128((k_at ^ (64 * (c & 1))) + 2048 * x +
+                                    (SPLIT ? C::OFF_V + (c >> 1) * Q_HALF : (NSTAGE - 1) * STAGE_BYTES + (c >> 1) * Q_HALF + wave * 4096));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float lo = E::up1((uint16_t)(t[i] & 0xffffu)) * a.q_scale;
+                const float hi = E::up1((uint16_t)(t[i] >> 16)) * a.q_scale;
+                t[i] = (uint32_t)E::cvt1(lo) | ((uint32_t)E::cvt1(hi) << 16);
+            }
+            if (!PACKED_ROWS && 4 * c + q4 > last_chunk) t = u32x4{0u, 0u, 0u, 0u};      // beyond the row: adds nothing
+            qf[x][c] = t;
         }
-        if (!PACKED_ROWS && 2 * s + hh > last_chunk) t = u32x4{0u, 0u, 0u, 0u};      // beyond the row: adds nothing
-        qf[s] = t;
-    }
 
     if constexpr (SPLIT) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (t_first < T) issue_own_v(t_first);
     }
     if constexpr (HALVES) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            kaddr[i] += 4096 * half;
-            vaddr[i >> 1][i & 1] += 4096 * half;
-        }
+        k_at += 4096 * half;
+        v_at += 4096 * half;
     }
 
-    // ---- running state: one query row per lane; both lane halves hold the same ref ----
-    f32x16 oacc[OB];                    // [2 * half + dblk]: 32 columns each
+    // ---- running state: of the query rows 16x + l16 what the products and sums need, of the row l32 (in both lane halves) what is
+    //      looked at once a tile ----
+    f32x4 oacc[2][DB];                  // 16 columns each
 #pragma unroll
-    for (int b = 0; b < OB; ++b)
+    for (int x = 0; x < 2; ++x)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) oacc[b][i] = 0.f;
+        for (int b = 0; b < DB; ++b) oacc[x][b] = f32x4{0.f, 0.f, 0.f, 0.f};
     float ref = 0.f;                    // reference point r, in accumulator units (log2 / pm)
     float rmax = -__builtin_inff();     // largest score seen when the maximum was last taken, minus r; -inf = no kept key yet
     int all_seen = 0;                   // wave-uniform: every row of this wavefront has met a kept key
-    float l_run = 0.f;                  // this lane's share of sum exp2(pm * (score - r))
-    u32x4 refb = {0u, 0u, 0u, 0u};      // -r as four 16-bit terms (lane half 0 only), B operand
+    float l_run[2] = {0.f, 0.f};        // this lane's share of sum exp2(pm * (score - r))
+    u32x2 refb[2] = {u32x2{0u, 0u}, u32x2{0u, 0u}};             // -r as four 16-bit terms (lanes 0 .. 15 only), B operand
     int ref_used = 0;                   // wave-uniform: 0 while r == 0 for every row: the extra MFMA is skipped
-    u32x4 ones = {E::ONES, E::ONES, E::ONES, E::ONES};
-    asm volatile("" : "+v"(ones));      // keep the constant operand resident in registers
 
     auto set_ref = [&](float r_wanted) __attribute__((always_inline)) -> float {      // returns the value actually represented
         float rest = -r_wanted, sum = 0.f;
@@ -744,9 +750,10 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
             rest -= got;
             sum += got;
         }
-        const uint32_t keep = hh == 0 ? 0xffffffffu : 0u;
-        refb.x = ((uint32_t)term[0] | ((uint32_t)term[1] << 16)) & keep;
-        refb.y = ((uint32_t)term[2] | ((uint32_t)term[3] << 16)) & keep;
+        const uint32_t keep = q4 == 0 ? 0xffffffffu : 0u;
+        const RowPair lo = of_rows((uint32_t)term[0] | ((uint32_t)term[1] << 16)), hi = of_rows((uint32_t)term[2] | ((uint32_t)term[3] << 16));
+#pragma unroll
+        for (int x = 0; x < 2; ++x) refb[x] = u32x2{lo.w[x] & keep, hi.w[x] & keep};
         return -sum;
     };
 
@@ -755,45 +762,62 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     // (SPLIT: `after_scores` runs when K has been read, `before_values` before V is.)
     constexpr int KB = HALVES ? 1 : 2;            // blocks of 32 keys that a wavefront takes of a tile
     auto compute_tile_with = [&](const u32x2 both, const uint32_t so, auto after_scores, auto before_values) __attribute__((always_inline)) {
-        const u32x2 w2 = HALVES ? u32x2{half ? both.y : both.x, 0u} : both;
+        const u32x2 w2 = HALVES ? u32x2{half ? both.y : both.x, 0u} : both;       // of row l32
         if (UNLIKELY(__builtin_amdgcn_ballot_w64((w2.x | w2.y) != 0u) == 0ull)) {
             after_scores();
             return;
         }
-        // ---- S^T: sacc[blk][4g+j] = log2 weight / pm of (key 32blk + 8g + 4hh + j, query l32) ----
-        f32x16 sacc[KB];
-        // The K fragments of MFMA step s + 1 are requested before the MFMAs of step s are issued, the
-        // first pair before the table look-ups below.  The scheduling barriers hold that order: left
-        // alone, the compiler requests each pair just before its MFMAs (it saves eight registers)
-        // and the wavefront sits out four LDS round trips per tile one after the other.
-        u32x4 kf[2][2];
-        kf[0][0] = lds_read_b128(kaddr[0] + so);
-        if constexpr (!HALVES) kf[0][1] = lds_read_b128(kaddr[0] + so + 4096);
+        asm volatile("" : "+v"(k_at), "+v"(v_at));       // or the compiler keeps a register for every address that follows from these
+        // Steps of two products: S^T of 16 keys and 32 columns each, then O^T += V^T P^T of 16 columns and 32 keys.  The operands of a step are
+        // requested AHEAD steps before it, and scheduling barriers hold that order: left alone, the compiler requests each just before
+        // its use (it saves registers) and the wavefront sits out one LDS round trip after the other.
+        constexpr int PH = 2 * KS, SCORES = KB * PH, VALUES = KB * DB;
+        u32x4 k_ring[AHEAD + 1], v_ring[V_AHEAD + 1];
+        auto fetch_k = [&](int n) __attribute__((always_inline)) {
+            const int blk = n / PH, kb = n & 1, c = n % PH >> 1;
+            if (n < SCORES) k_ring[n % (AHEAD + 1)] = lds_read_b128((k_at ^ (64 * (c & 1))) + so + (c >> 1) * TILE_BYTES + 4096 * blk + 2048 * kb);
+        };
+        auto fetch_v = [&](int n) __attribute__((always_inline)) {
+            if (n >= VALUES) return;
+            const int blk = n / DB, b = n % DB;
+            const uint32_t at = (v_at ^ (32 * (b & 3))) + so + (b >> 2) * TILE_BYTES + 4096 * blk;
+            const u32x2 lo = lds_read_tr16_b64(at), hi = lds_read_tr16_b64(at + 2048);
+            v_ring[n % (V_AHEAD + 1)] = u32x4{lo.x, lo.y, hi.x, hi.y};
+        };
+#pragma unroll
+        for (int n = 0; n < AHEAD; ++n) fetch_k(n);
         __builtin_amdgcn_sched_barrier(0);
+        constexpr int EARLY_V = SPLIT || (BYPRODUCTS && HDIM == 64) ? 0 : HDIM <= 64 ? 2 : 4;       // of V before the exponentials, where there are registers
+        // ---- S^T: sacc[blk][kb][x][j] = log2 weight / pm of (key 32blk + 16kb + 4q4 + j, query 16x + l16) ----
+        f32x4 sacc[KB][2][2];
 #pragma unroll
         for (int blk = 0; blk < KB; ++blk) {
-            const uint32_t wa = (blk == 0 ? w2.x : w2.y) << nib_shift;
+            const uint32_t wl = blk == 0 ? w2.x : w2.y;
+            const RowPair rows = of_rows(wl);
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const u32x4 b = lds_read_b128(lut_addr + ((wa >> (8 * g)) & 0xF0u));
-#pragma unroll
-                for (int j = 0; j < 4; ++j) sacc[blk][4 * g + j] = __builtin_bit_cast(float, (uint32_t)b[j]);
+            for (int x = 0; x < 2; ++x) {
+                const uint32_t wa = __builtin_amdgcn_alignbit(rows.w[x], rows.w[x], nib_rotate);
+                sacc[blk][0][x] = __builtin_bit_cast(f32x4, lds_read_b128(lut_addr + (wa & 0xF0u)));
+                sacc[blk][1][x] = __builtin_bit_cast(f32x4, lds_read_b128(lut_addr + ((wa >> 16) & 0xF0u)));
             }
         }
         if (UNLIKELY(ref_used)) {               // wave-uniform: some row of this wavefront has r != 0
-            sacc[0] = E::mfma(ones, refb, sacc[0]);
-            if constexpr (!HALVES) sacc[KB - 1] = E::mfma(ones, refb, sacc[KB - 1]);
+            const u32x4 ones = {E::ONES, E::ONES, E::ONES, E::ONES};
+#pragma unroll
+            for (int blk = 0; blk < KB; ++blk)
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                    for (int x = 0; x < 2; ++x) sacc[blk][kb][x] = E::mfma16(ones, u32x4{refb[x].x, refb[x].y, 0u, 0u}, sacc[blk][kb][x]);
         }
 #pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            if (s + 1 < KS) {
-                const uint32_t ka = kaddr[(s + 1) & 3] + so + ((s + 1) >> 2) * TILE_BYTES;
-                kf[(s + 1) & 1][0] = lds_read_b128(ka);
-                if constexpr (!HALVES) kf[(s + 1) & 1][1] = lds_read_b128(ka + 4096);
-            }
+        for (int n = 0; n < SCORES; ++n) {
+            fetch_k(n + AHEAD);
+            if (!SPLIT && n + EARLY_V >= SCORES) fetch_v(n + EARLY_V - SCORES);
             __builtin_amdgcn_sched_barrier(0);
-            sacc[0] = E::mfma(kf[s & 1][0], qf[s], sacc[0]);
-            if constexpr (!HALVES) sacc[KB - 1] = E::mfma(kf[s & 1][1], qf[s], sacc[KB - 1]);
+            const int blk = n / PH, kb = n & 1, c = n % PH >> 1;
+#pragma unroll
+            for (int x = 0; x < 2; ++x) sacc[blk][kb][x] = E::mfma16(k_ring[n % (AHEAD + 1)], qf[x][c], sacc[blk][kb][x]);
             __builtin_amdgcn_sched_barrier(0);
         }
         after_scores();
@@ -801,12 +825,18 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         // Moves the reference point when a row's scores leave the window [r-8, r+8] upwards, or when
         // the first kept score of a row lies below it.
         auto recentre = [&]() __attribute__((always_inline)) {
-            float mx = -__builtin_inff();
+            float m[2];
 #pragma unroll
-            for (int blk = 0; blk < KB; ++blk)
+            for (int x = 0; x < 2; ++x) {
+                m[x] = -__builtin_inff();
 #pragma unroll
-                for (int i = 0; i < 16; ++i) mx = __builtin_fmaxf(mx, sacc[blk][i]);
-            mx = xhalf_max(mx);
+                for (int blk = 0; blk < KB; ++blk)
+#pragma unroll
+                    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) m[x] = __builtin_fmaxf(m[x], sacc[blk][kb][x][j]);
+            }
+            const float mx = rows_max(m[0], m[1]);
             const float mxs = POSTMUL ? mx * pm : mx;
             const bool first = (rmax == -__builtin_inff());
             const bool move = (mxs > WINDOW_LOG2) | (first & (mxs < -WINDOW_LOG2) & (mx > -__builtin_inff()));
@@ -819,41 +849,47 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
                 const float alpha = first ? 1.0f : __builtin_amdgcn_exp2f(POSTMUL ? delta * pm : delta);
                 ref = new_ref;
                 ref_used = 1;
-                l_run *= alpha;
+                const RowPair da = of_rows(__builtin_bit_cast(uint32_t, delta)), al = of_rows(__builtin_bit_cast(uint32_t, alpha));
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
+                for (int x = 0; x < 2; ++x) {
+                    const float d = __builtin_bit_cast(float, da.w[x]), f = __builtin_bit_cast(float, al.w[x]);
+                    l_run[x] *= f;
 #pragma unroll
-                    for (int b = 0; b < OB; ++b) oacc[b][i] *= alpha;
-                    sacc[0][i] += delta;
-                    if constexpr (!HALVES) sacc[KB - 1][i] += delta;
+                    for (int b = 0; b < DB; ++b) oacc[x][b] *= f;
+#pragma unroll
+                    for (int blk = 0; blk < KB; ++blk)
+#pragma unroll
+                        for (int kb = 0; kb < 2; ++kb) sacc[blk][kb][x] += d;
                 }
                 rmax = top + delta;
             } else {
                 rmax = top;
             }
         };
-        // probabilities, packed as the B operands of the PV product; returns this lane's sum of them
-        uint32_t pb[KB][2][4];
-        auto exponentials = [&]() __attribute__((always_inline)) -> float {
-            float lsum = 0.f;
+        // probabilities, packed as the B operands of the PV product, and this lane's sums of them
+        u32x4 pb[KB][2];
+        float lsum[2];
+        auto exponentials = [&]() __attribute__((always_inline)) {
+            lsum[0] = lsum[1] = 0.f;
 #pragma unroll
             for (int blk = 0; blk < KB; ++blk)
 #pragma unroll
-                for (int u = 0; u < 2; ++u)
+                for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const float s0 = sacc[blk][8 * u + 2 * i], s1 = sacc[blk][8 * u + 2 * i + 1];
-                        const float p0 = __builtin_amdgcn_exp2f(POSTMUL ? s0 * pm : s0);
-                        const float p1 = __builtin_amdgcn_exp2f(POSTMUL ? s1 * pm : s1);
-                        const uint32_t pk = E::pack2_prob(p0, p1);
-                        pb[blk][u][i] = pk;
-                        lsum = E::add2(pk, lsum);
-                    }
-            return lsum;
+                    for (int i = 0; i < 2; ++i)
+#pragma unroll
+                        for (int x = 0; x < 2; ++x) {
+                            const float s0 = sacc[blk][kb][x][2 * i], s1 = sacc[blk][kb][x][2 * i + 1];
+                            const float p0 = __builtin_amdgcn_exp2f(POSTMUL ? s0 * pm : s0);
+                            const float p1 = __builtin_amdgcn_exp2f(POSTMUL ? s1 * pm : s1);
+                            const uint32_t pk = E::pack2_prob(p0, p1);
+                            pb[blk][x][2 * kb + i] = pk;
+                            lsum[x] = E::add2(pk, lsum[x]);
+                        }
         };
         // A row needs the maximum when it meets its first kept key (to choose its reference point)
         // and when a score runs away above the window.  The first is known beforehand; the second
-        // shows afterwards, in the sum of the exponentials (needed anyway): a weight above 2^14, an
+        // shows afterwards, in the sums of the exponentials (needed anyway): a weight above 2^14, an
         // infinity or a NaN makes a lane's sum of 32 weights exceed SUM_LIMIT, and no weight that
         // the window would have let pass (<= 2^8) can.  Only then are the maximum taken, the
         // reference moved and the exponentials redone.
@@ -865,31 +901,28 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
                 all_seen = __builtin_amdgcn_readfirstlane(__builtin_amdgcn_ballot_w64(rmax == -__builtin_inff()) == 0ull ? 1 : 0);
             }
         }
-        float lsum = exponentials();
-        if (UNLIKELY(__builtin_amdgcn_ballot_w64(!(lsum <= SUM_LIMIT)) != 0ull)) {
+        exponentials();
+        if (UNLIKELY(__builtin_amdgcn_ballot_w64(!(lsum[0] + lsum[1] <= SUM_LIMIT)) != 0ull)) {
             if (!with_max) {
                 recentre();
-                lsum = exponentials();
+                exponentials();
             }
         }
-        l_run += lsum;
+        l_run[0] += lsum[0];
+        l_run[1] += lsum[1];
         before_values();
-        // ---- O^T += V^T * P^T : oacc[b][4g+j] = out(query l32, d = 32b + 8g + 4hh + j) ----
+        // ---- O^T += V^T * P^T : oacc[x][b][j] = out(query 16x + l16, d = 16b + 4q4 + j) ----
 #pragma unroll
-        for (int blk = 0; blk < KB; ++blk)
+        for (int n = EARLY_V; n < V_AHEAD; ++n) fetch_v(n);
 #pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const u32x4 pv = {pb[blk][u][0], pb[blk][u][1], pb[blk][u][2], pb[blk][u][3]};
-                const uint32_t off = so + 4096 * blk + 2048 * u;
+        for (int n = 0; n < VALUES; ++n) {
+            fetch_v(n + V_AHEAD);
+            __builtin_amdgcn_sched_barrier(0);
+            const int blk = n / DB, b = n % DB;
 #pragma unroll
-                for (int b = 0; b < OB; ++b) {
-                    const uint32_t voff = off + (b >> 1) * TILE_BYTES;
-                    const u32x2 lo = lds_read_tr16_b64(vaddr[b & 1][0] + voff);
-                    const u32x2 hi = lds_read_tr16_b64(vaddr[b & 1][1] + voff);
-                    const u32x4 va = {lo.x, lo.y, hi.x, hi.y};
-                    oacc[b] = E::mfma(va, pv, oacc[b]);
-                }
-            }
+            for (int x = 0; x < 2; ++x) oacc[x][b] = E::mfma16(v_ring[n % (V_AHEAD + 1)], pb[blk][x], oacc[x][b]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     };
 
     auto compute_tile = [&](const u32x2 w2, const uint32_t so) __attribute__((always_inline)) {
@@ -1003,49 +1036,50 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         visit(tn, t, integral_constant<int, 1>{});
     }
     wait_vmcnt<0>();              // no copy may outlive the work-group's LDS allocation
+    float l_row = rows_sum(l_run[0], l_run[1]);
 
     if constexpr (SPLIT) {
         // Wavefronts 1 to 3 leave their sums in their own buffers, wavefront 0 adds them to its own, all of them
         // moved to the largest reference point of those that have met a kept key.
-        const bool seen = rmax > -__builtin_inff();
+        const f32x2 own = {rmax > -__builtin_inff() ? ref : -__builtin_inff(), l_row};
         if (wave != 0) {
 #pragma unroll
-            for (int b = 0; b < OB; ++b)
+            for (int x = 0; x < 2; ++x)
 #pragma unroll
-                for (int g = 0; g < 4; ++g)
-                    *(LDS_PTR(f32x4))(uintptr_t)(split_dst + (4 * b + g) * 1024 + lane * 16) =
-                        f32x4{oacc[b][4 * g], oacc[b][4 * g + 1], oacc[b][4 * g + 2], oacc[b][4 * g + 3]};
-            *(LDS_PTR(f32x2))(uintptr_t)(split_dst + OB * 4096 + lane * 8) = f32x2{seen ? ref : -__builtin_inff(), l_run};
+                for (int b = 0; b < DB; ++b)
+                    *(LDS_PTR(f32x4))(uintptr_t)(split_dst + (x * DB + b) * 1024 + lane * 16) = oacc[x][b];
+            *(LDS_PTR(f32x2))(uintptr_t)(split_dst + DB * 2048 + lane * 8) = own;
         }
         __syncthreads();
         if (wave != 0) return;
         f32x2 of_wave[4];
-        of_wave[0] = f32x2{seen ? ref : -__builtin_inff(), l_run};
-        float top = of_wave[0].x;
+        of_wave[0] = own;
+        float top = own.x;
 #pragma unroll
         for (int w = 1; w < 4; ++w) {
-            of_wave[w] = *(LDS_PTR(const f32x2))(uintptr_t)(lds0 + w * STAGE_BYTES + OB * 4096 + lane * 8);
+            of_wave[w] = *(LDS_PTR(const f32x2))(uintptr_t)(lds0 + w * STAGE_BYTES + DB * 2048 + lane * 8);
             top = __builtin_fmaxf(top, of_wave[w].x);
         }
         ref = top > -__builtin_inff() ? top : 0.f;
-        l_run = 0.f;
+        l_row = 0.f;
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
             // a wavefront that has met no kept key of the row has nothing to add (its factor is 0)
             const float d = of_wave[w].x - ref;
             const float f = __builtin_amdgcn_exp2f(POSTMUL ? d * pm : d);
-            l_run = __builtin_fmaf(of_wave[w].y, f, l_run);
+            l_row = __builtin_fmaf(of_wave[w].y, f, l_row);
+            const RowPair fx = of_rows(__builtin_bit_cast(uint32_t, f));
 #pragma unroll
-            for (int b = 0; b < OB; ++b)
+            for (int x = 0; x < 2; ++x)
 #pragma unroll
-                for (int g = 0; g < 4; ++g) {
+                for (int b = 0; b < DB; ++b) {
+                    const float g = __builtin_bit_cast(float, fx.w[x]);
                     if (w == 0) {
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) oacc[b][4 * g + j] *= f;
+                        oacc[x][b] *= g;
                     } else {
-                        const f32x4 o = *(LDS_PTR(const f32x4))(uintptr_t)(lds0 + w * STAGE_BYTES + (4 * b + g) * 1024 + lane * 16);
+                        const f32x4 o = *(LDS_PTR(const f32x4))(uintptr_t)(lds0 + w * STAGE_BYTES + (x * DB + b) * 1024 + lane * 16);
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) oacc[b][4 * g + j] = __builtin_fmaf(o[j], f, oacc[b][4 * g + j]);
+                        for (int j = 0; j < 4; ++j) oacc[x][b][j] = __builtin_fmaf(o[j], g, oacc[x][b][j]);
                     }
                 }
         }
@@ -1070,38 +1104,39 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         }
     }
 
-    constexpr int HALF_SUMS = OB * 4096 + 1024;          // of one wavefront
+    constexpr int HALF_SUMS = DB * 2048 + 1024;          // of one wavefront
     if constexpr (HALVES) {
         // Wavefronts 2 and 3 leave their sums for 0 and 1, which have the same rows, both moved to the larger reference point of
         // those that have met a kept key.
         const uint32_t sums = lds0 + (wave & 1) * HALF_SUMS;
-        const bool seen = rmax > -__builtin_inff();
+        const f32x2 own = {rmax > -__builtin_inff() ? ref : -__builtin_inff(), l_row};
         __syncthreads();                                  // the last tile has been read by all
         if (half == 1) {
 #pragma unroll
-            for (int b = 0; b < OB; ++b)
+            for (int x = 0; x < 2; ++x)
 #pragma unroll
-                for (int g = 0; g < 4; ++g)
-                    *(LDS_PTR(f32x4))(uintptr_t)(sums + (4 * b + g) * 1024 + lane * 16) =
-                        f32x4{oacc[b][4 * g], oacc[b][4 * g + 1], oacc[b][4 * g + 2], oacc[b][4 * g + 3]};
-            *(LDS_PTR(f32x2))(uintptr_t)(sums + OB * 4096 + lane * 8) = f32x2{seen ? ref : -__builtin_inff(), l_run};
+                for (int b = 0; b < DB; ++b)
+                    *(LDS_PTR(f32x4))(uintptr_t)(sums + (x * DB + b) * 1024 + lane * 16) = oacc[x][b];
+            *(LDS_PTR(f32x2))(uintptr_t)(sums + DB * 2048 + lane * 8) = own;
         }
         __syncthreads();
         if (half == 1) return;
-        const f32x2 other = *(LDS_PTR(const f32x2))(uintptr_t)(sums + OB * 4096 + lane * 8);
-        const float mine = seen ? ref : -__builtin_inff(), top = __builtin_fmaxf(mine, other.x);
+        const f32x2 other = *(LDS_PTR(const f32x2))(uintptr_t)(sums + DB * 2048 + lane * 8);
+        const float top = __builtin_fmaxf(own.x, other.x);
         ref = top > -__builtin_inff() ? top : 0.f;
         // one that has met no kept key of the row has nothing to add (its factor is 0)
-        const float dm = mine - ref, d = other.x - ref;
+        const float dm = own.x - ref, d = other.x - ref;
         const float fm = __builtin_amdgcn_exp2f(POSTMUL ? dm * pm : dm), f = __builtin_amdgcn_exp2f(POSTMUL ? d * pm : d);
-        l_run = __builtin_fmaf(other.y, f, l_run * fm);
+        l_row = __builtin_fmaf(other.y, f, l_row * fm);
+        const RowPair mine = of_rows(__builtin_bit_cast(uint32_t, fm)), its = of_rows(__builtin_bit_cast(uint32_t, f));
 #pragma unroll
-        for (int b = 0; b < OB; ++b)
+        for (int x = 0; x < 2; ++x)
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const f32x4 o = *(LDS_PTR(const f32x4))(uintptr_t)(sums + (4 * b + g) * 1024 + lane * 16);
+            for (int b = 0; b < DB; ++b) {
+                const f32x4 o = *(LDS_PTR(const f32x4))(uintptr_t)(sums + (x * DB + b) * 1024 + lane * 16);
+                const float g = __builtin_bit_cast(float, its.w[x]), gm = __builtin_bit_cast(float, mine.w[x]);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) oacc[b][4 * g + j] = __builtin_fmaf(o[j], f, oacc[b][4 * g + j] * fm);
+                for (int j = 0; j < 4; ++j) oacc[x][b][j] = __builtin_fmaf(o[j], g, oacc[x][b][j] * gm);
             }
     }
 
@@ -1114,19 +1149,19 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     // last occupant was tile T - 2, which every wave had finished before the barrier of the last
     // iteration, and no copy into it is in flight, so no further barrier is needed and a wave
     // that is done early stores early.
-    const float l_tot = xhalf_sum(l_run);
-    const float inv = (l_tot > 0.f) ? 1.0f / l_tot : 0.f;
+    const RowPair inv_of = of_rows(__builtin_bit_cast(uint32_t, l_row > 0.f ? 1.0f / l_row : 0.f));
+    const float inv[2] = {__builtin_bit_cast(float, inv_of.w[0]), __builtin_bit_cast(float, inv_of.w[1])};
     {
         const int row0 = row_base;
         const uint32_t ebase = SPLIT ? lds0 : HALVES ? lds0 + 2 * HALF_SUMS + wave * 4096 : lds0 + (uint32_t)(visits & 1) * STAGE_BYTES + wave * 4096;
-        store_rows<BF16, OB>(oacc, inv, ebase, SPLIT ? 4096 : HALVES ? 8192 : 16384, block_dst(a.out, a.out32, bi, hi, row0, D), a.out.p != nullptr,
+        store_rows16<BF16>(oacc, inv, ebase, SPLIT ? 4096 : HALVES ? 8192 : 16384, block_dst(a.out, a.out32, bi, hi, row0, D), a.out.p != nullptr,
                              BF16 && a.out32.p != nullptr, row0, N, lane);       // fp32 callers compute in bf16
     }
     if (qrow < N) {
         if (a.lse != nullptr && hh == 0) {
             // log2 of the row's sum of exp(scale * score) is pm * r + log2(l)
             a.lse[(size_t)bh * N + qrow] =
-                (l_tot > 0.f) ? __builtin_fmaf(pm * ref, 0.6931471805599453f, __builtin_logf(l_tot)) : -__builtin_inff();
+                (l_row > 0.f) ? __builtin_fmaf(pm * ref, 0.6931471805599453f, __builtin_logf(l_row)) : -__builtin_inff();
             // (an explicit fma: left to the compiler, the sum was contracted in some instantiations of
             // this kernel and not in others, and their lse differed in the last bit)
         }
