@@ -170,11 +170,11 @@ __device__ __forceinline__ void dq_rows(const AttnBwdArgs &a, unsigned char *sme
         const int qrow = qt * BM + wave * 32 + 16 * qb_ + l16;
         const int qr = qrow < N ? qrow : N - 1;
         u32x4 of[KS];
-        load_row16(qf[qb_], qb, a.q.sn, qr, q4, a.D);
-        load_row16(dof[qb_], dob, a.dout.sn, qr, q4, a.D);
+        load_row(qf[qb_], qb, a.q.sn, qr, q4, a.D);
+        load_row(dof[qb_], dob, a.dout.sn, qr, q4, a.D);
         float delta = 0.f, d2[2] = {0.f, 0.f};
         if constexpr (HAVE_DELTA) delta = a.delta[(size_t)bh * N + qr];
-        else load_row16(of, ob, a.out.sn, qr, q4, a.D);
+        else load_row(of, ob, a.out.sn, qr, q4, a.D);
 #pragma unroll
         for (int s = 0; s < KS; ++s)
 #pragma unroll
@@ -242,7 +242,7 @@ __device__ __forceinline__ void dq_rows(const AttnBwdArgs &a, unsigned char *sme
     const uint32_t lut_addr = lds0 + OFF_LUT;
     const uint32_t nib_rotate = (4u * q4 + 28u) & 31u;     // right: the nibble of keys 4q4 .. 4q4 + 3 comes to bits 4 .. 7
 
-    uint32_t row_at = make_tile_read16(lane).row, col_at = make_tile_read16(lane).col;
+    uint32_t row_at = make_tile_read(lane).row, col_at = make_tile_read(lane).col;
     // one key tile; the ring stage is a compile-time constant, as in the dK/dV kernel, so that every LDS address is a register plus an
     // immediate.  4 x 32 heads, N = 4096, D = 128: 1275 us, 1.29 PFLOP/s, the matrix cores busy two thirds of the time at 1.86 GHz
     auto tile = [&](int t, int t_next, auto st_c) __attribute__((always_inline)) {
@@ -321,7 +321,7 @@ __device__ __forceinline__ void dq_rows(const AttnBwdArgs &a, unsigned char *sme
             if (n >= 4 * PH) {
                 const int k = n - 4 * PH, b = k % DB;
 #pragma unroll
-                for (int x = 0; x < 2; ++x) oacc[x][b] = E::mfma16(r, pb[k / DB][x], oacc[x][b]);
+                for (int x = 0; x < 2; ++x) oacc[x][b] = E::mfma(r, pb[k / DB][x], oacc[x][b]);
                 if (k < DB) {
 #pragma unroll
                     for (int i = 0; i < (8 + DB - 1) / DB; ++i)
@@ -329,7 +329,7 @@ __device__ __forceinline__ void dq_rows(const AttnBwdArgs &a, unsigned char *sme
                 }
             } else if (ph == 0 || ph == 2) {
 #pragma unroll
-                for (int x = 0; x < 2; ++x) sacc[blk][kb][x] = E::mfma16(r, qf[x][c], sacc[blk][kb][x]);
+                for (int x = 0; x < 2; ++x) sacc[blk][kb][x] = E::mfma(r, qf[x][c], sacc[blk][kb][x]);
                 if (ph == 2) {
 #pragma unroll
                     for (int i = 0; i < (8 + PH - 1) / PH; ++i)
@@ -337,7 +337,7 @@ __device__ __forceinline__ void dq_rows(const AttnBwdArgs &a, unsigned char *sme
                 }
             } else {
 #pragma unroll
-                for (int x = 0; x < 2; ++x) dacc[blk][kb][x] = E::mfma16(r, dof[x][c], c == 0 ? from_delta[x] : dacc[blk][kb][x]);
+                for (int x = 0; x < 2; ++x) dacc[blk][kb][x] = E::mfma(r, dof[x][c], c == 0 ? from_delta[x] : dacc[blk][kb][x]);
 #pragma unroll
                 for (int i = 0; i < (16 + PH - 1) / PH; ++i)
                     if (m * ((16 + PH - 1) / PH) + i < 16) weight(blk, m * ((16 + PH - 1) / PH) + i);
@@ -356,7 +356,7 @@ __device__ __forceinline__ void dq_rows(const AttnBwdArgs &a, unsigned char *sme
     __syncthreads();              // every wave is done reading the stages
     const int row0 = qt * BM + wave * 32;
     if (row0 < N) {
-        store_gradient16<BF16, WIDE>(oacc, a.scale, lds0 + wave * 4096, a, a.dq, bi, hi, row0, lane);
+        store_gradient<BF16, WIDE>(oacc, a.scale, lds0 + wave * 4096, a, a.dq, bi, hi, row0, lane);
     }
 }
 
@@ -438,8 +438,8 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
     for (int kb = 0; kb < 2; ++kb) {
         const int key = key0 + 16 * kb + l16;         // a key beyond N has sums that are not stored
         u32x4 v_all[KS];
-        load_row16(kf[kb], kb_, a.k.sn, key < N ? key : N - 1, q4, a.D);
-        load_row16(v_all, vb, a.v.sn, key < N ? key : N - 1, q4, a.D);
+        load_row(kf[kb], kb_, a.k.sn, key < N ? key : N - 1, q4, a.D);
+        load_row(v_all, vb, a.v.sn, key < N ? key : N - 1, q4, a.D);
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
 #pragma unroll
@@ -505,7 +505,7 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
     aux_words += 128 * half;
     if constexpr (VLDS || OFF_AUX >= 65536) asm volatile("" : "+v"(aux_rows), "+v"(aux_words), "+v"(aux_lane));
 
-    uint32_t row_at = make_tile_read16(lane).row + 4096 * half, col_at = make_tile_read16(lane).col + 4096 * half;
+    uint32_t row_at = make_tile_read(lane).row + 4096 * half, col_at = make_tile_read(lane).col + 4096 * half;
     // one q tile; the ring stage is a compile-time constant so that every LDS address of the body is
     // a register plus an immediate
     auto tile = [&](int t, int t_next, auto st_c) __attribute__((always_inline)) {
@@ -593,10 +593,10 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
                 const u32x4 &r = ring[n % (AHEAD + 1)];
                 if (n < PH) {
 #pragma unroll
-                    for (int kb = 0; kb < 2; ++kb) sacc[rb][kb] = E::mfma16(r, kf[kb][c], sacc[rb][kb]);
+                    for (int kb = 0; kb < 2; ++kb) sacc[rb][kb] = E::mfma(r, kf[kb][c], sacc[rb][kb]);
                 } else if (n < 2 * PH) {
 #pragma unroll
-                    for (int kb = 0; kb < 2; ++kb) dacc[rb][kb] = E::mfma16(r, vs[c & 1][kb], dacc[rb][kb]);
+                    for (int kb = 0; kb < 2; ++kb) dacc[rb][kb] = E::mfma(r, vs[c & 1][kb], dacc[rb][kb]);
 #pragma unroll
                     for (int i = 0; i < (16 + PH - 1) / PH; ++i) {
                         const int e = m * ((16 + PH - 1) / PH) + i, er = e >> 3, ek = (e >> 2) & 1, j = e & 3;
@@ -617,7 +617,7 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
                 } else if (n < 2 * PH + DB) {          // dV^T += dO^T P
                     const int b = n - 2 * PH;
 #pragma unroll
-                    for (int kb = 0; kb < 2; ++kb) dvacc[kb][b] = E::mfma16(r, pp[kb], dvacc[kb][b]);
+                    for (int kb = 0; kb < 2; ++kb) dvacc[kb][b] = E::mfma(r, pp[kb], dvacc[kb][b]);
 #pragma unroll
                     for (int q = 0; q < (8 + DB - 1) / DB; ++q) {
                         const int i = b * ((8 + DB - 1) / DB) + q, ir = i >> 2, ik = (i >> 1) & 1, j = 2 * (i & 1);
@@ -627,7 +627,7 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
                 } else {                               // dK^T += Q^T dS
                     const int b = n - 2 * PH - DB;
 #pragma unroll
-                    for (int kb = 0; kb < 2; ++kb) dkacc[kb][b] = E::mfma16(r, ps[kb], dkacc[kb][b]);
+                    for (int kb = 0; kb < 2; ++kb) dkacc[kb][b] = E::mfma(r, ps[kb], dkacc[kb][b]);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -668,15 +668,15 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
                 }
         };
         add(dkacc, sums);
-        store_gradient16<BF16, WIDE>(dkacc, a.scale, lds0 + wave * (DB * 4096), a, a.dk, bi, hi, key0, lane);      // over its own sums
+        store_gradient<BF16, WIDE>(dkacc, a.scale, lds0 + wave * (DB * 4096), a, a.dk, bi, hi, key0, lane);      // over its own sums
         __builtin_amdgcn_sched_barrier(0);
         add(dvacc, sums + DB * 2048);
-        store_gradient16<BF16, WIDE>(dvacc, 1.0f, lds0 + wave * (DB * 4096), a, a.dv, bi, hi, key0, lane);
+        store_gradient<BF16, WIDE>(dvacc, 1.0f, lds0 + wave * (DB * 4096), a, a.dv, bi, hi, key0, lane);
         return;
     }
     if (wave_valid) {
-        store_gradient16<BF16, WIDE>(dkacc, a.scale, lds0 + wave * 4096, a, a.dk, bi, hi, key0, lane);
-        store_gradient16<BF16, WIDE>(dvacc, 1.0f, lds0 + wave * 4096, a, a.dv, bi, hi, key0, lane);
+        store_gradient<BF16, WIDE>(dkacc, a.scale, lds0 + wave * 4096, a, a.dk, bi, hi, key0, lane);
+        store_gradient<BF16, WIDE>(dvacc, 1.0f, lds0 + wave * 4096, a, a.dv, bi, hi, key0, lane);
     }
 }
 

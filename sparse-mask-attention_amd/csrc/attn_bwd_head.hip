@@ -4,8 +4,9 @@
 // S, dP and the exponentials are formed once where the two kernels of attn_bwd.hip form them twice (five N x N x D products
 // instead of seven), q, k, v and dO come from memory once, and there is one launch.  No sums between work-groups:
 // bit-reproducible.
-//   wavefront    32 KB keys, KB = 1 or 2 (lane = key, as in the dK/dV kernel); dK and dV are its accumulators, V fragments stay in
-//                registers.  With KB = 2 every Q and dO operand that is read from LDS serves two products.
+//   wavefront    32 KB keys, KB = 1 or 2, products of 16 x 16 x 32 (a lane has the keys lane % 16 and 16 more, as in the dK/dV kernel); dK and dV
+//                are its accumulators, V fragments stay in registers.  Every operand that is read from LDS serves two products, those of dV
+//                and dK 2 KB.
 //   rows         32 at a time, in a ring of two stages: Q, dO, the mask words of each wavefront's keys.  The wavefront that has copied
 //                eight rows also forms their delta (O comes with them) and Q scaled and rounded as the forward does it, so that
 //                the probabilities fit its lse, in the place of O.  Delta of all rows before the first, as the two kernels have it,
@@ -15,9 +16,9 @@
 //   dS           to LDS as [key][row], 64 bytes a key; after the next barrier the wavefronts share dQ^T = K^T dS^T of the 32 rows
 //                in blocks of 16 x 16.  Eight wavefronts have two such buffers and one barrier for 32 rows; four have one,
 //                so that two work-groups share a CU, and two barriers.
-// Swizzles: Q and dO as everywhere in the backward (bitrev3 of row / 2), K by 16 bytes with the bits of row / 2 in the order (2, 0, 1)
-// and dS by 8 bytes with those of key / 4 in the order (1, 2, 0): their row accesses and the transposing reads of 16 keys x 16
-// columns that dQ needs are free of bank conflicts (2.3 cycles a read on a full CU, 2.1 for a linear one).
+// Swizzles: Q and dO as everywhere in the backward (swizzle16 of row / 2), K by 16 bytes with the bits (2 ^ 1, 0, 1) of row / 2
+// and dS by 8 bytes with the bits (1, 0, 2) of key / 4: the row accesses (see swizzle16) and the transposing reads of 16 keys x 16
+// columns that dQ needs, keys 8q4 + 0 .. 3 and then + 4 .. 7 of the sixteens q4, stay free of bank conflicts.
 //
 // The backward alone, inputs in turn, in us, before (two kernels, up to 256 keys at head dims up to 64 an earlier form of this
 // one) -> now:
@@ -25,10 +26,17 @@
 //             2048 heads, N = 32: 26.6 -> 20.0
 //   D = 128   N = 256: 256 heads 54.0 -> 40.4, 1024: 212 -> 156;  1024 heads: N = 128 98.8 -> 64.3, N = 64 54.9 -> 31.9
 //   D =  32   1024 heads, N = 256: 66.1 -> 53.7;  192, N = 512: 45.3 -> 39.8;   D = 96   1024 heads, N = 128: 57.1 -> 48.1
-// What bounds it: on 256 heads, N = 512, D = 64 (66 us) a SIMD's 5800 cycles for 32 rows hold 2560 of the matrix cores, about 2700 of the
-// vector ALU and, for the CU, 3200 of LDS; the barrier keeps the eight wavefronts in the same phase, which is bound by one of them at a
-// time.  Starting half of the wavefronts with dQ and half with S changed nothing.  Prologue and epilogue, some 20000 cycles
-// of 130000, move 256 KB of every CU at what memory gives.
+// Products of 32 x 32 x 16 and exp2(fma(s, post_mul, -lse)) -> products of 16 x 16 x 32, the exponentials of one block of keys beside the products of
+// dP and dS beside dV's, accumulators that start from -lse, no multiplication where post_mul is 1 (the backward alone, us):
+//   D =  64   N = 512: 192 heads 52.1 -> 50.1, 256 58.6 -> 55.1, causal 49.2 -> 46.7;  640, N = 400: 131.9 -> 123.5;  1024, N = 256, causal 62.7 ->
+//             60.8;  1024, N = 128 28.2 -> 26.9;  192, N = 512, blocks 45.6 -> 42.7
+//   D = 128   1024 heads, N = 256 154 -> 146, 256 35.6 -> 34.1;  up to 128 keys, bound by memory, the same (1024, N = 128 50.3, 50.4)
+//   D =  32   192 heads, N = 512 37.6 -> 36.4;  1024, N = 256 47.0 -> 45.3
+// What bounds it: on 192 heads, N = 512, D = 64 some 5900 cycles for 32 rows: dQ's 16 products a wavefront 1400 to 2000 of them (LDS round trips and, for the
+// wavefronts that copy, the addresses of the mask words, 64 lines a copy), S to dK 4000 (of a SIMD's two wavefronts 2050 cycles of products, 1800 of vector ALU,
+// and LDS round trips that no registers are left to hide), the rest for delta, scaling and the barrier.  Starting half of the wavefronts with
+// dQ and half with S changed nothing; nor did four or six of dQ's operands on their way instead of two (57.2 us with the registers it took).  Prologue
+// and epilogue, some 20000 cycles of 115000, move 256 KB of every CU at what memory gives.
 #include <type_traits>
 
 #include "attn_bwd_common.h"
@@ -54,37 +62,29 @@ template <int HDIM, int NW, int KB> struct HeadCfg {
     static constexpr int LDS_BYTES = OFF_LIVE + 64;
 };
 
-// 16 x 16 x 32 products
-template <bool BF16> __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c)
-{
-    if constexpr (BF16)
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-}
 __device__ __forceinline__ u32x4 tr_pair(uint32_t lo, uint32_t hi)
 {
     const u32x2 x = lds_read_tr16_b64(lo), y = lds_read_tr16_b64(hi);
     return u32x4{x.x, x.y, y.x, y.y};
 }
 
-template <bool BF16, int HDIM, int NW, int KB, bool WIDE>
+template <bool BF16, int HDIM, int NW, int KB, bool POSTMUL, bool WIDE>
 __global__ __launch_bounds__(64 * NW, HDIM <= 64 && KB == 1 && NW == 4 ? 3 : 2) void attn_bwd_head_kernel(const AttnBwdArgs a)
 {
     using E = Elem<BF16>;
     using C = HeadCfg<HDIM, NW, KB>;
-    constexpr int NH = C::NH, KS = HDIM / 16, OB = HDIM / 32;
+    constexpr int NH = C::NH, KS = HDIM / 32, DB = HDIM / 16;
     __shared__ __attribute__((aligned(1024))) unsigned char smem[C::LDS_BYTES];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(LDS_PTR(unsigned char))smem;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int l32 = lane & 31, hh = lane >> 5;
+    const int l16 = lane & 15, q4 = lane >> 4;
     const int bh = renumber_block();
     const int N = a.N, nw = (N + 31) >> 5;
     const int RB = (N + 31) >> 5;                     // blocks of 32 rows
-    const float pm = a.post_mul;
+    const float pm = POSTMUL ? a.post_mul : 1.0f, lse_mul = -LOG2E / pm;        // pm is a power of two: exact
 
     const int bi = (int)fastdiv((uint32_t)bh, a.div_H), hi = bh - bi * a.H;
     const uint16_t *qb = slab(a.q, bi, hi), *dob = slab(a.dout, bi, hi), *ob = slab(a.out, bi, hi);
@@ -94,7 +94,7 @@ __global__ __launch_bounds__(64 * NW, HDIM <= 64 && KB == 1 && NW == 4 ? 3 : 2) 
     // ---- copies
     const int last_chunk = (a.D >> 3) - 1;
     auto chunk_at = [&](int c) __attribute__((always_inline)) -> uint32_t { return (uint32_t)(c < last_chunk ? c : last_chunk) << 4; };
-    auto k_swizzle = [](int row) __attribute__((always_inline)) { const int p = (row >> 1) & 7; return (p & 4) | ((p & 1) << 1) | ((p >> 1) & 1); };
+    auto k_swizzle = [](int row) __attribute__((always_inline)) { const int p = (row >> 1) & 7; return ((p ^ (p << 1)) & 4) | ((p & 1) << 1) | ((p >> 1) & 1); };
     const int key0 = wave * (32 * KB);                // this wavefront's keys
     const bool wave_valid = key0 < N;                 // wave-uniform
     const int part = wave & 3;
@@ -104,7 +104,7 @@ __global__ __launch_bounds__(64 * NW, HDIM <= 64 && KB == 1 && NW == 4 ? 3 : 2) 
         int ln = lane;
         asm volatile("" : "+v"(ln));                  // the few sums below are made again each time instead of kept
         const int prow = 8 * part + (ln >> 3);        // the row of a stage that this lane copies 16 bytes of
-        const int pc = (ln & 7) ^ bitrev3((prow >> 1) & 7);
+        const int pc = (ln & 7) ^ swizzle16((prow >> 1) & 7);
         const uint32_t pchunk = chunk_at(pc), pchunk2 = chunk_at(8 + pc);
         const int row = 32 * i + prow < N ? 32 * i + prow : N - 1;
         auto rows = [&](auto off_c, const uint16_t *mat, uint32_t sn) __attribute__((always_inline)) {
@@ -143,39 +143,36 @@ __global__ __launch_bounds__(64 * NW, HDIM <= 64 && KB == 1 && NW == 4 ? 3 : 2) 
     issue(0, std::integral_constant<int, 0>{});
 
     // ---- V^T fragments of this lane's keys
-    u32x4 vf[KB][KS];
+    u32x4 vf[2 * KB][KS];                             // blocks of 16 keys
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
-        const int key = key0 + 32 * kb + l32, kr = key < N ? key : N - 1;
+    for (int k = 0; k < 2 * KB; ++k) {
+        const int key = key0 + 16 * k + l16, kr = key < N ? key : N - 1;
         const uint16_t *vp = vb + (size_t)kr * a.v.sn;
 #pragma unroll
-        for (int s = 0; s < KS; ++s) {                // columns beyond the row's end: its last ones, set to zero
-            const int col = 16 * s + 8 * hh;
-            vf[kb][s] = *reinterpret_cast<const u32x4 *>(vp + (col < a.D ? col : a.D - 8)) & (col < a.D ? 0xffffffffu : 0u);
+        for (int c = 0; c < KS; ++c) {                // columns beyond the row's end: its last ones, set to zero
+            const int col = 32 * c + 8 * q4;
+            vf[k][c] = *reinterpret_cast<const u32x4 *>(vp + (col < a.D ? col : a.D - 8)) & (col < a.D ? 0xffffffffu : 0u);
         }
     }
     if (tid < 16) *(LDS_PTR(uint32_t))(uintptr_t)(lds0 + C::OFF_LIVE + 4 * tid) = 0u;
     const bool keys_end = key0 + 32 * KB > N;         // wave-uniform: some of this wavefront's keys do not exist
 
-    f32x16 dkacc[KB][OB], dvacc[KB][OB];
+    f32x4 dkacc[KB][2][DB], dvacc[KB][2][DB];
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-        for (int b = 0; b < OB; ++b)
+        for (int k = 0; k < 2; ++k)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                dkacc[kb][b][i] = 0.f;
-                dvacc[kb][b][i] = 0.f;
-            }
+            for (int b = 0; b < DB; ++b) dkacc[kb][k][b] = dvacc[kb][k][b] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     // ---- read addresses
     // One register per pattern: a step along a row flips bits of the swizzled chunk, eight (four) rows further down flip
     // another and add their bytes; the rest is an immediate.
-    uint32_t row_at = lds0 + C::OFF_STAGE + make_tile_read(lane).rowaddr[0], col_at = lds0 + C::OFF_STAGE + make_tile_read(lane).traddr[0][0];
-    uint32_t key_at = lds0 + (key0 + l32) * 128 + ((hh ^ k_swizzle(l32)) << 4);
-    auto ds_swizzle = [](int key) __attribute__((always_inline)) { const int x = key >> 2; return ((x & 2) << 1) | ((x & 4) >> 1) | (x & 1); };
-    uint32_t ds_at = lds0 + C::OFF_DS + (key0 + l32) * 64 + ((hh ^ ds_swizzle(l32)) << 3);
-    uint32_t half_at = lds0 + 16 * hh, lane_at = lds0 + 4 * lane;      // rows 8g + 4hh .. of the small data; this lane's word
+    uint32_t row_at = lds0 + C::OFF_STAGE + make_tile_read(lane).row, col_at = lds0 + C::OFF_STAGE + make_tile_read(lane).col;
+    uint32_t key_at = lds0 + (key0 + l16) * 128 + ((q4 ^ k_swizzle(l16)) << 4);
+    auto ds_swizzle = [](int key) __attribute__((always_inline)) { const int x = key >> 2; return ((x & 3) << 1) | ((x >> 2) & 1); };
+    uint32_t ds_at = lds0 + C::OFF_DS + (key0 + l16) * 64 + ((q4 ^ ds_swizzle(l16)) << 3);
+    uint32_t part_at = lds0 + 16 * q4, lane_at = lds0 + 4 * lane;      // rows 4q4 .. of the small data; this lane's word
 
     // dQ^T = K^T dS^T in blocks of 16 columns x 16 rows
     constexpr int NDB = HDIM / 16;
@@ -205,7 +202,7 @@ __global__ __launch_bounds__(64 * NW, HDIM <= 64 && KB == 1 && NW == 4 ? 3 : 2) 
         if (wave < 4) {
             int ln = lane;
             asm volatile("" : "+v"(ln));
-            const int prow = 8 * part + (ln >> 3), chunk = (ln & 7) ^ bitrev3((prow >> 1) & 7);
+            const int prow = 8 * part + (ln >> 3), chunk = (ln & 7) ^ swizzle16((prow >> 1) & 7);
             const uint32_t at = lds0 + 16 * ln + (SO + part * 1024);
             float delta = 0.f;
 #pragma unroll
@@ -234,7 +231,7 @@ __global__ __launch_bounds__(64 * NW, HDIM <= 64 && KB == 1 && NW == 4 ? 3 : 2) 
             const uint32_t at = lane_at + (SO + C::OFF_LSE);
             const float l = *(LDS_PTR(float))(uintptr_t)at;
             // rows that kept nothing or lie beyond N: probability 0
-            *(LDS_PTR(float))(uintptr_t)at = 32 * i + lane >= N || l == -__builtin_inff() ? -__builtin_inff() : -l * LOG2E;
+            *(LDS_PTR(float))(uintptr_t)at = 32 * i + lane >= N || l == -__builtin_inff() ? -__builtin_inff() : l * lse_mul;
         }
     };
     // ---- 32 query rows: dV, dK, and dS into LDS
@@ -243,8 +240,8 @@ __global__ __launch_bounds__(64 * NW, HDIM <= 64 && KB == 1 && NW == 4 ? 3 : 2) 
         constexpr int DS = C::DS_BUFS == 2 ? st * C::DS_BYTES : 0;
         constexpr int SB = st * C::STAGE_BYTES;
         // opaque: the compiler would keep a register for every address that follows from these
-        asm volatile("" : "+v"(row_at), "+v"(col_at), "+v"(key_at), "+v"(ds_at), "+v"(half_at), "+v"(lane_at));
-        const uint32_t word_at = lane_at + (C::OFF_STAGE + SB + C::OFF_WORDS + wave * 256), words_at = half_at + (C::OFF_STAGE + SB + C::OFF_WORDS + wave * 256);
+        asm volatile("" : "+v"(row_at), "+v"(col_at), "+v"(key_at), "+v"(ds_at), "+v"(part_at), "+v"(lane_at));
+        const uint32_t word_at = lane_at + (C::OFF_STAGE + SB + C::OFF_WORDS + wave * 256), words_at = part_at + (C::OFF_STAGE + SB + C::OFF_WORDS + wave * 256);
         uint32_t word = *(LDS_PTR(const uint32_t))(uintptr_t)(word_at);
         if (keys_end) {                               // nothing is kept of keys beyond N, whatever their bits
             int ln = lane;
@@ -253,125 +250,120 @@ __global__ __launch_bounds__(64 * NW, HDIM <= 64 && KB == 1 && NW == 4 ? 3 : 2) 
             word &= left >= 32 ? 0xffffffffu : left > 0 ? (1u << left) - 1u : 0u;
             *(LDS_PTR(uint32_t))(uintptr_t)(word_at) = word;
         }
+        // Steps of two products (four where both blocks of 32 keys take part), kb = 0, 1 in turn: S (PH of them), dP (as many); then dV and dK (DB
+        // each).  Operands are requested AHEAD steps before their use, and scheduling barriers hold that order: left alone, the compiler
+        // requests each just before it is needed, since registers are short, and the wavefront sits out some 30 LDS round
+        // trips one after the other.  The eight wavefronts go through these phases together, so what a wavefront's vector ALU does beside its own
+        // products counts: the exponentials of kb lie in its dP, its dS in the S of the next or in dV.
+        constexpr int PH = 2 * KS, SCORES = 2 * PH * KB, STEPS = SCORES + 2 * DB, AHEAD = KB == 2 ? HDIM == 64 ? 1 : 2 : 3;
+        const uint32_t rows = part_at + (C::OFF_STAGE + SB + C::OFF_LSE);
+        u32x4 ring[AHEAD + 1], kf[2][2];
+        auto fetch = [&](int n) __attribute__((always_inline)) {
+            u32x4 &r = ring[n % (AHEAD + 1)];
+            if (n < SCORES) {                             // row block m & 1, columns 32 (m >> 1) of Q or dO
+                const int m = n % PH, dp = n / PH & 1;
+                r = lds_read_b128((row_at ^ (64 * ((m >> 1) & 1))) + SB + (dp ? C::PART : C::LAND ? 2 * C::PART : 0) + (m >> 2) * 4096 + 2048 * (m & 1));
+            } else if (n < STEPS) {                       // dO^T, then Q^T, 16 columns
+                const int b = (n - SCORES) % DB;
+                const uint32_t at = (col_at ^ (32 * (b & 3))) + SB + (n - SCORES < DB ? C::PART : 0) + (b >> 2) * 4096;
+                r = tr_pair(at, at + 2048);
+            }
+        };
+        auto fetch_k = [&](int kb, int c) __attribute__((always_inline)) {
+#pragma unroll
+            for (int k = 0; k < 2; ++k) kf[c & 1][k] = lds_read_b128((key_at ^ (64 * (c & 1))) + (c >> 1) * C::K_HALF + 4096 * kb + 2048 * k);
+        };
+        u32x4 mw[2];                                      // mask words of 16 rows
+        f32x4 sacc[KB][2][2], dacc[KB][2][2];             // [kb][rb][k]: rows 16rb + 4q4 + j, key 32kb + 16k + l16
+        u32x4 pp[KB][2], ps[KB][2];
+        auto weight = [&](int kb, int e) __attribute__((always_inline)) {           // element e of 16
+            const int rb = e >> 3, k = (e >> 2) & 1, j = e & 3;
+            const uint32_t keep = (uint32_t)__builtin_amdgcn_sbfe((int)mw[rb][j], (uint32_t)(l16 + 16 * k), 1u);
+            const float x = __builtin_amdgcn_exp2f(POSTMUL ? sacc[kb][rb][k][j] * pm : sacc[kb][rb][k][j]);
+            float p = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & keep);
+            asm volatile("" : "+v"(p));                   // here: the compiler would keep both operands of all 16 for the first use
+            sacc[kb][rb][k][j] = p;
+        };
+        auto pack_weights = [&](int kb, int i) __attribute__((always_inline)) {     // pair i of 8
+            const int rb = i >> 2, k = (i >> 1) & 1, j = 2 * (i & 1);
+            pp[kb][k][2 * rb + (i & 1)] = E::pack2_rne(sacc[kb][rb][k][j], sacc[kb][rb][k][j + 1]);
+        };
+        auto dscore = [&](int kb, int i) __attribute__((always_inline)) {
+            const int rb = i >> 2, k = (i >> 1) & 1, j = 2 * (i & 1);
+            ps[kb][k][2 * rb + (i & 1)] = E::pack2_rne(sacc[kb][rb][k][j] * dacc[kb][rb][k][j], sacc[kb][rb][k][j + 1] * dacc[kb][rb][k][j + 1]);
+            if (i & 1)
+                *(LDS_PTR(u32x2))(uintptr_t)((ds_at ^ (32 * rb + 8 * k)) + DS + 2048 * kb + 1024 * k) = u32x2{ps[kb][k][2 * rb], ps[kb][k][2 * rb + 1]};
+        };
+        // the accumulators start from -lse (over pm) and -delta: the products leave s - lse and dP - delta, with no addition per element
+        auto from_lse = [&](int kb) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) sacc[kb][i][0] = sacc[kb][i][1] = __builtin_bit_cast(f32x4, lds_read_b128(rows + 64 * i));
+        };
+        if (NW == 8) __builtin_amdgcn_s_setprio(0);
+        from_lse(0);
+        fetch_k(0, 0);
+#pragma unroll
+        for (int n = 0; n < AHEAD; ++n) fetch(n);
+        __builtin_amdgcn_sched_barrier(0);                // requested before the words are looked at
         const bool live = __builtin_amdgcn_ballot_w64(word != 0u) != 0ull;         // dQ leaves out the others
         if (lane == 0) *(LDS_PTR(uint32_t))(uintptr_t)(lds0 + C::OFF_LIVE + (C::DS_BUFS == 2 ? 32 * st : 0) + 4 * wave) = live ? 1u : 0u;
         if (!live) return;
-        // Operands are requested a step ahead of their use, and scheduling barriers hold that order: left alone, the compiler
-        // requests each just before it is needed, since registers are short, and the wavefront sits out some 30 LDS round
-        // trips one after the other.
-        const uint32_t rows = half_at + (C::OFF_STAGE + SB + C::OFF_LSE);
-        auto q_frag = [&](int s) __attribute__((always_inline)) { return lds_read_b128((row_at ^ (32 * (s & 3))) + SB + (C::LAND ? 2 * C::PART : 0) + (s >> 2) * 4096); };
-        auto o_frag = [&](int s) __attribute__((always_inline)) { return lds_read_b128((row_at ^ (32 * (s & 3))) + SB + C::PART + (s >> 2) * 4096); };
-        auto k_frag = [&](int s, int kb) __attribute__((always_inline)) { return lds_read_b128((key_at ^ (32 * (s & 3))) + (s >> 2) * C::K_HALF + kb * 4096); };
-        auto mask_of = [&](int kb, int g) __attribute__((always_inline)) { return lds_read_b128(words_at + 128 * kb + 32 * g); };
-        auto lse_of = [&](int g) __attribute__((always_inline)) { return lds_read_b128(rows + 32 * g); };
-        f32x16 sacc[KB], dacc[KB];
-        auto from_delta = [&](int kb) __attribute__((always_inline)) {
+        static_assert(C::LAND || KB == 1, "one S of rows as they are");
+        if constexpr (!C::LAND) ring[0] = scaled(ring[0]);
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const u32x4 Dr = lds_read_b128(rows + (C::OFF_DELTA - C::OFF_LSE) + 32 * g);
+        for (int n = 0; n < STEPS; ++n) {
+            fetch(n + AHEAD);
+            const int kb = n / (2 * PH), m = n % PH, rb = m & 1, c = m >> 1;
+            const bool dp = n / PH & 1;
+            if (n < SCORES) {
+                if (!dp && rb == 0 && c + 1 < KS) fetch_k(kb, c + 1);
+                if (dp && kb + 1 < KB && m == PH - 1) fetch_k(kb + 1, 0);
+                if (!dp && m == PH - 2) {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) dacc[kb][4 * g + j] = __builtin_bit_cast(float, (uint32_t)Dr[j]);
-            }
-        };
-        if (NW == 8) __builtin_amdgcn_s_setprio(0);
-        u32x4 raw[2], qf[2], kf[2][KB], of[2], mg[2], Lr[2];
-        if constexpr (C::LAND) {
-            qf[0] = q_frag(0);
-        } else {
-            raw[0] = q_frag(0);
-            raw[1] = q_frag(1);
-        }
-#pragma unroll
-        for (int kb = 0; kb < KB; ++kb) {
-            kf[0][kb] = k_frag(0, kb);
-#pragma unroll
-            for (int e = 0; e < 16; ++e) sacc[kb][e] = 0.f;
-        }
-#pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            if constexpr (!C::LAND) qf[s & 1] = scaled(raw[s & 1]);
-            if (s + 1 < KS) {
-                if constexpr (C::LAND) qf[(s + 1) & 1] = q_frag(s + 1);
-                else if (s + 2 < KS) raw[s & 1] = q_frag(s + 2);
-#pragma unroll
-                for (int kb = 0; kb < KB; ++kb) kf[(s + 1) & 1][kb] = k_frag(s + 1, kb);
-            } else {
-                from_delta(0);
-                of[0] = o_frag(0);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int kb = 0; kb < KB; ++kb) sacc[kb] = E::mfma(qf[s & 1], kf[s & 1][kb], sacc[kb]);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            if (s + 1 < KS) {
-                of[(s + 1) & 1] = o_frag(s + 1);
-            } else {
-                mg[0] = mask_of(0, 0);
-                Lr[0] = lse_of(0);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            dacc[0] = E::mfma(of[s & 1], vf[0][s], dacc[0]);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        // P and dS, four rows at a time; with two blocks of keys the second's dP in the midst of the first's
-        uint32_t pp[KB][2][4], ps[KB][2][4];
-        u32x4 qa[2], oa[2];
-        auto columns = [&](int n) __attribute__((always_inline)) {           // Q^T and dO^T operands of the n-th pair of products
-            const int u = n / OB, b = n % OB, at = SB + 2048 * u + (b >> 1) * 4096;
-            const uint32_t c0 = col_at ^ (64 * (b & 1)), c1 = col_at ^ (64 * (b & 1) + 16);
-            oa[n & 1] = tr_pair(c0 + at + C::PART, c1 + at + 1024 + C::PART);
-            qa[n & 1] = tr_pair(c0 + at, c1 + at + 1024);
-        };
-#pragma unroll
-        for (int n = 0; n < 4 * KB; ++n) {
-            const int kb = n / 4, g = n % 4;
-            if (n + 1 < 4 * KB) {
-                mg[(n + 1) & 1] = mask_of((n + 1) / 4, (n + 1) % 4);
-                Lr[(n + 1) & 1] = lse_of((n + 1) % 4);
-            } else {
-                columns(0);
-            }
-            if (KB == 2 && n == 3) of[0] = o_frag(0);
-            __builtin_amdgcn_sched_barrier(0);
-            float p[4], d[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t keep = (uint32_t)__builtin_amdgcn_sbfe((int)mg[n & 1][j], (uint32_t)lane, 1u);       // bit lane % 32
-                const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[kb][4 * g + j], pm, __builtin_bit_cast(float, (uint32_t)Lr[n & 1][j])));
-                p[j] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, e) & keep);
-                d[j] = p[j] * dacc[kb][4 * g + j];
-            }
-            pp[kb][g >> 1][2 * (g & 1)] = E::pack2_rne(p[0], p[1]);
-            pp[kb][g >> 1][2 * (g & 1) + 1] = E::pack2_rne(p[2], p[3]);
-            const u32x2 ds = {E::pack2_rne(d[0], d[1]), E::pack2_rne(d[2], d[3])};
-            ps[kb][g >> 1][2 * (g & 1)] = ds.x;
-            ps[kb][g >> 1][2 * (g & 1) + 1] = ds.y;
-            *(LDS_PTR(u32x2))(uintptr_t)((ds_at ^ (16 * g)) + DS + 2048 * kb) = ds;
-            __builtin_amdgcn_sched_barrier(0);
-            if (KB == 2 && n == 3) {
-                from_delta(KB - 1);
-#pragma unroll
-                for (int s = 0; s < KS; ++s) {
-                    if (s + 1 < KS) of[(s + 1) & 1] = o_frag(s + 1);
-                    __builtin_amdgcn_sched_barrier(0);
-                    dacc[KB - 1] = E::mfma(of[s & 1], vf[KB - 1][s], dacc[KB - 1]);
-                    __builtin_amdgcn_sched_barrier(0);
+                    for (int i = 0; i < 2; ++i) {
+                        dacc[kb][i][0] = __builtin_bit_cast(f32x4, lds_read_b128(rows + (C::OFF_DELTA - C::OFF_LSE) + 64 * i));
+                        dacc[kb][i][1] = dacc[kb][i][0];
+                    }
                 }
+                if (!dp && m == PH - 1) mw[0] = lds_read_b128(words_at + 128 * kb);
+                if (dp && m == PH / 2 - 1) mw[1] = lds_read_b128(words_at + 128 * kb + 64);
+                if (dp && kb + 1 < KB && m == PH - 2) from_lse(kb + 1);
             }
-        }
-#pragma unroll
-        for (int n = 0; n < 2 * OB; ++n) {
-            const int u = n / OB, b = n % OB;
-            if (n + 1 < 2 * OB) columns(n + 1);
             __builtin_amdgcn_sched_barrier(0);
+            if (n < SCORES && !dp) {
 #pragma unroll
-            for (int kb = 0; kb < KB; ++kb) {
-                dvacc[kb][b] = E::mfma(oa[n & 1], u32x4{pp[kb][u][0], pp[kb][u][1], pp[kb][u][2], pp[kb][u][3]}, dvacc[kb][b]);
-                dkacc[kb][b] = E::mfma(qa[n & 1], u32x4{ps[kb][u][0], ps[kb][u][1], ps[kb][u][2], ps[kb][u][3]}, dkacc[kb][b]);
+                for (int k = 0; k < 2; ++k) sacc[kb][rb][k] = E::mfma(ring[n % (AHEAD + 1)], kf[c & 1][k], sacc[kb][rb][k]);
+                if constexpr (!C::LAND) {                 // the next step's
+                    if (m + 1 < PH) ring[(n + 1) % (AHEAD + 1)] = scaled(ring[(n + 1) % (AHEAD + 1)]);
+                }
+            } else if (n < SCORES) {
+                constexpr int EACH = (16 + PH - 1) / PH;
+#pragma unroll
+                for (int k = 0; k < 2; ++k) dacc[kb][rb][k] = E::mfma(ring[n % (AHEAD + 1)], vf[2 * kb + k][c], dacc[kb][rb][k]);
+#pragma unroll
+                for (int e = m * EACH; e < (m + 1) * EACH && e < 16; ++e) weight(kb, e);
+                if (m == PH - 1) {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        pack_weights(kb, i);
+                        if (kb + 1 < KB) dscore(kb, i);   // (at once: the registers that this frees are needed)
+                    }
+                }
+            } else {
+                const int b = (n - SCORES) % DB;
+                const u32x4 &r = ring[n % (AHEAD + 1)];
+#pragma unroll
+                for (int x = 0; x < KB; ++x)
+#pragma unroll
+                    for (int k = 0; k < 2; ++k) {
+                        if (n - SCORES < DB) dvacc[x][k][b] = E::mfma(r, pp[x][k], dvacc[x][k][b]);
+                        else dkacc[x][k][b] = E::mfma(r, ps[x][k], dkacc[x][k][b]);
+                    }
+                if (n - SCORES < DB) {
+                    constexpr int EACH = (8 + DB - 1) / DB;
+#pragma unroll
+                    for (int i = b * EACH; i < (b + 1) * EACH && i < 8; ++i) dscore(KB - 1, i);
+                }
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -386,7 +378,6 @@ __global__ __launch_bounds__(64 * NW, HDIM <= 64 && KB == 1 && NW == 4 ? 3 : 2) 
         int ln = lane;
         asm volatile("" : "+v"(ln));
         const uint32_t flag = *(LDS_PTR(const uint32_t))(uintptr_t)(lds0 + (C::OFF_LIVE + 32 * BUF) + 4 * (ln & (NW - 1)));
-        const uint32_t live = (uint32_t)__builtin_amdgcn_ballot_w64(flag != 0u) & ((1u << NW) - 1u);
 #pragma unroll
         for (int pass = 0; pass < PASSES; ++pass) {
             if (pass > 0 && wave + NW * pass >= NDB) break;
@@ -401,22 +392,22 @@ __global__ __launch_bounds__(64 * NW, HDIM <= 64 && KB == 1 && NW == 4 ? 3 : 2) 
             u32x4 kt[DEPTH], dst[DEPTH][RH];
             auto fetch = [&](int ks) __attribute__((always_inline)) {
                 constexpr int AT = BUF * C::DS_BYTES;
-                kt[ks % DEPTH] = tr_pair(dq_k + (pass * C::K_HALF + 4096 * ks), (dq_k ^ 16) + (pass * C::K_HALF + 4096 * ks + 512));
+                kt[ks % DEPTH] = tr_pair(dq_k + (pass * C::K_HALF + 4096 * ks), (dq_k ^ 80) + (pass * C::K_HALF + 4096 * ks + 512));
 #pragma unroll
                 for (int r = 0; r < RH; ++r)
-                    dst[ks % DEPTH][r] = tr_pair((dq_s ^ (32 * r)) + (AT + 2048 * ks), (dq_s ^ (32 * r + 8)) + (AT + 2048 * ks + 256));
+                    dst[ks % DEPTH][r] = tr_pair((dq_s ^ (32 * r)) + (AT + 2048 * ks), (dq_s ^ (32 * r + 16)) + (AT + 2048 * ks + 256));
             };
             auto product = [&](int ks) __attribute__((always_inline)) {
 #pragma unroll
-                for (int r = 0; r < RH; ++r) acc[r][ks % CH] = mfma16<BF16>(kt[ks % DEPTH], dst[ks % DEPTH][r], acc[r][ks % CH]);
+                for (int r = 0; r < RH; ++r) acc[r][ks % CH] = E::mfma(kt[ks % DEPTH], dst[ks % DEPTH][r], acc[r][ks % CH]);
             };
+#pragma unroll
+            for (int d = 0; d < DEPTH; ++d) fetch(d);     // before the flags are looked at
+            __builtin_amdgcn_sched_barrier(0);
+            const uint32_t live = (uint32_t)__builtin_amdgcn_ballot_w64(flag != 0u) & ((1u << NW) - 1u);
             if (live == (1u << NW) - 1u) {
 #pragma unroll
                 for (int ks = 0; ks < NW * KB; ++ks) {
-                    if (ks == 0) {
-#pragma unroll
-                        for (int d = 0; d < DEPTH; ++d) fetch(d);
-                    }
                     __builtin_amdgcn_sched_barrier(0);
                     product(ks);
                     if (ks + DEPTH < NW * KB) fetch(ks + DEPTH);
@@ -452,7 +443,7 @@ __global__ __launch_bounds__(64 * NW, HDIM <= 64 && KB == 1 && NW == 4 ? 3 : 2) 
 
     WAIT_VMCNT(0);
     if (a.D < HDIM && lane < 32 * KB) {               // columns of K beyond the row's end add nothing to the scores
-        for (int c = last_chunk + 1; c < 2 * KS; ++c)
+        for (int c = last_chunk + 1; c < 4 * KS; ++c)
             *(LDS_PTR(u32x4))(uintptr_t)(lds0 + (c >> 3) * C::K_HALF + (key0 + lane) * 128 + (((c & 7) ^ k_swizzle(lane)) << 4)) = u32x4{0u, 0u, 0u, 0u};
     }
     auto iteration = [&](int i, auto st_c) __attribute__((always_inline)) {
@@ -493,7 +484,9 @@ __global__ __launch_bounds__(64 * NW, HDIM <= 64 && KB == 1 && NW == 4 ? 3 : 2) 
 
 template <bool BF16, int HDIM, int NW, int KB, bool WIDE> void launch(hipStream_t stream, const AttnBwdArgs &a)
 {
-    hipLaunchKernelGGL((attn_bwd_head_kernel<BF16, HDIM, NW, KB, WIDE>), dim3((unsigned)a.BH), dim3(64 * NW), 0, stream, a);
+    // exp2(pm * s) needs its multiplication only then
+    const auto kernel = a.post_mul != 1.0f ? attn_bwd_head_kernel<BF16, HDIM, NW, KB, true, WIDE> : attn_bwd_head_kernel<BF16, HDIM, NW, KB, false, WIDE>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)a.BH), dim3(64 * NW), 0, stream, a);
 }
 template <bool BF16, bool WIDE> bool pick(hipStream_t stream, const AttnBwdArgs &a)
 {

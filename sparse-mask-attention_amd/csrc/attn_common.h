@@ -14,7 +14,6 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
@@ -34,11 +33,7 @@ template <bool BF16> struct Elem;
 
 template <> struct Elem<false> {
     static constexpr uint32_t ONES = 0x3c003c00u;           // two fp16 1.0
-    static __device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
-                                                      __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
+    static __device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
                                                       __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
     }
@@ -67,11 +62,7 @@ template <> struct Elem<false> {
 
 template <> struct Elem<true> {
     static constexpr uint32_t ONES = 0x3f803f80u;           // two bf16 1.0
-    static __device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
-                                                       __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
+    static __device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
                                                        __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
     }
@@ -276,47 +267,10 @@ __device__ __forceinline__ void store_landed(uint32_t lds_wave, const BlockDst &
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-// Transposed store of a 32 x COLS accumulator block (COLS = 64: acc[dblk][4g+j] = value(row l32,
-// column 32dblk + 8g + 4hh + j) with acc = {acc0, acc1}; COLS = 32: acc0 only) times `mult`.
-template <bool BF16, int COLS = 64>
-__device__ __forceinline__ void store_block(const f32x16 &acc0, const f32x16 &acc1, float mult, uint32_t lds_wave,
-                                            const BlockDst &dst, bool has_h, bool has_f, int row0, int N, int lane)
-{
-    const f32x16 acc[2] = {acc0, acc1};
-    using E = Elem<BF16>;
-    const int l32 = lane & 31, hh = lane >> 5;
-    const uint32_t wrow = lds_wave + l32 * 128 + hh * 8;
-    const int fo = (l32 >> 1) & 7;
-#pragma unroll
-    for (int dblk = 0; dblk < COLS / 32; ++dblk)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const u32x2 o = {E::pack2_rne(acc[dblk][4 * g + 0] * mult, acc[dblk][4 * g + 1] * mult),
-                             E::pack2_rne(acc[dblk][4 * g + 2] * mult, acc[dblk][4 * g + 3] * mult)};
-            *(LDS_PTR(u32x2))(uintptr_t)(wrow + (((4 * dblk + g) ^ fo) << 4)) = o;
-        }
-    store_landed<BF16, COLS>(lds_wave, dst, has_h, has_f, row0, N, lane);
-}
-// The same for all 32-column blocks of an output row (acc[2 * half + dblk]); `stride` LDS bytes between the
-// areas of the two column halves (0: one after the other through the same 4 KiB).
-template <bool BF16, int OB>
-__device__ __forceinline__ void store_rows(const f32x16 (&acc)[OB], float mult, uint32_t lds_wave, uint32_t stride,
-                                           const BlockDst &dst, bool has_h, bool has_f, int row0, int N, int lane)
-{
-    if constexpr (OB == 1) {
-        store_block<BF16, 32>(acc[0], acc[0], mult, lds_wave, dst, has_h, has_f, row0, N, lane);
-    } else {
-        store_block<BF16>(acc[0], acc[1], mult, lds_wave, dst, has_h, has_f, row0, N, lane);
-        if constexpr (OB == 3)
-            store_block<BF16, 32>(acc[2], acc[2], mult, lds_wave + stride, columns_from(dst, 64), has_h, has_f, row0, N, lane);
-        if constexpr (OB == 4)
-            store_block<BF16>(acc[2], acc[3], mult, lds_wave + stride, columns_from(dst, 64), has_h, has_f, row0, N, lane);
-    }
-}
-
-// The same from accumulators of 16 x 16 products: acc[rb][db][j] = value(row 16rb + lane % 16, column 16db + 4 (lane / 16) + j).
+// Transposed store of 32 rows from accumulators of 16 x 16 products, acc[rb][db][j] = value(row 16rb + lane % 16, column 16db + 4 (lane / 16) + j),
+// times `mult` of the row's block: COLS columns from block DB0 on, through 4 KiB of wave-private LDS ...
 template <bool BF16, int COLS, int DB0, int NB>
-__device__ __forceinline__ void store_block16(const f32x4 (&acc)[2][NB], const float (&mult)[2], uint32_t lds_wave,
+__device__ __forceinline__ void store_block(const f32x4 (&acc)[2][NB], const float (&mult)[2], uint32_t lds_wave,
                                               const BlockDst &dst, bool has_h, bool has_f, int row0, int N, int lane)
 {
     using E = Elem<BF16>;
@@ -333,13 +287,15 @@ __device__ __forceinline__ void store_block16(const f32x4 (&acc)[2][NB], const f
         }
     store_landed<BF16, COLS>(lds_wave, dst, has_h, has_f, row0, N, lane);
 }
+// ... and all columns, 64 at a time; `stride` LDS bytes between the areas of the two column halves (0: one after the other through
+// the same 4 KiB)
 template <bool BF16, int NB>
-__device__ __forceinline__ void store_rows16(const f32x4 (&acc)[2][NB], const float (&mult)[2], uint32_t lds_wave, uint32_t stride,
+__device__ __forceinline__ void store_rows(const f32x4 (&acc)[2][NB], const float (&mult)[2], uint32_t lds_wave, uint32_t stride,
                                              const BlockDst &dst, bool has_h, bool has_f, int row0, int N, int lane)
 {
-    store_block16<BF16, NB == 2 ? 32 : 64, 0>(acc, mult, lds_wave, dst, has_h, has_f, row0, N, lane);
+    store_block<BF16, NB == 2 ? 32 : 64, 0>(acc, mult, lds_wave, dst, has_h, has_f, row0, N, lane);
     if constexpr (NB > 4)
-        store_block16<BF16, NB == 6 ? 32 : 64, 4>(acc, mult, lds_wave + stride, columns_from(dst, 64), has_h, has_f, row0, N, lane);
+        store_block<BF16, NB == 6 ? 32 : 64, 4>(acc, mult, lds_wave + stride, columns_from(dst, 64), has_h, has_f, row0, N, lane);
 }
 
 }  // namespace

@@ -808,7 +808,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
 #pragma unroll
                 for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-                    for (int x = 0; x < 2; ++x) sacc[blk][kb][x] = E::mfma16(ones, u32x4{refb[x].x, refb[x].y, 0u, 0u}, sacc[blk][kb][x]);
+                    for (int x = 0; x < 2; ++x) sacc[blk][kb][x] = E::mfma(ones, u32x4{refb[x].x, refb[x].y, 0u, 0u}, sacc[blk][kb][x]);
         }
 #pragma unroll
         for (int n = 0; n < SCORES; ++n) {
@@ -817,7 +817,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
             __builtin_amdgcn_sched_barrier(0);
             const int blk = n / PH, kb = n & 1, c = n % PH >> 1;
 #pragma unroll
-            for (int x = 0; x < 2; ++x) sacc[blk][kb][x] = E::mfma16(k_ring[n % (AHEAD + 1)], qf[x][c], sacc[blk][kb][x]);
+            for (int x = 0; x < 2; ++x) sacc[blk][kb][x] = E::mfma(k_ring[n % (AHEAD + 1)], qf[x][c], sacc[blk][kb][x]);
             __builtin_amdgcn_sched_barrier(0);
         }
         after_scores();
@@ -920,7 +920,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
             __builtin_amdgcn_sched_barrier(0);
             const int blk = n / DB, b = n % DB;
 #pragma unroll
-            for (int x = 0; x < 2; ++x) oacc[x][b] = E::mfma16(v_ring[n % (V_AHEAD + 1)], pb[blk][x], oacc[x][b]);
+            for (int x = 0; x < 2; ++x) oacc[x][b] = E::mfma(v_ring[n % (V_AHEAD + 1)], pb[blk][x], oacc[x][b]);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -1154,7 +1154,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     {
         const int row0 = row_base;
         const uint32_t ebase = SPLIT ? lds0 : HALVES ? lds0 + 2 * HALF_SUMS + wave * 4096 : lds0 + (uint32_t)(visits & 1) * STAGE_BYTES + wave * 4096;
-        store_rows16<BF16>(oacc, inv, ebase, SPLIT ? 4096 : HALVES ? 8192 : 16384, block_dst(a.out, a.out32, bi, hi, row0, D), a.out.p != nullptr,
+        store_rows<BF16>(oacc, inv, ebase, SPLIT ? 4096 : HALVES ? 8192 : 16384, block_dst(a.out, a.out32, bi, hi, row0, D), a.out.p != nullptr,
                              BF16 && a.out32.p != nullptr, row0, N, lane);       // fp32 callers compute in bf16
     }
     if (qrow < N) {
