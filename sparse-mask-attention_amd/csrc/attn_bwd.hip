@@ -180,9 +180,7 @@ __device__ __forceinline__ void dq_rows(const AttnBwdArgs &a, unsigned char *sme
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 if constexpr (!HAVE_DELTA) d2[s & 1] = add_products<BF16>(dof[qb_][s][i], of[s][i], d2[s & 1]);
-                const float lo = E::up1((uint16_t)(qf[qb_][s][i] & 0xffffu)) * a.q_scale;
-                const float hi = E::up1((uint16_t)(qf[qb_][s][i] >> 16)) * a.q_scale;
-                qf[qb_][s][i] = (uint32_t)E::cvt1(lo) | ((uint32_t)E::cvt1(hi) << 16);
+                qf[qb_][s][i] = E::pack2_rne(E::up1((uint16_t)(qf[qb_][s][i] & 0xffffu)) * a.q_scale, E::up1((uint16_t)(qf[qb_][s][i] >> 16)) * a.q_scale);
             }
         if constexpr (!HAVE_DELTA) {
             delta = xhalf_sum(xrow_sum(d2[0])) + xhalf_sum(xrow_sum(d2[1]));
@@ -444,9 +442,7 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
         for (int s = 0; s < KS; ++s) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const float lo = E::up1((uint16_t)(kf[kb][s][i] & 0xffffu)) * a.q_scale;
-                const float hi = E::up1((uint16_t)(kf[kb][s][i] >> 16)) * a.q_scale;
-                kf[kb][s][i] = (uint32_t)E::cvt1(lo) | ((uint32_t)E::cvt1(hi) << 16);
+                kf[kb][s][i] = E::pack2_rne(E::up1((uint16_t)(kf[kb][s][i] & 0xffffu)) * a.q_scale, E::up1((uint16_t)(kf[kb][s][i] >> 16)) * a.q_scale);
             }
             if constexpr (VLDS) *(LDS_PTR(u32x4))(uintptr_t)(frag + (kb * KS + s) * 1024) = v_all[s];
             else vf[kb][VLDS ? 0 : s] = v_all[s];

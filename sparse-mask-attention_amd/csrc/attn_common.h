@@ -47,9 +47,9 @@ template <> struct Elem<false> {
         const f16x2 h = {(_Float16)a, (_Float16)b};
         return __builtin_bit_cast(uint32_t, h);
     }
-    static __device__ __forceinline__ float add2(uint32_t p, float acc) {
-        const f16x2 ones = {(_Float16)1.0f, (_Float16)1.0f};
-        return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, p), ones, acc, false);
+    // acc and the sum of a pair; `ones` is ONES (from a scalar register half the code of a literal)
+    static __device__ __forceinline__ float add2(uint32_t p, uint32_t ones, float acc) {
+        return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, p), __builtin_bit_cast(f16x2, ones), acc, false);
     }
     static __device__ __forceinline__ uint16_t cvt1(float a) {          // round to nearest even
         return __builtin_bit_cast(uint16_t, (_Float16)a);
@@ -75,9 +75,8 @@ template <> struct Elem<true> {
         const bf16x2 h = {(__bf16)a, (__bf16)b};
         return __builtin_bit_cast(uint32_t, h);
     }
-    static __device__ __forceinline__ float add2(uint32_t p, float acc) {
-        const bf16x2 ones = {(__bf16)1.0f, (__bf16)1.0f};
-        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, p), ones, acc, false);
+    static __device__ __forceinline__ float add2(uint32_t p, uint32_t ones, float acc) {
+        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, p), __builtin_bit_cast(bf16x2, ones), acc, false);
     }
     static __device__ __forceinline__ uint16_t cvt1(float a) {
         return __builtin_bit_cast(uint16_t, (__bf16)a);

@@ -584,6 +584,8 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         v_at = own0 + C::OFF_V + r * 128 + ((((l16 & 3) >> 1) ^ bitrev3(r >> 1)) << 4) + ((l16 & 1) << 3);
     }
     const uint32_t nib_rotate = (4u * q4 + 28u) & 31u;     // right: the nibble of keys 4q4 .. 4q4 + 3 comes to bits 4 .. 7
+    uint32_t nib_mask = 0xF0u, ones = E::ONES;             // in scalar registers: as literals they take four bytes more wherever they are used
+    asm volatile("" : "+s"(nib_mask), "+s"(ones));
 
     // ================================ prologue: one memory round trip ================================
     constexpr int Q_HALF = SPLIT ? 4096 : 16384;         // between the column halves of the staged q
@@ -708,9 +710,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
                                     (SPLIT ? C::OFF_V + (c >> 1) * Q_HALF : (NSTAGE - 1) * STAGE_BYTES + (c >> 1) * Q_HALF + wave * 4096));
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const float lo = E::up1((uint16_t)(t[i] & 0xffffu)) * a.q_scale;
-                const float hi = E::up1((uint16_t)(t[i] >> 16)) * a.q_scale;
-                t[i] = (uint32_t)E::cvt1(lo) | ((uint32_t)E::cvt1(hi) << 16);
+                t[i] = E::pack2_rne(E::up1((uint16_t)(t[i] & 0xffffu)) * a.q_scale, E::up1((uint16_t)(t[i] >> 16)) * a.q_scale);
             }
             if (!PACKED_ROWS && 4 * c + q4 > last_chunk) t = u32x4{0u, 0u, 0u, 0u};      // beyond the row: adds nothing
             qf[x][c] = t;
@@ -797,18 +797,18 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
 #pragma unroll
             for (int x = 0; x < 2; ++x) {
                 const uint32_t wa = __builtin_amdgcn_alignbit(rows.w[x], rows.w[x], nib_rotate);
-                sacc[blk][0][x] = __builtin_bit_cast(f32x4, lds_read_b128(lut_addr + (wa & 0xF0u)));
-                sacc[blk][1][x] = __builtin_bit_cast(f32x4, lds_read_b128(lut_addr + ((wa >> 16) & 0xF0u)));
+                sacc[blk][0][x] = __builtin_bit_cast(f32x4, lds_read_b128(lut_addr + (wa & nib_mask)));
+                sacc[blk][1][x] = __builtin_bit_cast(f32x4, lds_read_b128(lut_addr + ((wa >> 16) & nib_mask)));
             }
         }
         if (UNLIKELY(ref_used)) {               // wave-uniform: some row of this wavefront has r != 0
-            const u32x4 ones = {E::ONES, E::ONES, E::ONES, E::ONES};
+            const u32x4 all_ones = {ones, ones, ones, ones};
 #pragma unroll
             for (int blk = 0; blk < KB; ++blk)
 #pragma unroll
                 for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-                    for (int x = 0; x < 2; ++x) sacc[blk][kb][x] = E::mfma(ones, u32x4{refb[x].x, refb[x].y, 0u, 0u}, sacc[blk][kb][x]);
+                    for (int x = 0; x < 2; ++x) sacc[blk][kb][x] = E::mfma(all_ones, u32x4{refb[x].x, refb[x].y, 0u, 0u}, sacc[blk][kb][x]);
         }
 #pragma unroll
         for (int n = 0; n < SCORES; ++n) {
@@ -884,7 +884,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
                             const float p1 = __builtin_amdgcn_exp2f(POSTMUL ? s1 * pm : s1);
                             const uint32_t pk = E::pack2_prob(p0, p1);
                             pb[blk][x][2 * kb + i] = pk;
-                            lsum[x] = E::add2(pk, lsum[x]);
+                            lsum[x] = E::add2(pk, ones, lsum[x]);
                         }
         };
         // A row needs the maximum when it meets its first kept key (to choose its reference point)
