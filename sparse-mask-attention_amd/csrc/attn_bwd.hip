@@ -362,9 +362,8 @@ template <bool BF16, int HDIM, bool WIDE>
 __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_bwd_dq_kernel(const AttnBwdArgs a)
 {
     __shared__ __attribute__((aligned(1024))) unsigned char smem[Cfg<(HDIM > 64 ? 2 : 1)>::LDS_BYTES];
-    const int nid = renumber_block();
-    const int bh = (int)fastdiv((uint32_t)nid, a.div_qtiles);
-    dq_rows<BF16, HDIM, WIDE, false>(a, smem, bh, a.qtiles - 1 - (nid - bh * a.qtiles));      // last rows first, as in the forward
+    const Dealt d = deal(a.deal, a.qtiles, renumber_block());
+    dq_rows<BF16, HDIM, WIDE, false>(a, smem, d.head, a.qtiles - 1 - d.tile);      // last rows first, as in the forward
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -691,9 +690,8 @@ __global__ __launch_bounds__(64 * NW, HDIM == 128 ? NW / 4 : HDIM == 32 ? 4 : VL
             return;
         }
     }
-    const int nid = HDIM == 128 && NW == 8 ? renumber_block((int)blockIdx.x, a.whole_groups) : renumber_block();
-    const int bh = (int)fastdiv((uint32_t)nid, a.div_ktiles);
-    dkv_keys<BF16, HDIM, NW, VLDS, POSTMUL, WIDE>(a, smem, bh, nid - bh * a.ktiles);
+    const Dealt d = deal(a.deal, a.ktiles, HDIM == 128 && NW == 8 ? renumber_block((int)blockIdx.x, a.whole_groups) : renumber_block());
+    dkv_keys<BF16, HDIM, NW, VLDS, POSTMUL, WIDE>(a, smem, d.head, d.tile);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -746,10 +744,9 @@ __global__ __launch_bounds__(NTHREADS, HDIM == 128 ? 1 : HDIM > 64 ? 2 : 3) void
     constexpr bool VLDS = HDIM == 64 || HDIM == 128;
     constexpr int DQ = Cfg<(HDIM > 64 ? 2 : 1)>::LDS_BYTES, DKV = DkvCfg<HDIM, 4, VLDS>::LDS_BYTES;
     __shared__ __attribute__((aligned(1024))) unsigned char smem[DQ > DKV ? DQ : DKV];
-    const int nid = renumber_block();
-    const int bh = (int)fastdiv((uint32_t)nid, a.div_ktiles), i = nid - bh * 2 * a.qtiles;
-    if (i < a.qtiles) dkv_keys<BF16, HDIM, 4, VLDS, POSTMUL, WIDE>(a, smem, bh, i);
-    else dq_rows<BF16, HDIM, WIDE, true>(a, smem, bh, 2 * a.qtiles - 1 - i);
+    const Dealt d = deal(a.deal, a.ktiles, renumber_block());
+    if (d.tile < a.qtiles) dkv_keys<BF16, HDIM, 4, VLDS, POSTMUL, WIDE>(a, smem, d.head, d.tile);
+    else dq_rows<BF16, HDIM, WIDE, true>(a, smem, d.head, 2 * a.qtiles - 1 - d.tile);
 }
 
 template <bool BF16, int HDIM, bool POSTMUL, bool WIDE>
@@ -757,29 +754,33 @@ void launch_pair(hipStream_t stream, const AttnBwdArgs &args)
 {
     AttnBwdArgs a = args;
     const long long groups = (long long)a.BH * a.qtiles, cus = compute_units();
+    const bool alike = heads_alike(a.mask, a.H);
     // Both kinds of work-groups in one launch (see attn_bwd_both_kernel): while all are resident at once, or with a tile map
     if (2 * groups <= (HDIM == 128 ? 1 : HDIM > 64 ? 2 : 3) * cus ||
         (a.tile_map != nullptr && HDIM == 64 && groups < (1ll << 30))) {
-        a.ktiles = a.qtiles;
-        a.div_ktiles = make_fastdiv((uint32_t)(2 * a.qtiles));
+        a.ktiles = 2 * a.qtiles;
+        a.deal = make_deal(alike, a.BH, a.ktiles, (HDIM == 128 ? 1 : HDIM > 64 ? 2 : 3) * cus);
         hipLaunchKernelGGL((attn_bwd_delta_kernel<BF16>), dim3((unsigned)groups), dim3(NTHREADS), 0, stream, a);
         hipLaunchKernelGGL((attn_bwd_both_kernel<BF16, HDIM, POSTMUL, WIDE>), dim3((unsigned)(2 * groups)), dim3(NTHREADS), 0, stream, a);
         return;
     }
     // dQ first: it also fills the delta workspace that the dK/dV kernel reads (same stream)
+    a.deal = make_deal(alike, a.BH, a.qtiles, (HDIM > 64 ? 2 : HDIM == 64 ? 3 : 4) * cus);
     hipLaunchKernelGGL((attn_bwd_dq_kernel<BF16, HDIM, WIDE>), dim3((unsigned)(a.BH * a.qtiles)), dim3(NTHREADS), 0, stream, a);
     auto dkv = [&](auto nw_c, auto vlds_c) {
         constexpr int NW = decltype(nw_c)::value;
         a.ktiles = (a.N + 32 * NW - 1) / (32 * NW);
-        a.div_ktiles = make_fastdiv((uint32_t)a.ktiles);
         long long launched = (long long)a.BH * a.ktiles;
+        int whole = a.BH;
         if constexpr (HDIM == 128 && NW == 8) {
             // heads beyond the last full round in work-groups of 128 keys, if these are one round at most (see HALVES at the kernel)
             const long long full = cus > 0 ? (launched - 1) / cus * cus / a.ktiles : a.BH, rest = a.BH - full;
             a.whole_heads = rest * a.qtiles <= cus ? (int)full : a.BH;
+            whole = a.whole_heads;
             a.whole_groups = a.whole_heads * a.ktiles;
             launched = a.whole_groups + (long long)(a.BH - a.whole_heads) * a.qtiles;
         }
+        a.deal = make_deal(alike, whole, a.ktiles, (HDIM == 128 ? 1 : HDIM == 32 ? 4 : decltype(vlds_c)::value ? 3 : 2) * cus);
         hipLaunchKernelGGL((attn_bwd_dkv_kernel<BF16, HDIM, NW, decltype(vlds_c)::value, POSTMUL, WIDE>),
                            dim3((unsigned)launched), dim3(64 * NW), 0, stream, a);
     };

@@ -174,10 +174,17 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     const int l16 = lane & 15, q4 = lane >> 4;       // products: rows l16 and 16 + l16
 
     const int nid = renumber_block();
-    const int bh = (int)fastdiv((uint32_t)nid, a.div_qtiles);
     // last rows first: where rows keep more keys the later they come (causal masks), the longest
-    // work-groups of a head start first and the shortest fill the end of the launch
-    const int qt = a.qtiles - 1 - (nid - bh * a.qtiles);
+    // work-groups of a head (of several heads: see make_deal) start first and the shortest fill the end of the launch
+    int bh, qt;
+    if constexpr (BYTEMASK) {
+        bh = (int)fastdiv((uint32_t)nid, a.deal.div_groups);
+        qt = a.qtiles - 1 - (nid - bh * a.qtiles);
+    } else {
+        const Dealt d = deal(a.deal, a.qtiles, nid);
+        bh = d.head;
+        qt = a.qtiles - 1 - d.tile;
+    }
     const int half = HALVES ? wave >> 1 : 0;                             // which 32 keys of every tile
     const int row_base = SPLIT ? qt * 32 : HALVES ? qt * 64 + (wave & 1) * 32 : qt * BM + wave * 32;     // this wavefront's 32 query rows
     const int N = a.N, nw = (N + 31) >> 5;
@@ -1273,7 +1280,7 @@ hipError_t launch_attn_fwd(const AttnArgs &args, bool bf16, hipStream_t stream)
         a.qtiles = (a.N + 63) / 64;
         groups = (long long)a.BH * a.qtiles;
     }
-    a.div_qtiles = make_fastdiv((uint32_t)a.qtiles);
+    a.deal = make_deal(!split && !halves && !a.byte_mask && heads_alike(a.mask, a.H), a.BH, a.qtiles, (a.D <= HD ? 3 : 2) * cus);
     a.tail_start = (!split && groups > 2 * cus && groups <= 3 * cus) ? 0 : (int)groups;
     const dim3 grid((unsigned)groups), block(NTHREADS);
     const bool postmul = a.post_mul != 1.0f;

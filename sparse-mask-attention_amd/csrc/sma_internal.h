@@ -43,6 +43,52 @@ __host__ __device__ inline uint32_t fastdiv(uint32_t n, FastDiv f)
     return (uint32_t)(((uint64_t)n * f.mul) >> f.shift);
 }
 
+// How work-groups, each a tile of a head, are dealt out: `together` heads' tiles in turn, the first of all of them first.
+struct Deal {
+    int together;
+    FastDiv div_heads, div_groups;  // by `together` and by the tiles of so many heads
+};
+// One head after the other, unless neighbours have the same mask and there is more than one round of work-groups
+// (`resident` of them at once).  Then the tiles of the heads are alike, the longest come first (the last rows of a causal mask, its first
+// keys), and an XCD that takes as many heads in turn as it holds at once (a divisor of its share, so that no group lies on two) ends its
+// share with the short tiles of all heads instead of with the long and the short ones of the last.  One head after the other -> this, in us, bf16:
+//   forward, map      causal  D = 64: 64 heads, N = 2048 56.2 -> 39.9;  192, N = 1024 49.8 -> 38.5;  32, N = 4096 98.3 -> 76.2;  128, N = 4096 308 ->
+//                             289;  D = 128: 64, N = 2048 92.9 -> 75.8;  256, N = 1024 98.6 -> 84.2;  128, N = 4096 537 -> 528
+//                     blocks  192 heads, N = 1024: D = 32 25.8 -> 24.3, 64 35.2 -> 32.4, 128 60.6 -> 57.2;  N = 512, D = 128 25.4 -> 27.9 with one
+//                             mask a batch entry, 26.8 -> 25.8 with one for all
+//                     random  192 heads, N = 1024: 56.3 either way;  D = 128 97.5;  128, N = 4096, D = 64 527 -> 530
+//   forward, no map   causal  192 heads, N = 1024: D = 32 37.6 -> 31.4, 64 53.2 -> 43.6, 96 73.3 -> 60.7, 128 83.3 -> 71.7;  32, N = 4096: 97.9 ->
+//                             64.4, 106.8 -> 85.6, 139.0 -> 127.6, 163.9 -> 150.7;  128, N = 4096, D = 128 558.6 -> 547.9
+//                     blocks  192 heads, N = 1024: D = 32 32.4 -> 30.8, 64 41.5 -> 39.1, 128 67.5 -> 63.6
+//                     random  192 heads, N = 1024: D = 32 46.7 -> 47.7 (three tiles of a CU no longer read the same mask rows), 64 63.4 -> 63.9, 128
+//                             105.6 -> 106.1;  64, N = 2048, D = 32 57.6 -> 58.6, 64 80.3 -> 80.9, 128 132.2 either way
+//   backward, map     causal  192 heads, N = 1024: D = 32 95.4 -> 71.0, 64 130.0 -> 114.5, 128 257.5 -> 215.5;  64, N = 2048, D = 128 304 -> 223;  128, N =
+//                             4096: D = 64 942 -> 912, 128 1814 -> 1686
+//                     blocks  192 heads, N = 1024: D = 32 73.7 -> 66.3, 64 95.5 -> 88.8, 128 198.3 -> 192.1
+//                     random  D = 64: 192, N = 1024 182.9 -> 182.7;  128 heads, N = 4096: D = 64 1681 -> 1674, 128 2934 -> 2971
+//   backward, no map  causal  192 heads, N = 1024: D = 32 105 -> 83, 64 153 -> 132, 128 265 -> 229;  random, 128, N = 4096, D = 128 3021 -> 3017
+// With a mask for every head there is nothing alike to sort (forward, blocks, 192 heads, N = 1024: D = 64 33.9 -> 35.2, 128 58.6 -> 60.0).
+inline bool heads_alike(const PackedMask &mask, int H) { return (H > 1 ? mask.sh : mask.sb) == 0; }
+inline Deal make_deal(bool alike, int heads, int tiles, long long resident)
+{
+    int g = 1;
+    if (alike && heads % 8 == 0 && (long long)heads * tiles > resident) {
+        const long long want = (resident / 8 + tiles - 1) / tiles;
+        while (g < heads / 8 && (g < want || heads / 8 % g != 0)) ++g;
+    }
+    return Deal{g, make_fastdiv((uint32_t)g), make_fastdiv((uint32_t)(g * tiles))};
+}
+// Head and tile of work-group n.
+struct Dealt {
+    int head, tile;
+};
+__host__ __device__ inline Dealt deal(const Deal &d, int tiles, int n)
+{
+    const int first = (int)fastdiv((uint32_t)n, d.div_groups) * d.together, i = n - first * tiles;
+    const int tile = (int)fastdiv((uint32_t)i, d.div_heads);
+    return Dealt{first + i - tile * d.together, tile};
+}
+
 // Arguments of the fused forward kernel, already validated by the C-ABI layer.
 struct AttnArgs {
     Rows q, k, v;                   // inputs (never written)
@@ -63,7 +109,8 @@ struct AttnArgs {
     const uint32_t *tile_map;
     long long map_sb, map_sh;
     int qtiles;                     // ceil(N / 128): query tiles (work-groups) per (b,h)
-    FastDiv div_qtiles, div_H;      // filled in by the launcher
+    FastDiv div_H;                  // filled in by the launcher ...
+    Deal deal;                      // ... like this; with a boolean mask one head after the other
     // exp(scale * s) is evaluated as exp2(post_mul * (q_scale * q) . k): q is multiplied by
     // q_scale (sign of scale included, |q_scale| <= 1) when it is loaded, post_mul is a power of
     // two that is 1 unless |scale| * log2(e) > 1.
@@ -90,7 +137,8 @@ struct AttnBwdArgs {
     int D;                                     // head dim: a multiple of 8 up to 128
     int qtiles;                                // ceil(N / 128)
     int ktiles;                                // key tiles (work-groups of the dK/dV kernel) per (b,h) ...
-    FastDiv div_qtiles, div_ktiles, div_H;     // ... and these: filled in by the launcher
+    FastDiv div_qtiles, div_H;                 // ... and these: filled in by the launcher
+    Deal deal;                                 // of the kernel that is launched
     int whole_heads, whole_groups;             // head dim 128, eight wavefronts: the heads, and their work-groups, of 256 keys each
     float scale;                               // as given by the caller
     float q_scale, post_mul;                   // as in AttnArgs
