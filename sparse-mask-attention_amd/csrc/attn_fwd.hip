@@ -113,6 +113,17 @@ template <int NH, bool BYTEMASK, bool SPLIT> struct Cfg {
     static constexpr int LDS_BYTES = LUT_BYTES + (BYTEMASK && !SPLIT ? OFF_MAP_ARRIVED + 16 : OFF_MAP);
 };
 
+// The kernel's arguments where they lie.  What is read through this is requested no earlier than here: arguments are fetched from the host's
+// memory, and a work-group can request no data before those that the compiler has moved to its start have arrived.
+typedef const __attribute__((address_space(4))) AttnArgs *KernelArgs;
+__device__ __forceinline__ KernelArgs kernel_args()
+{
+    auto p = (KernelArgs)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return p;
+}
+__device__ __forceinline__ Rows rows_of(const __attribute__((address_space(4))) Rows &r) { return Rows{r.p, r.sb8, r.sh8, r.sn}; }
+
 template <int N> __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory"); }
 
 // PACKED_ROWS: the rows of q, k, v and out follow each other without gaps (row stride 64), as in
@@ -173,7 +184,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     const int l32 = lane & 31, hh = lane >> 5;       // mask: a row and a half of its words
     const int l16 = lane & 15, q4 = lane >> 4;       // products: rows l16 and 16 + l16
 
-    const int nid = renumber_block();
+    const int nid = SPLIT ? renumber_block() : renumber_block((int)blockIdx.x, a.groups);     // (SPLIT: 6.50 -> 6.37 us on 8 heads, N = 333, D = 32)
     // last rows first: where rows keep more keys the later they come (causal masks), the longest
     // work-groups of a head (of several heads: see make_deal) start first and the shortest fill the end of the launch
     int bh, qt;
@@ -706,6 +717,12 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     else if (PAIRS) wait_vmcnt<8>();                   // q has landed; 4 mask and 4 K/V copies may still be in flight
     else if (t_first < T) wait_vmcnt<C::COPIES>();     // q has landed; the copies of the first tile may still be in flight
     else wait_vmcnt<0>();
+    // What only the end needs of the arguments, while q is on its way from LDS.  Requested with the others at the start (as the compiler has it) ->
+    // behind the first copies -> here, the grid's size among the first arguments; small calls back to back: 2 heads, N = 128, D = 64 4.78 -> 4.64 ->
+    // 4.55 us; D = 128: 224, N = 18 5.38 -> 5.15 -> 5.14, 32, N = 64 5.05 -> 4.89 -> 4.83.
+    const KernelArgs late = kernel_args();
+    const Rows out = rows_of(late->out), out32 = rows_of(late->out32);
+    float *const lse = late->lse;
     // ---- Q^T as MFMA B operands, scaled by scale*log2(e)/post_mul:
     //      lane holds query rows 16x + l16, d = 32*c + 8*q4 .. +7
     u32x4 qf[2][KS];
@@ -1168,13 +1185,13 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     {
         const int row0 = row_base;
         const uint32_t ebase = SPLIT ? lds0 : HALVES ? lds0 + 2 * HALF_SUMS + wave * 4096 : lds0 + (uint32_t)(visits & 1) * STAGE_BYTES + wave * 4096;
-        store_rows<BF16>(oacc, inv, ebase, SPLIT ? 4096 : HALVES ? 8192 : 16384, block_dst(a.out, a.out32, bi, hi, row0, D), a.out.p != nullptr,
-                             BF16 && a.out32.p != nullptr, row0, N, lane);       // fp32 callers compute in bf16
+        store_rows<BF16>(oacc, inv, ebase, SPLIT ? 4096 : HALVES ? 8192 : 16384, block_dst(out, out32, bi, hi, row0, D), out.p != nullptr,
+                             BF16 && out32.p != nullptr, row0, N, lane);       // fp32 callers compute in bf16
     }
     if (qrow < N) {
-        if (a.lse != nullptr && hh == 0) {
+        if (lse != nullptr && hh == 0) {
             // log2 of the row's sum of exp(scale * score) is pm * r + log2(l)
-            a.lse[(size_t)bh * N + qrow] =
+            lse[(size_t)bh * N + qrow] =
                 (l_row > 0.f) ? __builtin_fmaf(pm * ref, 0.6931471805599453f, __builtin_logf(l_row)) : -__builtin_inff();
             // (an explicit fma: left to the compiler, the sum was contracted in some instantiations of
             // this kernel and not in others, and their lse differed in the last bit)
@@ -1289,6 +1306,7 @@ hipError_t launch_attn_fwd(const AttnArgs &args, bool bf16, hipStream_t stream)
     }
     a.deal = make_deal(!split && !halves && !a.byte_mask && heads_alike(a.mask, a.H), a.BH, a.qtiles, (a.D <= HD ? 3 : 2) * cus);
     a.tail_start = (!split && groups > 2 * cus && groups <= 3 * cus) ? 0 : (int)groups;
+    a.groups = (int)groups;
     const dim3 grid((unsigned)groups), block(NTHREADS);
     const bool postmul = a.post_mul != 1.0f;
     const int D = kernel_head_dim(a.D);

@@ -97,8 +97,10 @@ struct AttnArgs {
     PackedMask mask;                // byte_mask != 0: p names boolean bytes [Bm, Hm, N, N], strides in bytes
     Rows out, out32;                // 16-bit output and its fp32 copy (p names floats); p == nullptr: not wanted
     float *lse;                     // [BH, N] contiguous, or nullptr
-    int BH, H, N;
+    int groups;                     // work-groups of the launch: filled in by the launcher (the grid's own size lies behind all of this)
+    int H, N;
     int D;                          // head dim: a multiple of 8 up to 128
+    int BH;
     int byte_mask;                  // the mask is the caller's boolean tensor, not packed words
     uint32_t *mask_out;             // byte_mask only: nullptr, or where to leave the packed words [Bm, Hm, N, nw]
     uint32_t *map_out;              // byte_mask only: nullptr, or where to leave the tile map (layout as tile_map below)
