@@ -50,12 +50,29 @@ struct Deal {
 };
 // One head after the other, unless neighbours have the same mask and there is more than one round of work-groups
 // (`resident` of them at once).  Then the tiles of the heads are alike, the longest come first (the last rows of a causal mask, its first
-// keys), and an XCD that takes as many heads in turn as it holds at once (a divisor of its share, so that no group lies on two) ends its
-// share with the short tiles of all heads instead of with the long and the short ones of the last.  One head after the other -> this, in us, bf16:
+// keys), and an XCD that takes as many heads in turn as it holds at once ends its share with the short tiles of all heads instead of with the
+// long and the short ones of the last.  The group is the largest divisor of the share (no group lies on two XCDs) that is not more than that,
+// or, where that is half of it or less, the next one up to two thirds above.  What an XCD holds at once reads about as much K and V as its L2 has
+// room for (96 work-groups at head dim 64 3 MB, 64 at 128 4 MB); a much larger group sends every K and V out of it between the tiles of its head.
+// bf16, in us, one head after the other, groups of (held at once):
+//   forward, no map   D =  64  232 heads, N = 4096 causal 699, 29 (3) 1048, random 1042, 1086;  488, N = 2048 causal 387, 61 (6) 560;  1016, N = 512 causal
+//                              70.3, 127 (24) 91.2, random 87.6, 92.7;  40, N = 4096 causal 140.4, 5 (3) 134.7, random 182.0, 183.4
+//                     D = 128  104, N = 4096 causal 540, 13 (2) 807;  192, N = 512 random 31.3, 12 (16) 31.5, 24 32.6;  256, N = 512 random 41.0,
+//                              16 (16) 39.5, 32 46.7;  192, N = 800 random 79.2, 8 (10) 79.8, 24 85.4;  192, N = 1024 random 101.6, 8 (8) 102.5, 24 112.7
+//   forward, map      blocks, one mask a batch entry: D = 128  192 heads, N = 512, four masks drawn 25.8, 12 (16) 26.0, 24 27.5;  N = 1024 62.5, 8 (8) 57.5,
+//                              24 69.0;  D = 64 35.1, 12 (12) 32.4, 24 34.7
+//                     D = 128  104, N = 1024 causal 48.2, 13 (8) 38.4, random 64.6, 65.5;  24, N = 4096 causal 124.8, 3 (2) 106.9, random 189.8, 190.0
+//   backward, no map  D = 128  104, N = 1024 causal 168.9, 13 (8) 141.4;  232, N = 2048 causal 1047, 29 (4) 1120, random 1519, 1587
+// A causal mask with a map, whose far tiles are not visited, gains from the larger groups too (232 heads, N = 4096, D = 64: 597 -> 543), but nothing here
+// tells it from the others.
+// Neighbours with the same mask are enough: that a group reaches into another batch entry, with a mask of its own, costs nothing by itself (64 x 2 heads,
+// N = 2048, D = 64, groups of 1, 2, 4: causal, map 100.9, 95.6, 87.7, blocks 69.4, 67.9, 67.0, random 147.6, 149.5, 147.9).
+// Where two long heads in turn read more from memory than one after the other (4 x 32, N = 4096, D = 128, one mask a batch entry: forward 583 -> 773 MB, dQ
+// 852 -> 1043), they take no longer: random, forward 987 -> 974, backward 3052 -> 3021, causal 682 -> 677, 2030 -> 1934.
+// One head after the other -> groups, in us, bf16:
 //   forward, map      causal  D = 64: 64 heads, N = 2048 56.2 -> 39.9;  192, N = 1024 49.8 -> 38.5;  32, N = 4096 98.3 -> 76.2;  128, N = 4096 308 ->
 //                             289;  D = 128: 64, N = 2048 92.9 -> 75.8;  256, N = 1024 98.6 -> 84.2;  128, N = 4096 537 -> 528
-//                     blocks  192 heads, N = 1024: D = 32 25.8 -> 24.3, 64 35.2 -> 32.4, 128 60.6 -> 57.2;  N = 512, D = 128 25.4 -> 27.9 with one
-//                             mask a batch entry, 26.8 -> 25.8 with one for all
+//                     blocks  192 heads, N = 1024: D = 32 25.8 -> 24.3, 64 35.2 -> 32.4, 128 60.6 -> 57.2;  N = 512, D = 128: see above
 //                     random  192 heads, N = 1024: 56.3 either way;  D = 128 97.5;  128, N = 4096, D = 64 527 -> 530
 //   forward, no map   causal  192 heads, N = 1024: D = 32 37.6 -> 31.4, 64 53.2 -> 43.6, 96 73.3 -> 60.7, 128 83.3 -> 71.7;  32, N = 4096: 97.9 ->
 //                             64.4, 106.8 -> 85.6, 139.0 -> 127.6, 163.9 -> 150.7;  128, N = 4096, D = 128 558.6 -> 547.9
@@ -73,8 +90,16 @@ inline Deal make_deal(bool alike, int heads, int tiles, long long resident)
 {
     int g = 1;
     if (alike && heads % 8 == 0 && (long long)heads * tiles > resident) {
-        const long long want = (resident / 8 + tiles - 1) / tiles;
-        while (g < heads / 8 && (g < want || heads / 8 % g != 0)) ++g;
+        const int share = heads / 8;
+        const long long at_once = (resident / 8 + tiles - 1) / tiles;
+        const int holds = at_once < 1 ? 1 : at_once < share ? (int)at_once : share;
+        for (g = holds; share % g != 0;) --g;
+        if (2 * g <= holds)
+            for (int more = holds + 1; 3ll * more <= 5ll * holds && more <= share; ++more)
+                if (share % more == 0) {
+                    g = more;
+                    break;
+                }
     }
     return Deal{g, make_fastdiv((uint32_t)g), make_fastdiv((uint32_t)(g * tiles))};
 }
