@@ -465,20 +465,23 @@ def main():
     # ---- what this GPU sustains on a pure stream of the kernels' MFMA, and at what clock ----
     # (benchmark infrastructure in a library of its own, benchprobe/mfma_probe.h: not part of libsma_hip.so)
     probe_lib = ctypes.CDLL(os.path.join(PKG, "libsma_probe.so"))
-    probe_lib.sma_probe_mfma_stream.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
     n_cu = torch.cuda.get_device_properties(0).multi_processor_count
     stamps = torch.zeros(2 * n_cu, dtype=torch.int64, device=dev)
     probe = {}
-    for label, rnd in (("zero_operands", 0), ("random_operands", 1)):
+    for label, fn, rnd in (("zero_operands", "sma_probe_mfma_stream", 0), ("random_operands", "sma_probe_mfma_stream", 1),
+                           ("random_operands_32x32x16", "sma_probe_mfma_stream_32x32x16", 1)):
+        launch = getattr(probe_lib, fn)
+        launch.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
         iters = 20000
-        probe_lib.sma_probe_mfma_stream(rnd, 2000, n_cu, stamps.data_ptr(), stream)
-        ms = event_time_ms(lambda: probe_lib.sma_probe_mfma_stream(rnd, iters, n_cu, stamps.data_ptr(), stream), 1, 3, torch)
+        launch(rnd, 2000, n_cu, stamps.data_ptr(), stream)
+        ms = event_time_ms(lambda: launch(rnd, iters, n_cu, stamps.data_ptr(), stream), 1, 3, torch)
         st = stamps.view(n_cu, 2).double().cpu()
-        flops = n_cu * 12 * 8 * iters * 2.0 * 32 * 32 * 16
+        flops = n_cu * 12 * 8 * iters * 2.0 * 32 * 32 * 16            # 8 of 32 x 32 x 16 or 16 of 16 x 16 x 32 per iteration
         probe[label] = {"tflops": round(flops / (ms * 1e-3) / 1e12, 1),
                         "shader_clock_ghz": round(float((st[:, 0] / (st[:, 1] * 10.0)).mean()), 3)}
     result["mfma_stream_probe"] = dict(
-        probe, note="pure stream of v_mfma_f32_32x32x16_f16, three wavefronts per SIMD on every CU; the data-sheet "
+        probe, note="pure stream of v_mfma_f32_16x16x32_f16, which the kernels use, three wavefronts per SIMD on every CU (and of "
+                    "v_mfma_f32_32x32x16_f16); the data-sheet "
                     "peak (2516.6 TFLOP/s) assumes 2.4 GHz, the part lowers its clock under MFMAs on real data")
     sustained = probe["random_operands"]["tflops"]
     for key in ("roofline", "roofline_attn", "roofline_bwd"):

@@ -18,8 +18,8 @@ extern "C" {
 
 #define SMA_PROBE_MAX_ITERS (1 << 22)
 
-/* Launches `work_groups` (<= 65536) work-groups of 12 wavefronts that each issue 8 * iters MFMAs
- * (v_mfma_f32_32x32x16_f16; iters <= SMA_PROBE_MAX_ITERS) on operands that are all zero
+/* Launches `work_groups` (<= 65536) work-groups of 12 wavefronts that each issue 16 * iters MFMAs
+ * (v_mfma_f32_16x16x32_f16; iters <= SMA_PROBE_MAX_ITERS) on operands that are all zero
  * (random_operands == 0) or random fp16 numbers.  Thread 0 of work-group g leaves in stamps[2g] the
  * shader-clock ticks and in stamps[2g+1] the 100 MHz ticks that its loop took (stamps: device
  * memory, 2 * work_groups int64).  Time the launch to get the sustained MFMA rate; the quotient of
@@ -27,6 +27,9 @@ extern "C" {
  * NULL = the default stream).
  */
 int sma_probe_mfma_stream(int random_operands, int iters, int work_groups, long long *stamps, void *stream);
+
+/* The same of v_mfma_f32_32x32x16_f16, 8 * iters of them: as many operations. */
+int sma_probe_mfma_stream_32x32x16(int random_operands, int iters, int work_groups, long long *stamps, void *stream);
 
 #ifdef __cplusplus
 }

@@ -12,11 +12,11 @@
 // two, or both in one launch (attn_bwd_both_kernel):
 //
 //   attn_bwd_dq_kernel   one work-group = 128 query rows, walks the key tiles exactly like the
-//                        forward: S^T = K Q^T and dP^T = V dO^T on the MFMA (lane = query row, so
-//                        lse and delta are per-lane scalars and the mask enters as the accumulator's
+//                        forward: S^T = K Q^T and dP^T = V dO^T on the MFMA (a lane has two query rows, 16
+//                        apart, so lse and delta are two scalars each and the mask enters as the accumulator's
 //                        initial value), dS^T packed to 16 bit is the B operand of dQ^T += K^T dS^T
 //                        (K^T by transposing LDS reads).  Also writes delta to the workspace.
-//   attn_bwd_dkv_kernel  one work-group = 128 or 256 keys (lane = key), walks the query tiles:
+//   attn_bwd_dkv_kernel  one work-group = 128 or 256 keys (a lane has two, 16 apart), walks the query tiles:
 //                        S = Q K^T and dP = dO V^T with K, V fragments held in registers; -lse and
 //                        -delta of the tile's rows are read from LDS (broadcast reads) straight
 //                        into the accumulators as their initial values, so the products leave
@@ -27,7 +27,7 @@
 //                        register plus an immediate.
 //
 // Products of 16 x 16 x 32: what bounds these kernels at head dims 96 and 128 is the power the matrix cores draw, which lowers the clock, and a
-// stream of these on random operands sustains 1904 TFLOP/s at 1.89 GHz where 32 x 32 x 16 sustains 1689 at 1.69.  A lane holds two rows (dQ) or two
+// stream of these on random operands (benchprobe/) sustains 1968 TFLOP/s at 1.97 GHz where 32 x 32 x 16 sustains 1820 at 1.77.  A lane holds two rows (dQ) or two
 // keys (dK/dV), 16 apart, and every operand that is read from LDS serves both; of lse, delta and mask words half as many reads are left.  They are short, so
 // operands are requested two or three steps (of two products) ahead and the vector work of one step lies between the products of
 // another; scheduling barriers hold that order.  The compiler's own order, each read just before its use: dK/dV 1878 -> 2090 us on 4 x 32 heads,

@@ -15,7 +15,7 @@
 //                 exchanges (v_permlane16_swap, v_permlane32_swap).  P^T is already in
 //                 the B-operand layout of O^T += V^T * P^T: probabilities never leave registers.
 //                 The long grids run at the clock that the matrix cores' power leaves, and 16 x 16 x 32 draws
-//                 less than 32 x 32 x 16 (a stream on random operands: 1904 TFLOP/s at 1.89 GHz, 1689 at 1.69).
+//                 less than 32 x 32 x 16 (a stream on random operands, benchprobe/: 1968 TFLOP/s at 1.97 GHz, 1820 at 1.77).
 //                 These products are short, so their operands are requested two or three steps of two
 //                 products ahead (four or more of V while the exponentials run), in an order that scheduling barriers
 //                 hold.  Forward, 32 x 32 x 16 with operands one step ahead -> this, in us:

@@ -107,8 +107,9 @@ def load_probe():
         if not os.path.exists(path):
             raise RuntimeError(f"{path} is not built; run __graft_entry__.build()")
         lib = ctypes.CDLL(path)
-        lib.sma_probe_mfma_stream.restype = ctypes.c_int
-        lib.sma_probe_mfma_stream.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
+        for stream in (lib.sma_probe_mfma_stream, lib.sma_probe_mfma_stream_32x32x16):
+            stream.restype = ctypes.c_int
+            stream.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
         _probe = lib
     return _probe
 

@@ -418,8 +418,8 @@ def test_mfma_stream_probe_runs_and_reports_a_clock(dev):
     lib = _capi.load_probe()
     groups = 8
     stamps = torch.zeros(2 * groups, dtype=torch.int64, device=dev)
-    for random_operands in (0, 1):
-        assert lib.sma_probe_mfma_stream(random_operands, 2000, groups, stamps.data_ptr(), None) == 0
+    for stream, random_operands in ((lib.sma_probe_mfma_stream, 0), (lib.sma_probe_mfma_stream, 1), (lib.sma_probe_mfma_stream_32x32x16, 1)):
+        assert stream(random_operands, 2000, groups, stamps.data_ptr(), None) == 0
         torch.cuda.synchronize()
         st = stamps.view(groups, 2).double().cpu()
         assert (st > 0).all()
