@@ -759,13 +759,13 @@ void launch_pair(hipStream_t stream, const AttnBwdArgs &args)
     if (2 * groups <= (HDIM == 128 ? 1 : HDIM > 64 ? 2 : 3) * cus ||
         (a.tile_map != nullptr && HDIM == 64 && groups < (1ll << 30))) {
         a.ktiles = 2 * a.qtiles;
-        a.deal = make_deal(alike, a.BH, a.ktiles, (HDIM == 128 ? 1 : HDIM > 64 ? 2 : 3) * cus);
+        a.deal = make_deal(alike, a.BH, a.ktiles, (HDIM == 128 ? 1 : HDIM > 64 ? 2 : 3) * cus, 8ll * a.N * a.D);
         hipLaunchKernelGGL((attn_bwd_delta_kernel<BF16>), dim3((unsigned)groups), dim3(NTHREADS), 0, stream, a);
         hipLaunchKernelGGL((attn_bwd_both_kernel<BF16, HDIM, POSTMUL, WIDE>), dim3((unsigned)(2 * groups)), dim3(NTHREADS), 0, stream, a);
         return;
     }
     // dQ first: it also fills the delta workspace that the dK/dV kernel reads (same stream)
-    a.deal = make_deal(alike, a.BH, a.qtiles, (HDIM > 64 ? 2 : HDIM == 64 ? 3 : 4) * cus);
+    a.deal = make_deal(alike, a.BH, a.qtiles, (HDIM > 64 ? 2 : HDIM == 64 ? 3 : 4) * cus, 4ll * a.N * a.D);
     hipLaunchKernelGGL((attn_bwd_dq_kernel<BF16, HDIM, WIDE>), dim3((unsigned)(a.BH * a.qtiles)), dim3(NTHREADS), 0, stream, a);
     auto dkv = [&](auto nw_c, auto vlds_c) {
         constexpr int NW = decltype(nw_c)::value;
@@ -780,7 +780,7 @@ void launch_pair(hipStream_t stream, const AttnBwdArgs &args)
             a.whole_groups = a.whole_heads * a.ktiles;
             launched = a.whole_groups + (long long)(a.BH - a.whole_heads) * a.qtiles;
         }
-        a.deal = make_deal(alike, whole, a.ktiles, (HDIM == 128 ? 1 : HDIM == 32 ? 4 : decltype(vlds_c)::value ? 3 : 2) * cus);
+        a.deal = make_deal(alike, whole, a.ktiles, (HDIM == 128 ? 1 : HDIM == 32 ? 4 : decltype(vlds_c)::value ? 3 : 2) * cus, 4ll * a.N * a.D);
         hipLaunchKernelGGL((attn_bwd_dkv_kernel<BF16, HDIM, NW, decltype(vlds_c)::value, POSTMUL, WIDE>),
                            dim3((unsigned)launched), dim3(64 * NW), 0, stream, a);
     };

@@ -1304,7 +1304,7 @@ hipError_t launch_attn_fwd(const AttnArgs &args, bool bf16, hipStream_t stream)
         a.qtiles = (a.N + 63) / 64;
         groups = (long long)a.BH * a.qtiles;
     }
-    a.deal = make_deal(!split && !halves && !a.byte_mask && heads_alike(a.mask, a.H), a.BH, a.qtiles, (a.D <= HD ? 3 : 2) * cus);
+    a.deal = make_deal(!split && !halves && !a.byte_mask && heads_alike(a.mask, a.H), a.BH, a.qtiles, (a.D <= HD ? 3 : 2) * cus, 4ll * a.N * a.D);
     a.tail_start = (!split && groups > 2 * cus && groups <= 3 * cus) ? 0 : (int)groups;
     a.groups = (int)groups;
     const dim3 grid((unsigned)groups), block(NTHREADS);

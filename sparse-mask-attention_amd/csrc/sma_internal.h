@@ -51,16 +51,19 @@ struct Deal {
 // One head after the other, unless neighbours have the same mask and there is more than one round of work-groups
 // (`resident` of them at once).  Then the tiles of the heads are alike, the longest come first (the last rows of a causal mask, its first
 // keys), and an XCD that takes as many heads in turn as it holds at once ends its share with the short tiles of all heads instead of with the
-// long and the short ones of the last.  The group is the largest divisor of the share (no group lies on two XCDs) that is not more than that,
-// or, where that is half of it or less, the next one up to two thirds above.  What an XCD holds at once reads about as much K and V as its L2 has
-// room for (96 work-groups at head dim 64 3 MB, 64 at 128 4 MB); a much larger group sends every K and V out of it between the tiles of its head.
+// long and the short ones of the last.  The group is the largest divisor of the share (no group lies on two XCDs) that is not
+// more than that, or the next one up to two thirds above where its K and V fit an XCD's L2 (an eighth more is no loss yet) or the other is half of what is held or
+// less.  What an XCD holds at once reads about as much K and V as its L2 has room for (96 work-groups at head dim 64 3 MB, 64 at 128 4 MB); a much
+// larger group sends every K and V out of it between the tiles of its head.
 // bf16, in us, one head after the other, groups of (held at once):
 //   forward, no map   D =  64  232 heads, N = 4096 causal 699, 29 (3) 1048, random 1042, 1086;  488, N = 2048 causal 387, 61 (6) 560;  1016, N = 512 causal
 //                              70.3, 127 (24) 91.2, random 87.6, 92.7;  40, N = 4096 causal 140.4, 5 (3) 134.7, random 182.0, 183.4
 //                     D = 128  104, N = 4096 causal 540, 13 (2) 807;  192, N = 512 random 31.3, 12 (16) 31.5, 24 32.6;  256, N = 512 random 41.0,
-//                              16 (16) 39.5, 32 46.7;  192, N = 800 random 79.2, 8 (10) 79.8, 24 85.4;  192, N = 1024 random 101.6, 8 (8) 102.5, 24 112.7
-//   forward, map      blocks, one mask a batch entry: D = 128  192 heads, N = 512, four masks drawn 25.8, 12 (16) 26.0, 24 27.5;  N = 1024 62.5, 8 (8) 57.5,
+//                              16 (16) 39.5, 32 46.7;  192, N = 800 random 79.2, 8 (9) 79.8, 24 85.4;  192, N = 1024 random 101.6, 8 (8) 102.5, 24 112.7
+//   forward, map      blocks, one mask a batch entry: D = 128  192 heads, N = 512, mean of 24 masks drawn 26.0, 8 26.0, 12 (16) 26.6, 24 27.3;  N = 1024 62.5, 8 (8) 57.5,
 //                              24 69.0;  D = 64 35.1, 12 (12) 32.4, 24 34.7
+//                     D =  64  128 heads, N = 4096 causal 329, 2 309, 4 (3) 298;  192, N = 640 causal 21.9, 12 19.0, 24 (19) 18.4, blocks 19.6, 18.7, 18.2;  N = 700
+//                              causal 29.8, 12 25.1, 24 (16) 22.1, blocks 22.7, 22.8, 21.9, random without a map 34.9, 35.0, 35.2
 //                     D = 128  104, N = 1024 causal 48.2, 13 (8) 38.4, random 64.6, 65.5;  24, N = 4096 causal 124.8, 3 (2) 106.9, random 189.8, 190.0
 //   backward, no map  D = 128  104, N = 1024 causal 168.9, 13 (8) 141.4;  232, N = 2048 causal 1047, 29 (4) 1120, random 1519, 1587
 // A causal mask with a map, whose far tiles are not visited, gains from the larger groups too (232 heads, N = 4096, D = 64: 597 -> 543), but nothing here
@@ -86,20 +89,22 @@ struct Deal {
 //   backward, no map  causal  192 heads, N = 1024: D = 32 105 -> 83, 64 153 -> 132, 128 265 -> 229;  random, 128, N = 4096, D = 128 3021 -> 3017
 // With a mask for every head there is nothing alike to sort (forward, blocks, 192 heads, N = 1024: D = 64 33.9 -> 35.2, 128 58.6 -> 60.0).
 inline bool heads_alike(const PackedMask &mask, int H) { return (H > 1 ? mask.sh : mask.sb) == 0; }
-inline Deal make_deal(bool alike, int heads, int tiles, long long resident)
+constexpr long long L2_BYTES = 4ll << 20;         // of an XCD
+// head_bytes: what the tiles of a head all read (K and V, or Q and dO)
+inline Deal make_deal(bool alike, int heads, int tiles, long long resident, long long head_bytes)
 {
     int g = 1;
     if (alike && heads % 8 == 0 && (long long)heads * tiles > resident) {
         const int share = heads / 8;
-        const long long at_once = (resident / 8 + tiles - 1) / tiles;
-        const int holds = at_once < 1 ? 1 : at_once < share ? (int)at_once : share;
-        for (g = holds; share % g != 0;) --g;
-        if (2 * g <= holds)
-            for (int more = holds + 1; 3ll * more <= 5ll * holds && more <= share; ++more)
-                if (share % more == 0) {
-                    g = more;
-                    break;
-                }
+        const long long held = resident / 8;
+        while (g < share && (long long)(g + 1) * tiles <= held) ++g;
+        while (share % g != 0) --g;
+        const int below = g;
+        for (long long more = below + 1; more <= share && 3 * more * tiles <= 5 * held; ++more)
+            if (share % more == 0) {
+                if (2ll * below * tiles <= held || more * head_bytes <= L2_BYTES + L2_BYTES / 8) g = (int)more;
+                break;
+            }
     }
     return Deal{g, make_fastdiv((uint32_t)g), make_fastdiv((uint32_t)(g * tiles))};
 }

@@ -11,8 +11,8 @@ from _launches import launches, places
 pytestmark = pytest.mark.gpu
 
 
-# heads beyond one round of every kernel, in groups (at head dims up to 64, beyond) of: 4, 2 of a share of 4; 3 of 3; 5 of 5, a prime; 3, 2 of 6; 6 of 12, one
-# head with all the masks shared by the batch; 12 of 24 short ones; and one after the other (no multiple of 8)
+# heads beyond one round of every kernel, in groups (in the forward at head dims up to 64, at 128) of: 4, 2 of a share of 4; 3, 1 of 3; 5 of 5, a prime; 3, 2 of
+# 6; 12, 6 of 12, one head with all the masks shared by the batch; 24, 12 of 24 short ones; and one after the other (no multiple of 8)
 @pytest.mark.parametrize("B, H, N", [(2, 16, 3300), (3, 8, 4200), (5, 8, 2600), (4, 12, 4097), (96, 1, 1153), (16, 12, 577), (7, 3, 4750)])
 @pytest.mark.parametrize("D", [32, 64, 72, 128])
 @pytest.mark.parametrize("mapped", [False, True])

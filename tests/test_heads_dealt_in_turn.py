@@ -18,9 +18,9 @@ PROGRAM = r"""
 int main()
 {
     int heads, tiles, alike;
-    long long resident;
-    while (scanf("%d %d %lld %d", &heads, &tiles, &resident, &alike) == 4) {
-        const sma::Deal d = sma::make_deal(alike != 0, heads, tiles, resident);
+    long long resident, bytes;
+    while (scanf("%d %d %lld %d %lld", &heads, &tiles, &resident, &alike, &bytes) == 5) {
+        const sma::Deal d = sma::make_deal(alike != 0, heads, tiles, resident, bytes);
         std::vector<char> seen((size_t)heads * tiles);
         int ok = 1;
         for (int n = 0; n < heads * tiles; ++n) {
@@ -44,33 +44,41 @@ def _deals(tmp_path, grids):
     (tmp_path / "deal.cpp").write_text(PROGRAM)
     subprocess.run([compiler, "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__=1", "-Wno-deprecated-declarations", f"-I{CSRC}",
                     f"-I{os.environ.get('ROCM_PATH', '/opt/rocm')}/include", str(tmp_path / "deal.cpp"), "-o", str(tmp_path / "deal")], check=True)
-    text = "".join(f"{h} {t} {r} {int(a)}\n" for h, t, r, a in grids)
+    text = "".join(f"{h} {t} {r} {int(a)} {b}\n" for h, t, r, a, b in grids)
     out = subprocess.run([str(tmp_path / "deal")], input=text, capture_output=True, text=True, check=True).stdout.split()
     return [(int(g), ok == "1") for g, ok in zip(out[::2], out[1::2])]
 
 
+def _grid(heads, N, D, alike=True, cus=256):
+    """The forward's: 128 rows a work-group, three of them on a CU up to head dim 64 and two beyond."""
+    return heads, -(-N // 128), (3 if D <= 64 else 2) * cus, alike, 4 * N * D
+
+
 def test_groups(tmp_path):
-    grids = [(8 * share, tiles, resident, True)
-             for share in list(range(1, 33)) + [61, 96, 97, 127] for tiles in (1, 2, 3, 4, 5, 7, 8, 16, 21, 26, 32, 33, 64) for resident in (256, 512, 768, 1024)]
+    grids = [(8 * share, tiles, resident, True, 4 * 128 * tiles * D)
+             for share in list(range(1, 33)) + [61, 96, 97, 127] for tiles in (1, 2, 3, 4, 5, 7, 8, 16, 21, 26, 32, 33, 64) for resident in (256, 512, 768, 1024)
+             for D in (32, 128)]
     some = 0
-    for (heads, tiles, resident, _), (g, ok) in zip(grids, _deals(tmp_path, grids)):
-        share, holds = heads // 8, -(-(resident // 8) // tiles)
+    for (heads, tiles, resident, _, head_bytes), (g, ok) in zip(grids, _deals(tmp_path, grids)):
+        share, held = heads // 8, resident // 8 / tiles          # heads that an XCD holds at once
         assert ok and share % g == 0, (heads, tiles, resident, g)
         if heads * tiles <= resident:
             assert g == 1
             continue
         divisors = [x for x in range(1, share + 1) if share % x == 0]
-        most = max(x for x in divisors if x <= holds)
-        if 2 * most <= min(holds, share):                        # nothing near below it: at most two thirds above
-            most = min([x for x in divisors if holds < x <= holds * 5 / 3], default=most)
-        assert g == most <= holds * 5 / 3, (heads, tiles, resident, g)
+        below = max([x for x in divisors if x <= held], default=1)
+        above = min([x for x in divisors if x > below], default=below)
+        take = above * tiles * 3 <= resident // 8 * 5 and (2 * below * tiles <= resident // 8 or above * head_bytes <= 4.5 * 2 ** 20)
+        assert g == (above if take else below), (heads, tiles, resident, head_bytes, g)
+        assert g == 1 or g * tiles * 3 <= resident // 8 * 5
         some += g > 1
     assert some > 500
 
 
-def test_one_head_after_the_other(tmp_path):
-    grids = [(192, 8, 768, False), (190, 8, 768, True), (192, 4, 768, True), (192, 8, 0, True), (8, 8, 0, True),
-             (232, 32, 768, True), (1016, 4, 768, True)]                     # 29 and 127 heads a share, of which 3 and 24 are held at once
-    assert _deals(tmp_path, grids) == [(1, True)] * len(grids)
-    assert _deals(tmp_path, [(192, 8, 768, True), (192, 4, 512, True), (128, 32, 512, True), (104, 8, 512, True)]) == [
-        (12, True), (12, True), (2, True), (13, True)]
+def test_named_grids(tmp_path):
+    want = [(_grid(192, 1024, 64), 12), (_grid(192, 512, 128), 12), (_grid(128, 4096, 128), 2),                  # as many as are held, or most of them
+            (_grid(128, 4096, 64), 4), (_grid(192, 700, 64), 24), (_grid(192, 800, 128), 8),                     # the next above where K and V fit
+            (_grid(104, 1024, 128), 13),                                                                         # ... or where there is nothing near below
+            (_grid(232, 4096, 64), 1), (_grid(488, 2048, 64), 1), (_grid(1016, 512, 64), 1)]                     # 29, 61 and 127 heads a share
+    want += [(g, 1) for g in (_grid(192, 1024, 64, alike=False), _grid(190, 1024, 64), _grid(192, 512, 64), _grid(192, 1024, 64, cus=0), _grid(8, 1024, 64, cus=0))]
+    assert _deals(tmp_path, [g for g, _ in want]) == [(n, True) for _, n in want]
