@@ -719,10 +719,17 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     else wait_vmcnt<0>();
     // What only the end needs of the arguments, while q is on its way from LDS.  Requested with the others at the start (as the compiler has it) ->
     // behind the first copies -> here, the grid's size among the first arguments; small calls back to back: 2 heads, N = 128, D = 64 4.78 -> 4.64 ->
-    // 4.55 us; D = 128: 224, N = 18 5.38 -> 5.15 -> 5.14, 32, N = 64 5.05 -> 4.89 -> 4.83.
-    const KernelArgs late = kernel_args();
-    const Rows out = rows_of(late->out), out32 = rows_of(late->out32);
-    float *const lse = late->lse;
+    // 4.55 us; D = 128: 224, N = 18 5.38 -> 5.15 -> 5.14, 32, N = 64 5.05 -> 4.89 -> 4.83.  (Where by-products are asked for, in training, as the
+    // compiler has it: those kernels use all but a few scalar registers, and late costs them 192 heads, N = 577, D = 32 32.0 -> 32.2 us, fp32 queries, D = 80
+    // 43.75 -> 44.1, of which two are then spilled.)
+    Rows out = a.out, out32 = a.out32;
+    float *lse = a.lse;
+    if constexpr (!BYPRODUCTS) {
+        const KernelArgs late = kernel_args();
+        out = rows_of(late->out);
+        out32 = rows_of(late->out32);
+        lse = late->lse;
+    }
     // ---- Q^T as MFMA B operands, scaled by scale*log2(e)/post_mul:
     //      lane holds query rows 16x + l16, d = 32*c + 8*q4 .. +7
     u32x4 qf[2][KS];
@@ -734,8 +741,8 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
                                      (SPLIT ? C::OFF_V + (c >> 1) * Q_HALF : (NSTAGE - 1) * STAGE_BYTES + (c >> 1) * Q_HALF + wave * 4096));
     // All requested before the first is converted.  Left alone, the compiler read, waited and converted one after the other, up to eight round trips
     // of LDS in a row: small calls back to back, that -> this, 2 heads, N = 128, D = 64 4.86 -> 4.78 us; D = 128: 224, N = 18 5.51 -> 5.38, 32, N = 64
-    // 5.23 -> 5.05.
-    __builtin_amdgcn_sched_barrier(0);
+    // 5.23 -> 5.05.  (fp32 queries: the same either way, 6.69 us of a call of two launches, and 96 heads, N = 577, D = 80 43.5 us left alone, 43.9 held.)
+    if constexpr (!WIDE_Q) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int x = 0; x < 2; ++x)
 #pragma unroll
