@@ -156,12 +156,20 @@ template <bool BF16, bool POSTMUL, bool PACKED_ROWS, int HDIM, bool BYTEMASK = f
 __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ? 2 : 3) void attn_fwd_kernel(const AttnArgs a)
 {
     // HALVES: a work-group of 64 rows, two wavefronts to each 32 of them, which take 32 keys of every tile each and add their
-    // sums at the end.  A grid that leaves CUs without any 128-row work-group then has one on (almost) each, and a visit's chain of products,
-    // exponentials and products is half as long.  Forward, before -> now, D = 128: 7 heads, N = 2048 46.1 -> 36.1 us (packed 42.5 -> 32.0); 16,
+    // sums at the end.  A visit's chain of products, exponentials and products is half as long, which is what bounds a grid whose work-groups of 128
+    // rows are one or two to a CU.  Forward, before -> now, D = 128: 7 heads, N = 2048 46.1 -> 36.1 us (packed 42.5 -> 32.0); 16,
     // N = 1024 25.7 -> 21.0; 32, N = 512 15.6 -> 13.6; 32, N = 263 11.6 -> 10.7; D = 80: 5 heads, N = 3000 62.3 -> 52.3; 64, N = 192 8.7 -> 8.2.
-    static_assert(!HALVES || (HDIM > 64 && FETCH == 0 && !SPLIT), "HALVES: one tile's bytes at a time");
+    // D = 64: 24 heads, N = 2048 43.4 -> 35.1 us (packed 40.5 -> 32.8), 40, N = 1024 23.8 -> 19.3 (22.2 -> 17.7), 48, N = 990
+    // 26.4 -> 21.6; on masks that nothing has touched before 45.2 -> 42.0, 25.5 -> 22.7, 28.9 -> 26.0.
+    // The mask's bytes with HALVES: at head dims up to 64 always those of two tiles at once (FETCH != 0): each of the two wavefronts copies 16 of the 32
+    // rows for both, into one of two slots, two visits before the first of them is looked at.  32 bytes of a row, what a wavefront needs
+    // of a tile, copied by each for itself one or two visits ahead: on untouched masks 48 heads, N = 990 28.9 -> 30.4 us instead of 26.0.
+    static_assert(!HALVES || (!SPLIT && (!BYTEMASK || (HDIM <= 64) == (FETCH != 0))), "HALVES: pairs of tiles up to head dim 64");
     static_assert(FETCH == 0 || (BYTEMASK && HDIM <= 64 && !SPLIT), "PAIRS: byte mask, two byte slots");
     constexpr bool PAIRS = FETCH != 0, WHOLE = FETCH == 1;
+    // only the 32 keys of a tile that the wavefront takes: half the bytes to read from LDS and, without PAIRS, one copy instead of two.  (The
+    // by-products are made of whole tiles.)
+    constexpr bool HALF_BYTES = HALVES && BYTEMASK && !BYPRODUCTS;
     using E = Elem<BF16>;
     constexpr int NH = HDIM > 64 ? 2 : 1;         // 64-column tiles per matrix
     constexpr int KS = HDIM / 32;                 // MFMA steps of the QK^T chain
@@ -172,7 +180,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     constexpr bool SAME_HALVES = HDIM == 128 && PACKED_ROWS;
     using C = Cfg<NH, BYTEMASK, SPLIT>;
     constexpr int NSTAGE = C::NSTAGE, STAGE_BYTES = C::STAGE_BYTES, OFF_MASK = C::OFF_MASK;
-    constexpr int MASK_SLOT = C::MASK_SLOT;
+    constexpr int MASK_SLOT = C::MASK_SLOT, COPIES = C::COPIES - (HALF_BYTES ? 1 : 0);
     const int D = PACKED_ROWS ? HDIM : a.D;
     const int last_chunk = (D >> 3) - 1;          // 16-byte chunks per global row, minus one
     __shared__ __attribute__((aligned(1024))) unsigned char smem[C::LDS_BYTES];
@@ -254,9 +262,10 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     if constexpr (BYTEMASK) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            const int row = 16 * j + (lane >> 2);
+            // (HALF_BYTES: row i/2, position i%2, of the wavefront's two chunks the one at position ^ ((row >> 3) & 1))
+            const int row = HALF_BYTES ? lane >> 1 : 16 * j + (lane >> 2);
             const int grow = row_base + row;
-            mb_chunk[j] = (uint32_t)(((lane & 3) ^ ((row >> 2) & 3)) << 4);
+            mb_chunk[j] = HALF_BYTES ? (uint32_t)(32 * half + (((lane & 1) ^ ((row >> 3) & 1)) << 4)) : (uint32_t)(((lane & 3) ^ ((row >> 2) & 3)) << 4);
             mb_voff[j] = (uint32_t)(grow < N ? grow : N - 1) * (uint32_t)N + mb_chunk[j];
         }
     }
@@ -281,7 +290,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
                 }
             }
             async_copy_b128_at<OFF_MASK + SLOT * MASK_SLOT>(mask_dst, src, mb_voff[0]);
-            async_copy_b128_at<OFF_MASK + SLOT * MASK_SLOT + 1024>(mask_dst, src, mb_voff[1]);
+            if constexpr (!HALF_BYTES) async_copy_b128_at<OFF_MASK + SLOT * MASK_SLOT + 1024>(mask_dst, src, mb_voff[1]);
         } else {
             if (UNLIKELY(x == odd_tile)) m_voff -= (lane & 1) * 4;      // the last tile: none follows it
             async_copy_b32_at<OFF_MASK + SLOT * MASK_SLOT>(mask_dst, mb + 2u * (uint32_t)x, m_voff);
@@ -294,7 +303,14 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     if constexpr (PAIRS) pair_voff = (uint32_t)(row_base + (lane >> 3)) * (uint32_t)N + (uint32_t)(((lane & 7) ^ (lane >> 4)) << 4);
     auto issue_mask_pair = [&](int p) __attribute__((always_inline)) {      // bytes of tiles 2p and 2p + 1
         const uint8_t *src = reinterpret_cast<const uint8_t *>(mb) + (size_t)p * (2 * BN);
-        const uint32_t dst = lds0 + wave * 4096;
+        // HALVES: the two wavefronts of 32 rows copy 16 of them each, for both, into one of two slots
+        const uint32_t dst = HALVES ? lds0 + (p & 1) * 8192 + (wave & 1) * 4096 + half * 2048 : lds0 + wave * 4096;
+        if constexpr (WHOLE && HALVES) {
+            src += (size_t)(16 * half) * N;
+            async_copy_b128_at<OFF_MASK>(dst, src, pair_voff);
+            async_copy_b128_at<OFF_MASK + 1024>(dst, src + (size_t)8 * N, pair_voff ^ 64u);
+            return;
+        }
         if constexpr (WHOLE) {                   // the low seven bits of the lane offset are the chunk alone
             async_copy_b128_at<OFF_MASK>(dst, src, pair_voff);
             async_copy_b128_at<OFF_MASK + 1024>(dst, src + (size_t)8 * N, pair_voff ^ 64u);
@@ -327,6 +343,12 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
                 vo[j] += back;
                 if (end > row_end) vo[j] -= end - row_end;
             }
+        }
+        if constexpr (HALVES) {
+            src += 2 * half * step;
+            async_copy_b128_at<OFF_MASK>(dst, src, half ? vo[2] : vo[0]);
+            async_copy_b128_at<OFF_MASK + 1024>(dst, src + step, half ? vo[3] : vo[1]);
+            return;
         }
         async_copy_b128_at<OFF_MASK>(dst, src, vo[0]);
         async_copy_b128_at<OFF_MASK + 1024>(dst, src + step, vo[1]);
@@ -364,22 +386,46 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     // slots occupy otherwise; the 16-byte chunks of a row are swizzled like K's (position ^ ((row >> 1)
     // & 7), applied on the global side), which keeps the reads below free of bank conflicts.
     // `pair_half` (0 or 1) says which tile of the pair; -1: the ordinary slots.
-    const uint32_t pair_base = lds0 + OFF_MASK + wave * 4096 + l32 * 128;
+    const uint32_t pair_base = lds0 + OFF_MASK + (HALVES ? wave & 1 : wave) * 4096 + l32 * 128;
     const int psw = (l32 >> 1) & 7;
     auto mask_words = [&](int x, int slot, int pair_half = -1) __attribute__((always_inline)) -> u32x2 {
         u32x2 w;
-        if constexpr (BYTEMASK) {
+        // a byte counts as "attend" when it is non-zero, as in the packer: nz() leaves 0x80 in
+        // every non-zero byte, the dot products weigh those with 1, 2, 4 .. 128 (times 128)
+        auto nz = [](uint32_t x) -> uint32_t { return (((x & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x) & 0x80808080u; };
+        if constexpr (HALF_BYTES) {
+            // this lane: 16 bytes of row l32, keys 32 half + 16hh .. + 15
+            const u32x4 d = lds_read_b128(PAIRS ? pair_base + slot * 8192 + (((4 * pair_half + 2 * half + hh) ^ psw) << 4)
+                                                : mask_dst + OFF_MASK + slot * MASK_SLOT + l32 * 32 + ((hh ^ ((l32 >> 3) & 1)) << 4));
+            uint32_t mine;
+            if (LIKELY(__builtin_amdgcn_ballot_w64(((d.x | d.y | d.z | d.w) & 0xfefefefeu) != 0u) == 0ull)) {
+                uint32_t b0 = __builtin_amdgcn_udot4(d.x, 0x08040201u, 0u, false);
+                uint32_t b1 = __builtin_amdgcn_udot4(d.z, 0x08040201u, 0u, false);
+                b0 = __builtin_amdgcn_udot4(d.y, 0x80402010u, b0, false);
+                b1 = __builtin_amdgcn_udot4(d.w, 0x80402010u, b1, false);
+                mine = b0 | (b1 << 8);
+            } else {
+                uint32_t b0 = __builtin_amdgcn_udot4(nz(d.x), 0x08040201u, 0u, false);
+                uint32_t b1 = __builtin_amdgcn_udot4(nz(d.z), 0x08040201u, 0u, false);
+                b0 = __builtin_amdgcn_udot4(nz(d.y), 0x80402010u, b0, false);
+                b1 = __builtin_amdgcn_udot4(nz(d.w), 0x80402010u, b1, false);
+                mine = (b0 >> 7) | (b1 << 1);                        // each partial value is 128 x (8 bits): bits 7..14
+            }
+            const int row_end = N - x * BN;
+            if (UNLIKELY(x == cut_tile) && (row_end >> 4) == 2 * half + hh) mine >>= (16 - (row_end & 15)) & 15;     // see below
+            const auto r = __builtin_amdgcn_permlane32_swap(mine, mine, false, false);
+            w.x = (uint32_t)r[0] | ((uint32_t)r[1] << 16);
+            if (UNLIKELY(x == cut_tile)) w.x &= half ? a.last_mask1 : a.last_mask0;
+            w.y = w.x;
+        } else if constexpr (BYTEMASK) {
             // this lane: the 32 bytes of row l32 for keys 32hh .. 32hh+31 -> one word
             const uint32_t a0 = !PAIRS || pair_half < 0 ? maddr + slot * MASK_SLOT + (((2 * hh) ^ msw) << 4)
-                                                        : pair_base + (((4 * pair_half + 2 * hh) ^ psw) << 4);
+                                                        : pair_base + (HALVES ? slot * 8192 : 0) + (((4 * pair_half + 2 * hh) ^ psw) << 4);
             const uint32_t a1 = !PAIRS || pair_half < 0 ? maddr + slot * MASK_SLOT + (((2 * hh + 1) ^ msw) << 4)
-                                                        : pair_base + (((4 * pair_half + 2 * hh + 1) ^ psw) << 4);
+                                                        : pair_base + (HALVES ? slot * 8192 : 0) + (((4 * pair_half + 2 * hh + 1) ^ psw) << 4);
             const u32x4 d0 = lds_read_b128(a0);
             const u32x4 d1 = lds_read_b128(a1);
-            // a byte counts as "attend" when it is non-zero, as in the packer: nz() leaves 0x80 in
-            // every non-zero byte, the dot products weigh those with 1, 2, 4 .. 128 (times 128)
-            auto nz = [](uint32_t x) -> uint32_t { return (((x & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x) & 0x80808080u; };
-            // ... which costs three instructions per four bytes.  Bytes that are all 0 or 1 (every
+            // nz() costs three instructions per four bytes.  Bytes that are all 0 or 1 (every
             // mask PyTorch itself made) need none of it: one look at the wavefront's 2 KiB decides.
             const uint32_t other = (d0.x | d0.y | d0.z | d0.w | d1.x | d1.y | d1.z | d1.w) & 0xfefefefeu;
             uint32_t mine;
@@ -714,8 +760,8 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         yield_at = n_visits / 4;
     }
     if (SPLIT) { if (t_first < T) wait_vmcnt<8 * NH + C::MASK_COPIES>(); else wait_vmcnt<0>(); }
-    else if (PAIRS) wait_vmcnt<8>();                   // q has landed; 4 mask and 4 K/V copies may still be in flight
-    else if (t_first < T) wait_vmcnt<C::COPIES>();     // q has landed; the copies of the first tile may still be in flight
+    else if (PAIRS) wait_vmcnt<HALVES ? 6 : 8>();      // q has landed; 4 (2) mask and 4 K/V copies may still be in flight
+    else if (t_first < T) wait_vmcnt<COPIES>();        // q has landed; the copies of the first tile may still be in flight
     else wait_vmcnt<0>();
     // What only the end needs of the arguments, while q is on its way from LDS.  Requested with the others at the start (as the compiler has it) ->
     // behind the first copies -> here, the grid's size among the first arguments; small calls back to back: 2 heads, N = 128, D = 64 4.78 -> 4.64 ->
@@ -1045,21 +1091,30 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         // a pair are always followed by exactly four younger copies when they are needed.  (The stores
         // of the by-products, when asked for, only add to the count: copies complete in the order of
         // their requests, so "at most four outstanding" still means that all older copies are in.)
+        // HALVES: a wavefront reads bytes that another has copied, behind the even visit's barrier; the next pair's are requested then
+        // into the other slot, whose bytes were read before the odd visit's barrier.
         for (int t = 0; t < T; t += 2) {
             progress();
-            wait_vmcnt<4>();                                  // this wave's bytes of the pair have landed
-            const u32x2 w_even = mask_words(t, 0, 0);
-            u32x2 w_odd = {0u, 0u};
-            if (WHOLE || t + 1 < T) w_odd = mask_words(t + 1, 0, 1);
+            u32x2 w_even, w_odd = {0u, 0u};
+            auto words = [&]() __attribute__((always_inline)) {
+                const int slot = HALVES ? (t >> 1) & 1 : 0;
+                w_even = mask_words(t, slot, 0);
+                if (WHOLE || t + 1 < T) w_odd = mask_words(t + 1, slot, 1);
+            };
+            if constexpr (!HALVES) {
+                wait_vmcnt<4>();                              // this wave's bytes of the pair have landed
+                words();
+            }
             wait_vmcnt<0>();                                  // K/V of tile t
             if (!WHOLE && UNLIKELY(t == cut_tile)) zero_tail_rows(t, 0);
             __syncthreads();
+            if constexpr (HALVES) words();
             if (WHOLE || t + 1 < T) issue_kv(t + 1, integral_constant<int, 1>{});
             if (LIKELY(t + 2 < T)) issue_mask_pair((t >> 1) + 1);     // the words above are in registers: the bytes may go
             compute_tile(w_even, 0u);
             if (!WHOLE && t + 1 >= T) break;
             progress();
-            if (t + 2 < T) wait_vmcnt<4>(); else wait_vmcnt<0>();   // K/V of tile t + 1 (the next pair's bytes may be on their way)
+            if (t + 2 < T) wait_vmcnt<HALVES ? 2 : 4>(); else wait_vmcnt<0>();   // K/V of tile t + 1 (the next pair's bytes may be on their way)
             if (!WHOLE && UNLIKELY(t + 1 == cut_tile)) zero_tail_rows(t + 1, 1);
             __syncthreads();
             if (LIKELY(t + 2 < T)) issue_kv(t + 2, integral_constant<int, 0>{});
@@ -1210,7 +1265,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
 
 // The instance for (fp32 q, element type, post-multiplier, row strides) and the kind of mask: 0 packed words, 1
 // boolean bytes, 2 the same with by-products, 3 and 4 those with two tiles' bytes per request, 5 to 7 the first
-// three with the keys split between the wavefronts, 8 and 9 as 3 and 4 at any N, 10 to 12 the first three in halves.  This file is
+// three with the keys split between the wavefronts, 8 and 9 as 3 and 4 at any N; 10 to 14, 18 and 19 those ten less in halves.  This file is
 // compiled once per head dim for the instances, side by side, and once for the launcher.
 typedef void (*FwdKernel)(const AttnArgs);
 #ifdef SMA_FWD_HEAD_DIM
@@ -1230,11 +1285,15 @@ template <int HDIM, bool BF16, bool POSTMUL, bool PACKED_ROWS, bool WIDE_Q = fal
         case 4: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true, 1, false, WIDE_Q>;
         case 8: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, false, 2, false, WIDE_Q>;
         case 9: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true, 2, false, WIDE_Q>;
+        case 13: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, false, 1, false, WIDE_Q, true>;
+        case 14: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true, 1, false, WIDE_Q, true>;
+        case 18: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, false, 2, false, WIDE_Q, true>;
+        case 19: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true, 2, false, WIDE_Q, true>;
         }
     }
+    if (mask_kind == 10) return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, false, false, 0, false, WIDE_Q, true>;
     if constexpr (HDIM > 64) {
         switch (mask_kind) {
-        case 10: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, false, false, 0, false, WIDE_Q, true>;
         case 11: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, false, 0, false, WIDE_Q, true>;
         case 12: return attn_fwd_kernel<BF16, POSTMUL, PACKED_ROWS, HDIM, true, true, 0, false, WIDE_Q, true>;
         }
@@ -1302,11 +1361,18 @@ hipError_t launch_attn_fwd(const AttnArgs &args, bool bf16, hipStream_t stream)
             if (e != hipSuccess) return e;
         }
     }
-    // Beyond that line work-groups of 64 rows (HALVES at the kernel) while one on a CU holds them all, at head dims beyond 64.  With two on a
-    // CU they lose (8 x 8 heads, N = 512, D = 128: 17.0 -> 17.8 us), up to 64, where three share a CU, they gain and lose by turns (packed, 48 heads,
-    // N = 1024: 24.3 -> 22.2; 64, N = 512: 11.7 -> 12.1, boolean 13.1), and up to 128 keys there is nothing to share (6.6 us either way).
-    // The split stays ahead where it fits: 8 heads, N = 1024 16.9 against 21.3 us.
-    const bool halves = !split && a.D > HD && a.N > 2 * BN && (long long)a.BH * ((a.N + 63) / 64) <= cus;
+    // Beyond that line work-groups of 64 rows (HALVES at the kernel), `g64` of them:
+    //   head dims beyond 64, where two share a CU: while one on a CU holds them all.  With two on a CU they lose (8 x 8 heads, N = 512, D = 128: 17.0 -> 17.8 us;
+    //       32, N = 1024 22.9 -> 23.1, boolean 24.7 -> 25.3), but at head dim 96 from 1024 rows on, where they gain as long as these are one round: 10 heads, N = 2048
+    //       35.5 -> 30.7 (boolean 39.5 -> 36.6, untouched masks 42.1 -> 39.9), 32, N = 1024 20.5 -> 19.5 (22.3 -> 22.0, 24.7 -> 24.8); 64, N = 512 13.5 -> 14.0;
+    //   up to 64, where three do: when they are one round of two to three on a CU and work-groups of 128 rows would be one on some CUs and two on others.  Up
+    //       to two on a CU, packed masks gain and boolean ones lose (32 heads, N = 1024: 16.4 -> 15.2; untouched 18.3 -> 18.7), and with a second
+    //       round all do (28, N = 2048: 40.7 -> 45.8, boolean 44.6 -> 61.5).  Beyond ten tiles, where the chain is most of a call: 48, N = 1024 24.2 -> 20.3, 160, N = 256
+    //       9.7 -> 8.9; and a training step on up to 640 rows, whose backward holds whole heads, keeps a head's bits however many heads there are.
+    // Up to 128 keys there is nothing to share (6.6 us either way).  The split stays ahead where it fits: 8 heads, N = 1024 16.9 against 21.3 us.
+    const long long g64 = (long long)a.BH * ((a.N + 63) / 64);
+    const bool halves = !split && a.N > 2 * BN &&
+                        (a.D > HD ? g64 <= (a.D <= 96 && a.N >= 1024 ? 2 * cus : cus) : a.N > 10 * BN && g64 > 2 * cus && g64 <= 3 * cus);
     if (halves) {
         a.qtiles = (a.N + 63) / 64;
         groups = (long long)a.BH * a.qtiles;
@@ -1322,7 +1388,7 @@ hipError_t launch_attn_fwd(const AttnArgs &args, bool bf16, hipStream_t stream)
     const bool byproducts = a.mask_out != nullptr || a.map_out != nullptr;
     // two tiles' mask bytes per request (see PAIRS at the kernel), unless the grid is the single round of work-groups in
     // step for which tail_start was set to 0 above
-    const bool further = !split && !halves && a.byte_mask && D <= HD && a.tail_start != 0;
+    const bool further = !split && a.byte_mask && D <= HD && (halves || a.tail_start != 0);
     if (a.q_f32 && !bf16) return hipErrorInvalidValue;         // fp32 callers compute in bf16
     if (a.byte_mask && a.N < 16) return hipErrorInvalidValue;  // a row holds at least one 16-byte copy (checked by the C-ABI layer)
     const int mask_kind = (split ? 5 : halves ? 10 : 0) + (!a.byte_mask ? 0 : (!further ? 1 : a.N % (2 * BN) == 0 ? 3 : 8) + (byproducts ? 1 : 0));

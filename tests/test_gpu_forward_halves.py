@@ -1,5 +1,5 @@
 """The forward whose work-groups have 64 rows and whose wavefronts share the keys of every tile (head dims beyond 64, grids of at most one such
-work-group on a CU)."""
+work-group on a CU; the others further down)."""
 import importlib
 import sys
 
@@ -92,3 +92,44 @@ def test_map_by_product(dev, heads, N):
     plain = sa.sparse_attention(*leaves, mask)
     assert torch.equal(out, plain)
     assert all(torch.equal(x, y) for x, y in zip(torch.autograd.grad(out, leaves, do), torch.autograd.grad(plain, leaves, do)))
+
+
+# Head dims up to 64 (three work-groups share a CU): one round of more than two of 64 rows on each, beyond ten tiles; and head dim 96 from 1024 rows on, up
+# to two.  Pairs of tiles that end in either of their tiles, whole ones (N a multiple of 128), one key beyond a tile and one short of it, a walk over two map
+# words.
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("heads, N, D", [(50, 641, 64), (48, 704, 32), (44, 705, 64), (60, 767, 40), (50, 768, 32), (33, 1023, 64), (33, 1024, 64), (36, 1025, 48),
+                                         (17, 2100, 64), (30, 1025, 80), (10, 2048, 96)])
+def test_one_round_of_64_row_groups(dev, heads, N, D, dtype):
+    sa = _sa()
+    g = torch.Generator(device=dev).manual_seed(N + D)
+    q, k, v = (torch.randn(1, heads, N, D, device=dev, generator=g).to(dtype) for _ in range(3))
+    nb = (N + 63) // 64
+    blocks = torch.rand(1, 1, nb, nb, device=dev, generator=g) < 0.6
+    mask = (torch.rand(1, 1, N, N, device=dev, generator=g) < 0.3) & blocks.repeat_interleave(64, 2)[:, :, :N].repeat_interleave(64, 3)[..., :N]
+    mask[..., 3, :] = False
+    mask[..., 4, :] = torch.arange(N, device=dev) == N - 1
+    odd = (mask.to(torch.uint8) * 6).view(torch.bool)                  # bytes that are neither 0 nor 1
+    packed = sa.pack_mask(mask)
+    tile_map = sa.tile_map(packed, min_skip=0.0)
+    leaves = [t.detach().requires_grad_(True) for t in (q, k, v)]
+    made = []
+    ran = launches(lambda: made.extend([sa.sparse_attention_func(q, k, v, mask), sa.sparse_attention_func(q, k, v, odd),
+                                        sa.sparse_attention_func(q, k, v, None, mask_packed=packed),
+                                        sa.sparse_attention_func(q, k, v, None, mask_packed=packed, tile_map=tile_map),
+                                        sa.sparse_attention(*leaves, mask, tile_map=True)]))
+    assert [args[9] for name, args, _ in ran if name == "attn_fwd_kernel"] == ["true"] * 5, ran           # HALVES
+    out = made[0]
+    assert all(torch.equal(out, x) for x in made[1:])
+    lse, words = made[4].grad_fn.saved_tensors[4:6]
+    assert torch.equal(words.view_as(packed), packed) and torch.equal(made[4].grad_fn.tile_map.flatten(), tile_map.flatten())
+    # the bounds of the first test
+    eps = 2.0 ** (-10 if dtype == torch.float16 else -7)
+    for h in (0, heads - 1):
+        one = [t[:, h:h + 1].double() if dtype != torch.float32 else t[:, h:h + 1].bfloat16().double() for t in (q, k, v)]
+        x = ((one[0] * D ** -0.5) @ one[1].transpose(-1, -2)).masked_fill(~mask, float("-inf"))
+        ref, want_lse = torch.softmax(x, -1).nan_to_num() @ one[2], torch.logsumexp(x, -1)
+        shift = (eps * (one[0].abs() * D ** -0.5) @ one[1].abs().transpose(-1, -2)).masked_fill(~mask, 0).amax(-1)
+        err = (out[:, h:h + 1].double() - ref).abs()
+        assert (err <= 1e-4 + one[2].abs().max() * (4 * eps + 2 * shift[..., None])).all(), float(err.max())
+        assert ((lse[:, h:h + 1].double() - want_lse).abs() <= 1e-4 + shift)[torch.isfinite(want_lse)].all() and torch.isinf(lse[:, h, 3]).all()
