@@ -35,7 +35,7 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 LIB_NAME = "libsma_hip.so"
 MODULE_NAME = "sparse_attn_cuda"
 HIP_SOURCES = ["attn_fwd.hip", "attn_bwd.hip", "attn_bwd_head.hip", "pack_mask.hip", "capi.hip"]
-FWD_HEAD_DIMS = (32, 64, 96, 128)      # attn_fwd.hip is compiled once for each, for their kernels
+FWD_HEAD_DIMS = (32, 64, 80, 96, 128)      # attn_fwd.hip is compiled once for each, for their kernels
 PROBE_DIR = os.path.join(HERE, "benchprobe")
 PROBE_LIB_NAME = "libsma_probe.so"
 GPU_ARCH = "gfx950"

@@ -47,7 +47,7 @@
 // halves, the others (dQ, dK, dV) fill one pair of accumulators per half.  Head dim 32 uses half a tile: the copies fill the upper half of
 // every LDS row with copies of the row's last 16 bytes, which are never read;
 // contractions over the head dim take one MFMA step and the outputs have two 16-column blocks.  Head dim 96
-// is 128 with such a half tile as its second half: three steps, six blocks.
+// is 128 with such a half tile as its second half: three steps, six blocks; 80 the same with five.
 #include "attn_bwd_common.h"
 
 namespace sma {
@@ -140,7 +140,7 @@ __device__ __forceinline__ void dq_rows(const AttnBwdArgs &a, unsigned char *sme
 {
     using E = Elem<BF16>;
     constexpr int NH = HDIM > 64 ? 2 : 1;         // 64-column tiles per matrix
-    constexpr int KS = HDIM / 32;                 // MFMA steps of a contraction over the head dim
+    constexpr int KS = (HDIM + 31) / 32;          // MFMA steps of a contraction over the head dim
     constexpr int DB = HDIM / 16;                 // 16-column accumulator blocks of an output
     constexpr int AHEAD = HDIM <= 64 ? 2 : 3;     // steps by which an operand is requested before its use
     using C = Cfg<NH>;
@@ -390,7 +390,7 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
 {
     using E = Elem<BF16>;
     constexpr int NH = HDIM > 64 ? 2 : 1;
-    constexpr int KS = HDIM / 32;
+    constexpr int KS = (HDIM + 31) / 32;
     constexpr int DB = HDIM / 16;
     constexpr int AHEAD = VLDS || HDIM == 32 ? 2 : 3;             // one more where there are registers for it
     using C = DkvCfg<HDIM, NW, VLDS>;
@@ -830,6 +830,7 @@ hipError_t launch_attn_bwd(const AttnBwdArgs &args, bool bf16, hipStream_t strea
     switch (kernel_head_dim(a.D)) {
     case 128: launch_head_dim<128>(bf16, stream, a); break;
     case 96: launch_head_dim<96>(bf16, stream, a); break;
+    case 80: launch_head_dim<80>(bf16, stream, a); break;
     case 64: launch_head_dim<64>(bf16, stream, a); break;
     default: launch_head_dim<32>(bf16, stream, a); break;
     }

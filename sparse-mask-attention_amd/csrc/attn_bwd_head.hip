@@ -533,7 +533,7 @@ template <bool BF16, bool WIDE> bool pick(hipStream_t stream, const AttnBwdArgs 
         return true;
     };
     return D == 32 ? narrow(std::integral_constant<int, 32>{}) : D == 64 ? narrow(std::integral_constant<int, 64>{})
-           : D == 96 ? wide(std::integral_constant<int, 96>{}) : wide(std::integral_constant<int, 128>{});
+           : D <= 96 ? wide(std::integral_constant<int, 96>{}) : wide(std::integral_constant<int, 128>{});
 }
 
 }  // namespace

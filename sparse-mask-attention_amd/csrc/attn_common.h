@@ -294,7 +294,7 @@ __device__ __forceinline__ void store_rows(const f32x4 (&acc)[2][NB], const floa
 {
     store_block<BF16, NB == 2 ? 32 : 64, 0>(acc, mult, lds_wave, dst, has_h, has_f, row0, N, lane);
     if constexpr (NB > 4)
-        store_block<BF16, NB == 6 ? 32 : 64, 4>(acc, mult, lds_wave + stride, columns_from(dst, 64), has_h, has_f, row0, N, lane);
+        store_block<BF16, NB < 8 ? 16 * (NB - 4) : 64, 4>(acc, mult, lds_wave + stride, columns_from(dst, 64), has_h, has_f, row0, N, lane);
 }
 
 }  // namespace

@@ -81,6 +81,7 @@ constexpr float SUM_LIMIT = 16384.0f;     // a lane's 32 weights of a tile sum t
 //        two 16-column blocks of V.
 //   96   128 with such a half tile as its second half: three steps, six blocks.  D = 80 and 96 ran in the
 //        128 kernel before, through zero-padded copies (16 x 8 heads, N = 1088, D = 96: 156 -> 81 us)
+//   80   as 96 with five blocks (what that gives stands at kernel_head_dim)
 //
 // BYTEMASK: the mask arrives as the caller's boolean bytes (one per score, 0 or 1) instead of packed
 // words.  Each wavefront copies the 32 x 64 bytes of a tile for its rows into LDS and turns them
@@ -172,7 +173,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     constexpr bool HALF_BYTES = HALVES && BYTEMASK && !BYPRODUCTS;
     using E = Elem<BF16>;
     constexpr int NH = HDIM > 64 ? 2 : 1;         // 64-column tiles per matrix
-    constexpr int KS = HDIM / 32;                 // MFMA steps of the QK^T chain
+    constexpr int KS = (HDIM + 31) / 32;          // MFMA steps of the QK^T chain
     constexpr int DB = HDIM / 16;                 // 16-column accumulator blocks of O
     constexpr int AHEAD = SPLIT ? 4 : HDIM <= 64 ? 2 : 3;              // steps by which an operand is requested before its use: scores
     constexpr int V_AHEAD = SPLIT ? DB * 2 < 8 ? DB * 2 : 8 : HDIM <= 64 ? 4 : 6;             // ... and values, when the scores' registers are free
@@ -797,7 +798,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 t[i] = E::pack2_rne(E::up1((uint16_t)(t[i] & 0xffffu)) * a.q_scale, E::up1((uint16_t)(t[i] >> 16)) * a.q_scale);
-            if (!PACKED_ROWS && 4 * c + q4 > last_chunk) t = u32x4{0u, 0u, 0u, 0u};      // beyond the row: adds nothing
+            if ((!PACKED_ROWS || HDIM % 32 != 0) && 4 * c + q4 > last_chunk) t = u32x4{0u, 0u, 0u, 0u};      // beyond the row: adds nothing
         }
 
     if constexpr (SPLIT) {
@@ -1323,6 +1324,7 @@ FwdKernel SMA_NAME(SMA_FWD_HEAD_DIM)(int variant, int mask_kind) { return pick<S
 #else
 FwdKernel fwd_kernel_32(int variant, int mask_kind);
 FwdKernel fwd_kernel_64(int variant, int mask_kind);
+FwdKernel fwd_kernel_80(int variant, int mask_kind);
 FwdKernel fwd_kernel_96(int variant, int mask_kind);
 FwdKernel fwd_kernel_128(int variant, int mask_kind);
 
@@ -1394,7 +1396,7 @@ hipError_t launch_attn_fwd(const AttnArgs &args, bool bf16, hipStream_t stream)
     const int mask_kind = (split ? 5 : halves ? 10 : 0) + (!a.byte_mask ? 0 : (!further ? 1 : a.N % (2 * BN) == 0 ? 3 : 8) + (byproducts ? 1 : 0));
     const int variant = (a.q_f32 ? 8 : 0) | (bf16 ? 4 : 0) | (postmul ? 2 : 0) | (packed ? 1 : 0);
     const FwdKernel kernel = D == 32 ? fwd_kernel_32(variant, mask_kind) : D == 64 ? fwd_kernel_64(variant, mask_kind)
-                             : D == 96 ? fwd_kernel_96(variant, mask_kind) : fwd_kernel_128(variant, mask_kind);
+                             : D == 80 ? fwd_kernel_80(variant, mask_kind) : D == 96 ? fwd_kernel_96(variant, mask_kind) : fwd_kernel_128(variant, mask_kind);
     hipLaunchKernelGGL(kernel, grid, block, 0, stream, a);
     return hipGetLastError();
 }

@@ -177,10 +177,16 @@ struct AttnBwdArgs {
     uint32_t last_mask0, last_mask1;
 };
 
-// The kernels exist for head dims of 32, 64, 96 and 128; any multiple of 8 in between runs in the next larger
+// The kernels exist for head dims of 32, 64, 80, 96 and 128; any multiple of 8 in between runs in the next larger
 // one: the copies fill an LDS row beyond the tensor's with its last 16 bytes once more, the fragments that the
 // wavefronts hold in registers are zero there, and results beyond it are not stored.
-inline int kernel_head_dim(int D) { return D <= 32 ? 32 : D <= 64 ? 64 : D <= 96 ? 96 : 128; }
+// 80 differs from 96 in what has the head dim as its result (O, dQ, dK, dV): five blocks of 16 columns instead of six, one product in 12 less in the
+// forward, in 18 in dQ, in 12 in dK/dV, with the operands read for them; the contractions take three steps of 32 in either.  (The whole-head backward, up
+// to 256 keys, has none of its own.)  The kernels for 96 -> this, us, D = 80: training 128 heads, N = 2048 838 -> 801, 64, N = 1500 258 -> 246, 4,
+// N = 3000 121 -> 116, 192, N = 1024, blocks with a map 211 -> 202, 128, N = 700 151 -> 147;  forward 64, N = 1500 82.2 -> 79.6, 128, N = 2048, packed 214 -> 206,
+// causal 132 -> 125, 1024, N = 64 12.5 -> 11.7, 2, N = 333 9.98 -> 9.28, 128, N = 700, bound by the mask's bytes, 41.9 either way.  D = 72 the same (512 heads,
+// N = 300, training 144.7 -> 140.9).
+inline int kernel_head_dim(int D) { return D <= 32 ? 32 : D <= 64 ? 64 : D <= 80 ? 80 : D <= 96 ? 96 : 128; }
 
 // Number of compute units of the current device (asked for once).
 int compute_units();

@@ -6,6 +6,7 @@ import sys
 import pytest
 import torch
 
+from _launches import launches
 from oracle import sma_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -44,3 +45,44 @@ def test_head_dims_between_the_kernels(dev, N, D):
         assert torch.equal(a.float(), b)                     # fp32 callers get the bf16 results, widened
     for got, want in zip(results[torch.float32], [ref.detach()] + [t.grad for t in refs]):
         assert ((got.cpu() - want).abs() <= 1e-4 + 2e-2 * want.abs().max() + 2e-2 * want.abs()).all()
+
+
+# 65 to 80 have kernels with five blocks of 16 result columns: the second 64 columns of a row's store are 16 wide.  One key beyond whole tiles, few heads (dQ
+# and dK/dV in one launch) and more than fit that, a walk over tiles of a map.
+@pytest.mark.parametrize("D", [72, 80])
+@pytest.mark.parametrize("heads, N, blocks", [(3, 257, False), (80, 300, False), (60, 577, True), (34, 1024, False), (4, 1025, True)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_kernels_for_80(dev, heads, N, blocks, D, dtype):
+    importlib.import_module("python.sparse_attention")
+    sa = sys.modules["python.sparse_attention"]
+    g = torch.Generator(device=dev).manual_seed(N + D)
+    rounded = torch.bfloat16 if dtype == torch.float32 else dtype
+    leaves = []
+    for _ in range(4):                                       # rows between columns of NaN
+        buf = torch.full((1, N, heads, D + 8), float("nan"), dtype=dtype, device=dev)
+        view = buf[..., :D].transpose(1, 2)
+        view.copy_(torch.randn(1, heads, N, D, device=dev, generator=g).to(rounded))
+        leaves.append(view)
+    q, k, v, do = leaves
+    mask = torch.rand(1, 1, N, N, device=dev, generator=g) < 0.3
+    if blocks:
+        nb = (N + 63) // 64
+        mask &= (torch.rand(1, 1, nb, nb, device=dev, generator=g) < 0.5).repeat_interleave(64, 2)[:, :, :N].repeat_interleave(64, 3)[..., :N]
+    mask[..., 5, :] = False
+    qkv = [t.detach().requires_grad_(True) for t in (q, k, v)]
+    made = []
+
+    def step():
+        out = sa.sparse_attention(*qkv, mask, tile_map=True if blocks else None)
+        made.extend([out.detach(), *torch.autograd.grad(out, qkv, do)])
+    ran = [(name, args) for name, args, _ in launches(step) if name.startswith("attn_") and name != "attn_bwd_delta_kernel"]
+    assert {name: args[3 if name == "attn_fwd_kernel" else 1] for name, args in ran} == {name: "80" for name, _ in ran}, ran
+    dense = [t.contiguous().detach().requires_grad_(True) for t in (q, k, v)]
+    out = sa.sparse_attention(*dense, mask, tile_map=True if blocks else None)
+    assert all(torch.equal(a, b) for a, b in zip(made, [out.detach(), *torch.autograd.grad(out, dense, do.contiguous())]))
+    for h in (0, heads - 1):
+        one = [t[:, h:h + 1].detach().double().requires_grad_(True) for t in (q, k, v)]
+        ref = O.sparse_attention_ref(*one, mask)
+        wanted = [ref.detach(), *torch.autograd.grad(ref, one, do[:, h:h + 1].double())]
+        for got, want in zip(made, wanted):                  # the bound of the test above
+            assert ((got[:, h:h + 1].double() - want).abs() <= 1e-4 + 2e-2 * want.abs().max() + 2e-2 * want.abs()).all()
