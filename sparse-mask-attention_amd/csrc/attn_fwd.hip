@@ -88,14 +88,23 @@ constexpr float SUM_LIMIT = 16384.0f;     // a lane's 32 weights of a tile sum t
 // into the two words per row itself (eight dot products with the weights 1, 2, 4 .. 128 per lane
 // and one exchange between the lane halves): the separate packing pass, its launch and the
 // round trip of the words through memory disappear for a mask that is used once.
-template <int NH, bool BYTEMASK, bool SPLIT> struct Cfg {
+// SECOND: bytes of a row in the second column half's tile (head dims beyond 64).  At head dims 80 and 96, but with SPLIT, the rows there are only as long as
+// what is used of them: 32 and 64 bytes, of which one request fills 32 or 16 rows.  A wavefront requests five or six pieces of K and V a tile instead of eight, and a stage is 20
+// or 24 KiB instead of 32, which is what lets three work-groups share a CU (see three_on_a_cu).  Whole rows -> this with two on a CU all the same: D = 80, 512 heads, N = 320 33.7 ->
+// 32.4 us, N = 512 67.1 -> 65.4; D = 96 36.4 -> 35.9, 69.9 -> 68.5.  64 bytes where by-products are asked for at 80 (two on a CU: 32, whose reads of K's last step
+// meet in a bank, cost 64 heads, N = 1500 in training 281 -> 285 us, 64 282), and whole rows for fp32 queries at 96 (64, N = 1500 104.0 -> 109.5).
+constexpr int second_row(int hdim, bool split, bool byproducts, bool wide_q)
+{
+    return hdim <= 64 ? 0 : split || hdim == 128 || (hdim == 96 && wide_q) ? 128 : hdim == 96 || byproducts ? 64 : 32;
+}
+template <int NH, bool BYTEMASK, bool SPLIT, int SECOND> struct Cfg {
     // SPLIT: one K and one V buffer for each of the four wavefronts, else a ring of two stages: copies run one tile ahead
     static constexpr int NSTAGE = SPLIT ? 4 : 2;
     static constexpr int MASK_COPIES = BYTEMASK ? 2 : 1;
-    static constexpr int COPIES = MASK_COPIES + 4 * NH;             // async copies per wave and tile
+    static constexpr int COPIES = MASK_COPIES + 4 + (SECOND == 32 ? 1 : SECOND / 32);    // async copies per wave and tile
     // LDS map (bytes), after the 256 of the table of the mask bias, which lies first: a read's immediate offset reaches 64 KiB
-    static constexpr int STAGE_BYTES = 2 * NH * TILE_BYTES;         // K halves, then V halves
-    static constexpr int OFF_V = NH * TILE_BYTES;                   // V inside a stage
+    static constexpr int OFF_V = TILE_BYTES + BN * SECOND;          // V inside a stage
+    static constexpr int STAGE_BYTES = 2 * OFF_V;                   // K halves, then V halves
     // mask: packed words in NSTAGE slots of 4 waves x 64 words; bytes in slots of 4 waves x 2 KiB,
     // two of them for head dims up to 64 and, for want of LDS, ONE for 128: a wave has turned its
     // bytes into words before it requests the next tile's (see the main loop), so one slot is
@@ -113,6 +122,18 @@ template <int NH, bool BYTEMASK, bool SPLIT> struct Cfg {
     static constexpr int LUT_BYTES = 256;                           // 16 x 16 B
     static constexpr int LDS_BYTES = LUT_BYTES + (BYTEMASK && !SPLIT ? OFF_MAP_ARRIVED + 16 : OFF_MAP);
 };
+
+// Head dims beyond 64 of which three work-groups share a CU (but with SPLIT): where 168 registers hold the loop, with operands requested no further ahead
+// than at head dim 64 (by-products: 34 spilled at 80;  fp32 queries at 96: 32), and the LDS three of them (the boolean mask's bytes at 96 do not fit).  A visit is bound by its chain of
+// products, exponentials and products, which a third wavefront on the SIMD fills.  Two (with whole rows in the second half) -> three, us:
+//   D = 80   packed 128 heads, N = 2048 206 -> 183, causal 125 -> 116;  192, N = 1024, blocks with a map 55.8 -> 49.0;  192, N = 512 27.1 -> 22.6;  512, N = 256 21.5 -> 19.2;
+//            2048, N = 64 20.0 -> 17.2;  boolean 64, N = 1500 79.6 -> 73.0;  128, N = 700 41.9 -> 37.5;  fp32 64, N = 1500 99.6 -> 93.1
+//   D = 96   packed 128, N = 2048 220 -> 202, causal 133 -> 125;  64, N = 1500 66.2 -> 58.0;  192, N = 1024, blocks with a map 58.1 -> 52.8;  192, N = 512 26.6 -> 23.2
+// Work-groups of 64 rows (HALVES) have the registers anyway: 8 heads, N = 3000, boolean D = 80 50.8 -> 49.1, 96 56.4 -> 50.9.
+constexpr bool three_on_a_cu(int hdim, bool bytemask, bool byproducts, bool wide_q)
+{
+    return !byproducts && (hdim == 80 || (hdim == 96 && !bytemask && !wide_q));
+}
 
 // The kernel's arguments where they lie.  What is read through this is requested no earlier than here: arguments are fetched from the host's
 // memory, and a work-group can request no data before those that the compiler has moved to its start have arrived.
@@ -154,7 +175,7 @@ template <int N> __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_
 // 1.4 times as long.
 template <bool BF16, bool POSTMUL, bool PACKED_ROWS, int HDIM, bool BYTEMASK = false, bool BYPRODUCTS = false,
           int FETCH = 0, bool SPLIT = false, bool WIDE_Q = false, bool HALVES = false>
-__global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ? 2 : 3) void attn_fwd_kernel(const AttnArgs a)
+__global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ? (three_on_a_cu(HDIM, BYTEMASK, BYPRODUCTS, WIDE_Q) ? 3 : 2) : 3) void attn_fwd_kernel(const AttnArgs a)
 {
     // HALVES: a work-group of 64 rows, two wavefronts to each 32 of them, which take 32 keys of every tile each and add their
     // sums at the end.  A visit's chain of products, exponentials and products is half as long, which is what bounds a grid whose work-groups of 128
@@ -175,11 +196,14 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     constexpr int NH = HDIM > 64 ? 2 : 1;         // 64-column tiles per matrix
     constexpr int KS = (HDIM + 31) / 32;          // MFMA steps of the QK^T chain
     constexpr int DB = HDIM / 16;                 // 16-column accumulator blocks of O
-    constexpr int AHEAD = SPLIT ? 4 : HDIM <= 64 ? 2 : 3;              // steps by which an operand is requested before its use: scores
-    constexpr int V_AHEAD = SPLIT ? DB * 2 < 8 ? DB * 2 : 8 : HDIM <= 64 ? 4 : 6;             // ... and values, when the scores' registers are free
+    constexpr bool THIRD = !SPLIT && !HALVES && three_on_a_cu(HDIM, BYTEMASK, BYPRODUCTS, WIDE_Q);
+    constexpr int AHEAD = SPLIT ? 4 : HDIM <= 64 || THIRD ? 2 : 3;              // steps by which an operand is requested before its use: scores
+    constexpr int V_AHEAD = SPLIT ? DB * 2 < 8 ? DB * 2 : 8 : HDIM <= 64 || THIRD ? 4 : 6;             // ... and values, when the scores' registers are free
     // second column half at a constant distance from the first in every row
     constexpr bool SAME_HALVES = HDIM == 128 && PACKED_ROWS;
-    using C = Cfg<NH, BYTEMASK, SPLIT>;
+    constexpr int SECOND = second_row(HDIM, SPLIT, BYPRODUCTS, WIDE_Q);
+    constexpr bool NARROW = SECOND == 32 || SECOND == 64;
+    using C = Cfg<NH, BYTEMASK, SPLIT, SECOND>;
     constexpr int NSTAGE = C::NSTAGE, STAGE_BYTES = C::STAGE_BYTES, OFF_MASK = C::OFF_MASK;
     constexpr int MASK_SLOT = C::MASK_SLOT, COPIES = C::COPIES - (HALF_BYTES ? 1 : 0);
     const int D = PACKED_ROWS ? HDIM : a.D;
@@ -259,15 +283,17 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     // holds the end are shifted to their places below, those of later chunks cleared as pad bits.
     const int mrow = BYTEMASK ? 0 : row_base + (lane >> 1);
     uint32_t m_voff = BYTEMASK ? 0u : (uint32_t)(((size_t)(mrow < N ? mrow : N - 1) * nw + (lane & 1)) * 4);
-    uint32_t mb_voff[2] = {0u, 0u}, mb_chunk[2] = {0u, 0u};
+    uint32_t mb_voff[2] = {0u, 0u};
+    auto mb_chunk = [&](int l) __attribute__((always_inline)) -> uint32_t {
+        return HALF_BYTES ? 32 * half + (((l & 1) ^ ((l >> 4) & 1)) << 4) : ((l & 3) ^ ((l >> 4) & 3)) << 4;
+    };
     if constexpr (BYTEMASK) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             // (HALF_BYTES: row i/2, position i%2, of the wavefront's two chunks the one at position ^ ((row >> 3) & 1))
             const int row = HALF_BYTES ? lane >> 1 : 16 * j + (lane >> 2);
             const int grow = row_base + row;
-            mb_chunk[j] = HALF_BYTES ? (uint32_t)(32 * half + (((lane & 1) ^ ((row >> 3) & 1)) << 4)) : (uint32_t)(((lane & 3) ^ ((row >> 2) & 3)) << 4);
-            mb_voff[j] = (uint32_t)(grow < N ? grow : N - 1) * (uint32_t)N + mb_chunk[j];
+            mb_voff[j] = (uint32_t)(grow < N ? grow : N - 1) * (uint32_t)N + mb_chunk(lane);
         }
     }
     const uint32_t mask_dst = lds0 + wave * (BYTEMASK ? 2048 : 256);
@@ -284,10 +310,13 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
                 // row_end = N >= 16 and nothing goes below zero)
                 const uint32_t back = x > 0 ? 16u : 0u;
                 src -= back;
+                int l = lane;
+                if constexpr (NARROW) asm volatile("" : "+v"(l));      // opaque: no register across the loop for what follows from it
+                const uint32_t end = mb_chunk(l) + 16;
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
                     mb_voff[j] += back;
-                    if (mb_chunk[j] + 16 > row_end) mb_voff[j] -= mb_chunk[j] + 16 - row_end;
+                    if (end > row_end) mb_voff[j] -= end - row_end;
                 }
             }
             async_copy_b128_at<OFF_MASK + SLOT * MASK_SLOT>(mask_dst, src, mb_voff[0]);
@@ -528,13 +557,17 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         }
         return w;
     };
+    auto narrow_swizzle = [](int row) __attribute__((always_inline)) { return (0x1320 >> (4 * ((row >> 2) & 3))) & 3; };      // 0, 2, 3, 1
     // ---- K/V tiles: async copies --------------------------------------------------------------
     // One global_load_lds_dwordx4 fills 1 KiB = 8 tile rows.  Wave w copies row blocks 2w, 2w+1 of
     // K and of V.  Lane i fills LDS chunk (row = 8*blk + i/8, position i%8) with the global chunk
     // position ^ swz(row):   K: swz(row) = (row >> 1) & 7      V: swz(row) = bitrev3((row >> 1) & 7)
     // (a chunk beyond the row's last is read as that one)
     auto chunk_at = [&](int c) __attribute__((always_inline)) -> uint32_t { return (uint32_t)(c < last_chunk ? c : last_chunk) << 4; };
+    // NARROW (short rows in the second half): the second halves' tiles, K then V, as one series of pieces of 1 KiB (lane i: row i / 2 or i / 4 of it); at 64 bytes a row wave w copies piece w of
+    // either, at 32 piece w of the four.  Their swizzle, K and V alike, is narrow_swizzle: none at 32 bytes.
     uint32_t kv_voff[2][2], kv_voff2[2][2];       // first and second column half
+    auto row2_of = [&](int l) __attribute__((always_inline)) { return SECOND == 32 ? 32 * (wave & 1) + (l >> 1) : 16 * wave + (l >> 2); };      // the tile row of a lane's piece
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const int row = 8 * (SPLIT ? j : 2 * wave + j) + (lane >> 3);       // SPLIT: the wave copies rows 16i + these too
@@ -547,6 +580,15 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         kv_voff2[0][j] = SAME_HALVES ? kv_voff[0][j] + 2 * HD : __umul24(row, k_rb) + chunk_at(8 + (pos ^ f));
         kv_voff2[1][j] = SAME_HALVES ? kv_voff[1][j] + 2 * HD : __umul24(row, v_rb) + chunk_at(8 + (pos ^ fr));
     }
+    const bool takes_v2 = SECOND == 32 && wave >= 2;
+    const uint32_t rb2 = takes_v2 ? v_rb : k_rb;
+    if constexpr (NARROW) {
+        const int row2 = row2_of(lane);
+        const uint32_t c = chunk_at(8 + (SECOND == 32 ? lane & 1 : (lane & 3) ^ narrow_swizzle(row2)));
+        kv_voff2[0][0] = __umul24(row2, rb2) + c;
+        kv_voff2[1][0] = __umul24(row2, v_rb) + c;
+    }
+    const uint32_t kv_dst2 = lds0 + TILE_BYTES + (SECOND == 32 ? (takes_v2 ? C::OFF_V : 0) + (wave & 1) * 1024 : wave * 1024);
     const uint32_t kv_dst = lds0 + wave * 2048;
     auto issue_kv = [&](int t, auto stage_c) __attribute__((always_inline)) {
         constexpr int SO = decltype(stage_c)::value * STAGE_BYTES;
@@ -556,25 +598,39 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         if (UNLIKELY(t == cut_tile)) {        // rows beyond N: copy row N-1 instead (zeroed later); no tile follows this one
             int last0 = key0;
             asm volatile("" : "+s"(last0));   // opaque: keeps this once-only arithmetic out of the loop's registers
+            int l = lane;
+            if constexpr (NARROW) asm volatile("" : "+v"(l));
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                const int row = 8 * (2 * wave + j) + (lane >> 3);
+                const int row = 8 * (2 * wave + j) + (l >> 3);
                 const int over = last0 + row - (N - 1);
                 if (over > 0) {
                     kv_voff[0][j] -= __umul24(over, k_rb); kv_voff[1][j] -= __umul24(over, v_rb);
-                    kv_voff2[0][j] -= __umul24(over, k_rb); kv_voff2[1][j] -= __umul24(over, v_rb);
+                    if constexpr (!NARROW) { kv_voff2[0][j] -= __umul24(over, k_rb); kv_voff2[1][j] -= __umul24(over, v_rb); }
+                }
+            }
+            if constexpr (NARROW) {
+                const int over = last0 + row2_of(l) - (N - 1);
+                if (over > 0) {
+                    kv_voff2[0][0] -= __umul24(over, rb2);
+                    kv_voff2[1][0] -= __umul24(over, v_rb);
                 }
             }
         }
         async_copy2_b128_at<SO, SO + 1024>(kv_dst, ksrc, kv_voff[0][0], kv_voff[0][1]);
         if constexpr (SAME_HALVES) {          // 128 bytes further along each row
             async_copy2_b128_at<SO + TILE_BYTES, SO + TILE_BYTES + 1024>(kv_dst, ksrc + HD, kv_voff[0][0], kv_voff[0][1]);
-        } else if constexpr (NH == 2) {
+        } else if constexpr (NH == 2 && !NARROW) {
             async_copy2_b128_at<SO + TILE_BYTES, SO + TILE_BYTES + 1024>(kv_dst, ksrc, kv_voff2[0][0], kv_voff2[0][1]);
         }
         async_copy2_b128_at<SO + C::OFF_V, SO + C::OFF_V + 1024>(kv_dst, vsrc, kv_voff[1][0], kv_voff[1][1]);
         if constexpr (SAME_HALVES) {
             async_copy2_b128_at<SO + C::OFF_V + TILE_BYTES, SO + C::OFF_V + TILE_BYTES + 1024>(kv_dst, vsrc + HD, kv_voff[1][0], kv_voff[1][1]);
+        } else if constexpr (SECOND == 64) {
+            async_copy_b128_at<SO>(kv_dst2, ksrc, kv_voff2[0][0]);
+            async_copy_b128_at<SO + C::OFF_V>(kv_dst2, vsrc, kv_voff2[1][0]);
+        } else if constexpr (SECOND == 32) {
+            async_copy_b128_at<SO>(kv_dst2, takes_v2 ? vsrc : ksrc, kv_voff2[0][0]);
         } else if constexpr (NH == 2) {
             async_copy2_b128_at<SO + C::OFF_V + TILE_BYTES, SO + C::OFF_V + TILE_BYTES + 1024>(kv_dst, vsrc, kv_voff2[1][0], kv_voff2[1][1]);
         }
@@ -625,14 +681,25 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     };
     auto zero_tail_rows = [&](int t, int stage) __attribute__((always_inline)) {   // after the copies of the last tile have landed
         const int key0 = t * BN;
+        int l = lane;
+        if constexpr (NARROW) asm volatile("" : "+v"(l));        // as in issue_kv
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            const int row = 8 * (2 * wave + j) + (lane >> 3);
+            const int row = 8 * (2 * wave + j) + (l >> 3);
             if (key0 + row >= N) {
-                const uint32_t p = lds0 + stage * STAGE_BYTES + wave * 2048 + j * 1024 + lane * 16;
+                const uint32_t p = lds0 + stage * STAGE_BYTES + wave * 2048 + j * 1024 + l * 16;
                 const u32x4 z = {0u, 0u, 0u, 0u};
 #pragma unroll
-                for (int part = 0; part < 2 * NH; ++part) *(LDS_PTR(u32x4))(uintptr_t)(p + part * TILE_BYTES) = z;
+                for (int part = 0; part < (NARROW ? 2 : 2 * NH); ++part)
+                    *(LDS_PTR(u32x4))(uintptr_t)(p + (NARROW ? part * C::OFF_V : part * TILE_BYTES)) = z;
+            }
+        }
+        if constexpr (NARROW) {
+            if (key0 + row2_of(l) >= N) {
+                const uint32_t p = kv_dst2 + stage * STAGE_BYTES + l * 16;
+                const u32x4 z = {0u, 0u, 0u, 0u};
+                *(LDS_PTR(u32x4))(uintptr_t)p = z;
+                if constexpr (SECOND == 64) *(LDS_PTR(u32x4))(uintptr_t)(p + C::OFF_V) = z;
             }
         }
     };
@@ -641,12 +708,19 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     // K operand (block of 16 keys kb, step c): row 16kb + l16, chunk 4c + q4           -> (k_at ^ 64 (c % 2)) + 2048kb
     // V operand (16 columns db, block of 32 keys), read by ds_read_b64_tr_b16: the lane supplies
     //   rows 16x + 4q4 + (l16 >> 2), columns 16db + 4(l16 & 3) .. +3, x = 0, 1                -> (v_at ^ 32 (db % 4)) + 2048x
-    uint32_t k_at, v_at;
+    // NARROW, second column half: K's row and chunk at k2_at + SECOND (rows beyond), V's at v2_at, ^ 32: 16 columns further
+    uint32_t k_at, v_at, k2_at = 0u, v2_at = 0u;
     {
         const uint32_t own0 = SPLIT ? split_dst : lds0;
         const int r = 4 * q4 + (l16 >> 2);
         k_at = own0 + l16 * 128 + ((q4 ^ (l16 >> 1)) << 4);
         v_at = own0 + C::OFF_V + r * 128 + ((((l16 & 3) >> 1) ^ bitrev3(r >> 1)) << 4) + ((l16 & 1) << 3);
+        if constexpr (NARROW) {
+            // (80: what the lanes of the last two chunks read meets zeros of q, as where rows are whole; it is the row's last chunk there too)
+            const int chunk = SECOND == 32 ? (q4 < 1 ? q4 : 1) : q4 ^ narrow_swizzle(l16);
+            k2_at = own0 + TILE_BYTES + l16 * SECOND + (chunk << 4);
+            v2_at = own0 + C::OFF_V + TILE_BYTES + r * SECOND + ((((l16 & 3) >> 1) ^ (SECOND == 32 ? 0 : narrow_swizzle(r))) << 4) + ((l16 & 1) << 3);
+        }
     }
     const uint32_t nib_rotate = (4u * q4 + 28u) & 31u;     // right: the nibble of keys 4q4 .. 4q4 + 3 comes to bits 4 .. 7
     uint32_t nib_mask = 0xF0u, ones = E::ONES;             // in scalar registers: as literals they take four bytes more wherever they are used
@@ -663,7 +737,14 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     // compiler's waits for these loads also wait for the copies issued after them, which it knows nothing of.  As an instance of its own: decided at
     // run time, the other element types' loops came out 0.5 to 1 % slower.
     const uint32_t q_dst = SPLIT ? split_dst + C::OFF_V : lds0 + (NSTAGE - 1) * STAGE_BYTES + wave * 4096;
-    f32x4 wide[WIDE_Q ? 4 * NH : 1][2];
+    // NARROW: the second half of q behind the four wavefronts' first halves, SECOND bytes a row, in as many pieces
+    constexpr int Q2_PIECES = NARROW ? SECOND / 32 : 0;
+    const uint32_t q2_dst = lds0 + (NSTAGE - 1) * STAGE_BYTES + 16384 + wave * (32 * SECOND);
+    auto q2_row = [&](int j) __attribute__((always_inline)) { return SECOND == 32 ? lane >> 1 : 16 * j + (lane >> 2); };
+    auto q2_chunk = [&](int j) __attribute__((always_inline)) { return 8 + (SECOND == 32 ? lane & 1 : (lane & 3) ^ narrow_swizzle(q2_row(j))); };
+    f32x4 wide[WIDE_Q ? 4 * NH : 1][2], wide2[WIDE_Q && NARROW ? Q2_PIECES : 1][2];
+    constexpr int Q_PARTS = NARROW ? 1 : NH;             // column halves in whole rows
+    static_assert(!NARROW || 16384 + 128 * SECOND <= STAGE_BYTES, "q fits a stage");
     {
         const int qbase = row_base < N ? row_base : N - 1;   // wave-uniform
         const uint16_t *qsrc = qb + (size_t)qbase * q_sn;
@@ -679,7 +760,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
                 const float *src = reinterpret_cast<const float *>(a.q.p) + ((size_t)bi * a.q.sb8 + (size_t)hi * a.q.sh8) * 8 +
                                    (size_t)(qbase + lrow) * q_sn;
 #pragma unroll
-                for (int half = 0; half < NH; ++half) {
+                for (int half = 0; half < Q_PARTS; ++half) {
                     const f32x4 *x = reinterpret_cast<const f32x4 *>(src + (chunk_at(8 * half + c) >> 1));
                     wide[NH * j + half][0] = x[0];
                     wide[NH * j + half][1] = x[1];
@@ -687,7 +768,20 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
                 continue;
             }
             async_copy_b128(dst + j * 1024, qsrc, __umul24(lrow, q_rb) + chunk_at(c));
-            if constexpr (NH == 2) async_copy_b128(dst + Q_HALF + j * 1024, qsrc, __umul24(lrow, q_rb) + chunk_at(8 + c));
+            if constexpr (NH == 2 && !NARROW) async_copy_b128(dst + Q_HALF + j * 1024, qsrc, __umul24(lrow, q_rb) + chunk_at(8 + c));
+        }
+#pragma unroll
+        for (int j = 0; j < Q2_PIECES; ++j) {
+            const int row = q2_row(j), lrow = row < last ? row : last;
+            if constexpr (WIDE_Q) {
+                const float *src = reinterpret_cast<const float *>(a.q.p) + ((size_t)bi * a.q.sb8 + (size_t)hi * a.q.sh8) * 8 +
+                                   (size_t)(qbase + lrow) * q_sn;
+                const f32x4 *x = reinterpret_cast<const f32x4 *>(src + (chunk_at(q2_chunk(j)) >> 1));
+                wide2[j][0] = x[0];
+                wide2[j][1] = x[1];
+            } else {
+                async_copy_b128(q2_dst + j * 1024, qsrc, __umul24(lrow, q_rb) + chunk_at(q2_chunk(j)));
+            }
         }
     }
     using std::integral_constant;
@@ -724,7 +818,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         return base_t + b;
     };
     const int t_first = next_tile();
-    const bool even_progress = NH == 1 && (int)blockIdx.x >= a.tail_start;   // three work-groups per CU
+    const bool even_progress = (NH == 1 || THIRD) && (int)blockIdx.x >= a.tail_start;   // three work-groups per CU
     if (t_first < T) {
         if constexpr (SPLIT) {          // V waits until q, which sits in its buffer, has been read
             issue_own_k(t_first);
@@ -739,18 +833,21 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     }
     if constexpr (WIDE_Q) {
         uint16_t *q16 = a.q16.p != nullptr && (SPLIT ? wave == 0 : half == 0) ? slab(a.q16, bi, hi) : nullptr;
+        auto land = [&](const f32x4 lo, const f32x4 hi4, uint32_t at, int row, int chunk) __attribute__((always_inline)) {
+            const u32x4 t = {E::pack2_rne(lo.x, lo.y), E::pack2_rne(lo.z, lo.w), E::pack2_rne(hi4.x, hi4.y), E::pack2_rne(hi4.z, hi4.w)};
+            *(LDS_PTR(u32x4))(uintptr_t)at = t;
+            if (q16 != nullptr && row_base + row < N && chunk <= last_chunk)
+                *reinterpret_cast<u32x4 *>(q16 + (size_t)(row_base + row) * a.q16.sn + 8 * chunk) = t;
+        };
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int row = 8 * j + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
 #pragma unroll
-            for (int half = 0; half < NH; ++half) {
-                const f32x4 lo = wide[NH * j + half][0], hi4 = wide[NH * j + half][1];
-                const u32x4 t = {E::pack2_rne(lo.x, lo.y), E::pack2_rne(lo.z, lo.w), E::pack2_rne(hi4.x, hi4.y), E::pack2_rne(hi4.z, hi4.w)};
-                *(LDS_PTR(u32x4))(uintptr_t)(q_dst + half * Q_HALF + j * 1024 + lane * 16) = t;
-                if (q16 != nullptr && row_base + row < N && 8 * half + c <= last_chunk)
-                    *reinterpret_cast<u32x4 *>(q16 + (size_t)(row_base + row) * a.q16.sn + 8 * (8 * half + c)) = t;
-            }
+            for (int half = 0; half < Q_PARTS; ++half)
+                land(wide[NH * j + half][0], wide[NH * j + half][1], q_dst + half * Q_HALF + j * 1024 + lane * 16, row, 8 * half + c);
         }
+#pragma unroll
+        for (int j = 0; j < Q2_PIECES; ++j) land(wide2[j][0], wide2[j][1], q2_dst + j * 1024 + lane * 16, q2_row(j), q2_chunk(j));
     }
     // small LDS table for the mask: entry n (16 B) holds four floats, float j = (bit j of n) ? 0 : -inf
     if (tid < 64)
@@ -784,7 +881,8 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     for (int x = 0; x < 2; ++x)
 #pragma unroll
         for (int c = 0; c < KS; ++c)
-            qf[x][c] = lds_read_b128((k_at ^ (64 * (c & 1))) + 2048 * x +
+            qf[x][c] = NARROW && c == 2 ? lds_read_b128(k2_at - TILE_BYTES + (NSTAGE - 1) * STAGE_BYTES + 16384 + wave * (32 * SECOND) + 16 * SECOND * x)
+                                        : lds_read_b128((k_at ^ (64 * (c & 1))) + 2048 * x +
                                      (SPLIT ? C::OFF_V + (c >> 1) * Q_HALF : (NSTAGE - 1) * STAGE_BYTES + (c >> 1) * Q_HALF + wave * 4096));
     // All requested before the first is converted.  Left alone, the compiler read, waited and converted one after the other, up to eight round trips
     // of LDS in a row: small calls back to back, that -> this, 2 heads, N = 128, D = 64 4.86 -> 4.78 us; D = 128: 224, N = 18 5.51 -> 5.38, 32, N = 64
@@ -808,6 +906,8 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     if constexpr (HALVES) {
         k_at += 4096 * half;
         v_at += 4096 * half;
+        k2_at += 32 * SECOND * half;
+        v2_at += 32 * SECOND * half;
     }
 
     // ---- running state: of the query rows 16x + l16 what the products and sums need, of the row l32 (in both lane halves) what is
@@ -852,6 +952,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
             after_scores();
             return;
         }
+        if constexpr (NARROW) asm volatile("" : "+v"(k2_at), "+v"(v2_at));
         asm volatile("" : "+v"(k_at), "+v"(v_at));       // or the compiler keeps a register for every address that follows from these
         // Steps of two products: S^T of 16 keys and 32 columns each, then O^T += V^T P^T of 16 columns and 32 keys.  The operands of a step are
         // requested AHEAD steps before it, and scheduling barriers hold that order: left alone, the compiler requests each just before
@@ -860,19 +961,21 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         u32x4 k_ring[AHEAD + 1], v_ring[V_AHEAD + 1];
         auto fetch_k = [&](int n) __attribute__((always_inline)) {
             const int blk = n / PH, kb = n & 1, c = n % PH >> 1;
-            if (n < SCORES) k_ring[n % (AHEAD + 1)] = lds_read_b128((k_at ^ (64 * (c & 1))) + so + (c >> 1) * TILE_BYTES + 4096 * blk + 2048 * kb);
+            if (NARROW && c == 2 && n < SCORES) k_ring[n % (AHEAD + 1)] = lds_read_b128(k2_at + so + SECOND * (32 * blk + 16 * kb));
+            else if (n < SCORES) k_ring[n % (AHEAD + 1)] = lds_read_b128((k_at ^ (64 * (c & 1))) + so + (c >> 1) * TILE_BYTES + 4096 * blk + 2048 * kb);
         };
         auto fetch_v = [&](int n) __attribute__((always_inline)) {
             if (n >= VALUES) return;
             const int blk = n / DB, b = n % DB;
-            const uint32_t at = (v_at ^ (32 * (b & 3))) + so + (b >> 2) * TILE_BYTES + 4096 * blk;
-            const u32x2 lo = lds_read_tr16_b64(at), hi = lds_read_tr16_b64(at + 2048);
+            const bool second = NARROW && b >= 4;
+            const uint32_t at = second ? (v2_at ^ (32 * (b & 3))) + so + 32 * SECOND * blk : (v_at ^ (32 * (b & 3))) + so + (b >> 2) * TILE_BYTES + 4096 * blk;
+            const u32x2 lo = lds_read_tr16_b64(at), hi = lds_read_tr16_b64(at + (second ? 16 * SECOND : 2048));
             v_ring[n % (V_AHEAD + 1)] = u32x4{lo.x, lo.y, hi.x, hi.y};
         };
 #pragma unroll
         for (int n = 0; n < AHEAD; ++n) fetch_k(n);
         __builtin_amdgcn_sched_barrier(0);
-        constexpr int EARLY_V = SPLIT || (BYPRODUCTS && HDIM == 64) ? 0 : HDIM <= 64 ? 2 : 4;       // of V before the exponentials, where there are registers
+        constexpr int EARLY_V = SPLIT || (BYPRODUCTS && HDIM == 64) || THIRD ? 0 : HDIM <= 64 ? 2 : 4;       // of V before the exponentials, where there are registers
         // ---- S^T: sacc[blk][kb][x][j] = log2 weight / pm of (key 32blk + 16kb + 4q4 + j, query 16x + l16) ----
         f32x4 sacc[KB][2][2];
 #pragma unroll
@@ -1248,7 +1351,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     {
         const int row0 = row_base;
         const uint32_t ebase = SPLIT ? lds0 : HALVES ? lds0 + 2 * HALF_SUMS + wave * 4096 : lds0 + (uint32_t)(visits & 1) * STAGE_BYTES + wave * 4096;
-        store_rows<BF16>(oacc, inv, ebase, SPLIT ? 4096 : HALVES ? 8192 : 16384, block_dst(out, out32, bi, hi, row0, D), out.p != nullptr,
+        store_rows<BF16>(oacc, inv, ebase, SPLIT ? 4096 : HALVES ? 8192 : NARROW ? 0 : 16384, block_dst(out, out32, bi, hi, row0, D), out.p != nullptr,
                              BF16 && out32.p != nullptr, row0, N, lane);       // fp32 callers compute in bf16
     }
     if (qrow < N) {
@@ -1379,15 +1482,15 @@ hipError_t launch_attn_fwd(const AttnArgs &args, bool bf16, hipStream_t stream)
         a.qtiles = (a.N + 63) / 64;
         groups = (long long)a.BH * a.qtiles;
     }
-    a.deal = make_deal(!split && !halves && !a.byte_mask && heads_alike(a.mask, a.H), a.BH, a.qtiles, (a.D <= HD ? 3 : 2) * cus, 4ll * a.N * a.D);
+    const int D = kernel_head_dim(a.D);
+    const bool byproducts = a.mask_out != nullptr || a.map_out != nullptr, three = D <= HD || three_on_a_cu(D, a.byte_mask != 0, byproducts, a.q_f32 != 0);
+    a.deal = make_deal(!split && !halves && !a.byte_mask && heads_alike(a.mask, a.H), a.BH, a.qtiles, (three ? 3 : 2) * cus, 4ll * a.N * a.D);
     a.tail_start = (!split && groups > 2 * cus && groups <= 3 * cus) ? 0 : (int)groups;
     a.groups = (int)groups;
     const dim3 grid((unsigned)groups), block(NTHREADS);
     const bool postmul = a.post_mul != 1.0f;
-    const int D = kernel_head_dim(a.D);
     const bool packed = a.D == D && (int)a.q.sn == D && (int)a.k.sn == D && (int)a.v.sn == D;
-    if (D > HD) a.tail_start = (int)groups;                   // two work-groups per CU: nobody yields
-    const bool byproducts = a.mask_out != nullptr || a.map_out != nullptr;
+    if (!three) a.tail_start = (int)groups;                   // two work-groups per CU: nobody yields
     // two tiles' mask bytes per request (see PAIRS at the kernel), unless the grid is the single round of work-groups in
     // step for which tail_start was set to 0 above
     const bool further = !split && a.byte_mask && D <= HD && (halves || a.tail_start != 0);
@@ -1397,7 +1500,11 @@ hipError_t launch_attn_fwd(const AttnArgs &args, bool bf16, hipStream_t stream)
     const int variant = (a.q_f32 ? 8 : 0) | (bf16 ? 4 : 0) | (postmul ? 2 : 0) | (packed ? 1 : 0);
     const FwdKernel kernel = D == 32 ? fwd_kernel_32(variant, mask_kind) : D == 64 ? fwd_kernel_64(variant, mask_kind)
                              : D == 80 ? fwd_kernel_80(variant, mask_kind) : D == 96 ? fwd_kernel_96(variant, mask_kind) : fwd_kernel_128(variant, mask_kind);
-    hipLaunchKernelGGL(kernel, grid, block, 0, stream, a);
+    // Three on a CU lose where the work is all bytes, two tiles a work-group and a head to each, over several rounds: 12 KiB more of LDS keep it at two.  D = 80, 2048 heads,
+    // packed, two -> three on a CU: N = 112 38.3 -> 39.2 us, 128 42.4 -> 44.5 (boolean 47.3 -> 51.0), D = 96 42.9 -> 44.1;  512 heads 10.1 either way;  one tile, N = 64,
+    // 19.3 -> 17.2, three, N = 136, 62.8 -> 55.3.
+    const bool two = three && D > HD && !halves && !split && a.N > BN && a.N <= BM && groups > 3 * cus;
+    hipLaunchKernelGGL(kernel, grid, block, two ? 12288 : 0, stream, a);
     return hipGetLastError();
 }
 #endif

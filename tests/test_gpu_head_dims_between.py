@@ -86,3 +86,35 @@ def test_kernels_for_80(dev, heads, N, blocks, D, dtype):
         wanted = [ref.detach(), *torch.autograd.grad(ref, one, do[:, h:h + 1].double())]
         for got, want in zip(made, wanted):                  # the bound of the test above
             assert ((got[:, h:h + 1].double() - want).abs() <= 1e-4 + 2e-2 * want.abs().max() + 2e-2 * want.abs()).all()
+
+
+# The forward's tiles whose second column half has short rows (65 to 80: 32 bytes, in training 64; 81 to 96: 64, fp32 whole ones): one tile and two, keys that end in either half
+# and in the first or last of the rows that one request fills, work-groups of 64 rows (from 1024 rows on), two on a CU by the launcher's choice (800 heads).  With a whole head dim
+# (80, 96) and rows that end before it.
+@pytest.mark.parametrize("D", [72, 80, 88, 96])
+@pytest.mark.parametrize("heads, N", [(3, 33), (800, 65), (800, 128), (110, 127), (110, 129), (60, 656), (60, 673), (90, 720), (20, 1025), (12, 1104)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_short_rows_of_the_second_half(dev, heads, N, D, dtype):
+    importlib.import_module("python.sparse_attention")
+    sa = sys.modules["python.sparse_attention"]
+    g = torch.Generator(device=dev).manual_seed(N + D)
+    q, k, v = (torch.randn(1, heads, N, D, device=dev, generator=g).to(dtype) for _ in range(3))
+    mask = torch.rand(1, 1, N, N, device=dev, generator=g) < 0.3
+    mask[..., 3, :] = False
+    mask[..., 4, :] = torch.arange(N, device=dev) == N - 1
+    packed = sa.pack_mask(mask)
+    out = sa.sparse_attention_func(q, k, v, mask)
+    odd = (mask.to(torch.uint8) * 6).view(torch.bool)                  # bytes that are neither 0 nor 1
+    leaves = [t.detach().requires_grad_(True) for t in (q, k, v)]
+    strided = [torch.nn.functional.pad(t, (0, 8), value=float("nan"))[..., :D] for t in (q, k, v)]
+    for x in (sa.sparse_attention_func(q, k, v, odd), sa.sparse_attention_func(q, k, v, None, mask_packed=packed), sa.sparse_attention_func(*strided, mask),
+              sa.sparse_attention_func(q, k, v, None, mask_packed=packed, tile_map=sa.tile_map(packed, min_skip=0.0)), sa.sparse_attention(*leaves, mask)):
+        assert torch.equal(out, x)
+    # the bound of the work-groups of 64 rows: the probabilities and the result are rounded once each, relative to the largest value of a row's mean
+    eps = 2.0 ** (-10 if dtype == torch.float16 else -7)
+    for h in (0, heads - 1):
+        one = [t[:, h:h + 1].double() if dtype != torch.float32 else t[:, h:h + 1].bfloat16().double() for t in (q, k, v)]
+        x = ((one[0] * D ** -0.5) @ one[1].transpose(-1, -2)).masked_fill(~mask, float("-inf"))
+        ref = torch.softmax(x, -1).nan_to_num() @ one[2]
+        shift = (eps * (one[0].abs() * D ** -0.5) @ one[1].abs().transpose(-1, -2)).masked_fill(~mask, 0).amax(-1)
+        assert ((out[:, h:h + 1].double() - ref).abs() <= 1e-4 + one[2].abs().max() * (4 * eps + 2 * shift[..., None])).all()
