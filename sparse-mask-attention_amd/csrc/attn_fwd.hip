@@ -53,7 +53,7 @@
 //                 skips its GEMMs and its softmax for that tile.
 //   head dim    = the description above is for 64.  128 runs the same code on two column halves of
 //                 64 (see Cfg below): twice the MFMAs per tile for the same softmax work, a ring of
-//                 two stages and two work-groups per CU.  32 uses half of every tile row.
+//                 two stages and two work-groups per CU.  32, 80 and 96 keep short rows (second_row).
 #include <atomic>
 #include <type_traits>
 
@@ -76,8 +76,8 @@ constexpr float SUM_LIMIT = 16384.0f;     // a lane's 32 weights of a tile sum t
 //        QK^T chain runs over both halves of K and q, and P multiplies each half of V into its own
 //        pair of accumulators.  A stage is twice as large (32 KiB) and the kernel needs about 224
 //        registers, so two work-groups share a CU.
-//   32   half a tile: the copies fill the upper half of every LDS row with copies of the row's last
-//        16 bytes, which are never read; the QK^T chain has one step instead of two and P multiplies
+//   32   half a tile: rows of 64 bytes (with SPLIT of 128, of which the copies fill the upper half with the row's last
+//        16 bytes, which are never read); the QK^T chain has one step instead of two and P multiplies
 //        two 16-column blocks of V.
 //   96   128 with such a half tile as its second half: three steps, six blocks.  D = 80 and 96 ran in the
 //        128 kernel before, through zero-padded copies (16 x 8 heads, N = 1088, D = 96: 156 -> 81 us)
@@ -88,22 +88,27 @@ constexpr float SUM_LIMIT = 16384.0f;     // a lane's 32 weights of a tile sum t
 // into the two words per row itself (eight dot products with the weights 1, 2, 4 .. 128 per lane
 // and one exchange between the lane halves): the separate packing pass, its launch and the
 // round trip of the words through memory disappear for a mask that is used once.
-// SECOND: bytes of a row in the second column half's tile (head dims beyond 64).  At head dims 80 and 96, but with SPLIT, the rows there are only as long as
+// SECOND: bytes of a row in the second column half's tile (head dims beyond 64; at 32, but with SPLIT, all of the row: there is no first half).  At head dims 80 and 96, but with SPLIT, the rows there are only as long as
 // what is used of them: 32 and 64 bytes, of which one request fills 32 or 16 rows.  A wavefront requests five or six pieces of K and V a tile instead of eight, and a stage is 20
 // or 24 KiB instead of 32, which is what lets three work-groups share a CU (see three_on_a_cu).  Whole rows -> this with two on a CU all the same: D = 80, 512 heads, N = 320 33.7 ->
 // 32.4 us, N = 512 67.1 -> 65.4; D = 96 36.4 -> 35.9, 69.9 -> 68.5.  64 bytes where by-products are asked for at 80 (two on a CU: 32, whose reads of K's last step
 // meet in a bank, cost 64 heads, N = 1500 in training 281 -> 285 us, 64 282), and whole rows for fp32 queries at 96 (64, N = 1500 104.0 -> 109.5).
+// Head dim 32, two requests a tile instead of four, stages of 8 KiB instead of 16, with which the boolean mask's bytes leave room for four work-groups on a CU instead of three, whole rows -> this:
+// boolean 2048 heads, N = 32 11.6 -> 9.8 us, N = 100 16.1 -> 14.5, N = 200 45.7 -> 42.3;  256, N = 1000 78.3 -> 73.4;  192, N = 1024 55.2 -> 52.6;  packed 2048, N = 200 33.2 -> 31.5, 128, N = 2048 96.4 -> 93.8,
+// causal 60.5 -> 60.3;  where two tiles a head of whole rows are all there is 3 % slower, at 4.4 TB/s (2048, N = 128, packed 14.8 -> 15.2; boolean 18.2 -> 17.9; N = 112 13.3 -> 13.0).
 constexpr int second_row(int hdim, bool split, bool byproducts, bool wide_q)
 {
-    return hdim <= 64 ? 0 : split || hdim == 128 || (hdim == 96 && wide_q) ? 128 : hdim == 96 || byproducts ? 64 : 32;
+    return hdim == 32 ? (split ? 0 : 64) : hdim <= 64 ? 0 : split || hdim == 128 || (hdim == 96 && wide_q) ? 128 : hdim == 96 || byproducts ? 64 : 32;
 }
 template <int NH, bool BYTEMASK, bool SPLIT, int SECOND> struct Cfg {
     // SPLIT: one K and one V buffer for each of the four wavefronts, else a ring of two stages: copies run one tile ahead
     static constexpr int NSTAGE = SPLIT ? 4 : 2;
     static constexpr int MASK_COPIES = BYTEMASK ? 2 : 1;
-    static constexpr int COPIES = MASK_COPIES + 4 + (SECOND == 32 ? 1 : SECOND / 32);    // async copies per wave and tile
+    static constexpr int FIRST = NH == 1 && SECOND != 0 ? 0 : TILE_BYTES;                // the first half's tile: none at head dim 32, all of whose row is short
+    static constexpr int KV_COPIES = (FIRST != 0 ? 4 : 0) + (SECOND == 32 ? 1 : SECOND / 32);
+    static constexpr int COPIES = MASK_COPIES + KV_COPIES;          // async copies per wave and tile
     // LDS map (bytes), after the 256 of the table of the mask bias, which lies first: a read's immediate offset reaches 64 KiB
-    static constexpr int OFF_V = TILE_BYTES + BN * SECOND;          // V inside a stage
+    static constexpr int OFF_V = FIRST + BN * SECOND;               // V inside a stage
     static constexpr int STAGE_BYTES = 2 * OFF_V;                   // K halves, then V halves
     // mask: packed words in NSTAGE slots of 4 waves x 64 words; bytes in slots of 4 waves x 2 KiB,
     // two of them for head dims up to 64 and, for want of LDS, ONE for 128: a wave has turned its
@@ -120,7 +125,8 @@ template <int NH, bool BYTEMASK, bool SPLIT, int SECOND> struct Cfg {
     static constexpr int OFF_MAP = OFF_MASK + (BYTEMASK ? BYTE_SLOTS * 8192 : SPLIT ? 1024 : NSTAGE * 1024);
     static constexpr int OFF_MAP_ARRIVED = OFF_MAP + 4 * MAP_WORDS * 8;
     static constexpr int LUT_BYTES = 256;                           // 16 x 16 B
-    static constexpr int LDS_BYTES = LUT_BYTES + (BYTEMASK && !SPLIT ? OFF_MAP_ARRIVED + 16 : OFF_MAP);
+    // head dim 32, packed words: the rows leave through 4 KiB a wavefront of their own (a stage is smaller than that)
+    static constexpr int LDS_BYTES = LUT_BYTES + (BYTEMASK && !SPLIT ? OFF_MAP_ARRIVED + 16 : OFF_MAP + (FIRST == 0 ? 16384 : 0));
 };
 
 // Head dims beyond 64 of which three work-groups share a CU (but with SPLIT): where 168 registers hold the loop, with operands requested no further ahead
@@ -204,6 +210,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     constexpr int SECOND = second_row(HDIM, SPLIT, BYPRODUCTS, WIDE_Q);
     constexpr bool NARROW = SECOND == 32 || SECOND == 64;
     using C = Cfg<NH, BYTEMASK, SPLIT, SECOND>;
+    constexpr int FIRST = C::FIRST, SHORT_CHUNK = FIRST != 0 ? 8 : 0;        // (NARROW: where the short rows begin in LDS, and their first 16-byte chunk)
     constexpr int NSTAGE = C::NSTAGE, STAGE_BYTES = C::STAGE_BYTES, OFF_MASK = C::OFF_MASK;
     constexpr int MASK_SLOT = C::MASK_SLOT, COPIES = C::COPIES - (HALF_BYTES ? 1 : 0);
     const int D = PACKED_ROWS ? HDIM : a.D;
@@ -584,11 +591,11 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     const uint32_t rb2 = takes_v2 ? v_rb : k_rb;
     if constexpr (NARROW) {
         const int row2 = row2_of(lane);
-        const uint32_t c = chunk_at(8 + (SECOND == 32 ? lane & 1 : (lane & 3) ^ narrow_swizzle(row2)));
+        const uint32_t c = chunk_at(SHORT_CHUNK + (SECOND == 32 ? lane & 1 : (lane & 3) ^ narrow_swizzle(row2)));
         kv_voff2[0][0] = __umul24(row2, rb2) + c;
         kv_voff2[1][0] = __umul24(row2, v_rb) + c;
     }
-    const uint32_t kv_dst2 = lds0 + TILE_BYTES + (SECOND == 32 ? (takes_v2 ? C::OFF_V : 0) + (wave & 1) * 1024 : wave * 1024);
+    const uint32_t kv_dst2 = lds0 + FIRST + (SECOND == 32 ? (takes_v2 ? C::OFF_V : 0) + (wave & 1) * 1024 : wave * 1024);
     const uint32_t kv_dst = lds0 + wave * 2048;
     auto issue_kv = [&](int t, auto stage_c) __attribute__((always_inline)) {
         constexpr int SO = decltype(stage_c)::value * STAGE_BYTES;
@@ -617,13 +624,13 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
                 }
             }
         }
-        async_copy2_b128_at<SO, SO + 1024>(kv_dst, ksrc, kv_voff[0][0], kv_voff[0][1]);
+        if constexpr (FIRST != 0) async_copy2_b128_at<SO, SO + 1024>(kv_dst, ksrc, kv_voff[0][0], kv_voff[0][1]);
         if constexpr (SAME_HALVES) {          // 128 bytes further along each row
             async_copy2_b128_at<SO + TILE_BYTES, SO + TILE_BYTES + 1024>(kv_dst, ksrc + HD, kv_voff[0][0], kv_voff[0][1]);
         } else if constexpr (NH == 2 && !NARROW) {
             async_copy2_b128_at<SO + TILE_BYTES, SO + TILE_BYTES + 1024>(kv_dst, ksrc, kv_voff2[0][0], kv_voff2[0][1]);
         }
-        async_copy2_b128_at<SO + C::OFF_V, SO + C::OFF_V + 1024>(kv_dst, vsrc, kv_voff[1][0], kv_voff[1][1]);
+        if constexpr (FIRST != 0) async_copy2_b128_at<SO + C::OFF_V, SO + C::OFF_V + 1024>(kv_dst, vsrc, kv_voff[1][0], kv_voff[1][1]);
         if constexpr (SAME_HALVES) {
             async_copy2_b128_at<SO + C::OFF_V + TILE_BYTES, SO + C::OFF_V + TILE_BYTES + 1024>(kv_dst, vsrc + HD, kv_voff[1][0], kv_voff[1][1]);
         } else if constexpr (SECOND == 64) {
@@ -686,7 +693,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const int row = 8 * (2 * wave + j) + (l >> 3);
-            if (key0 + row >= N) {
+            if (FIRST != 0 && key0 + row >= N) {
                 const uint32_t p = lds0 + stage * STAGE_BYTES + wave * 2048 + j * 1024 + l * 16;
                 const u32x4 z = {0u, 0u, 0u, 0u};
 #pragma unroll
@@ -718,8 +725,8 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         if constexpr (NARROW) {
             // (80: what the lanes of the last two chunks read meets zeros of q, as where rows are whole; it is the row's last chunk there too)
             const int chunk = SECOND == 32 ? (q4 < 1 ? q4 : 1) : q4 ^ narrow_swizzle(l16);
-            k2_at = own0 + TILE_BYTES + l16 * SECOND + (chunk << 4);
-            v2_at = own0 + C::OFF_V + TILE_BYTES + r * SECOND + ((((l16 & 3) >> 1) ^ (SECOND == 32 ? 0 : narrow_swizzle(r))) << 4) + ((l16 & 1) << 3);
+            k2_at = own0 + FIRST + l16 * SECOND + (chunk << 4);
+            v2_at = own0 + C::OFF_V + FIRST + r * SECOND + ((((l16 & 3) >> 1) ^ (SECOND == 32 ? 0 : narrow_swizzle(r))) << 4) + ((l16 & 1) << 3);
         }
     }
     const uint32_t nib_rotate = (4u * q4 + 28u) & 31u;     // right: the nibble of keys 4q4 .. 4q4 + 3 comes to bits 4 .. 7
@@ -739,12 +746,12 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     const uint32_t q_dst = SPLIT ? split_dst + C::OFF_V : lds0 + (NSTAGE - 1) * STAGE_BYTES + wave * 4096;
     // NARROW: the second half of q behind the four wavefronts' first halves, SECOND bytes a row, in as many pieces
     constexpr int Q2_PIECES = NARROW ? SECOND / 32 : 0;
-    const uint32_t q2_dst = lds0 + (NSTAGE - 1) * STAGE_BYTES + 16384 + wave * (32 * SECOND);
+    const uint32_t q2_dst = lds0 + (NSTAGE - 1) * STAGE_BYTES + 2 * FIRST + wave * (32 * SECOND);
     auto q2_row = [&](int j) __attribute__((always_inline)) { return SECOND == 32 ? lane >> 1 : 16 * j + (lane >> 2); };
-    auto q2_chunk = [&](int j) __attribute__((always_inline)) { return 8 + (SECOND == 32 ? lane & 1 : (lane & 3) ^ narrow_swizzle(q2_row(j))); };
+    auto q2_chunk = [&](int j) __attribute__((always_inline)) { return SHORT_CHUNK + (SECOND == 32 ? lane & 1 : (lane & 3) ^ narrow_swizzle(q2_row(j))); };
     f32x4 wide[WIDE_Q ? 4 * NH : 1][2], wide2[WIDE_Q && NARROW ? Q2_PIECES : 1][2];
-    constexpr int Q_PARTS = NARROW ? 1 : NH;             // column halves in whole rows
-    static_assert(!NARROW || 16384 + 128 * SECOND <= STAGE_BYTES, "q fits a stage");
+    constexpr int Q_PARTS = FIRST == 0 ? 0 : NARROW ? 1 : NH;             // column halves in whole rows
+    static_assert(!NARROW || 2 * FIRST + 128 * SECOND <= STAGE_BYTES, "q fits a stage");
     {
         const int qbase = row_base < N ? row_base : N - 1;   // wave-uniform
         const uint16_t *qsrc = qb + (size_t)qbase * q_sn;
@@ -767,7 +774,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
                 }
                 continue;
             }
-            async_copy_b128(dst + j * 1024, qsrc, __umul24(lrow, q_rb) + chunk_at(c));
+            if constexpr (FIRST != 0) async_copy_b128(dst + j * 1024, qsrc, __umul24(lrow, q_rb) + chunk_at(c));
             if constexpr (NH == 2 && !NARROW) async_copy_b128(dst + Q_HALF + j * 1024, qsrc, __umul24(lrow, q_rb) + chunk_at(8 + c));
         }
 #pragma unroll
@@ -858,7 +865,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         yield_at = n_visits / 4;
     }
     if (SPLIT) { if (t_first < T) wait_vmcnt<8 * NH + C::MASK_COPIES>(); else wait_vmcnt<0>(); }
-    else if (PAIRS) wait_vmcnt<HALVES ? 6 : 8>();      // q has landed; 4 (2) mask and 4 K/V copies may still be in flight
+    else if (PAIRS) wait_vmcnt<C::KV_COPIES + (HALVES ? 2 : 4)>();      // q has landed; 4 (2) mask and the K/V copies may still be in flight
     else if (t_first < T) wait_vmcnt<COPIES>();        // q has landed; the copies of the first tile may still be in flight
     else wait_vmcnt<0>();
     // What only the end needs of the arguments, while q is on its way from LDS.  Requested with the others at the start (as the compiler has it) ->
@@ -881,7 +888,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     for (int x = 0; x < 2; ++x)
 #pragma unroll
         for (int c = 0; c < KS; ++c)
-            qf[x][c] = NARROW && c == 2 ? lds_read_b128(k2_at - TILE_BYTES + (NSTAGE - 1) * STAGE_BYTES + 16384 + wave * (32 * SECOND) + 16 * SECOND * x)
+            qf[x][c] = NARROW && 4 * c == SHORT_CHUNK ? lds_read_b128(k2_at + FIRST + (NSTAGE - 1) * STAGE_BYTES + wave * (32 * SECOND) + 16 * SECOND * x)
                                         : lds_read_b128((k_at ^ (64 * (c & 1))) + 2048 * x +
                                      (SPLIT ? C::OFF_V + (c >> 1) * Q_HALF : (NSTAGE - 1) * STAGE_BYTES + (c >> 1) * Q_HALF + wave * 4096));
     // All requested before the first is converted.  Left alone, the compiler read, waited and converted one after the other, up to eight round trips
@@ -961,13 +968,13 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         u32x4 k_ring[AHEAD + 1], v_ring[V_AHEAD + 1];
         auto fetch_k = [&](int n) __attribute__((always_inline)) {
             const int blk = n / PH, kb = n & 1, c = n % PH >> 1;
-            if (NARROW && c == 2 && n < SCORES) k_ring[n % (AHEAD + 1)] = lds_read_b128(k2_at + so + SECOND * (32 * blk + 16 * kb));
+            if (NARROW && 4 * c == SHORT_CHUNK && n < SCORES) k_ring[n % (AHEAD + 1)] = lds_read_b128(k2_at + so + SECOND * (32 * blk + 16 * kb));
             else if (n < SCORES) k_ring[n % (AHEAD + 1)] = lds_read_b128((k_at ^ (64 * (c & 1))) + so + (c >> 1) * TILE_BYTES + 4096 * blk + 2048 * kb);
         };
         auto fetch_v = [&](int n) __attribute__((always_inline)) {
             if (n >= VALUES) return;
             const int blk = n / DB, b = n % DB;
-            const bool second = NARROW && b >= 4;
+            const bool second = NARROW && 2 * b >= SHORT_CHUNK;
             const uint32_t at = second ? (v2_at ^ (32 * (b & 3))) + so + 32 * SECOND * blk : (v_at ^ (32 * (b & 3))) + so + (b >> 2) * TILE_BYTES + 4096 * blk;
             const u32x2 lo = lds_read_tr16_b64(at), hi = lds_read_tr16_b64(at + (second ? 16 * SECOND : 2048));
             v_ring[n % (V_AHEAD + 1)] = u32x4{lo.x, lo.y, hi.x, hi.y};
@@ -1192,9 +1199,9 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         // Copies in flight, oldest first, at the top of an even visit t: the bytes of the pair
         // (t, t + 1), then K/V of t; after its barrier K/V of t + 1 and then the bytes of the next
         // pair are requested, and the odd visit requests K/V of t + 2 after its barrier: the bytes of
-        // a pair are always followed by exactly four younger copies when they are needed.  (The stores
+        // a pair are always followed by exactly one tile's younger copies (KV_COPIES) when they are needed.  (The stores
         // of the by-products, when asked for, only add to the count: copies complete in the order of
-        // their requests, so "at most four outstanding" still means that all older copies are in.)
+        // their requests, so "at most so many outstanding" still means that all older copies are in.)
         // HALVES: a wavefront reads bytes that another has copied, behind the even visit's barrier; the next pair's are requested then
         // into the other slot, whose bytes were read before the odd visit's barrier.
         for (int t = 0; t < T; t += 2) {
@@ -1206,7 +1213,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
                 if (WHOLE || t + 1 < T) w_odd = mask_words(t + 1, slot, 1);
             };
             if constexpr (!HALVES) {
-                wait_vmcnt<4>();                              // this wave's bytes of the pair have landed
+                wait_vmcnt<C::KV_COPIES>();                   // this wave's bytes of the pair have landed
                 words();
             }
             wait_vmcnt<0>();                                  // K/V of tile t
@@ -1350,7 +1357,10 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
     const float inv[2] = {__builtin_bit_cast(float, inv_of.w[0]), __builtin_bit_cast(float, inv_of.w[1])};
     {
         const int row0 = row_base;
-        const uint32_t ebase = SPLIT ? lds0 : HALVES ? lds0 + 2 * HALF_SUMS + wave * 4096 : lds0 + (uint32_t)(visits & 1) * STAGE_BYTES + wave * 4096;
+        // Head dim 32, whose stages are smaller: through an area of the wavefront's own, with pairs of tiles' bytes that of the bytes; with one tile's
+        // through both stages, behind a barrier.
+        if constexpr (FIRST == 0 && BYTEMASK && !PAIRS && !HALVES) __syncthreads();
+        const uint32_t ebase = FIRST == 0 && !HALVES ? lds0 + (PAIRS ? OFF_MASK : BYTEMASK ? 0 : C::OFF_MAP) + wave * 4096 : SPLIT ? lds0 : HALVES ? lds0 + 2 * HALF_SUMS + wave * 4096 : lds0 + (uint32_t)(visits & 1) * STAGE_BYTES + wave * 4096;
         store_rows<BF16>(oacc, inv, ebase, SPLIT ? 4096 : HALVES ? 8192 : NARROW ? 0 : 16384, block_dst(out, out32, bi, hi, row0, D), out.p != nullptr,
                              BF16 && out32.p != nullptr, row0, N, lane);       // fp32 callers compute in bf16
     }

@@ -88,10 +88,10 @@ def test_kernels_for_80(dev, heads, N, blocks, D, dtype):
             assert ((got[:, h:h + 1].double() - want).abs() <= 1e-4 + 2e-2 * want.abs().max() + 2e-2 * want.abs()).all()
 
 
-# The forward's tiles whose second column half has short rows (65 to 80: 32 bytes, in training 64; 81 to 96: 64, fp32 whole ones): one tile and two, keys that end in either half
+# The forward's tiles that have short rows (head dims to 32: 64 bytes;  in the second column half 65 to 80: 32 bytes, in training 64; 81 to 96: 64, fp32 whole ones): one tile and two, keys that end in either half
 # and in the first or last of the rows that one request fills, work-groups of 64 rows (from 1024 rows on), two on a CU by the launcher's choice (800 heads).  With a whole head dim
 # (80, 96) and rows that end before it.
-@pytest.mark.parametrize("D", [72, 80, 88, 96])
+@pytest.mark.parametrize("D", [24, 32, 72, 80, 88, 96])
 @pytest.mark.parametrize("heads, N", [(3, 33), (800, 65), (800, 128), (110, 127), (110, 129), (60, 656), (60, 673), (90, 720), (20, 1025), (12, 1104)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 def test_short_rows_of_the_second_half(dev, heads, N, D, dtype):
