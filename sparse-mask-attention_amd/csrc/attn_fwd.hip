@@ -624,9 +624,15 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
                 }
             }
         }
+        // The two pieces of a row follow each other: its end and the next row's begin share lines, which two tiles a work-group are too short-lived to
+        // find in the cache again.  K and V first, then their ends (and q likewise) -> this, us, at head dim 96, where rows all whole were the faster on
+        // two tiles: inputs from memory, packed, 1024 heads, N = 104 20.9 -> 20.2 (whole 20.2), 384, N = 112 9.10 -> 8.88 (8.85);  boolean 384, N = 96
+        // 9.44 -> 9.09 (9.16), 2048, N = 127 48.3 -> 48.1 (47.9), 256, N = 512 43.1 -> 42.4 (43.9).
         if constexpr (FIRST != 0) async_copy2_b128_at<SO, SO + 1024>(kv_dst, ksrc, kv_voff[0][0], kv_voff[0][1]);
         if constexpr (SAME_HALVES) {          // 128 bytes further along each row
             async_copy2_b128_at<SO + TILE_BYTES, SO + TILE_BYTES + 1024>(kv_dst, ksrc + HD, kv_voff[0][0], kv_voff[0][1]);
+        } else if constexpr (SECOND == 64) {
+            async_copy_b128_at<SO>(kv_dst2, ksrc, kv_voff2[0][0]);
         } else if constexpr (NH == 2 && !NARROW) {
             async_copy2_b128_at<SO + TILE_BYTES, SO + TILE_BYTES + 1024>(kv_dst, ksrc, kv_voff2[0][0], kv_voff2[0][1]);
         }
@@ -634,7 +640,6 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         if constexpr (SAME_HALVES) {
             async_copy2_b128_at<SO + C::OFF_V + TILE_BYTES, SO + C::OFF_V + TILE_BYTES + 1024>(kv_dst, vsrc + HD, kv_voff[1][0], kv_voff[1][1]);
         } else if constexpr (SECOND == 64) {
-            async_copy_b128_at<SO>(kv_dst2, ksrc, kv_voff2[0][0]);
             async_copy_b128_at<SO + C::OFF_V>(kv_dst2, vsrc, kv_voff2[1][0]);
         } else if constexpr (SECOND == 32) {
             async_copy_b128_at<SO>(kv_dst2, takes_v2 ? vsrc : ksrc, kv_voff2[0][0]);
@@ -776,18 +781,22 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
             }
             if constexpr (FIRST != 0) async_copy_b128(dst + j * 1024, qsrc, __umul24(lrow, q_rb) + chunk_at(c));
             if constexpr (NH == 2 && !NARROW) async_copy_b128(dst + Q_HALF + j * 1024, qsrc, __umul24(lrow, q_rb) + chunk_at(8 + c));
+            if constexpr (NARROW) {           // the rows' ends behind the last of their first pieces, as in issue_kv
+                constexpr int EVERY = 4 / Q2_PIECES;
+                const int i = j / EVERY, end_row = q2_row(i);
+                if (j % EVERY == EVERY - 1)
+                    async_copy_b128(q2_dst + i * 1024, qsrc, __umul24(end_row < last ? end_row : last, q_rb) + chunk_at(q2_chunk(i)));
+            }
         }
+        if constexpr (WIDE_Q && NARROW) {
 #pragma unroll
-        for (int j = 0; j < Q2_PIECES; ++j) {
-            const int row = q2_row(j), lrow = row < last ? row : last;
-            if constexpr (WIDE_Q) {
+            for (int j = 0; j < Q2_PIECES; ++j) {
+                const int row = q2_row(j), lrow = row < last ? row : last;
                 const float *src = reinterpret_cast<const float *>(a.q.p) + ((size_t)bi * a.q.sb8 + (size_t)hi * a.q.sh8) * 8 +
                                    (size_t)(qbase + lrow) * q_sn;
                 const f32x4 *x = reinterpret_cast<const f32x4 *>(src + (chunk_at(q2_chunk(j)) >> 1));
                 wide2[j][0] = x[0];
                 wide2[j][1] = x[1];
-            } else {
-                async_copy_b128(q2_dst + j * 1024, qsrc, __umul24(lrow, q_rb) + chunk_at(q2_chunk(j)));
             }
         }
     }
