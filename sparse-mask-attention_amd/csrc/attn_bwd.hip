@@ -377,12 +377,13 @@ __global__ __launch_bounds__(NTHREADS, HDIM > 64 ? 2 : 3) void attn_bwd_dq_kerne
 //        launcher): 16 x 12 heads, N = 512, this kernel alone on warm inputs: 41.0 -> 37.3 us (691 TFLOP/s)
 template <int HDIM, int NW, bool VLDS> struct DkvCfg {
     static constexpr int NH = HDIM > 64 ? 2 : 1;
+    static constexpr int KS = (HDIM + 31) / 32;             // MFMA steps of a contraction over the head dim
     static constexpr int STAGE_BYTES = 2 * NH * TILE_BYTES;
     static constexpr int OFF_B = NH * TILE_BYTES;           // dO inside a stage
     static constexpr int AUX = NW * 256 + 512;              // per wavefront its mask words of 64 rows, then lse, delta
     static constexpr int OFF_AUX = NSTAGE * STAGE_BYTES;
     static constexpr int OFF_FRAG = OFF_AUX + NSTAGE * AUX; // V fragments of each wavefront
-    static constexpr int FRAG = VLDS ? HDIM / 16 * 1024 : 0;
+    static constexpr int FRAG = VLDS ? 2 * KS * 1024 : 0;   // of two blocks of 16 keys
     static constexpr int LDS_BYTES = OFF_FRAG + NW * FRAG;
 };
 template <bool BF16, int HDIM, int NW, bool VLDS, bool POSTMUL, bool WIDE, bool HALVES = false>
@@ -390,10 +391,10 @@ __device__ __forceinline__ void dkv_keys(const AttnBwdArgs &a, unsigned char *sm
 {
     using E = Elem<BF16>;
     constexpr int NH = HDIM > 64 ? 2 : 1;
-    constexpr int KS = (HDIM + 31) / 32;
+    using C = DkvCfg<HDIM, NW, VLDS>;
+    constexpr int KS = C::KS;
     constexpr int DB = HDIM / 16;
     constexpr int AHEAD = VLDS || HDIM == 32 ? 2 : 3;             // one more where there are registers for it
-    using C = DkvCfg<HDIM, NW, VLDS>;
     constexpr int STAGE_BYTES = C::STAGE_BYTES, OFF_AUX = C::OFF_AUX, AUX_BYTES = C::AUX;
     constexpr int OFF_LSE = NW * 256, OFF_DELTA = OFF_LSE + 256;       // inside the small data of a stage
     const uint32_t lds0 = (uint32_t)(uintptr_t)(LDS_PTR(unsigned char))smem;

@@ -134,3 +134,17 @@ def test_forward_requests_the_pieces_of_a_row_together(tmp_path):
             tiles = [rest[i:i + 6] for i in range(0, len(rest), copies)]
         assert tiles and len(set(q)) == 1, name
         assert all(t[0] == t[1] == t[2] and t[3] == t[4] == t[5] for t in tiles), (name, tiles)
+
+
+def test_lds_of_the_value_fragments(tmp_path):
+    """dK/dV with V's fragments in LDS: a wavefront's area holds what it writes there, two fragments of 1 KiB for each step of 32 columns, at every head dim."""
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("no hipcc")
+    source = tmp_path / "frag.hip"
+    source.write_text('#include "attn_bwd.hip"\n'
+                      "template <int HDIM> constexpr bool holds() { return sma::DkvCfg<HDIM, 4, true>::FRAG >= 2 * ((HDIM + 31) / 32) * 1024; }\n"
+                      'static_assert(holds<32>() && holds<64>() && holds<80>() && holds<96>() && holds<128>(), "V fragments");\n')
+    csrc = os.path.join(os.path.dirname(_capi.LIB), "csrc")
+    include = os.path.join(os.path.dirname(os.path.dirname(_capi.LIB)), "include")
+    subprocess.run([hipcc, "--offload-host-only", "-fsyntax-only", "-std=c++17", "-I" + include, "-I" + csrc, str(source)], check=True)
