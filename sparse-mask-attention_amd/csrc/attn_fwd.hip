@@ -834,7 +834,7 @@ __global__ __launch_bounds__(NTHREADS, SPLIT ? (HDIM > 64 ? 1 : 2) : HDIM > 64 ?
         return base_t + b;
     };
     const int t_first = next_tile();
-    const bool even_progress = (NH == 1 || THIRD) && (int)blockIdx.x >= a.tail_start;   // three work-groups per CU
+    const bool even_progress = (NH == 1 || THIRD) && (int)blockIdx.x >= a.tail_start;   // three work-groups per CU, or four
     if (t_first < T) {
         if constexpr (SPLIT) {          // V waits until q, which sits in its buffer, has been read
             issue_own_k(t_first);
@@ -1468,7 +1468,7 @@ hipError_t launch_attn_fwd(const AttnArgs &args, bool bf16, hipStream_t stream)
     a.div_H = make_fastdiv((uint32_t)a.H);
     long long groups = (long long)a.BH * a.qtiles;
     if (groups == 0) return hipSuccess;
-    // Only a grid that is resident all at once with three work-groups on (almost) every CU evens out
+    // Only a grid that is resident all at once with three work-groups (or four) on (almost) every CU evens out
     // its progress; with several rounds oldest-first is what frees slots for the waiting ones, and
     // applying it to the last round only measured neutral.
     const long long cus = compute_units();
@@ -1504,15 +1504,21 @@ hipError_t launch_attn_fwd(const AttnArgs &args, bool bf16, hipStream_t stream)
     const int D = kernel_head_dim(a.D);
     const bool byproducts = a.mask_out != nullptr || a.map_out != nullptr, three = D <= HD || three_on_a_cu(D, a.byte_mask != 0, byproducts, a.q_f32 != 0);
     a.deal = make_deal(!split && !halves && !a.byte_mask && heads_alike(a.mask, a.H), a.BH, a.qtiles, (three ? 3 : 2) * cus, 4ll * a.N * a.D);
-    a.tail_start = (!split && groups > 2 * cus && groups <= 3 * cus) ? 0 : (int)groups;
+    // Four share a CU at head dim 32, but with by-products (132 to 137 registers): one round of those evens out its progress too.  Oldest first -> this, us: packed
+    // 256 heads, N = 512 17.1 -> 15.5, causal 16.1 -> 14.5, blocks with a map 13.1 -> 11.8;  128, N = 1024 29.5 -> 27.2;  boolean 512, N = 256 13.9 -> 13.0, 132, N = 700 25.5 -> 23.0, 74, N = 1500
+    // 53.1 -> 50.9;  fp32 149, N = 700 36.9 -> 34.7.  Not with a map of more than one word, from whose first alone a wavefront knows the visits ahead of it (32 heads, N = 4096, causal 55.5 -> 59.6).
+    // The rest of the launcher stays with three: the deal keeps heads in turn on such a grid (its ends taken for a second round; without, 128, N = 1024, causal 18.1 -> 26.3), and the
+    // boolean mask its pairs of tiles (one tile's bytes: 512, N = 256 13.0 -> 12.3, but 74, N = 1500 50.9 -> 58.3).
+    const bool four = D == 32 && !byproducts && (a.tile_map == nullptr || a.N <= 32 * BN);
+    a.tail_start = (!split && groups > 2 * cus && groups <= (four ? 4 : 3) * cus) ? 0 : (int)groups;
     a.groups = (int)groups;
     const dim3 grid((unsigned)groups), block(NTHREADS);
     const bool postmul = a.post_mul != 1.0f;
     const bool packed = a.D == D && (int)a.q.sn == D && (int)a.k.sn == D && (int)a.v.sn == D;
     if (!three) a.tail_start = (int)groups;                   // two work-groups per CU: nobody yields
-    // two tiles' mask bytes per request (see PAIRS at the kernel), unless the grid is the single round of work-groups in
+    // two tiles' mask bytes per request (see PAIRS at the kernel), unless the grid is the single round of three work-groups on a CU in
     // step for which tail_start was set to 0 above
-    const bool further = !split && a.byte_mask && D <= HD && (halves || a.tail_start != 0);
+    const bool further = !split && a.byte_mask && D <= HD && (halves || a.tail_start != 0 || groups > 3 * cus);
     if (a.q_f32 && !bf16) return hipErrorInvalidValue;         // fp32 callers compute in bf16
     if (a.byte_mask && a.N < 16) return hipErrorInvalidValue;  // a row holds at least one 16-byte copy (checked by the C-ABI layer)
     const int mask_kind = (split ? 5 : halves ? 10 : 0) + (!a.byte_mask ? 0 : (!further ? 1 : a.N % (2 * BN) == 0 ? 3 : 8) + (byproducts ? 1 : 0));

@@ -150,7 +150,7 @@ struct AttnArgs {
     float post_mul;
     uint32_t last_mask0, last_mask1;   // valid-bit masks of the two mask words of the last key tile
     // Work-groups with a linear id >= tail_start lower their waves' priority as they advance, so
-    // that the (up to three) work-groups of a CU finish together instead of oldest first.  The
+    // that the (up to four) work-groups of a CU finish together instead of oldest first.  The
     // launcher sets 0 when the whole grid is resident at once, else the grid size (nobody yields).
     int tail_start;
 };

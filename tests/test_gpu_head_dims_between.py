@@ -6,7 +6,7 @@ import sys
 import pytest
 import torch
 
-from _launches import launches
+from _launches import launches, places
 from oracle import sma_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -112,6 +112,35 @@ def test_short_rows_of_the_second_half(dev, heads, N, D, dtype):
         assert torch.equal(out, x)
     # the bound of the work-groups of 64 rows: the probabilities and the result are rounded once each, relative to the largest value of a row's mean
     eps = 2.0 ** (-10 if dtype == torch.float16 else -7)
+    for h in (0, heads - 1):
+        one = [t[:, h:h + 1].double() if dtype != torch.float32 else t[:, h:h + 1].bfloat16().double() for t in (q, k, v)]
+        x = ((one[0] * D ** -0.5) @ one[1].transpose(-1, -2)).masked_fill(~mask, float("-inf"))
+        ref = torch.softmax(x, -1).nan_to_num() @ one[2]
+        shift = (eps * (one[0].abs() * D ** -0.5) @ one[1].abs().transpose(-1, -2)).masked_fill(~mask, 0).amax(-1)
+        assert ((out[:, h:h + 1].double() - ref).abs() <= 1e-4 + one[2].abs().max() * (4 * eps + 2 * shift[..., None])).all()
+
+
+# Head dim 32 in one round of more than three work-groups on a CU, which four share: wavefronts yield to each other as they advance, by the visits that a map of one
+# word leaves them (a longer map: they don't).  Whole tiles and a last one of one key, pairs of tiles that end in either of theirs.
+@pytest.mark.parametrize("N, tiles", [(257, 3), (320, 3), (512, 4), (700, 6), (2048, 16), (2100, 17)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_one_round_of_four_on_a_cu(dev, N, tiles, dtype):
+    importlib.import_module("python.sparse_attention")
+    sa = sys.modules["python.sparse_attention"]
+    D, heads = 32, 4 * places() // tiles
+    assert 3 * places() < heads * tiles <= 4 * places()
+    g = torch.Generator(device=dev).manual_seed(N)
+    q, k, v = (torch.randn(1, heads, N, D, device=dev, generator=g).to(dtype) for _ in range(3))
+    nb = (N + 63) // 64
+    mask = torch.rand(1, 1, N, N, device=dev, generator=g) < 0.3
+    mask &= (torch.rand(1, 1, nb, nb, device=dev, generator=g) < 0.5).repeat_interleave(64, 2)[:, :, :N].repeat_interleave(64, 3)[..., :N]
+    mask[..., 3, :] = False
+    packed = sa.pack_mask(mask)
+    out = sa.sparse_attention_func(q, k, v, mask)
+    for x in (sa.sparse_attention_func(q, k, v, None, mask_packed=packed),
+              sa.sparse_attention_func(q, k, v, None, mask_packed=packed, tile_map=sa.tile_map(packed, min_skip=0.0))):
+        assert torch.equal(out, x)
+    eps = 2.0 ** (-10 if dtype == torch.float16 else -7)               # the bound of the short rows' test
     for h in (0, heads - 1):
         one = [t[:, h:h + 1].double() if dtype != torch.float32 else t[:, h:h + 1].bfloat16().double() for t in (q, k, v)]
         x = ((one[0] * D ** -0.5) @ one[1].transpose(-1, -2)).masked_fill(~mask, float("-inf"))
