@@ -297,7 +297,7 @@ int sma_attn_bwd_map_strided(const sma_tensor *dout, const sma_tensor *q, const 
 
 /* Forward and backward with everything optional in one argument block, for what the functions above do
  * not take: any head dim that is a multiple of 8 up to 128 without padding copies (the kernels exist
- * for 32, 64, 96 and 128; D = 80 runs in the one for 96), and fp32 results next to or instead of the
+ * for 32, 64, 80, 96 and 128; D = 72 runs in the one for 80), and fp32 results next to or instead of the
  * bf16 ones (the rounded bf16 values widened; dtype must be bf16), for callers that keep fp32 tensors.
  * Pointers that are marked optional may be NULL; everything else is as in sma_attn_fwd_map_strided,
  * sma_attn_fwd_bool_mask_strided and sma_attn_bwd_map_strided.

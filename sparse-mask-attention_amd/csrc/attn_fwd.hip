@@ -1,4 +1,4 @@
-// Fused masked-attention forward for gfx950 (MI355X), head_dim 32, 64, 96 or 128, fp16 / bf16, fp32 accumulate.
+// Fused masked-attention forward for gfx950 (MI355X), head_dim 32, 64, 80, 96 or 128, fp16 / bf16, fp32 accumulate.
 //
 // Stands in for sparse_attn_wmma_full_fp16 (csrc/sparse_attention.cu:82-412 of the reference) and
 // for its scalar bf16 kernel (csrc/sparse_attention.cu:418-543); the design below is specific to
@@ -93,9 +93,12 @@ constexpr float SUM_LIMIT = 16384.0f;     // a lane's 32 weights of a tile sum t
 // or 24 KiB instead of 32, which is what lets three work-groups share a CU (see three_on_a_cu).  Whole rows -> this with two on a CU all the same: D = 80, 512 heads, N = 320 33.7 ->
 // 32.4 us, N = 512 67.1 -> 65.4; D = 96 36.4 -> 35.9, 69.9 -> 68.5.  64 bytes where by-products are asked for at 80 (two on a CU: 32, whose reads of K's last step
 // meet in a bank, cost 64 heads, N = 1500 in training 281 -> 285 us, 64 282), and whole rows for fp32 queries at 96 (64, N = 1500 104.0 -> 109.5).
-// Head dim 32, two requests a tile instead of four, stages of 8 KiB instead of 16, with which the boolean mask's bytes leave room for four work-groups on a CU instead of three, whole rows -> this:
+// Head dim 32, two requests a tile instead of four, stages of 8 KiB instead of 16, with which the boolean mask's bytes leave room for four work-groups on a CU instead of three (the packed words did already; with by-products
+// 132 to 137 registers keep it at three, and in 128 of them 2 to 34 are spilled: the forward of a training step, 2048 heads, N = 100 19.0 -> 19.6 us, 256, N = 512 24.0 -> 22.5), whole rows -> this:
 // boolean 2048 heads, N = 32 11.6 -> 9.8 us, N = 100 16.1 -> 14.5, N = 200 45.7 -> 42.3;  256, N = 1000 78.3 -> 73.4;  192, N = 1024 55.2 -> 52.6;  packed 2048, N = 200 33.2 -> 31.5, 128, N = 2048 96.4 -> 93.8,
-// causal 60.5 -> 60.3;  where two tiles a head of whole rows are all there is 3 % slower, at 4.4 TB/s (2048, N = 128, packed 14.8 -> 15.2; boolean 18.2 -> 17.9; N = 112 13.3 -> 13.0).
+// causal 60.5 -> 60.3;  2048, N = 128 boolean 18.2 -> 17.9.  Two packed tiles a head that are all but full, all bytes at 4.8 TB/s, win and lose by the number of work-groups on a CU, with inputs in the caches (from memory):
+// N = 128, seven 12.8 -> 13.4 (13.6 -> 13.6), eight 14.5 -> 14.6 (15.3 -> 15.4), nine 15.7 -> 16.5 (17.3 -> 17.4), twelve 19.0 -> 19.2 (23.8 -> 22.6);  N = 120, 7 12.4 -> 12.7 (12.4 -> 12.7), 12 19.0 -> 18.6, 24 39.6 -> 38.8;
+// an instance with whole rows for them gave as much back as it got.
 constexpr int second_row(int hdim, bool split, bool byproducts, bool wide_q)
 {
     return hdim == 32 ? (split ? 0 : 64) : hdim <= 64 ? 0 : split || hdim == 128 || (hdim == 96 && wide_q) ? 128 : hdim == 96 || byproducts ? 64 : 32;
@@ -1486,13 +1489,17 @@ hipError_t launch_attn_fwd(const AttnArgs &args, bool bf16, hipStream_t stream)
         }
     }
     // Beyond that line work-groups of 64 rows (HALVES at the kernel), `g64` of them:
-    //   head dims beyond 64, where two share a CU: while one on a CU holds them all.  With two on a CU they lose (8 x 8 heads, N = 512, D = 128: 17.0 -> 17.8 us;
-    //       32, N = 1024 22.9 -> 23.1, boolean 24.7 -> 25.3), but at head dim 96 from 1024 rows on, where they gain as long as these are one round: 10 heads, N = 2048
-    //       35.5 -> 30.7 (boolean 39.5 -> 36.6, untouched masks 42.1 -> 39.9), 32, N = 1024 20.5 -> 19.5 (22.3 -> 22.0, 24.7 -> 24.8); 64, N = 512 13.5 -> 14.0;
-    //   up to 64, where three do: when they are one round of two to three on a CU and work-groups of 128 rows would be one on some CUs and two on others.  Up
+    //   head dims beyond 64: while one on a CU holds them all.  With two on a CU they lose at 128 (8 x 8 heads, N = 512: 17.0 -> 17.8 us;
+    //       32, N = 1024 22.9 -> 23.1, boolean 24.7 -> 25.3), but up to 96 they gain from 1024 rows on, as long as these are one round.  D = 96: 10 heads, N = 2048
+    //       35.5 -> 30.7 (boolean 39.5 -> 36.6, untouched masks 42.1 -> 39.9), 32, N = 1024 20.5 -> 19.5 (22.3 -> 22.0, 24.7 -> 24.8); 64, N = 512 13.5 -> 14.0.  D = 80: 16, N = 2048
+    //       32.9 -> 30.9 (boolean 36.3 -> 34.7, with by-products 41.3 -> 39.3, blocks with a map 23.0 -> 16.5, causal 31.6 -> 29.5), 20, N = 1600 36.5 -> 25.6 (boolean 39.5 -> 28.5); one loses
+    //       there, 8, N = 4000 with by-products 81.5 -> 88.7.  Up to three on a CU, where that many share one at 80 and 96 (three_on_a_cu), by-products, which leave it at two, lose: D = 80, 24, N = 2000 packed
+    //       47.2 -> 43.0, but boolean 55.9 -> 62.9, a training step 207 -> 235;
+    //   up to 64, where three share a CU: when they are one round of two to three on a CU and work-groups of 128 rows would be one on some CUs and two on others.  Up
     //       to two on a CU, packed masks gain and boolean ones lose (32 heads, N = 1024: 16.4 -> 15.2; untouched 18.3 -> 18.7), and with a second
-    //       round all do (28, N = 2048: 40.7 -> 45.8, boolean 44.6 -> 61.5).  Beyond ten tiles, where the chain is most of a call: 48, N = 1024 24.2 -> 20.3, 160, N = 256
-    //       9.7 -> 8.9; and a training step on up to 640 rows, whose backward holds whole heads, keeps a head's bits however many heads there are.
+    //       round all do (28, N = 2048: 40.7 -> 45.8, boolean 44.6 -> 61.5; any number of rounds, but with a map only: blocks 192, N = 1024 36.9 -> 36.4, 384, N = 512 25.2 -> 27.0, causal
+    //       42.6 -> 51.2).  Beyond ten tiles: 48, N = 1024 24.2 -> 20.3.  Shorter ones keep the order of their sums from before this rule; by time it could begin at four tiles (D = 64, N = 200
+    //       to 640: 7 to 18 % less, blocks with a map up to 27; three tiles packed 7.6 -> 7.8).
     // Up to 128 keys there is nothing to share (6.6 us either way).  The split stays ahead where it fits: 8 heads, N = 1024 16.9 against 21.3 us.
     const long long g64 = (long long)a.BH * ((a.N + 63) / 64);
     const bool halves = !split && a.N > 2 * BN &&

@@ -596,10 +596,10 @@ void refuse_tangents(const Tensor &q, const Tensor &k, const Tensor &v)
 //   inference from 2^20 elements on -8 to +0.5 % (200 grids): 64, 256, 64 12.5 -> 11.7;  192, 512, 128 75.8 -> 69.8;  128, 1000, 32 51.0 -> 49.8.  0.8 to
 //             1 million: -6 to +4 %, -1 to -3 on average;  around 0.72 million -1.4 % on average at head dim 64, +0.5 at 128.  Below: 64, 128, 64
 //             9.2 -> 9.7;  128, 128, 32 9.3 -> 9.6;  64, 64, 128 9.4 -> 10.1
-//   training  (from 2^20 elements on) it also writes the rounded rows.  Long sequences hide that: 160, 768, 128 113.5 -> 108.2;  96, 512, 80 36.7 -> 34.7;
-//             200, 1024, 64 117 -> 112;  at worst 300, 512, 80 92.3 -> 94.1.  Short ones don't (512, 64, 128 24.6 -> 27.3;  200, 320, 80 43.7 -> 47.3;
-//             192, 200, 128 33.5 -> 34.2), nor does head dim 32 (300, 512 42.3 -> 43.9), and where every head has a boolean mask of its own, whose bytes
+//   training  (from 2^20 elements on) it also writes the rounded rows.  Long sequences hide that: 160, 768, 128 113.5 -> 108.2;  200, 1024, 64 117 -> 112.  Short ones don't (512, 64, 128 24.6 -> 27.3;  192, 200, 128 33.5 -> 34.2), nor does head dim 32 (300, 512 42.3 -> 43.9), and where every head has a boolean mask of its own, whose bytes
 //             bound it, nothing is gained (200, 600, 64 72.1 -> 77.1;  96, 1024, 64 69.0 -> 67.5)
+//   with the kernels for 80, GPU time: inference 32, 512, 80 18.4 -> 17.0;  100, 256, 80 21.2 -> 19.1;  around the line 40, 256 12.4 -> 11.9;  below it 24, 256 10.4 -> 10.6;  12, 512
+//             12.5 -> 12.7.  Whole training steps 96, 512, 80 88.5 -> 86.4;  300, 512 227 -> 222;  48, 2048 343 -> 339;  below 512 keys 200, 320 109 -> 111, packed 107 -> 104;  64, 448 59.7 -> 58.4
 bool forward_rounds_q(const Call &c, const Tensor &q, bool training)
 {
     if (!training) return q.numel() >= 11 * (int64_t(1) << 16);

@@ -29,7 +29,7 @@ What differs from the reference, on purpose:
   size and shared between batch entries / heads by the kernels (the reference needs the expanded
   ``[B, H, N, N]`` tensor).  A mask passed as an ``expand``-ed view is recognised by its zero
   strides and treated the same way.
-* Head dims: the kernels exist for 64 (the reference's only one), 32, 96 and 128.  Any multiple of 8 in
+* Head dims: the kernels exist for 64 (the reference's only one), 32, 80, 96 and 128.  Any multiple of 8 in
   between runs in the next larger one as it is; any other D <= 128 is computed exactly by zero-padding q, k, v (the
   scores and the first D output columns do not change; the scale stays 1/sqrt(D)) at the price of the padding copies.
 * The mask is not packed in a pass of its own: where the kernel's limits allow (any q, k, v the strided kernels take,
